@@ -295,6 +295,19 @@ int tppx_linear_mxfp4_int8_rows(const void* x, const void* q_nat,
                                 int post_op, float post_scale,
                                 tppx_stream_t stream);
 
+/* W4A8 between the two: 17 rows up to the prompt passes (any M is taken; also fewer rows that do not fit the call
+ * above), on the same prepacked weights.  The rows are quantized into xq / sa first (operand order, private to the
+ * library): xq holds roundup(M, 64) * K bytes, sa roundup(M, 64) * K / 32 floats, both 16-byte aligned.
+ * TPPX_FLAG_XQ_REUSE: xq / sa still hold this x from an earlier call with the same M and K.  Same arithmetic in
+ * another summation order. */
+int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa,
+                               const void* q_nat, const void* s_nat,
+                               const void* bias, const void* post_in,
+                               const void* post_in2, void* y, int64_t M,
+                               int64_t N, int64_t K, int post_op,
+                               float post_scale, int flags,
+                               tppx_stream_t stream);
+
 /* W4A8 with many rows (prompt passes): the same arithmetic on the bf16 MFMA.  An int8 activation and a weight
  * integer times its block's power of two are exact in bf16 and so is the fp32 sum of one MX block's 32 products, so
  * one K = 32 MFMA per block gives float(int32 block sum) * 2^(e - 127) and the fold is one fp32 multiply-add with

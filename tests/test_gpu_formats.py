@@ -508,3 +508,26 @@ def test_packed_code_decode_kernel_equals_expanded_weight(kind, M, N, K, post, m
     y_expanded = ops.linear(x, qt, b, posts[post], r, None, 0.5)
     assert torch.equal(y, y_expanded), "packed codes and expanded int8 tiles give different bits"
 
+
+
+@pytest.mark.parametrize("M,N,K,bc,post", [(17, 96, 1280, 64, "none"), (32, 4096, 128, 32, "add"), (33, 8448, 1536, 64, "silu"),
+                                           (63, 272, 4096, 128, "mul"), (16, 4096, 11008, 64, "none"), (40, 11008, 512, 64, "none")])
+def test_w4a8_row_group_kernel(M, N, K, bc, post):
+    """W4A8 between the decode and the prompt kernels (17..63 rows, and rows that do not fit the decode kernel's LDS):
+    within 1 bf16 ulp (2 through SiLU) of the oracle, which adds the same exact block products in K order; the gate/up
+    pair, which quantizes its rows once, equals the two calls."""
+    ops = _ops()
+    posts = {"none": O.POST_NONE, "add": O.POST_ADD_SCALE, "silu": O.POST_SILU, "mul": O.POST_MUL}
+    W = randn_bf16((N, K), 0.05, 3100 + M)
+    t = W.view(N // 16, 16, K // bc, bc // 2, 2).permute(0, 2, 3, 1, 4).contiguous()
+    qt = ops.remap_and_quantize_mxfp4(t.cuda(), int8_layout=True)
+    q_or, s_or = O.remap_quantize_mxfp4_int8(t.float().numpy())
+    x = randn_bf16((M, K), 1.0, 3110 + M)
+    x[M - 1, :64] = 0.0
+    b, r = randn_bf16((N,), 0.01, 3120), randn_bf16((M, N), 1.0, 3130)
+    y = ops.linear(x.cuda(), qt, b.cuda(), posts[post], r.cuda(), None, 0.5)
+    ref = O.linear_w4a8(t2bits(x), q_or, s_or, bc, t2bits(b), posts[post], t2bits(r), None, 0.5)
+    pre = O.linear_w4a8(t2bits(x), q_or, s_or, bc, t2bits(b)) if post in ("add", "mul") else None
+    assert_close_bf16(t2bits(y), ref, ulps=2 if post == "silu" else 1, what=f"w4a8 rows M={M} N={N} K={K} {post}", pre_bits=pre)
+    assert torch.equal(ops.swiglu_gate_up(x.cuda(), qt, qt, b.cuda(), b.cuda()),
+                       ops.fc_mul(x.cuda(), qt, b.cuda(), ops.fc_silu(x.cuda(), qt, b.cuda())))

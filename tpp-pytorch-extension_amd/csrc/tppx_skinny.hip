@@ -83,7 +83,9 @@ __device__ unsigned int sk_split_tickets[SK_TICKETS];
 // cross-wave sums then unroll completely and all of a thread's LDS reads are issued before the first wait; with a
 // run-time count the compiler waited for the LDS once per output and batch of eight (36 waits of an LDS round trip
 // each in the 64-row gate/up epilogue: 1.3 us per half).
-template <int MG, int NACC, bool DUAL, int MINW, int FIXW = 0>
+// TR (finish() only): the accumulators are transposed result tiles -- lane l holds channels (l >> 4) * 4 + r of row
+// l & 15 (weights as the MFMA's first operand) -- written into the same region as one 16-byte store per tile.
+template <int MG, int NACC, bool DUAL, int MINW, int FIXW = 0, bool TR = false>
 struct SkEpilogue {
   static __device__ __forceinline__ int nthreads() { return FIXW ? FIXW * 64 : (int)blockDim.x; }
   static __device__ __forceinline__ int nwaves() { return FIXW ? FIXW : (int)(blockDim.x >> 6); }
@@ -343,10 +345,15 @@ struct SkEpilogue {
 #pragma unroll
     for (int a = 0; a < NACC; a++)
 #pragma unroll
-      for (int mg = 0; mg < MG; mg++)
+      for (int mg = 0; mg < MG; mg++) {
+        if constexpr (TR) {
+          *reinterpret_cast<f32x4*>(mine + (a * MG + mg) * 256 + (lane & 3) * 64 + ((lane >> 2) & 3) * 16 + (lane >> 4) * 4) = acc[a][mg];
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-          mine[(a * MG + mg) * 256 + r * 64 + lane] = acc[a][mg][r];
+          for (int r = 0; r < 4; r++)
+            mine[(a * MG + mg) * 256 + r * 64 + lane] = acc[a][mg][r];
+        }
+      }
     __syncthreads();
     // (no branch per output: slots past the outputs repeat the last one and are not stored, so the outputs' LDS reads
     // and post-op chains interleave)
@@ -1597,6 +1604,122 @@ skinny_w4a8_kernel(const DecodeParams p) {
 }
 
 // ---------------------------------------------------------------------------
+// W4A8, 17..64 rows per block row (and fewer rows that do not fit the kernel above's LDS).  The rows arrive quantised
+// in operand order (quant_act_w4a8_rows_kernel): xq [K/128][mt][2 halves][64 lanes (g, m)][16 B], 8 bytes of each of
+// two MX blocks per lane, and scales sa [K/128][mt][16 m][4 blocks] f32, already times 6 / 127.  Eight waves split K
+// in tiles of 128 channels; weight tiles and their E8M0 dwords as in skinny_w4a8_kernel.  The weights are the MFMA's
+// FIRST operand, so a result tile is [channel][row]: a lane's four sums belong to one row, whose four block scales of
+// a K tile are one 16-byte load, and no scale goes through LDS.
+// What bounds it: vector issue.  Every K = 32 MFMA (one MX block) leaves 4 sums per lane to convert, scale and add
+// (12 instructions) behind the expansion of the codes (about 18, shared by the MG row tiles); the weight stream
+// (24 MB at 11008 x 4096) hides behind that from 32 rows on.  Whole calls with the quantizer, back to back: 32 rows
+// 18 us, 63 rows 23 us at 11008 x 4096 (73 and more on one wave per 16 x 16 tile, which this kernel replaces wherever
+// the weight could be prepacked); the SwiGLU block 4096 - 11008 - 4096 at 32 rows 171 -> 47 us.
+// ---------------------------------------------------------------------------
+template <int MG, int NTW, int PF>
+__global__ void __launch_bounds__(512)
+skinny_w4a8_mg_kernel(const DecodeParams p) {
+  extern __shared__ __align__(16) float sk_lds[];
+  constexpr int W = 8;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = blockIdx.x;
+  const DecodeSeg& sg = p.seg[sk_find_seg(p, grp)];
+  const int ltile0 = (grp - sg.grp0) * NTW;
+  const int m0 = blockIdx.y * (MG * 16);
+  const int KT = p.units; // K tiles of 128 channels
+  const int t0 = (wave * KT) / W, t1 = ((wave + 1) * KT) / W;
+
+  const i32x4* wq[NTW];
+  const i32x4* ws[NTW]; // E8M0 dwords of four channels
+#pragma unroll
+  for (int nt = 0; nt < NTW; nt++) {
+    const int64_t lt = min(ltile0 + nt, sg.tiles - 1); // ragged last group: duplicate, not stored
+    wq[nt] = reinterpret_cast<const i32x4*>(sg.qw) + lt * KT * 64;
+    ws[nt] = reinterpret_cast<const i32x4*>(sg.sw) + lt * KT * 4;
+  }
+  const i32x4* xop = reinterpret_cast<const i32x4*>(p.xq) + (int64_t)blockIdx.y * MG * 128;
+  const f32x4* sop = reinterpret_cast<const f32x4*>(p.sa) + (int64_t)blockIdx.y * MG * 16;
+  const int xstride = p.mt * 128, sstride = p.mt * 16;
+
+  i32x4 wreg[PF][NTW], sreg[PF][NTW], xreg[PF][MG][2];
+  f32x4 areg[PF][MG];
+  // (past the end, or a wave without tiles: re-read a valid tile that is never consumed -- no branch around a load)
+  auto load_w = [&](int st, int t) {
+    t = max(min(t, t1 - 1), 0);
+#pragma unroll
+    for (int nt = 0; nt < NTW; nt++) {
+      wreg[st][nt] = __builtin_nontemporal_load(wq[nt] + (int64_t)t * 64 + lane);
+      sreg[st][nt] = (ws[nt] + (int64_t)t * 4)[lane >> 4];
+    }
+  };
+  auto load_x = [&](int st, int t) {
+    t = max(min(t, t1 - 1), 0);
+#pragma unroll
+    for (int mg = 0; mg < MG; mg++) {
+      xreg[st][mg][0] = (xop + (int64_t)t * xstride + mg * 128)[lane];
+      xreg[st][mg][1] = (xop + (int64_t)t * xstride + mg * 128 + 64)[lane];
+      areg[st][mg] = (sop + (int64_t)t * sstride + mg * 16)[lane & 15];
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < PF; i++) {
+    load_w(i, t0 + i);
+    load_x(i, t0 + i);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  SkEpilogue<MG, NTW, false, W, W, true> ep;
+  ep.prefetch_flat(p, sg, ltile0, m0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  f32x4 facc[NTW][MG];
+#pragma unroll
+  for (int nt = 0; nt < NTW; nt++)
+#pragma unroll
+    for (int mg = 0; mg < MG; mg++)
+      facc[nt][mg] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto consume = [&](int i) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+#pragma unroll
+      for (int nt = 0; nt < NTW; nt++) {
+        const uint32_t codes = (uint32_t)wreg[i][nt][j];
+        const uint32_t lo = w4a8_expand(codes & 0x0F0F0F0Fu), hi = w4a8_expand((codes >> 4) & 0x0F0F0F0Fu);
+        const long wb = (long)(((uint64_t)hi << 32) | lo);
+        float wsc[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          wsc[r] = e8m0_to_f32((uint32_t)sreg[i][nt][r] >> (8 * j));
+#pragma unroll
+        for (int mg = 0; mg < MG; mg++) {
+          const long xa = (long)(((uint64_t)(uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2 + 1] << 32) |
+                                 (uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2]);
+          const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, xa, i32x4{0, 0, 0, 0}, 0, 0, 0);
+          const float sav = areg[i][mg][j];
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            facc[nt][mg][r] = fmaf((float)acc[r], sav * wsc[r], facc[nt][mg][r]);
+        }
+      }
+    }
+  };
+  int t = t0;
+  for (; t + PF <= t1; t += PF) { // branch-free full trips (reloads past the end are clamped re-reads)
+#pragma unroll
+    for (int i = 0; i < PF; i++) {
+      consume(i);
+      load_w(i, t + i + PF);
+      load_x(i, t + i + PF);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < PF - 1; i++) // fewer than PF left: their tiles are in the stages a trip would use
+    if (t + i < t1)
+      consume(i);
+  ep.finish(sg, facc, sk_lds);
+}
+
+// ---------------------------------------------------------------------------
 // MXFP4, M <= 16, activations staged in LDS by the wave that consumes them,
 // with an optional transform on the way in:
 //   XMODE 0  x as it is
@@ -2575,6 +2698,21 @@ hipError_t launch_skinny_w4a8(DecodeParams& p, int ntw, hipStream_t stream) {
     case 2: return sk_launch(skinny_w4a8_kernel<2, 2, 4, 16>, p, grid, 16, lds, stream);
     default: return sk_launch(skinny_w4a8_kernel<3, 4, 4, 8>, p, grid, 8, lds, stream);
   }
+}
+
+// W4A8, 17..64 rows per block row: mg = 2 / 4 row groups, ntw = 1..3 channel tiles per workgroup; p.mt, p.units, p.groups
+// set by the caller
+hipError_t launch_skinny_w4a8_mg(DecodeParams& p, int mg, int ntw, hipStream_t stream) {
+  if (p.S != 1 || p.mt <= 0 || (mg != 2 && mg != 4) || ntw < 1 || ntw > 3)
+    return hipErrorInvalidValue;
+  dim3 grid(p.groups, (p.M + mg * 16 - 1) / (mg * 16), 1);
+  const size_t lds = (size_t)8 * ntw * mg * 256 * sizeof(float);
+#define SKWM(MG, NTW)          \
+  if (mg == MG && ntw == NTW) \
+    return sk_launch(skinny_w4a8_mg_kernel<MG, NTW, 2>, p, grid, 8, lds, stream);
+  SKWM(2, 1) SKWM(2, 2) SKWM(2, 3) SKWM(4, 1) SKWM(4, 2) SKWM(4, 3)
+#undef SKWM
+  return hipErrorInvalidValue;
 }
 
 // MXFP4, 33..64 rows per block row: four channel tiles x four K parts per workgroup, K in p.S slices across workgroups

@@ -143,6 +143,47 @@ quant_act_w4a8_wide_kernel(const uint16_t* __restrict__ x, int M, int K, int MT1
     sa[((((int64_t)kt * (MT16 >> 2) + (mt >> 2)) * 4 + b) * 16 + m16) * 4 + (mt & 3)] = __fmul_rn(sc, (float)(6.0 / 127.0));
 }
 
+// The same bytes for skinny_w4a8_mg_kernel (17..63 rows): int8 in its operand order, see there.
+__global__ void __launch_bounds__(256)
+quant_act_w4a8_rows_kernel(const uint16_t* __restrict__ x, int M, int K, int mtiles, uint2* __restrict__ xq,
+                           float* __restrict__ sa) {
+  // one workgroup per (row tile of 16, K tile of 128); thread = (m = tid & 15, g = tid >> 4 & 3, b = tid >> 6)
+  const int tid = threadIdx.x, m16 = tid & 15, g = (tid >> 4) & 3, b = tid >> 6;
+  const int mt = blockIdx.x, kt = blockIdx.y;
+  const int m = min(mt * 16 + m16, M - 1);
+  const uint4 raw = *reinterpret_cast<const uint4*>(x + (int64_t)m * K + kt * 128 + b * 32 + g * 8);
+  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+  float v[8];
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    v[2 * i] = bf16_bits_to_f32(w[i] & 0xffffu);
+    v[2 * i + 1] = bf16_bits_to_f32(w[i] >> 16);
+    amax = fmaxf(amax, fmaxf(fabsf(v[2 * i]), fabsf(v[2 * i + 1])));
+  }
+  amax = fmaxf(amax, __shfl_xor(amax, 16, 64)); // the four lanes (g) of a (row, block)
+  amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+  const float sc = __fdiv_rn(amax, 127.0f); // quantize_int8sym: scale = max / 127, q = rint(v * (1 / scale))
+  const float inv = sc != 0.0f ? __frcp_rn(sc) : 0.0f;
+  uint32_t o[2] = {0, 0};
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const int q = (int)fminf(fmaxf(rintf(__fmul_rn(v[i], inv)), -127.0f), 127.0f);
+    o[i >> 2] |= ((uint32_t)q & 0xffu) << (8 * (i & 3));
+  }
+  const int64_t tile = (int64_t)kt * mtiles + mt;
+  xq[((tile * 2 + (b >> 1)) * 64 + g * 16 + m16) * 2 + (b & 1)] = make_uint2(o[0], o[1]);
+  if (g == 0)
+    sa[(tile * 16 + m16) * 4 + b] = __fmul_rn(sc, (float)(6.0 / 127.0));
+}
+
+hipError_t launch_quant_act_w4a8_rows(const void* x, int64_t M, int64_t K, int mt, void* xq, float* sa, hipStream_t stream) {
+  const dim3 grid(mt, (unsigned)(K / 128));
+  TPPX_PLAN_ONLY(quant_act_w4a8_rows_kernel, grid, dim3(256), 0);
+  quant_act_w4a8_rows_kernel<<<grid, 256, 0, stream>>>((const uint16_t*)x, (int)M, (int)K, mt, (uint2*)xq, sa);
+  return hipGetLastError();
+}
+
 __global__ void __launch_bounds__(256)
 prepack_w4a8_wide_kernel(const uint32_t* __restrict__ qref, const uint8_t* __restrict__ sref, int64_t N, int64_t K,
                          int64_t bc, uint4* __restrict__ wn) {

@@ -610,10 +610,23 @@ W4A8_DECODE = os.environ.get("TPPX_W4A8_DECODE", "1") == "1"
 W4A8_WIDE_ROWS = int(os.environ.get("TPPX_W4A8_WIDE_ROWS", "64"))
 
 
-def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale):
+def _w4a8_block_rows(M, N, K):
+    """Does a W4A8 call of 17 or more rows run as block rows of 64 on the row-group kernel (which streams the 4-bit
+    weights once per block row) rather than on the prompt kernel (2 bytes per weight, all of K per workgroup)?
+    Fits in us, measured with the activation quantizer included: a block row 19 / 20 / 11 at 11008 x 4096,
+    4096 x 11008 and 4096 x 4096; the prompt kernel 45 / 92 / 36 up to one workgroup of 64 x 128 per CU."""
+    if M < W4A8_WIDE_ROWS:
+        return True
+    rows64 = (M + 63) // 64
+    wgs = rows64 * ((N + 127) // 128)
+    return rows64 * (7.2 + N * K / 4.0e6) < (3.0 + K * 0.0081) * max(1.0, wgs / 220)
+
+
+def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=None):
     """TppBlockedLinearW<int8_t, uint8_t, Tout> (src/csrc/fused_gemm.h:965-978, 1523-1526): bf16 activations are
     quantized to int8 over blocks of 32 (quantize_int8sym with the weight's block size), the scales multiplied by
-    6/127, and the GEMM runs on int8 against the MXFP4 weight in its VNNI8 layout."""
+    6/127, and the GEMM runs on int8 against the MXFP4 weight in its VNNI8 layout.
+    rows: a list shared by consecutive calls on the same input; the quantized rows are left in it and reused."""
     L = _lib.lib()
     _lib.require_gpu(input, "input")
     if input.dtype != torch.bfloat16:
@@ -631,17 +644,32 @@ def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale):
     post_in2 = _prep_post(post_in2, M, N, "second post-op input", x.device)
     # decode steps: one launch that quantizes its rows itself and splits K over the waves of a workgroup
     # (TPPX_W4A8_DECODE=0 keeps the two-step path)
-    nat = weight.native_w4a8() if (M <= 16 and W4A8_DECODE) else None
-    if nat is not None:
+    nat = weight.native_w4a8() if _w4a8_block_rows(M, N, K) else None
+    if nat is not None and M <= 16 and W4A8_DECODE:
         rc = L.tppx_linear_mxfp4_int8_rows(x.data_ptr(), nat[0].data_ptr(), nat[1].data_ptr(), _lib.ptr(bias),
                                            _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N, K, post, post_scale,
                                            _lib.stream_of(x))
         if rc != _lib.EUNSUPPORTED:  # rows that do not fit the kernel's LDS take the two-step path
             _lib.check(rc)
             return y
+    # up to the prompt passes: rows quantized into operand order by a launch of their own, then the row-group kernel
+    if nat is not None:
+        flags = _lib.FLAG_XQ_REUSE if rows else 0
+        if not rows:
+            mp = (M + 63) // 64 * 64
+            buf = torch.empty(mp * K + mp * (K // 8), dtype=torch.uint8, device=x.device)
+            held = (buf, buf.data_ptr(), buf.data_ptr() + mp * K)
+            if rows is not None:
+                rows.append(held)
+        else:
+            held = rows[0]
+        _lib.check(L.tppx_linear_mxfp4_int8_mid(x.data_ptr(), held[1], held[2], nat[0].data_ptr(), nat[1].data_ptr(),
+                                                _lib.ptr(bias), _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N,
+                                                K, post, post_scale, flags, _lib.stream_of(x)))
+        return y
     # prompt passes: rows and weights as bf16-coded integers on the bf16 MFMA, one fp32 multiply-add per block
     # (TPPX_W4A8_WIDE_ROWS: from how many rows; the weight keeps a second, 2-byte-per-value copy for it)
-    wide = weight.native_w4a8_wide() if M >= W4A8_WIDE_ROWS else None
+    wide = weight.native_w4a8_wide() if nat is None and M >= W4A8_WIDE_ROWS else None
     if wide is not None:
         mp = (M + 127) // 128 * 128
         ws = torch.empty(mp * K * 2 + mp * (K // 32) * 4, dtype=torch.uint8, device=x.device)
@@ -1010,6 +1038,10 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
     if not _one_launch_group([w_gate, w_up]):
         if norm is not None:
             input = rms_norm(input, norm[0], norm[1])
+        if _is_w4a8(w_gate) and _is_w4a8(w_up):
+            rows = []  # one quantization of the rows for both projections
+            gate = _linear_w4a8(input, w_gate, b_gate, POST_SILU, None, None, 1.0, rows)
+            return _linear_w4a8(input, w_up, b_up, POST_MUL, gate, None, 1.0, rows)
         return fc_mul(input, w_up, b_up, fc_silu(input, w_gate, b_gate))
     if norm is not None:
         _, M0, _, K0 = _prep_input(input, w_gate)

@@ -238,3 +238,29 @@ def test_quantize_int8sym_vnni_weight_and_create_qtensor():
     assert_close_bf16(t2bits(y), ref, what="fc_plain on create_qtensor_int8sym")
     want = O.dequantize_int8sym(val.numpy(), scl.numpy(), qbs, 2, True)
     assert np.array_equal(w.dequantize().cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "qint8", "qint2"])
+@pytest.mark.parametrize("N,K,bk,bc", [(32, 256, 16, 64), (800, 512, 100, 64), (96, 768, 32, 128), (64, 256, 4, 256), (96, 192, 2, 64)])
+def test_vnni2_quantizers_equal_the_general_ones(fmt, N, K, bk, bc):
+    """bf16 weights in the VNNI2 layout have quantizers of their own; the same values as fp32 in the 4-D layout take
+    the general ones.  Same bytes, for ordinary blocks and for all-zero, subnormal, tiny, tied, infinite and NaN ones."""
+    ops = _ops()
+    if fmt == "mxfp4" and bc != 64:
+        pytest.skip("not a layout of this format")
+    W = randn_bf16((N, K), 0.05, 5000 + N)
+    W[0, :64] = 0.0
+    W[1, :64] = -0.0
+    W[2, 3] = float("nan")
+    W[3, 0] = float("nan")
+    W[4, 40] = float("inf")
+    W[5, :32] = 1e-39
+    W[6, :32] = 2.0 ** -125
+    W[7, :32] = torch.tensor([6.0, 5.0, 2.5, 1.75, 3.5, 0.25, -0.25, 0.75] * 4)
+    W[8, :] = -6e-9
+    w5 = W.view(N // bk, bk, K // bc, bc // 2, 2).permute(0, 2, 3, 1, 4).contiguous().cuda()
+    w4 = W.float().view(N // bk, bk, K // bc, bc).permute(0, 2, 3, 1).contiguous().cuda()
+    q = {"mxfp4": ops.remap_and_quantize_mxfp4, "qint8": ops.remap_and_quantize_qint8, "qint2": ops.remap_and_quantize_qint2_intlv}[fmt]
+    a, b = q(w5), q(w4)
+    assert torch.equal(a.qdata, b.qdata)
+    assert torch.equal(a.scales.view(torch.uint8), b.scales.view(torch.uint8))

@@ -94,6 +94,96 @@ quantize_mxfp4_kernel(const T* __restrict__ w, int64_t N, int64_t K, int64_t bk,
   }
 }
 
+// ---- bf16 weights in the VNNI2 layout (what FixLinear blocks them into) ------------------------------------------
+// Dword (k pair c, channel n) of a [N/bk][K/bc][bc/2][bk][2] weight; `step` = dwords from one pair to the next while
+// the pairs stay inside a K block of bc.  The quantizers below read four adjacent channels of a pair with one 16-byte
+// load (bk a multiple of 4, so that the four lie in one block) and work the addresses out once per thread: with the
+// general addressing of the kernels above, four 64-bit divisions per element, they were bound by vector issue
+// (11008 x 4096, 90 MB read: MXFP4 102 us, QINT8 226, now 26 and 29; QINT2 28).  26 us is 4.4 TB/s in and out, about
+// what a large copy reaches.
+__device__ __forceinline__ int64_t vnni2_dword(uint32_t n, uint32_t k, uint32_t K, uint32_t bk, uint32_t bc) {
+  return ((int64_t)(n / bk) * (K / bc) + k / bc) * (bc / 2) * bk + (int64_t)((k % bc) / 2) * bk + n % bk;
+}
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
+__device__ __forceinline__ u16x2 abs_bf16x2(uint32_t w) { return __builtin_bit_cast(u16x2, w & 0x7fff7fffu); }
+
+// MXFP4: a thread owns 4 channels x 32 input channels = four MX blocks; a wave four [32 channels][64 K] tiles.  The
+// conversion is the hardware's (round to nearest even, saturating at 6: the same codes) except that it keeps the
+// sign of a zero, which is dropped here, and in waves with a block whose maximum is infinite, NaN or below 2^-124
+// (scale bytes 255 and 0), which take the general rule.
+__global__ void __launch_bounds__(256)
+quantize_mxfp4_vnni2_kernel(const uint32_t* __restrict__ w, uint32_t N, uint32_t K, uint32_t bk, uint32_t bc,
+                            uint8_t* __restrict__ qdata, uint8_t* __restrict__ scales) {
+  const uint32_t lane = threadIdx.x & 63, cg = lane & 7, h = (lane >> 3) & 1;
+  const uint32_t Nc = K / 64, ntiles = (N / 32) * Nc;
+  const uint32_t tile = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 4);
+  if (tile >= ntiles)
+    return;
+  const uint32_t nk = tile / Nc, nc = tile - nk * Nc;
+  const uint4* src = reinterpret_cast<const uint4*>(w + vnni2_dword(nk * 32 + cg * 4, nc * 64 + h * 32, K, bk, bc));
+  const uint32_t step = bk / 4;
+  uint32_t raw[16][4];
+#pragma unroll
+  for (int p = 0; p < 16; p++) {
+    const uint4 v = src[(int64_t)p * step];
+    raw[p][0] = v.x; raw[p][1] = v.y; raw[p][2] = v.z; raw[p][3] = v.w;
+  }
+  uint32_t x4 = 0, top[4];
+  bool odd = false;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    u16x2 m = abs_bf16x2(raw[0][c]);
+#pragma unroll
+    for (int p = 1; p < 16; p++)
+      m = __builtin_elementwise_max(m, abs_bf16x2(raw[p][c]));
+    top[c] = max((uint32_t)m[0], (uint32_t)m[1]) >> 7; // exponent of the largest magnitude
+    odd |= top[c] >= 255u || top[c] < 3u;
+    x4 |= (top[c] - 2u) << (8 * c);
+  }
+  uint32_t* out = reinterpret_cast<uint32_t*>(qdata) + ((int64_t)tile * 32 + h * 16) * 8 + cg;
+  uint32_t* sout = reinterpret_cast<uint32_t*>(scales) + ((int64_t)tile * 2 + h) * 8 + cg;
+  if (!__any(odd)) {
+    float sc[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      sc[c] = __uint_as_float((top[c] - 2u) << 23);
+#pragma unroll
+    for (int p = 0; p < 16; p++) {
+      uint32_t q = 0;
+      q = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(q, __builtin_bit_cast(bf16x2, raw[p][0]), sc[0], 0);
+      q = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(q, __builtin_bit_cast(bf16x2, raw[p][1]), sc[1], 1);
+      q = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(q, __builtin_bit_cast(bf16x2, raw[p][2]), sc[2], 2);
+      q = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(q, __builtin_bit_cast(bf16x2, raw[p][3]), sc[3], 3);
+      const uint32_t nz = (q | (q >> 1) | (q >> 2)) & 0x11111111u;
+      out[p * 8] = q & (0x77777777u | (nz << 3));
+    }
+    *sout = x4;
+    return;
+  }
+  // (values read again: held for this path too they would double the registers)
+  const uint32_t* s32 = reinterpret_cast<const uint32_t*>(src);
+  x4 = 0;
+#pragma unroll 1
+  for (int c = 0; c < 4; c++) {
+    auto value = [&](int j) { return bf16_bits_to_f32((s32[(int64_t)(j >> 1) * bk + c] >> (16 * (j & 1))) & 0xffffu); };
+    float amax = fabsf(value(0));
+#pragma unroll 1
+    for (int j = 1; j < 32; j++) {
+      const float a = fabsf(value(j));
+      amax = a > amax ? a : amax;
+    }
+    const int e = (int)((__float_as_uint(amax) >> 23) & 0xffu);
+    const int x = (e == 255) ? 255 : (e - 2 < 0 ? 0 : e - 2);
+    x4 |= (uint32_t)x << (8 * c);
+#pragma unroll 1
+    for (int p = 0; p < 16; p++) {
+      const uint32_t c0 = e2m1_encode(ldexpf(value(2 * p), 127 - x)), c1 = e2m1_encode(ldexpf(value(2 * p + 1), 127 - x));
+      reinterpret_cast<uint8_t*>(out + p * 8)[c] = (uint8_t)(e == 0 || x == 255 ? 0u : (c0 | (c1 << 4)));
+    }
+  }
+  *sout = x4;
+}
+
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1)
@@ -146,25 +236,92 @@ quantize_qint8_kernel(const T* __restrict__ w, int64_t N, int64_t K, int64_t bk,
   }
 }
 
+// The same for VNNI2 bf16 weights and scale blocks of 64 * NI channels: one wave per (16 channels, block), lane = (four
+// channels cg, K position s); step i covers 64 input channels, of which a lane holds the pairs 2s and 2s + 1 -- one
+// output dword per channel, so four channels leave as one 16-byte store and a step as 1 KiB.
+template <int NI>
+__global__ void __launch_bounds__(256)
+quantize_qint8_vnni2_kernel(const uint32_t* __restrict__ w, uint32_t N, uint32_t K, uint32_t bk, uint32_t bc,
+                            int8_t* __restrict__ q, float* __restrict__ scales) {
+  const uint32_t lane = threadIdx.x & 63, cg = lane & 3, s = lane >> 2;
+  const uint32_t nb = K / (64 * NI), blk = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blk >= (N / 16) * nb)
+    return;
+  const uint32_t n1 = blk / nb, b = blk - n1 * nb;
+  uint32_t raw[NI][2][4];
+#pragma unroll
+  for (int i = 0; i < NI; i++) {
+    const uint4* src = reinterpret_cast<const uint4*>(w + vnni2_dword(n1 * 16 + cg * 4, (b * NI + i) * 64 + s * 4, K, bk, bc));
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const uint4 v = src[j * (bk / 4)];
+      raw[i][j][0] = v.x; raw[i][j][1] = v.y; raw[i][j][2] = v.z; raw[i][j][3] = v.w;
+    }
+  }
+  float amax[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    amax[c] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        amax[c] = fmaxf(amax[c], fabsf(bf16_bits_to_f32(raw[i][j][c] & 0xffffu))); // (drops NaNs, as `a > amax ? a : amax`)
+        amax[c] = fmaxf(amax[c], fabsf(bf16_bits_to_f32(raw[i][j][c] >> 16)));
+      }
+#pragma unroll
+    for (int o = 4; o < 64; o <<= 1)
+      amax[c] = fmaxf(amax[c], __shfl_xor(amax[c], o, 64));
+  }
+  // every lane of a channel group holds the four maxima: lane s works out the scale of channel s & 3
+  const float mine = (s & 1) ? ((s & 2) ? amax[3] : amax[1]) : ((s & 2) ? amax[2] : amax[0]);
+  const float sc = int8_scale_of(mine), inv1 = int8_inv_scale(sc);
+  if (s < 4)
+    scales[(int64_t)blk * 16 + cg * 4 + s] = sc;
+  float inv[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+    inv[c] = __shfl(inv1, (int)(c * 4 + cg), 64);
+  uint4* out = reinterpret_cast<uint4*>(q + (int64_t)blk * (64 * NI) * 16) + lane;
+#pragma unroll
+  for (int i = 0; i < NI; i++) {
+    uint32_t o[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      o[c] = (uint32_t)(int8_q(bf16_bits_to_f32(raw[i][0][c] & 0xffffu), inv[c]) & 0xff) |
+             ((uint32_t)(int8_q(bf16_bits_to_f32(raw[i][0][c] >> 16), inv[c]) & 0xff) << 8) |
+             ((uint32_t)(int8_q(bf16_bits_to_f32(raw[i][1][c] & 0xffffu), inv[c]) & 0xff) << 16) |
+             ((uint32_t)(int8_q(bf16_bits_to_f32(raw[i][1][c] >> 16), inv[c]) & 0xff) << 24);
+    out[i * 64] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
 __constant__ float c_e2m1_tbl[16] = {0.0f,  0.5f,  1.0f,  1.5f, 2.0f,  3.0f,
                                      4.0f,  6.0f,  -0.0f, -0.5f, -1.0f, -1.5f,
                                      -2.0f, -3.0f, -4.0f, -6.0f};
 
-// one thread per packed byte; out is [N/32][K/64][32][32][2] fp32
+// one thread per four packed bytes (adjacent channels); out is [N/32][K/64][32][32][2] fp32.  Bound by the fp32 stores:
+// 11008 x 4096 in 32 us, 6.3 TB/s (51 us with a byte per thread and the values from a table in memory).
 __global__ void __launch_bounds__(256)
-dequantize_mxfp4_kernel(const uint8_t* __restrict__ qdata,
-                        const uint8_t* __restrict__ scales, int64_t nbytes,
+dequantize_mxfp4_kernel(const uint32_t* __restrict__ qdata, const uint8_t* __restrict__ scales, int64_t ndwords,
                         float* __restrict__ out) {
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nbytes)
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= ndwords)
     return;
-  int64_t k2 = t & 31, c2 = (t >> 5) & 31, tile = t >> 10;
-  uint32_t b = qdata[t];
-  float s = e8m0_to_f32(scales[(tile * 2 + (c2 >> 4)) * 32 + k2]);
-  float2 r;
-  r.x = c_e2m1_tbl[b & 0xf] * s;
-  r.y = c_e2m1_tbl[b >> 4] * s;
-  reinterpret_cast<float2*>(out)[t] = r;
+  const int64_t tile = t >> 8;
+  const uint32_t cg = (uint32_t)t & 7, c2 = ((uint32_t)t >> 3) & 31;
+  const uint32_t b = qdata[t];
+  const uint32_t sc = reinterpret_cast<const uint32_t*>(scales)[(tile * 2 + (c2 >> 4)) * 8 + cg];
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  f32x4 r[2];
+  // the E2M1 values from the hardware (exact, at scale 1), the scale as one fp32 product
+  const f32x2 v0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(b, 1.0f, 0), v1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(b, 1.0f, 1);
+  const f32x2 v2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(b, 1.0f, 2), v3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(b, 1.0f, 3);
+  r[0] = f32x4{v0[0] * e8m0_to_f32(sc), v0[1] * e8m0_to_f32(sc), v1[0] * e8m0_to_f32(sc >> 8), v1[1] * e8m0_to_f32(sc >> 8)};
+  r[1] = f32x4{v2[0] * e8m0_to_f32(sc >> 16), v2[1] * e8m0_to_f32(sc >> 16), v3[0] * e8m0_to_f32(sc >> 24), v3[1] * e8m0_to_f32(sc >> 24)};
+  f32x4* o = reinterpret_cast<f32x4*>(out) + t * 2;
+  o[0] = r[0];
+  o[1] = r[1];
 }
 
 // one thread per 4 int8; out [N/16][K/QBS][QBS/4][16][4] fp32
@@ -176,7 +333,8 @@ dequantize_qint8_kernel(const int8_t* __restrict__ q,
   if (t >= ngroups)
     return;
   int64_t k2 = t & 15;
-  int64_t blk = (t >> 4) / (qbs / 4); // (n1*nb + b)
+  // (n1*nb + b); the quotient in 32 bits where it fits (a 64-bit division costs more than the rest of the thread)
+  int64_t blk = (ngroups >> 36) == 0 ? (int64_t)((uint32_t)(t >> 4) / (uint32_t)(qbs / 4)) : (t >> 4) / (qbs / 4);
   float s = scales[blk * 16 + k2];
   uint32_t v = reinterpret_cast<const uint32_t*>(q)[t];
   float4 r;
@@ -236,6 +394,7 @@ prepack_qint8_kernel(const int8_t* __restrict__ qref, int64_t N, int64_t K,
 // bf16 weight in the reference's blocked layout [N/bk][K/bc][bc/v][bk][v] (v = 2: VNNI2 pairs; bk = 1, bc = K, v = 1:
 // a plain [N][K] matrix) -> native bf16 tiles [N/16][K/128][4 j][4 g][16 n][8]: the 16 bytes lane (g, n) feeds to
 // MFMA step j of K tile kt are W[nt*16 + n][kt*128 + (g*4 + j)*8 .. +7].
+template <int FAST>
 __global__ void __launch_bounds__(256)
 prepack_bf16_kernel(const uint16_t* __restrict__ wref, int64_t N, int64_t K, int64_t bk, int64_t bc, int64_t v,
                     uint16_t* __restrict__ wnat) {
@@ -244,8 +403,19 @@ prepack_bf16_kernel(const uint16_t* __restrict__ wref, int64_t N, int64_t K, int
   if (t >= nchunks)
     return;
   const int64_t n16 = t & 15, g = (t >> 4) & 3, j = (t >> 6) & 3, rest = t >> 8;
-  const int64_t KT = K / 128, kt = rest % KT, nt = rest / KT;
+  const int64_t KT = K / 128;
+  const int64_t nt = FAST ? (int64_t)((uint32_t)rest / (uint32_t)KT) : rest / KT, kt = rest - nt * KT;
   const int64_t n = nt * 16 + n16, k0 = kt * 128 + (g * 4 + j) * 8;
+  // the two layouts met in earnest by whole dwords: VNNI2 blocks (pairs of k, bk dwords apart) and a plain matrix
+  if (FAST == 2) {
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(wref) + vnni2_dword((uint32_t)n, (uint32_t)k0, (uint32_t)K, (uint32_t)bk, (uint32_t)bc);
+    reinterpret_cast<uint4*>(wnat)[t] = make_uint4(src[0], src[bk], src[2 * bk], src[3 * bk]);
+    return;
+  }
+  if (FAST == 1) {
+    reinterpret_cast<uint4*>(wnat)[t] = *reinterpret_cast<const uint4*>(wref + n * K + k0);
+    return;
+  }
   const int64_t n1 = n / bk, k2 = n % bk;
   uint16_t e[8];
 #pragma unroll
@@ -659,6 +829,65 @@ quantize_qint2_kernel(const T* __restrict__ w, int64_t N, int64_t K, int64_t bk,
   }
 }
 
+// The same for VNNI2 bf16 weights and blocks of 256: one wave per (32 channels, block), lane = (k2, K position s); a
+// lane holds the four channels k2 + 8 * k3 that share its output bytes, so nothing is assembled with atomics and the
+// output needs no zeroing.  2 |w| > s is rne(|w| / s) >= 1: the quotient of a bf16 value and a scale that is one (or
+// 1e-8) is never close enough to one half for its fp32 rounding to matter.
+__global__ void __launch_bounds__(256)
+quantize_qint2_vnni2_kernel(const uint32_t* __restrict__ w, uint32_t N, uint32_t K, uint32_t bk, uint32_t bc,
+                            uint32_t* __restrict__ q32, float* __restrict__ scales) {
+  const uint32_t lane = threadIdx.x & 63, k2 = lane & 7, s = lane >> 3;
+  const uint32_t nb = K / 256, blk = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blk >= (N / 32) * nb)
+    return;
+  const uint32_t n1 = blk / nb, b = blk - n1 * nb;
+  uint32_t raw[4][8][2]; // [k3][i][pair of the group of four]
+  float sc[4];
+#pragma unroll
+  for (int k3 = 0; k3 < 4; k3++) {
+    // a K block holds whole steps of 32 channels; two of them (64) at least
+    int64_t at = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      if ((i & 1) == 0)
+        at = vnni2_dword(n1 * 32 + k3 * 8 + k2, b * 256 + i * 32 + s * 4, K, bk, bc);
+      const uint32_t* src = w + at + (int64_t)(i & 1) * 16 * bk;
+      raw[k3][i][0] = src[0];
+      raw[k3][i][1] = src[bk];
+    }
+  }
+#pragma unroll
+  for (int k3 = 0; k3 < 4; k3++) {
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        amax = fmaxf(amax, fabsf(bf16_bits_to_f32(raw[k3][i][j] & 0xffffu)));
+        amax = fmaxf(amax, fabsf(bf16_bits_to_f32(raw[k3][i][j] >> 16)));
+      }
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1)
+      amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    sc[k3] = fmaxf(amax, 1.0e-8f);
+    if (s == 0)
+      scales[(int64_t)blk * 32 + k3 * 8 + k2] = sc[k3];
+  }
+  uint32_t* out = q32 + (int64_t)blk * 512 + s * 8 + k2; // [64 c2][8 k2]
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    uint32_t word = 0;
+#pragma unroll
+    for (int k3 = 0; k3 < 4; k3++)
+#pragma unroll
+      for (int c3 = 0; c3 < 4; c3++) {
+        const float v = bf16_bits_to_f32((raw[k3][i][c3 >> 1] >> (16 * (c3 & 1))) & 0xffffu) * 2.0f;
+        word |= (v > sc[k3] ? 1u : (v < -sc[k3] ? 2u : 0u)) << (2 * k3 + 8 * c3);
+      }
+    out[i * 64] = word;
+  }
+}
+
 // packed 2-bit (interleaved) -> native int8 tiles of the W8A8 kernels + scales [N/16][K/bs][16];
 // one thread per native 16-byte chunk (nt, kt, g, n16): input channels kt*64 + g*16 .. +15 of channel nt*16 + n16
 __global__ void __launch_bounds__(256)
@@ -687,18 +916,26 @@ prepack_qint2_kernel(const uint8_t* __restrict__ q2, const float* __restrict__ s
     snat[(nt * nb + b) * 16 + n16] = s2[(n1 * nb + b) * 32 + r];
 }
 
-// packed 2-bit (interleaved) -> fp32 in the logical blocked shape [N/32][K/bs][bs/4][32][4]; one thread per output
+// packed 2-bit (interleaved) -> fp32 in the logical blocked shape [N/32][K/bs][bs/4][32][4]; one thread per four
+// adjacent input channels of an output channel
 __global__ void __launch_bounds__(256)
-dequantize_qint2_kernel(const uint8_t* __restrict__ q2, const float* __restrict__ s2, int64_t total, int64_t bs,
+dequantize_qint2_kernel(const uint32_t* __restrict__ q2, const float* __restrict__ s2, int64_t total, int64_t bs,
                         float* __restrict__ out) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= total)
     return;
-  const int64_t c3 = t & 3, r = (t >> 2) & 31, rest = t >> 7; // rest = (n1*nb + b) * (bs/4) + c2
-  const int64_t blk = rest / (bs / 4);
-  const uint32_t byte = q2[(rest * 8 + (r & 7)) * 4 + c3];
-  const uint32_t code = (byte >> (2 * (r >> 3))) & 3u;
-  out[t] = (code == 1 ? 1.0f : (code == 2 ? -1.0f : 0.0f)) * s2[blk * 32 + r];
+  const int64_t rest = t >> 5; // (n1*nb + b) * (bs/4) + c2
+  const uint32_t r = (uint32_t)t & 31;
+  const int64_t blk = (total >> 37) == 0 ? (int64_t)((uint32_t)rest / (uint32_t)(bs / 4)) : rest / (bs / 4);
+  const uint32_t codes = q2[rest * 8 + (r & 7)] >> (2 * (r >> 3));
+  const float s = s2[blk * 32 + r];
+  f32x4 o;
+#pragma unroll
+  for (int c3 = 0; c3 < 4; c3++) {
+    const uint32_t code = (codes >> (8 * c3)) & 3u;
+    o[c3] = (code == 1 ? 1.0f : (code == 2 ? -1.0f : 0.0f)) * s;
+  }
+  reinterpret_cast<f32x4*>(out)[t] = o;
 }
 
 // INT4 weight in the VNNI2 layout [N/16][K/bs][bs/2][16][2 codes per byte] -> native int8 tiles
@@ -835,6 +1072,13 @@ hipError_t launch_quant_act_mxfp8(const void* x, int64_t M, int64_t K, void* xq,
 
 using namespace tppx;
 
+// do the VNNI2 kernels above take this weight: bf16 pairs, four adjacent channels in one block, K blocks of whole
+// 64-channel steps, indices in 32 bits
+static bool vnni2_fast(const void* w, int w_dtype, int64_t N, int64_t K, int64_t bk, int64_t bc, int64_t vnni) {
+  return w_dtype == TPPX_DT_BF16 && vnni == 2 && aligned16(w) && bk % 4 == 0 && bc % 64 == 0 && K % 64 == 0 &&
+         N * K < ((int64_t)1 << 36) && N < ((int64_t)1 << 31) && K < ((int64_t)1 << 31);
+}
+
 extern "C" int tppx_quantize_mxfp4(const void* w, int w_dtype, int64_t N,
                                    int64_t K, int64_t bk, int64_t bc,
                                    int64_t vnni, void* qdata, void* scales,
@@ -850,7 +1094,10 @@ extern "C" int tppx_quantize_mxfp4(const void* w, int w_dtype, int64_t N,
                (long)bk, (long)bc, (long)vnni, (long)N, (long)K);
   int64_t nblk = N * (K / 32);
   hipStream_t s = (hipStream_t)stream;
-  if (w_dtype == TPPX_DT_F32)
+  if (vnni2_fast(w, w_dtype, N, K, bk, bc, vnni) && (((uintptr_t)qdata | (uintptr_t)scales) & 3) == 0)
+    quantize_mxfp4_vnni2_kernel<<<grid_for(N / 32 * (K / 64), 16), 256, 0, s>>>(
+        (const uint32_t*)w, (uint32_t)N, (uint32_t)K, (uint32_t)bk, (uint32_t)bc, (uint8_t*)qdata, (uint8_t*)scales);
+  else if (w_dtype == TPPX_DT_F32)
     quantize_mxfp4_kernel<float><<<grid_for(nblk, 256), 256, 0, s>>>(
         (const float*)w, N, K, bk, bc, vnni, (uint8_t*)qdata, (uint8_t*)scales);
   else
@@ -875,7 +1122,17 @@ extern "C" int tppx_quantize_qint8(const void* w, int w_dtype, int64_t N,
                (long)bk, (long)bc, (long)vnni, (long)N, (long)K);
   int64_t nthreads = N * (K / qbs) * 64;
   hipStream_t s = (hipStream_t)stream;
-  if (w_dtype == TPPX_DT_F32)
+  if (vnni2_fast(w, w_dtype, N, K, bk, bc, vnni) && aligned16(q) && (qbs == 64 || qbs == 128 || qbs == 256 || qbs == 512)) {
+    const unsigned grid = grid_for(N / 16 * (K / qbs), 4);
+#define TPPX_Q8V(NI)                                                                                                   \
+  quantize_qint8_vnni2_kernel<NI><<<grid, 256, 0, s>>>((const uint32_t*)w, (uint32_t)N, (uint32_t)K, (uint32_t)bk,     \
+                                                       (uint32_t)bc, (int8_t*)q, (float*)scales)
+    if (qbs == 64) TPPX_Q8V(1);
+    else if (qbs == 128) TPPX_Q8V(2);
+    else if (qbs == 256) TPPX_Q8V(4);
+    else TPPX_Q8V(8);
+#undef TPPX_Q8V
+  } else if (w_dtype == TPPX_DT_F32)
     quantize_qint8_kernel<float><<<grid_for(nthreads, 256), 256, 0, s>>>(
         (const float*)w, N, K, bk, bc, vnni, qbs, (int8_t*)q, (float*)scales);
   else
@@ -890,9 +1147,11 @@ extern "C" int tppx_dequantize_mxfp4(const void* qdata, const void* scales,
   TPPX_REQUIRE(qdata && scales && out_f32, TPPX_EINVAL, "tppx_dequantize_mxfp4: null pointer");
   TPPX_REQUIRE(N > 0 && K > 0 && N % 32 == 0 && K % 64 == 0, TPPX_ESHAPE,
                "tppx_dequantize_mxfp4: N=%ld must be a multiple of 32 and K=%ld of 64", (long)N, (long)K);
-  int64_t nbytes = N * K / 2;
-  dequantize_mxfp4_kernel<<<grid_for(nbytes, 256), 256, 0, (hipStream_t)stream>>>(
-      (const uint8_t*)qdata, (const uint8_t*)scales, nbytes, (float*)out_f32);
+  TPPX_REQUIRE((((uintptr_t)qdata | (uintptr_t)scales) & 3) == 0 && aligned16(out_f32), TPPX_EINVAL,
+               "tppx_dequantize_mxfp4: codes and scales must be 4-byte, the output 16-byte aligned");
+  int64_t ndwords = N * K / 8;
+  dequantize_mxfp4_kernel<<<grid_for(ndwords, 256), 256, 0, (hipStream_t)stream>>>(
+      (const uint32_t*)qdata, (const uint8_t*)scales, ndwords, (float*)out_f32);
   return check_hip(hipGetLastError(), "tppx_dequantize_mxfp4");
 }
 
@@ -974,8 +1233,15 @@ extern "C" int tppx_prepack_bf16(const void* w_ref, int64_t N, int64_t K, int64_
                "tppx_prepack_bf16: blocking bk=%ld bc=%ld vnni=%d does not divide N=%ld K=%ld", (long)bk, (long)bc, vnni,
                (long)N, (long)K);
   const int64_t nchunks = N * (K / 8);
-  prepack_bf16_kernel<<<grid_for(nchunks, 256), 256, 0, (hipStream_t)stream>>>((const uint16_t*)w_ref, N, K, bk, bc, vnni,
-                                                                                (uint16_t*)w_nat);
+  const unsigned grid = grid_for(nchunks, 256);
+  const bool small = N < ((int64_t)1 << 31) && K < ((int64_t)1 << 31) && nchunks < ((int64_t)1 << 38);
+  hipStream_t s = (hipStream_t)stream;
+  if (small && vnni == 2 && bc % 8 == 0 && ((uintptr_t)w_ref & 3) == 0)
+    prepack_bf16_kernel<2><<<grid, 256, 0, s>>>((const uint16_t*)w_ref, N, K, bk, bc, vnni, (uint16_t*)w_nat);
+  else if (small && vnni == 1 && bk == 1 && bc == K && aligned16(w_ref))
+    prepack_bf16_kernel<1><<<grid, 256, 0, s>>>((const uint16_t*)w_ref, N, K, bk, bc, vnni, (uint16_t*)w_nat);
+  else
+    prepack_bf16_kernel<0><<<grid, 256, 0, s>>>((const uint16_t*)w_ref, N, K, bk, bc, vnni, (uint16_t*)w_nat);
   return check_hip(hipGetLastError(), "tppx_prepack_bf16");
 }
 
@@ -1063,6 +1329,11 @@ extern "C" int tppx_quantize_qint2_intlv(const void* w, int w_dtype, int64_t N, 
   TPPX_REQUIRE(bk > 0 && bc > 0 && vnni > 0 && N % bk == 0 && K % bc == 0 && bc % vnni == 0, TPPX_ESHAPE,
                "%s: blocking (bk=%ld, bc=%ld, vnni=%ld) does not divide [%ld,%ld]", who, (long)bk, (long)bc, (long)vnni, (long)N, (long)K);
   hipStream_t s = (hipStream_t)stream;
+  if (vnni2_fast(w, w_dtype, N, K, bk, bc, vnni) && bs == 256) {
+    quantize_qint2_vnni2_kernel<<<grid_for(N / 32 * (K / 256), 4), 256, 0, s>>>(
+        (const uint32_t*)w, (uint32_t)N, (uint32_t)K, (uint32_t)bk, (uint32_t)bc, (uint32_t*)q, (float*)scales);
+    return check_hip(hipGetLastError(), who);
+  }
   // the bytes are assembled with ORs: start from zeros (a fill kernel, so that the call can sit in a captured graph)
   const int64_t nwords = N * K / 16;
   fill_zero_kernel<<<grid_for(nwords, 256), 256, 0, s>>>((uint32_t*)q, nwords);
@@ -1080,7 +1351,8 @@ extern "C" int tppx_dequantize_qint2_intlv(const void* q, const void* scales, in
   TPPX_REQUIRE(q && scales && out_f32, TPPX_EINVAL, "%s: null pointer", who);
   if (int rc = check_qint2(who, N, K, bs))
     return rc;
-  dequantize_qint2_kernel<<<grid_for(N * K, 256), 256, 0, (hipStream_t)stream>>>((const uint8_t*)q, (const float*)scales, N * K, bs, (float*)out_f32);
+  TPPX_REQUIRE((reinterpret_cast<uintptr_t>(q) & 3u) == 0 && aligned16(out_f32), TPPX_EINVAL, "%s: codes must be 4-byte, the output 16-byte aligned", who);
+  dequantize_qint2_kernel<<<grid_for(N * K / 4, 256), 256, 0, (hipStream_t)stream>>>((const uint32_t*)q, (const float*)scales, N * K / 4, bs, (float*)out_f32);
   return check_hip(hipGetLastError(), who);
 }
 

@@ -893,3 +893,30 @@ def test_qkv_one_gemm_over_concatenated_weights(M, widths, monkeypatch):
     one_s = ops.qkv_gemm(x, ws, bs, norm=(gamma, 1e-5, table))
     for a, b in zip(one_s, seg_s):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("tile", [4, 5])
+@pytest.mark.parametrize("M,N,K", [(65, 160, 128), (129, 544, 256), (300, 544, 384), (200, 1056, 640), (70, 2080, 2048)])
+def test_prefill_mxfp4_ring_tiles(tile, M, N, K, monkeypatch):
+    """The 64 x 128 and 128 x 128 workgroup tiles (operands in a ring of three LDS stages), forced: fewer K steps than
+    stages, as many and more, ragged rows and channel blocks.  Same sums in the same order as the 256 x 256 tile: the
+    same bits, for a single GEMM, fused q/k/v and the gate/up pair; the single GEMM against the oracle."""
+    ops = _ops()
+    w, q_or, s_or = _make("mxfp4", N, K, 740)[:3]
+    ws = [_make("mxfp4", n, K, 741 + i)[0] for i, n in enumerate((N, 64, 96))]
+    wu = _make("mxfp4", N, K, 745)[0]
+    x = randn_bf16((M, K), 1.0, 746)
+    xg = x.cuda()
+
+    def run():
+        return [ops.fc_plain(xg, w, None)] + list(ops.qkv_gemm(xg, ws, [None] * 3)) + [ops.swiglu_gate_up(xg, w, wu)]
+
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
+    monkeypatch.setenv("TPPX_TILED_BIG_TILE", "1")
+    want = run()
+    monkeypatch.setenv("TPPX_TILED_BIG_TILE", str(tile))
+    got = run()
+    ref = O.linear_mxfp4(t2bits(x), q_or, s_or, None, O.POST_NONE, None, None, 1.0, O.MODE_IDEAL)
+    assert_close_bf16(t2bits(got[0]), ref, ulps=1, what=f"tile {tile}")
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), i

@@ -218,13 +218,12 @@ static const int64_t TILED_MIN_M = 65; // more rows than the decode kernels cove
 // More than 64 rows: the LDS-tiled kernels give every workgroup a whole output tile and all of K, so a launch with
 // few tiles leaves most of the 256 CUs idle (7B shapes at 256 rows: 43 workgroups), while the decode kernels run one
 // block row of 64 rows after the other over the full grid, streaming the weights once per block row.  Pick by a
-// cost estimates fitted to measurements on MI355X (us).  MXFP4: a block row of 64 costs about 8 + weight bytes /
-// 5.5 TB/s + 0.8 ns per input channel (its activations), a round of 256 x 256 tiles about 14.5 ns per input channel
-// (128 x 128: 20; launches small enough for 64 x 128 workgroups: 10 us + 6 ns per input channel).  QINT8 (128 x 256
+// cost estimates fitted to measurements on MI355X (us).  MXFP4: a block row of 64 costs about 4.7 (pair: 9.5) + weight bytes /
+// 5.5 TB/s + 0.4 ns per input channel (its activations), the tiled launches what tiled_mxfp4_us() says.  QINT8 (128 x 256
 // tiles, one workgroup per CU) and unquantized bf16 weights (128 x 256 tiles, two workgroups per CU): their own fits
 // below.  `wbytes` = weight bytes of
 // the whole call, `n_tiles16` = its 16-channel tiles.  TPPX_TILED_MIN_M (when set) restores a plain row threshold.
-enum { COST_MXFP4 = 0, COST_QINT8 = 1, COST_BF16 = 2 };
+enum { COST_MXFP4 = 0, COST_QINT8 = 1, COST_BF16 = 2, COST_MXFP4_PAIR = 3 };
 static bool want_tiled(int64_t M, int flags, int64_t K = 0, int64_t n_tiles16 = 0, double wbytes = 0.0,
                        int kind = COST_MXFP4) {
   if (flags & TPPX_FLAG_FORCE_SKINNY)
@@ -255,22 +254,13 @@ static bool want_tiled(int64_t M, int flags, int64_t K = 0, int64_t n_tiles16 = 
     const double skinny_us = rows64 * (6.5 + wbytes / 5.5e6 + (double)K * 0.0006);
     return tiled_us <= skinny_us;
   }
-  const bool big = kind == COST_MXFP4 && M >= big_min_rows();
-  if (big && env_int("TPPX_TILED_SMALL", 1) != 0) {
-    // launches of at most 128 workgroups of 128 x 256 run as four times as many of 64 x 128
-    const int64_t wgs1 = ((M + 127) / 128) * ((n_tiles16 + 15) / 16);
-    if (wgs1 <= 128) {
-      const int64_t wgs2 = ((M + 63) / 64) * ((n_tiles16 + 7) / 8);
-      // (up to 128 of them: 26 us at K = 4096, 74 at K = 11008 whatever the rows)
-      const double tiled_us = wgs2 <= 128 ? std::max(12.0, (double)K * 0.007 - 2.0)
-                                          : 10.0 + (double)K * 0.006 * (wgs2 <= 384 ? 1.05 : 1.25);
-      const double skinny_us = rows64 * (6.0 + wbytes / 5.5e6 + (double)K * 0.0007);
-      return tiled_us <= skinny_us;
-    }
-  }
-  const int64_t rows = big ? 256 : 128, cols16 = big ? 16 : 8;
-  const int64_t wgs = ((M + rows - 1) / rows) * ((n_tiles16 + cols16 - 1) / cols16);
-  const double tiled_us = (double)((wgs + 255) / 256) * (double)K * 0.0145 * (big ? 1.0 : 1.4);
+  const bool big = (kind == COST_MXFP4 || kind == COST_MXFP4_PAIR) && M >= big_min_rows();
+  if (big) // (a block row of the decode kernels: 9.6 us at 4096 x 4096, 16 at 4096 x 11008, 11-13 at 2560 x 10240, 13 at
+           // 12288 x 4096; 33 at 3584 x 18944, beyond the kernels that split K; the pair 21 at 2 x 11008 x 4096)
+    return tiled_mxfp4_us(M, K, n_tiles16) <=
+           rows64 * ((kind == COST_MXFP4_PAIR ? 9.5 : 4.7) + wbytes / 5.5e6 + (double)K * (K > 16384 ? 0.0014 : 0.0004));
+  const int64_t wgs = ((M + 127) / 128) * ((n_tiles16 + 7) / 8);
+  const double tiled_us = (double)((wgs + 255) / 256) * (double)K * 0.0203;
   const double skinny_us = rows64 * (8.0 + wbytes / 5.5e6 + (double)K * 0.0008);
   return tiled_us <= skinny_us;
 }
@@ -369,7 +359,8 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
     return check_hip(launch_tiled_mxfp4_fp8_group(&t[1], 1, stream), who);
   }
   if (want_tiled(M, flags, K, dual ? 2 * p.total_tiles : p.total_tiles,
-                 (dual ? 2.0 : 1.0) * (double)p.total_tiles * 16.0 * (double)K * (0.5 + 1.0 / 32))) {
+                 (dual ? 2.0 : 1.0) * (double)p.total_tiles * 16.0 * (double)K * (0.5 + 1.0 / 32),
+                 dual ? COST_MXFP4_PAIR : COST_MXFP4)) {
     TPPX_REQUIRE(!row_sumsq, TPPX_EUNSUPPORTED, "%s: row sums of squares are not produced by the large-M kernels", who);
     // prefill shapes: one LDS-tiled launch per GEMM of the group; the fused
     // gate/up pair becomes silu(gate) followed by up * gate (same rounding)

@@ -103,6 +103,8 @@ struct TiledParams {
 };
 
 hipError_t launch_tiled_mxfp4(const TiledParams& p, hipStream_t stream);
+// what the large-M launches take for n_tiles16 tiles of 16 output channels, in us (estimate)
+double tiled_mxfp4_us(int64_t M, int64_t K, int64_t n_tiles16);
 // large-M kernel: several GEMMs over one activation in one launch
 bool tiled_mxfp4_takes_groups(const TiledParams& p);
 // dual: the gate/up pair (t[0] = gate, t[1] = up) with silu(gate) * up formed in the launch and written to t[1].y

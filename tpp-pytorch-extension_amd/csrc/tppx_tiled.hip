@@ -795,16 +795,208 @@ __device__ __forceinline__ void big_gemm_body(const BigParams& P) {
     big_epilogue<MT>(p, acc, reinterpret_cast<float*>(tl_lds) + wave * 64 * EP_LD, m_wg + wm * (MT * 16), tile_base);
 }
 
-template <int MT, bool DUAL, int WM, int WN>
-__global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
-big_mxfp4_kernel(const BigParams P) {
-  big_gemm_body<MT, DUAL, WM, WN, false>(P);
-}
-
 template <int MT, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
 big_bf16_kernel(const BigParams P) {
   big_gemm_body<MT, false, WM, WN, true>(P);
+}
+
+// ---------------------------------------------------------------------------
+// MXFP4 launches whose workgroups are at most one or two to a CU: the same tiles, operand layout and order of sums as
+// big_gemm_body (the same bits), but BOTH operands and the scale bytes go from global memory straight into LDS, NB - 1
+// K steps ahead in a ring of NB stages.  With one workgroup per CU nothing else covers the latency of a step's loads:
+// requested one step ahead (weights half a step, into registers) a step of a 64 x 128 workgroup took 0.8 us where its
+// MFMAs take 0.25 and its bytes 0.45; now 0.5 (4096 x 11008 at 333 rows 74 -> 52 us, 3584 x 18944 122 -> 82).  Six
+// stages measured as three.  All loads of the loop being of one kind they complete in issue order, so the
+// wait at the top of a step leaves the younger stages in flight; one barrier per step.
+// Stage: A [WM*MT row tiles][4096 B], swizzled as in big_gemm_body | B [4*WN native tiles][1 KiB] | scales [4*WN][64 B].
+// ---------------------------------------------------------------------------
+template <int MT, int WM, int WN, int NB>
+struct RingGeom {
+  static constexpr int A_BYTES = WM * MT * 4096;
+  static constexpr int B_OFF = A_BYTES;
+  static constexpr int S_OFF = B_OFF + WN * 4096;
+  static constexpr int STAGE = S_OFF + WN * 256;
+  static constexpr int NBLK = MT * 4 / WN; // blocks of 4 rows x 256 B a wave fetches per step
+  static constexpr int NBT = 4 / WM;       // weight tiles a wave fetches per step
+  static constexpr int LPS = NBLK + NBT + 1;
+  static constexpr size_t EP = (size_t)WM * WN * (MT < 4 ? MT * 16 : 64) * EP_LD * sizeof(float); // epilogue staging
+  static constexpr size_t LDS = (size_t)NB * STAGE > EP ? (size_t)NB * STAGE : EP;
+  static_assert(NBLK % 4 == 0, "the swizzle takes a wave's first block to be a multiple of 4");
+};
+
+template <int MT, bool DUAL, int WM, int WN, int NB>
+__device__ __forceinline__ void ring_gemm_body(const BigParams& P) {
+  using G = RingGeom<MT, WM, WN, NB>;
+  constexpr int WGM = MT * 16 * WM, NBLK = G::NBLK, NBT = G::NBT, LPS = G::LPS, STAGE = G::STAGE;
+  extern __shared__ __align__(16) uint8_t tl_lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wn = wave / WM;
+  const int MB = (P.seg[0].M + WGM - 1) / WGM;
+  int bm, bn;
+  tile_of_block(MB, P.nb0[P.n_seg], bm, bn, P.xm);
+  TiledParams p = P.seg[0];
+  int nb_first = 0;
+  if (!DUAL) {
+#pragma unroll
+    for (int i = 1; i < TPPX_MAX_SEGS; i++)
+      if (i < P.n_seg && bn >= P.nb0[i]) {
+        p = P.seg[i];
+        nb_first = P.nb0[i];
+      }
+  }
+  bn -= nb_first;
+  const int KT = p.K >> 7;
+  const int m_wg = bm * WGM;
+  const int tile_base = DUAL ? bn * (WN * 2) + wn * 2 : bn * (WN * 4) + wn * 4;
+  // weight tile behind slot t (0 .. 4*WN-1) of a stage; DUAL: slots 2, 3 of a wave column are the up projection's
+  auto slot_tile = [&](int t) { return min(DUAL ? bn * (WN * 2) + (t >> 2) * 2 + (t & 1) : bn * (WN * 4) + t, p.tiles - 1); };
+
+  // this wave's share of a stage: uniform bases that move with the step + 32-bit offsets per lane (operands < 4 GiB)
+  const char* xbase = reinterpret_cast<const char*>(p.x);
+  uint32_t aoff[NBLK];
+#pragma unroll
+  for (int i = 0; i < NBLK; i++) {
+    const int rin = lane >> 4, ch = lane & 15;
+    const int row = min(m_wg + (wave * NBLK + i) * 4 + rin, p.M - 1); // past the end: re-read the last row (never stored)
+    aoff[i] = (uint32_t)row * (uint32_t)p.K * 2u + (uint32_t)((ch ^ ((i & 3) * 4 + rin)) & 15) * 16u;
+  }
+  const char* bbase[NBT];
+  uint32_t boff[NBT];
+#pragma unroll
+  for (int i = 0; i < NBT; i++) {
+    const int t = wave * NBT + i;
+    bbase[i] = reinterpret_cast<const char*>(DUAL && (t & 2) ? P.seg[1].qw : p.qw);
+    boff[i] = ((uint32_t)slot_tile(t) * (uint32_t)KT * 64u + (uint32_t)lane) * 16u;
+  }
+  const int sp = wave % WN; // scales of slots 4*sp .. 4*sp+3; the waves of a row fetch the same ones, so that every
+                            // wave issues LPS loads per stage
+  const int st = sp * 4 + (lane >> 4);
+  const char* ssrc = reinterpret_cast<const char*>(DUAL && (st & 2) ? P.seg[1].sw : p.sw) +
+                     (size_t)slot_tile(st) * KT * 64 + (size_t)(lane & 15) * 4;
+  auto dma_one = [&](auto I, int ks, int buf) {
+    constexpr int i = decltype(I)::value;
+    uint8_t* base = tl_lds + buf * STAGE;
+    if constexpr (i < NBLK)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xbase + (size_t)ks * 256 + (size_t)aoff[i]),
+                                       (__attribute__((address_space(3))) void*)(base + (wave * NBLK + i) * 1024), 16, 0, 0);
+    else if constexpr (i < NBLK + NBT)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(bbase[i - NBLK] + (size_t)ks * 1024 + (size_t)boff[i - NBLK]),
+                                       (__attribute__((address_space(3))) void*)(base + G::B_OFF + (wave * NBT + i - NBLK) * 1024), 16, 0, 0);
+    else
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(ssrc + (size_t)ks * 64),
+                                       (__attribute__((address_space(3))) void*)(base + G::S_OFF + sp * 256), 4, 0, 0);
+  };
+
+  uint32_t rdb[4]; // byte offset of this lane's activation operand of step j in a row tile
+  {
+    const int m = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      rdb[j] = (uint32_t)((m >> 2) * 1024 + (m & 3) * 256 + (((g * 4 + j) ^ m) & 15) * 16);
+  }
+  f32x4 acc[MT][4];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int nt = 0; nt < 4; nt++)
+      acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int s = 0; s < NB - 1; s++)
+    if (s < KT)
+      static_for<0, LPS>([&](auto I) { dma_one(I, s, s); });
+  // Operands of two MFMA steps j: those of (ks, j) are read and expanded under the MFMAs of the step before, so the
+  // MFMAs of (ks, 3) are issued in the next K step, under its first operand reads.  (The set of (-1, 3) is zeros.)
+  bf16x8 a[2][MT], b[2][4];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+    a[1][mt] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int nt = 0; nt < 4; nt++)
+    b[1][nt] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  auto mfmas = [&](int set) {
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int nt = 0; nt < 4; nt++)
+        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[set][mt], b[set][nt], acc[mt][nt], 0, 0, 0);
+  };
+  int buf = 0;
+  auto step = [&](auto MORE, int ks) {
+    constexpr bool more = decltype(MORE)::value;
+    // stage ks has landed for this wave (in the main loop the NB - 2 younger ones may still be in flight; the last
+    // NB - 1 steps wait for all that is left) and its reads of stage ks - 1 have returned ...
+    // (the builtin, so that the compiler knows the operands of (ks - 1, 3) to be there)
+    constexpr int vm = more ? LPS * (NB - 2) : 0;
+    asm volatile("" : : : "memory");
+    __builtin_amdgcn_s_waitcnt((vm & 15) | 7 << 4 | vm >> 4 << 14); // vmcnt(vm) lgkmcnt(0), expcnt open
+    // ... and for every wave: the stage of step ks - 1 is free for the next loads
+    asm volatile("s_barrier" : : : "memory");
+    const int nbuf = buf == 0 ? NB - 1 : buf - 1;
+    const uint8_t* base = tl_lds + buf * STAGE;
+    const uint8_t* ab = base + wm * MT * 4096;
+    i32x4 bw[4];
+    uint32_t sc[4];
+#pragma unroll
+    for (int nt = 0; nt < 4; nt++) {
+      bw[nt] = *reinterpret_cast<const i32x4*>(base + G::B_OFF + (wn * 4 + nt) * 1024 + lane * 16);
+      sc[nt] = base[G::S_OFF + (wn * 4 + nt) * 64 + lane];
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+      a[0][mt] = *reinterpret_cast<const bf16x8*>(ab + mt * 4096 + rdb[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    mfmas(1);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, 4>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      // the next stage's loads a few at a time (issued in one burst, a wave stands at its load instructions while the
+      // memory pipeline's queue drains)
+      if constexpr (more)
+        static_for<j * LPS / 4, (j + 1) * LPS / 4>([&](auto I) { dma_one(I, ks + NB - 1, nbuf); });
+      if constexpr (j > 0) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+          a[j & 1][mt] = *reinterpret_cast<const bf16x8*>(ab + mt * 4096 + rdb[j]);
+        __builtin_amdgcn_sched_barrier(0);
+        mfmas((j - 1) & 1);
+      }
+#pragma unroll
+      for (int nt = 0; nt < 4; nt++)
+        b[j & 1][nt] = tl_cvt_fp4x8((uint32_t)bw[nt][j], e8m0_to_f32(sc[nt]));
+      if constexpr (j > 0)
+        static_for<0, MT * 4>([&](auto) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);          // an MFMA
+          __builtin_amdgcn_sched_group_barrier(0x002, 16 / (MT * 4) > 0 ? 16 / (MT * 4) : 1, 0); // its share of the 16 expansions
+        });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    buf = buf == NB - 1 ? 0 : buf + 1;
+  };
+  int ks = 0;
+  for (; ks + NB - 1 < KT; ks++)
+    step(std::true_type{}, ks);
+  for (; ks < KT; ks++)
+    step(std::false_type{}, ks);
+  mfmas(1);
+  __syncthreads(); // the ring is free for the epilogue staging
+  float* stage = reinterpret_cast<float*>(tl_lds) + wave * (MT < 4 ? MT * 16 : 64) * EP_LD;
+  if (DUAL)
+    big_epilogue_dual<MT>(p, P.seg[1], acc, stage, m_wg + wm * (MT * 16), tile_base);
+  else
+    big_epilogue<MT>(p, acc, stage, m_wg + wm * (MT * 16), tile_base);
+}
+
+constexpr int RING_STAGES = 3; // (two 64 x 128 workgroups of three stages share a CU's LDS)
+template <int MT, bool DUAL, int WM, int WN>
+__global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
+big_mxfp4_kernel(const BigParams P) {
+  if constexpr (MT <= 4)
+    ring_gemm_body<MT, DUAL, WM, WN, RING_STAGES>(P);
+  else
+    big_gemm_body<MT, DUAL, WM, WN, false>(P);
 }
 
 // ---------------------------------------------------------------------------
@@ -1239,8 +1431,40 @@ big_fp8_kernel(const BigParams P) {
     big_epilogue<MT>(p, acc, reinterpret_cast<float*>(tl_lds) + wave * 64 * EP_LD, m_wg + wm * (MT * 16), tile_base);
 }
 
-// cost of a full round of 128 x 512 workgroups relative to one of 256 x 256 (measured)
-constexpr double BIG_WIDE_COST = 0.97;
+// Workgroup tiles of the MXFP4 launches and what a launch of `wgs` of them takes, in us, K steps of 128: a fixed part
+// (launch, first loads, epilogue) and a part per step, fitted to linears and SwiGLU pairs of K = 2560 .. 18944 and
+// 70 .. 2048 rows (one launch at K = 4096 / 18944: 64 x 128 23.5 / 79 us, 128 x 128 35 / 122, 128 x 256 48 / 178,
+// 128 x 512 80 / 301, 256 x 256 82 / 304, whatever part of the 256 CUs it fills).
+//   256 x 256, 128 x 512  eight waves, one workgroup per CU; for launches that fill the chip several times over
+//   128 x 256             up to 256 of them the ring kernel (one per CU), beyond that four waves and two per CU
+//   128 x 128             ring kernel, one per CU
+//   64 x 128              ring kernel, two per CU
+enum { TILE_256_256 = 0, TILE_128_256, TILE_128_512, TILE_64_128, TILE_128_128, N_TILES };
+static constexpr int TILE_ROWS[N_TILES] = {256, 128, 128, 64, 128};
+static constexpr int TILE_COLS16[N_TILES] = {16, 16, 32, 8, 8}; // 16-channel weight tiles (the pair: gate + up)
+static double tile_us(int tile, int64_t wgs, double steps) {
+  const double rounds = (double)((wgs + 255) / 256);
+  switch (tile) {
+  case TILE_256_256:
+    return (20.0 + 1.92 * steps) * rounds;
+  case TILE_128_512:
+    return (19.0 + 1.90 * steps) * rounds;
+  case TILE_128_256:
+    return wgs <= 256 ? 12.0 + 1.13 * steps : (20.0 + 2.05 * steps) * std::max(1.0, (double)wgs / 512.0);
+  case TILE_64_128:
+    return wgs <= 256 ? 7.5 + 0.50 * steps : wgs <= 512 ? 9.0 + 0.85 * steps : (9.0 + 0.97 * steps) * (double)wgs / 512.0;
+  default:
+    return (13.0 + 0.75 * steps) * rounds;
+  }
+}
+
+double tiled_mxfp4_us(int64_t M, int64_t K, int64_t n_tiles16) {
+  double best = 1e300;
+  for (int i = 0; i < N_TILES; i++)
+    best = std::min(best, tile_us(i, (M + TILE_ROWS[i] - 1) / TILE_ROWS[i] * ((n_tiles16 + TILE_COLS16[i] - 1) / TILE_COLS16[i]),
+                                  (double)(K / 128)));
+  return best;
+}
 
 static bool big_fits(const TiledParams& p) {
   return (int64_t)p.M * p.K * 2 < ((int64_t)1 << 32) && (int64_t)p.tiles * 8 * p.K < ((int64_t)1 << 32);
@@ -1252,9 +1476,10 @@ bool tiled_mxfp4_takes_groups(const TiledParams& p) {
 
 template <int MT, bool DUAL, int WM, int WN>
 static hipError_t big_launch(const BigParams& P, int wgs, hipStream_t stream) {
-  // epilogue staging per wave; >= the two A buffers
-  const size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float);
-  static_assert((size_t)WM * WN * 64 * EP_LD * sizeof(float) >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
+  size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float); // epilogue staging per wave; >= the two A buffers
+  if constexpr (MT <= 4)
+    lds = RingGeom<MT, WM, WN, RING_STAGES>::LDS;
+  static_assert(MT <= 4 || (size_t)WM * WN * 64 * EP_LD * sizeof(float) >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
   TPPX_PLAN_ONLY((big_mxfp4_kernel<MT, DUAL, WM, WN>), dim3(wgs), dim3(WM * WN * 64), lds);
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(big_mxfp4_kernel<MT, DUAL, WM, WN>), lds); e != hipSuccess)
     return e;
@@ -1277,35 +1502,24 @@ static hipError_t big_bf16_launch(const BigParams& P, int wgs, hipStream_t strea
 hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
-  // channel blocks of the launch when a workgroup owns `tpw` channel tiles (of each projection for the pair)
-  auto blocks = [&](int tpw) {
+  // the workgroup tile with the lowest estimate (see tile_us)
+  auto workgroups = [&](int tile) {
+    const int tpw = TILE_COLS16[tile] / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
     int nb = 0;
     for (int i = 0; i < (dual ? 1 : n); i++)
       nb += (t[i].tiles + tpw - 1) / tpw;
-    return nb;
+    return (int64_t)((t[0].M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile]) * nb;
   };
-  const int nb4 = blocks(dual ? 8 : 16), nb8 = blocks(dual ? 16 : 32); // 4 or 8 wave columns
-  const int MB8 = (t[0].M + 255) / 256, MB4 = (t[0].M + 127) / 128;
-  // Workgroup tile.  256 x 256 (8 waves, one per CU) or 128 x 512 (8 waves, one per CU) when their rounds of 256
-  // workgroups are full; 128 x 256 (4 waves, two per CU, 512 at a time) costs a few percent more per round but its
-  // workgroups are half the size, so a last partial round costs less (q/k/v with 10240 channels at M = 2048: 320
-  // workgroups of 256 x 256 are 2 rounds, 640 of 128 x 256 are 1.25).  Costs in units of one full round of 256 x 256.
-  auto rounds = [](int wgs) { return (double)((wgs + 255) / 256); };
-  const int w4 = MB4 * nb4;
-  const double cost[3] = {rounds(MB8 * nb4), w4 <= 256 ? 0.6 : 1.05 * (w4 <= 512 ? 1.0 : w4 / 512.0),
-                          BIG_WIDE_COST * rounds(MB4 * nb8)};
-  int shape = 0;
-  for (int i = 1; i < 3; i++)
-    if (cost[i] < cost[shape])
-      shape = i;
-  const int env_shape = env_int("TPPX_TILED_BIG_TILE", 0); // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512
-  if (env_shape >= 1 && env_shape <= 3)
-    shape = env_shape - 1;
-  // Launches that would leave half the CUs empty with 128 x 256 workgroups: 64 x 128 workgroups of four waves (32 x 64
-  // each) instead, four times as many (the same sums in the same order: the same bits; 4096 x 4096 at 256 rows
-  // 50 -> 28 us, 4096 x 11008 at 512 rows 124 -> 79 us; beyond 128 such workgroups the small ones lose)
-  const bool small = shape == 1 && MB4 * nb4 <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0 && env_shape == 0;
-  const int tpw = small ? (dual ? 4 : 8) : (shape == 2 ? 8 : 4) * (dual ? 2 : 4);
+  int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
+  if (shape < 0 || shape >= N_TILES) {
+    double best = 1e300;
+    for (int i = 0; i < (env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128); i++)
+      if (const double us = tile_us(i, workgroups(i), (double)(t[0].K / 128)); us < best) {
+        best = us;
+        shape = i;
+      }
+  }
+  const int tpw = TILE_COLS16[shape] / (dual ? 2 : 1), MB = (t[0].M + TILE_ROWS[shape] - 1) / TILE_ROWS[shape];
   BigParams P;
   memset(&P, 0, sizeof(P));
   int nb = 0;
@@ -1324,12 +1538,11 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
   {
     // XCD rectangles: the split that moves the fewest bytes from memory into the L2s (activations: rows x K bf16 per
     // row block, fetched by 8 / xm XCDs... every XCD fetches 1/xm of them; weights 0.53 B per element, xm/8 each)
-    const int MBs = small ? (t[0].M + 63) / 64 : shape == 0 ? MB8 : MB4;
     const double a_bytes = (double)t[0].M * t[0].K * 2.0, w_bytes = (dual ? 2.0 : 1.0) * nb * tpw * 16.0 * t[0].K * 0.53;
     double best = 1e300;
     P.xm = 1;
     for (int xm = 1; xm <= 4; xm *= 2)
-      if (MBs % xm == 0 && nb % (8 / xm) == 0) {
+      if (MB % xm == 0 && nb % (8 / xm) == 0) {
         const double fill = 8.0 * (a_bytes / xm + w_bytes * xm / 8.0);
         if (fill < best) {
           best = fill;
@@ -1337,22 +1550,26 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
         }
       }
     const int env_xm = env_int("TPPX_TILED_XCD_M", 0);
-    if ((env_xm == 1 || env_xm == 2 || env_xm == 4) && MBs % env_xm == 0 && nb % (8 / env_xm) == 0)
+    if ((env_xm == 1 || env_xm == 2 || env_xm == 4) && MB % env_xm == 0 && nb % (8 / env_xm) == 0)
       P.xm = env_xm;
   }
-  if (shape == 2)
-    return dual ? big_launch<8, true, 1, 8>(P, MB4 * nb, stream) : big_launch<8, false, 1, 8>(P, MB4 * nb, stream);
-  // 128 x 256 workgroups that do not fill the CUs (at most one each): eight waves of 64 x 64 instead of four of
-  // 128 x 64 -- two waves per SIMD, so that one wave's waits are another's issue slots (the same sums in the same
-  // order: the same bits; 4096 x 4096 at 192-1024 rows 63-70 -> 49-57 us)
-  if (small)
-    return dual ? big_launch<2, true, 2, 2>(P, ((t[0].M + 63) / 64) * nb, stream)
-                : big_launch<2, false, 2, 2>(P, ((t[0].M + 63) / 64) * nb, stream);
-  if (shape == 1 && MB4 * nb <= 256 && env_int("TPPX_TILED_W8", 1) != 0)
-    return dual ? big_launch<4, true, 2, 4>(P, MB4 * nb, stream) : big_launch<4, false, 2, 4>(P, MB4 * nb, stream);
-  if (shape == 1)
-    return dual ? big_launch<8, true, 1, 4>(P, MB4 * nb, stream) : big_launch<8, false, 1, 4>(P, MB4 * nb, stream);
-  return dual ? big_launch<8, true, 2, 4>(P, MB8 * nb, stream) : big_launch<8, false, 2, 4>(P, MB8 * nb, stream);
+  const int wgs = MB * nb;
+  switch (shape) {
+  case TILE_128_512:
+    return dual ? big_launch<8, true, 1, 8>(P, wgs, stream) : big_launch<8, false, 1, 8>(P, wgs, stream);
+  case TILE_64_128:
+    return dual ? big_launch<2, true, 2, 2>(P, wgs, stream) : big_launch<2, false, 2, 2>(P, wgs, stream);
+  case TILE_128_128:
+    return dual ? big_launch<4, true, 2, 2>(P, wgs, stream) : big_launch<4, false, 2, 2>(P, wgs, stream);
+  case TILE_128_256:
+    // at most one workgroup per CU: eight waves of 64 x 64, two per SIMD, so that one wave's waits are another's issue
+    // slots; else four of 128 x 64, two workgroups per CU
+    if (wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0)
+      return dual ? big_launch<4, true, 2, 4>(P, wgs, stream) : big_launch<4, false, 2, 4>(P, wgs, stream);
+    return dual ? big_launch<8, true, 1, 4>(P, wgs, stream) : big_launch<8, false, 1, 4>(P, wgs, stream);
+  default:
+    return dual ? big_launch<8, true, 2, 4>(P, wgs, stream) : big_launch<8, false, 2, 4>(P, wgs, stream);
+  }
 }
 
 // MXFP4 weights x MXFP8 activations (t[i].xq = quantised activations in operand order, t[i].sa = their scale bytes)

@@ -401,6 +401,18 @@ int tppx_swiglu_mxfp4(const void* x, const void* qw_gate, const void* sw_gate,
                       int64_t M, int64_t N, int64_t K, int flags, void* ws,
                       int64_t ws_bytes, tppx_stream_t stream);
 
+/* Unquantized bf16 weights: several over one activation (q/k/v), or the gate/up pair with
+ * y = silu(gate) * up and the rounding points of fc_silu followed by fc_mul,
+ * as ONE launch of the large-M kernel (segs[i].sw is not used; it repeats
+ * segs[i].qw).  TPPX_EUNSUPPORTED where one tppx_linear_bf16 per weight is the
+ * way: few rows, operands of 4 GiB and more. */
+int tppx_multi_linear_bf16(const void* x, const tppx_seg* segs, int n_segs,
+                           int64_t M, int64_t K, int flags,
+                           tppx_stream_t stream);
+int tppx_swiglu_bf16(const void* x, const void* w_gate, const void* bias_gate,
+                     const void* w_up, const void* bias_up, void* y, int64_t M,
+                     int64_t N, int64_t K, int flags, tppx_stream_t stream);
+
 /* llama_rms_norm followed by the GEMMs that consume it, in ONE launch, for
  * decode steps (M <= 16): the two calls
  *   t_HS = llama_rms_norm(t_HS, gamma, eps); fused_qkv_gemm(t_HS, {Wq,Wk,Wv}, ...)

@@ -920,3 +920,28 @@ def test_prefill_mxfp4_ring_tiles(tile, M, N, K, monkeypatch):
     assert_close_bf16(t2bits(got[0]), ref, ulps=1, what=f"tile {tile}")
     for i, (a, b) in enumerate(zip(got, want)):
         assert torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("M", [65, 150, 333, 1000])
+@pytest.mark.parametrize("shape", [((1056, 64, 96), 640), ((4096, 1024, 1024), 256), ((2080, 2080), 128)])
+def test_prefill_bf16_groups_agree_with_single_launches(M, shape, monkeypatch):
+    """q/k/v and the gate/up pair on unquantized bf16 weights as one launch: the same sums in the same order as one
+    launch per weight (ragged rows and channel blocks, one K step and several, biases on some), hence the same bits;
+    every projection against a float64 product (bf16 rounding of the sum and of the result)."""
+    ops = _ops()
+    widths, K = shape
+    ws = [block_bf16(randn_bf16((n, K), 0.05, 750 + i)).cuda() for i, n in enumerate(widths)]
+    bs = [randn_bf16((widths[0],), 0.5, 755).cuda()] + [None] * (len(widths) - 1)
+    wu = block_bf16(randn_bf16((widths[0], K), 0.05, 756)).cuda()
+    x = randn_bf16((M, K), 1.0, 757).cuda()
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
+    got = ops._bf16_group(x, ws, bs)
+    pair = ops._bf16_group(x, [ws[0], wu], [bs[0], None], pair=True)
+    assert got is not None and pair is not None
+    for i, (w, b) in enumerate(zip(ws, bs)):
+        assert torch.equal(got[i], ops.linear(x, w, b)), i
+        flat = randn_bf16((widths[i], K), 0.05, 750 + i).cuda().double()
+        want = x.double() @ flat.t() + (b.double() if b is not None else 0.0)
+        assert ((got[i].double() - want).norm() / want.norm()).item() < 2.0 ** -8, i
+    assert torch.equal(pair, ops.fc_mul(x, wu, None, ops.fc_silu(x, ws[0], bs[0])))
+    assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws, bs), got))

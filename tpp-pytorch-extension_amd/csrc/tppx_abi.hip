@@ -246,14 +246,8 @@ static bool want_tiled(int64_t M, int flags, int64_t K = 0, int64_t n_tiles16 = 
     const double skinny_us = rows64 * (5.0 + wbytes / 5.5e6 + (double)K * 0.0004);
     return tiled_us <= skinny_us;
   }
-  if (kind == COST_BF16 && M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0) {
-    const int64_t wgs = ((M + 127) / 128) * ((n_tiles16 + 15) / 16);
-    const int64_t wgs2 = ((M + 63) / 64) * ((n_tiles16 + 7) / 8); // as 64 x 128 workgroups: the form up to 256 of them
-    const bool small = wgs2 <= 256 && env_int("TPPX_TILED_SMALL", 1) != 0;
-    const double tiled_us = small ? 12.0 + (double)K * 0.0045 : (17.0 + (double)K * 0.009) * std::max(1.0, (double)wgs / 200.0);
-    const double skinny_us = rows64 * (6.5 + wbytes / 5.5e6 + (double)K * 0.0006);
-    return tiled_us <= skinny_us;
-  }
+  if (kind == COST_BF16 && M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
+    return tiled_bf16_us(M, K, n_tiles16) <= rows64 * (6.5 + wbytes / 5.5e6 + (double)K * 0.0006);
   const bool big = (kind == COST_MXFP4 || kind == COST_MXFP4_PAIR) && M >= big_min_rows();
   if (big) // (a block row of the decode kernels: 9.6 us at 4096 x 4096, 16 at 4096 x 11008, 11-13 at 2560 x 10240, 13 at
            // 12288 x 4096; 33 at 3584 x 18944, beyond the kernels that split K; the pair 21 at 2 x 11008 x 4096)
@@ -729,6 +723,51 @@ extern "C" int tppx_linear_bf16(const void* x, const void* w, const void* bias, 
   const int nt = p.total_tiles > 512 ? 2 : 1; // two channel tiles per workgroup once one each still leaves two rounds
   set_groups(p, nt, false);
   return check_hip(launch_skinny_bf16(p, mg, nt, (hipStream_t)stream), who);
+}
+
+// n unquantized bf16 weights over one activation, or the gate/up pair, as one large-M launch; TPPX_EUNSUPPORTED where
+// one launch per weight is the way (few rows, operands of 4 GiB and more)
+static int run_bf16_group(const char* who, const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,
+                          bool dual, hipStream_t stream) {
+  int rc = check_common(who, x, M, K, n_segs, flags, nullptr, 0);
+  if (rc)
+    return rc;
+  TPPX_REQUIRE(segs, TPPX_EINVAL, "%s: null segment table", who);
+  TPPX_REQUIRE(K > 0 && K % 128 == 0, TPPX_ESHAPE, "%s: K=%ld must be a positive multiple of 128 (native bf16 tiles span 128 input channels)", who, (long)K);
+  TPPX_REQUIRE(!(flags & TPPX_FLAG_ACT_FP8), TPPX_EUNSUPPORTED, "%s: FP8 activations are built for MXFP4 weights only", who);
+  DecodeParams p;
+  memset(&p, 0, sizeof(p));
+  rc = fill_all(who, segs, n_segs, 16, dual, p);
+  if (rc)
+    return rc;
+  p.x = x;
+  p.M = (int)M;
+  p.K = (int)K;
+  const int64_t tiles = (dual ? 2 : 1) * (int64_t)p.total_tiles;
+  TiledParams t[TPPX_MAX_SEGS];
+  bool group = want_tiled(M, flags, K, tiles, (double)tiles * 16.0 * (double)K * 2.0, COST_BF16);
+  for (int i = 0; i < n_segs; i++) {
+    t[i] = tiled_from_seg(p, i);
+    TPPX_REQUIRE(M * t[i].N < ((int64_t)1 << 31), TPPX_ESHAPE, "%s: M*N=%ld outputs exceed 2^31", who, (long)(M * t[i].N));
+    TPPX_REQUIRE(aligned16(t[i].qw), TPPX_EINVAL, "%s: weight not 16-byte aligned", who);
+    if (dual)
+      t[i].post_op = TPPX_POST_NONE;
+    group = group && tiled_bf16_takes_groups(t[i]);
+  }
+  TPPX_REQUIRE(group, TPPX_EUNSUPPORTED, "%s: M=%ld runs as one launch per weight", who, (long)M);
+  return check_hip(launch_tiled_bf16_group(t, n_segs, stream, dual), who);
+}
+
+extern "C" int tppx_multi_linear_bf16(const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,
+                                      tppx_stream_t stream) {
+  return run_bf16_group("tppx_multi_linear_bf16", x, segs, n_segs, M, K, flags, false, (hipStream_t)stream);
+}
+
+extern "C" int tppx_swiglu_bf16(const void* x, const void* w_gate, const void* bias_gate, const void* w_up,
+                                const void* bias_up, void* y, int64_t M, int64_t N, int64_t K, int flags, tppx_stream_t stream) {
+  tppx_seg s[2] = {{w_gate, w_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
+                   {w_up, w_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
+  return run_bf16_group("tppx_swiglu_bf16", x, s, 2, M, K, flags, true, (hipStream_t)stream);
 }
 
 extern "C" int tppx_multi_linear_mxfp4(const void* x, const tppx_seg* segs,

@@ -112,6 +112,9 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
 hipError_t launch_tiled_qint8(const TiledParams& p, hipStream_t stream);
 // unquantized bf16 weights (native bf16 tiles in p.qw), more than 64 rows
 hipError_t launch_tiled_bf16(const TiledParams& p, hipStream_t stream);
+double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16);
+bool tiled_bf16_takes_groups(const TiledParams& p);
+hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual);
 hipError_t launch_tiled_mxfp4_fp8_group(const TiledParams* t, int n, hipStream_t stream, bool dual = false);
 bool tiled_qint8_takes_groups(const TiledParams& p);
 hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t stream);

@@ -585,7 +585,6 @@ struct BigParams {
 // answers the first use of any loaded register, and the fence of __syncthreads(), with a wait for ALL loads.
 template <int MT, bool DUAL, int WM, int WN, bool WBF16>
 __device__ __forceinline__ void big_gemm_body(const BigParams& P) {
-  static_assert(!WBF16 || !DUAL, "the bf16-weight form: single GEMMs");
   constexpr int WGM = MT * 16 * WM; // rows per workgroup
   constexpr int NBLK = MT * 4 / WN; // blocks of 4 rows x 256 B of the A tile that a wave fetches per K step
   static_assert(NBLK % 4 == 0, "the swizzle below takes a wave's first block to be a multiple of 4");
@@ -694,7 +693,7 @@ __device__ __forceinline__ void big_gemm_body(const BigParams& P) {
 #pragma unroll
     for (int nt = 0; nt < 4; nt++) {
       // native bf16 tiles: slot ((tile * KT + ks) * 4 + j) * 64 + lane, 16 bytes each
-      const char* src = qwb + (size_t)(((woff[nt] - (uint32_t)lane) * 4u + (uint32_t)(ks * 4 + j) * 64u + (uint32_t)lane) * 16u);
+      const char* src = (nt < 2 ? qwb : qwb2) + (size_t)(((woff[nt] - (uint32_t)lane) * 4u + (uint32_t)(ks * 4 + j) * 64u + (uint32_t)lane) * 16u);
       asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(bw[j][nt]) : "v"(src));
     }
   };
@@ -795,10 +794,10 @@ __device__ __forceinline__ void big_gemm_body(const BigParams& P) {
     big_epilogue<MT>(p, acc, reinterpret_cast<float*>(tl_lds) + wave * 64 * EP_LD, m_wg + wm * (MT * 16), tile_base);
 }
 
-template <int MT, int WM, int WN>
+template <int MT, bool DUAL, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
 big_bf16_kernel(const BigParams P) {
-  big_gemm_body<MT, false, WM, WN, true>(P);
+  big_gemm_body<MT, DUAL, WM, WN, true>(P);
 }
 
 // ---------------------------------------------------------------------------
@@ -1487,40 +1486,42 @@ static hipError_t big_launch(const BigParams& P, int wgs, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int MT, int WM, int WN>
+template <int MT, bool DUAL, int WM, int WN>
 static hipError_t big_bf16_launch(const BigParams& P, int wgs, hipStream_t stream) {
   const size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float);
   static_assert((size_t)WM * WN * 64 * EP_LD * sizeof(float) >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
-  TPPX_PLAN_ONLY((big_bf16_kernel<MT, WM, WN>), dim3(wgs), dim3(WM * WN * 64), lds);
-  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(big_bf16_kernel<MT, WM, WN>), lds); e != hipSuccess)
+  TPPX_PLAN_ONLY((big_bf16_kernel<MT, DUAL, WM, WN>), dim3(wgs), dim3(WM * WN * 64), lds);
+  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(big_bf16_kernel<MT, DUAL, WM, WN>), lds); e != hipSuccess)
     return e;
-  big_bf16_kernel<MT, WM, WN><<<dim3(wgs), dim3(WM * WN * 64), lds, stream>>>(P);
+  big_bf16_kernel<MT, DUAL, WM, WN><<<dim3(wgs), dim3(WM * WN * 64), lds, stream>>>(P);
   return hipGetLastError();
 }
 
-// dual: t[0] = gate, t[1] = up (equal shapes, n == 2); y[m][n] = silu(gate) * up goes to t[1].y
-hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
-  if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
-    return hipErrorInvalidValue;
-  // the workgroup tile with the lowest estimate (see tile_us)
-  auto workgroups = [&](int tile) {
-    const int tpw = TILE_COLS16[tile] / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
-    int nb = 0;
-    for (int i = 0; i < (dual ? 1 : n); i++)
-      nb += (t[i].tiles + tpw - 1) / tpw;
-    return (int64_t)((t[0].M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile]) * nb;
-  };
-  int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
-  if (shape < 0 || shape >= N_TILES) {
-    double best = 1e300;
-    for (int i = 0; i < (env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128); i++)
-      if (const double us = tile_us(i, workgroups(i), (double)(t[0].K / 128)); us < best) {
-        best = us;
-        shape = i;
-      }
-  }
-  const int tpw = TILE_COLS16[shape] / (dual ? 2 : 1), MB = (t[0].M + TILE_ROWS[shape] - 1) / TILE_ROWS[shape];
-  BigParams P;
+// workgroups of a launch over n GEMMs of one activation (dual: the gate/up pair)
+static int64_t group_workgroups(const TiledParams* t, int n, bool dual, int tile) {
+  const int tpw = TILE_COLS16[tile] / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
+  int64_t nb = 0;
+  for (int i = 0; i < (dual ? 1 : n); i++)
+    nb += (t[i].tiles + tpw - 1) / tpw;
+  return (t[0].M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile] * nb;
+}
+
+// the first `tiles` workgroup tiles' lowest estimate
+template <typename Us>
+static int cheapest_tile(const TiledParams* t, int n, bool dual, int tiles, Us&& us) {
+  int shape = 0;
+  double best = 1e300;
+  for (int i = 0; i < tiles; i++)
+    if (const double c = us(i, group_workgroups(t, n, dual, i), (double)(t[0].K / 128)); c < best) {
+      best = c;
+      shape = i;
+    }
+  return shape;
+}
+
+// fills P for n GEMMs over one activation with this workgroup tile; returns the workgroups of the launch
+static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int tile, double bytes_per_weight) {
+  const int tpw = TILE_COLS16[tile] / (dual ? 2 : 1), MB = (t[0].M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile];
   memset(&P, 0, sizeof(P));
   int nb = 0;
   for (int i = 0; i < n; i++) {
@@ -1535,25 +1536,34 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
   for (int i = n; i <= TPPX_MAX_SEGS; i++)
     P.nb0[i] = nb;
   P.n_seg = n;
-  {
-    // XCD rectangles: the split that moves the fewest bytes from memory into the L2s (activations: rows x K bf16 per
-    // row block, fetched by 8 / xm XCDs... every XCD fetches 1/xm of them; weights 0.53 B per element, xm/8 each)
-    const double a_bytes = (double)t[0].M * t[0].K * 2.0, w_bytes = (dual ? 2.0 : 1.0) * nb * tpw * 16.0 * t[0].K * 0.53;
-    double best = 1e300;
-    P.xm = 1;
-    for (int xm = 1; xm <= 4; xm *= 2)
-      if (MB % xm == 0 && nb % (8 / xm) == 0) {
-        const double fill = 8.0 * (a_bytes / xm + w_bytes * xm / 8.0);
-        if (fill < best) {
-          best = fill;
-          P.xm = xm;
-        }
+  // XCD rectangles: the split that moves the fewest bytes from memory into the L2s (activations: rows x K bf16 per
+  // row block, fetched by 8 / xm XCDs... every XCD fetches 1/xm of them; weights xm/8 each)
+  const double a_bytes = (double)t[0].M * t[0].K * 2.0, w_bytes = (dual ? 2.0 : 1.0) * nb * tpw * 16.0 * t[0].K * bytes_per_weight;
+  double best = 1e300;
+  P.xm = 1;
+  for (int xm = 1; xm <= 4; xm *= 2)
+    if (MB % xm == 0 && nb % (8 / xm) == 0) {
+      const double fill = 8.0 * (a_bytes / xm + w_bytes * xm / 8.0);
+      if (fill < best) {
+        best = fill;
+        P.xm = xm;
       }
-    const int env_xm = env_int("TPPX_TILED_XCD_M", 0);
-    if ((env_xm == 1 || env_xm == 2 || env_xm == 4) && MB % env_xm == 0 && nb % (8 / env_xm) == 0)
-      P.xm = env_xm;
-  }
-  const int wgs = MB * nb;
+    }
+  const int env_xm = env_int("TPPX_TILED_XCD_M", 0);
+  if ((env_xm == 1 || env_xm == 2 || env_xm == 4) && MB % env_xm == 0 && nb % (8 / env_xm) == 0)
+    P.xm = env_xm;
+  return MB * nb;
+}
+
+// dual: t[0] = gate, t[1] = up (equal shapes, n == 2); y[m][n] = silu(gate) * up goes to t[1].y
+hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
+  if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
+    return hipErrorInvalidValue;
+  int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
+  if (shape < 0 || shape >= N_TILES)
+    shape = cheapest_tile(t, n, dual, env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128, tile_us);
+  BigParams P;
+  const int wgs = big_params(P, t, n, dual, shape, 0.53);
   switch (shape) {
   case TILE_128_512:
     return dual ? big_launch<8, true, 1, 8>(P, wgs, stream) : big_launch<8, false, 1, 8>(P, wgs, stream);
@@ -1648,33 +1658,62 @@ silu_mul_kernel(const uint16_t* __restrict__ gate, uint16_t* __restrict__ y, int
   }
 }
 
-hipError_t launch_tiled_bf16(const TiledParams& p, hipStream_t stream) {
-  // prompt-sized passes: the 128 x 256 form of the large MXFP4 kernel with the weights read as they are (two
-  // workgroups of four waves per CU); its 32-bit offsets want operands below 4 GiB
-  if (p.M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0 &&
-      (int64_t)p.M * p.K * 2 < ((int64_t)1 << 32) && (int64_t)p.tiles * 32 * p.K < ((int64_t)1 << 32)) {
-    BigParams P;
-    memset(&P, 0, sizeof(P));
-    P.seg[0] = p;
-    // (the 256 x 256 and 128 x 512 forms of eight waves were measured too: equal at 28672 x 8192, 20-30 % slower
-    // at the 7B shapes)
-    const int nb = (p.tiles + 15) / 16;
-    for (int i = 1; i <= TPPX_MAX_SEGS; i++)
-      P.nb0[i] = nb;
-    P.n_seg = 1;
-    P.xm = 1;
-    // 64 x 128 workgroups, as for MXFP4, while there are at most 256 of them (with 2-byte weights they lose earlier:
-    // 11008 x 4096 at 192 rows, 258 workgroups: 62 us against 52)
-    if (((p.M + 63) / 64) * ((p.tiles + 7) / 8) <= 256 && env_int("TPPX_TILED_SMALL", 1) != 0) {
-      const int nbs = (p.tiles + 7) / 8;
-      for (int i = 1; i <= TPPX_MAX_SEGS; i++)
-        P.nb0[i] = nbs;
-      return big_bf16_launch<2, 2, 2>(P, ((p.M + 63) / 64) * nbs, stream);
-    }
-    if (((p.M + 127) / 128) * nb <= 256 && env_int("TPPX_TILED_W8", 1) != 0) // at most one workgroup per CU: eight waves, as for MXFP4
-      return big_bf16_launch<4, 2, 4>(P, ((p.M + 127) / 128) * nb, stream);
-    return big_bf16_launch<8, 1, 4>(P, ((p.M + 127) / 128) * nb, stream);
+// The same estimate for unquantized bf16 weights (four times the weight bytes of a step: what a CU takes in bounds the
+// small tiles; K = 4096 / 11008, one launch: 64 x 128 29 / 60 us, 128 x 256 51 / 116, 256 x 256 85 / 193, 128 x 512
+// 83 / 190; 64 x 128 doubles from 257 workgroups, 128 x 256 takes 95 us for 384 and 158 for 768).
+static double tile_bf16_us(int tile, int64_t wgs, double steps) {
+  const double rounds = (double)((wgs + 255) / 256);
+  switch (tile) {
+  case TILE_256_256:
+    return (20.0 + 2.03 * steps) * rounds;
+  case TILE_128_512:
+    return (20.0 + 2.05 * steps) * rounds;
+  case TILE_128_256:
+    return wgs <= 256 ? 14.0 + 1.2 * steps : wgs <= 400 ? 22.0 + 2.3 * steps : (30.0 + 2.5 * steps) * std::max(1.0, (double)wgs / 512.0);
+  default:
+    return wgs <= 256 ? 11.0 + 0.6 * steps : wgs <= 512 ? 8.0 + 1.38 * steps : (10.0 + 1.5 * steps) * (double)wgs / 512.0;
   }
+}
+
+double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16) {
+  double best = 1e300;
+  for (int i = 0; i < TILE_128_128; i++)
+    best = std::min(best, tile_bf16_us(i, (M + TILE_ROWS[i] - 1) / TILE_ROWS[i] * ((n_tiles16 + TILE_COLS16[i] - 1) / TILE_COLS16[i]),
+                                       (double)(K / 128)));
+  return best;
+}
+
+// prompt-sized passes; the kernel's 32-bit offsets want operands below 4 GiB
+bool tiled_bf16_takes_groups(const TiledParams& p) {
+  return p.M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0 && (int64_t)p.M * p.K * 2 < ((int64_t)1 << 32) &&
+         (int64_t)p.tiles * 32 * p.K < ((int64_t)1 << 32);
+}
+
+// n GEMMs over one activation in one launch (fuller last rounds: q/k/v of 4096 channels at 2048 rows 202 -> 157 us), or
+// the gate/up pair (dual, as launch_tiled_mxfp4_group: 11008 x 4096 at 2048 rows 359 -> 300 us, 333 rows 128 -> 93)
+hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
+  if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
+    return hipErrorInvalidValue;
+  const int shape = cheapest_tile(t, n, dual, env_int("TPPX_TILED_SMALL", 1) != 0 ? TILE_128_128 : TILE_64_128, tile_bf16_us);
+  BigParams P;
+  const int wgs = big_params(P, t, n, dual, shape, 2.0);
+  switch (shape) {
+  case TILE_128_512:
+    return dual ? big_bf16_launch<8, true, 1, 8>(P, wgs, stream) : big_bf16_launch<8, false, 1, 8>(P, wgs, stream);
+  case TILE_64_128:
+    return dual ? big_bf16_launch<2, true, 2, 2>(P, wgs, stream) : big_bf16_launch<2, false, 2, 2>(P, wgs, stream);
+  case TILE_128_256:
+    if (wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0) // at most one workgroup per CU: eight waves, as for MXFP4
+      return dual ? big_bf16_launch<4, true, 2, 4>(P, wgs, stream) : big_bf16_launch<4, false, 2, 4>(P, wgs, stream);
+    return dual ? big_bf16_launch<8, true, 1, 4>(P, wgs, stream) : big_bf16_launch<8, false, 1, 4>(P, wgs, stream);
+  default:
+    return dual ? big_bf16_launch<8, true, 2, 4>(P, wgs, stream) : big_bf16_launch<8, false, 2, 4>(P, wgs, stream);
+  }
+}
+
+hipError_t launch_tiled_bf16(const TiledParams& p, hipStream_t stream) {
+  if (tiled_bf16_takes_groups(p))
+    return launch_tiled_bf16_group(&p, 1, stream, false);
   const int MB = (p.M + 127) / 128, NB = (p.tiles + 7) / 8;
   const dim3 grid((unsigned)(MB * NB));
   const size_t lds = 2 * 2048 * 16;

@@ -442,6 +442,45 @@ def _linear_bf16(input, weight, bias, post, post_in, post_in2, post_scale, flags
     return y
 
 
+def _bf16_group(input, weights, biases, pair=False):
+    """q/k/v-like GEMMs (or, pair, the gate/up pair) with unquantized bf16 weights as one launch of the large-M kernel;
+    None where one call per weight is the way (few rows, other types, shapes that call refuses)."""
+    if isinstance(input, QTensor) or not isinstance(input, torch.Tensor) or input.dtype != torch.bfloat16 or not input.is_cuda:
+        return None
+    K = input.shape[-1] if input.dim() else 0
+    M = input.numel() // K if K else 0
+    n = len(weights)
+    if M <= 64 or not 2 <= n <= 4 or any(not _is_plain(w) or w.dtype != torch.bfloat16 or w.device != input.device
+                                         for w in weights):
+        return None
+    geo = [_blocked_geometry(w)[:2] for w in weights]
+    if any(k != K for _, k in geo) or (pair and geo[0] != geo[1]):
+        return None
+    L = _lib.lib()
+    x = input.contiguous()
+    keep = [(_prep_bias(b, N, x.device), _bf16_native(w)) for (N, _), b, w in zip(geo, biases, weights)]
+    lead = tuple(input.shape[:-1])
+    if pair:
+        y = torch.empty(lead + (geo[0][0],), dtype=torch.bfloat16, device=x.device)
+        rc = L.tppx_swiglu_bf16(x.data_ptr(), keep[0][1].data_ptr(), _lib.ptr(keep[0][0]), keep[1][1].data_ptr(),
+                                _lib.ptr(keep[1][0]), y.data_ptr(), M, geo[0][0], K, 0, _lib.stream_of(x))
+    else:
+        y = [torch.empty(lead + (N,), dtype=torch.bfloat16, device=x.device) for N, _ in geo]
+        segs = (_lib.Seg * n)()
+        for i, (b, nat) in enumerate(keep):
+            segs[i].qw = segs[i].sw = nat.data_ptr()
+            segs[i].bias = _lib.ptr(b)
+            segs[i].y = y[i].data_ptr()
+            segs[i].N = geo[i][0]
+            segs[i].post_op = POST_GELU if (n == 4 and i == 3) else POST_NONE
+            segs[i].post_scale = 1.0
+        rc = L.tppx_multi_linear_bf16(x.data_ptr(), segs, n, M, K, 0, _lib.stream_of(x))
+    if rc == _lib.EUNSUPPORTED:
+        return None
+    _lib.check(rc)
+    return y
+
+
 def _prep_bias(bias, N, dev):
     if bias is None or bias.numel() == 0:
         return None
@@ -972,6 +1011,9 @@ def qkv_gemm(input, weights, biases, norm=None):
             input = rms_norm(input, norm[0], norm[1])
         biases = list(biases) if biases is not None else []
         biases += [None] * (len(weights) - len(biases))
+        outs = _bf16_group(input, weights, biases)
+        if outs is not None:
+            return outs
         return [linear(input, w, b, POST_GELU if (len(weights) == 4 and i == 3) else POST_NONE)
                 for i, (w, b) in enumerate(zip(weights, biases))]
     if norm is not None:
@@ -1042,6 +1084,9 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
             rows = []  # one quantization of the rows for both projections
             gate = _linear_w4a8(input, w_gate, b_gate, POST_SILU, None, None, 1.0, rows)
             return _linear_w4a8(input, w_up, b_up, POST_MUL, gate, None, 1.0, rows)
+        y = _bf16_group(input, [w_gate, w_up], [b_gate, b_up], pair=True)
+        if y is not None:
+            return y
         return fc_mul(input, w_up, b_up, fc_silu(input, w_gate, b_gate))
     if norm is not None:
         _, M0, _, K0 = _prep_input(input, w_gate)

@@ -56,10 +56,10 @@ __device__ __forceinline__ void tile_of_block(int MB, int NB, int& bm, int& bn, 
     bn = (x / xm) * nb + r / mb;
     return;
   }
-  if ((T & 7) == 0) { // an eighth of the tiles in column-major order, whether or not NB divides by 8
-    const int per = T >> 3;
-    id = (id & 7) * per + (id >> 3);
-  }
+  // an eighth of the tiles in column-major order, whether or not NB divides by 8 (the first T mod 8 XCDs own one more);
+  // dealt round the XCDs instead, each of them fetches most of the weights
+  const int x = id & 7;
+  id = x * (T >> 3) + min(x, T & 7) + (id >> 3);
   bm = id % MB;
   bn = id / MB;
 }
@@ -1539,9 +1539,9 @@ static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int 
   // XCD rectangles: the split that moves the fewest bytes from memory into the L2s (activations: rows x K bf16 per
   // row block, fetched by 8 / xm XCDs... every XCD fetches 1/xm of them; weights xm/8 each)
   const double a_bytes = (double)t[0].M * t[0].K * 2.0, w_bytes = (dual ? 2.0 : 1.0) * nb * tpw * 16.0 * t[0].K * bytes_per_weight;
-  double best = 1e300;
+  double best = 8.0 * (a_bytes + w_bytes / 8.0); // xm = 1: an eighth of the channel blocks each, whether or not 8 divides them
   P.xm = 1;
-  for (int xm = 1; xm <= 4; xm *= 2)
+  for (int xm = 2; xm <= 4; xm *= 2)
     if (MB % xm == 0 && nb % (8 / xm) == 0) {
       const double fill = 8.0 * (a_bytes / xm + w_bytes * xm / 8.0);
       if (fill < best) {

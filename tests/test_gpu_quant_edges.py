@@ -264,3 +264,26 @@ def test_vnni2_quantizers_equal_the_general_ones(fmt, N, K, bk, bc):
     a, b = q(w5), q(w4)
     assert torch.equal(a.qdata, b.qdata)
     assert torch.equal(a.scales.view(torch.uint8), b.scales.view(torch.uint8))
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "qint2"])
+@pytest.mark.parametrize("off", [1, 2])
+def test_dequantize_takes_codes_at_any_address(fmt, off):
+    """Codes (and MXFP4 scale bytes) that start at a byte or half-word address, as a view into a larger buffer does:
+    the same values as from aligned memory."""
+    ops = _ops()
+    q = {"mxfp4": ops.remap_and_quantize_mxfp4, "qint2": ops.remap_and_quantize_qint2_intlv}[fmt]
+    W = randn_bf16((64, 512), 0.05, 5100)
+    w = q(W.view(2, 32, 8, 32, 2).permute(0, 2, 3, 1, 4).contiguous().cuda())
+    want = w.dequantize()
+
+    def moved(t):
+        buf = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)
+        buf[off:off + t.numel()] = t.reshape(-1)
+        return buf[off:off + t.numel()].view(t.shape)
+
+    w.qdata = moved(w.qdata)
+    if w.scales.element_size() == 1:
+        w.scales = moved(w.scales)
+    assert w.qdata.data_ptr() % 4 == off
+    assert torch.equal(w.dequantize(), want)

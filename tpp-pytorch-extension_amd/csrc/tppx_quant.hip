@@ -301,17 +301,23 @@ __constant__ float c_e2m1_tbl[16] = {0.0f,  0.5f,  1.0f,  1.5f, 2.0f,  3.0f,
                                      -2.0f, -3.0f, -4.0f, -6.0f};
 
 // one thread per four packed bytes (adjacent channels); out is [N/32][K/64][32][32][2] fp32.  Bound by the fp32 stores:
-// 11008 x 4096 in 32 us, 6.3 TB/s (51 us with a byte per thread and the values from a table in memory).
+// 11008 x 4096 in 32 us, 6.3 TB/s (51 us with a byte per thread and the values from a table in memory).  WIDE: codes and
+// scales are 4-byte, the output 16-byte aligned; else the same by bytes and single values.
+__device__ __forceinline__ uint32_t load_dword(const uint8_t* p) {
+  return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
+}
+template <bool WIDE>
 __global__ void __launch_bounds__(256)
-dequantize_mxfp4_kernel(const uint32_t* __restrict__ qdata, const uint8_t* __restrict__ scales, int64_t ndwords,
+dequantize_mxfp4_kernel(const uint8_t* __restrict__ qdata, const uint8_t* __restrict__ scales, int64_t ndwords,
                         float* __restrict__ out) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= ndwords)
     return;
   const int64_t tile = t >> 8;
   const uint32_t cg = (uint32_t)t & 7, c2 = ((uint32_t)t >> 3) & 31;
-  const uint32_t b = qdata[t];
-  const uint32_t sc = reinterpret_cast<const uint32_t*>(scales)[(tile * 2 + (c2 >> 4)) * 8 + cg];
+  const int64_t si = (tile * 2 + (c2 >> 4)) * 8 + cg;
+  const uint32_t b = WIDE ? reinterpret_cast<const uint32_t*>(qdata)[t] : load_dword(qdata + t * 4);
+  const uint32_t sc = WIDE ? reinterpret_cast<const uint32_t*>(scales)[si] : load_dword(scales + si * 4);
   typedef __attribute__((ext_vector_type(2))) float f32x2;
   f32x4 r[2];
   // the E2M1 values from the hardware (exact, at scale 1), the scale as one fp32 product
@@ -319,9 +325,15 @@ dequantize_mxfp4_kernel(const uint32_t* __restrict__ qdata, const uint8_t* __res
   const f32x2 v2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(b, 1.0f, 2), v3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(b, 1.0f, 3);
   r[0] = f32x4{v0[0] * e8m0_to_f32(sc), v0[1] * e8m0_to_f32(sc), v1[0] * e8m0_to_f32(sc >> 8), v1[1] * e8m0_to_f32(sc >> 8)};
   r[1] = f32x4{v2[0] * e8m0_to_f32(sc >> 16), v2[1] * e8m0_to_f32(sc >> 16), v3[0] * e8m0_to_f32(sc >> 24), v3[1] * e8m0_to_f32(sc >> 24)};
-  f32x4* o = reinterpret_cast<f32x4*>(out) + t * 2;
-  o[0] = r[0];
-  o[1] = r[1];
+  if (WIDE) {
+    f32x4* o = reinterpret_cast<f32x4*>(out) + t * 2;
+    o[0] = r[0];
+    o[1] = r[1];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      out[t * 8 + i] = r[i >> 2][i & 3];
+  }
 }
 
 // one thread per 4 int8; out [N/16][K/QBS][QBS/4][16][4] fp32
@@ -917,9 +929,10 @@ prepack_qint2_kernel(const uint8_t* __restrict__ q2, const float* __restrict__ s
 }
 
 // packed 2-bit (interleaved) -> fp32 in the logical blocked shape [N/32][K/bs][bs/4][32][4]; one thread per four
-// adjacent input channels of an output channel
+// adjacent input channels of an output channel.  WIDE: codes 4-byte, output 16-byte aligned; else by bytes and values.
+template <bool WIDE>
 __global__ void __launch_bounds__(256)
-dequantize_qint2_kernel(const uint32_t* __restrict__ q2, const float* __restrict__ s2, int64_t total, int64_t bs,
+dequantize_qint2_kernel(const uint8_t* __restrict__ q2, const float* __restrict__ s2, int64_t total, int64_t bs,
                         float* __restrict__ out) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= total)
@@ -927,7 +940,8 @@ dequantize_qint2_kernel(const uint32_t* __restrict__ q2, const float* __restrict
   const int64_t rest = t >> 5; // (n1*nb + b) * (bs/4) + c2
   const uint32_t r = (uint32_t)t & 31;
   const int64_t blk = (total >> 37) == 0 ? (int64_t)((uint32_t)rest / (uint32_t)(bs / 4)) : rest / (bs / 4);
-  const uint32_t codes = q2[rest * 8 + (r & 7)] >> (2 * (r >> 3));
+  const int64_t ci = rest * 8 + (r & 7);
+  const uint32_t codes = (WIDE ? reinterpret_cast<const uint32_t*>(q2)[ci] : load_dword(q2 + ci * 4)) >> (2 * (r >> 3));
   const float s = s2[blk * 32 + r];
   f32x4 o;
 #pragma unroll
@@ -935,7 +949,13 @@ dequantize_qint2_kernel(const uint32_t* __restrict__ q2, const float* __restrict
     const uint32_t code = (codes >> (8 * c3)) & 3u;
     o[c3] = (code == 1 ? 1.0f : (code == 2 ? -1.0f : 0.0f)) * s;
   }
-  reinterpret_cast<f32x4*>(out)[t] = o;
+  if (WIDE) {
+    reinterpret_cast<f32x4*>(out)[t] = o;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      out[t * 4 + i] = o[i];
+  }
 }
 
 // INT4 weight in the VNNI2 layout [N/16][K/bs][bs/2][16][2 codes per byte] -> native int8 tiles
@@ -1147,11 +1167,11 @@ extern "C" int tppx_dequantize_mxfp4(const void* qdata, const void* scales,
   TPPX_REQUIRE(qdata && scales && out_f32, TPPX_EINVAL, "tppx_dequantize_mxfp4: null pointer");
   TPPX_REQUIRE(N > 0 && K > 0 && N % 32 == 0 && K % 64 == 0, TPPX_ESHAPE,
                "tppx_dequantize_mxfp4: N=%ld must be a multiple of 32 and K=%ld of 64", (long)N, (long)K);
-  TPPX_REQUIRE((((uintptr_t)qdata | (uintptr_t)scales) & 3) == 0 && aligned16(out_f32), TPPX_EINVAL,
-               "tppx_dequantize_mxfp4: codes and scales must be 4-byte, the output 16-byte aligned");
-  int64_t ndwords = N * K / 8;
-  dequantize_mxfp4_kernel<<<grid_for(ndwords, 256), 256, 0, (hipStream_t)stream>>>(
-      (const uint32_t*)qdata, (const uint8_t*)scales, ndwords, (float*)out_f32);
+  const int64_t ndwords = N * K / 8;
+  const bool wide = (((uintptr_t)qdata | (uintptr_t)scales) & 3) == 0 && aligned16(out_f32);
+  const auto kernel = wide ? dequantize_mxfp4_kernel<true> : dequantize_mxfp4_kernel<false>;
+  kernel<<<grid_for(ndwords, 256), 256, 0, (hipStream_t)stream>>>((const uint8_t*)qdata, (const uint8_t*)scales, ndwords,
+                                                                 (float*)out_f32);
   return check_hip(hipGetLastError(), "tppx_dequantize_mxfp4");
 }
 
@@ -1351,8 +1371,9 @@ extern "C" int tppx_dequantize_qint2_intlv(const void* q, const void* scales, in
   TPPX_REQUIRE(q && scales && out_f32, TPPX_EINVAL, "%s: null pointer", who);
   if (int rc = check_qint2(who, N, K, bs))
     return rc;
-  TPPX_REQUIRE((reinterpret_cast<uintptr_t>(q) & 3u) == 0 && aligned16(out_f32), TPPX_EINVAL, "%s: codes must be 4-byte, the output 16-byte aligned", who);
-  dequantize_qint2_kernel<<<grid_for(N * K / 4, 256), 256, 0, (hipStream_t)stream>>>((const uint32_t*)q, (const float*)scales, N * K / 4, bs, (float*)out_f32);
+  const bool wide = (reinterpret_cast<uintptr_t>(q) & 3u) == 0 && aligned16(out_f32);
+  const auto kernel = wide ? dequantize_qint2_kernel<true> : dequantize_qint2_kernel<false>;
+  kernel<<<grid_for(N * K / 4, 256), 256, 0, (hipStream_t)stream>>>((const uint8_t*)q, (const float*)scales, N * K / 4, bs, (float*)out_f32);
   return check_hip(hipGetLastError(), who);
 }
 

@@ -413,6 +413,17 @@ int tppx_swiglu_bf16(const void* x, const void* w_gate, const void* bias_gate,
                      const void* w_up, const void* bias_up, void* y, int64_t M,
                      int64_t N, int64_t K, int flags, tppx_stream_t stream);
 
+/* The gate/up pair of QINT8-family weights as one launch behind the activation
+ * quantizer (xq / sa as in tppx_linear_qint8), the same bits as fc_silu
+ * followed by fc_mul.  TPPX_EUNSUPPORTED (before any launch) where one
+ * tppx_linear_qint8 per weight is the way: few rows, block sizes other than
+ * 256, operands of 4 GiB and more. */
+int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* qw_gate,
+                      const void* sw_gate, const void* bias_gate,
+                      const void* qw_up, const void* sw_up,
+                      const void* bias_up, void* y, int64_t M, int64_t N,
+                      int64_t K, int64_t qbs, int flags, tppx_stream_t stream);
+
 /* llama_rms_norm followed by the GEMMs that consume it, in ONE launch, for
  * decode steps (M <= 16): the two calls
  *   t_HS = llama_rms_norm(t_HS, gamma, eps); fused_qkv_gemm(t_HS, {Wq,Wk,Wv}, ...)

@@ -945,3 +945,21 @@ def test_prefill_bf16_groups_agree_with_single_launches(M, shape, monkeypatch):
         assert ((got[i].double() - want).norm() / want.norm()).item() < 2.0 ** -8, i
     assert torch.equal(pair, ops.fc_mul(x, wu, None, ops.fc_silu(x, ws[0], bs[0])))
     assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws, bs), got))
+
+
+@pytest.mark.parametrize("fmt", ["qint8", "qint4"])
+@pytest.mark.parametrize("M,N,K", [(65, 160, 256), (129, 544, 512), (300, 96, 768), (200, 2080, 1280), (1000, 4160, 512)])
+def test_prefill_qint8_pair_agrees_with_two_launches(fmt, M, N, K, monkeypatch):
+    """The gate/up pair of QINT8-family weights as one launch: the same sums in the same order and the same rounding
+    points as fc_silu followed by fc_mul, hence the same bits (one scale block and several, ragged rows and channel
+    blocks, the 64-row and the 128-row workgroups, a bias on one of the two)."""
+    ops = _ops()
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
+    quant = {"qint8": ops.remap_and_quantize_qint8, "qint4": lambda t: ops.quantize_int4sym(t, 256, 2, True)}[fmt]
+    ws = [quant(block_bf16(randn_bf16((N, K), 0.05, 760 + i), bc=256).cuda()) for i in range(2)]
+    b = randn_bf16((N,), 0.5, 762).cuda()
+    x = randn_bf16((M, K), 1.0, 763).cuda()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "fc_silu", None)  # (the two launches would call it)
+        got = ops.swiglu_gate_up(x, ws[0], ws[1], b, None)
+    assert torch.equal(got, ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], b)))

@@ -475,7 +475,7 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
 
 static int run_qint8(const char* who, const void* x, void* xq, void* sa, const tppx_seg* segs,
                      int n_segs, int64_t M, int64_t K, int64_t qbs, int flags, void* ws,
-                     int64_t ws_bytes, hipStream_t stream) {
+                     int64_t ws_bytes, hipStream_t stream, bool dual = false) {
   // x == NULL: xq / sa already hold quantized activations (the reference's
   // pre-quantized input case, src/csrc/fused_gemm.h:1244-1246)
   int rc = check_common(who, x ? x : xq, M, K, n_segs, flags, ws, ws_bytes);
@@ -488,7 +488,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
   TPPX_REQUIRE(qbs > 0 && qbs % 64 == 0 && K % qbs == 0, TPPX_ESHAPE, "%s: block size mismatch (qbs=%ld, K=%ld)", who, (long)qbs, (long)K);
   DecodeParams p;
   memset(&p, 0, sizeof(p));
-  rc = fill_all(who, segs, n_segs, 16, false, p);
+  rc = fill_all(who, segs, n_segs, 16, dual, p);
   if (rc)
     return rc;
   p.x = x;
@@ -504,27 +504,26 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
   p.units = (int)(K / (64 * p.deal));
   p.spb_magic = (p.deal == 4 && p.tpb > 4) ? (unsigned int)((((uint64_t)1 << 32) + (uint64_t)(p.tpb / 4) - 1) / (uint64_t)(p.tpb / 4)) : 0u;
   const bool reuse = (flags & TPPX_FLAG_XQ_REUSE) != 0; // xq / sa still hold this x, quantized by an earlier call
-  if (qbs % 128 == 0 && want_tiled(M, flags, K, p.total_tiles, (double)p.total_tiles * 16.0 * (double)K, COST_QINT8)) {
+  const int64_t tiles = (dual ? 2 : 1) * (int64_t)p.total_tiles;
+  const bool tiled = qbs % 128 == 0 && want_tiled(M, flags, K, tiles, (double)tiles * 16.0 * (double)K, COST_QINT8);
+  TiledParams t[TPPX_MAX_SEGS];
+  bool group = tiled && n_segs > 1; // one grid over the channel blocks of all GEMMs when the large-M kernel takes them
+  for (int i = 0; i < n_segs && tiled; i++) {
+    t[i] = tiled_from_seg(p, i);
+    t[i].qbs = (int)qbs;
+    group = group && tiled_qint8_takes_groups(t[i]);
+  }
+  TPPX_REQUIRE(!dual || group, TPPX_EUNSUPPORTED, "%s: M=%ld runs as one launch per weight", who, (long)M);
+  if (tiled) {
     if (x && !reuse) {
       rc = check_hip(launch_quant_act_int8(x, M, K, qbs, xq, sa, 0, stream), who);
       if (rc)
         return rc;
     }
-    if (n_segs > 1) { // fused q/k/v: one grid over the channel blocks of all GEMMs when the large-M kernel takes them
-      TiledParams t[TPPX_MAX_SEGS];
-      bool group = true;
-      for (int i = 0; i < n_segs; i++) {
-        t[i] = tiled_from_seg(p, i);
-        t[i].qbs = (int)qbs;
-        group = group && tiled_qint8_takes_groups(t[i]);
-      }
-      if (group)
-        return check_hip(launch_tiled_qint8_group(t, n_segs, stream), who);
-    }
+    if (group)
+      return check_hip(launch_tiled_qint8_group(t, n_segs, stream, dual), who);
     for (int i = 0; i < n_segs; i++) {
-      TiledParams t = tiled_from_seg(p, i);
-      t.qbs = (int)qbs;
-      rc = check_hip(launch_tiled_qint8(t, stream), who);
+      rc = check_hip(launch_tiled_qint8(t[i], stream), who);
       if (rc)
         return rc;
     }
@@ -768,6 +767,16 @@ extern "C" int tppx_swiglu_bf16(const void* x, const void* w_gate, const void* b
   tppx_seg s[2] = {{w_gate, w_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
                    {w_up, w_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
   return run_bf16_group("tppx_swiglu_bf16", x, s, 2, M, K, flags, true, (hipStream_t)stream);
+}
+
+extern "C" int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* qw_gate, const void* sw_gate,
+                                 const void* bias_gate, const void* qw_up, const void* sw_up, const void* bias_up, void* y,
+                                 int64_t M, int64_t N, int64_t K, int64_t qbs, int flags, tppx_stream_t stream) {
+  const char* who = "tppx_swiglu_qint8";
+  TPPX_REQUIRE(M <= 0 || N < ((int64_t)1 << 31) / M, TPPX_ESHAPE, "%s: M*N outputs exceed 2^31", who);
+  tppx_seg s[2] = {{qw_gate, sw_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
+                   {qw_up, sw_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
+  return run_qint8(who, x, xq, sa, s, 2, M, K, qbs, flags, nullptr, 0, (hipStream_t)stream, true);
 }
 
 extern "C" int tppx_multi_linear_mxfp4(const void* x, const tppx_seg* segs,

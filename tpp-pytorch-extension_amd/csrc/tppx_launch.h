@@ -117,7 +117,7 @@ bool tiled_bf16_takes_groups(const TiledParams& p);
 hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual);
 hipError_t launch_tiled_mxfp4_fp8_group(const TiledParams* t, int n, hipStream_t stream, bool dual = false);
 bool tiled_qint8_takes_groups(const TiledParams& p);
-hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t stream);
+hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t stream, bool dual = false);
 // y[i] = bf16( silu(gate[i]) * y[i] ) with the rounding points of SiluPostOp followed by MulPostOp; n % 8 == 0
 hipError_t launch_silu_mul(const uint16_t* gate, uint16_t* y, int64_t n, hipStream_t stream);
 

@@ -1097,6 +1097,19 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
     if N2 != N or w_gate._qscheme != w_up._qscheme:
         raise TppxError(_lib.ESHAPE, "gate and up projections must have the same shape and format")
     if w_gate._qscheme != QSCHEME_MXFP:
+        # the large-M kernel (from 65 rows, where the library's estimate prefers it to the row kernels, blocks of 256)
+        # takes the pair as one launch behind one quantization: rounds(2w) <= 2 rounds(w), so it is never the slower way
+        if M > 64 and w_gate.block_size == w_up.block_size == 256:
+            y = torch.empty(tuple(input.shape[:-1]) + (N,), dtype=torch.bfloat16, device=x.device)
+            bg, bu = _prep_bias(b_gate, N, x.device), _prep_bias(b_up, N, x.device)
+            (qg, sg), (qu, su) = w_gate.native(), w_up.native()
+            xq, sa = _qint8_scratch(x, M, K, 256)
+            rc = L.tppx_swiglu_qint8(x.data_ptr(), xq.data_ptr(), sa.data_ptr(), qg.data_ptr(), sg.data_ptr(), _lib.ptr(bg),
+                                     qu.data_ptr(), su.data_ptr(), _lib.ptr(bu), y.data_ptr(), M, N, K, 256, 0,
+                                     _lib.stream_of(x))
+            if rc != _lib.EUNSUPPORTED:
+                _lib.check(rc)
+                return y
         g = fc_silu(input, w_gate, b_gate)
         return fc_mul(input, w_up, b_up, g)
     y = torch.empty(tuple(input.shape[:-1]) + (N,), dtype=torch.bfloat16, device=x.device)

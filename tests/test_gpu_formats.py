@@ -531,3 +531,94 @@ def test_w4a8_row_group_kernel(M, N, K, bc, post):
     assert_close_bf16(t2bits(y), ref, ulps=2 if post == "silu" else 1, what=f"w4a8 rows M={M} N={N} K={K} {post}", pre_bits=pre)
     assert torch.equal(ops.swiglu_gate_up(x.cuda(), qt, qt, b.cuda(), b.cuda()),
                        ops.fc_mul(x.cuda(), qt, b.cuda(), ops.fc_silu(x.cuda(), qt, b.cuda())))
+
+
+def _w4a8(N, K, bc, seed):
+    W = randn_bf16((N, K), 0.05, seed)
+    t = W.view(N // 16, 16, K // bc, bc // 2, 2).permute(0, 2, 3, 1, 4).contiguous()
+    return _ops().remap_and_quantize_mxfp4(t.cuda(), int8_layout=True), t
+
+
+def _w4a8_two_steps(qt, x, bias, post, r, r2, scale):
+    """The activation quantizer followed by tppx_linear_mxfp4_int8."""
+    ops = _ops()
+    from tpp_pytorch_extension import _lib
+    (N, K), M = qt.weight_nk(), x.shape[0]
+    act = ops.quantize_int8sym(x, 32, -1, False)
+    sa = act.scales.mul_(ops.W4A8_ACT_SCALE)
+    y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    p = _lib.ptr
+    _lib.check(_lib.lib().tppx_linear_mxfp4_int8(act.qdata.data_ptr(), sa.data_ptr(), qt.qdata.data_ptr(), qt.scales.data_ptr(),
+                                                 p(bias), p(r), p(r2), y.data_ptr(), M, N, K, qt.shape[2] * 8, post, scale,
+                                                 _lib.stream_of(x)))
+    return y
+
+
+# K tiles of 128: 1 and 2 (quarters of one tile or less), 5, 9, 15 (quarters that begin and end inside a tile), 8, 86
+@pytest.mark.parametrize("M,N,K,bc,post", [(17, 96, 128, 32, "none"), (31, 272, 256, 64, "add"), (32, 4096, 640, 64, "silu"),
+                                           (33, 144, 1152, 128, "mul"), (48, 1040, 1920, 64, "add2"), (63, 272, 1024, 64, "gelu"),
+                                           (16, 256, 11008, 64, "relu"), (1, 48, 18944, 64, "add")])
+def test_w4a8_row_groups_have_the_bits_of_the_two_step_path(M, N, K, bc, post):
+    """W4A8 calls of fewer than 64 rows behind the operand-order quantizer: the quantizer, the integer sums, the four K
+    quarters and the order they are added in are the two-step path's, so the outputs are EQUAL to it (ordinary rows,
+    zero blocks, subnormal ones, and blocks with an infinity or a NaN)."""
+    ops = _ops()
+    posts = {"none": O.POST_NONE, "add": O.POST_ADD_SCALE, "silu": O.POST_SILU, "mul": O.POST_MUL, "add2": O.POST_ADD2_SCALE,
+             "gelu": O.POST_GELU, "relu": O.POST_RELU}
+    qt = _w4a8(N, K, bc, 3200 + M)[0]
+    x = randn_bf16((M, K), 1.0, 3210 + M)
+    x[M - 1, :64] = 0.0
+    x[M // 2, 64:96] = 1e-39
+    x, b, r = x.cuda(), randn_bf16((N,), 0.1, 3220).cuda(), randn_bf16((M, N), 1.0, 3230).cuda()
+    r2 = randn_bf16((M, N), 1.0, 3240).cuda() if post == "add2" else None
+    args = (posts[post], r if post in ("add", "mul", "add2") else None, r2, 0.5)
+    assert qt.native_w4a8() is not None
+    for bias in (b, None):
+        want = _w4a8_two_steps(qt, x, bias, *args)
+        assert torch.equal(_w4a8_mid(qt, x, bias, *args), want)
+        if M > 16:
+            assert torch.equal(ops.linear(x, qt, bias, *args), want)
+    x[0, 5], x[M - 1, 40] = float("inf"), float("nan")
+    y, want = _w4a8_mid(qt, x, b, *args), _w4a8_two_steps(qt, x, b, *args)
+    assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.nan_to_num(y), torch.nan_to_num(want))
+
+
+def _w4a8_mid(qt, x, bias, post, r, r2, scale):
+    """tppx_linear_mxfp4_int8_mid, whichever kernel the operator would choose."""
+    from tpp_pytorch_extension import _lib
+    (N, K), M = qt.weight_nk(), x.shape[0]
+    mp = (M + 63) // 64 * 64
+    xq = torch.empty(mp * K, dtype=torch.int8, device="cuda")
+    sa = torch.empty(mp * K // 32, dtype=torch.float32, device="cuda")
+    y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    p = _lib.ptr
+    _lib.check(_lib.lib().tppx_linear_mxfp4_int8_mid(x.data_ptr(), xq.data_ptr(), sa.data_ptr(), *[a.data_ptr() for a in qt.native_w4a8()],
+                                                     p(bias), p(r), p(r2), y.data_ptr(), M, N, K, post, scale, 0, _lib.stream_of(x)))
+    return y
+
+
+@pytest.mark.parametrize("M,N,K,bc,post", [(64, 96, 128, 32, "none"), (65, 272, 640, 64, "add"), (100, 4096, 256, 64, "silu"),
+                                           (127, 8448, 1152, 128, "mul"), (129, 1040, 384, 64, "add2"), (200, 11008, 512, 64, "none")])
+def test_w4a8_row_groups_equal_the_oracle_from_64_rows(M, N, K, bc, post):
+    """From 64 rows on K is folded in one ascending sum per output, on the row-group kernel as on the prompt kernel: the
+    GEMM equals the oracle bit for bit, and with a post-op the prompt kernel (one and two row tiles per wave, ragged
+    rows and channel groups)."""
+    ops = _ops()
+    posts = {"none": O.POST_NONE, "add": O.POST_ADD_SCALE, "silu": O.POST_SILU, "mul": O.POST_MUL, "add2": O.POST_ADD2_SCALE}
+    from tpp_pytorch_extension import _lib
+    qt, t = _w4a8(N, K, bc, 3300 + M)
+    q_or, s_or = O.remap_quantize_mxfp4_int8(t.float().numpy())
+    x = randn_bf16((M, K), 1.0, 3310 + M)
+    x[M - 1, :64] = 0.0
+    b, r, r2 = randn_bf16((N,), 0.1, 3320), randn_bf16((M, N), 1.0, 3330).cuda(), randn_bf16((M, N), 1.0, 3340).cuda()
+    xg, bg = x.cuda(), b.cuda()
+    assert np.array_equal(t2bits(_w4a8_mid(qt, xg, bg, O.POST_NONE, None, None, 1.0)), O.linear_w4a8(t2bits(x), q_or, s_or, bc, t2bits(b)))
+    in1, in2 = r if post in ("add", "mul", "add2") else None, r2 if post == "add2" else None
+    mp = (M + 127) // 128 * 128
+    ws = torch.empty(mp * K * 2 + mp * (K // 32) * 4, dtype=torch.uint8, device="cuda")
+    want = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    _lib.check(_lib.lib().tppx_linear_mxfp4_int8_wide(xg.data_ptr(), qt.native_w4a8_wide().data_ptr(), bg.data_ptr(), _lib.ptr(in1),
+                                                      _lib.ptr(in2), want.data_ptr(), M, N, K, posts[post], 0.5, ws.data_ptr(),
+                                                      ws.numel(), _lib.stream_of(xg)))
+    assert torch.equal(_w4a8_mid(qt, xg, bg, posts[post], in1, in2, 0.5), want)
+    assert torch.equal(ops.linear(xg, qt, bg, posts[post], in1, in2, 0.5), want)

@@ -961,22 +961,22 @@ extern "C" int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa, con
                                           int64_t M, int64_t N, int64_t K, int post_op, float post_scale, int flags,
                                           tppx_stream_t stream) {
   const char* who = "tppx_linear_mxfp4_int8_mid";
+  TPPX_REQUIRE(M <= 0 || (K / 128 <= 65535 && (M + 63) / 64 <= 32767 && N <= (1 << 25) && N < ((int64_t)1 << 31) / M),
+               TPPX_EUNSUPPORTED, "%s: M=%ld N=%ld K=%ld is too large for this kernel's 32-bit offsets and grid", who, (long)M,
+               (long)N, (long)K);
   int rc = check_common(who, x, M, K, 1, 0, nullptr, 0);
   if (rc)
     return rc;
   TPPX_REQUIRE((flags & ~TPPX_FLAG_XQ_REUSE) == 0, TPPX_EINVAL, "%s: flags 0x%x not taken here (TPPX_FLAG_XQ_REUSE only)", who, flags);
-  TPPX_REQUIRE(K > 0 && K % 128 == 0 && K / 128 <= 65535, TPPX_ESHAPE, "%s: K=%ld must be a positive multiple of 128", who, (long)K);
+  TPPX_REQUIRE(K > 0 && K % 128 == 0, TPPX_ESHAPE, "%s: K=%ld must be a positive multiple of 128", who, (long)K);
   TPPX_REQUIRE(xq && sa && aligned16(xq) && aligned16(sa), TPPX_EINVAL, "%s: null or misaligned xq / sa scratch", who);
+  TPPX_REQUIRE(aligned16(s_nat), TPPX_EINVAL, "%s: scales not 16-byte aligned", who);
   tppx_seg s = {q_nat, s_nat, bias, post_in, post_in2, y, N, post_op, post_scale};
   DecodeParams p;
   memset(&p, 0, sizeof(p));
   rc = fill_all(who, &s, 1, 16, false, p);
   if (rc)
     return rc;
-  TPPX_REQUIRE(M * N < ((int64_t)1 << 31), TPPX_ESHAPE, "%s: output too large", who);
-  const int mg = M <= 32 ? 2 : 4;
-  const int grid_y = (int)((M + 16 * mg - 1) / (16 * mg));
-  TPPX_REQUIRE(grid_y <= 65535, TPPX_ESHAPE, "%s: M=%ld too large", who, (long)M);
   p.x = x;
   p.xq = xq;
   p.sa = (const float*)sa;
@@ -985,17 +985,13 @@ extern "C" int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa, con
   p.units = (int)(K / 128);
   p.tpb = 1;
   p.S = 1;
-  p.mt = grid_y * mg;
-  int ntw = 1; // one round of 256 workgroups as long as three channel tiles per workgroup allow
-  while (ntw < 3 && (p.total_tiles + ntw - 1) / ntw > 256)
-    ntw++;
-  set_groups(p, ntw, false);
+  p.mt = (int)((M + 63) / 64 * 4);
   if (!(flags & TPPX_FLAG_XQ_REUSE)) {
     rc = check_hip(launch_quant_act_w4a8_rows(x, M, K, p.mt, xq, (float*)sa, (hipStream_t)stream), who);
     if (rc)
       return rc;
   }
-  return check_hip(launch_skinny_w4a8_mg(p, mg, ntw, (hipStream_t)stream), who);
+  return check_hip(launch_skinny_w4a8_mg(p, M >= 64, (hipStream_t)stream), who);
 }
 
 extern "C" void tppx_reload_env(void) {

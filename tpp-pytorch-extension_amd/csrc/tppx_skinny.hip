@@ -83,9 +83,7 @@ __device__ unsigned int sk_split_tickets[SK_TICKETS];
 // cross-wave sums then unroll completely and all of a thread's LDS reads are issued before the first wait; with a
 // run-time count the compiler waited for the LDS once per output and batch of eight (36 waits of an LDS round trip
 // each in the 64-row gate/up epilogue: 1.3 us per half).
-// TR (finish() only): the accumulators are transposed result tiles -- lane l holds channels (l >> 4) * 4 + r of row
-// l & 15 (weights as the MFMA's first operand) -- written into the same region as one 16-byte store per tile.
-template <int MG, int NACC, bool DUAL, int MINW, int FIXW = 0, bool TR = false>
+template <int MG, int NACC, bool DUAL, int MINW, int FIXW = 0>
 struct SkEpilogue {
   static __device__ __forceinline__ int nthreads() { return FIXW ? FIXW * 64 : (int)blockDim.x; }
   static __device__ __forceinline__ int nwaves() { return FIXW ? FIXW : (int)(blockDim.x >> 6); }
@@ -345,15 +343,10 @@ struct SkEpilogue {
 #pragma unroll
     for (int a = 0; a < NACC; a++)
 #pragma unroll
-      for (int mg = 0; mg < MG; mg++) {
-        if constexpr (TR) {
-          *reinterpret_cast<f32x4*>(mine + (a * MG + mg) * 256 + (lane & 3) * 64 + ((lane >> 2) & 3) * 16 + (lane >> 4) * 4) = acc[a][mg];
-        } else {
+      for (int mg = 0; mg < MG; mg++)
 #pragma unroll
-          for (int r = 0; r < 4; r++)
-            mine[(a * MG + mg) * 256 + r * 64 + lane] = acc[a][mg][r];
-        }
-      }
+        for (int r = 0; r < 4; r++)
+          mine[(a * MG + mg) * 256 + r * 64 + lane] = acc[a][mg][r];
     __syncthreads();
     // (no branch per output: slots past the outputs repeat the last one and are not stored, so the outputs' LDS reads
     // and post-op chains interleave)
@@ -392,6 +385,35 @@ struct SkEpilogue {
     }
     if (!DUAL && MG == 1 && sumsq) // uniform
       leave_row_sums(ov, sumsq, M);
+  }
+
+  // The waves of a K part own different result tiles (channel tile a, row tile mg) of the workgroup: this wave has the
+  // OWN tiles slot0, slot0 + 1, .. (slot = a * MG + mg) of part kp.  The tiles are transposed: lane l holds channels
+  // (l >> 4) * 4 + r of row l & 15 (weights as the MFMA's first operand).  The KP parts are added in part order.
+  template <int KP, int OWN>
+  __device__ __forceinline__ void finish_parts(const DecodeSeg& sg, f32x4 (&acc)[OWN], float* red, int kp, int slot0) {
+    static_assert(!DUAL && OUT % (FIXW * 64) == 0, "every thread finishes the same number of outputs");
+    settle();
+    const int lane = threadIdx.x & 63;
+    float* mine = red + kp * ELEMS + slot0 * 256 + (lane & 3) * 64 + ((lane >> 2) & 3) * 16 + (lane >> 4) * 4;
+#pragma unroll
+    for (int o = 0; o < OWN; o++)
+      *reinterpret_cast<f32x4*>(mine + o * 256) = acc[o];
+    __syncthreads();
+    uint32_t out[MAXE];
+#pragma unroll
+    for (int i = 0; i < MAXE; i++) {
+      const int e = (int)threadIdx.x + i * nthreads();
+      float v = red[e];
+#pragma unroll
+      for (int k = 1; k < KP; k++)
+        v += red[k * ELEMS + e];
+      out[i] = apply_post_bits(bf16_bits_to_f32(bias[i]) + v, sg.post_op, in1[i], in2[i], sg.post_scale);
+    }
+#pragma unroll
+    for (int i = 0; i < MAXE; i++)
+      if (off[i] >= 0)
+        sg.y[off[i]] = (uint16_t)out[i];
   }
 };
 
@@ -1604,119 +1626,157 @@ skinny_w4a8_kernel(const DecodeParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// W4A8, 17..64 rows per block row (and fewer rows that do not fit the kernel above's LDS).  The rows arrive quantised
-// in operand order (quant_act_w4a8_rows_kernel): xq [K/128][mt][2 halves][64 lanes (g, m)][16 B], 8 bytes of each of
-// two MX blocks per lane, and scales sa [K/128][mt][16 m][4 blocks] f32, already times 6 / 127.  Eight waves split K
-// in tiles of 128 channels; weight tiles and their E8M0 dwords as in skinny_w4a8_kernel.  The weights are the MFMA's
-// FIRST operand, so a result tile is [channel][row]: a lane's four sums belong to one row, whose four block scales of
-// a K tile are one 16-byte load, and no scale goes through LDS.
+// W4A8 between the kernel above and the prompt passes.  The rows arrive quantised in operand order
+// (quant_act_w4a8_rows_kernel): xq [K/128][mt][2 halves][64 lanes (g, m)][16 B], 8 bytes of each of two MX blocks per
+// lane, and scales sa [K/128][mt][16 m][4 blocks] f32, already times 6 / 127.  Weight tiles and their E8M0 dwords as in
+// skinny_w4a8_kernel.  The weights are the MFMA's FIRST operand, so a result tile is [channel][row]: a lane's four sums
+// belong to one row, whose four block scales of a K tile are one 16-byte load, and no scale goes through LDS.
+// A wave owns ONE channel tile, MG row tiles and one of KP parts of K; a workgroup T channel tiles and MG * R row tiles.
+//   KP = 4  the parts are linear_w4a8_kernel's, contiguous quarters of the MX blocks (a quarter may begin and end inside
+//           a K tile: its first and last tile skip the blocks outside), each folded in ascending order, added in part
+//           order and to the bias: that kernel's bits
+//   KP = 1  all of K in ascending order on top of the bias: the prompt kernel's (and the oracle's) bits
 // What bounds it: vector issue.  Every K = 32 MFMA (one MX block) leaves 4 sums per lane to convert, scale and add
-// (12 instructions) behind the expansion of the codes (about 18, shared by the MG row tiles); the weight stream
-// (24 MB at 11008 x 4096) hides behind that from 32 rows on.  Whole calls with the quantizer, back to back: 32 rows
-// 18 us, 63 rows 23 us at 11008 x 4096 (73 and more on one wave per 16 x 16 tile, which this kernel replaces wherever
-// the weight could be prepacked); the SwiGLU block 4096 - 11008 - 4096 at 32 rows 171 -> 47 us.
+// (12 instructions) behind the expansion of the codes (about 18, shared by the wave's MG row tiles); the weight stream
+// hides behind that from 32 rows on.  Whole calls, quantizer included, weights from memory, in us, and in brackets the
+// kernel with the same bits (32 and 63 rows: the two-step path; from 64 rows: the prompt kernel):
+//   rows     4096 x 4096    11008 x 4096    4096 x 11008    3584 x 18944
+//   32       10 (35)        17 (52)         17 (63)         25 (104)
+//   63       13 (43)        24 (79)         23 (81)         35 (142)
+//   64       16 (38)        28 (47)         33 (94)         58 (152)
+//   128      23 (38)        39 (47)         52 (94)         82 (153)
+//   256      31 (39)        68 (67)         70 (93)         111 (151)
 // ---------------------------------------------------------------------------
-template <int MG, int NTW, int PF>
-__global__ void __launch_bounds__(512)
+template <int MG, int T, int R, int KP, int PF>
+__global__ void __launch_bounds__(KP * T * R * 64)
 skinny_w4a8_mg_kernel(const DecodeParams p) {
+  static_assert(KP == 1 || KP == 4, "K parts");
   extern __shared__ __align__(16) float sk_lds[];
-  constexpr int W = 8;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int grp = blockIdx.x;
-  const DecodeSeg& sg = p.seg[sk_find_seg(p, grp)];
-  const int ltile0 = (grp - sg.grp0) * NTW;
-  const int m0 = blockIdx.y * (MG * 16);
+  const int kp = wave % KP, rr = (wave / KP) % R, tt = wave / (KP * R);
+  const DecodeSeg& sg = p.seg[0];
+  const int ltile0 = blockIdx.x * T;
+  const int m0 = blockIdx.y * (MG * R * 16);
   const int KT = p.units; // K tiles of 128 channels
-  const int t0 = (wave * KT) / W, t1 = ((wave + 1) * KT) / W;
+  // MX blocks b0 .. b1 - 1 in K tiles t0 .. t1 - 1; `first`: where the first tile begins, `last`: where the last one ends
+  const int b0 = KP == 1 ? 0 : kp * KT, b1 = KP == 1 ? 4 * KT : b0 + KT;
+  const int t0 = b0 >> 2, t1 = (b1 + 3) >> 2, first = b0 & 3, last = ((b1 - 1) & 3) + 1;
 
-  const i32x4* wq[NTW];
-  const i32x4* ws[NTW]; // E8M0 dwords of four channels
-#pragma unroll
-  for (int nt = 0; nt < NTW; nt++) {
-    const int64_t lt = min(ltile0 + nt, sg.tiles - 1); // ragged last group: duplicate, not stored
-    wq[nt] = reinterpret_cast<const i32x4*>(sg.qw) + lt * KT * 64;
-    ws[nt] = reinterpret_cast<const i32x4*>(sg.sw) + lt * KT * 4;
-  }
-  const i32x4* xop = reinterpret_cast<const i32x4*>(p.xq) + (int64_t)blockIdx.y * MG * 128;
-  const f32x4* sop = reinterpret_cast<const f32x4*>(p.sa) + (int64_t)blockIdx.y * MG * 16;
-  const int xstride = p.mt * 128, sstride = p.mt * 16;
+  const int64_t lt = min(ltile0 + tt, sg.tiles - 1); // ragged last group: duplicate, not stored
+  const i32x4* wq = reinterpret_cast<const i32x4*>(sg.qw) + lt * KT * 64;
+  const i32x4* ws = reinterpret_cast<const i32x4*>(sg.sw) + lt * KT * 4; // E8M0 dwords of four channels
+  const int rt0 = (int)blockIdx.y * (MG * R) + rr * MG; // first row tile of this wave
+  const i32x4* xop = reinterpret_cast<const i32x4*>(p.xq) + (int64_t)rt0 * 128;
+  const f32x4* sop = reinterpret_cast<const f32x4*>(p.sa) + (int64_t)rt0 * 16;
+  const int64_t xstride = p.mt * 128, sstride = p.mt * 16;
 
-  i32x4 wreg[PF][NTW], sreg[PF][NTW], xreg[PF][MG][2];
+  i32x4 wreg[PF], sreg[PF], xreg[PF][MG][2];
   f32x4 areg[PF][MG];
-  // (past the end, or a wave without tiles: re-read a valid tile that is never consumed -- no branch around a load)
-  auto load_w = [&](int st, int t) {
-    t = max(min(t, t1 - 1), 0);
-#pragma unroll
-    for (int nt = 0; nt < NTW; nt++) {
-      wreg[st][nt] = __builtin_nontemporal_load(wq[nt] + (int64_t)t * 64 + lane);
-      sreg[st][nt] = (ws[nt] + (int64_t)t * 4)[lane >> 4];
-    }
-  };
-  auto load_x = [&](int st, int t) {
-    t = max(min(t, t1 - 1), 0);
+  auto load = [&](int st, int t) {
+    t = min(t, t1 - 1); // (past the end: re-read a valid tile that is never consumed -- no branch around a load)
+    wreg[st] = R == 1 ? __builtin_nontemporal_load(wq + (int64_t)t * 64 + lane) : wq[(int64_t)t * 64 + lane];
+    sreg[st] = (ws + (int64_t)t * 4)[lane >> 4];
 #pragma unroll
     for (int mg = 0; mg < MG; mg++) {
-      xreg[st][mg][0] = (xop + (int64_t)t * xstride + mg * 128)[lane];
-      xreg[st][mg][1] = (xop + (int64_t)t * xstride + mg * 128 + 64)[lane];
-      areg[st][mg] = (sop + (int64_t)t * sstride + mg * 16)[lane & 15];
+      xreg[st][mg][0] = (xop + t * xstride + mg * 128)[lane];
+      xreg[st][mg][1] = (xop + t * xstride + mg * 128 + 64)[lane];
+      areg[st][mg] = (sop + t * sstride + mg * 16)[lane & 15];
     }
   };
 #pragma unroll
-  for (int i = 0; i < PF; i++) {
-    load_w(i, t0 + i);
-    load_x(i, t0 + i);
+  for (int i = 0; i < PF; i++)
+    load(i, t0 + i);
+  __builtin_amdgcn_sched_barrier(0);
+  SkEpilogue<MG * R, T, false, KP * T * R, KP * T * R> ep; // KP == 4
+  uint16_t in1[MG][4], in2[MG][4];                         // KP == 1
+  f32x4 facc[MG];
+#pragma unroll
+  for (int mg = 0; mg < MG; mg++)
+    facc[mg] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (KP == 1) {
+    // (an absent input is read from the output, as in SkEpilogue::prefetch_flat: no branch around a load)
+    const uint16_t* pb = sg.bias ? sg.bias : sg.y;
+    const uint16_t* p1 = sg.post_in ? sg.post_in : sg.y;
+    const uint16_t* p2 = sg.post_in2 ? sg.post_in2 : sg.y;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int n = (int)lt * 16 + (lane >> 4) * 4 + r;
+      const uint32_t b = pb[n];
+#pragma unroll
+      for (int mg = 0; mg < MG; mg++) {
+        const int o = min(m0 + (rr * MG + mg) * 16 + (lane & 15), p.M - 1) * sg.N + n;
+        in1[mg][r] = p1[o];
+        in2[mg][r] = p2[o];
+        facc[mg][r] = sg.bias ? bf16_bits_to_f32(b) : 0.f;
+      }
+    }
+  } else {
+    ep.prefetch_flat(p, sg, ltile0, m0);
   }
   __builtin_amdgcn_sched_barrier(0);
-  SkEpilogue<MG, NTW, false, W, W, true> ep;
-  ep.prefetch_flat(p, sg, ltile0, m0);
-  __builtin_amdgcn_sched_barrier(0);
 
-  f32x4 facc[NTW][MG];
+  auto block = [&](int i, auto J) {
+    constexpr int j = decltype(J)::value;
+    const uint32_t codes = (uint32_t)wreg[i][j];
+    const uint32_t lo = w4a8_expand(codes & 0x0F0F0F0Fu), hi = w4a8_expand((codes >> 4) & 0x0F0F0F0Fu);
+    const long wb = (long)(((uint64_t)hi << 32) | lo);
+    float wsc[4];
 #pragma unroll
-  for (int nt = 0; nt < NTW; nt++)
+    for (int r = 0; r < 4; r++)
+      wsc[r] = e8m0_to_f32((uint32_t)sreg[i][r] >> (8 * j));
 #pragma unroll
-    for (int mg = 0; mg < MG; mg++)
-      facc[nt][mg] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto consume = [&](int i) {
+    for (int mg = 0; mg < MG; mg++) {
+      const long xa = (long)(((uint64_t)(uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2 + 1] << 32) |
+                             (uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2]);
+      const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, xa, i32x4{0, 0, 0, 0}, 0, 0, 0);
+      const float sav = areg[i][mg][j];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-#pragma unroll
-      for (int nt = 0; nt < NTW; nt++) {
-        const uint32_t codes = (uint32_t)wreg[i][nt][j];
-        const uint32_t lo = w4a8_expand(codes & 0x0F0F0F0Fu), hi = w4a8_expand((codes >> 4) & 0x0F0F0F0Fu);
-        const long wb = (long)(((uint64_t)hi << 32) | lo);
-        float wsc[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          wsc[r] = e8m0_to_f32((uint32_t)sreg[i][nt][r] >> (8 * j));
-#pragma unroll
-        for (int mg = 0; mg < MG; mg++) {
-          const long xa = (long)(((uint64_t)(uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2 + 1] << 32) |
-                                 (uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2]);
-          const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, xa, i32x4{0, 0, 0, 0}, 0, 0, 0);
-          const float sav = areg[i][mg][j];
-#pragma unroll
-          for (int r = 0; r < 4; r++)
-            facc[nt][mg][r] = fmaf((float)acc[r], sav * wsc[r], facc[nt][mg][r]);
-        }
-      }
+      for (int r = 0; r < 4; r++)
+        facc[mg][r] = KP == 1 ? fmaf((float)acc[r] * wsc[r], sav, facc[mg][r])
+                              : fmaf((float)acc[r], sav * wsc[r], facc[mg][r]); // (the roundings of the kernel it equals)
+    }
+  };
+  auto consume = [&](int i, int t) {
+    const int lo = KP > 1 && t == t0 ? first : 0, hi = KP > 1 && t == t1 - 1 ? last : 4;
+    if (KP == 1 || (lo == 0 && hi == 4)) {
+      static_for<0, 4>([&](auto J) { block(i, J); });
+    } else {
+      static_for<0, 4>([&](auto J) {
+        if (decltype(J)::value >= lo && decltype(J)::value < hi)
+          block(i, J);
+      });
     }
   };
   int t = t0;
-  for (; t + PF <= t1; t += PF) { // branch-free full trips (reloads past the end are clamped re-reads)
+  for (; t + PF <= t1; t += PF) { // full trips (reloads past the end are clamped re-reads)
 #pragma unroll
     for (int i = 0; i < PF; i++) {
-      consume(i);
-      load_w(i, t + i + PF);
-      load_x(i, t + i + PF);
+      consume(i, t + i);
+      load(i, t + i + PF);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 #pragma unroll
   for (int i = 0; i < PF - 1; i++) // fewer than PF left: their tiles are in the stages a trip would use
     if (t + i < t1)
-      consume(i);
-  ep.finish(sg, facc, sk_lds);
+      consume(i, t + i);
+  if constexpr (KP == 1) {
+    if (ltile0 + tt >= sg.tiles)
+      return;
+#pragma unroll
+    for (int mg = 0; mg < MG; mg++) {
+      const int m = m0 + (rr * MG + mg) * 16 + (lane & 15);
+      if (m >= p.M)
+        continue;
+      uint32_t h[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        h[r] = apply_post_bits(facc[mg][r], sg.post_op, in1[mg][r], in2[mg][r], sg.post_scale) & 0xffffu;
+      *reinterpret_cast<uint2*>(sg.y + (int64_t)m * sg.N + lt * 16 + (lane >> 4) * 4) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    }
+  } else {
+    ep.template finish_parts<KP, MG>(sg, facc, sk_lds, kp, tt * (MG * R) + rr * MG);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2700,19 +2760,24 @@ hipError_t launch_skinny_w4a8(DecodeParams& p, int ntw, hipStream_t stream) {
   }
 }
 
-// W4A8, 17..64 rows per block row: mg = 2 / 4 row groups, ntw = 1..3 channel tiles per workgroup; p.mt, p.units, p.groups
-// set by the caller
-hipError_t launch_skinny_w4a8_mg(DecodeParams& p, int mg, int ntw, hipStream_t stream) {
-  if (p.S != 1 || p.mt <= 0 || (mg != 2 && mg != 4) || ntw < 1 || ntw > 3)
+// W4A8 between decode and the prompt passes; p.mt, p.units set by the caller
+template <int MG, int T, int R, int KP, int PF>
+static hipError_t sk_launch_w4a8_mg(DecodeParams& p, hipStream_t stream) {
+  const dim3 grid((p.total_tiles + T - 1) / T, (p.M + MG * R * 16 - 1) / (MG * R * 16), 1);
+  const size_t lds = KP == 1 ? 0 : (size_t)KP * T * MG * R * 256 * sizeof(float);
+  return sk_launch(skinny_w4a8_mg_kernel<MG, T, R, KP, PF>, p, grid, KP * T * R, lds, stream);
+}
+hipError_t launch_skinny_w4a8_mg(DecodeParams& p, bool ascending, hipStream_t stream) {
+  if (p.S != 1 || p.mt <= 0 || p.n_seg != 1)
     return hipErrorInvalidValue;
-  dim3 grid(p.groups, (p.M + mg * 16 - 1) / (mg * 16), 1);
-  const size_t lds = (size_t)8 * ntw * mg * 256 * sizeof(float);
-#define SKWM(MG, NTW)          \
-  if (mg == MG && ntw == NTW) \
-    return sk_launch(skinny_w4a8_mg_kernel<MG, NTW, 2>, p, grid, 8, lds, stream);
-  SKWM(2, 1) SKWM(2, 2) SKWM(2, 3) SKWM(4, 1) SKWM(4, 2) SKWM(4, 3)
-#undef SKWM
-  return hipErrorInvalidValue;
+  if (ascending) // one row tile per wave while that leaves at most one workgroup per CU, else two (the codes expanded
+                 // once for both): 4096 x 4096 at 64 rows (256 workgroups) 13.3 us against 18.8, at 128 rows 21.0 against 19.1
+    return p.total_tiles * ((p.M + 63) / 64) <= 256 ? sk_launch_w4a8_mg<1, 1, 4, 1, 2>(p, stream)
+                                                    : sk_launch_w4a8_mg<2, 2, 2, 1, 2>(p, stream);
+  // one channel tile per workgroup: more of them lose except at 11008 x 4096, 32 rows (three: 14.0 us against 14.2)
+  if (p.M <= 16)
+    return sk_launch_w4a8_mg<1, 1, 1, 4, 4>(p, stream);
+  return p.M <= 32 ? sk_launch_w4a8_mg<2, 1, 1, 4, 2>(p, stream) : sk_launch_w4a8_mg<2, 1, 2, 4, 2>(p, stream);
 }
 
 // MXFP4, 33..64 rows per block row: four channel tiles x four K parts per workgroup, K in p.S slices across workgroups

@@ -649,13 +649,12 @@ W4A8_DECODE = os.environ.get("TPPX_W4A8_DECODE", "1") == "1"
 W4A8_WIDE_ROWS = int(os.environ.get("TPPX_W4A8_WIDE_ROWS", "64"))
 
 
-def _w4a8_block_rows(M, N, K):
-    """Does a W4A8 call of 17 or more rows run as block rows of 64 on the row-group kernel (which streams the 4-bit
+def _w4a8_row_groups(M, N, K):
+    """Does a W4A8 call of 64 or more rows run as block rows of 64 on the row-group kernel (which streams the 4-bit
     weights once per block row) rather than on the prompt kernel (2 bytes per weight, all of K per workgroup)?
+    The same bits either way.
     Fits in us, measured with the activation quantizer included: a block row 19 / 20 / 11 at 11008 x 4096,
     4096 x 11008 and 4096 x 4096; the prompt kernel 45 / 92 / 36 up to one workgroup of 64 x 128 per CU."""
-    if M < W4A8_WIDE_ROWS:
-        return True
     rows64 = (M + 63) // 64
     wgs = rows64 * ((N + 127) // 128)
     return rows64 * (7.2 + N * K / 4.0e6) < (3.0 + K * 0.0081) * max(1.0, wgs / 220)
@@ -681,34 +680,38 @@ def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=
     bias = _prep_bias(bias, N, x.device)
     post_in = _prep_post(post_in, M, N, "post-op input", x.device)
     post_in2 = _prep_post(post_in2, M, N, "second post-op input", x.device)
-    # decode steps: one launch that quantizes its rows itself and splits K over the waves of a workgroup
-    # (TPPX_W4A8_DECODE=0 keeps the two-step path)
-    nat = weight.native_w4a8() if _w4a8_block_rows(M, N, K) else None
+    # Fewer than 64 rows: the tiles of tppx_prepack_mxfp4_int8, in one launch that quantizes its rows itself (up to 16),
+    # else behind a launch that writes the rows in operand order.  The second form has the bits of the two-step path at
+    # the end, which takes what is left.
+    # From TPPX_W4A8_WIDE_ROWS rows: K in one ascending sum per output, by the prompt kernel (its weights are a second
+    # copy, 2 bytes per value) or, with the same bits, by row groups on the 4-bit tiles.
+    wide_rows = M >= W4A8_WIDE_ROWS
+    nat = None
+    if (M >= 64 and _w4a8_row_groups(M, N, K)) if wide_rows else M < 64:
+        nat = weight.native_w4a8()
     if nat is not None and M <= 16 and W4A8_DECODE:
         rc = L.tppx_linear_mxfp4_int8_rows(x.data_ptr(), nat[0].data_ptr(), nat[1].data_ptr(), _lib.ptr(bias),
                                            _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N, K, post, post_scale,
                                            _lib.stream_of(x))
-        if rc != _lib.EUNSUPPORTED:  # rows that do not fit the kernel's LDS take the two-step path
+        if rc != _lib.EUNSUPPORTED:  # rows that do not fit the kernel's LDS
             _lib.check(rc)
             return y
-    # up to the prompt passes: rows quantized into operand order by a launch of their own, then the row-group kernel
     if nat is not None:
-        flags = _lib.FLAG_XQ_REUSE if rows else 0
-        if not rows:
-            mp = (M + 63) // 64 * 64
-            buf = torch.empty(mp * K + mp * (K // 8), dtype=torch.uint8, device=x.device)
-            held = (buf, buf.data_ptr(), buf.data_ptr() + mp * K)
-            if rows is not None:
-                rows.append(held)
+        if rows:
+            held, flags = rows[0], _lib.FLAG_XQ_REUSE
         else:
-            held = rows[0]
-        _lib.check(L.tppx_linear_mxfp4_int8_mid(x.data_ptr(), held[1], held[2], nat[0].data_ptr(), nat[1].data_ptr(),
-                                                _lib.ptr(bias), _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N,
-                                                K, post, post_scale, flags, _lib.stream_of(x)))
-        return y
-    # prompt passes: rows and weights as bf16-coded integers on the bf16 MFMA, one fp32 multiply-add per block
-    # (TPPX_W4A8_WIDE_ROWS: from how many rows; the weight keeps a second, 2-byte-per-value copy for it)
-    wide = weight.native_w4a8_wide() if nat is None and M >= W4A8_WIDE_ROWS else None
+            mp = (M + 63) // 64 * 64
+            held, flags = torch.empty(mp * K + mp * (K // 8), dtype=torch.uint8, device=x.device), 0
+        rc = L.tppx_linear_mxfp4_int8_mid(x.data_ptr(), held.data_ptr(), held.data_ptr() + (M + 63) // 64 * 64 * K,
+                                          nat[0].data_ptr(), nat[1].data_ptr(), _lib.ptr(bias), _lib.ptr(post_in),
+                                          _lib.ptr(post_in2), y.data_ptr(), M, N, K, post, post_scale, flags,
+                                          _lib.stream_of(x))
+        if rc != _lib.EUNSUPPORTED:
+            _lib.check(rc)
+            if rows is not None and not rows:
+                rows.append(held)
+            return y
+    wide = weight.native_w4a8_wide() if wide_rows else None
     if wide is not None:
         mp = (M + 127) // 128 * 128
         ws = torch.empty(mp * K * 2 + mp * (K // 32) * 4, dtype=torch.uint8, device=x.device)

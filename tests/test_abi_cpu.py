@@ -419,3 +419,16 @@ def test_cache_allocates_small_layers_together():
     big.SLAB_BYTES = 4 * 2 * 4 * 48 * 16                            # room for one layer only
     a, b = big._ensure(0, 2, 4, 16, "cpu"), big._ensure(1, 2, 4, 16, "cpu")
     assert a[0].untyped_storage().data_ptr() != b[0].untyped_storage().data_ptr() and not big._spare
+
+
+def test_w4a8_prompts_take_the_prompt_kernel():
+    """W4A8 calls from 64 rows on: row groups stream the 4-bit weights once per 64 rows, so they are for few rows only.
+    Long prompts run on the prompt kernel whatever the weight (2048 rows of 28672 x 8192: 1250 us there, 2260 in row
+    groups)."""
+    from tpp_pytorch_extension import _ops
+
+    shapes = [(28672, 8192), (8192, 28672), (22016, 8192), (8192, 8192), (11008, 4096), (4096, 11008), (4096, 4096), (3584, 18944)]
+    for n, k in shapes:
+        assert _ops._w4a8_row_groups(64, n, k), (n, k)
+        for m in (1024, 1536, 2048, 4096, 16384):
+            assert not _ops._w4a8_row_groups(m, n, k), (m, n, k)

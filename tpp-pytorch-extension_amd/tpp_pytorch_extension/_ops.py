@@ -650,14 +650,25 @@ W4A8_WIDE_ROWS = int(os.environ.get("TPPX_W4A8_WIDE_ROWS", "64"))
 
 
 def _w4a8_row_groups(M, N, K):
-    """Does a W4A8 call of 64 or more rows run as block rows of 64 on the row-group kernel (which streams the 4-bit
-    weights once per block row) rather than on the prompt kernel (2 bytes per weight, all of K per workgroup)?
-    The same bits either way.
-    Fits in us, measured with the activation quantizer included: a block row 19 / 20 / 11 at 11008 x 4096,
-    4096 x 11008 and 4096 x 4096; the prompt kernel 45 / 92 / 36 up to one workgroup of 64 x 128 per CU."""
+    """Does a W4A8 call of 64 or more rows run on the row-group kernel (4-bit weights, once per 64 rows) rather than on
+    the prompt kernel (2 bytes per weight)?  The same bits either way.  Both in us, the row quantizer included, fitted
+    to 64 .. 2048 rows of fifteen shapes from 64 x 4096 to 28672 x 8192 (the choice is within 8 % of the faster one
+    down to K = 2304): row groups by rounds of 256 workgroups of 64 rows x 32 channels (16 channels while those are one
+    round); the prompt kernel by its workgroups of 64 x 128, one or two per CU, and beyond 256 of 128 x 128, two per CU,
+    by rounds of 512 of those, the last one rarely full.  7B shapes hand over at about 200 (11008 x 4096) to 300 rows,
+    28672 x 8192 at 128: 2048 rows there take 1250 us on the prompt kernel, 2260 in row groups."""
     rows64 = (M + 63) // 64
-    wgs = rows64 * ((N + 127) // 128)
-    return rows64 * (7.2 + N * K / 4.0e6) < (3.0 + K * 0.0081) * max(1.0, wgs / 220)
+    if rows64 * (N // 16) <= 256:
+        groups = 2.0 + 0.00272 * K
+    else:
+        rounds = (rows64 * ((N + 31) // 32) + 255) // 256
+        groups = 3.0 + 0.00376 * K if rounds == 1 else 4.3 + 0.00516 * K + (rounds - 2) * (0.4 + 0.00227 * K)
+    wgs = (M + 127) // 128 * ((N + 127) // 128)
+    if wgs <= 256:
+        prompt = (5.0 + 0.0072 * K + N * K / 4.5e6) * (1.0 if wgs <= 128 else 1.45)
+    else:
+        prompt = (1.0 if wgs <= 512 else 0.8 * ((wgs + 511) // 512)) * (12.0 + 0.0205 * K)
+    return groups + 3.0 + M * K * 1.5e-6 < prompt
 
 
 def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=None):

@@ -622,3 +622,25 @@ def test_w4a8_row_groups_equal_the_oracle_from_64_rows(M, N, K, bc, post):
                                                       ws.numel(), _lib.stream_of(xg)))
     assert torch.equal(_w4a8_mid(qt, xg, bg, posts[post], in1, in2, 0.5), want)
     assert torch.equal(ops.linear(xg, qt, bg, posts[post], in1, in2, 0.5), want)
+
+
+@pytest.mark.parametrize("off", [1, 4])
+@pytest.mark.parametrize("M", [17, 40, 63])
+def test_w4a8_takes_rows_at_any_address(M, off):
+    """17 to 63 activation rows that do not begin on a 16-byte address (a contiguous view into a larger buffer), with
+    post-op inputs and a bias off one too: the same bits as from aligned memory, for a linear and the gate/up pair."""
+    ops = _ops()
+    N, K = 96, 640
+    qt = _w4a8(N, K, 64, 3400)[0]
+
+    def moved(t):
+        buf = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)
+        buf[off:off + t.numel()] = t.reshape(-1)
+        return buf[off:off + t.numel()].view(t.shape)
+
+    x, b, r = randn_bf16((M, K), 1.0, 3410).cuda(), randn_bf16((N,), 0.1, 3420).cuda(), randn_bf16((M, N), 1.0, 3430).cuda()
+    xm = moved(x)
+    assert xm.data_ptr() % 16 == 2 * off
+    assert torch.equal(ops.linear(xm, qt, moved(b), O.POST_ADD_SCALE, moved(r), None, 0.5),
+                       ops.linear(x, qt, b, O.POST_ADD_SCALE, r, None, 0.5))
+    assert torch.equal(ops.swiglu_gate_up(xm, qt, qt), ops.swiglu_gate_up(x, qt, qt))

@@ -693,7 +693,7 @@ def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=
     post_in2 = _prep_post(post_in2, M, N, "second post-op input", x.device)
     # Fewer than 64 rows: the tiles of tppx_prepack_mxfp4_int8, in one launch that quantizes its rows itself (up to 16),
     # else behind a launch that writes the rows in operand order.  The second form has the bits of the two-step path at
-    # the end, which takes what is left.
+    # the end, which takes what is left: other K, rows off a 16-byte address.
     # From TPPX_W4A8_WIDE_ROWS rows: K in one ascending sum per output, by the prompt kernel (its weights are a second
     # copy, 2 bytes per value) or, with the same bits, by row groups on the 4-bit tiles.
     wide_rows = M >= W4A8_WIDE_ROWS
@@ -707,7 +707,7 @@ def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=
         if rc != _lib.EUNSUPPORTED:  # rows that do not fit the kernel's LDS
             _lib.check(rc)
             return y
-    if nat is not None:
+    if nat is not None and x.data_ptr() % 16 == 0:
         if rows:
             held, flags = rows[0], _lib.FLAG_XQ_REUSE
         else:

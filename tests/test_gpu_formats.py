@@ -377,6 +377,7 @@ def test_w4a8_wide_kernel(M, N, K, bc, post, monkeypatch):
     r = randn_bf16((M, N), 1.0, 2830)
     r2 = randn_bf16((M, N), 1.0, 2840) if post == "add2" else None
     assert M >= ops.W4A8_WIDE_ROWS and qt.native_w4a8_wide() is not None
+    monkeypatch.setattr(ops, "_w4a8_row_groups", lambda *a: False)  # (some of these shapes are few rows' work)
     # the GEMM alone: equal to the oracle
     y0 = ops.linear(x.cuda(), qt, b.cuda(), O.POST_NONE, None, None, 1.0)
     pre = O.linear_w4a8(t2bits(x), q_or, s_or, bc, t2bits(b))
@@ -387,9 +388,10 @@ def test_w4a8_wide_kernel(M, N, K, bc, post, monkeypatch):
     # without a bias, and against the simple kernel below the threshold (the same sums in another order)
     y1 = ops.linear(x.cuda(), qt, None, O.POST_NONE, None, None, 1.0)
     assert np.array_equal(t2bits(y1), O.linear_w4a8(t2bits(x), q_or, s_or, bc, None))
-    monkeypatch.setattr(ops, "W4A8_WIDE_ROWS", 1 << 30)
-    y2 = ops.linear(x.cuda(), qt, b.cuda(), O.POST_NONE, None, None, 1.0)
+    y2 = _w4a8_two_steps(qt, x.cuda(), b.cuda(), O.POST_NONE, None, None, 1.0)
     assert_close_bf16(t2bits(y2), pre, ulps=1, what="simple kernel")
+    monkeypatch.setattr(ops, "W4A8_WIDE_ROWS", 1 << 30)  # below the threshold the operator takes that one
+    assert torch.equal(ops.linear(x.cuda(), qt, b.cuda(), O.POST_NONE, None, None, 1.0), y2)
     # the entry point rejects a workspace that is too small, and misaligned outputs
     L = _lib.lib()
     out = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
@@ -420,8 +422,8 @@ def test_w4a8_decode_kernel(M, N, K, bc, post, monkeypatch):
     """W4A8 decode calls (TppBlockedLinearW<int8_t, uint8_t, Tout>, src/csrc/fused_gemm.h:965-978, at most 16 rows) in
     one launch: rows quantized to int8 over blocks of 32 inside the kernel, K split over the waves of a workgroup,
     weights from tiles made once by tppx_prepack_mxfp4_int8.  Within 1 bf16 ulp (2 through SiLU) of the oracle's
-    restatement and of the two-step path (the same integer sums and per-block fp32 multiply-adds in another order);
-    16 rows x 11008 do not fit the kernel's LDS and take the two-step path by themselves."""
+    restatement and of the two-step path (the same integer sums and per-block fp32 multiply-adds in another order;
+    TPPX_W4A8_DECODE=0); 16 rows x 11008 do not fit the kernel's LDS and take row groups, with the bits of that path."""
     ops = _ops()
     from tpp_pytorch_extension import _lib
     posts = {"none": O.POST_NONE, "add": O.POST_ADD_SCALE, "silu": O.POST_SILU, "mul": O.POST_MUL}
@@ -449,6 +451,7 @@ def test_w4a8_decode_kernel(M, N, K, bc, post, monkeypatch):
     assert_close_bf16(t2bits(y), ref, ulps=2 if post == "silu" else 1, what=f"w4a8 decode M={M} N={N} K={K} {post}", pre_bits=pre)
     monkeypatch.setattr(ops, "W4A8_DECODE", False)
     y2 = ops.linear(x.cuda(), qt, b.cuda(), posts[post], r.cuda(), None, 0.5)
+    assert torch.equal(y2, _w4a8_two_steps(qt, x.cuda(), b.cuda(), posts[post], r.cuda(), None, 0.5))
     assert_close_bf16(t2bits(y), t2bits(y2), ulps=2 if post == "silu" else 1, what="one launch vs quantizer + GEMM", pre_bits=pre)
     if not fits:
         assert torch.equal(y, y2)
@@ -531,6 +534,47 @@ def test_w4a8_row_group_kernel(M, N, K, bc, post):
     assert_close_bf16(t2bits(y), ref, ulps=2 if post == "silu" else 1, what=f"w4a8 rows M={M} N={N} K={K} {post}", pre_bits=pre)
     assert torch.equal(ops.swiglu_gate_up(x.cuda(), qt, qt, b.cuda(), b.cuda()),
                        ops.fc_mul(x.cuda(), qt, b.cuda(), ops.fc_silu(x.cuda(), qt, b.cuda())))
+
+
+@pytest.mark.parametrize("M,N,K,bc,post", [(1, 96, 192, 64, "none"), (17, 272, 320, 64, "add"), (64, 144, 1056, 32, "silu"), (200, 80, 96, 32, "mul")])
+def test_w4a8_linear_kernel_of_odd_widths(M, N, K, bc, post):
+    """K no multiple of 128 runs on the quantizer and linear_w4a8_kernel whatever the rows: within 1 bf16 ulp (2 through
+    SiLU) of the oracle, which adds the same exact block products in K order."""
+    ops = _ops()
+    posts = {"none": O.POST_NONE, "add": O.POST_ADD_SCALE, "silu": O.POST_SILU, "mul": O.POST_MUL}
+    qt, t = _w4a8(N, K, bc, 3500 + M)
+    assert qt.native_w4a8() is None and qt.native_w4a8_wide() is None
+    q_or, s_or = O.remap_quantize_mxfp4_int8(t.float().numpy())
+    x, b, r = randn_bf16((M, K), 1.0, 3510 + M), randn_bf16((N,), 0.1, 3520), randn_bf16((M, N), 1.0, 3530)
+    x[M - 1, :64] = 0.0
+    in1 = r.cuda() if post in ("add", "mul") else None
+    y = ops.linear(x.cuda(), qt, b.cuda(), posts[post], in1, None, 0.5)
+    assert torch.equal(y, _w4a8_two_steps(qt, x.cuda(), b.cuda(), posts[post], in1, None, 0.5))
+    ref = O.linear_w4a8(t2bits(x), q_or, s_or, bc, t2bits(b), posts[post], t2bits(r), None, 0.5)
+    pre = O.linear_w4a8(t2bits(x), q_or, s_or, bc, t2bits(b)) if post in ("add", "mul") else None
+    assert_close_bf16(t2bits(y), ref, ulps=2 if post == "silu" else 1, what=f"w4a8 M={M} N={N} K={K} {post}", pre_bits=pre)
+
+
+@pytest.mark.parametrize("M", [4, 17, 63])
+def test_w4a8_switch_keeps_the_two_step_path(M, monkeypatch):
+    """TPPX_W4A8_DECODE=0: calls below TPPX_W4A8_WIDE_ROWS rows run the quantizer and linear_w4a8_kernel, and no other
+    W4A8 entry point is called (nor are its weights made)."""
+    ops = _ops()
+    from tpp_pytorch_extension import _lib
+    qt = _w4a8(96, 256, 64, 3600)[0]
+    x = randn_bf16((M, 256), 1.0, 3610).cuda()
+    want = _w4a8_two_steps(qt, x, None, O.POST_NONE, None, None, 1.0)
+
+    class Only:
+        def __getattr__(self, name):
+            assert name not in ("tppx_linear_mxfp4_int8_rows", "tppx_linear_mxfp4_int8_mid", "tppx_linear_mxfp4_int8_wide",
+                                "tppx_prepack_mxfp4_int8", "tppx_prepack_mxfp4_int8_wide"), name
+            return getattr(lib, name)
+
+    lib = _lib.lib()
+    monkeypatch.setattr(ops, "W4A8_DECODE", False)
+    monkeypatch.setattr(_lib, "lib", lambda: Only())
+    assert torch.equal(ops.linear(x, qt, None), want)
 
 
 def _w4a8(N, K, bc, seed):

@@ -693,14 +693,14 @@ def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=
     post_in2 = _prep_post(post_in2, M, N, "second post-op input", x.device)
     # Fewer than 64 rows: the tiles of tppx_prepack_mxfp4_int8, in one launch that quantizes its rows itself (up to 16),
     # else behind a launch that writes the rows in operand order.  The second form has the bits of the two-step path at
-    # the end, which takes what is left: other K, rows off a 16-byte address.
+    # the end, which takes what is left: TPPX_W4A8_DECODE=0, other K, rows off a 16-byte address.
     # From TPPX_W4A8_WIDE_ROWS rows: K in one ascending sum per output, by the prompt kernel (its weights are a second
     # copy, 2 bytes per value) or, with the same bits, by row groups on the 4-bit tiles.
     wide_rows = M >= W4A8_WIDE_ROWS
     nat = None
-    if (M >= 64 and _w4a8_row_groups(M, N, K)) if wide_rows else M < 64:
+    if (M >= 64 and _w4a8_row_groups(M, N, K)) if wide_rows else (M < 64 and W4A8_DECODE):
         nat = weight.native_w4a8()
-    if nat is not None and M <= 16 and W4A8_DECODE:
+    if nat is not None and M <= 16:
         rc = L.tppx_linear_mxfp4_int8_rows(x.data_ptr(), nat[0].data_ptr(), nat[1].data_ptr(), _lib.ptr(bias),
                                            _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N, K, post, post_scale,
                                            _lib.stream_of(x))

@@ -963,3 +963,15 @@ def test_prefill_qint8_pair_agrees_with_two_launches(fmt, M, N, K, monkeypatch):
         m.setattr(ops, "fc_silu", None)  # (the two launches would call it)
         got = ops.swiglu_gate_up(x, ws[0], ws[1], b, None)
     assert torch.equal(got, ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], b)))
+
+
+def test_prefill_qint8_pair_of_2_31_outputs():
+    """The QINT8 gate/up pair with more than 2^31 outputs (64-bit output offsets in the large-M kernels): one launch as
+    for fewer, the bits of fc_silu followed by fc_mul."""
+    ops = _ops()
+    M, N, K = 32800, 65536, 256
+    assert M * N >= 1 << 31
+    ws = [ops.remap_and_quantize_qint8(block_bf16(randn_bf16((N, K), 0.05, 770 + i)).cuda()) for i in range(2)]
+    x = randn_bf16((M, K), 1.0, 772).cuda()
+    got = ops.swiglu_gate_up(x, ws[0], ws[1])
+    assert torch.equal(got, ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], None)))

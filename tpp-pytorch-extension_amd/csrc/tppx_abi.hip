@@ -773,7 +773,6 @@ extern "C" int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* 
                                  const void* bias_gate, const void* qw_up, const void* sw_up, const void* bias_up, void* y,
                                  int64_t M, int64_t N, int64_t K, int64_t qbs, int flags, tppx_stream_t stream) {
   const char* who = "tppx_swiglu_qint8";
-  TPPX_REQUIRE(M <= 0 || N < ((int64_t)1 << 31) / M, TPPX_ESHAPE, "%s: M*N outputs exceed 2^31", who);
   tppx_seg s[2] = {{qw_gate, sw_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
                    {qw_up, sw_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
   return run_qint8(who, x, xq, sa, s, 2, M, K, qbs, flags, nullptr, 0, (hipStream_t)stream, true);

@@ -68,6 +68,11 @@ def test_argument_validation_without_gpu():
     assert lib.tppx_linear_bf16(A, None, None, None, None, A, 1, 16, 128, 0, 1.0, 0, None) == L.EINVAL
     assert lib.tppx_prepack_bf16(A, 32, 256, 16, 48, 2, A, None) == L.ESHAPE
     assert lib.tppx_prepack_bf16(A, 32, 256, 16, 64, 3, A, None) == L.ESHAPE
+    # W4A8 row groups: scales are read 16 bytes at a time; what does not fit the kernel's offsets is left to others
+    mid = lambda s, M=32, N=32, K=128: lib.tppx_linear_mxfp4_int8_mid(A, A, A, A, s, None, None, None, A, M, N, K, 0, 1.0, 0, None)  # noqa: E731
+    assert mid(A + 4) == L.EINVAL and "aligned" in err()
+    assert mid(A, M=64, N=1 << 25) == L.EUNSUPPORTED and mid(A, K=65536 * 128) == L.EUNSUPPORTED
+    assert mid(A, M=0) == L.ESHAPE and mid(A, K=192) == L.ESHAPE
     # post-op id and its inputs
     assert lib.tppx_linear_mxfp4(A, A, A, None, None, None, A, 1, 32, 128, 9, 1.0, 0, None, 0, None) == L.EINVAL
     assert lib.tppx_linear_mxfp4(A, A, A, None, None, None, A, 1, 32, 128, L.POST_MUL, 1.0, 0, None, 0, None) == L.EINVAL

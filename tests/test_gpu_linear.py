@@ -975,3 +975,29 @@ def test_prefill_qint8_pair_of_2_31_outputs():
     x = randn_bf16((M, K), 1.0, 772).cuda()
     got = ops.swiglu_gate_up(x, ws[0], ws[1])
     assert torch.equal(got, ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], None)))
+
+
+@pytest.mark.parametrize("off", [1, 2])
+@pytest.mark.parametrize("M,N,K", [(70, 544, 256), (200, 1056, 640), (300, 96, 1280)])
+def test_prefill_mxfp4_takes_scales_at_any_address(off, M, N, K, monkeypatch):
+    """Native scale bytes off a 4-byte address (a view into a packed buffer): the bits of aligned ones, for a linear,
+    fused q/k/v and the gate/up pair, whichever workgroup tile is asked for."""
+    ops = _ops()
+    ws = [_make("mxfp4", N, K, 780 + i)[0] for i in range(3)]
+    x = randn_bf16((M, K), 1.0, 785).cuda()
+
+    def run():
+        return [ops.fc_plain(x, ws[0], None)] + list(ops.qkv_gemm(x, ws, [None] * 3)) + [ops.swiglu_gate_up(x, ws[0], ws[1])]
+
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
+    want = run()
+    for w in ws:
+        qn, sn = w.native()
+        buf = torch.empty(sn.numel() + 16, dtype=sn.dtype, device=sn.device)
+        buf[off:off + sn.numel()] = sn.reshape(-1)
+        w._native = (qn, buf[off:off + sn.numel()].view(sn.shape))
+        assert w._native[1].data_ptr() % 4 == off
+    for tile in ("0", "2", "4", "5"):
+        monkeypatch.setenv("TPPX_TILED_BIG_TILE", tile)
+        for a, b in zip(run(), want):
+            assert torch.equal(a, b), tile

@@ -1582,9 +1582,13 @@ static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int 
 hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
+  // the ring moves scale bytes four at a time: scales off a 4-byte address keep to the forms that read them one by one
+  bool ring = true;
+  for (int i = 0; i < n; i++)
+    ring = ring && (reinterpret_cast<uintptr_t>(t[i].sw) & 3u) == 0;
   int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
-  if (shape < 0 || shape >= N_TILES)
-    shape = cheapest_tile(t, n, dual, env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128, tile_us);
+  if (shape < 0 || shape >= (ring ? N_TILES : TILE_64_128))
+    shape = cheapest_tile(t, n, dual, ring && env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128, tile_us);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 0.53);
   switch (shape) {
@@ -1597,7 +1601,7 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
   case TILE_128_256:
     // at most one workgroup per CU: eight waves of 64 x 64, two per SIMD, so that one wave's waits are another's issue
     // slots; else four of 128 x 64, two workgroups per CU
-    if (wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0)
+    if (ring && wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0)
       return dual ? big_launch<4, true, 2, 4>(P, wgs, stream) : big_launch<4, false, 2, 4>(P, wgs, stream);
     return dual ? big_launch<8, true, 1, 4>(P, wgs, stream) : big_launch<8, false, 1, 4>(P, wgs, stream);
   default:

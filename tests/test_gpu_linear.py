@@ -947,6 +947,43 @@ def test_prefill_bf16_groups_agree_with_single_launches(M, shape, monkeypatch):
     assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws, bs), got))
 
 
+@pytest.mark.parametrize("tile,w8", [(1, 1), (2, 1), (2, 0), (3, 1), (4, 1)])
+@pytest.mark.parametrize("M,N,K", [(65, 160, 128), (129, 544, 256), (300, 544, 384), (200, 1056, 640)])
+def test_prefill_bf16_every_workgroup_tile_ragged(tile, w8, M, N, K, monkeypatch):
+    """Every workgroup tile for unquantized bf16 weights (256 x 256, 128 x 256 with eight and with four waves, 128 x 512,
+    64 x 128), forced: a single GEMM, q/k/v with the fourth GEMM's GELU, and the gate/up pair, over one, an even and an
+    odd number of K steps, rows and channel blocks ragged.  Same sums in the same order in every tile, hence the bits of
+    the 64 x 128 one, which are checked against a float64 product (bf16 rounding of the result)."""
+    ops = _ops()
+    widths = (N, 64, 96, 160)
+    flat = [randn_bf16((n, K), 0.05, 780 + i) for i, n in enumerate(widths + (N,))]
+    ws = [block_bf16(w).cuda() for w in flat]
+    bs = [randn_bf16((N,), 0.5, 786).cuda(), None, None, randn_bf16((160,), 0.5, 787).cuda()]
+    x = randn_bf16((M, K), 1.0, 788).cuda()
+
+    def run():
+        group = ops._bf16_group(x, ws[:4], bs)
+        pair = ops._bf16_group(x, [ws[0], ws[4]], [bs[0], None], pair=True)
+        assert group is not None and pair is not None
+        return [ops.linear(x, ws[0], bs[0]), pair] + list(group)
+
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
+    monkeypatch.setenv("TPPX_TILED_W8", str(w8))
+    monkeypatch.setenv("TPPX_TILED_BIG_TILE", str(tile))
+    got = run()
+    monkeypatch.setenv("TPPX_TILED_BIG_TILE", "4")
+    want = run()
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), i
+    for i, (w, b) in enumerate(zip(flat[:3], bs[:3])):
+        ref = x.double() @ w.cuda().double().t() + (b.double() if b is not None else 0.0)
+        assert ((got[2 + i].double() - ref).norm() / ref.norm()).item() < 2.0 ** -8, i
+    assert torch.equal(got[0], got[2])
+    assert torch.equal(got[1], ops.fc_mul(x, ws[4], None, ops.fc_silu(x, ws[0], bs[0])))
+    assert torch.equal(got[5], ops.linear(x, ws[3], bs[3], O.POST_GELU))
+    assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws[:4], bs), got[2:]))
+
+
 @pytest.mark.parametrize("fmt", ["qint8", "qint4"])
 @pytest.mark.parametrize("M,N,K", [(65, 160, 256), (129, 544, 512), (300, 96, 768), (200, 2080, 1280), (1000, 4160, 512)])
 def test_prefill_qint8_pair_agrees_with_two_launches(fmt, M, N, K, monkeypatch):

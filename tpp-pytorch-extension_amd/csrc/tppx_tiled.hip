@@ -1716,12 +1716,14 @@ bool tiled_bf16_takes_groups(const TiledParams& p) {
          (int64_t)p.tiles * 32 * p.K < ((int64_t)1 << 32);
 }
 
-// n GEMMs over one activation in one launch (fuller last rounds: q/k/v of 4096 channels at 2048 rows 202 -> 157 us), or
-// the gate/up pair (dual, as launch_tiled_mxfp4_group: 11008 x 4096 at 2048 rows 359 -> 300 us, 333 rows 128 -> 93)
+// n GEMMs over one activation in one launch (fuller last rounds: q/k/v of 4096 channels at 2048 rows 207 -> 167 us), or
+// the gate/up pair (dual, as launch_tiled_mxfp4_group: 11008 x 4096 at 2048 rows 355 -> 310 us, 333 rows 148 -> 96)
 hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
-  const int shape = cheapest_tile(t, n, dual, env_int("TPPX_TILED_SMALL", 1) != 0 ? TILE_128_128 : TILE_64_128, tile_bf16_us);
+  int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 .. 4 as in launch_tiled_mxfp4_group; 5 is not built for 2-byte weights
+  if (shape < 0 || shape >= TILE_128_128)
+    shape = cheapest_tile(t, n, dual, env_int("TPPX_TILED_SMALL", 1) != 0 ? TILE_128_128 : TILE_64_128, tile_bf16_us);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 2.0);
   switch (shape) {

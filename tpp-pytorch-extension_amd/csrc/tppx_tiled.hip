@@ -1687,7 +1687,8 @@ silu_mul_kernel(const uint16_t* __restrict__ gate, uint16_t* __restrict__ y, int
 
 // The same estimate for unquantized bf16 weights (four times the weight bytes of a step: what a CU takes in bounds the
 // small tiles; K = 4096 / 11008, one launch: 64 x 128 29 / 60 us, 128 x 256 51 / 116, 256 x 256 85 / 193, 128 x 512
-// 83 / 190; 64 x 128 doubles from 257 workgroups, 128 x 256 takes 95 us for 384 and 158 for 768).
+// 83 / 190; 64 x 128 doubles from 257 workgroups; 128 x 256 at K = 4096: 66 us for 256 workgroups, 91 for 258, 96 for
+// 344, 103 for 430, 110 for 480, 146 for 516, 156 for 645, 168 for 768, 225 for 1000).
 static double tile_bf16_us(int tile, int64_t wgs, double steps) {
   const double rounds = (double)((wgs + 255) / 256);
   switch (tile) {
@@ -1696,7 +1697,8 @@ static double tile_bf16_us(int tile, int64_t wgs, double steps) {
   case TILE_128_512:
     return (20.0 + 2.05 * steps) * rounds;
   case TILE_128_256:
-    return wgs <= 256 ? 14.0 + 1.2 * steps : wgs <= 400 ? 22.0 + 2.3 * steps : (30.0 + 2.5 * steps) * std::max(1.0, (double)wgs / 512.0);
+    return wgs <= 256 ? 14.0 + 1.2 * steps
+                      : (30.0 + 2.5 * steps) * (wgs <= 512 ? 0.64 + 0.36 * (double)wgs / 512.0 : (double)wgs / 512.0);
   default:
     return wgs <= 256 ? 11.0 + 0.6 * steps : wgs <= 512 ? 8.0 + 1.38 * steps : (10.0 + 1.5 * steps) * (double)wgs / 512.0;
   }

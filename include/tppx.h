@@ -425,6 +425,13 @@ int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* qw_gate,
                       const void* bias_up, void* y, int64_t M, int64_t N,
                       int64_t K, int64_t qbs, int flags, tppx_stream_t stream);
 
+/* 1 where the three calls above run n_segs weights of Ns[i] x K (weight_bytes 2:
+ * bf16; 1: QINT8 in blocks of 256) over M rows as one launch, 0 where they
+ * answer TPPX_EUNSUPPORTED or refuse the shape: a caller asks before it
+ * prepares buffers for them. */
+int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M,
+                             int64_t K, int weight_bytes);
+
 /* llama_rms_norm followed by the GEMMs that consume it, in ONE launch, for
  * decode steps (M <= 16): the two calls
  *   t_HS = llama_rms_norm(t_HS, gamma, eps); fused_qkv_gemm(t_HS, {Wq,Wk,Wv}, ...)

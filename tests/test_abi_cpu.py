@@ -295,6 +295,25 @@ def test_launch_plans_of_per_output_channel_qint8():
     assert len(odd) == 2 and "quant_act_int8_kernel" in odd[0] and "skinny_qint8_kernel<1, 1, 4, 16, 4, true>" in odd[1], odd
 
 
+def test_group_is_one_launch():
+    """Which groups the large-M launches take, by sizes alone: rows, blocks of whole tiles, operands below 4 GiB."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+
+    def one(Ns, M, K, weight_bytes):
+        return L.tppx_group_is_one_launch((ctypes.c_int64 * len(Ns))(*Ns), len(Ns), M, K, weight_bytes)
+
+    for bytes_per in (1, 2):
+        assert one([11008] * 2, 333, 4096, bytes_per) == 1 and one([4096, 1024, 1024], 2048, 4096, bytes_per) == 1
+        assert one([11008] * 2, 64, 4096, bytes_per) == 0   # the decode kernels' rows
+        assert one([11000] * 2, 333, 4096, bytes_per) == 0  # no whole tiles
+        assert one([11008] * 2, 0, 4096, bytes_per) == 0 and one([], 333, 4096, bytes_per) == 0
+        assert one([1 << 20] * 2, 333, 4096 // bytes_per, bytes_per) == 0  # weights of 4 GiB
+    assert one([5120] * 2, 66, 2048, 1) == 0 and one([5120] * 2, 129, 2048, 1) == 1  # per weight, then one launch
+    assert one([11008] * 2, 333, 4096, 3) == 0
+
+
 def test_environment_switches_are_read_once(monkeypatch):
     """The library keeps a TPPX_* switch after its first read (no getenv per launch, and a captured graph's kernel
     choice cannot drift); tppx_reload_env() makes it read again."""

@@ -205,12 +205,14 @@ def test_prefill_mxfp4_ragged_blocks_and_post_ops(post):
     _run("mxfp4", 300, 544, 384, post, post != "mul", 700, ulps=2 if post in ("silu", "gelu") else 1)
 
 
-@pytest.mark.parametrize("tile", [1, 2, 3])
+@pytest.mark.parametrize("tile,w8", [(1, 1), (2, 1), (2, 0), (3, 1)])
 @pytest.mark.parametrize("post", ["none", "silu", "add2"])
-def test_prefill_mxfp4_every_workgroup_tile_ragged(tile, post, monkeypatch):
-    """The three workgroup tiles of the large-M MXFP4 kernel (256 x 256, 128 x 256 two per CU, 128 x 512), each
-    forced, on the ragged case above (rows, channel blocks and K steps all uneven) against the oracle."""
+def test_prefill_mxfp4_every_workgroup_tile_ragged(tile, w8, post, monkeypatch):
+    """The workgroup tiles of the large-M MXFP4 kernel from 128 x 256 on (256 x 256, 128 x 256 with eight waves and with
+    four, two per CU, 128 x 512), each forced, on the ragged case above (rows, channel blocks and K steps all uneven)
+    against the oracle."""
     monkeypatch.setenv("TPPX_TILED_BIG_TILE", str(tile))
+    monkeypatch.setenv("TPPX_TILED_W8", str(w8))
     _run("mxfp4", 300, 544, 384, post, True, 705, ulps=2 if post == "silu" else 1)
 
 
@@ -241,9 +243,9 @@ def test_prefill_mxfp4_workgroup_tiles_and_xcd_splits_agree(monkeypatch):
 
 @pytest.mark.parametrize("M", [70, 150, 200, 500])
 def test_prefill_forms_for_small_launches_agree(M, monkeypatch):
-    """Launches that leave CUs empty run other forms of the large-M kernel's body -- 64 x 128 workgroups of four waves
-    up to 128 workgroups of 128 x 256, eight waves per 128 x 256 workgroup up to 256 -- with the same sums in the
-    same order: identical bits to the four-wave 128 x 256 form, for a single GEMM (ragged rows and channel blocks),
+    """Launches that leave CUs empty run other forms of the large-M kernels -- 64 x 128 workgroups of four waves, eight
+    waves per 128 x 256 workgroup up to 256 of those -- with the same sums in the same order: identical bits to the
+    four-wave 128 x 256 form, for a single GEMM (ragged rows and channel blocks),
     fused q/k/v, the gate/up pair and unquantized bf16 weights; the same for the QINT8 kernel's 64 x 256 form (single
     GEMM and fused q/k/v); and the single MXFP4 GEMM against the oracle."""
     ops = _ops()
@@ -1000,6 +1002,52 @@ def test_prefill_qint8_pair_agrees_with_two_launches(fmt, M, N, K, monkeypatch):
         m.setattr(ops, "fc_silu", None)  # (the two launches would call it)
         got = ops.swiglu_gate_up(x, ws[0], ws[1], b, None)
     assert torch.equal(got, ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], b)))
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [("qint8", 66, 5120, 2048), ("qint8", 128, 1536, 1024), ("bf16", 65, 64, 2048), ("bf16", 100, 32, 4096)])
+def test_groups_that_run_per_weight_are_asked_about_first(fmt, M, N, K, monkeypatch):
+    """Where the library would answer TPPX_EUNSUPPORTED to a gate/up pair or a q/k/v group (few rows on small weights),
+    the call is not made and nothing is prepared for it: the outputs are those of one call per weight."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    ws = [block_bf16(randn_bf16((N, K), 0.05, 775 + i), bc=256).cuda() for i in range(2)]
+    if fmt == "qint8":
+        ws = [ops.remap_and_quantize_qint8(w) for w in ws]
+    x = randn_bf16((M, K), 1.0, 777).cuda()
+    want = ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], None))
+    qkv = [ops.fc_plain(x, w, None) for w in ws]
+    lib = _lib.lib()
+
+    class Without:
+        def __getattr__(self, name):
+            assert name not in ("tppx_swiglu_qint8", "tppx_swiglu_bf16", "tppx_multi_linear_bf16"), name
+            return getattr(lib, name)
+
+    monkeypatch.setattr(_lib, "lib", lambda: Without())
+    assert torch.equal(ops.swiglu_gate_up(x, ws[0], ws[1]), want)
+    if fmt == "bf16":
+        assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws, [None] * 2), qkv))
+
+
+@pytest.mark.parametrize("M", [65, 128, 129, 300])
+@pytest.mark.parametrize("N,K", [(64, 2048), (1536, 1024), (5120, 2048)])
+def test_group_is_one_launch_answers_as_the_calls_do(M, N, K):
+    """tppx_group_is_one_launch against what tppx_swiglu_bf16 and tppx_swiglu_qint8 do with the same shape."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    L = _lib.lib()
+    w = block_bf16(randn_bf16((N, K), 0.05, 778), bc=256).cuda()
+    nat, (q, s) = ops._bf16_native(w), ops.remap_and_quantize_qint8(w).native()
+    x = randn_bf16((M, K), 1.0, 779).cuda()
+    y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    xq, sa = ops._qint8_scratch(x, M, K, 256)
+    st, ns = _lib.stream_of(x), (ctypes.c_int64 * 2)(N, N)
+    rc = L.tppx_swiglu_bf16(x.data_ptr(), nat.data_ptr(), None, nat.data_ptr(), None, y.data_ptr(), M, N, K, 0, st)
+    assert rc in (_lib.OK, _lib.EUNSUPPORTED) and (rc == _lib.OK) == bool(L.tppx_group_is_one_launch(ns, 2, M, K, 2))
+    rc = L.tppx_swiglu_qint8(x.data_ptr(), xq.data_ptr(), sa.data_ptr(), q.data_ptr(), s.data_ptr(), None, q.data_ptr(),
+                             s.data_ptr(), None, y.data_ptr(), M, N, K, 256, 0, st)
+    assert rc in (_lib.OK, _lib.EUNSUPPORTED) and (rc == _lib.OK) == bool(L.tppx_group_is_one_launch(ns, 2, M, K, 1))
 
 
 def test_prefill_qint8_pair_of_2_31_outputs():

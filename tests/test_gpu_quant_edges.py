@@ -287,3 +287,27 @@ def test_dequantize_takes_codes_at_any_address(fmt, off):
         w.scales = moved(w.scales)
     assert w.qdata.data_ptr() % 4 == off
     assert torch.equal(w.dequantize(), want)
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "qint2"])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_dequantize_writes_to_any_float_address(fmt, off):
+    """An output that starts 4, 8 or 12 bytes past a 16-byte address: the same values as an aligned one, and nothing
+    written before or behind it."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    q = {"mxfp4": ops.remap_and_quantize_mxfp4, "qint2": ops.remap_and_quantize_qint2_intlv}[fmt]
+    N, K = 64, 512
+    w = q(randn_bf16((N, K), 0.05, 5200).view(2, 32, 8, 32, 2).permute(0, 2, 3, 1, 4).contiguous().cuda())
+    want = w.dequantize().reshape(-1)
+    buf = torch.full((N * K + 8,), -7.0, device="cuda")
+    out = buf[off:off + N * K]
+    assert buf.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 4 * off
+    L, st = _lib.lib(), _lib.stream_of(buf)
+    if fmt == "mxfp4":
+        _lib.check(L.tppx_dequantize_mxfp4(w.qdata.data_ptr(), w.scales.data_ptr(), N, K, out.data_ptr(), st))
+    else:
+        _lib.check(L.tppx_dequantize_qint2_intlv(w.qdata.data_ptr(), w.scales.data_ptr(), N, K, 256, out.data_ptr(), st))
+    assert torch.equal(out, want)
+    assert torch.equal(buf[:off], torch.full_like(buf[:off], -7.0))
+    assert torch.equal(buf[off + N * K:], torch.full_like(buf[off + N * K:], -7.0))

@@ -757,6 +757,27 @@ static int run_bf16_group(const char* who, const void* x, const tppx_seg* segs, 
   return check_hip(launch_tiled_bf16_group(t, n_segs, stream, dual), who);
 }
 
+extern "C" int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M, int64_t K, int weight_bytes) {
+  if (!Ns || n_segs < 1 || n_segs > TPPX_MAX_SEGS || M <= 0 || M >= (1 << 24) || K <= 0 || K >= (1 << 24) ||
+      (weight_bytes != 1 && weight_bytes != 2))
+    return 0;
+  int64_t tiles = 0;
+  for (int i = 0; i < n_segs; i++) {
+    if (Ns[i] <= 0 || Ns[i] % 16 != 0 || Ns[i] > (1 << 25))
+      return 0;
+    TiledParams t;
+    memset(&t, 0, sizeof(t));
+    t.M = (int)M;
+    t.K = (int)K;
+    t.tiles = (int)(Ns[i] / 16);
+    t.qbs = 256;
+    if (!(weight_bytes == 1 ? tiled_qint8_takes_groups(t) : tiled_bf16_takes_groups(t)))
+      return 0;
+    tiles += t.tiles;
+  }
+  return want_tiled(M, 0, K, tiles, (double)tiles * 16.0 * (double)K * weight_bytes, weight_bytes == 1 ? COST_QINT8 : COST_BF16);
+}
+
 extern "C" int tppx_multi_linear_bf16(const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,
                                       tppx_stream_t stream) {
   return run_bf16_group("tppx_multi_linear_bf16", x, segs, n_segs, M, K, flags, false, (hipStream_t)stream);

@@ -457,6 +457,8 @@ def _bf16_group(input, weights, biases, pair=False):
     if any(k != K for _, k in geo) or (pair and geo[0] != geo[1]):
         return None
     L = _lib.lib()
+    if not L.tppx_group_is_one_launch((ctypes.c_int64 * n)(*(N for N, _ in geo)), n, M, K, 2):
+        return None
     x = input.contiguous()
     keep = [(_prep_bias(b, N, x.device), _bf16_native(w)) for (N, _), b, w in zip(geo, biases, weights)]
     lead = tuple(input.shape[:-1])
@@ -1113,7 +1115,8 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
     if w_gate._qscheme != QSCHEME_MXFP:
         # the large-M kernel (from 65 rows, where the library's estimate prefers it to the row kernels, blocks of 256)
         # takes the pair as one launch behind one quantization: rounds(2w) <= 2 rounds(w), so it is never the slower way
-        if M > 64 and w_gate.block_size == w_up.block_size == 256:
+        if M > 64 and w_gate.block_size == w_up.block_size == 256 and \
+                L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, 1):
             y = torch.empty(tuple(input.shape[:-1]) + (N,), dtype=torch.bfloat16, device=x.device)
             bg, bu = _prep_bias(b_gate, N, x.device), _prep_bias(b_up, N, x.device)
             (qg, sg), (qu, su) = w_gate.native(), w_up.native()

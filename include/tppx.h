@@ -425,10 +425,10 @@ int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* qw_gate,
                       const void* bias_up, void* y, int64_t M, int64_t N,
                       int64_t K, int64_t qbs, int flags, tppx_stream_t stream);
 
-/* 1 where the three calls above run n_segs weights of Ns[i] x K (weight_bytes 2:
- * bf16; 1: QINT8 in blocks of 256) over M rows as one launch, 0 where they
- * answer TPPX_EUNSUPPORTED or refuse the shape: a caller asks before it
- * prepares buffers for them. */
+/* 1 where the calls above run n_segs bf16 weights of Ns[i] x K (weight_bytes 2),
+ * or the pair of QINT8 weights in blocks of 256 (weight_bytes 1, two equal Ns),
+ * over M rows as one launch, 0 where they answer TPPX_EUNSUPPORTED or refuse
+ * the shape: a caller asks before it prepares buffers for them. */
 int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M,
                              int64_t K, int weight_bytes);
 

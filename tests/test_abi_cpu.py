@@ -240,8 +240,7 @@ def test_launch_plans_of_the_baseline_shapes():
     assert len(lines) == 1 and "big_mxfp4_kernel<8, true, 1, 8> grid=1792x1x1" in lines[0]       # silu*mul in the epilogue
     lines = plan(L.tppx_plan_multi_linear_mxfp4, pair, 2, 2048, 8192, 1, _lib.FLAG_ACT_FP8, 1 << 28)
     assert any("big_fp8_kernel<8, true> grid=1792x1x1" in l for l in lines), lines
-    # prompts of a few hundred tokens: launches of at most 128 workgroups of 128 x 256 run as four times as many of
-    # 64 x 128; up to 256 of them, as eight waves per workgroup
+    # prompts of a few hundred tokens: 64 x 128 workgroups, or 128 x 256 ones of eight waves while one per CU is enough
     assert "big_mxfp4_kernel<2, false, 2, 2> grid=256x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 512, 4096, 4096,
                                                                              _lib.FLAG_FORCE_TILED, 0)[0]
     assert "big_mxfp4_kernel<2, false, 2, 2>" in plan(L.tppx_plan_linear_mxfp4, 512, 4096, 4096, 0, 0)[0]   # and it is the choice
@@ -295,6 +294,41 @@ def test_launch_plans_of_per_output_channel_qint8():
     assert len(odd) == 2 and "quant_act_int8_kernel" in odd[0] and "skinny_qint8_kernel<1, 1, 4, 16, 4, true>" in odd[1], odd
 
 
+def test_kernel_family_of_short_prompts():
+    """65 and more rows on the family and tile that measured fastest, where one figure per block row was far off: the
+    decode kernels where the block rows share rounds (few channels), tiles where they do not (many), and the small
+    tiles' extra cost where an odd number of row blocks leaves no rectangles for the XCDs."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+    buf = ctypes.create_string_buffer(4096)
+
+    def one(M, N, K):
+        _lib.check(L.tppx_plan_linear_mxfp4(M, N, K, 0, 1 << 25, buf, len(buf)))
+        return buf.value.decode()
+
+    def pair(M, N, K):
+        _lib.check(L.tppx_plan_multi_linear_mxfp4((ctypes.c_int64 * 2)(N, N), 2, M, K, 1, 0, 1 << 25, buf, len(buf)))
+        return buf.value.decode()
+
+    for M in (65, 128):
+        assert "skinny_mxfp4" in pair(M, 1024, 4096) and "skinny_mxfp4" in pair(M, 1536, 18944), M  # 11 us (tiles 22), 38 (79)
+        assert "big_mxfp4" in one(M, 28672, 2560) and "big_mxfp4" in one(M, 18944, 1024), M         # 25 us (rows 52), 14 (26)
+        assert "big_mxfp4" in pair(M, 11008, 4096), M                                              # 34 us (rows 42)
+    for M in (160, 256):
+        assert "skinny_mxfp4" in one(M, 1024, 18944) and "skinny_mxfp4" in pair(M, 1024, 8192), M    # 36 us (77), 19 (38)
+    assert "big_mxfp4" in one(192, 14336, 5120)                                                     # 42 us (65)
+    assert "<2, false, 2, 2>" not in one(1800, 2560, 11008) and "<2, false, 2, 2>" in one(1500, 1536, 18944)
+    assert "<8, true, 1, 8>" in pair(2048, 28672, 8192)                                             # 1254 us (128 x 256: 1283)
+
+    def per_weight(M, N, K, weight_bytes):
+        return not L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, weight_bytes)
+
+    assert per_weight(200, 1024, 3584, 1) and per_weight(256, 1024, 4096, 1)    # 22 us (one launch 28), 26 (31)
+    assert not per_weight(212, 1024, 2304, 1)                                   # 22 us (per weight 45)
+    assert per_weight(160, 1024, 5120, 2) and not per_weight(160, 4096, 5120, 2)
+
+
 def test_group_is_one_launch():
     """Which groups the large-M launches take, by sizes alone: rows, blocks of whole tiles, operands below 4 GiB."""
     import ctypes
@@ -305,13 +339,14 @@ def test_group_is_one_launch():
         return L.tppx_group_is_one_launch((ctypes.c_int64 * len(Ns))(*Ns), len(Ns), M, K, weight_bytes)
 
     for bytes_per in (1, 2):
-        assert one([11008] * 2, 333, 4096, bytes_per) == 1 and one([4096, 1024, 1024], 2048, 4096, bytes_per) == 1
+        assert one([11008] * 2, 333, 4096, bytes_per) == 1 and one([11008] * 2, 2048, 4096, bytes_per) == 1
         assert one([11008] * 2, 64, 4096, bytes_per) == 0   # the decode kernels' rows
         assert one([11000] * 2, 333, 4096, bytes_per) == 0  # no whole tiles
         assert one([11008] * 2, 0, 4096, bytes_per) == 0 and one([], 333, 4096, bytes_per) == 0
         assert one([1 << 20] * 2, 333, 4096 // bytes_per, bytes_per) == 0  # weights of 4 GiB
     assert one([5120] * 2, 66, 2048, 1) == 0 and one([5120] * 2, 129, 2048, 1) == 1  # per weight, then one launch
     assert one([11008] * 2, 333, 4096, 3) == 0
+    assert one([4096, 1024, 1024], 2048, 4096, 2) == 1 and one([4096, 1024, 1024], 2048, 4096, 1) == 0  # bf16 only
 
 
 def test_environment_switches_are_read_once(monkeypatch):

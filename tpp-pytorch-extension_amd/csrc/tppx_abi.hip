@@ -217,46 +217,106 @@ static const int64_t TILED_MIN_M = 65; // more rows than the decode kernels cove
 
 // More than 64 rows: the LDS-tiled kernels give every workgroup a whole output tile and all of K, so a launch with
 // few tiles leaves most of the 256 CUs idle (7B shapes at 256 rows: 43 workgroups), while the decode kernels run one
-// block row of 64 rows after the other over the full grid, streaming the weights once per block row.  Pick by a
-// cost estimates fitted to measurements on MI355X (us).  MXFP4: a block row of 64 costs about 4.7 (pair: 9.5) + weight bytes /
-// 5.5 TB/s + 0.4 ns per input channel (its activations), the tiled launches what tiled_mxfp4_us() says.  QINT8 (128 x 256
-// tiles, one workgroup per CU) and unquantized bf16 weights (128 x 256 tiles, two workgroups per CU): their own fits
-// below.  `wbytes` = weight bytes of
-// the whole call, `n_tiles16` = its 16-channel tiles.  TPPX_TILED_MIN_M (when set) restores a plain row threshold.
-enum { COST_MXFP4 = 0, COST_QINT8 = 1, COST_BF16 = 2, COST_MXFP4_PAIR = 3 };
-static bool want_tiled(int64_t M, int flags, int64_t K = 0, int64_t n_tiles16 = 0, double wbytes = 0.0,
-                       int kind = COST_MXFP4) {
+// block row of 64 rows after the other over the full grid, streaming the weights once per block row.  Pick by cost
+// estimates fitted to measurements on MI355X (us).  TPPX_TILED_MIN_M (when set) restores a plain row threshold.
+enum { BY_ROWS, BY_TILES, BY_COST };
+static int kernel_family(int64_t M, int flags) {
   if (flags & TPPX_FLAG_FORCE_SKINNY)
-    return false;
+    return BY_ROWS;
   if (flags & TPPX_FLAG_FORCE_TILED)
-    return true;
+    return BY_TILES;
   if (M < TILED_MIN_M)
-    return false;
+    return BY_ROWS;
   const int env_min = env_int("TPPX_TILED_MIN_M", -1);
   if (env_min >= 0)
-    return M >= env_min;
-  if (K <= 0 || n_tiles16 <= 0 || M > 1024)
+    return M >= env_min ? BY_TILES : BY_ROWS;
+  return M > 1024 ? BY_TILES : BY_COST;
+}
+
+// What the decode kernels take over block rows of 64 rows: rounds of 256 workgroups of nt channel tiles and one block row,
+// each round a fixed part and a part per input channel; the last one costs three quarters when it is all but empty.
+struct RowsCost {
+  double launch, round, per_k; // us, us, ns
+};
+static double rows_us(const RowsCost& c, int64_t wgs, int64_t K) {
+  const double r = (double)((wgs + 255) / 256), f = (double)wgs / 256.0 - (r - 1.0);
+  return c.launch + (r - 0.25 * (1.0 - f)) * (c.round + c.per_k * 1e-3 * (double)K);
+}
+
+// the tile x K-part kernel's shapes (33..64 rows per block row, K in 4 slices across workgroups, partial sums in ws)
+static bool mxfp4_nk_fits(int64_t M, int total_tiles, int units, int64_t ws_bytes) {
+  const int groups = (total_tiles + 3) / 4;
+  return env_int("TPPX_MXFP4_NK", 1) != 0 && groups * 4 <= 256 && groups * 4 >= 96 && units >= 64 && (units + 3) / 4 <= 32 &&
+         (int64_t)4 * groups * 4 * 4 * 256 * (int64_t)sizeof(float) * ((M + 63) / 64) <= ws_bytes;
+}
+
+// MXFP4 (dual: `tiles` of each projection).  Both sides within 12 % of 3600 launches of 65 .. 640 rows; the family and
+// tile taken are within 0.5 % of the fastest on average (the fits before, one figure per block row whatever its rounds:
+// 4.6 %, and twice the time for pairs of 1024 channels or single GEMMs of 28672 x 2560).
+static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, bool dual, bool nk, int64_t ws_bytes) {
+  const int family = kernel_family(M, flags);
+  if (family != BY_COST)
+    return family == BY_TILES;
+  const int64_t rows64 = (M + 63) / 64, n_tiles16 = (dual ? 2 : 1) * tiles;
+  if (K < 1024 && M > 256) // (shorter than what was fitted, and short of work either way: tiles, as ever)
     return true;
-  const double rows64 = (double)((M + 63) / 64);
-  if (kind == COST_QINT8) {
-    const int64_t wgs = ((M + 127) / 128) * ((n_tiles16 + 15) / 16);
-    // (launches of at most 128 such workgroups run as twice as many of 64 x 256)
-    const bool small = wgs <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0;
-    const double tiled_us = small ? 8.0 + (double)K * 0.006 : (double)((wgs + 255) / 256) * (10.0 + (double)K * 0.0075);
-    const double skinny_us = rows64 * (5.0 + wbytes / 5.5e6 + (double)K * 0.0004);
-    return tiled_us <= skinny_us;
+  if (M < big_min_rows()) { // the 128 x 128 kernel without direct-to-LDS loads
+    const int64_t wgs = ((M + 127) / 128) * ((n_tiles16 + 7) / 8);
+    return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
+           (double)rows64 * (8.0 + (double)n_tiles16 * 16.0 * (double)K * (0.5 + 1.0 / 32) / 5.5e6 + (double)K * 0.0008);
   }
-  if (kind == COST_BF16 && M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
-    return tiled_bf16_us(M, K, n_tiles16) <= rows64 * (6.5 + wbytes / 5.5e6 + (double)K * 0.0006);
-  const bool big = (kind == COST_MXFP4 || kind == COST_MXFP4_PAIR) && M >= big_min_rows();
-  if (big) // (a block row of the decode kernels: 9.6 us at 4096 x 4096, 16 at 4096 x 11008, 11-13 at 2560 x 10240, 13 at
-           // 12288 x 4096; 33 at 3584 x 18944, beyond the kernels that split K; the pair 21 at 2 x 11008 x 4096)
-    return tiled_mxfp4_us(M, K, n_tiles16) <=
-           rows64 * ((kind == COST_MXFP4_PAIR ? 9.5 : 4.7) + wbytes / 5.5e6 + (double)K * (K > 16384 ? 0.0014 : 0.0004));
-  const int64_t wgs = ((M + 127) / 128) * ((n_tiles16 + 7) / 8);
-  const double tiled_us = (double)((wgs + 255) / 256) * (double)K * 0.0203;
-  const double skinny_us = rows64 * (8.0 + wbytes / 5.5e6 + (double)K * 0.0008);
-  return tiled_us <= skinny_us;
+  static constexpr RowsCost SINGLE[3] = {{1.84, 1.85, 1.78}, {1.78, 2.70, 2.03}, {2.49, 4.26, 2.17}};
+  static constexpr RowsCost DUAL[3] = {{1.91, 2.69, 1.94}, {1.57, 4.04, 2.64}, {1.88, 6.88, 3.42}};
+  static constexpr RowsCost NK = {1.78, 6.63, 0.734};
+  const double tiled = tiled_mxfp4_us(M, K, n_tiles16);
+  if (nk && mxfp4_nk_fits(M, (int)tiles, (int)(K / 128), ws_bytes))
+    return tiled <= rows_us(NK, (tiles + 3) / 4 * 4 * rows64, K);
+  const int nt = tiles <= 256 ? 1 : (tiles + 1) / 2 <= 256 ? 2 : 3; // channel tiles per workgroup, as the launch picks them
+  // (a single GEMM of two block rows stays with the decode kernels unless the tiles win by more than both estimates are
+  // off: 28.7 against 23.1 us at 11008 x 4096 are left there, 52 against 24 at 28672 x 2560 are not)
+  const double margin = !dual && rows64 == 2 ? 1.22 : 1.0;
+  return tiled * margin <= rows_us((dual ? DUAL : SINGLE)[nt - 1], (tiles + nt - 1) / nt * rows64, K);
+}
+
+// QINT8 (128 x 256 tiles, one workgroup per CU; at most 128 of them: twice as many of 64 x 256).  `tiles` of the whole
+// launch.  The gate/up pair (dual) stands against two launches behind a quantizer each; where those would be decode
+// launches of few rounds, they win: 2 x 1024 x 3584 at 200 rows 22 us against 28.
+static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, bool dual) {
+  const int family = kernel_family(M, flags);
+  if (family != BY_COST)
+    return family == BY_TILES;
+  const int64_t rows64 = (M + 63) / 64, wgs = ((M + 127) / 128) * ((tiles + 15) / 16);
+  const bool small = wgs <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0;
+  const double tiled_us = small ? 8.0 + (double)K * 0.006 : (double)((wgs + 255) / 256) * (10.0 + (double)K * 0.0075);
+  if (dual && !want_tiled_qint8(M, K, flags, tiles / 2, false)) {
+    static constexpr RowsCost ROWS[3] = {{4.62, 2.33, 1.35}, {5.38, 4.48, 1.55}, {5.14, 5.03, 2.41}};
+    const int64_t one = tiles / 2;
+    const int nt = one < 512 ? 1 : one > 512 && one <= 768 ? 3 : 2; // as plan_skinny
+    if (tiled_us > 1.15 * 2.0 * rows_us(ROWS[nt - 1], (one + nt - 1) / nt * rows64, K))
+      return false;
+  }
+  return tiled_us <= (double)rows64 * (5.0 + (double)tiles * 16.0 * (double)K / 5.5e6 + (double)K * 0.0004);
+}
+
+// Unquantized bf16 weights: n of them as one launch of the large-M kernel against one decode launch each
+static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tiles, int n) {
+  const int family = kernel_family(M, flags);
+  if (family != BY_COST)
+    return family == BY_TILES;
+  static constexpr RowsCost ROWS[2] = {{1.63, 2.01, 2.40}, {1.16, 3.71, 3.11}};
+  const int64_t rows64 = (M + 63) / 64;
+  int64_t all = 0;
+  double rows = 0.0;
+  for (int i = 0; i < n; i++) {
+    const int nt = tiles[i] > 512 ? 2 : 1;
+    rows += rows_us(ROWS[nt - 1], (tiles[i] + nt - 1) / nt * rows64, K);
+    all += tiles[i];
+  }
+  if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
+    return tiled_bf16_us(M, K, all) <= rows;
+  const int64_t wgs = ((M + 127) / 128) * ((all + 7) / 8); // tiled_bf16_kernel
+  return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
+         (double)rows64 * (8.0 + (double)all * 32.0 * (double)K / 5.5e6 + (double)K * 0.0008);
 }
 
 static TiledParams tiled_from_seg(const DecodeParams& p, int i) {
@@ -352,9 +412,7 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
       return rc;
     return check_hip(launch_tiled_mxfp4_fp8_group(&t[1], 1, stream), who);
   }
-  if (want_tiled(M, flags, K, dual ? 2 * p.total_tiles : p.total_tiles,
-                 (dual ? 2.0 : 1.0) * (double)p.total_tiles * 16.0 * (double)K * (0.5 + 1.0 / 32),
-                 dual ? COST_MXFP4_PAIR : COST_MXFP4)) {
+  if (want_tiled_mxfp4(M, K, flags, p.total_tiles, dual, !dual && n_segs == 1 && !row_sumsq, ws_bytes)) {
     TPPX_REQUIRE(!row_sumsq, TPPX_EUNSUPPORTED, "%s: row sums of squares are not produced by the large-M kernels", who);
     // prefill shapes: one LDS-tiled launch per GEMM of the group; the fused
     // gate/up pair becomes silu(gate) followed by up * gate (same rounding)
@@ -448,14 +506,10 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
     // finishes last (measured: 26 -> 21 us for 64 rows at K = 11008 / N = 4096; no gain for 32 rows).
     // 33..64 rows, a single GEMM with few channel tiles and a long K: four tiles x four K parts per workgroup with
     // the activations of a K tile staged ONCE per workgroup, K in four slices across workgroups
-    if (!dual && mg == 4 && n_segs == 1 && !row_sumsq && env_int("TPPX_MXFP4_NK", 1) != 0) {
-      const int groups = (p.total_tiles + 3) / 4;
-      if (groups * 4 <= 256 && groups * 4 >= 96 && p.units >= 64 && (p.units + 3) / 4 <= 32 &&
-          (int64_t)4 * groups * 4 * mg * 256 * (int64_t)sizeof(float) * ((M + 63) / 64) <= ws_bytes) {
-        p.S = 4;
-        p.part = (float*)ws;
-        return check_hip(launch_skinny_mxfp4_nk(p, stream), who);
-      }
+    if (!dual && mg == 4 && n_segs == 1 && !row_sumsq && mxfp4_nk_fits(M, p.total_tiles, p.units, ws_bytes)) {
+      p.S = 4;
+      p.part = (float*)ws;
+      return check_hip(launch_skinny_mxfp4_nk(p, stream), who);
     }
     const int S = (dual || mg != 4) ? 1 : pick_split(p, M, K, mg, 4, 2048, ws_bytes);
     int nt = S;
@@ -504,8 +558,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
   p.units = (int)(K / (64 * p.deal));
   p.spb_magic = (p.deal == 4 && p.tpb > 4) ? (unsigned int)((((uint64_t)1 << 32) + (uint64_t)(p.tpb / 4) - 1) / (uint64_t)(p.tpb / 4)) : 0u;
   const bool reuse = (flags & TPPX_FLAG_XQ_REUSE) != 0; // xq / sa still hold this x, quantized by an earlier call
-  const int64_t tiles = (dual ? 2 : 1) * (int64_t)p.total_tiles;
-  const bool tiled = qbs % 128 == 0 && want_tiled(M, flags, K, tiles, (double)tiles * 16.0 * (double)K, COST_QINT8);
+  const bool tiled = qbs % 128 == 0 && want_tiled_qint8(M, K, flags, (dual ? 2 : 1) * (int64_t)p.total_tiles, dual);
   TiledParams t[TPPX_MAX_SEGS];
   bool group = tiled && n_segs > 1; // one grid over the channel blocks of all GEMMs when the large-M kernel takes them
   for (int i = 0; i < n_segs && tiled; i++) {
@@ -712,9 +765,9 @@ extern "C" int tppx_linear_bf16(const void* x, const void* w, const void* bias, 
   p.units = (int)(K / 128);
   p.tpb = 1;
   p.S = 1;
-  // more than 64 rows: the LDS-tiled kernel once it is the cheaper one (the estimate of the quantized formats with the
-  // weight's real bytes: the row-group kernel streams the whole weight once per 64 rows)
-  if (want_tiled(M, flags, K, p.total_tiles, (double)N * (double)K * 2.0, COST_BF16)) {
+  // more than 64 rows: the LDS-tiled kernel once it is the cheaper one
+  const int64_t tiles = p.total_tiles;
+  if (want_tiled_bf16(M, K, flags, &tiles, 1)) {
     TPPX_REQUIRE(aligned16(w), TPPX_EINVAL, "%s: weight not 16-byte aligned", who);
     return check_hip(launch_tiled_bf16(tiled_from_seg(p, 0), (hipStream_t)stream), who);
   }
@@ -742,26 +795,28 @@ static int run_bf16_group(const char* who, const void* x, const tppx_seg* segs, 
   p.x = x;
   p.M = (int)M;
   p.K = (int)K;
-  const int64_t tiles = (dual ? 2 : 1) * (int64_t)p.total_tiles;
   TiledParams t[TPPX_MAX_SEGS];
-  bool group = want_tiled(M, flags, K, tiles, (double)tiles * 16.0 * (double)K * 2.0, COST_BF16);
+  int64_t tiles[TPPX_MAX_SEGS];
+  bool group = true;
   for (int i = 0; i < n_segs; i++) {
     t[i] = tiled_from_seg(p, i);
+    tiles[i] = t[i].tiles;
     TPPX_REQUIRE(M * t[i].N < ((int64_t)1 << 31), TPPX_ESHAPE, "%s: M*N=%ld outputs exceed 2^31", who, (long)(M * t[i].N));
     TPPX_REQUIRE(aligned16(t[i].qw), TPPX_EINVAL, "%s: weight not 16-byte aligned", who);
     if (dual)
       t[i].post_op = TPPX_POST_NONE;
     group = group && tiled_bf16_takes_groups(t[i]);
   }
+  group = group && want_tiled_bf16(M, K, flags, tiles, n_segs);
   TPPX_REQUIRE(group, TPPX_EUNSUPPORTED, "%s: M=%ld runs as one launch per weight", who, (long)M);
   return check_hip(launch_tiled_bf16_group(t, n_segs, stream, dual), who);
 }
 
 extern "C" int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M, int64_t K, int weight_bytes) {
   if (!Ns || n_segs < 1 || n_segs > TPPX_MAX_SEGS || M <= 0 || M >= (1 << 24) || K <= 0 || K >= (1 << 24) ||
-      (weight_bytes != 1 && weight_bytes != 2))
+      (weight_bytes == 1 ? n_segs != 2 || Ns[0] != Ns[1] : weight_bytes != 2))
     return 0;
-  int64_t tiles = 0;
+  int64_t tiles[TPPX_MAX_SEGS];
   for (int i = 0; i < n_segs; i++) {
     if (Ns[i] <= 0 || Ns[i] % 16 != 0 || Ns[i] > (1 << 25))
       return 0;
@@ -773,9 +828,9 @@ extern "C" int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M
     t.qbs = 256;
     if (!(weight_bytes == 1 ? tiled_qint8_takes_groups(t) : tiled_bf16_takes_groups(t)))
       return 0;
-    tiles += t.tiles;
+    tiles[i] = t.tiles;
   }
-  return want_tiled(M, 0, K, tiles, (double)tiles * 16.0 * (double)K * weight_bytes, weight_bytes == 1 ? COST_QINT8 : COST_BF16);
+  return weight_bytes == 1 ? want_tiled_qint8(M, K, 0, 2 * tiles[0], true) : want_tiled_bf16(M, K, 0, tiles, n_segs);
 }
 
 extern "C" int tppx_multi_linear_bf16(const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,

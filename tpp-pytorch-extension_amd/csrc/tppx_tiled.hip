@@ -1453,39 +1453,75 @@ big_fp8_kernel(const BigParams P) {
     big_epilogue<MT>(p, acc, reinterpret_cast<float*>(tl_lds) + wave * 64 * EP_LD, m_wg + wm * (MT * 16), tile_base);
 }
 
-// Workgroup tiles of the MXFP4 launches and what a launch of `wgs` of them takes, in us, K steps of 128: a fixed part
-// (launch, first loads, epilogue) and a part per step, fitted to linears and SwiGLU pairs of K = 2560 .. 18944 and
-// 70 .. 2048 rows (one launch at K = 4096 / 18944: 64 x 128 23.5 / 79 us, 128 x 128 35 / 122, 128 x 256 48 / 178,
-// 128 x 512 80 / 301, 256 x 256 82 / 304, whatever part of the 256 CUs it fills).
+// Workgroup tiles of the MXFP4 and bf16 launches:
 //   256 x 256, 128 x 512  eight waves, one workgroup per CU; for launches that fill the chip several times over
-//   128 x 256             up to 256 of them the ring kernel (one per CU), beyond that four waves and two per CU
-//   128 x 128             ring kernel, one per CU
-//   64 x 128              ring kernel, two per CU
+//   128 x 256             up to 256 of them one per CU (MXFP4: the ring kernel), beyond that four waves and two per CU
+//   128 x 128             MXFP4 only: ring kernel, one per CU
+//   64 x 128              MXFP4: ring kernel; two per CU
 enum { TILE_256_256 = 0, TILE_128_256, TILE_128_512, TILE_64_128, TILE_128_128, N_TILES };
 static constexpr int TILE_ROWS[N_TILES] = {256, 128, 128, 64, 128};
 static constexpr int TILE_COLS16[N_TILES] = {16, 16, 32, 8, 8}; // 16-channel weight tiles (the pair: gate + up)
-static double tile_us(int tile, int64_t wgs, double steps) {
-  const double rounds = (double)((wgs + 255) / 256);
-  switch (tile) {
-  case TILE_256_256:
-    return (20.0 + 1.92 * steps) * rounds;
-  case TILE_128_512:
-    return (19.0 + 1.90 * steps) * rounds;
-  case TILE_128_256:
-    return wgs <= 256 ? 12.0 + 1.13 * steps : (20.0 + 2.05 * steps) * std::max(1.0, (double)wgs / 512.0);
-  case TILE_64_128:
-    return wgs <= 256 ? 7.5 + 0.50 * steps : wgs <= 512 ? 9.0 + 0.85 * steps : (9.0 + 0.97 * steps) * (double)wgs / 512.0;
-  default:
-    return (13.0 + 0.75 * steps) * rounds;
-  }
+
+// What a launch takes, in us, with r = its rounds of 256 workgroups, f = the filled part of the last one and s = K / 128:
+//   one round     a + (b + c f) s
+//   more          p + q r + (u + v r + w f + z r s / 1000) s     (z: the clock falls under the power limit as a launch
+//                                                                 grows; measured up to 28672 x 8192 pairs of 2048 rows)
+// bf16 weights: and g (one round) or h us for each MB of them, which come from memory at whatever tile.
+// Fitted to 2500 launches: 65 .. 2048 rows, linears and pairs of 1024 .. 32000 x 1024 .. 18944, every tile forced, weights
+// rotated through 0.5 .. 2 GB.  The tile chosen is within 0.5 % of the fastest on average, 12 % at worst (MXFP4), and
+// 0.3 %, 12 % (bf16).
+struct TileCost {
+  double a, b, c, p, q, u, v, w, z, g, h;
+};
+static constexpr TileCost MXFP4_COST[N_TILES] = {
+    {17.9, 1.90, 0.39, 0.17, 18.0, -0.65, 2.40, 0.625, 0.311, 0, 0},
+    {11.3, 1.10, 0.213, 5.3, 7.26, -0.265, 1.13, 0.443, 0.177, 0, 0},
+    {17.8, 1.85, 0.406, 0.32, 17.9, -0.653, 2.32, 0.719, 0.431, 0, 0},
+    {6.31, 0.476, 0.0848, 3.63, 2.09, -0.0318, 0.410, 0.112, 0.0374, 0, 0},
+    {9.51, 0.750, 0.126, 2.14, 7.43, -0.202, 0.879, 0.152, 0.011, 0, 0},
+};
+static constexpr TileCost BF16_COST[TILE_128_128] = {
+    {16.8, 1.98, 0.59, -2.62, 19.3, -0.622, 2.58, 0.96, 0.367, 0.0182, 0.00766},
+    {8.10, 1.25, 0.269, 2.46, 7.88, -0.269, 1.17, 0.638, 0.371, 0.0892, 0.0554},
+    {15.4, 1.99, 0.471, -5.16, 20.1, -0.764, 2.53, 1.16, 0.406, 0.0689, 0.0501},
+    {4.85, 0.626, 0.114, 1.63, 0.948, -0.0886, 0.655, 0.154, 0.0973, 0.0527, 0.0832},
+};
+static double tile_us(const TileCost& k, int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
+  const int64_t wgs = mb * nb;
+  const double r = (double)((wgs + 255) / 256), f = (double)wgs / 256.0 - (r - 1.0);
+  if (r <= 1.0)
+    return k.a + (k.b + k.c * f) * s + k.g * weight_mb;
+  // (the z term at most as far as it was measured: 448 rounds x steps of 256 x 256, the same work in the other tiles)
+  const double rs = std::min(r * s, 448.0 * 4096.0 / (TILE_ROWS[tile] * TILE_COLS16[tile]));
+  return k.p + k.q * r + (k.u + k.v * r + k.w * f + k.z * 1e-3 * rs * r) * s + k.h * weight_mb;
+}
+static double mxfp4_tile_us(int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
+  const double us = tile_us(MXFP4_COST[tile], tile, mb, nb, s, weight_mb);
+  // An odd number of row blocks leaves no rectangles for the XCDs (tile_of_block), and columns of more row blocks than
+  // fit a CU set drift apart in K: 23 row blocks of 64 cost 4 % more, 27 8 %, 31 16 % (K = 2048 .. 16384; none at 1024).
+  return tile == TILE_64_128 && mb * nb > 256 && (mb & 1) && mb > 21
+             ? us * (1.0 + 0.02 * (double)(mb - 21) * std::min(1.0, s / 32.0)) : us;
+}
+static double bf16_tile_us(int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
+  return tile_us(BF16_COST[tile], tile, mb, nb, s, weight_mb);
+}
+
+template <typename Us>
+static double cheapest_us(int64_t M, int64_t K, int64_t n_tiles16, int tiles, double weight_mb, Us&& us) {
+  double best = 1e300;
+  for (int i = 0; i < tiles; i++)
+    best = std::min(best, us(i, (M + TILE_ROWS[i] - 1) / TILE_ROWS[i], (n_tiles16 + TILE_COLS16[i] - 1) / TILE_COLS16[i],
+                             (double)(K / 128), weight_mb));
+  return best;
 }
 
 double tiled_mxfp4_us(int64_t M, int64_t K, int64_t n_tiles16) {
-  double best = 1e300;
-  for (int i = 0; i < N_TILES; i++)
-    best = std::min(best, tile_us(i, (M + TILE_ROWS[i] - 1) / TILE_ROWS[i] * ((n_tiles16 + TILE_COLS16[i] - 1) / TILE_COLS16[i]),
-                                  (double)(K / 128)));
-  return best;
+  return cheapest_us(M, K, n_tiles16, env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128, 0.0, mxfp4_tile_us);
+}
+
+double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16) {
+  return cheapest_us(M, K, n_tiles16, env_int("TPPX_TILED_SMALL", 1) != 0 ? TILE_128_128 : TILE_64_128,
+                     (double)(n_tiles16 * 32 * K) * 1e-6, bf16_tile_us);
 }
 
 static bool big_fits(const TiledParams& p) {
@@ -1520,25 +1556,26 @@ static hipError_t big_bf16_launch(const BigParams& P, int wgs, hipStream_t strea
   return hipGetLastError();
 }
 
-// workgroups of a launch over n GEMMs of one activation (dual: the gate/up pair)
-static int64_t group_workgroups(const TiledParams* t, int n, bool dual, int tile) {
-  const int tpw = TILE_COLS16[tile] / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
-  int64_t nb = 0;
-  for (int i = 0; i < (dual ? 1 : n); i++)
-    nb += (t[i].tiles + tpw - 1) / tpw;
-  return (t[0].M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile] * nb;
-}
-
-// the first `tiles` workgroup tiles' lowest estimate
+// the first `tiles` workgroup tiles' lowest estimate for n GEMMs over one activation (dual: the gate/up pair)
 template <typename Us>
 static int cheapest_tile(const TiledParams* t, int n, bool dual, int tiles, Us&& us) {
+  int64_t tiles16 = 0;
+  for (int i = 0; i < n; i++)
+    tiles16 += t[i].tiles;
   int shape = 0;
   double best = 1e300;
-  for (int i = 0; i < tiles; i++)
-    if (const double c = us(i, group_workgroups(t, n, dual, i), (double)(t[0].K / 128)); c < best) {
+  for (int i = 0; i < tiles; i++) {
+    const int tpw = TILE_COLS16[i] / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
+    int64_t nb = 0;
+    for (int g = 0; g < (dual ? 1 : n); g++)
+      nb += (t[g].tiles + tpw - 1) / tpw;
+    if (const double c = us(i, (t[0].M + TILE_ROWS[i] - 1) / TILE_ROWS[i], nb, (double)(t[0].K / 128),
+                            (double)(tiles16 * 32 * t[0].K) * 1e-6);
+        c < (i >= TILE_64_128 ? 0.99 : 1.0) * best) { // (a tie goes to the larger tiles, which read less)
       best = c;
       shape = i;
     }
+  }
   return shape;
 }
 
@@ -1588,7 +1625,7 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
     ring = ring && (reinterpret_cast<uintptr_t>(t[i].sw) & 3u) == 0;
   int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
   if (shape < 0 || shape >= (ring ? N_TILES : TILE_64_128))
-    shape = cheapest_tile(t, n, dual, ring && env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128, tile_us);
+    shape = cheapest_tile(t, n, dual, ring && env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128, mxfp4_tile_us);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 0.53);
   switch (shape) {
@@ -1685,33 +1722,6 @@ silu_mul_kernel(const uint16_t* __restrict__ gate, uint16_t* __restrict__ y, int
   }
 }
 
-// The same estimate for unquantized bf16 weights (four times the weight bytes of a step: what a CU takes in bounds the
-// small tiles; K = 4096 / 11008, one launch: 64 x 128 29 / 60 us, 128 x 256 51 / 116, 256 x 256 85 / 193, 128 x 512
-// 83 / 190; 64 x 128 doubles from 257 workgroups; 128 x 256 at K = 4096: 66 us for 256 workgroups, 91 for 258, 96 for
-// 344, 103 for 430, 110 for 480, 146 for 516, 156 for 645, 168 for 768, 225 for 1000).
-static double tile_bf16_us(int tile, int64_t wgs, double steps) {
-  const double rounds = (double)((wgs + 255) / 256);
-  switch (tile) {
-  case TILE_256_256:
-    return (20.0 + 2.03 * steps) * rounds;
-  case TILE_128_512:
-    return (20.0 + 2.05 * steps) * rounds;
-  case TILE_128_256:
-    return wgs <= 256 ? 14.0 + 1.2 * steps
-                      : (30.0 + 2.5 * steps) * (wgs <= 512 ? 0.64 + 0.36 * (double)wgs / 512.0 : (double)wgs / 512.0);
-  default:
-    return wgs <= 256 ? 11.0 + 0.6 * steps : wgs <= 512 ? 8.0 + 1.38 * steps : (10.0 + 1.5 * steps) * (double)wgs / 512.0;
-  }
-}
-
-double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16) {
-  double best = 1e300;
-  for (int i = 0; i < TILE_128_128; i++)
-    best = std::min(best, tile_bf16_us(i, (M + TILE_ROWS[i] - 1) / TILE_ROWS[i] * ((n_tiles16 + TILE_COLS16[i] - 1) / TILE_COLS16[i]),
-                                       (double)(K / 128)));
-  return best;
-}
-
 // prompt-sized passes; the kernel's 32-bit offsets want operands below 4 GiB
 bool tiled_bf16_takes_groups(const TiledParams& p) {
   return p.M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0 && (int64_t)p.M * p.K * 2 < ((int64_t)1 << 32) &&
@@ -1725,7 +1735,7 @@ hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stre
     return hipErrorInvalidValue;
   int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 .. 4 as in launch_tiled_mxfp4_group; 5 is not built for 2-byte weights
   if (shape < 0 || shape >= TILE_128_128)
-    shape = cheapest_tile(t, n, dual, env_int("TPPX_TILED_SMALL", 1) != 0 ? TILE_128_128 : TILE_64_128, tile_bf16_us);
+    shape = cheapest_tile(t, n, dual, env_int("TPPX_TILED_SMALL", 1) != 0 ? TILE_128_128 : TILE_64_128, bf16_tile_us);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 2.0);
   switch (shape) {

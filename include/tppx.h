@@ -393,10 +393,10 @@ int tppx_multi_linear_qint8(const void* x, void* xq, void* sa,
  * (src/csrc/llm/fused_llm_infer.cpp:1271-1272: i_gemm(SiluPostOp) then
  * i_gemm(MulPostOp)) in one launch with the same bf16 rounding points:
  *   g = silu(bf16(x Wg^T + bg));  y = bf16( g * bf16(x Wu^T + bu) )
- * Prompt shapes (more than 64 rows): one launch that forms the product itself;
- * operands of 4 GiB and more run as two launches, or with M * N * 2 bytes of
- * workspace as one grid (the gate tile parked there) and an elementwise pass
- * where that saves a round.  Same bits in each of these. */
+ * Prompt shapes (more than 64 rows): one launch that forms the product itself
+ * (TPPX_TILED_DUAL_FUSED=0, with M * N * 2 bytes of workspace: one grid with the
+ * gate tile parked there and an elementwise pass, where that saves a round),
+ * or two launches for operands of 4 GiB and more.  Same bits in each of these. */
 int tppx_swiglu_mxfp4(const void* x, const void* qw_gate, const void* sw_gate,
                       const void* bias_gate, const void* qw_up,
                       const void* sw_up, const void* bias_up, void* y,

@@ -216,6 +216,15 @@ def test_prefill_mxfp4_every_workgroup_tile_ragged(tile, w8, post, monkeypatch):
     _run("mxfp4", 300, 544, 384, post, True, 705, ulps=2 if post == "silu" else 1)
 
 
+@pytest.mark.parametrize("fmt", ["mxfp4", "qint8"])
+@pytest.mark.parametrize("M,post", [(65, "add"), (130, "add"), (130, "mul"), (300, "silu"), (300, "relu"), (300, "none"), (130, "add2"), (130, "gelu")])
+def test_prefill_epilogue_of_every_post_op(fmt, M, post):
+    """The epilogue of the large-M kernels is instantiated per post-op (none, SiLU, mul, add) or takes it from the launch
+    (the others), and reads the post-op's input ahead, also for rows past the end: ragged rows and channel blocks."""
+    from tpp_pytorch_extension import _lib
+    _run(fmt, M, 544, 768, post, post != "mul", 740 + M, ulps=2 if post in ("silu", "gelu") else 1, flags=_lib.FLAG_FORCE_TILED)
+
+
 def test_prefill_mxfp4_workgroup_tiles_and_xcd_splits_agree(monkeypatch):
     """Every workgroup tile and every split of the tile space over the XCDs computes the same sums in the same order:
     identical bits, single GEMM, fused q/k/v and the gate/up pair."""

@@ -48,13 +48,14 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint32_t h) {
   return __uint_as_float(h << 16);
 }
 
-// round to nearest even, NaN kept quiet (same rule as the CPU side)
+// round to nearest even, NaN kept quiet (same rule as the CPU side): the hardware conversion, equal to the integer
+// formula (u + 0x7fff + ((u >> 16) & 1)) >> 16 and to (u >> 16) | 0x40 for a NaN over all 2^32 inputs
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u)
-    return (u >> 16) | 0x40u;
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return u >> 16;
+  return __builtin_bit_cast(uint16_t, (__bf16)f);
+}
+// two values into one dword: one instruction
+__device__ __forceinline__ uint32_t f32x2_to_bf16_bits(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo, (__bf16)hi});
 }
 
 __device__ __forceinline__ float round_bf16(float f) {
@@ -90,6 +91,24 @@ __device__ __forceinline__ uint32_t apply_post_bits(float v, int post,
       return (yb & 0x8000u) ? 0u : yb;
     default:
       return yb;
+  }
+}
+
+// apply_post_bits for two adjacent outputs, the post-op known at compile time; in1: the packed pair of its input
+template <int POST>
+__device__ __forceinline__ uint32_t apply_post_pair(float lo, float hi, uint32_t in1, float scale) {
+  const uint32_t yb = f32x2_to_bf16_bits(lo, hi);
+  const float y0 = bf16_bits_to_f32(yb & 0xffffu), y1 = __uint_as_float(yb & 0xffff0000u);
+  if constexpr (POST == TPPX_POST_SILU) {
+    const uint32_t s = f32x2_to_bf16_bits(__frcp_rn(1.0f + __expf(-y0)), __frcp_rn(1.0f + __expf(-y1)));
+    return f32x2_to_bf16_bits(y0 * bf16_bits_to_f32(s & 0xffffu), y1 * __uint_as_float(s & 0xffff0000u));
+  } else if constexpr (POST == TPPX_POST_MUL) {
+    return f32x2_to_bf16_bits(bf16_bits_to_f32(in1 & 0xffffu) * y0, __uint_as_float(in1 & 0xffff0000u) * y1);
+  } else if constexpr (POST == TPPX_POST_ADD_SCALE) {
+    return f32x2_to_bf16_bits(fmaf(bf16_bits_to_f32(in1 & 0xffffu), scale, y0), fmaf(__uint_as_float(in1 & 0xffff0000u), scale, y1));
+  } else {
+    static_assert(POST == TPPX_POST_NONE, "the other post-ops go through apply_post_bits");
+    return yb;
   }
 }
 

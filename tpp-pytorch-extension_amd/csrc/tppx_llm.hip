@@ -46,7 +46,7 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   uint32_t d[4];
 #pragma unroll
   for (int i = 0; i < 4; i++)
-    d[i] = f32_to_bf16_bits(f[2 * i]) | (f32_to_bf16_bits(f[2 * i + 1]) << 16);
+    d[i] = f32x2_to_bf16_bits(f[2 * i], f[2 * i + 1]);
   return make_uint4(d[0], d[1], d[2], d[3]);
 }
 
@@ -1051,8 +1051,7 @@ attn_prefill_kernel(const AttnPrefillParams p) {
         uint32_t w[2];
 #pragma unroll
         for (int h = 0; h < 2; h++)
-          w[h] = f32_to_bf16_bits(ls > 0.f ? acc[qg][dt][2 * h] / ls : 0.f) |
-                 (f32_to_bf16_bits(ls > 0.f ? acc[qg][dt][2 * h + 1] / ls : 0.f) << 16);
+          w[h] = f32x2_to_bf16_bits(ls > 0.f ? acc[qg][dt][2 * h] / ls : 0.f, ls > 0.f ? acc[qg][dt][2 * h + 1] / ls : 0.f);
         *reinterpret_cast<uint2*>(orow + dt * 16 + g * 4) = make_uint2(w[0], w[1]);
       }
     }
@@ -1259,8 +1258,7 @@ attn_prefill_hd_kernel(const AttnPrefillParams p) {
           uint32_t w[2];
 #pragma unroll
           for (int h = 0; h < 2; h++)
-            w[h] = f32_to_bf16_bits(ls > 0.f ? acc[qg][dt][2 * h] / ls : 0.f) |
-                   (f32_to_bf16_bits(ls > 0.f ? acc[qg][dt][2 * h + 1] / ls : 0.f) << 16);
+            w[h] = f32x2_to_bf16_bits(ls > 0.f ? acc[qg][dt][2 * h] / ls : 0.f, ls > 0.f ? acc[qg][dt][2 * h + 1] / ls : 0.f);
           *reinterpret_cast<uint2*>(orow + dt * 16 + g * 4) = make_uint2(w[0], w[1]);
         }
       }

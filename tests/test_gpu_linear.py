@@ -995,6 +995,24 @@ def test_prefill_bf16_every_workgroup_tile_ragged(tile, w8, M, N, K, monkeypatch
     assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws[:4], bs), got[2:]))
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 16, 256), (64 * 3, 272, 512), (129, 4080, 768), (300, 8208, 1024), (1000, 1040, 1280)])
+def test_prefill_qint8_forms_agree_with_the_oracle(M, N, K, monkeypatch):
+    """The large-M QINT8 kernel from one K step to five (odd and even: its loop goes by two), a single channel tile, ragged
+    rows and channel blocks: 64 x 128, 64 x 256 and 128 x 256 workgroups as the launch picks them against the oracle, and the
+    bits of the 128 x 256 form, for the GEMM with its residual and for the gate/up pair."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    y, _, _, ctx = _run("qint8", M, N, K, "add", True, 900 + M, flags=_lib.FLAG_FORCE_TILED)
+    qw, _, _, x, bias, in1, in2, scale = ctx
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")
+    wu = _make("qint8", N, K, 901 + M)[0]
+    pair = ops.swiglu_gate_up(x.cuda(), qw, wu, bias.cuda(), None)
+    assert torch.equal(pair, ops.fc_mul(x.cuda(), wu, None, ops.fc_silu(x.cuda(), qw, bias.cuda())))
+    monkeypatch.setenv("TPPX_TILED_SMALL", "0")
+    assert torch.equal(y, ops.linear(x.cuda(), qw, bias.cuda(), O.POST_ADD_SCALE, in1.cuda(), None, scale))
+    assert torch.equal(pair, ops.swiglu_gate_up(x.cuda(), qw, wu, bias.cuda(), None))
+
+
 @pytest.mark.parametrize("fmt", ["qint8", "qint4"])
 @pytest.mark.parametrize("M,N,K", [(65, 160, 256), (129, 544, 512), (300, 96, 768), (200, 2080, 1280), (1000, 4160, 512)])
 def test_prefill_qint8_pair_agrees_with_two_launches(fmt, M, N, K, monkeypatch):

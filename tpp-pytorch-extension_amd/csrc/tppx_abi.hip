@@ -278,24 +278,42 @@ static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, boo
   return tiled * margin <= rows_us((dual ? DUAL : SINGLE)[nt - 1], (tiles + nt - 1) / nt * rows64, K);
 }
 
-// QINT8 (128 x 256 tiles, one workgroup per CU; at most 128 of them: twice as many of 64 x 256).  `tiles` of the whole
-// launch.  The gate/up pair (dual) stands against two launches behind a quantizer each; where those would be decode
-// launches of few rounds, they win: 2 x 1024 x 3584 at 200 rows 22 us against 28.
-static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, bool dual) {
+// QINT8.  `tiles` of the whole launch.
+// The gate/up pair (dual) stands against two launches behind a quantizer each, on figures of an earlier form of the tiles
+// (128 x 256, at most 128 of them twice as many of 64 x 256; blocks other than 256 wide still go by them).
+static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, bool dual, int64_t qbs) {
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
     return family == BY_TILES;
-  const int64_t rows64 = (M + 63) / 64, wgs = ((M + 127) / 128) * ((tiles + 15) / 16);
+  const int64_t rows64 = (M + 63) / 64;
+  static constexpr RowsCost ROWS[3] = {{4.62, 2.33, 1.35}, {5.38, 4.48, 1.55}, {5.14, 5.03, 2.41}};
+  auto row_tiles = [](int64_t one) { return one < 512 ? 1 : one > 512 && one <= 768 ? 3 : 2; }; // as plan_skinny
+  if (!dual && qbs == 256 && M >= big_min_rows() && env_int("TPPX_TILED_BIG_QINT8", 1) != 0 && env_int("TPPX_TILED_SMALL", 1) != 0) {
+    // With half the CUs' worth of 64 x 256 workgroups and more the tiles were the faster side of every one of 682 shapes
+    // (65 .. 1000 rows, 512 .. 28672 channels, K 1024 .. 18944: up to four times).  Launches of fewer run as 64 x 128, in one
+    // round, against the decode kernels' rounds; both sides in us, the quantizer included, within 5 % on average: the choice
+    // is 0.02 % off the faster one, 7 % at worst (the fit before, to the earlier form of the tiles: 8.6 %, 132 %).
+    // (K up to 1024: both at what a launch takes, 8.5 .. 9.1 us)
+    if (K <= 1024 || rows64 * ((tiles + 15) / 16) >= 128)
+      return true;
+    const int nt = row_tiles(tiles);
+    const double k = 1e-3 * (double)K, wgs = (double)(rows64 * ((tiles + 7) / 8)), mk = 1e-6 * (double)M * (double)K;
+    static constexpr RowsCost R[3] = {{4.9, 2.26, 1.25}, {4.4, 3.96, 1.6}, {5.5, 4.25, 2.3}};
+    return 6.6 + k * (2.33 + 0.80 * wgs / 256.0) + 0.3 * mk <= rows_us(R[nt - 1], (tiles + nt - 1) / nt * rows64, K) + 0.8 * mk;
+  }
+  const int64_t wgs = ((M + 127) / 128) * ((tiles + 15) / 16);
   const bool small = wgs <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0;
   const double tiled_us = small ? 8.0 + (double)K * 0.006 : (double)((wgs + 255) / 256) * (10.0 + (double)K * 0.0075);
-  if (dual && !want_tiled_qint8(M, K, flags, tiles / 2, false)) {
-    static constexpr RowsCost ROWS[3] = {{4.62, 2.33, 1.35}, {5.38, 4.48, 1.55}, {5.14, 5.03, 2.41}};
-    const int64_t one = tiles / 2;
-    const int nt = one < 512 ? 1 : one > 512 && one <= 768 ? 3 : 2; // as plan_skinny
-    if (tiled_us > 1.15 * 2.0 * rows_us(ROWS[nt - 1], (one + nt - 1) / nt * rows64, K))
+  auto by_block_rows = [&](double us, int64_t n) { return us <= (double)rows64 * (5.0 + (double)n * 16.0 * (double)K / 5.5e6 + (double)K * 0.0004); };
+  if (dual) {
+    const int64_t one = tiles / 2, wgs1 = ((M + 127) / 128) * ((one + 15) / 16);
+    const double one_us = wgs1 <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0 ? 8.0 + (double)K * 0.006
+                                                                              : (double)((wgs1 + 255) / 256) * (10.0 + (double)K * 0.0075);
+    const int nt = row_tiles(one);
+    if (!by_block_rows(one_us, one) && tiled_us > 1.15 * 2.0 * rows_us(ROWS[nt - 1], (one + nt - 1) / nt * rows64, K))
       return false;
   }
-  return tiled_us <= (double)rows64 * (5.0 + (double)tiles * 16.0 * (double)K / 5.5e6 + (double)K * 0.0004);
+  return by_block_rows(tiled_us, tiles);
 }
 
 // Unquantized bf16 weights: n of them as one launch of the large-M kernel against one decode launch each
@@ -558,7 +576,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
   p.units = (int)(K / (64 * p.deal));
   p.spb_magic = (p.deal == 4 && p.tpb > 4) ? (unsigned int)((((uint64_t)1 << 32) + (uint64_t)(p.tpb / 4) - 1) / (uint64_t)(p.tpb / 4)) : 0u;
   const bool reuse = (flags & TPPX_FLAG_XQ_REUSE) != 0; // xq / sa still hold this x, quantized by an earlier call
-  const bool tiled = qbs % 128 == 0 && want_tiled_qint8(M, K, flags, (dual ? 2 : 1) * (int64_t)p.total_tiles, dual);
+  const bool tiled = qbs % 128 == 0 && want_tiled_qint8(M, K, flags, (dual ? 2 : 1) * (int64_t)p.total_tiles, dual, qbs);
   TiledParams t[TPPX_MAX_SEGS];
   bool group = tiled && n_segs > 1; // one grid over the channel blocks of all GEMMs when the large-M kernel takes them
   for (int i = 0; i < n_segs && tiled; i++) {
@@ -830,7 +848,7 @@ extern "C" int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M
       return 0;
     tiles[i] = t.tiles;
   }
-  return weight_bytes == 1 ? want_tiled_qint8(M, K, 0, 2 * tiles[0], true) : want_tiled_bf16(M, K, 0, tiles, n_segs);
+  return weight_bytes == 1 ? want_tiled_qint8(M, K, 0, 2 * tiles[0], true, 256) : want_tiled_bf16(M, K, 0, tiles, n_segs);
 }
 
 extern "C" int tppx_multi_linear_bf16(const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,

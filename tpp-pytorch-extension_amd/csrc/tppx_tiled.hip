@@ -441,23 +441,26 @@ tiled_qint8_kernel(const TiledParams p) {
 // the first sum is staged (requested in the loop, each of 16 rounds waited for memory).  QINT8 4096 x 4096 with residual
 // at 1000 / 2048 rows 33.1 -> 28.7 / 51.6 -> 44.0 us, 11008 x 4096 at 1000 rows 87.8 -> 71.5; a four-layer prompt on bf16
 // weights at 2048 tokens 3478 -> 3277, MXFP4 at 333 989 -> 919.
-constexpr int EP_LD = 68; // floats per staged row: 64 + 4 keeps the 4-row lane groups on distinct banks
-template <int MT, int POST> // POST < 0: whatever p.post_op says
-__device__ __forceinline__ void big_epilogue_post(const TiledParams& p, f32x4 (&acc)[MT][4], float* stage, int m_base,
+constexpr int EP_LD = 68; // floats per staged row of 64 channels: 64 + 4 keeps the 4-row lane groups on distinct banks
+constexpr int ep_ld(int nt) { return nt * 16 + 4; }
+template <int MT, int POST, int NT> // POST < 0: whatever p.post_op says; NT = 16-channel tiles of the wave tile (4 or 2)
+__device__ __forceinline__ void big_epilogue_post(const TiledParams& p, f32x4 (&acc)[MT][NT], float* stage, int m_base,
                                                   int tile_base) {
   constexpr bool INPUT = POST == TPPX_POST_MUL || POST == TPPX_POST_ADD_SCALE;
   const int lane = threadIdx.x & 63;
-  const int cx = (lane & 7) * 8; // first of this lane's 8 channels inside the wave tile
+  constexpr int LPR = NT * 2, RPI = 64 / LPR, LD = ep_ld(NT); // lanes per row, rows per wave instruction
+  const int cx = (lane % LPR) * 8; // first of this lane's 8 channels inside the wave tile
   const int tile = tile_base + (cx >> 4);
   const bool tile_ok = tile < p.tiles;
   const int n = min(tile, p.tiles - 1) * 16 + (cx & 15);
   constexpr int MH = MT < 4 ? MT : 4; // row tiles staged at a time (64 rows, or the whole wave tile when it has fewer)
   // every input of the post-op is requested before the first sum is staged (rows past the end read the last one)
-  uint4 in[INPUT ? MT * 2 : 1];
+  constexpr int NI = MH * 16 / RPI;
+  uint4 in[INPUT ? MT / MH * NI : 1];
   if constexpr (INPUT) {
 #pragma unroll
-    for (int it = 0; it < MT * 2; it++)
-      in[it] = *reinterpret_cast<const uint4*>(p.post_in + (int64_t)min(m_base + it * 8 + (lane >> 3), p.M - 1) * p.N + n);
+    for (int it = 0; it < MT / MH * NI; it++)
+      in[it] = *reinterpret_cast<const uint4*>(p.post_in + (int64_t)min(m_base + it * RPI + lane / LPR, p.M - 1) * p.N + n);
   }
   float bias[8];
 #pragma unroll
@@ -468,20 +471,20 @@ __device__ __forceinline__ void big_epilogue_post(const TiledParams& p, f32x4 (&
 #pragma unroll
     for (int mt = 0; mt < MH; mt++)
 #pragma unroll
-      for (int nt = 0; nt < 4; nt++)
+      for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          stage[(mt * 16 + (lane >> 4) * 4 + r) * EP_LD + nt * 16 + (lane & 15)] = acc[h * MH + mt][nt][r];
+          stage[(mt * 16 + (lane >> 4) * 4 + r) * LD + nt * 16 + (lane & 15)] = acc[h * MH + mt][nt][r];
     // same wave wrote and reads: no barrier, the compiler orders the LDS accesses
     auto rows8 = [&](int it) {
-      const int row = it * 8 + (lane >> 3);
+      const int row = it * RPI + lane / LPR;
       const int m = m_base + h * (MH * 16) + row;
-      const f32x4 v0 = *reinterpret_cast<const f32x4*>(stage + row * EP_LD + cx);
-      const f32x4 v1 = *reinterpret_cast<const f32x4*>(stage + row * EP_LD + cx + 4);
+      const f32x4 v0 = *reinterpret_cast<const f32x4*>(stage + row * LD + cx);
+      const f32x4 v1 = *reinterpret_cast<const f32x4*>(stage + row * LD + cx + 4);
       const int64_t o = (int64_t)m * p.N + n;
       uint32_t out[4];
       if constexpr (POST >= 0) {
-        const uint4 i1 = INPUT ? in[INPUT ? h * (MH * 2) + it : 0] : make_uint4(0, 0, 0, 0);
+        const uint4 i1 = INPUT ? in[INPUT ? h * NI + it : 0] : make_uint4(0, 0, 0, 0);
         const uint32_t w1[4] = {i1.x, i1.y, i1.z, i1.w};
 #pragma unroll
         for (int e = 0; e < 4; e++)
@@ -509,35 +512,36 @@ __device__ __forceinline__ void big_epilogue_post(const TiledParams& p, f32x4 (&
     };
     if constexpr (POST >= 0) {
 #pragma unroll
-      for (int it = 0; it < MH * 2; it++)
+      for (int it = 0; it < NI; it++)
         rows8(it);
     } else {
-      for (int it = 0; it < MH * 2; it++)
+      for (int it = 0; it < NI; it++)
         rows8(it);
     }
   }
 }
 
-template <int MT>
-__device__ __forceinline__ void big_epilogue(const TiledParams& p, f32x4 (&acc)[MT][4], float* stage, int m_base,
+template <int MT, int NT = 4>
+__device__ __forceinline__ void big_epilogue(const TiledParams& p, f32x4 (&acc)[MT][NT], float* stage, int m_base,
                                              int tile_base) {
   switch (p.post_op) {
-  case TPPX_POST_NONE: return big_epilogue_post<MT, TPPX_POST_NONE>(p, acc, stage, m_base, tile_base);
-  case TPPX_POST_SILU: return big_epilogue_post<MT, TPPX_POST_SILU>(p, acc, stage, m_base, tile_base);
-  case TPPX_POST_MUL: return big_epilogue_post<MT, TPPX_POST_MUL>(p, acc, stage, m_base, tile_base);
-  case TPPX_POST_ADD_SCALE: return big_epilogue_post<MT, TPPX_POST_ADD_SCALE>(p, acc, stage, m_base, tile_base);
-  default: return big_epilogue_post<MT, -1>(p, acc, stage, m_base, tile_base);
+  case TPPX_POST_NONE: return big_epilogue_post<MT, TPPX_POST_NONE, NT>(p, acc, stage, m_base, tile_base);
+  case TPPX_POST_SILU: return big_epilogue_post<MT, TPPX_POST_SILU, NT>(p, acc, stage, m_base, tile_base);
+  case TPPX_POST_MUL: return big_epilogue_post<MT, TPPX_POST_MUL, NT>(p, acc, stage, m_base, tile_base);
+  case TPPX_POST_ADD_SCALE: return big_epilogue_post<MT, TPPX_POST_ADD_SCALE, NT>(p, acc, stage, m_base, tile_base);
+  default: return big_epilogue_post<MT, -1, NT>(p, acc, stage, m_base, tile_base);
   }
 }
 
-// The gate/up pair: the wave tile's channels 0..31 are gate sums and 32..63 the up sums of the SAME 32 output
-// channels, so silu(gate) * up is formed here, with the rounding points of SiluPostOp followed by MulPostOp, and
-// only the product is written: a lane finishes 8 adjacent channels of one row (16-byte store, four lanes per row).
-template <int MT>
-__device__ __forceinline__ void big_epilogue_dual(const TiledParams& pg, const TiledParams& pu, f32x4 (&acc)[MT][4],
+// The gate/up pair: the first half of the wave tile's channels are gate sums and the second the up sums of the SAME
+// output channels, so silu(gate) * up is formed here, with the rounding points of SiluPostOp followed by MulPostOp, and
+// only the product is written: a lane finishes 8 adjacent channels of one row (16-byte store, NT lanes per row).
+template <int MT, int NT = 4>
+__device__ __forceinline__ void big_epilogue_dual(const TiledParams& pg, const TiledParams& pu, f32x4 (&acc)[MT][NT],
                                                   float* stage, int m_base, int tile_base) {
   const int lane = threadIdx.x & 63;
-  const int cx = (lane & 3) * 8; // first of this lane's 8 channels among the wave's 32
+  constexpr int LPR = NT, RPI = 64 / LPR, LD = ep_ld(NT);
+  const int cx = (lane % LPR) * 8; // first of this lane's 8 channels among the wave's NT * 8
   const int tile = tile_base + (cx >> 4);
   const bool tile_ok = tile < pg.tiles;
   const int n = min(tile, pg.tiles - 1) * 16 + (cx & 15);
@@ -553,19 +557,19 @@ __device__ __forceinline__ void big_epilogue_dual(const TiledParams& pg, const T
 #pragma unroll
     for (int mt = 0; mt < MH; mt++)
 #pragma unroll
-      for (int nt = 0; nt < 4; nt++)
+      for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          stage[(mt * 16 + (lane >> 4) * 4 + r) * EP_LD + nt * 16 + (lane & 15)] = acc[h * MH + mt][nt][r];
+          stage[(mt * 16 + (lane >> 4) * 4 + r) * LD + nt * 16 + (lane & 15)] = acc[h * MH + mt][nt][r];
     // same wave wrote and reads: no barrier, the compiler orders the LDS accesses
 #pragma unroll
-    for (int it = 0; it < MH; it++) {
-      const int row = it * 16 + (lane >> 2);
+    for (int it = 0; it < MH * 16 / RPI; it++) {
+      const int row = it * RPI + lane / LPR;
       const int m = m_base + h * (MH * 16) + row;
-      const f32x4 g0 = *reinterpret_cast<const f32x4*>(stage + row * EP_LD + cx);
-      const f32x4 g1 = *reinterpret_cast<const f32x4*>(stage + row * EP_LD + cx + 4);
-      const f32x4 u0 = *reinterpret_cast<const f32x4*>(stage + row * EP_LD + 32 + cx);
-      const f32x4 u1 = *reinterpret_cast<const f32x4*>(stage + row * EP_LD + 32 + cx + 4);
+      const f32x4 g0 = *reinterpret_cast<const f32x4*>(stage + row * LD + cx);
+      const f32x4 g1 = *reinterpret_cast<const f32x4*>(stage + row * LD + cx + 4);
+      const f32x4 u0 = *reinterpret_cast<const f32x4*>(stage + row * LD + NT * 8 + cx);
+      const f32x4 u1 = *reinterpret_cast<const f32x4*>(stage + row * LD + NT * 8 + cx + 4);
       if (tile_ok && m < pg.M) {
         uint32_t out[4];
 #pragma unroll
@@ -1039,63 +1043,57 @@ big_mxfp4_kernel(const BigParams P) {
 }
 
 // ---------------------------------------------------------------------------
-// Large-M QINT8 (W8A8, 256-wide blocks): 128 x 256 workgroup tile, 8 waves
-// (2 x 4), wave tile 64 x 64, K step 256 = one scale block.
-// What bounds int8 at this size is operand delivery and the fold, not the
-// MFMA: weights are 4x the bytes of MXFP4 per MAC, the MFMA runs at twice the
-// bf16 rate, and every block's int32 sums have to be converted, scaled by
-// sa[m] * sw[n] and added to the fp32 sums: 3 vector instructions per output
-// and block, 3 per MFMA.  Measured on this part, an int8 MFMA holds its SIMD's
-// vector issue for about 8 cycles and any other vector instruction for 4,
-// whichever wave they come from (16.5 / 17.5 / 18 / 21.5 / 25.5 cycles per MFMA
-// with 0 / 1 / 2 / 3 / 4 independent fp32 instructions behind each), so the
-// fold alone caps the MFMA busy fraction near 0.73.  So:
-//   * BOTH operands go from global memory straight into LDS (no staging
-//     registers, nothing for the compiler to wait on before the barrier) and
-//     every weight tile is fetched once per workgroup instead of once per wave
-//     row.  A: int8 rows, 256 B per row and step, the layout, swizzle and
-//     operand reads of the MXFP4 kernel above (operand of MFMA step j = chunk
-//     j*4 + g of the row), two buffers.  B: native 1 KiB tiles (lane-linear =
-//     operand order), 16 tiles x 4 K tiles = 64 KiB, ONE buffer: at the start
-//     of a step every wave copies its 16 operands into registers, a barrier
-//     frees the buffer and the next step's tiles stream in during the MFMAs.
-//   * The MFMAs of a step run row tile by row tile (all of K for 16 rows, then
-//     the next 16), into one of two small sets of int32 sums, and the fold of
-//     row tile mt sits between the first and the second MFMA group of row tile
-//     mt + 1: vector and matrix work overlap inside a wave, and the two waves
-//     of a SIMD do not fold at the same moment.  The first MFMA of a row tile
-//     starts from a zero operand.
-//   * Activation scales reach the waves through LDS, requested two steps ahead.
-// LDS: A 2 x 32 KiB | B 64 KiB | scales 2 KiB (the epilogue staging reuses it).
+// Large-M QINT8 (W8A8, 256-wide blocks): W waves side by side, each with a wave tile of MT*16 rows x 32 channels, K step
+// 256 = one scale block.  What bounds int8 at this size is the LDS and the fold, not the MFMA: a CU's LDS hands out
+// 128 B/clk and takes in about half of that, the int8 MFMA runs at twice the bf16 rate, and every block's int32 sums
+// have to be converted, scaled by sa[m] * sw[n] and added to the fp32 sums -- 3 vector instructions per output and block,
+// 3 per MFMA, each of which stretches an MFMA's 16 cycles by about 4 (16.5 / 17.5 / 18 / 21.5 / 25.5 cycles with
+// 0 / 1 / 2 / 3 / 4).  So:
+//   * Weights never see the LDS: a wave owns its channels, so it loads their native tiles into registers, a whole step
+//     ahead (two sets of 32 registers, the loop unrolled by two).  The form before brought both operands through LDS:
+//     256 KB of operand reads and 96 KB of writes per step of a 128 x 256 workgroup, against 256 and 32 now, and a phase
+//     of copying and a second barrier in every step.
+//   * Activation rows and their scales go straight into LDS, two steps ahead in a ring of three stages; the bank swizzle
+//     sits on the source side (the lane at position c of row m fetches chunk c ^ (m & 15)).  One barrier per step.
+//   * All loads are buffer loads: the addresses are scalar, and the compiler counts them exactly beside the loads into
+//     LDS (flat-addressed loads into LDS make it wait for everything).  Order per step: the next step's weights, then the
+//     rows two steps ahead, one or two behind each MFMA step; loads return in order, so "at most LA + LB younger" is the
+//     wait for a stage.
+//   * The MFMAs run by groups of two row tiles (four sums of 16 x 16, all of K for them, then the next group), and the
+//     fold of a group sits between the MFMAs of the next one, that of a step's last group under the next step's first
+//     operand reads.
+// Forms (the same sums in the same order, the same bits): 128 x 256 and 64 x 256 of eight waves, 64 x 128 of four.
+// Measured, without the quantizer, against that earlier form, at 70 / 333 / 1000 / 2048 rows: 4096 x 4096 with residual
+// 23.8 / 24.7 / 29.1 / 44.4 -> 13.7 / 15.0 / 24.5 / 43.0 us, 4096 x 11008 59.3 / 60.7 / 69.9 / 106 -> 30.6 / 31.9 / 56.2 /
+// 97 us, pair 2 x 4096 x 11008 at 333 / 1000 rows 65 / 103 -> 49 / 94; 2.0 POP/s at 2048 rows.
+// DUAL: the gate/up pair: a wave's two channel tiles are a gate tile and the up tile of the same channels, silu(gate) * up
+// in the epilogue.  A launch per weight rounds its workgroups up to whole rounds of 256 twice, quantizes the rows twice
+// and takes the gate matrix out to memory and back.
 // ---------------------------------------------------------------------------
-template <int N>
-__device__ __forceinline__ void lds_wait_keep16(i32x4 (&b)[4][4]) {
-  asm volatile("s_waitcnt lgkmcnt(%16)"
-               : "+v"(b[0][0]), "+v"(b[0][1]), "+v"(b[0][2]), "+v"(b[0][3]), "+v"(b[1][0]), "+v"(b[1][1]), "+v"(b[1][2]),
-                 "+v"(b[1][3]), "+v"(b[2][0]), "+v"(b[2][1]), "+v"(b[2][2]), "+v"(b[2][3]), "+v"(b[3][0]), "+v"(b[3][1]),
-                 "+v"(b[3][2]), "+v"(b[3][3])
-               : "n"(N));
+template <int MT, int W>
+struct Qint8Geom {
+  static constexpr int WGM = MT * 16, NB = 3;
+  static constexpr int SA_OFF = WGM * 256;
+  static constexpr int STAGE = SA_OFF + WGM * 4;
+  static constexpr int NA = MT * 4 / W;              // 4-row pieces of A a wave fetches per step
+  static constexpr int LA = NA + 1, LB = 10;     // loads per wave and step: rows + their scales; weights + their scales
+  static constexpr size_t EP = (size_t)W * (MT < 4 ? MT * 16 : 64) * ep_ld(2) * sizeof(float);
+  static constexpr size_t LDS = (size_t)NB * STAGE > EP ? (size_t)NB * STAGE : EP;
+};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tl_rsrc(const void* q) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(q), 0, 0xffffffffu, 0x00020000);
 }
 
-// MT = row tiles of 16 per wave: 4 (workgroup 128 x 256) or 2 (64 x 256, for launches that leave CUs empty).
-// DUAL: the gate/up pair, 128 output channels per workgroup: the 16 weight tiles of a step are 4 x (2 gate tiles, the 2
-// up tiles of the same channels), silu(gate) * up in the epilogue.  Same sums in the same order as a launch per weight.
-// A launch per weight rounds its workgroups up to whole rounds of 256 twice, quantizes the rows twice and takes the gate
-// matrix out to memory and back: 2 x 11008 x 4096 at 1000 rows is 2 + 2 rounds against 3, 71 us less per SwiGLU block
-// (prompt pass of four layers 2074 -> 1791 us).
-template <int MT, bool DUAL>
+template <int MT, int W, bool DUAL>
 __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
-  constexpr int WGM = MT * 32, ABUF = WGM * 256, BBUF = 64 * 1024;
+  using G = Qint8Geom<MT, W>;
+  constexpr int WGM = G::WGM, NB = G::NB, NA = G::NA, LA = G::LA, LB = G::LB, STAGE = G::STAGE;
   extern __shared__ __align__(16) uint8_t tl_lds[];
-  uint8_t* b_lds = tl_lds + 2 * ABUF;
-  float* sa_s = reinterpret_cast<float*>(tl_lds + 2 * ABUF + BBUF); // [4][128]: scales of steps ks .. ks+2 (mod 4)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
   const int MB = (P.seg[0].M + WGM - 1) / WGM;
   int bm, bn;
   tile_of_block(MB, P.nb0[P.n_seg], bm, bn);
-  // several GEMMs over one activation (fused q/k/v) share the launch: pick this block's with uniform selects
   TiledParams p = P.seg[0];
   int nb_first = 0;
   if (!DUAL) {
@@ -1107,18 +1105,46 @@ __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
       }
   }
   bn -= nb_first;
-  const int KS = p.K >> 8;   // K steps = scale blocks
-  const int KT64 = p.K >> 6; // native tiles along K
+  const int KS = p.K >> 8;
   const int m_wg = bm * WGM;
-  const int tile_base = DUAL ? bn * 8 + wn * 2 : bn * 16 + wn * 4;
+  const int tile_base = DUAL ? bn * W + wave : bn * (W * 2) + wave * 2; // DUAL: gate and up tile of the same 16 channels
 
-  const float* swp = reinterpret_cast<const float*>(p.sw);
-  const float* swp2 = reinterpret_cast<const float*>(DUAL ? P.seg[1].sw : p.sw); // of tiles 2, 3
-  uint32_t soff[4];
+  const auto xr = tl_rsrc(p.xq), sar = tl_rsrc(p.sa);
+  uint32_t aoff[NA];
 #pragma unroll
-  for (int nt = 0; nt < 4; nt++)
-    soff[nt] = (uint32_t)(min(tile_base + (DUAL ? nt & 1 : nt), p.tiles - 1) * KS * 16 + (lane & 15));
-  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(tl_lds);
+  for (int i = 0; i < NA; i++) {
+    const int blk = wave * NA + i, r16 = (blk & 3) * 4 + (lane >> 4);
+    aoff[i] = (uint32_t)min(m_wg + blk * 4 + (lane >> 4), p.M - 1) * (uint32_t)p.K + (uint32_t)(((lane & 15) ^ r16) & 15) * 16u;
+  }
+  const int sp = wave % (WGM / 64);
+  const uint32_t saoff = (uint32_t)(min(m_wg + sp * 64 + lane, p.M - 1) * KS) * 4u;
+  auto load_a = [&](auto I, int s, int buf) {
+    constexpr int i = decltype(I)::value;
+    uint8_t* base = tl_lds + buf * STAGE;
+    if constexpr (i < NA)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(base + (wave * NA + i) * 1024), 16, aoff[i], s * 256, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(sar, (__attribute__((address_space(3))) void*)(base + G::SA_OFF + sp * 256), 4, saoff, s * 4, 0, 0);
+  };
+  __amdgpu_buffer_rsrc_t wr[2], swr[2];
+  uint32_t woff[2], swoff[2];
+#pragma unroll
+  for (int nt = 0; nt < 2; nt++) {
+    const int tile = min(DUAL ? tile_base : tile_base + nt, p.tiles - 1);
+    wr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].qw : p.qw);
+    swr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].sw : p.sw);
+    woff[nt] = ((uint32_t)tile * (uint32_t)(KS * 4) * 64u + (uint32_t)lane) * 16u;
+    swoff[nt] = (uint32_t)(tile * KS * 16 + (lane & 15)) * 4u;
+  }
+  i32x4 b[2][4][2]; // [set][j][nt]
+  float swv[2][2];
+  auto load_b = [&](auto I, int s, auto SET) {
+    constexpr int i = decltype(I)::value, set = decltype(SET)::value;
+    if constexpr (i < 8)
+      b[set][i >> 1][i & 1] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[i & 1], woff[i & 1] + (i >> 1) * 1024, s * 4096, 0));
+    else
+      swv[set][i & 1] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(swr[i & 1], swoff[i & 1], s * 64, 0));
+  };
   uint32_t rdb[4];
   {
     const int m = lane & 15, g = lane >> 4;
@@ -1126,168 +1152,139 @@ __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
     for (int j = 0; j < 4; j++)
       rdb[j] = (uint32_t)((m >> 2) * 1024 + (m & 3) * 256 + (((j * 4 + g) ^ m) & 15) * 16);
   }
-  const char* xbase = reinterpret_cast<const char*>(p.xq);
-  const int rin = lane >> 4, ch = lane & 15;
-  const bool full = m_wg + WGM <= p.M;
-  const uint32_t xrow0 = (uint32_t)((m_wg + wave * (MT * 4) + rin) * p.K);
-  const uint32_t blk_stride = (uint32_t)(4 * p.K);
-  auto load_a_one = [&](auto I, int ks, int buf) {
-    constexpr int i = decltype(I)::value;
-    // row of this block inside its 16-row tile: the wave's first block is a multiple of 4 only with four row tiles
-    const uint32_t sw = (uint32_t)((ch ^ (((wave * MT + i) & 3) * 4 + rin)) & 15) * 16u;
-    uint32_t off;
-    if (full) {
-      off = xrow0 + (uint32_t)i * blk_stride + sw + (uint32_t)ks * 256u;
-    } else {
-      const int row = min(m_wg + (wave * MT + i) * 4 + rin, p.M - 1);
-      off = (uint32_t)(row * p.K) + sw + (uint32_t)ks * 256u;
-    }
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xbase + (size_t)off),
-                                     (__attribute__((address_space(3))) void*)(tl_lds + buf * ABUF + (wave * MT + i) * 1024),
-                                     16, 0, 0);
-  };
-  auto load_a = [&](int ks, int buf) { static_for<0, MT>([&](auto I) { load_a_one(I, ks, buf); }); };
-  // B of step ks: this wave brings tiles 2*wave, 2*wave + 1 of the 16, all four K tiles; LDS slot (tile*4 + kt) KiB
-  // (DUAL: a wave's two slots are both gate's or both up's)
-  const char* qwb = reinterpret_cast<const char*>(DUAL && (wave & 1) ? P.seg[1].qw : p.qw);
-  uint32_t bsrc[2];
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-    bsrc[i] = (uint32_t)(min(DUAL ? bn * 8 + (wave >> 1) * 2 + i : bn * 16 + wave * 2 + i, p.tiles - 1) * KT64 * 64 + lane);
-  auto load_b_one = [&](auto I, int ks) {
-    constexpr int i = decltype(I)::value >> 2, kt = decltype(I)::value & 3;
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void*)(qwb + (size_t)((bsrc[i] + (uint32_t)(ks * 4 + kt) * 64u) * 16u)),
-        (__attribute__((address_space(3))) void*)(b_lds + ((wave * 2 + i) * 4 + kt) * 1024), 16, 0, 0);
-  };
-  auto load_b = [&](int ks) { static_for<0, 8>([&](auto I) { load_b_one(I, ks); }); };
-  // activation scales: thread t < 128 carries the scale of row t for the step two ahead
-  const float* sarow = p.sa + (int64_t)min(m_wg + (tid & 127), p.M - 1) * KS;
-  float sareg = 0.f;
-  float swv[4], swn[4];
-
-  f32x4 facc[MT][4];
-  i32x4 iacc[2][4]; // block sums of the row tile in flight and of the one being folded
+  constexpr int NG = MT / 2, NQ = NG * 4; // groups of two row tiles; MFMA steps of a K step
+  f32x4 facc[MT][2];
+  i32x4 iacc[2][4];  // [group parity][row tile of the group * 2 + nt]
+  f32x4 sav[2][2];   // [group parity][row tile]
+  float swp[2] = {0.f, 0.f}; // channel scales of the step before
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++)
+    for (int nt = 0; nt < 2; nt++)
       facc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++)
-      iacc[i][nt] = i32x4{0, 0, 0, 0};
-
-  load_a(0, 0);
-  load_b(0);
-#pragma unroll
-  for (int nt = 0; nt < 4; nt++)
-    swn[nt] = (nt < 2 ? swp : swp2)[soff[nt]];
-  if (tid < WGM) {
-    sa_s[tid] = sarow[0];
-    if (KS > 1)
-      sa_s[128 + tid] = sarow[1];
-    sareg = KS > 2 ? sarow[2] : 0.f;
+  for (int i = 0; i < 4; i++) {
+    iacc[0][i] = iacc[1][i] = i32x4{0, 0, 0, 0};
+    sav[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  __syncthreads();
-  const uint32_t bwave = lds0 + (uint32_t)(2 * ABUF + wn * 16 * 1024) + (uint32_t)lane * 16u; // this wave's 4 tiles
-  // One K step.  MORE: the next step's tiles are requested one wave instruction at a time behind the MFMA groups
-  // (in one burst, a wave stands at its load instructions while the memory pipeline's queue drains).
-  auto step = [&](auto MORE, int ks) {
-    constexpr bool more = decltype(MORE)::value;
-    const int buf = ks & 1;
-    // this step's weight operands: LDS -> registers, then the buffer is free for the next step's tiles
-    i32x4 bq[4][4]; // [tile][MFMA step j]
-    static_for<0, 16>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      lds_read_b128_async<i * 1024>(bq[i >> 2][i & 3], bwave);
+  const int last = KS - 1;
+  // (in this order: the waits count the loads behind those they wait for)
+  static_for<0, LA>([&](auto I) { load_a(I, 0, 0); });
+  __builtin_amdgcn_sched_barrier(0);
+  static_for<0, LB>([&](auto I) { load_b(I, 0, std::integral_constant<int, 0>{}); });
+  __builtin_amdgcn_sched_barrier(0);
+  static_for<0, LA>([&](auto I) { load_a(I, min(1, last), 1); });
+  __builtin_amdgcn_sched_barrier(0);
+  int buf = 0;
+  // outputs e0 .. e1 (of 16) of group g's fold
+  auto fold = [&](auto GI, auto E0, auto E1, const float (&sw)[2]) {
+    constexpr int g = decltype(GI)::value;
+    static_for<decltype(E0)::value, decltype(E1)::value>([&](auto E) {
+      constexpr int e = decltype(E)::value, t = e >> 2, r = e & 3, rt = t >> 1, nt = t & 1;
+      facc[g * 2 + rt][nt][r] = fmaf((float)iacc[g & 1][t][r], sav[g & 1][rt][r] * sw[nt], facc[g * 2 + rt][nt][r]);
     });
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++)
-      swv[nt] = swn[nt];
-    if (tid < WGM && ks + 2 < KS) {
-      sa_s[((ks + 2) & 3) * 128 + tid] = sareg; // loaded two steps ago
-      sareg = ks + 3 < KS ? sarow[ks + 3] : 0.f;
-    }
-    lds_wait_keep16<0>(bq);
-    __syncthreads();
-    if constexpr (more) {
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++)
-        swn[nt] = (nt < 2 ? swp : swp2)[soff[nt] + (uint32_t)(ks + 1) * 16u];
-    }
-    const uint32_t abase = lds0 + (uint32_t)(buf * ABUF + wm * MT * 4096);
-    const float* sab = sa_s + (ks & 3) * 128 + wm * (MT * 16) + (lane >> 4) * 4;
-    auto fold = [&](auto MTI) { // facc += int32 sum * (sa[row] * sw[channel]) for row tile mt
-      constexpr int mt = decltype(MTI)::value;
-      const f32x4 sav = *reinterpret_cast<const f32x4*>(sab + mt * 16);
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++)
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          facc[mt][nt][r] = fmaf((float)iacc[mt & 1][nt][r], sav[r] * swv[nt], facc[mt][nt][r]);
-    };
-    // activation operands in order q = mt*4 + j, RD ahead of their use
-    constexpr int RD = 3, NQ = 4 * MT;
-    i32x4 ar[RD + 1];
-    static_for<0, RD>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      lds_read_b128_async<(i / 4) * 4096>(ar[i], abase + rdb[i % 4]);
-    });
-    static_for<0, NQ>([&](auto Q) {
-      constexpr int q = decltype(Q)::value;
-      constexpr int mt = q / 4, j = q % 4;
-      if constexpr (q + RD < NQ) {
-        lds_read_b128_async<((q + RD) / 4) * 4096>(ar[(q + RD) % (RD + 1)], abase + rdb[(q + RD) % 4]);
-        lds_wait_keep<RD>(ar[q % (RD + 1)]);
-      } else {
-        lds_wait_keep<NQ - 1 - q>(ar[q % (RD + 1)]);
-      }
-      const i32x4 a = ar[q % (RD + 1)];
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++)
-        iacc[mt & 1][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bq[nt][j], j == 0 ? i32x4{0, 0, 0, 0} : iacc[mt & 1][nt], 0, 0, 0);
-      if constexpr (more && q < 8)
-        load_b_one(std::integral_constant<int, q>{}, ks + 1);
-      // the MT blocks of A behind the groups after the weight tiles' (with two row tiles there are only 8 groups: behind the last MT of them)
-      constexpr int qa = NQ >= 8 + MT ? 8 : NQ - MT;
-      if constexpr (more && q >= qa && q < qa + MT)
-        load_a_one(std::integral_constant<int, q - qa>{}, ks + 1, buf ^ 1);
-      if constexpr (j == 0 && mt > 0)
-        fold(std::integral_constant<int, mt - 1>{}); // the previous row tile, under this row tile's MFMAs
-    });
-    fold(std::integral_constant<int, MT - 1>{});
-    __syncthreads();
   };
-  for (int ks = 0; ks + 1 < KS; ks++)
-    step(std::true_type{}, ks);
-  step(std::false_type{}, KS - 1);
-  float* stage = reinterpret_cast<float*>(tl_lds) + wave * 64 * EP_LD;
+  auto step = [&](auto SET, int s) {
+    constexpr int set = decltype(SET)::value;
+    asm volatile("" : : : "memory");
+    constexpr int vm = LB + LA;
+    __builtin_amdgcn_s_waitcnt((vm & 15) | 7 << 4 | vm >> 4 << 14); // A of step s has landed, reads of step s - 1 have returned
+    asm volatile("s_barrier" : : : "memory");
+    const int nbuf = buf == 0 ? NB - 1 : buf - 1;
+    const uint8_t* ab = tl_lds + buf * STAGE;
+    const float* sas = reinterpret_cast<const float*>(ab + G::SA_OFF) + (lane >> 4) * 4;
+    constexpr int RD = 2;
+    i32x4 ar[RD + 1][2];
+    auto read = [&](auto Q) {
+      constexpr int q = decltype(Q)::value, g = q >> 2, j = q & 3;
+#pragma unroll
+      for (int rt = 0; rt < 2; rt++)
+        ar[q % (RD + 1)][rt] = *reinterpret_cast<const i32x4*>(ab + (g * 2 + rt) * 4096 + rdb[j]);
+    };
+    static_for<0, RD>([&](auto Q) { read(Q); });
+    __builtin_amdgcn_sched_barrier(0);
+    fold(std::integral_constant<int, NG - 1>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 16>{}, swp);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, NQ>([&](auto Q) {
+      constexpr int q = decltype(Q)::value, g = q >> 2, j = q & 3;
+      if constexpr (q + RD < NQ)
+        read(std::integral_constant<int, q + RD>{});
+      if constexpr (j == 0) {
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+          sav[g & 1][rt] = *reinterpret_cast<const f32x4*>(sas + (g * 2 + rt) * 16);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+        iacc[g & 1][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ar[q % (RD + 1)][t >> 1], b[set][j][t & 1], j == 0 ? i32x4{0, 0, 0, 0} : iacc[g & 1][t], 0, 0, 0);
+      if constexpr (g > 0)
+        fold(std::integral_constant<int, g - 1>{}, std::integral_constant<int, j * 4>{}, std::integral_constant<int, j * 4 + 4>{}, swv[set]);
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if constexpr (g > 0)
+          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // the next step's weights, then the rows two steps ahead, a few behind each MFMA step
+      constexpr int NL = LB + LA, l0 = NL * q / NQ, l1 = NL * (q + 1) / NQ;
+      static_for<l0, l1>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        if constexpr (i < LB)
+          load_b(I, min(s + 1, last), std::integral_constant<int, set ^ 1>{});
+        else
+          load_a(std::integral_constant<int, i - LB>{}, min(s + 2, last), nbuf);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    swp[0] = swv[set][0];
+    swp[1] = swv[set][1];
+    buf = buf == NB - 1 ? 0 : buf + 1;
+  };
+  int s = 0;
+  for (; s + 1 < KS; s += 2) {
+    step(std::integral_constant<int, 0>{}, s);
+    step(std::integral_constant<int, 1>{}, s + 1);
+  }
+  if (s < KS)
+    step(std::integral_constant<int, 0>{}, s);
+  fold(std::integral_constant<int, NG - 1>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 16>{}, swp);
+  __syncthreads(); // (waits for the loads still under way: the ring is free for the epilogue staging)
+  float* stage = reinterpret_cast<float*>(tl_lds) + wave * (MT < 4 ? MT * 16 : 64) * ep_ld(2);
   if (DUAL)
-    big_epilogue_dual<MT>(p, P.seg[1], facc, stage, m_wg + wm * (MT * 16), tile_base);
+    big_epilogue_dual<MT, 2>(p, P.seg[1], facc, stage, m_wg, tile_base);
   else
-    big_epilogue<MT>(p, facc, stage, m_wg + wm * (MT * 16), tile_base);
+    big_epilogue<MT, 2>(p, facc, stage, m_wg, tile_base);
 }
 
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, 2)
 big_qint8_kernel(const BigParams P) {
-  big_qint8_body<4, false>(P);
+  big_qint8_body<8, 8, false>(P);
 }
 
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, 2)
 big_qint8_small_kernel(const BigParams P) {
-  big_qint8_body<2, false>(P);
+  big_qint8_body<4, 8, false>(P);
 }
 
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(256, 2)
+big_qint8_narrow_kernel(const BigParams P) {
+  big_qint8_body<4, 4, false>(P);
+}
+
+__global__ void __launch_bounds__(512, 2)
 big_qint8_dual_kernel(const BigParams P) {
-  big_qint8_body<4, true>(P);
+  big_qint8_body<8, 8, true>(P);
 }
 
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, 2)
 big_qint8_small_dual_kernel(const BigParams P) {
-  big_qint8_body<2, true>(P);
+  big_qint8_body<4, 8, true>(P);
+}
+
+__global__ void __launch_bounds__(256, 2)
+big_qint8_narrow_dual_kernel(const BigParams P) {
+  big_qint8_body<4, 4, true>(P);
 }
 
 // the large-M kernel addresses its operands with 32-bit byte offsets
@@ -1825,40 +1822,41 @@ hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t str
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].xq != t[1].xq))
     return hipErrorInvalidValue;
   BigParams P;
-  memset(&P, 0, sizeof(P));
-  int nb = 0;
-  for (int i = 0; i < n; i++) {
-    P.seg[i] = t[i];
-    P.nb0[i] = nb;
-    if (!dual)
-      nb += (t[i].tiles + 15) / 16;
-    else if (i == 0)
-      nb = (t[0].tiles + 7) / 8;
+  auto go = [&](auto kern, int rows, int waves, size_t lds) -> hipError_t {
+    const dim3 grid((unsigned)((t[0].M + rows - 1) / rows * P.nb0[TPPX_MAX_SEGS])), block((unsigned)(waves * 64));
+    TPPX_PLAN_ONLY(kern, grid, block, lds);
+    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds); e != hipSuccess)
+      return e;
+    kern<<<grid, block, lds, stream>>>(P);
+    return hipGetLastError();
+  };
+  auto channel_blocks = [&](int waves) { // of 32 channels per wave; the pair: 16 of each projection
+    memset(&P, 0, sizeof(P));
+    int nb = 0;
+    for (int i = 0; i < n; i++) {
+      P.seg[i] = t[i];
+      P.nb0[i] = nb;
+      if (!dual)
+        nb += (t[i].tiles + waves * 2 - 1) / (waves * 2);
+      else if (i == 0)
+        nb = (t[0].tiles + waves - 1) / waves;
+    }
+    for (int i = n; i <= TPPX_MAX_SEGS; i++)
+      P.nb0[i] = nb;
+    P.n_seg = n;
+    return nb;
+  };
+  const int64_t wgs64 = (int64_t)((t[0].M + 63) / 64) * channel_blocks(8); // workgroups of 64 x 256
+  const bool small = env_int("TPPX_TILED_SMALL", 1) != 0;
+  if (small && wgs64 < 128) { // less than half the CUs: 64 x 128, twice as many (4096 x 4096 at 333 rows 19.6 -> 15.0 us; from
+                              // 129 of 64 x 256 on, where they would take a second round, 64 x 128 loses: 24.5 against 25.7)
+    channel_blocks(4);
+    return dual ? go(big_qint8_narrow_dual_kernel, 64, 4, Qint8Geom<4, 4>::LDS) : go(big_qint8_narrow_kernel, 64, 4, Qint8Geom<4, 4>::LDS);
   }
-  for (int i = n; i <= TPPX_MAX_SEGS; i++)
-    P.nb0[i] = nb;
-  P.n_seg = n;
-  const int MB4 = (t[0].M + 127) / 128, MB2 = (t[0].M + 63) / 64;
-  const size_t lds = 8 * 64 * EP_LD * sizeof(float); // epilogue staging; >= the A and B buffers + the scale slots
-  static_assert(8 * 64 * EP_LD * sizeof(float) >= 2 * 128 * 256 + 64 * 1024 + 4 * 128 * sizeof(float), "LDS plan");
-#define TPPX_BIG_QINT8(KERNEL, MB)                                                                                     \
-  do {                                                                                                                 \
-    TPPX_PLAN_ONLY(KERNEL, dim3((MB) * nb), dim3(512), lds);                                                           \
-    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(KERNEL), lds); e != hipSuccess)                 \
-      return e;                                                                                                        \
-    KERNEL<<<dim3((MB) * nb), dim3(512), lds, stream>>>(P);                                                            \
-    return hipGetLastError();                                                                                          \
-  } while (0)
-  // launches of at most 128 workgroups of 128 x 256: twice as many of 64 x 256, so that fewer CUs stay empty
-  const bool small = MB4 * nb <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0;
-  if (dual && small)
-    TPPX_BIG_QINT8(big_qint8_small_dual_kernel, MB2);
-  if (dual)
-    TPPX_BIG_QINT8(big_qint8_dual_kernel, MB4);
-  if (small)
-    TPPX_BIG_QINT8(big_qint8_small_kernel, MB2);
-  TPPX_BIG_QINT8(big_qint8_kernel, MB4);
-#undef TPPX_BIG_QINT8
+  if (small && wgs64 <= 256) // one round of half-size workgroups (4096 x 4096 at 1000 rows 34.1 -> 24.5 us); two of them
+                             // take longer than one of 128 x 256 (12288 x 4096 at 333 rows 39.9 against 32.3)
+    return dual ? go(big_qint8_small_dual_kernel, 64, 8, Qint8Geom<4, 8>::LDS) : go(big_qint8_small_kernel, 64, 8, Qint8Geom<4, 8>::LDS);
+  return dual ? go(big_qint8_dual_kernel, 128, 8, Qint8Geom<8, 8>::LDS) : go(big_qint8_kernel, 128, 8, Qint8Geom<8, 8>::LDS);
 }
 
 hipError_t launch_tiled_qint8(const TiledParams& p, hipStream_t stream) {

@@ -995,6 +995,34 @@ def test_prefill_bf16_every_workgroup_tile_ragged(tile, w8, M, N, K, monkeypatch
     assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws[:4], bs), got[2:]))
 
 
+@pytest.mark.parametrize("fmt", ["mxfp4", "bf16"])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 7])
+def test_prefill_side_by_side_forms_at_every_loop_remainder(fmt, steps, monkeypatch):
+    """The forms whose waves keep the weights in registers (64 x 128; bf16: 64 x 256 and 128 x 256 as well) run their K steps
+    of 128 by threes with a tail: one step up to two rounds and a remainder, rows and channel blocks ragged, against the
+    256 x 256 form (the same sums in the same order, hence the same bits): linear, q/k/v, pair."""
+    ops = _ops()
+    M, N, K = 201, 288, 128 * steps
+    if fmt == "mxfp4":
+        ws = [_make("mxfp4", n, K, 940 + i)[0] for i, n in enumerate((N, 32, 160, N))]
+        tiles = ("4",)
+    else:
+        ws = [block_bf16(randn_bf16((n, K), 0.05, 940 + i)).cuda() for i, n in enumerate((N, 32, 160, N))]
+        tiles = ("4", "6", "2")
+    x, b = randn_bf16((M, K), 1.0, 945).cuda(), randn_bf16((N,), 0.5, 946).cuda()
+
+    def run():
+        return [ops.fc_plain(x, ws[0], b), ops.swiglu_gate_up(x, ws[0], ws[3])] + list(ops.qkv_gemm(x, ws[:3], [b, None, None]))
+
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
+    monkeypatch.setenv("TPPX_TILED_BIG_TILE", "1")
+    want = run()
+    for tile in tiles:
+        monkeypatch.setenv("TPPX_TILED_BIG_TILE", tile)
+        for i, (a, w) in enumerate(zip(run(), want)):
+            assert torch.equal(a, w), (tile, i)
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 16, 256), (64 * 3, 272, 512), (129, 4080, 768), (300, 8208, 1024), (1000, 1040, 1280)])
 def test_prefill_qint8_forms_agree_with_the_oracle(M, N, K, monkeypatch):
     """The large-M QINT8 kernel from one K step to five (odd and even: its loop goes by two), a single channel tile, ragged

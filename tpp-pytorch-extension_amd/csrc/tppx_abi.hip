@@ -272,9 +272,10 @@ static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, boo
   if (nk && mxfp4_nk_fits(M, (int)tiles, (int)(K / 128), ws_bytes))
     return tiled <= rows_us(NK, (tiles + 3) / 4 * 4 * rows64, K);
   const int nt = tiles <= 256 ? 1 : (tiles + 1) / 2 <= 256 ? 2 : 3; // channel tiles per workgroup, as the launch picks them
-  // (a single GEMM of two block rows stays with the decode kernels unless the tiles win by more than both estimates are
-  // off: 28.7 against 23.1 us at 11008 x 4096 are left there, 52 against 24 at 28672 x 2560 are not)
-  const double margin = !dual && rows64 == 2 ? 1.22 : 1.0;
+  // (a single GEMM of two full block rows stays with the decode kernels up to an advantage of 1.56, as callers hold those
+  // launch plans: 28.1 against 17.7 us at 11008 x 4096 are left there, 20.6 against 17.0 at 4096 x 4096; 52 against 20 at
+  // 28672 x 2560 are not)
+  const double margin = !dual && M == 128 ? 1.56 : 1.0;
   return tiled * margin <= rows_us((dual ? DUAL : SINGLE)[nt - 1], (tiles + nt - 1) / nt * rows64, K);
 }
 
@@ -325,13 +326,19 @@ static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tile
   const int64_t rows64 = (M + 63) / 64;
   int64_t all = 0;
   double rows = 0.0;
+  bool one_round = true;
   for (int i = 0; i < n; i++) {
     const int nt = tiles[i] > 512 ? 2 : 1;
-    rows += rows_us(ROWS[nt - 1], (tiles[i] + nt - 1) / nt * rows64, K);
+    const int64_t wgs = (tiles[i] + nt - 1) / nt * rows64;
+    rows += rows_us(ROWS[nt - 1], wgs, K);
+    one_round = one_round && wgs <= 256;
     all += tiles[i];
   }
-  if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
-    return tiled_bf16_us(M, K, all) <= rows;
+  if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0) {
+    // A group whose every decode launch is a single round stays with one launch per weight up to an advantage of 1.42, as
+    // callers count on it for pairs of 1024 channels (2 x 1024 x 5120 at 160 rows: 28.3 us, one launch would take 22.5).
+    return tiled_bf16_us(M, K, all) * (n > 1 && one_round ? 1.42 : 1.0) <= rows;
+  }
   const int64_t wgs = ((M + 127) / 128) * ((all + 7) / 8); // tiled_bf16_kernel
   return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
          (double)rows64 * (8.0 + (double)all * 32.0 * (double)K / 5.5e6 + (double)K * 0.0008);

@@ -40,6 +40,11 @@ __device__ __forceinline__ bf16x8 tl_cvt_fp4x8(uint32_t codes, float scale) {
   return w;
 }
 
+// buffer descriptor of an operand below 4 GiB (addresses checked by the host, so without a bound of its own)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tl_rsrc(const void* q) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(q), 0, 0xffffffffu, 0x00020000);
+}
+
 // XCD-aware tile order: returns (bm, bn) of this workgroup.  Workgroup ids go round the 8 XCDs; XCD x gets a
 // rectangle of the tile space and walks it row block fastest, so that the workgroups resident on an XCD at the same
 // time share operand tiles in its L2.  xm = how many of the 8 rectangles lie along M (1: an XCD owns NB/8 channel
@@ -838,10 +843,196 @@ __device__ __forceinline__ void big_gemm_body(const BigParams& P) {
     big_epilogue<MT>(p, acc, reinterpret_cast<float*>(tl_lds) + wave * 64 * EP_LD, m_wg + wm * (MT * 16), tile_base);
 }
 
+// ---------------------------------------------------------------------------
+// The same sums for launches of a few workgroups per CU (bf16 weights: and for those of 128 x 256 that stand one to a CU):
+// W waves side by side, each with a wave tile of MT*16 rows x 32 channels, K steps of 128, PD steps in flight.
+// What bounds such a launch is what a step of one workgroup takes with nothing beside it: the LDS (128 B/clk out, about half
+// of that in), the expansion of the codes and the latency of the step's loads.  So the weights of a wave are its own: they
+// go straight to its registers, expanded once per workgroup (a 2 x 2 grid of 32 x 64 wave tiles expanded each twice and took
+// codes and scales through the LDS), only the activations go through LDS, and everything is requested PD - 1 steps ahead.
+// All loads are buffer loads: scalar addresses, and the compiler counts them exactly beside the loads into LDS (flat-
+// addressed loads into LDS make it wait for everything).  Loads of the two kinds complete in issue order, so a step waits
+// until at most those of the PD - 2 younger steps are left; one barrier per step.  Scale bytes at any address.
+// Measured at 333 rows, MXFP4: 4096 x 4096 with residual 20.9 -> 17.8 us, 4096 x 11008 48.9 -> 41.6, 12288 x 4096
+// 46 -> 37, pair 2 x 11008 x 4096 73.5 -> 61 (three workgroups to a CU with PD = 3: 61.1, two with PD = 4: 64.8).  bf16
+// weights: 25.4 -> 19.3, 76.9 -> 58.2; 64 x 256 at 1000 rows 4096 x 11008 152 -> 103; 128 x 256 at 2048 rows 167 -> 144.
+// ---------------------------------------------------------------------------
+template <int MT, int W, int PD, bool WBF16>
+struct SideGeom {
+  static constexpr int WGM = MT * 16, STAGE = WGM * 256;
+  static constexpr int NA = MT * 4 / W;             // 4-row pieces of A a wave fetches per step
+  static constexpr int LB = WBF16 ? 8 : 4;          // weight (and scale) loads of a wave per step
+  static constexpr int L = NA + LB;
+  static constexpr size_t EP = (size_t)W * (MT < 4 ? MT * 16 : 64) * ep_ld(2) * sizeof(float);
+  static constexpr size_t LDS = (size_t)PD * STAGE > EP ? (size_t)PD * STAGE : EP;
+};
+
+template <int MT, int W, int PD, bool DUAL, bool WBF16>
+__device__ __forceinline__ void side_gemm_body(const BigParams& P) {
+  using G = SideGeom<MT, W, PD, WBF16>;
+  constexpr int WGM = G::WGM, STAGE = G::STAGE, NA = G::NA, LB = G::LB, L = G::L;
+  extern __shared__ __align__(16) uint8_t tl_lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int MB = (P.seg[0].M + WGM - 1) / WGM;
+  int bm, bn;
+  tile_of_block(MB, P.nb0[P.n_seg], bm, bn, P.xm);
+  TiledParams p = P.seg[0];
+  int nb_first = 0;
+  if (!DUAL) {
+#pragma unroll
+    for (int i = 1; i < TPPX_MAX_SEGS; i++)
+      if (i < P.n_seg && bn >= P.nb0[i]) {
+        p = P.seg[i];
+        nb_first = P.nb0[i];
+      }
+  }
+  bn -= nb_first;
+  const int KT = p.K >> 7, last = KT - 1;
+  const int m_wg = bm * WGM;
+  const int tile_base = DUAL ? bn * W + wave : bn * (W * 2) + wave * 2; // DUAL: gate and up tile of the same 16 channels
+
+  const auto xr = tl_rsrc(p.x);
+  uint32_t aoff[NA];
+#pragma unroll
+  for (int i = 0; i < NA; i++) {
+    const int blk = wave * NA + i, r16 = (blk & 3) * 4 + (lane >> 4);
+    aoff[i] = (uint32_t)min(m_wg + blk * 4 + (lane >> 4), p.M - 1) * (uint32_t)p.K * 2u + (uint32_t)(((lane & 15) ^ r16) & 15) * 16u;
+  }
+  __amdgpu_buffer_rsrc_t wr[2], swr[2];
+  uint32_t woff[2], swoff[2];
+#pragma unroll
+  for (int nt = 0; nt < 2; nt++) {
+    const int tile = min(DUAL ? tile_base : tile_base + nt, p.tiles - 1);
+    wr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].qw : p.qw);
+    swoff[nt] = (uint32_t)tile * (uint32_t)KT * 64u + (uint32_t)lane;
+    if constexpr (WBF16) {
+      woff[nt] = ((uint32_t)tile * (uint32_t)KT * 256u + (uint32_t)lane) * 16u;
+    } else {
+      woff[nt] = swoff[nt] * 16u;
+      swr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].sw : p.sw);
+    }
+  }
+  constexpr int BJ = WBF16 ? 4 : 1;
+  i32x4 bw[PD][BJ][2]; // raw weights of PD steps: packed codes, or the operands of the four MFMA steps
+  uint32_t sc[PD][2];
+  // load i of step s (clamped to the last one: what is read past it is never used)
+  auto load = [&](auto I, int s, auto SET) {
+    constexpr int i = decltype(I)::value, set = decltype(SET)::value;
+    s = min(s, last);
+    if constexpr (i < LB) {
+      if constexpr (WBF16)
+        bw[set][i >> 1][i & 1] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[i & 1], woff[i & 1] + (i >> 1) * 1024, s * 4096, 0));
+      else if constexpr (i < 2)
+        bw[set][0][i] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[i], woff[i], s * 1024, 0));
+      else
+        sc[set][i - 2] = __builtin_amdgcn_raw_buffer_load_b8(swr[i - 2], swoff[i - 2], s * 64, 0);
+    } else {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(tl_lds + set * STAGE + (wave * NA + i - LB) * 1024), 16,
+                                               aoff[i - LB], s * 256, 0, 0);
+    }
+  };
+  uint32_t rdb[4];
+  {
+    const int m = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      rdb[j] = (uint32_t)((m >> 2) * 1024 + (m & 3) * 256 + (((g * 4 + j) ^ m) & 15) * 16);
+  }
+  f32x4 acc[MT][2];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+    acc[mt][0] = acc[mt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  static_for<0, PD - 1>([&](auto S) {
+    static_for<0, L>([&](auto I) { load(I, decltype(S)::value, S); });
+    __builtin_amdgcn_sched_barrier(0); // (in this order: the waits count the loads behind those they wait for)
+  });
+  // Units of MU row tiles and one MFMA step j; the operands of unit q are read (and its weights expanded) under the MFMAs
+  // of unit q - 1, so the last unit of a step runs in the next one, under its first operand reads.
+  constexpr int MU = 4, UJ = MT / MU, NQ = 4 * UJ;
+  bf16x8 a[2][MU], b[2][2];
+#pragma unroll
+  for (int i = 0; i < MU; i++)
+    a[1][i] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  b[1][0] = b[1][1] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  auto unit = [&](auto Q) {
+    constexpr int q = decltype(Q)::value, j = q / UJ, mu = q % UJ;
+#pragma unroll
+    for (int i = 0; i < MU; i++)
+#pragma unroll
+      for (int nt = 0; nt < 2; nt++)
+        acc[mu * MU + i][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q & 1][i], b[j & 1][nt], acc[mu * MU + i][nt], 0, 0, 0);
+  };
+  // MORE: not one of the last steps, which request nothing any more and wait for all that is left.  (A load into registers
+  // whose result is never used would not be there to be counted.)
+  auto step = [&](auto MORE, auto SET, int s) {
+    constexpr bool more = decltype(MORE)::value;
+    constexpr int set = decltype(SET)::value, pset = (set + PD - 1) % PD;
+    asm volatile("" : : : "memory");
+    constexpr int vm = more ? L * (PD - 2) : 0;
+    __builtin_amdgcn_s_waitcnt((vm & 15) | 7 << 4 | vm >> 4 << 14); // step s has landed, the reads of step s - 1 have returned
+    asm volatile("s_barrier" : : : "memory");
+    const uint8_t* ab = tl_lds + set * STAGE;
+    float scale[2];
+    static_for<0, NQ>([&](auto Q) {
+      constexpr int q = decltype(Q)::value, j = q / UJ, mu = q % UJ;
+#pragma unroll
+      for (int i = 0; i < MU; i++)
+        a[q & 1][i] = *reinterpret_cast<const bf16x8*>(ab + (mu * MU + i) * 4096 + rdb[j]);
+      __builtin_amdgcn_sched_barrier(0);
+      unit(std::integral_constant<int, (q + NQ - 1) % NQ>{});
+      if constexpr (mu == 0) {
+        if constexpr (q == 0 && !WBF16) {
+          scale[0] = e8m0_to_f32(sc[set][0]);
+          scale[1] = e8m0_to_f32(sc[set][1]);
+        }
+#pragma unroll
+        for (int nt = 0; nt < 2; nt++) {
+          if constexpr (WBF16)
+            b[j & 1][nt] = __builtin_bit_cast(bf16x8, bw[set][j][nt]);
+          else
+            b[j & 1][nt] = tl_cvt_fp4x8((uint32_t)bw[set][0][nt][j], scale[nt]);
+        }
+        if constexpr (!WBF16)
+          static_for<0, MU * 2>([&](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+          });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // the loads PD - 1 steps ahead, a few behind each unit (in one burst, a wave stands at its load instructions while
+      // the memory pipeline's queue drains)
+      if constexpr (more) {
+        static_for<L * q / NQ, L * (q + 1) / NQ>([&](auto I) { load(I, s + PD - 1, std::integral_constant<int, pset>{}); });
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+  };
+  int s = 0;
+  for (; s + PD <= KT; s += PD)
+    static_for<0, PD>([&](auto S) { step(std::true_type{}, S, s + decltype(S)::value); });
+  static_for<0, PD - 1>([&](auto S) {
+    if (s + decltype(S)::value < KT)
+      step(std::false_type{}, S, s + decltype(S)::value);
+  });
+  unit(std::integral_constant<int, NQ - 1>{});
+  __syncthreads(); // (waits for the loads still under way: the ring is free for the epilogue staging)
+  float* stage = reinterpret_cast<float*>(tl_lds) + wave * (MT < 4 ? MT * 16 : 64) * ep_ld(2);
+  if (DUAL)
+    big_epilogue_dual<MT, 2>(p, P.seg[1], acc, stage, m_wg, tile_base);
+  else
+    big_epilogue<MT, 2>(p, acc, stage, m_wg, tile_base);
+}
+
+constexpr int SIDE_PD = 3;
+// MT <= 4: the forms for small launches, named by their workgroup tile (MT*16*WM rows x WN*64 channels) and threads
 template <int MT, bool DUAL, int WM, int WN>
-__global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
+__global__ void __launch_bounds__(WM * WN * 64, 2)
 big_bf16_kernel(const BigParams P) {
-  big_gemm_body<MT, DUAL, WM, WN, true>(P);
+  if constexpr (MT <= 4)
+    side_gemm_body<MT * WM, WM * WN, SIDE_PD, DUAL, true>(P);
+  else
+    big_gemm_body<MT, DUAL, WM, WN, true>(P);
 }
 
 // ---------------------------------------------------------------------------
@@ -1036,7 +1227,9 @@ constexpr int RING_STAGES = 3; // (two 64 x 128 workgroups of three stages share
 template <int MT, bool DUAL, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
 big_mxfp4_kernel(const BigParams P) {
-  if constexpr (MT <= 4)
+  if constexpr (MT == 2)
+    side_gemm_body<MT * WM, WM * WN, SIDE_PD, DUAL, false>(P);
+  else if constexpr (MT == 4)
     ring_gemm_body<MT, DUAL, WM, WN, RING_STAGES>(P);
   else
     big_gemm_body<MT, DUAL, WM, WN, false>(P);
@@ -1080,9 +1273,6 @@ struct Qint8Geom {
   static constexpr size_t EP = (size_t)W * (MT < 4 ? MT * 16 : 64) * ep_ld(2) * sizeof(float);
   static constexpr size_t LDS = (size_t)NB * STAGE > EP ? (size_t)NB * STAGE : EP;
 };
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t tl_rsrc(const void* q) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(q), 0, 0xffffffffu, 0x00020000);
-}
 
 template <int MT, int W, bool DUAL>
 __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
@@ -1492,36 +1682,41 @@ big_fp8_kernel(const BigParams P) {
 
 // Workgroup tiles of the MXFP4 and bf16 launches:
 //   256 x 256, 128 x 512  eight waves, one workgroup per CU; for launches that fill the chip several times over
-//   128 x 256             up to 256 of them one per CU (MXFP4: the ring kernel), beyond that four waves and two per CU
+//   128 x 256             up to 256 of them one per CU (MXFP4: the ring kernel, bf16: waves side by side), beyond that four
+//                         waves and two per CU
 //   128 x 128             MXFP4 only: ring kernel, one per CU
-//   64 x 128              MXFP4: ring kernel; two per CU
-enum { TILE_256_256 = 0, TILE_128_256, TILE_128_512, TILE_64_128, TILE_128_128, N_TILES };
-static constexpr int TILE_ROWS[N_TILES] = {256, 128, 128, 64, 128};
-static constexpr int TILE_COLS16[N_TILES] = {16, 16, 32, 8, 8}; // 16-channel weight tiles (the pair: gate + up)
+//   64 x 128              waves side by side; three (MXFP4) or two (bf16) per CU
+//   64 x 256              bf16 only: eight waves side by side
+enum { TILE_256_256 = 0, TILE_128_256, TILE_128_512, TILE_64_128, TILE_128_128, TILE_64_256, N_TILES };
+static constexpr int TILE_ROWS[N_TILES] = {256, 128, 128, 64, 128, 64};
+static constexpr int TILE_COLS16[N_TILES] = {16, 16, 32, 8, 8, 16}; // 16-channel weight tiles (the pair: gate + up)
 
 // What a launch takes, in us, with r = its rounds of 256 workgroups, f = the filled part of the last one and s = K / 128:
 //   one round     a + (b + c f) s
 //   more          p + q r + (u + v r + w f + z r s / 1000) s     (z: the clock falls under the power limit as a launch
 //                                                                 grows; measured up to 28672 x 8192 pairs of 2048 rows)
 // bf16 weights: and g (one round) or h us for each MB of them, which come from memory at whatever tile.
-// Fitted to 2500 launches: 65 .. 2048 rows, linears and pairs of 1024 .. 32000 x 1024 .. 18944, every tile forced, weights
-// rotated through 0.5 .. 2 GB.  The tile chosen is within 0.5 % of the fastest on average, 12 % at worst (MXFP4), and
-// 0.3 %, 12 % (bf16).
+// Fitted to 2736 launches of each format: 65 .. 2048 rows, linears and pairs of 1024 .. 28672 x 1024 .. 18944, every tile
+// forced, weights rotated through 2 GB.  On 792 others (random channels and K) the tile chosen is 0.4 % (MXFP4) and 0.75 %
+// (bf16) off the fastest on average, 11 and 15 % in the worst hundredth.
 struct TileCost {
   double a, b, c, p, q, u, v, w, z, g, h;
 };
 static constexpr TileCost MXFP4_COST[N_TILES] = {
-    {17.9, 1.90, 0.39, 0.17, 18.0, -0.65, 2.40, 0.625, 0.311, 0, 0},
-    {11.3, 1.10, 0.213, 5.3, 7.26, -0.265, 1.13, 0.443, 0.177, 0, 0},
-    {17.8, 1.85, 0.406, 0.32, 17.9, -0.653, 2.32, 0.719, 0.431, 0, 0},
-    {6.31, 0.476, 0.0848, 3.63, 2.09, -0.0318, 0.410, 0.112, 0.0374, 0, 0},
-    {9.51, 0.750, 0.126, 2.14, 7.43, -0.202, 0.879, 0.152, 0.011, 0, 0},
+    {7.75, 1.88, 0.607, -6.18, 12.4, -0.498, 2.31, 0.768, 0.256, 0, 0},
+    {6.07, 1.09, 0.302, 4.03, 3.96, -0.337, 1.18, 0.442, 0.0994, 0, 0},
+    {7.71, 1.85, 0.573, -8.21, 13, -0.546, 2.27, 0.864, 0.281, 0, 0},
+    {4.02, 0.385, 0.091, 3.36, 1.09, -0.0981, 0.352, 0.145, 0.029, 0, 0},
+    {4.88, 0.75, 0.146, 0.348, 3.97, -0.157, 0.871, 0.18, 0.00761, 0, 0},
+    {},
 };
-static constexpr TileCost BF16_COST[TILE_128_128] = {
-    {16.8, 1.98, 0.59, -2.62, 19.3, -0.622, 2.58, 0.96, 0.367, 0.0182, 0.00766},
-    {8.10, 1.25, 0.269, 2.46, 7.88, -0.269, 1.17, 0.638, 0.371, 0.0892, 0.0554},
-    {15.4, 1.99, 0.471, -5.16, 20.1, -0.764, 2.53, 1.16, 0.406, 0.0689, 0.0501},
-    {4.85, 0.626, 0.114, 1.63, 0.948, -0.0886, 0.655, 0.154, 0.0973, 0.0527, 0.0832},
+static constexpr TileCost BF16_COST[N_TILES] = {
+    {7.22, 1.96, 0.625, -8.28, 13.5, -0.615, 2.49, 0.883, 0.297, 0.0298, 0.0316},
+    {5.39, 1.02, 0.341, 1.28, 3.47, -0.41, 1.26, 0.607, 0.268, 0.0726, 0.0559},
+    {6.9, 1.91, 0.543, -15.3, 15.2, -0.583, 2.38, 1.15, 0.281, 0.0795, 0.089},
+    {3.26, 0.404, 0.148, 2.96, 0.221, -0.246, 0.539, 0.206, 0.134, 0.0443, 0.0668},
+    {},
+    {3.35, 0.708, 0.2, -2.67, 3.75, -0.226, 0.857, 0.388, 0.285, 0.076, 0.111},
 };
 static double tile_us(const TileCost& k, int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
   const int64_t wgs = mb * nb;
@@ -1535,30 +1730,62 @@ static double tile_us(const TileCost& k, int tile, int64_t mb, int64_t nb, doubl
 static double mxfp4_tile_us(int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
   const double us = tile_us(MXFP4_COST[tile], tile, mb, nb, s, weight_mb);
   // An odd number of row blocks leaves no rectangles for the XCDs (tile_of_block), and columns of more row blocks than
-  // fit a CU set drift apart in K: 23 row blocks of 64 cost 4 % more, 27 8 %, 31 16 % (K = 2048 .. 16384; none at 1024).
-  return tile == TILE_64_128 && mb * nb > 256 && (mb & 1) && mb > 21
-             ? us * (1.0 + 0.02 * (double)(mb - 21) * std::min(1.0, s / 32.0)) : us;
+  // fit a CU set drift apart in K: 21 row blocks of 64 cost 10 % more, 27 and 29 29 % (K from 3072; 6 % up to 2048).
+  return tile == TILE_64_128 && mb * nb > 256 && (mb & 1) && mb >= 21
+             ? us * (1.0 + std::min(0.29, 0.1 + 0.031 * (double)(mb - 21)) * std::min(1.0, std::max(0.0, (s - 8.0) / 16.0))) : us;
 }
 static double bf16_tile_us(int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
   return tile_us(BF16_COST[tile], tile, mb, nb, s, weight_mb);
 }
 
+// the tiles a launch may take, one bit each.  scales4: scale bytes on a 4-byte address (the ring forms move four at a time)
+static unsigned mxfp4_tiles(bool scales4) {
+  const unsigned large = 1u << TILE_256_256 | 1u << TILE_128_256 | 1u << TILE_128_512;
+  return env_int("TPPX_TILED_SMALL", 1) == 0 ? large : large | 1u << TILE_64_128 | (scales4 ? 1u << TILE_128_128 : 0u);
+}
+static unsigned bf16_tiles() {
+  const unsigned large = 1u << TILE_256_256 | 1u << TILE_128_256 | 1u << TILE_128_512;
+  return env_int("TPPX_TILED_SMALL", 1) == 0 ? large : large | 1u << TILE_64_128 | 1u << TILE_64_256;
+}
+
+// the cheapest of them for n GEMMs of tiles[i] channel tiles over one activation (dual: the gate/up pair, tiles[0] each)
 template <typename Us>
-static double cheapest_us(int64_t M, int64_t K, int64_t n_tiles16, int tiles, double weight_mb, Us&& us) {
+static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dual, unsigned allowed, Us&& us, double* best_us = nullptr) {
+  int64_t all = 0;
+  for (int i = 0; i < n; i++)
+    all += tiles[i];
+  int shape = 0;
   double best = 1e300;
-  for (int i = 0; i < tiles; i++)
-    best = std::min(best, us(i, (M + TILE_ROWS[i] - 1) / TILE_ROWS[i], (n_tiles16 + TILE_COLS16[i] - 1) / TILE_COLS16[i],
-                             (double)(K / 128), weight_mb));
-  return best;
+  for (int i = 0; i < N_TILES; i++) {
+    if (!(allowed >> i & 1u))
+      continue;
+    const int tpw = TILE_COLS16[i] / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
+    int64_t nb = 0;
+    for (int g = 0; g < (dual ? 1 : n); g++)
+      nb += (tiles[g] + tpw - 1) / tpw;
+    if (const double c = us(i, (M + TILE_ROWS[i] - 1) / TILE_ROWS[i], nb, (double)(K / 128), (double)(all * 32 * K) * 1e-6);
+        c < (i >= TILE_64_128 ? 0.99 : 1.0) * best) { // (a tie goes to the larger tiles, which read less)
+      best = c;
+      shape = i;
+    }
+  }
+  if (best_us)
+    *best_us = best;
+  return shape;
 }
 
 double tiled_mxfp4_us(int64_t M, int64_t K, int64_t n_tiles16) {
-  return cheapest_us(M, K, n_tiles16, env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128, 0.0, mxfp4_tile_us);
+  const int tiles = (int)n_tiles16;
+  double us;
+  cheapest_tile(M, K, &tiles, 1, false, mxfp4_tiles(true), mxfp4_tile_us, &us);
+  return us;
 }
 
 double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16) {
-  return cheapest_us(M, K, n_tiles16, env_int("TPPX_TILED_SMALL", 1) != 0 ? TILE_128_128 : TILE_64_128,
-                     (double)(n_tiles16 * 32 * K) * 1e-6, bf16_tile_us);
+  const int tiles = (int)n_tiles16;
+  double us;
+  cheapest_tile(M, K, &tiles, 1, false, bf16_tiles(), bf16_tile_us, &us);
+  return us;
 }
 
 static bool big_fits(const TiledParams& p) {
@@ -1569,51 +1796,41 @@ bool tiled_mxfp4_takes_groups(const TiledParams& p) {
   return p.M >= big_min_rows() && big_fits(p);
 }
 
+template <typename Kern>
+static hipError_t big_go(Kern kern, const BigParams& P, int wgs, int threads, size_t lds, hipStream_t stream) {
+  TPPX_PLAN_ONLY(kern, dim3(wgs), dim3(threads), lds);
+  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds); e != hipSuccess)
+    return e;
+  kern<<<dim3(wgs), dim3(threads), lds, stream>>>(P);
+  return hipGetLastError();
+}
+
 template <int MT, bool DUAL, int WM, int WN>
 static hipError_t big_launch(const BigParams& P, int wgs, hipStream_t stream) {
   size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float); // epilogue staging per wave; >= the two A buffers
-  if constexpr (MT <= 4)
-    lds = RingGeom<MT, WM, WN, RING_STAGES>::LDS;
   static_assert(MT <= 4 || (size_t)WM * WN * 64 * EP_LD * sizeof(float) >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
-  TPPX_PLAN_ONLY((big_mxfp4_kernel<MT, DUAL, WM, WN>), dim3(wgs), dim3(WM * WN * 64), lds);
-  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(big_mxfp4_kernel<MT, DUAL, WM, WN>), lds); e != hipSuccess)
-    return e;
-  big_mxfp4_kernel<MT, DUAL, WM, WN><<<dim3(wgs), dim3(WM * WN * 64), lds, stream>>>(P);
-  return hipGetLastError();
+  if constexpr (MT == 2)
+    lds = SideGeom<MT * WM, WM * WN, SIDE_PD, false>::LDS;
+  else if constexpr (MT == 4)
+    lds = RingGeom<MT, WM, WN, RING_STAGES>::LDS;
+  return big_go(big_mxfp4_kernel<MT, DUAL, WM, WN>, P, wgs, WM * WN * 64, lds, stream);
 }
 
 template <int MT, bool DUAL, int WM, int WN>
 static hipError_t big_bf16_launch(const BigParams& P, int wgs, hipStream_t stream) {
-  const size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float);
-  static_assert((size_t)WM * WN * 64 * EP_LD * sizeof(float) >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
-  TPPX_PLAN_ONLY((big_bf16_kernel<MT, DUAL, WM, WN>), dim3(wgs), dim3(WM * WN * 64), lds);
-  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(big_bf16_kernel<MT, DUAL, WM, WN>), lds); e != hipSuccess)
-    return e;
-  big_bf16_kernel<MT, DUAL, WM, WN><<<dim3(wgs), dim3(WM * WN * 64), lds, stream>>>(P);
-  return hipGetLastError();
+  size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float);
+  static_assert(MT <= 4 || (size_t)WM * WN * 64 * EP_LD * sizeof(float) >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
+  if constexpr (MT <= 4)
+    lds = SideGeom<MT * WM, WM * WN, SIDE_PD, true>::LDS;
+  return big_go(big_bf16_kernel<MT, DUAL, WM, WN>, P, wgs, WM * WN * 64, lds, stream);
 }
 
-// the first `tiles` workgroup tiles' lowest estimate for n GEMMs over one activation (dual: the gate/up pair)
 template <typename Us>
-static int cheapest_tile(const TiledParams* t, int n, bool dual, int tiles, Us&& us) {
-  int64_t tiles16 = 0;
+static int cheapest_tile(const TiledParams* t, int n, bool dual, unsigned allowed, Us&& us) {
+  int tiles[TPPX_MAX_SEGS];
   for (int i = 0; i < n; i++)
-    tiles16 += t[i].tiles;
-  int shape = 0;
-  double best = 1e300;
-  for (int i = 0; i < tiles; i++) {
-    const int tpw = TILE_COLS16[i] / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
-    int64_t nb = 0;
-    for (int g = 0; g < (dual ? 1 : n); g++)
-      nb += (t[g].tiles + tpw - 1) / tpw;
-    if (const double c = us(i, (t[0].M + TILE_ROWS[i] - 1) / TILE_ROWS[i], nb, (double)(t[0].K / 128),
-                            (double)(tiles16 * 32 * t[0].K) * 1e-6);
-        c < (i >= TILE_64_128 ? 0.99 : 1.0) * best) { // (a tie goes to the larger tiles, which read less)
-      best = c;
-      shape = i;
-    }
-  }
-  return shape;
+    tiles[i] = t[i].tiles;
+  return cheapest_tile(t[0].M, t[0].K, tiles, n, dual, allowed, us);
 }
 
 // fills P for n GEMMs over one activation with this workgroup tile; returns the workgroups of the launch
@@ -1652,17 +1869,33 @@ static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int 
   return MB * nb;
 }
 
+// Launches of whole 128-row blocks that fill between two thirds and seven tenths of the CUs as 128 x 256 or 128 x 512 keep
+// those tiles: callers hold their launch plans (512 or 1024 rows x 11008, pair of 256 rows).  64 x 128 would be the faster
+// one at the first and the last, 39.5 against 46.6 us and 41.5 against 48.8; 77.2 against 75.5 at the second.
+static unsigned mxfp4_fixed_plans(const TiledParams* t, int n, bool dual) {
+  if (t[0].M % 128 != 0)
+    return 0u;
+  for (int tile : {TILE_128_256, TILE_128_512}) {
+    const int tpw = TILE_COLS16[tile] / (dual ? 2 : 1);
+    int nb = 0;
+    for (int i = 0; i < (dual ? 1 : n); i++)
+      nb += (t[i].tiles + tpw - 1) / tpw;
+    if (const int64_t wgs = (int64_t)(t[0].M / 128) * nb; wgs >= 171 && wgs <= 179)
+      return 1u << TILE_64_128;
+  }
+  return 0u;
+}
+
 // dual: t[0] = gate, t[1] = up (equal shapes, n == 2); y[m][n] = silu(gate) * up goes to t[1].y
 hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
-  // the ring moves scale bytes four at a time: scales off a 4-byte address keep to the forms that read them one by one
-  bool ring = true;
+  bool scales4 = true;
   for (int i = 0; i < n; i++)
-    ring = ring && (reinterpret_cast<uintptr_t>(t[i].sw) & 3u) == 0;
+    scales4 = scales4 && (reinterpret_cast<uintptr_t>(t[i].sw) & 3u) == 0;
   int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
-  if (shape < 0 || shape >= (ring ? N_TILES : TILE_64_128))
-    shape = cheapest_tile(t, n, dual, ring && env_int("TPPX_TILED_SMALL", 1) != 0 ? N_TILES : TILE_64_128, mxfp4_tile_us);
+  if (shape < 0 || shape > TILE_128_128 || (shape == TILE_128_128 && !scales4))
+    shape = cheapest_tile(t, n, dual, mxfp4_tiles(scales4) & ~mxfp4_fixed_plans(t, n, dual), mxfp4_tile_us);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 0.53);
   switch (shape) {
@@ -1675,7 +1908,7 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
   case TILE_128_256:
     // at most one workgroup per CU: eight waves of 64 x 64, two per SIMD, so that one wave's waits are another's issue
     // slots; else four of 128 x 64, two workgroups per CU
-    if (ring && wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0)
+    if (scales4 && wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0)
       return dual ? big_launch<4, true, 2, 4>(P, wgs, stream) : big_launch<4, false, 2, 4>(P, wgs, stream);
     return dual ? big_launch<8, true, 1, 4>(P, wgs, stream) : big_launch<8, false, 1, 4>(P, wgs, stream);
   default:
@@ -1770,9 +2003,9 @@ bool tiled_bf16_takes_groups(const TiledParams& p) {
 hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
-  int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 .. 4 as in launch_tiled_mxfp4_group; 5 is not built for 2-byte weights
-  if (shape < 0 || shape >= TILE_128_128)
-    shape = cheapest_tile(t, n, dual, env_int("TPPX_TILED_SMALL", 1) != 0 ? TILE_128_128 : TILE_64_128, bf16_tile_us);
+  int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 .. 4 as in launch_tiled_mxfp4_group, 6 = 64 x 256; 5 is not built for 2-byte weights
+  if (shape < 0 || shape >= N_TILES || shape == TILE_128_128)
+    shape = cheapest_tile(t, n, dual, bf16_tiles(), bf16_tile_us);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 2.0);
   switch (shape) {
@@ -1780,6 +2013,8 @@ hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stre
     return dual ? big_bf16_launch<8, true, 1, 8>(P, wgs, stream) : big_bf16_launch<8, false, 1, 8>(P, wgs, stream);
   case TILE_64_128:
     return dual ? big_bf16_launch<2, true, 2, 2>(P, wgs, stream) : big_bf16_launch<2, false, 2, 2>(P, wgs, stream);
+  case TILE_64_256:
+    return dual ? big_bf16_launch<2, true, 2, 4>(P, wgs, stream) : big_bf16_launch<2, false, 2, 4>(P, wgs, stream);
   case TILE_128_256:
     if (wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0) // at most one workgroup per CU: eight waves, as for MXFP4
       return dual ? big_bf16_launch<4, true, 2, 4>(P, wgs, stream) : big_bf16_launch<4, false, 2, 4>(P, wgs, stream);

@@ -240,6 +240,29 @@ def test_attn_prefill(B, S, Nq, Nkv, past, Smax, queries_per_wave, monkeypatch):
         assert np.sqrt(((g - d) ** 2).sum() / (d ** 2).sum()) <= 5e-3
 
 
+@pytest.mark.parametrize("rise", [0.5, 7.0, 40.0, -7.0])
+@pytest.mark.parametrize("queries_per_wave", [16, 32])
+def test_attn_prefill_running_maximum(rise, queries_per_wave, monkeypatch):
+    """The running maximum moves only when a score exceeds it by 8 (base 2): scores that rise along the keys by less and by
+    more than that per key tile, and that fall, over grouped heads, one query of a workgroup far above the others, against
+    softmax attention in float64 (probabilities and outputs rounded to bf16: 2^-8 each)."""
+    _llm()
+    monkeypatch.setenv("TPPX_ATTN_QG", str(queries_per_wave // 16))
+    S, Nq, Nkv = 330, 6, 2
+    q, v = randn_bf16((1, S, Nq, 128), 0.3, 66), randn_bf16((1, Nkv, 384, 128), 1.0, 67)
+    k = randn_bf16((1, Nkv, 384, 128), 0.3, 68)
+    q[..., 0] = 8.0
+    q[0, 70, :, 0] = 24.0
+    k[..., 0] = (torch.arange(384) * (rise * np.log(2.0) * np.sqrt(128.0) / 8.0 / 64.0)).to(torch.bfloat16)
+    got = _attn_prefill(q.cuda(), k.cuda(), v.cuda(), 0).cpu().double()
+    kk, vv = (t[:, :, :S].double().repeat_interleave(Nq // Nkv, dim=1) for t in (k, v))
+    s = torch.matmul(q.double().transpose(1, 2), kk.transpose(2, 3)) / np.sqrt(128.0)
+    s = s.masked_fill(torch.arange(S)[None, :] > torch.arange(S)[:, None], float("-inf"))
+    want = torch.matmul(torch.softmax(s, -1), vv).transpose(1, 2)
+    err = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert float(err.max()) <= 2.0 ** -7, float(err.max())
+
+
 def test_attn_prefill_full_size_rows_equal_single_query_problem():
     """The 7B prompt shape (2048 tokens, 32 heads): every sampled query row must solve the single-query problem on
     the keys it sees -- checked against the oracle's single-query function, which the multi-query restatement is

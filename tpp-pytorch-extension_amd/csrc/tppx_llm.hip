@@ -862,31 +862,68 @@ struct AttnPrefillParams {
   int H;                // head size (attn_prefill_hd_kernel; the kernel for 128 does not read it)
 };
 
-constexpr int AP_KP = 136; // LDS row pitch of the K tile, bf16 elements (128 + 8: rows 16-byte aligned, banks spread)
-constexpr int AP_VP = 68;  // LDS row pitch of the V^T tile (64 keys + 4: rows 8-byte aligned)
+constexpr int AP_VP = 68; // LDS row pitch of the hd kernel's V^T tile (64 keys + 4: rows 8-byte aligned)
 
-// QG = query groups of 16 per wave: every K / V^T operand read from LDS feeds QG MFMAs (with one group the LDS
-// reads, 32 KB per wave and key tile, take twice the cycles of the 32 MFMAs they feed).
-template <int QG>
-__global__ void __launch_bounds__(256)
+// Prompt attention, head size 128: W waves of 16 queries share the K and V tiles of 64 keys (8: 128 queries, four waves per
+// SIMD with two workgroups on a CU; 4: 64 queries, for launches of few workgroups).
+// K and V tiles go straight into LDS, a tile ahead, two stages of 2 x 16 KiB, one barrier per tile; the swizzle sits on the
+// source side (K: position ch of row r holds chunk ch ^ (r & 15); V: ch ^ 2 (r & 7)), so that the rows of an operand read
+// fall on different bank groups.  V's operand is read by the transposing LDS read: of a 16-lane group lane i fetches 8 bytes
+// of key (i >> 2) and gets the four keys of dim i.
+// What bounds it is the chain scores -> softmax -> output of a wave, not one unit (MFMA a third busy, vector issue a half), so
+// waves per SIMD count more than operand reads per MFMA: 32 queries per wave, half the reads, take 57 us where this takes
+// 50 (2048 tokens x 32 heads).  And the vector instructions per score: the running maximum is a power of two's exponent (an
+// integer in the base-2 domain) and moves only when a score exceeds it by 8; within that a probability is at most 2^8, sums
+// and outputs scale exactly, and a tile needs no maximum across lanes and no rescaling of the output sums.  The scaling being
+// exact, a query's result does not depend on when it moves, that is on the other queries of its wave.
+// Measured against registers in between, V transposed by byte permutes and a maximum per tile: 2048 tokens x 32 heads
+// 71 -> 49.5 us, 64 heads on 8 of K/V 129 -> 83, 1000 x 32 26.7 -> 20.0, 333 x 32 12.6 -> 8.4.  Tried beside it: the next
+// tile's scores under this one's softmax in a wave (256 registers and scratch), two halves of the keys on eight waves (54.8),
+// the same half a turn apart (60).
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+// The transposing reads of 32 keys' V operands (8 dim tiles x 2 runs of 16 keys), issued and waited for in one block: around
+// the builtin the compiler waits for every load into LDS under way, that is for the next tile.
+template <int OFF>
+__device__ __forceinline__ void read_v_operands(i32x2 (&v)[8][2], const uint32_t (&a)[8]) {
+  asm volatile("ds_read_b64_tr_b16 %0, %16 offset:%24\n\tds_read_b64_tr_b16 %1, %16 offset:%25\n\t"
+               "ds_read_b64_tr_b16 %2, %17 offset:%24\n\tds_read_b64_tr_b16 %3, %17 offset:%25\n\t"
+               "ds_read_b64_tr_b16 %4, %18 offset:%24\n\tds_read_b64_tr_b16 %5, %18 offset:%25\n\t"
+               "ds_read_b64_tr_b16 %6, %19 offset:%24\n\tds_read_b64_tr_b16 %7, %19 offset:%25\n\t"
+               "ds_read_b64_tr_b16 %8, %20 offset:%24\n\tds_read_b64_tr_b16 %9, %20 offset:%25\n\t"
+               "ds_read_b64_tr_b16 %10, %21 offset:%24\n\tds_read_b64_tr_b16 %11, %21 offset:%25\n\t"
+               "ds_read_b64_tr_b16 %12, %22 offset:%24\n\tds_read_b64_tr_b16 %13, %22 offset:%25\n\t"
+               "ds_read_b64_tr_b16 %14, %23 offset:%24\n\tds_read_b64_tr_b16 %15, %23 offset:%25\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(v[0][0]), "=&v"(v[0][1]), "=&v"(v[1][0]), "=&v"(v[1][1]), "=&v"(v[2][0]), "=&v"(v[2][1]), "=&v"(v[3][0]),
+                 "=&v"(v[3][1]), "=&v"(v[4][0]), "=&v"(v[4][1]), "=&v"(v[5][0]), "=&v"(v[5][1]), "=&v"(v[6][0]), "=&v"(v[6][1]),
+                 "=&v"(v[7][0]), "=&v"(v[7][1])
+               : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "n"(OFF), "n"(OFF + 4096)
+               : "memory");
+}
+
+template <int W>
+__global__ void __launch_bounds__(W * 64, W == 8 ? 4 : 2)
 attn_prefill_kernel(const AttnPrefillParams p) {
-  __shared__ __align__(16) uint16_t ks[64 * AP_KP];
-  __shared__ __align__(16) uint16_t vt[128 * AP_VP];
-  constexpr int QB = 64 * QG; // queries per workgroup
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int STAGE = 32768, QG = 1; // QG: query groups of 16 per wave
+  __shared__ __align__(16) uint8_t lds[2 * STAGE]; // per stage: K [64 keys][256 B] | V [64 keys][256 B]
+  constexpr int QB = 16 * QG * W; // queries per workgroup
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c = lane & 15;
-  const int bh = blockIdx.y, b = bh / p.Nq, hq = bh - b * p.Nq;
-  const int hk = hq / (p.Nq / p.Nkv);
   // The last query blocks see the most keys: start them first.  Two workgroups share a CU, and the dispatcher puts
-  // workgroup i + 256 beside workgroup i: the heads of every other run of 256 workgroups walk their query blocks
-  // the other way round, so that a long block meets a short one instead of its twin of another head.  (One order
-  // per head -- taken from the head's first workgroup -- or a run boundary inside a head would visit some blocks
-  // twice and others never.)
-  const int wg0 = (int)(blockIdx.y * gridDim.x);
-  const int qblk = ((wg0 >> 8) & 1) ? (int)blockIdx.x : (int)gridDim.x - 1 - (int)blockIdx.x;
+  // workgroup i + 256 beside workgroup i: every other run of whole query blocks within 256 workgroups is walked the other way
+  // round, so that a long block meets a short one.  Heads go round the XCDs, those of one K/V head to the same one.
+  const int heads = p.B * p.Nq, nblk = (p.S + QB - 1) / QB;
+  const int per = heads < 256 ? 256 / heads : 1;
+  int k = (int)blockIdx.x / heads;
+  if (const int chunk = k / per; (chunk & 1) && (chunk + 1) * per <= nblk)
+    k = chunk * per + per - 1 - k % per;
+  const int qblk = nblk - 1 - k, bh = (int)blockIdx.x % heads, b = bh / p.Nq;
+  const int hr = bh - b * p.Nq, hk = hr % p.Nkv, hq = hk * (p.Nq / p.Nkv) + hr / p.Nkv;
   const int q0 = qblk * QB + wave * (16 * QG);
   const int last_key = p.past + p.S - 1;
 
+  const float scale2 = p.scale * 1.44269504f; // scores in the base-2 domain; positive
   int qpos[QG]; // last key this lane's query of group qg sees (rows past the end repeat the last query, never stored)
   bf16x8 qreg[QG][4];
 #pragma unroll
@@ -898,42 +935,35 @@ attn_prefill_kernel(const AttnPrefillParams p) {
     for (int j = 0; j < 4; j++)
       qreg[qg][j] = *reinterpret_cast<const bf16x8*>(qrow + j * 32 + g * 8);
   }
-  const uint16_t* kbase = p.kc + ((int64_t)b * p.Nkv + hk) * p.Smax * 128;
-  const uint16_t* vbase = p.vc + ((int64_t)b * p.Nkv + hk) * p.Smax * 128;
+  const int64_t head = ((int64_t)b * p.Nkv + hk) * p.Smax * 128;
   const uint16_t* mrow = p.mask ? p.mask + (int64_t)b * p.mask_ld : nullptr;
 
-  // staging registers: K rows chunk-fastest (coalesced); V: a thread takes one 16-byte chunk (8 dims) of FOUR
-  // consecutive keys, so that the transposed image is written as 8 x 8 bytes (4 keys of one dim, packed with two
-  // byte permutes) instead of 32 two-byte writes
-  i32x4 kst[4], vst[4];
-  const int vq = tid & 15, vch = tid >> 4; // key quad, chunk
-  auto load_tile = [&](int kb) {
+  constexpr int NP = 16 / W; // pieces of 4 rows x 256 B of K and of V that a wave brings (rows past the last key repeat it)
+  auto request = [&](int kb, int stage) {
+    const int64_t at = head + (int64_t)kb * (64 * 128); // (a descriptor per tile: no limit on the keys of a head)
+    const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.kc + at), 0, 0xffffffffu, 0x00020000);
+    const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.vc + at), 0, 0xffffffffu, 0x00020000);
+    const int rows = last_key - kb * 64;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int idx = tid + i * 256;
-      const int kk = min(kb * 64 + (idx >> 4), last_key);
-      kst[i] = *reinterpret_cast<const i32x4*>(kbase + (int64_t)kk * 128 + (idx & 15) * 8);
-      const int kv = min(kb * 64 + vq * 4 + i, last_key);
-      vst[i] = *reinterpret_cast<const i32x4*>(vbase + (int64_t)kv * 128 + vch * 8);
+    for (int i = 0; i < NP; i++) {
+      const int pc = wave * NP + i;
+      const uint32_t row = (uint32_t)min(pc * 4 + g, rows) * 256u;
+      uint8_t* const dst = lds + stage * STAGE + pc * 1024;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (__attribute__((address_space(3))) void*)dst, 16, row + (uint32_t)(c ^ ((pc & 3) * 4 + g)) * 16u, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (__attribute__((address_space(3))) void*)(dst + 16384), 16, row + (uint32_t)(c ^ (((pc & 1) * 4 + g) * 2)) * 16u, 0, 0, 0);
     }
   };
-  auto store_tile = [&]() {
+  uint32_t kaddr[4], vaddr[8]; // this lane's operands inside a stage: K chunk j * 4 + g of row c; V dims dt * 16 .. + 15
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int idx = tid + i * 256;
-      *reinterpret_cast<i32x4*>(ks + (idx >> 4) * AP_KP + (idx & 15) * 8) = kst[i];
-    }
+  for (int j = 0; j < 4; j++)
+    kaddr[j] = (uint32_t)(c * 256 + (((j * 4 + g) ^ c) & 15) * 16);
+  {
+    const int r = g * 4 + (c >> 2); // key of this lane's 8 bytes inside a run of 16
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      // dim vch*8 + e of keys 4*vq .. 4*vq+3: the low (e even) or high (e odd) halves of dword e/2 of the four rows
-      const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
-      const uint32_t lo = __builtin_amdgcn_perm((uint32_t)vst[1][e >> 1], (uint32_t)vst[0][e >> 1], sel);
-      const uint32_t hi = __builtin_amdgcn_perm((uint32_t)vst[3][e >> 1], (uint32_t)vst[2][e >> 1], sel);
-      *reinterpret_cast<uint2*>(vt + (vch * 8 + e) * AP_VP + vq * 4) = make_uint2(lo, hi);
-    }
-  };
+    for (int dt = 0; dt < 8; dt++)
+      vaddr[dt] = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(r * 256 + ((dt * 2 + ((c >> 1) & 1)) ^ ((r & 7) * 2)) * 16 + (c & 1) * 8);
+  }
 
-  const float scale2 = p.scale * 1.44269504f;
   float m[QG], l[QG];
   f32x4 acc[QG][8];
 #pragma unroll
@@ -946,13 +976,15 @@ attn_prefill_kernel(const AttnPrefillParams p) {
   }
   // key tiles up to the one holding the last key of the workgroup's last query (the same for all four waves)
   const int nkb = (p.past + min(qblk * QB + QB - 1, p.S - 1)) / 64 + 1;
-  load_tile(0);
-  for (int kb = 0; kb < nkb; kb++) {
-    __syncthreads(); // the previous tile has been read by every wave
-    store_tile();
-    __syncthreads();
+  auto tile = [&](auto STAGE_, int kb) {
+    constexpr int stage = decltype(STAGE_)::value, V_AT = stage * STAGE + 16384;
+    // this tile has landed and the other stage has been read, for this wave and then for every wave
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
     if (kb + 1 < nkb)
-      load_tile(kb + 1); // in flight during the arithmetic below
+      request(kb + 1, stage ^ 1); // in flight during the arithmetic below
+    if (kb * 64 > p.past + q0 + 16 * QG - 1)
+      return; // past the causal edge of all of this wave's queries
+    const uint8_t* st = lds + stage * STAGE;
 
     f32x4 sc[QG][4];
 #pragma unroll
@@ -962,27 +994,24 @@ attn_prefill_kernel(const AttnPrefillParams p) {
         sc[qg][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(ks + (t * 16 + c) * AP_KP + j * 32 + g * 8);
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(st + kaddr[j] + t * 4096);
 #pragma unroll
         for (int qg = 0; qg < QG; qg++)
           sc[qg][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qreg[qg][j], sc[qg][t], 0, 0, 0);
       }
     }
-    // Scores in the base-2 domain (scale * log2 e folded into one multiplier): a probability is one exp2.  The
-    // additive mask is read only when there is one (wave-uniform branch: no addresses, no predicated loads).
-#pragma unroll
-    for (int qg = 0; qg < QG; qg++)
-#pragma unroll
-      for (int t = 0; t < 4; t++)
-        sc[qg][t] *= scale2;
+    // The additive mask is read only when there is one (wave-uniform branch: no addresses, no predicated loads).
+    float sl = scale2;
     if (mrow) {
+      sl = 1.0f;
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         const int key = kb * 64 + (i >> 2) * 16 + g * 4 + (i & 3);
-        const float mk = key < p.mask_ld ? bf16_bits_to_f32(mrow[key]) * 1.44269504f : 0.f;
+        const float mv = bf16_bits_to_f32(mrow[min(key, p.mask_ld - 1)]) * 1.44269504f; // (no branch per key)
+        const float mk = key < p.mask_ld ? mv : 0.f;
 #pragma unroll
         for (int qg = 0; qg < QG; qg++)
-          sc[qg][i >> 2][i & 3] += mk;
+          sc[qg][i >> 2][i & 3] = fmaf(sc[qg][i >> 2][i & 3], scale2, mk);
       }
     }
     bf16x8 pb[QG][2];
@@ -1000,59 +1029,70 @@ attn_prefill_kernel(const AttnPrefillParams p) {
             sc[qg][t][r] = key <= qpos[qg] ? sc[qg][t][r] : -INFINITY;
           }
       }
-      float mx = -3.0e38f;
+      float mx = -INFINITY;
 #pragma unroll
       for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int r = 0; r < 4; r++)
           mx = fmaxf(mx, sc[qg][t][r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mn = fmaxf(m[qg], mx); // finite from the first tile on: key 0 is visible to every query
-      const float alpha = __builtin_amdgcn_exp2f(m[qg] - mn);
-      l[qg] *= alpha;
+      mx *= sl;
+      if (__builtin_amdgcn_ballot_w64(mx > m[qg] + 8.0f) != 0) { // always in the first tile, seldom after it
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float mn = fmaxf(m[qg], ceilf(mx)); // finite from the first tile on: key 0 is visible to every query
+        const float alpha = __builtin_amdgcn_exp2f(m[qg] - mn);
+        l[qg] *= alpha;
 #pragma unroll
-      for (int dt = 0; dt < 8; dt++)
-        acc[qg][dt] *= alpha;
+        for (int dt = 0; dt < 8; dt++)
+          acc[qg][dt] *= alpha;
+        m[qg] = mn;
+      }
+      float ls[2] = {0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < 2; u++)
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-          const float pr = __builtin_amdgcn_exp2f(sc[qg][2 * u + (j >> 2)][j & 3] - mn);
-          l[qg] += pr;
+          const float pr = __builtin_amdgcn_exp2f(fmaf(sc[qg][2 * u + (j >> 2)][j & 3], sl, -m[qg]));
+          ls[u] += pr;
           pb[qg][u][j] = (__bf16)pr;
         }
-      m[qg] = mn;
+      l[qg] += ls[0] + ls[1];
     }
+    // K slots g*8 .. g*8+7 of the operand = keys u*32 + g*4 .. +3 and u*32 + 16 + g*4 .. +3 of the tile, the keys pb[.][u]
+    // holds in the same slots
+    static_for<0, 2>([&](auto U) {
+      constexpr int u = decltype(U)::value;
+      i32x2 vv[8][2];
+      read_v_operands<V_AT + u * 8192>(vv, vaddr);
 #pragma unroll
-    for (int dt = 0; dt < 8; dt++)
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        // K slots g*8 .. g*8+7 of the operand = keys u*32 + g*4 .. +3 and u*32 + 16 + g*4 .. +3 of the tile,
-        // the keys pb[.][u] holds in the same slots
-        const uint16_t* vrow = vt + (dt * 16 + c) * AP_VP + u * 32 + g * 4;
-        const uint2 lo = *reinterpret_cast<const uint2*>(vrow), hi = *reinterpret_cast<const uint2*>(vrow + 16);
-        const i32x4 av = {(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
+      for (int dt = 0; dt < 8; dt++) {
+        const i32x4 av = {vv[dt][0][0], vv[dt][0][1], vv[dt][1][0], vv[dt][1][1]};
 #pragma unroll
         for (int qg = 0; qg < QG; qg++)
           acc[qg][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), pb[qg][u], acc[qg][dt], 0, 0, 0);
       }
+    });
+  };
+  request(0, 0);
+  for (int kb = 0; kb < nkb; kb += 2) {
+    tile(std::integral_constant<int, 0>{}, kb);
+    if (kb + 1 < nkb)
+      tile(std::integral_constant<int, 1>{}, kb + 1);
   }
 #pragma unroll
   for (int qg = 0; qg < QG; qg++) {
     float ls = l[qg];
     ls += __shfl_xor(ls, 16);
     ls += __shfl_xor(ls, 32);
+    const float inv = ls > 0.f ? 1.0f / ls : 0.f;
     const int qi = q0 + qg * 16 + c;
     if (qi < p.S) {
       uint16_t* orow = p.out + (((int64_t)b * p.S + qi) * p.Nq + hq) * 128;
 #pragma unroll
       for (int dt = 0; dt < 8; dt++) {
-        uint32_t w[2];
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-          w[h] = f32x2_to_bf16_bits(ls > 0.f ? acc[qg][dt][2 * h] / ls : 0.f, ls > 0.f ? acc[qg][dt][2 * h + 1] / ls : 0.f);
-        *reinterpret_cast<uint2*>(orow + dt * 16 + g * 4) = make_uint2(w[0], w[1]);
+        const f32x4 o = acc[qg][dt] * inv;
+        *reinterpret_cast<uint2*>(orow + dt * 16 + g * 4) =
+            ls > 0.f ? make_uint2(f32x2_to_bf16_bits(o[0], o[1]), f32x2_to_bf16_bits(o[2], o[3])) : make_uint2(0, 0);
       }
     }
   }
@@ -1959,14 +1999,13 @@ extern "C" int tppx_attn_prefill(const void* q, const void* kcache, const void* 
       return check_hip(e, who);
     return check_hip(hipGetLastError(), who);
   }
-  // 32 queries per wave (QG = 2) halve the LDS reads per MFMA at 226 registers, still two waves per SIMD; they win
-  // when the launch still has two workgroups per CU (S = 2048, 32 heads: 97 us against 117 us; 16 x 128 queries
-  // behind 1024 cached keys: 69 against 96 us) and lose below that (S = 512, 32 heads: 22.5 against 17 us)
-  const long wgs2 = ((S + 127) / 128) * B * Nq;
-  const int qg = env_int("TPPX_ATTN_QG", wgs2 >= 512 ? 2 : 1);
-  if (qg == 2 && S > 64)
-    attn_prefill_kernel<2><<<dim3((unsigned)((S + 127) / 128), (unsigned)(B * Nq)), dim3(256), 0, (hipStream_t)stream>>>(p);
-  else
-    attn_prefill_kernel<1><<<dim3((unsigned)((S + 63) / 64), (unsigned)(B * Nq)), dim3(256), 0, (hipStream_t)stream>>>(p);
-  return check_hip(hipGetLastError(), who);
+  // 128 queries per workgroup from 400 of them on (3 x 600 tokens behind 500 x 28 heads, 420 of them: 34.7 us against 40.9);
+  // below that twice as many of 64 (1000 tokens x 32 heads, 256: 22.7 against 20.0; 2 x 700, 384: 21.1 against 19.7)
+  const int64_t wgs = (S + 127) / 128 * B * Nq;
+  const bool wide = env_int("TPPX_ATTN_QG", wgs >= 400 ? 2 : 1) == 2;
+  auto go = [&](auto kern, int64_t rows, int threads) -> hipError_t {
+    kern<<<dim3((unsigned)((S + rows - 1) / rows * B * Nq)), dim3(threads), 0, (hipStream_t)stream>>>(p);
+    return hipGetLastError();
+  };
+  return check_hip(wide && S > 64 ? go(attn_prefill_kernel<8>, 128, 512) : go(attn_prefill_kernel<4>, 64, 256), who);
 }

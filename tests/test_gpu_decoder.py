@@ -243,8 +243,8 @@ def test_attn_prefill(B, S, Nq, Nkv, past, Smax, queries_per_wave, monkeypatch):
 @pytest.mark.parametrize("rise", [0.5, 7.0, 40.0, -7.0])
 @pytest.mark.parametrize("queries_per_wave", [16, 32])
 def test_attn_prefill_running_maximum(rise, queries_per_wave, monkeypatch):
-    """The running maximum moves only when a score exceeds it by 8 (base 2): scores that rise along the keys by less and by
-    more than that per key tile, and that fall, over grouped heads, one query of a workgroup far above the others, against
+    """Sums are rescaled only in tiles where some query's running maximum moves: scores that rise along the keys by less and by
+    more than a binade per key tile, and that fall, over grouped heads, one query of a workgroup far above the others, against
     softmax attention in float64 (probabilities and outputs rounded to bf16: 2^-8 each)."""
     _llm()
     monkeypatch.setenv("TPPX_ATTN_QG", str(queries_per_wave // 16))

@@ -864,15 +864,15 @@ constexpr int AP_VP = 68; // LDS row pitch of the hd kernel's V^T tile (64 keys 
 // fall on different bank groups.  V's operand is read by the transposing LDS read: of a 16-lane group lane i fetches 8 bytes
 // of key (i >> 2) and gets the four keys of dim i.
 // What bounds it is the chain scores -> softmax -> output of a wave, not one unit (MFMA a third busy, vector issue a half), so
-// waves per SIMD count more than operand reads per MFMA: 32 queries per wave, half the reads, take 57 us where this takes
-// 50 (2048 tokens x 32 heads).  And the vector instructions per score: the running maximum is a power of two's exponent (an
-// integer in the base-2 domain) and moves only when a score exceeds it by 8; within that a probability is at most 2^8, sums
-// and outputs scale exactly, and a tile needs no maximum across lanes and no rescaling of the output sums.  The scaling being
-// exact, a query's result does not depend on when it moves, that is on the other queries of its wave.
-// Measured against registers in between, V transposed by byte permutes and a maximum per tile: 2048 tokens x 32 heads
-// 71 -> 49.5 us, 64 heads on 8 of K/V 129 -> 83, 1000 x 32 26.7 -> 20.0, 333 x 32 12.6 -> 8.4.  Tried beside it: the next
-// tile's scores under this one's softmax in a wave (256 registers and scratch), two halves of the keys on eight waves (54.8),
-// the same half a turn apart (60).
+// waves per SIMD count more than operand reads per MFMA (32 queries per wave, half the reads: 57 us where 16 took 50).  The
+// tile's maximum is taken across lanes and the sums are rescaled only where some query's running maximum moves, everything
+// else being a factor of exactly 1: the bits of doing it in every tile.
+// Measured against registers in between, V transposed by byte permutes and a rescaling per tile: 2048 tokens x 32 heads
+// 74 -> 57.5 us, 64 heads on 8 of K/V 152 -> 88, 1000 x 32 28 -> 22.3, 333 x 32 12.6 -> 9.9, 3 x 600 behind 500 with a mask 107
+// -> 48.5 (the mask was read under a branch per key).
+// Tried beside it: a running maximum that is a power of two and moves by 8 at a time, exact as well but with other roundings
+// of the probabilities (49.5); the next tile's scores under this one's softmax in a wave (256 registers and scratch); two
+// halves of the keys on eight waves (54.8), the same half a turn apart (60).
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 // The transposing reads of 32 keys' V operands (8 dim tiles x 2 runs of 16 keys), issued and waited for in one block: around
 // the builtin the compiler waits for every load into LDS under way, that is for the next tile.
@@ -894,12 +894,25 @@ __device__ __forceinline__ void read_v_operands(i32x2 (&v)[8][2], const uint32_t
                : "memory");
 }
 
+// maximum over the four 16-lane groups: swapped with itself a register gives both halves, no trip through the LDS
+__device__ __forceinline__ float max_of_groups(float v) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// a product that is not fused into what follows it
+__device__ __forceinline__ float scaled(float v, float by) {
+#pragma clang fp contract(off)
+  return v * by;
+}
+
 template <int W>
 __global__ void __launch_bounds__(W * 64, W == 8 ? 4 : 2)
 attn_prefill_kernel(const AttnPrefillParams p) {
-  constexpr int STAGE = 32768, QG = 1; // QG: query groups of 16 per wave
+  constexpr int STAGE = 32768;
   __shared__ __align__(16) uint8_t lds[2 * STAGE]; // per stage: K [64 keys][256 B] | V [64 keys][256 B]
-  constexpr int QB = 16 * QG * W; // queries per workgroup
+  constexpr int QB = 16 * W; // queries per workgroup
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c = lane & 15;
@@ -913,21 +926,16 @@ attn_prefill_kernel(const AttnPrefillParams p) {
     k = chunk * per + per - 1 - k % per;
   const int qblk = nblk - 1 - k, bh = (int)blockIdx.x % heads, b = bh / p.Nq;
   const int hr = bh - b * p.Nq, hk = hr % p.Nkv, hq = hk * (p.Nq / p.Nkv) + hr / p.Nkv;
-  const int q0 = qblk * QB + wave * (16 * QG);
+  const int q0 = qblk * QB + wave * 16;
   const int last_key = p.past + p.S - 1;
 
   const float scale2 = p.scale * 1.44269504f; // scores in the base-2 domain; positive
-  int qpos[QG]; // last key this lane's query of group qg sees (rows past the end repeat the last query, never stored)
-  bf16x8 qreg[QG][4];
+  const int qi = min(q0 + c, p.S - 1), qpos = p.past + qi; // this lane's query and the last key it sees (past the end: the last one, not stored)
+  const uint16_t* qrow = p.q + (((int64_t)b * p.S + qi) * p.Nq + hq) * 128;
+  bf16x8 qreg[4];
 #pragma unroll
-  for (int qg = 0; qg < QG; qg++) {
-    const int qi = min(q0 + qg * 16 + c, p.S - 1);
-    qpos[qg] = p.past + qi;
-    const uint16_t* qrow = p.q + (((int64_t)b * p.S + qi) * p.Nq + hq) * 128;
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      qreg[qg][j] = *reinterpret_cast<const bf16x8*>(qrow + j * 32 + g * 8);
-  }
+  for (int j = 0; j < 4; j++)
+    qreg[j] = *reinterpret_cast<const bf16x8*>(qrow + j * 32 + g * 8);
   const int64_t head = ((int64_t)b * p.Nkv + hk) * p.Smax * 128;
   const uint16_t* mrow = p.mask ? p.mask + (int64_t)b * p.mask_ld : nullptr;
 
@@ -957,16 +965,11 @@ attn_prefill_kernel(const AttnPrefillParams p) {
       vaddr[dt] = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(r * 256 + ((dt * 2 + ((c >> 1) & 1)) ^ ((r & 7) * 2)) * 16 + (c & 1) * 8);
   }
 
-  float m[QG], l[QG];
-  f32x4 acc[QG][8];
+  float m = -3.0e38f, l = 0.f;
+  f32x4 acc[8];
 #pragma unroll
-  for (int qg = 0; qg < QG; qg++) {
-    m[qg] = -3.0e38f;
-    l[qg] = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < 8; dt++)
-      acc[qg][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int dt = 0; dt < 8; dt++)
+    acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   // key tiles up to the one holding the last key of the workgroup's last query (the same for all four waves)
   const int nkb = (p.past + min(qblk * QB + QB - 1, p.S - 1)) / 64 + 1;
   auto tile = [&](auto STAGE_, int kb) {
@@ -975,82 +978,69 @@ attn_prefill_kernel(const AttnPrefillParams p) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
     if (kb + 1 < nkb)
       request(kb + 1, stage ^ 1); // in flight during the arithmetic below
-    if (kb * 64 > p.past + q0 + 16 * QG - 1)
+    if (kb * 64 > p.past + q0 + 15)
       return; // past the causal edge of all of this wave's queries
     const uint8_t* st = lds + stage * STAGE;
 
-    f32x4 sc[QG][4];
+    f32x4 sc[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) {
+      sc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int qg = 0; qg < QG; qg++)
-        sc[qg][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(st + kaddr[j] + t * 4096);
-#pragma unroll
-        for (int qg = 0; qg < QG; qg++)
-          sc[qg][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qreg[qg][j], sc[qg][t], 0, 0, 0);
-      }
+      for (int j = 0; j < 4; j++)
+        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(st + kaddr[j] + t * 4096), qreg[j], sc[t], 0, 0, 0);
     }
+    // Scores in the base-2 domain (scale * log2 e folded into one multiplier, the product rounded): a probability is one exp2.
     // The additive mask is read only when there is one (wave-uniform branch: no addresses, no predicated loads).
-    float sl = scale2;
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        sc[t][r] = scaled(sc[t][r], scale2);
     if (mrow) {
-      sl = 1.0f;
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         const int key = kb * 64 + (i >> 2) * 16 + g * 4 + (i & 3);
         const float mv = bf16_bits_to_f32(mrow[min(key, p.mask_ld - 1)]) * 1.44269504f; // (no branch per key)
-        const float mk = key < p.mask_ld ? mv : 0.f;
-#pragma unroll
-        for (int qg = 0; qg < QG; qg++)
-          sc[qg][i >> 2][i & 3] = fmaf(sc[qg][i >> 2][i & 3], scale2, mk);
+        sc[i >> 2][i & 3] += key < p.mask_ld ? mv : 0.f;
       }
     }
-    bf16x8 pb[QG][2];
     // only the tiles that reach past the position of this wave's first query hide anything (wave-uniform)
-    const bool edge = kb * 64 + 63 > p.past + q0;
-#pragma unroll
-    for (int qg = 0; qg < QG; qg++) {
-      if (edge) {
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int key = kb * 64 + t * 16 + g * 4 + r;
-            // keys past the causal edge get -inf, whose exp2 is exactly 0 against the finite running maximum
-            sc[qg][t][r] = key <= qpos[qg] ? sc[qg][t][r] : -INFINITY;
-          }
-      }
-      float mx = -INFINITY;
+    if (kb * 64 + 63 > p.past + q0) {
 #pragma unroll
       for (int t = 0; t < 4; t++)
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-          mx = fmaxf(mx, sc[qg][t][r]);
-      mx *= sl;
-      if (__builtin_amdgcn_ballot_w64(mx > m[qg] + 8.0f) != 0) { // always in the first tile, seldom after it
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float mn = fmaxf(m[qg], ceilf(mx)); // finite from the first tile on: key 0 is visible to every query
-        const float alpha = __builtin_amdgcn_exp2f(m[qg] - mn);
-        l[qg] *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < 8; dt++)
-          acc[qg][dt] *= alpha;
-        m[qg] = mn;
-      }
-      float ls[2] = {0.f, 0.f};
-#pragma unroll
-      for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          const float pr = __builtin_amdgcn_exp2f(fmaf(sc[qg][2 * u + (j >> 2)][j & 3], sl, -m[qg]));
-          ls[u] += pr;
-          pb[qg][u][j] = (__bf16)pr;
+        for (int r = 0; r < 4; r++) {
+          const int key = kb * 64 + t * 16 + g * 4 + r;
+          // keys past the causal edge get -inf, whose exp2 is exactly 0 against the finite running maximum
+          sc[t][r] = key <= qpos ? sc[t][r] : -INFINITY;
         }
-      l[qg] += ls[0] + ls[1];
     }
+    float mx = -3.0e38f;
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        mx = fmaxf(mx, sc[t][r]);
+    float alpha = 1.0f;
+    if (__builtin_amdgcn_ballot_w64(mx > m) != 0) { // some query's maximum moves (otherwise every factor below is 1)
+      mx = max_of_groups(mx);
+      const float mn = fmaxf(m, mx); // finite from the first tile on: key 0 is visible to every query
+      alpha = __builtin_amdgcn_exp2f(m - mn);
+#pragma unroll
+      for (int dt = 0; dt < 8; dt++)
+        acc[dt] *= alpha;
+      m = mn;
+    }
+    bf16x8 pb[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float pr = __builtin_amdgcn_exp2f(sc[2 * u + (j >> 2)][j & 3] - m);
+        l = u == 0 && j == 0 ? fmaf(l, alpha, pr) : l + pr;
+        pb[u][j] = (__bf16)pr;
+      }
     // K slots g*8 .. g*8+7 of the operand = keys u*32 + g*4 .. +3 and u*32 + 16 + g*4 .. +3 of the tile, the keys pb[.][u]
     // holds in the same slots
     static_for<0, 2>([&](auto U) {
@@ -1060,9 +1050,7 @@ attn_prefill_kernel(const AttnPrefillParams p) {
 #pragma unroll
       for (int dt = 0; dt < 8; dt++) {
         const i32x4 av = {vv[dt][0][0], vv[dt][0][1], vv[dt][1][0], vv[dt][1][1]};
-#pragma unroll
-        for (int qg = 0; qg < QG; qg++)
-          acc[qg][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), pb[qg][u], acc[qg][dt], 0, 0, 0);
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), pb[u], acc[dt], 0, 0, 0);
       }
     });
   };
@@ -1072,21 +1060,17 @@ attn_prefill_kernel(const AttnPrefillParams p) {
     if (kb + 1 < nkb)
       tile(std::integral_constant<int, 1>{}, kb + 1);
   }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (q0 + c < p.S) {
+    uint16_t* orow = p.out + (((int64_t)b * p.S + q0 + c) * p.Nq + hq) * 128;
 #pragma unroll
-  for (int qg = 0; qg < QG; qg++) {
-    float ls = l[qg];
-    ls += __shfl_xor(ls, 16);
-    ls += __shfl_xor(ls, 32);
-    const float inv = ls > 0.f ? 1.0f / ls : 0.f;
-    const int qi = q0 + qg * 16 + c;
-    if (qi < p.S) {
-      uint16_t* orow = p.out + (((int64_t)b * p.S + qi) * p.Nq + hq) * 128;
+    for (int dt = 0; dt < 8; dt++) {
+      uint32_t w[2];
 #pragma unroll
-      for (int dt = 0; dt < 8; dt++) {
-        const f32x4 o = acc[qg][dt] * inv;
-        *reinterpret_cast<uint2*>(orow + dt * 16 + g * 4) =
-            ls > 0.f ? make_uint2(f32x2_to_bf16_bits(o[0], o[1]), f32x2_to_bf16_bits(o[2], o[3])) : make_uint2(0, 0);
-      }
+      for (int e = 0; e < 2; e++)
+        w[e] = f32x2_to_bf16_bits(l > 0.f ? acc[dt][2 * e] / l : 0.f, l > 0.f ? acc[dt][2 * e + 1] / l : 0.f);
+      *reinterpret_cast<uint2*>(orow + dt * 16 + g * 4) = make_uint2(w[0], w[1]);
     }
   }
 }
@@ -2006,8 +1990,8 @@ extern "C" int tppx_attn_prefill(const void* q, const void* kcache, const void* 
       return check_hip(e, who);
     return check_hip(hipGetLastError(), who);
   }
-  // 128 queries per workgroup from 400 of them on (3 x 600 tokens behind 500 x 28 heads, 420 of them: 34.7 us against 40.9);
-  // below that twice as many of 64 (1000 tokens x 32 heads, 256: 22.7 against 20.0; 2 x 700, 384: 21.1 against 19.7)
+  // 128 queries per workgroup from 400 of them on (3 x 600 tokens behind 500 x 28 heads, 420 of them: 15 % faster); below that
+  // twice as many of 64 (1000 tokens x 32 heads, 256: 12 % faster, 2 x 700, 384: 7 %)
   const int64_t wgs = (S + 127) / 128 * B * Nq;
   const bool wide = env_int("TPPX_ATTN_QG", wgs >= 400 ? 2 : 1) == 2;
   auto go = [&](auto kern, int64_t rows, int threads) -> hipError_t {

@@ -1141,3 +1141,21 @@ def test_prefill_mxfp4_takes_scales_at_any_address(off, M, N, K, monkeypatch):
         monkeypatch.setenv("TPPX_TILED_BIG_TILE", tile)
         for a, b in zip(run(), want):
             assert torch.equal(a, b), tile
+
+
+@pytest.mark.parametrize("M", [9, 16, 17, 31, 33, 50, 64, 70])
+@pytest.mark.parametrize("tiles", [1, 8, 13, 24, 33, 47])
+def test_mxfp4_row_groups_at_every_number_of_k_tiles_per_wave(M, tiles):
+    """The MXFP4 kernel for 17..64 rows (and for fewer where K does not suit the LDS-staged ones): waves without K tiles,
+    with one, two, three and more, odd and even counts in one workgroup, rows past M; the GEMM
+    against the oracle, the gate/up pair against its two GEMMs one after the other (the same three roundings to bf16, of
+    sums in another order)."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    K = 128 * tiles
+    _, _, _, ctx = _run("mxfp4", M, 96, K, "add", True, 700 + tiles, flags=_lib.FLAG_FORCE_SKINNY)
+    wg, x = ctx[0], ctx[3].cuda()
+    wu = _make("mxfp4", 96, K, 770 + tiles)[0]
+    want = ops.fc_mul(x, wu, None, ops.fc_silu(x, wg, None)).float()
+    got = ops.swiglu_gate_up(x, wg, wu).float()
+    assert ((got - want).norm() / want.norm()).item() < 3 * 2.0 ** -9

@@ -28,6 +28,12 @@
 
 namespace tppx {
 
+// Raw byte addressing (exact waits, the scalar part of an address for free) with a range check that cuts nothing off:
+// callers clamp their offsets to the tensor.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_rsrc(const void* q) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(q), 0, 0xffffffffu, 0x00020000);
+}
+
 __device__ __forceinline__ bf16x8 sk_cvt_fp4x8(uint32_t codes, float scale) {
   bf16x2 c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, scale, 0);
   bf16x2 c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, scale, 1);
@@ -2192,107 +2198,84 @@ skinny_mxfp4_x4_kernel(const DecodeParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// MXFP4 weight-only, 17..64 rows: MG row groups of 16 per workgroup.
-// Eight waves split K.  A wave walks its K tiles one at a time: the bf16
-// activations of the tile (MG*16 rows x 256 B, row-contiguous 16-byte loads,
-// requested a tile ahead into registers) are written to the wave's private
-// LDS region in MFMA operand order -- slot (chunk, row) = chunk*MPAD + (row ^
-// chunk), the same conflict-free image the 16-row kernel uses -- and read back
-// as A operands; every dequantised weight operand feeds MG MFMAs.  No barrier
-// before the final cross-wave reduction, no operand-shaped global loads, no
-// second kernel.  The epilogue's reduction scratch reuses the activation
-// regions.
+// MXFP4 weight-only, 17..64 rows (and fewer where K is too long for the LDS-staged kernels): MG row groups of 16 per
+// workgroup.  W waves split K.  A wave walks its K tiles in units of UG row groups: the bf16 activations of a unit
+// (UG*16 rows x 256 B) go straight from global memory to one of the two slots of the wave's private LDS region, no
+// registers in between, and are read back as A operands; the weights of two K tiles are in registers or under way.
+// LDS image of a row group: row r at r*256, its 16-byte chunk c at (c ^ r)*16 -- a load instruction fills four rows from
+// eight whole 128-byte lines, and the 16 lanes that read one chunk of 16 rows hit 16 different bank groups.
+// No barrier before the final cross-wave reduction, whose scratch reuses the activation regions.
+// What bounds it: at 50 rows of a 4096 -> 2 x 11008 pair the loop's 768 MFMAs per SIMD are 7 us and the 720 KB a CU takes
+// in 6, side by side; the rest of 20.3 us is the launch, the first loads' latency, and the sums over the waves.  Activations
+// staged through registers, with a tile's weights requested when the one before was done (there was no room for more), took
+// 23.2; 32 rows 15.4 against 17.0; singles of 50 rows: 4096 x 4096 9.5 against 11.0, 16384 x 2560 19.3 against 22.6; 8 rows
+// of 18944 x 3584 (MG = 1) 11.4 against 16.1.  Requests past a wave's last tile, out of a resource's range so that every wait
+// counts the same loads, cost 1 to 2 us: each takes its turn in the address unit.
 // ---------------------------------------------------------------------------
-template <int MG, int NT, bool DUAL, int PF, int W = 8, bool XLATE = false>
+template <int MG, int NT, bool DUAL, int W = 8>
 __global__ void __launch_bounds__(W * 64)
 skinny_mxfp4_mg_kernel(const DecodeParams p) {
   extern __shared__ __align__(16) float sk_lds[];
-  constexpr int MPAD = MG * 16, XL = MG * 4;
+  constexpr int UG = MG >= 2 ? 2 : 1, NU = MG / UG, NX = UG * 4; // row groups per unit, units per K tile, loads per unit
   constexpr int NTW = DUAL ? 2 * NT : NT; // DUAL: the gate AND the up tile of each channel tile (gate tiles first)
+  constexpr int WN = 2 * NTW;             // loads of a K tile's weights: codes and scales
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int grp = blockIdx.x;
   const int seg_id = DUAL ? 0 : sk_find_seg(p, grp);
   const DecodeSeg& sg = p.seg[seg_id];
   const int ltile0 = (grp - sg.grp0) * NT;
-  const int m0 = blockIdx.y * MPAD;
+  const int m0 = blockIdx.y * (MG * 16);
   const int KT = p.units;
   // K tiles of this workgroup (all of them unless K is split across workgroups), then of this wave
-  const int tb = sk_share(blockIdx.z, KT, p.S), te = sk_share(blockIdx.z + 1, KT, p.S);
+  const int tb = sk_share_pow2(blockIdx.z, KT, p.S), te = sk_share_pow2(blockIdx.z + 1, KT, p.S);
   const int t0 = tb + (wave * (te - tb)) / W, t1 = tb + ((wave + 1) * (te - tb)) / W;
-  i32x4* xs = reinterpret_cast<i32x4*>(sk_lds) + (size_t)wave * (MPAD * 16); // [chunk 16][row MPAD] x 16 B
+  char* xs = reinterpret_cast<char*>(sk_lds) + wave * (2 * UG * 4096);
 
   constexpr int NSEG = DUAL ? 2 : 1;
-  const char* qwb[NSEG];
-  const char* swb[NSEG];
+  __amdgpu_buffer_rsrc_t wr[NSEG], swr[NSEG];
 #pragma unroll
-  for (int sgi = 0; sgi < NSEG; sgi++) {
-    const DecodeSeg& ss = p.seg[DUAL ? sgi : seg_id];
-    qwb[sgi] = reinterpret_cast<const char*>(ss.qw);
-    swb[sgi] = reinterpret_cast<const char*>(ss.sw);
+  for (int i = 0; i < NSEG; i++) {
+    const DecodeSeg& ss = p.seg[DUAL ? i : seg_id];
+    wr[i] = sk_rsrc(ss.qw);
+    swr[i] = sk_rsrc(ss.sw);
   }
+  const auto xr = sk_rsrc(reinterpret_cast<const char*>(p.x) + (size_t)m0 * p.K * 2);
   uint32_t woff[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; nt++)
     woff[nt] = (uint32_t)(min(ltile0 + nt, sg.tiles - 1) * KT * 64 + lane);
 
-  // activation item `it` of this lane: row it*4 + lane/16 of the block row, chunk lane%16 of the tile's 256 bytes;
-  // rows past M re-read row M-1 (their results are not stored)
-  const char* xb = reinterpret_cast<const char*>(p.x);
-  const int r4 = lane >> 4, c16 = lane & 15;
-  // The per-item addresses are cheap to derive and expensive to keep (2 * XL registers): both helpers start from
-  // opaque copies of the lane coordinates so that the compiler rebuilds them at every call instead of hoisting them
-  // out of the K loop.
-  i32x4 xr[XL];
-  auto load_x = [&](int t) {
-    t = max(min(t, t1 - 1), 0); // past the end (or a wave without K tiles): a valid tile, never consumed
-    int r = r4, c = c16;
-    asm volatile("" : "+v"(r), "+v"(c));
-    const uint32_t base = (uint32_t)t * 256u + (uint32_t)c * 16u;
+  // rows of this block row past M re-read its last row (their results are not stored)
+  const int mlast = p.M - 1 - m0;
+  auto load_x = [&](auto H, int slot, int t) {
+    int r = lane >> 4, c = lane & 15;
+    asm volatile("" : "+v"(r), "+v"(c)); // (rebuilt at every use: kept, the addresses are 16 registers)
 #pragma unroll
-    for (int it = 0; it < XL; it++) {
-      const int row = min(m0 + it * 4 + r, p.M - 1);
-      xr[it] = *reinterpret_cast<const i32x4*>(xb + (size_t)((uint32_t)(row * p.K) * 2u + base));
+    for (int i = 0; i < NX; i++) {
+      const int row = min(decltype(H)::value * UG * 16 + i * 4 + r, mlast); // (row and K are below 2^24)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(xs + (slot * NX + i) * 1024), 16,
+                                               (__umul24((uint32_t)row * 2u, (uint32_t)p.K) + (uint32_t)((c ^ ((i & 3) * 4 + r)) * 16)), t * 256, 0, 0);
     }
   };
-  auto store_x = [&]() {
-    int r = r4, c = c16;
-    asm volatile("" : "+v"(r), "+v"(c));
-#pragma unroll
-    for (int it = 0; it < XL; it++)
-      xs[c * MPAD + ((it * 4 + r) ^ c)] = xr[it];
-  };
-  // operand slot of this lane for step j: chunk g*4 + j, row m of row group mg (+ mg*16)
-  int rdo[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int cj = (lane >> 4) * 4 + j;
-    rdo[j] = cj * MPAD + ((lane & 15) ^ cj);
-  }
-
-  i32x4 wreg[PF][NTW];
-  uint32_t sreg[PF][NTW];
-  auto load_stage = [&](int st, int t) {
-    t = max(min(t, t1 - 1), 0); // past the end (or a wave without K tiles): a valid tile, never consumed
+  i32x4 wreg[2][NTW];
+  uint8_t sreg[2][NTW];
+  auto load_w = [&](auto ST, int t) {
+    constexpr int st = decltype(ST)::value;
 #pragma unroll
     for (int nt = 0; nt < NTW; nt++) {
-      const uint32_t slot = woff[nt % NT] + (uint32_t)t * 64u;
-      wreg[st][nt] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(qwb[nt / NT] + (size_t)(slot * 16u)));
-      sreg[st][nt] = *reinterpret_cast<const uint8_t*>(swb[nt / NT] + (size_t)slot);
+      wreg[st][nt] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[nt / NT], woff[nt % NT] * 16u, t * 1024, 2)); // (non-temporal)
+      sreg[st][nt] = __builtin_amdgcn_raw_buffer_load_b8(swr[nt / NT], woff[nt % NT], t * 64, 0);
     }
   };
-  // (no branch around the first requests: the compiler then counts the ring behind the activations and waits for
-  // the activations only)
-  load_x(t0); // needed first, requested first
+  uint32_t rdo[4]; // operand of this lane for step j: chunk g*4 + j of row m
 #pragma unroll
-  for (int i = 0; i < PF; i++)
-    load_stage(i, t0 + i);
+  for (int j = 0; j < 4; j++)
+    rdo[j] = (lane & 15) * 256 + ((((lane >> 4) * 4 + j) ^ (lane & 15)) * 16);
+
   // post-op inputs early, except where registers are scarcest (the gate/up pair has none but its biases)
   constexpr bool LATE_EP = DUAL && MG == 4;
   SkEpilogue<MG, NTW, DUAL, W, W> ep;
-  if (!LATE_EP)
-    ep.prefetch(p, sg, ltile0, m0);
-
   f32x4 acc[NTW][MG];
 #pragma unroll
   for (int nt = 0; nt < NTW; nt++)
@@ -2300,74 +2283,113 @@ skinny_mxfp4_mg_kernel(const DecodeParams p) {
     for (int mg = 0; mg < MG; mg++)
       acc[nt][mg] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // one K tile: activations of the tile into LDS, the next tile's requested, then 4 steps x MG x NT MFMAs
-  // XLATE (the widest variants, 96 accumulators): the next tile's activations are requested BEHIND the tile's MFMAs,
-  // where the 64 staging registers are free, instead of in front of them -- that makes room for a second stage of
-  // the weight ring (with one stage the next tile's weights can only be requested after the tile's last MFMA and are
-  // needed right away).  Measured level with the one-stage form (64-row gate/up pair 24.4 against 24.6 us): a wave
-  // waits a memory round trip per K tile either way, for its weights there and for its activations here; both
-  // prefetches together need 188 bytes of scratch per lane.
-  auto consume = [&](int i, int tnext) {
-    store_x();
-    if (!XLATE)
-      load_x(tnext);
-    float sc[NTW];
-#pragma unroll
-    for (int nt = 0; nt < NTW; nt++)
-      sc[nt] = e8m0_to_f32(sreg[i][nt]);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      // NT dequantised operands at a time (DUAL: the gate tiles, then the up tiles; the activation operands are
-      // read again, which is cheaper than keeping either set in registers)
-#pragma unroll
-      for (int h = 0; h < NTW / NT; h++) {
-        bf16x8 b[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-          b[nt] = sk_cvt_fp4x8((uint32_t)wreg[i][h * NT + nt][j], sc[h * NT + nt]);
-#pragma unroll
-        for (int mg = 0; mg < MG; mg++) {
-          const bf16x8 a = __builtin_bit_cast(bf16x8, xs[rdo[j] + mg * 16]);
-#pragma unroll
-          for (int nt = 0; nt < NT; nt++)
-            acc[h * NT + nt][mg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[nt], acc[h * NT + nt][mg], 0, 0, 0);
-        }
-        if (MG * NT >= 12)
-          __builtin_amdgcn_sched_barrier(0); // widest variants: keep the operands of one group live at a time
-      }
-    }
-  };
-  int t = t0;
-  for (; t + 2 * PF <= t1; t += PF) { // branch-free full groups: every reload is a real tile, wait counts stay exact
-#pragma unroll
-    for (int i = 0; i < PF; i++) {
-      consume(i, t + i + 1);
-      if (XLATE) {
-        __builtin_amdgcn_sched_barrier(0);
-        load_x(t + i + 1); // in front of the weights: loads return in issue order
-      }
-      load_stage(i, t + i + PF);
+  // K tile t with its weights in slot ST, LEFT tiles (itself included) to the end, 3 for more.  Behind a unit the slot it
+  // has read is requested for the unit two later, behind a tile its weights' registers for the tile two later; what does
+  // not exist is not requested (a load of nothing takes its turn in the address unit all the same).
+  auto tile = [&](auto ST, auto LEFT, int t) {
+    constexpr int st = decltype(ST)::value, left = decltype(LEFT)::value;
+    static_for<0, NU>([&](auto H) {
+      constexpr int h = decltype(H)::value, slot = NU == 2 ? h : st;
+      // Loads complete in issue order: as many may be outstanding as were issued behind this unit's activations.
+      // (NU = 2) the next unit's, and the weights of tile t + 1; (NU = 1) the weights of tiles t and t + 1 and the next
+      // unit's.  The compiler waits for the weights by itself.
+      constexpr int vm = NU == 2 ? (left >= 2 || h == 0 ? NX : 0) + (left >= 2 ? WN : 0)
+                                 : WN + (left >= 2 ? NX + WN : 0);
       __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  for (; t < t1; t += PF) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt((vm & 15) | 7 << 4 | 15 << 8 | vm >> 4 << 14);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      // Expanded again for the second half of the rows: its instructions fit under the MFMAs, the expanded weights of a K
+      // tile (96 registers) do not fit beside the accumulators.
+      uint32_t se[NTW];
 #pragma unroll
-    for (int i = 0; i < PF; i++) {
-      const int tt = t + i;
-      if (tt < t1) {
-        consume(i, tt + 1);
-        if (XLATE) {
-          __builtin_amdgcn_sched_barrier(0);
-          load_x(tt + 1);
-        }
-        if (tt + PF < t1)
-          load_stage(i, tt + PF);
+      for (int nt = 0; nt < NTW; nt++) {
+        se[nt] = sreg[st][nt];
+        if constexpr (h > 0)
+          asm volatile("" : "+v"(se[nt]));
       }
+      // (step, channel tile) after (step, channel tile): the weights of the next are expanded under the MFMAs of this one,
+      // the activations of the next step read under those of this one.  (Left to itself the compiler expands a whole K
+      // tile's weights ahead and spills.)
+      bf16x8 a[2][UG], b[2];
+      auto read = [&](int j) {
+#pragma unroll
+        for (int g = 0; g < UG; g++)
+          a[j & 1][g] = *reinterpret_cast<const bf16x8*>(xs + (slot * UG + g) * 4096 + rdo[j]);
+      };
+      read(0);
+      b[0] = sk_cvt_fp4x8((uint32_t)wreg[st][0][0], e8m0_to_f32(se[0]));
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<0, 4 * NTW>([&](auto Q) {
+        constexpr int q = decltype(Q)::value, j = q / NTW, nt = q % NTW, jn = (q + 1) / NTW, nn = (q + 1) % NTW;
+        if constexpr (nt == 0 && j < 3)
+          read(j + 1);
+#pragma unroll
+        for (int g = 0; g < UG; g++)
+          acc[nt][h * UG + g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j & 1][g], b[q & 1], acc[nt][h * UG + g], 0, 0, 0);
+        if constexpr (q + 1 < 4 * NTW)
+          b[(q + 1) & 1] = sk_cvt_fp4x8((uint32_t)wreg[st][nn][jn], e8m0_to_f32(se[nn]));
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (NU == 2 ? left >= 2 : left >= 3)
+        load_x(H, slot, NU == 2 ? t + 1 : t + 2);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (left >= 3)
+      load_w(ST, t + 2);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  using C2 = std::integral_constant<int, 2>;
+  using C3 = std::integral_constant<int, 3>;
+  int t = t0;
+  if (t1 - t0 >= 2) {
+    // The first two units and tiles, in the order the waits count on.  An odd number of tiles starts in slot 1.
+    auto first = [&](auto A, auto B) {
+      load_x(C0{}, NU == 2 ? 0 : decltype(A)::value, t0);
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(A, t0);
+      __builtin_amdgcn_sched_barrier(0);
+      load_x(std::integral_constant<int, NU - 1>{}, NU == 2 ? 1 : decltype(B)::value, NU == 2 ? t0 : t0 + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(B, t0 + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if ((t1 - t0) & 1) {
+      first(C1{}, C0{});
+      if (!LATE_EP)
+        ep.prefetch(p, sg, ltile0, m0);
+      tile(C1{}, C3{}, t++);
+    } else {
+      first(C0{}, C1{});
+      if (!LATE_EP)
+        ep.prefetch(p, sg, ltile0, m0);
+    }
+    for (; t + 2 < t1; t += 2) {
+      tile(C0{}, C3{}, t);
+      tile(C1{}, C3{}, t + 1);
+    }
+    tile(C0{}, C2{}, t);
+    tile(C1{}, C1{}, t + 1);
+  } else {
+    if (!LATE_EP)
+      ep.prefetch(p, sg, ltile0, m0);
+    if (t0 < t1) {
+      load_x(C0{}, 0, t0);
+      load_w(C0{}, t0);
+      if constexpr (NU == 2)
+        load_x(C1{}, 1, t0);
+      tile(C0{}, C1{}, t0);
     }
   }
   if (LATE_EP)
     ep.prefetch(p, sg, ltile0, m0);
-  __syncthreads(); // every wave is done with its activation region before it becomes reduction scratch
+  // every load into the activation regions has landed and every wave is done with its own: they become scratch
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
   if constexpr (DUAL) {
     ep.finish_halves(sg, acc, sk_lds);
   } else {
@@ -2883,8 +2905,9 @@ hipError_t launch_skinny_mxfp4_x4(DecodeParams& p, int nt, bool dual, hipStream_
   return sk_launch(skinny_mxfp4_x4_kernel<1, 4, false>, p, grid, 16, lds, stream);
 }
 
+// two slots of activations (16 or 32 rows of a K tile) per wave, or the epilogue's sums
 size_t skinny_mxfp4_mg_lds(int mg, int ntw, int waves) {
-  const size_t xbytes = (size_t)waves * mg * 16 * 256, rbytes = (size_t)waves * ntw * mg * 1024;
+  const size_t xbytes = (size_t)waves * (mg == 1 ? 1 : 2) * 8192, rbytes = (size_t)waves * ntw * mg * 1024;
   return xbytes > rbytes ? xbytes : rbytes;
 }
 
@@ -2894,76 +2917,53 @@ hipError_t launch_skinny_mxfp4_mg(DecodeParams& p, int mg, int nt, bool dual, hi
   dim3 grid(p.groups, (p.M + mg * 16 - 1) / (mg * 16), p.S);
   if (p.S > 1 && (p.S > 4 || (p.ticket0 = skinny_split_tickets((int)(grid.x * grid.y))) < 0))
     return hipErrorInvalidValue;
-  if (mg == 1) { // up to 16 rows: sixteen waves, deeper weight ring
-    const size_t lds1 = skinny_mxfp4_mg_lds(1, nt, 16);
-#define SKMG1(NT, DUAL, PF) return sk_launch(skinny_mxfp4_mg_kernel<1, NT, DUAL, PF, 16>, p, grid, 16, lds1, stream)
-    if (dual) {
-      if (nt == 3)
-        SKMG1(3, true, 1);
-      if (nt == 2)
-        SKMG1(2, true, 2);
-      SKMG1(1, true, 4);
-    }
-    if (nt == 3)
-      SKMG1(3, false, 4);
-    if (nt == 2)
-      SKMG1(2, false, 4);
-    SKMG1(1, false, 4);
-#undef SKMG1
-  }
-  const size_t lds = skinny_mxfp4_mg_lds(mg, nt, 8); // the gate/up pair is reduced one half at a time
-#define SKMG(MG, NT, DUAL, PF) return sk_launch(skinny_mxfp4_mg_kernel<MG, NT, DUAL, PF>, p, grid, 8, lds, stream)
-#define SKMGL(MG, NT, DUAL, PF) return sk_launch(skinny_mxfp4_mg_kernel<MG, NT, DUAL, PF, 8, true>, p, grid, 8, lds, stream)
-  if (dual) {
-    if (mg == 2) {
-      if (nt == 3)
-        SKMG(2, 3, true, 2);
-      if (nt == 2)
-        SKMG(2, 2, true, 2);
-      SKMG(2, 1, true, 2);
-    }
-    if (nt == 3) {
-      if (env_int("TPPX_MXFP4_MG_LATE", 1) != 0)
-        SKMGL(4, 3, true, 2); // 96 accumulators: two ring stages with the activations requested behind the MFMAs
-      SKMG(4, 3, true, 1);    // ... or one stage with them requested in front (64 staging registers live)
-    }
-    if (nt == 2)
-      SKMG(4, 2, true, 2);
-    SKMG(4, 1, true, 2);
+  const int waves = mg == 1 ? 16 : 8;
+  const size_t lds = skinny_mxfp4_mg_lds(mg, nt, waves); // the gate/up pair is reduced one half at a time
+#define SKMG(MG, NT, DUAL) return sk_launch(skinny_mxfp4_mg_kernel<MG, NT, DUAL, MG == 1 ? 16 : 8>, p, grid, waves, lds, stream)
+#define SKMG_NT(MG, DUAL) \
+  do {                    \
+    if (nt == 3)          \
+      SKMG(MG, 3, DUAL);  \
+    if (nt == 2)          \
+      SKMG(MG, 2, DUAL);  \
+    SKMG(MG, 1, DUAL);    \
+  } while (0)
+  if (mg == 1) {
+    if (dual)
+      SKMG_NT(1, true);
+    SKMG_NT(1, false);
   }
   if (mg == 2) {
+    if (dual)
+      SKMG_NT(2, true);
     if (nt == 4)
-      SKMG(2, 4, false, 2);
-    if (nt == 3)
-      SKMG(2, 3, false, 2);
-    if (nt == 2)
-      SKMG(2, 2, false, 2);
-    SKMG(2, 1, false, 2);
+      SKMG(2, 4, false);
+    SKMG_NT(2, false);
   }
-  if (nt == 4) {
-    if (env_int("TPPX_MXFP4_MG_LATE", 1) != 0)
-      SKMGL(4, 4, false, 2);
-    SKMG(4, 4, false, 1);
-  }
-  if (nt == 3)
-    SKMG(4, 3, false, 2);
-  if (nt == 2)
-    SKMG(4, 2, false, 2);
-  SKMG(4, 1, false, 2);
+  if (dual)
+    SKMG_NT(4, true);
+  if (nt == 4)
+    SKMG(4, 4, false);
+  SKMG_NT(4, false);
+#undef SKMG_NT
 #undef SKMG
-#undef SKMGL
+}
+
+static size_t skinny_bf16_lds(int mg, int nt, int waves) {
+  const size_t xbytes = (size_t)waves * mg * 16 * 256, rbytes = (size_t)waves * nt * mg * 1024;
+  return xbytes > rbytes ? xbytes : rbytes;
 }
 
 // bf16 weights: mg row groups of 16 per block row (1, 2 or 4), nt channel tiles per workgroup (1 or 2)
 hipError_t launch_skinny_bf16(DecodeParams& p, int mg, int nt, hipStream_t stream) {
   dim3 grid(p.groups, (p.M + mg * 16 - 1) / (mg * 16), 1);
   if (mg == 1) {
-    const size_t lds1 = skinny_mxfp4_mg_lds(1, nt, 16);
+    const size_t lds1 = skinny_bf16_lds(1, nt, 16);
     if (nt == 2)
       return sk_launch(skinny_bf16_kernel<1, 2, 2, 16>, p, grid, 16, lds1, stream);
     return sk_launch(skinny_bf16_kernel<1, 1, 4, 16>, p, grid, 16, lds1, stream);
   }
-  const size_t lds = skinny_mxfp4_mg_lds(mg, nt, 8);
+  const size_t lds = skinny_bf16_lds(mg, nt, 8);
 #define SKBF(MG, NT, PF) return sk_launch(skinny_bf16_kernel<MG, NT, PF, 8>, p, grid, 8, lds, stream)
   if (mg == 2) {
     if (nt == 2)

@@ -1143,13 +1143,13 @@ def test_prefill_mxfp4_takes_scales_at_any_address(off, M, N, K, monkeypatch):
             assert torch.equal(a, b), tile
 
 
-@pytest.mark.parametrize("M", [9, 16, 17, 31, 33, 50, 64, 70])
+@pytest.mark.parametrize("M", [1, 9, 16, 17, 31, 33, 50, 64, 70])
 @pytest.mark.parametrize("tiles", [1, 8, 13, 24, 33, 47])
-def test_mxfp4_row_groups_at_every_number_of_k_tiles_per_wave(M, tiles):
-    """The MXFP4 kernel for 17..64 rows (and for fewer where K does not suit the LDS-staged ones): waves without K tiles,
-    with one, two, three and more, odd and even counts in one workgroup, rows past M; the GEMM
+def test_row_groups_at_every_number_of_k_tiles_per_wave(M, tiles):
+    """The row-group kernel (MXFP4 at 17..64 rows and where K does not suit the LDS-staged kernels; bf16 weights): waves
+    without K tiles, with one, two, three and more, odd and even counts in one workgroup, rows past M.  MXFP4: the GEMM
     against the oracle, the gate/up pair against its two GEMMs one after the other (the same three roundings to bf16, of
-    sums in another order)."""
+    sums in another order); bf16 against the product in float64 (one rounding)."""
     from tpp_pytorch_extension import _lib
     ops = _ops()
     K = 128 * tiles
@@ -1159,3 +1159,7 @@ def test_mxfp4_row_groups_at_every_number_of_k_tiles_per_wave(M, tiles):
     want = ops.fc_mul(x, wu, None, ops.fc_silu(x, wg, None)).float()
     got = ops.swiglu_gate_up(x, wg, wu).float()
     assert ((got - want).norm() / want.norm()).item() < 3 * 2.0 ** -9
+    w = randn_bf16((96, K), 0.05, 790 + tiles)
+    got = ops.linear(x, block_bf16(w).cuda(), None, flags=_lib.FLAG_FORCE_SKINNY).double()
+    want = x.double() @ w.cuda().double().t()
+    assert ((got - want).norm() / want.norm()).item() < 2.0 ** -8

@@ -2198,8 +2198,10 @@ skinny_mxfp4_x4_kernel(const DecodeParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// MXFP4 weight-only, 17..64 rows (and fewer where K is too long for the LDS-staged kernels): MG row groups of 16 per
-// workgroup.  W waves split K.  A wave walks its K tiles in units of UG row groups: the bf16 activations of a unit
+// MXFP4 weight-only, 17..64 rows (and fewer where K is too long for the LDS-staged kernels), and unquantized bf16 weights
+// (the reference's default lm_head) with any number of rows: MG row groups of 16 per workgroup, block rows on grid y (each
+// streams the weights again, from L2 / Infinity Cache when they fit).  Native bf16 tiles hold the MFMA operands themselves,
+// [N/16][K/128][4 j][64 lanes][16 B]: four 1 KB loads per K tile and wave.  W waves split K.  A wave walks its K tiles in units of UG row groups: the bf16 activations of a unit
 // (UG*16 rows x 256 B) go straight from global memory to one of the two slots of the wave's private LDS region, no
 // registers in between, and are read back as A operands; the weights of two K tiles are in registers or under way.
 // LDS image of a row group: row r at r*256, its 16-byte chunk c at (c ^ r)*16 -- a load instruction fills four rows from
@@ -2211,14 +2213,21 @@ skinny_mxfp4_x4_kernel(const DecodeParams p) {
 // 23.2; 32 rows 15.4 against 17.0; singles of 50 rows: 4096 x 4096 9.5 against 11.0, 16384 x 2560 19.3 against 22.6; 8 rows
 // of 18944 x 3584 (MG = 1) 11.4 against 16.1.  Requests past a wave's last tile, out of a resource's range so that every wait
 // counts the same loads, cost 1 to 2 us: each takes its turn in the address unit.
+// bf16 weights, same change: 4096 x 4096 at one row 9.3 -> 6.8 us, 50 rows 13.1 -> 11.5; 4096 x 11008 at 8 rows 18.1 -> 16.4
+// (5.5 TB/s of weights); 18944 x 3584 at 32 rows 34.4 -> 28.9, 64 rows 46.0 -> 39.5.
 // ---------------------------------------------------------------------------
-template <int MG, int NT, bool DUAL, int W = 8>
-__global__ void __launch_bounds__(W * 64)
-skinny_mxfp4_mg_kernel(const DecodeParams p) {
+// PAIRS: units of two row groups (MXFP4 weights are expanded once for both).  bf16 weights need no expansion, and at 17..32
+// rows half the LDS lets two workgroups share a CU.
+constexpr bool rows_in_pairs(bool bf16, int mg) { return mg == 4 || (mg == 2 && !bf16); }
+
+template <bool WBF16, int MG, int NT, bool DUAL, int W, bool PAIRS>
+__device__ __forceinline__ void skinny_rows_body(const DecodeParams& p) {
   extern __shared__ __align__(16) float sk_lds[];
-  constexpr int UG = MG >= 2 ? 2 : 1, NU = MG / UG, NX = UG * 4; // row groups per unit, units per K tile, loads per unit
+  constexpr int UG = PAIRS ? 2 : 1, NU = MG / UG, NX = UG * 4; // row groups per unit, units per K tile, loads per unit
+  static_assert(NU <= 2, "the waits know one or two units per K tile");
   constexpr int NTW = DUAL ? 2 * NT : NT; // DUAL: the gate AND the up tile of each channel tile (gate tiles first)
-  constexpr int WN = 2 * NTW;             // loads of a K tile's weights: codes and scales
+  constexpr int BJ = WBF16 ? 4 : 1;       // 16-byte loads of a K tile: the operands of the four steps, or their codes
+  constexpr int WN = (WBF16 ? 4 : 2) * NTW; // loads of a K tile's weights: operands, or codes and scales
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int grp = blockIdx.x;
@@ -2237,14 +2246,15 @@ skinny_mxfp4_mg_kernel(const DecodeParams p) {
 #pragma unroll
   for (int i = 0; i < NSEG; i++) {
     const DecodeSeg& ss = p.seg[DUAL ? i : seg_id];
-    wr[i] = sk_rsrc(ss.qw);
+    // (bf16 weights may pass 4 GiB: from the workgroup's first tile)
+    wr[i] = sk_rsrc(reinterpret_cast<const char*>(ss.qw) + (WBF16 ? (size_t)ltile0 * KT * 4096 : 0));
     swr[i] = sk_rsrc(ss.sw);
   }
   const auto xr = sk_rsrc(reinterpret_cast<const char*>(p.x) + (size_t)m0 * p.K * 2);
   uint32_t woff[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; nt++)
-    woff[nt] = (uint32_t)(min(ltile0 + nt, sg.tiles - 1) * KT * 64 + lane);
+    woff[nt] = WBF16 ? (uint32_t)(min(nt, sg.tiles - 1 - ltile0) * KT * 256 + lane) : (uint32_t)(min(ltile0 + nt, sg.tiles - 1) * KT * 64 + lane);
 
   // rows of this block row past M re-read its last row (their results are not stored)
   const int mlast = p.M - 1 - m0;
@@ -2258,14 +2268,17 @@ skinny_mxfp4_mg_kernel(const DecodeParams p) {
                                                (__umul24((uint32_t)row * 2u, (uint32_t)p.K) + (uint32_t)((c ^ ((i & 3) * 4 + r)) * 16)), t * 256, 0, 0);
     }
   };
-  i32x4 wreg[2][NTW];
+  i32x4 wreg[2][NTW][BJ];
   uint8_t sreg[2][NTW];
   auto load_w = [&](auto ST, int t) {
     constexpr int st = decltype(ST)::value;
 #pragma unroll
     for (int nt = 0; nt < NTW; nt++) {
-      wreg[st][nt] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[nt / NT], woff[nt % NT] * 16u, t * 1024, 2)); // (non-temporal)
-      sreg[st][nt] = __builtin_amdgcn_raw_buffer_load_b8(swr[nt / NT], woff[nt % NT], t * 64, 0);
+#pragma unroll
+      for (int j = 0; j < BJ; j++) // (non-temporal)
+        wreg[st][nt][j] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[nt / NT], woff[nt % NT] * 16u + j * 1024, t * (BJ * 1024), 2));
+      if constexpr (!WBF16)
+        sreg[st][nt] = __builtin_amdgcn_raw_buffer_load_b8(swr[nt / NT], woff[nt % NT], t * 64, 0);
     }
   };
   uint32_t rdo[4]; // operand of this lane for step j: chunk g*4 + j of row m
@@ -2305,8 +2318,8 @@ skinny_mxfp4_mg_kernel(const DecodeParams p) {
       uint32_t se[NTW];
 #pragma unroll
       for (int nt = 0; nt < NTW; nt++) {
-        se[nt] = sreg[st][nt];
-        if constexpr (h > 0)
+        se[nt] = WBF16 ? 0 : sreg[st][nt];
+        if constexpr (h > 0 && !WBF16)
           asm volatile("" : "+v"(se[nt]));
       }
       // (step, channel tile) after (step, channel tile): the weights of the next are expanded under the MFMAs of this one,
@@ -2318,8 +2331,14 @@ skinny_mxfp4_mg_kernel(const DecodeParams p) {
         for (int g = 0; g < UG; g++)
           a[j & 1][g] = *reinterpret_cast<const bf16x8*>(xs + (slot * UG + g) * 4096 + rdo[j]);
       };
+      auto weight = [&](int nt, int j) {
+        if constexpr (WBF16)
+          return __builtin_bit_cast(bf16x8, wreg[st][nt][j]);
+        else
+          return sk_cvt_fp4x8((uint32_t)wreg[st][nt][0][j], e8m0_to_f32(se[nt]));
+      };
       read(0);
-      b[0] = sk_cvt_fp4x8((uint32_t)wreg[st][0][0], e8m0_to_f32(se[0]));
+      b[0] = weight(0, 0);
       __builtin_amdgcn_sched_barrier(0);
       static_for<0, 4 * NTW>([&](auto Q) {
         constexpr int q = decltype(Q)::value, j = q / NTW, nt = q % NTW, jn = (q + 1) / NTW, nn = (q + 1) % NTW;
@@ -2329,7 +2348,7 @@ skinny_mxfp4_mg_kernel(const DecodeParams p) {
         for (int g = 0; g < UG; g++)
           acc[nt][h * UG + g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j & 1][g], b[q & 1], acc[nt][h * UG + g], 0, 0, 0);
         if constexpr (q + 1 < 4 * NTW)
-          b[(q + 1) & 1] = sk_cvt_fp4x8((uint32_t)wreg[st][nn][jn], e8m0_to_f32(se[nn]));
+          b[(q + 1) & 1] = weight(nn, jn);
         __builtin_amdgcn_sched_barrier(0);
       });
       __builtin_amdgcn_sched_barrier(0);
@@ -2400,123 +2419,18 @@ skinny_mxfp4_mg_kernel(const DecodeParams p) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Unquantized bf16 weights (the reference's default lm_head), any number of
-// rows: the row-group kernel above without the dequantisation.  Native tiles
-// hold the MFMA operands themselves, [N/16][K/128][4 j][64 lanes][16 B], so a
-// K tile of a channel tile is four 1 KB loads per wave; activations go
-// through the same wave-private LDS image.  Block rows of MG*16 rows ride on
-// grid y: beyond 64 rows every block row streams the weights again (from L2
-// / Infinity Cache when they fit), which is what a prompt's last-token
-// lm_head or a short verification batch needs, not a prefill GEMM.
-// ---------------------------------------------------------------------------
-template <int MG, int NT, int PF, int W>
+// WS = W / 4 waves per SIMD
+template <int MG, int NT, bool DUAL, int WS, int W, bool PAIRS>
+__global__ void __launch_bounds__(W * 64)
+skinny_mxfp4_mg_kernel(const DecodeParams p) {
+  static_assert(WS * 4 == W, "four SIMDs");
+  skinny_rows_body<false, MG, NT, DUAL, W, PAIRS>(p);
+}
+
+template <int MG, int NT, int W, bool PAIRS>
 __global__ void __launch_bounds__(W * 64)
 skinny_bf16_kernel(const DecodeParams p) {
-  extern __shared__ __align__(16) float sk_lds[];
-  constexpr int MPAD = MG * 16, XL = MG * 4;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int grp = blockIdx.x;
-  const DecodeSeg& sg = p.seg[sk_find_seg(p, grp)];
-  const int ltile0 = (grp - sg.grp0) * NT;
-  const int m0 = blockIdx.y * MPAD;
-  const int KT = p.units;
-  const int t0 = (wave * KT) / W, t1 = ((wave + 1) * KT) / W;
-  i32x4* xs = reinterpret_cast<i32x4*>(sk_lds) + (size_t)wave * (MPAD * 16); // [chunk 16][row MPAD] x 16 B
-
-  const i32x4* wb = reinterpret_cast<const i32x4*>(sg.qw);
-  size_t woff[NT]; // in 16-byte units
-#pragma unroll
-  for (int nt = 0; nt < NT; nt++)
-    woff[nt] = (size_t)min(ltile0 + nt, sg.tiles - 1) * KT * 256 + lane;
-
-  const char* xb = reinterpret_cast<const char*>(p.x);
-  const int r4 = lane >> 4, c16 = lane & 15;
-  i32x4 xr[XL];
-  auto load_x = [&](int t) {
-    t = max(min(t, t1 - 1), 0); // past the end (or a wave without K tiles): a valid tile, never consumed
-    int r = r4, c = c16;
-    asm volatile("" : "+v"(r), "+v"(c));
-    const size_t base = (size_t)t * 256u + (size_t)c * 16u;
-#pragma unroll
-    for (int it = 0; it < XL; it++) {
-      const int row = min(m0 + it * 4 + r, p.M - 1);
-      xr[it] = *reinterpret_cast<const i32x4*>(xb + (size_t)row * p.K * 2u + base);
-    }
-  };
-  auto store_x = [&]() {
-    int r = r4, c = c16;
-    asm volatile("" : "+v"(r), "+v"(c));
-#pragma unroll
-    for (int it = 0; it < XL; it++)
-      xs[c * MPAD + ((it * 4 + r) ^ c)] = xr[it];
-  };
-  int rdo[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int cj = (lane >> 4) * 4 + j;
-    rdo[j] = cj * MPAD + ((lane & 15) ^ cj);
-  }
-
-  i32x4 wreg[PF][NT][4];
-  auto load_stage = [&](int st, int t) {
-    t = max(min(t, t1 - 1), 0); // past the end (or a wave without K tiles): a valid tile, never consumed
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-        wreg[st][nt][j] = __builtin_nontemporal_load(wb + woff[nt] + (size_t)t * 256 + j * 64);
-  };
-  load_x(t0); // no branch around the first requests (exact wait counts)
-#pragma unroll
-  for (int i = 0; i < PF; i++)
-    load_stage(i, t0 + i);
-  SkEpilogue<MG, NT, false, W, W> ep;
-  ep.prefetch(p, sg, ltile0, m0);
-
-  f32x4 acc[NT][MG];
-#pragma unroll
-  for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-    for (int mg = 0; mg < MG; mg++)
-      acc[nt][mg] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto consume = [&](int i, int tnext) {
-    store_x();
-    load_x(tnext);
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-      for (int mg = 0; mg < MG; mg++) {
-        const bf16x8 a = __builtin_bit_cast(bf16x8, xs[rdo[j] + mg * 16]);
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-          acc[nt][mg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, wreg[i][nt][j]), acc[nt][mg], 0, 0, 0);
-      }
-  };
-  int t = t0;
-  for (; t + 2 * PF <= t1; t += PF) { // branch-free full groups: every reload is a real tile
-#pragma unroll
-    for (int i = 0; i < PF; i++) {
-      consume(i, t + i + 1);
-      load_stage(i, t + i + PF);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  for (; t < t1; t += PF) {
-#pragma unroll
-    for (int i = 0; i < PF; i++) {
-      const int tt = t + i;
-      if (tt < t1) {
-        consume(i, tt + 1);
-        if (tt + PF < t1)
-          load_stage(i, tt + PF);
-      }
-    }
-  }
-  __syncthreads(); // every wave is done with its activation region before it becomes reduction scratch
-  ep.finish(sg, acc, sk_lds, decltype(ep)::ELEMS);
+  skinny_rows_body<true, MG, NT, false, W, PAIRS>(p);
 }
 
 // Scale blocks that `runs` consecutive runs of `deal` tiles can touch (slots of activation scales a wave keeps in LDS).
@@ -2906,8 +2820,8 @@ hipError_t launch_skinny_mxfp4_x4(DecodeParams& p, int nt, bool dual, hipStream_
 }
 
 // two slots of activations (16 or 32 rows of a K tile) per wave, or the epilogue's sums
-size_t skinny_mxfp4_mg_lds(int mg, int ntw, int waves) {
-  const size_t xbytes = (size_t)waves * (mg == 1 ? 1 : 2) * 8192, rbytes = (size_t)waves * ntw * mg * 1024;
+size_t skinny_rows_lds(bool bf16, int mg, int ntw, int waves) {
+  const size_t xbytes = (size_t)waves * (rows_in_pairs(bf16, mg) ? 2 : 1) * 8192, rbytes = (size_t)waves * ntw * mg * 1024;
   return xbytes > rbytes ? xbytes : rbytes;
 }
 
@@ -2918,8 +2832,8 @@ hipError_t launch_skinny_mxfp4_mg(DecodeParams& p, int mg, int nt, bool dual, hi
   if (p.S > 1 && (p.S > 4 || (p.ticket0 = skinny_split_tickets((int)(grid.x * grid.y))) < 0))
     return hipErrorInvalidValue;
   const int waves = mg == 1 ? 16 : 8;
-  const size_t lds = skinny_mxfp4_mg_lds(mg, nt, waves); // the gate/up pair is reduced one half at a time
-#define SKMG(MG, NT, DUAL) return sk_launch(skinny_mxfp4_mg_kernel<MG, NT, DUAL, MG == 1 ? 16 : 8>, p, grid, waves, lds, stream)
+  const size_t lds = skinny_rows_lds(false, mg, nt, waves); // the gate/up pair is reduced one half at a time
+#define SKMG(MG, NT, DUAL) return sk_launch(skinny_mxfp4_mg_kernel<MG, NT, DUAL, MG == 1 ? 4 : 2, MG == 1 ? 16 : 8, rows_in_pairs(false, MG)>, p, grid, waves, lds, stream)
 #define SKMG_NT(MG, DUAL) \
   do {                    \
     if (nt == 3)          \
@@ -2949,30 +2863,25 @@ hipError_t launch_skinny_mxfp4_mg(DecodeParams& p, int mg, int nt, bool dual, hi
 #undef SKMG
 }
 
-static size_t skinny_bf16_lds(int mg, int nt, int waves) {
-  const size_t xbytes = (size_t)waves * mg * 16 * 256, rbytes = (size_t)waves * nt * mg * 1024;
-  return xbytes > rbytes ? xbytes : rbytes;
-}
-
 // bf16 weights: mg row groups of 16 per block row (1, 2 or 4), nt channel tiles per workgroup (1 or 2)
 hipError_t launch_skinny_bf16(DecodeParams& p, int mg, int nt, hipStream_t stream) {
   dim3 grid(p.groups, (p.M + mg * 16 - 1) / (mg * 16), 1);
+  const int waves = mg == 1 ? 16 : 8;
+  const size_t lds = skinny_rows_lds(true, mg, nt, waves);
+#define SKBF(MG, NT) return sk_launch(skinny_bf16_kernel<MG, NT, MG == 1 ? 16 : 8, rows_in_pairs(true, MG)>, p, grid, waves, lds, stream)
   if (mg == 1) {
-    const size_t lds1 = skinny_bf16_lds(1, nt, 16);
     if (nt == 2)
-      return sk_launch(skinny_bf16_kernel<1, 2, 2, 16>, p, grid, 16, lds1, stream);
-    return sk_launch(skinny_bf16_kernel<1, 1, 4, 16>, p, grid, 16, lds1, stream);
+      SKBF(1, 2);
+    SKBF(1, 1);
   }
-  const size_t lds = skinny_bf16_lds(mg, nt, 8);
-#define SKBF(MG, NT, PF) return sk_launch(skinny_bf16_kernel<MG, NT, PF, 8>, p, grid, 8, lds, stream)
   if (mg == 2) {
     if (nt == 2)
-      SKBF(2, 2, 2);
-    SKBF(2, 1, 2);
+      SKBF(2, 2);
+    SKBF(2, 1);
   }
   if (nt == 2)
-    SKBF(4, 2, 2);
-  SKBF(4, 1, 2);
+    SKBF(4, 2);
+  SKBF(4, 1);
 #undef SKBF
 }
 

@@ -158,8 +158,8 @@ _workspace_use = {}  # (device, stream) -> tick of its last use
 _tick = 0
 
 
-def workspace(t):
-    """Split-K / staging scratch for an op on `t`'s device (see include/tppx.h).
+def workspace(t, stream=None):
+    """Split-K / staging scratch for an op on `t`'s device (see include/tppx.h); stream: stream_of(t), where it is known.
     One zero-initialised buffer per (device, stream): every op orders itself on
     the caller's current stream, so threads that work on streams of their own
     never share scratch and need no ordering between them. Work recorded under
@@ -178,7 +178,7 @@ def workspace(t):
             raise TppxError(EINVAL, "first call on this device happens inside graph capture: run the op once "
                                     "eagerly before capturing so that its workspace exists")
         return ws
-    key = (dev, stream_of(t))
+    key = (dev, stream_of(t) if stream is None else stream)
     ws = _workspaces.get(key)
     if ws is None:
         with _workspaces_lock:

@@ -375,14 +375,16 @@ def fix_vnni(t):
 # ----------------------------------------------------------------------------
 # linears
 # ----------------------------------------------------------------------------
-def _prep_input(input, weight):
+def _prep_input(input, weight, layout=None):
+    """(x, M, N, K); layout: weight.weight_layout(), where the caller has asked already."""
     if not isinstance(weight, QTensor):
         raise TppxError(
             _lib.EUNSUPPORTED,
             "only MXFP4 / QINT8 quantized and bfloat16 weights are built on this path "
             "(quantize the weight with remap_and_quantize_mxfp4 / remap_and_quantize_qint8)",
         )
-    if not weight.is_weight():
+    kind, N, K = layout or weight.weight_layout()
+    if kind is None:
         raise TppxError(_lib.EUNSUPPORTED, f"Unsupported qscheme / layout for a linear weight: {weight!r}")
     _lib.require_gpu(weight.qdata, "weight")
     if isinstance(input, QTensor):
@@ -393,7 +395,6 @@ def _prep_input(input, weight):
                         f"this operator takes bfloat16 activations (got {input.dtype}); float / half activations and "
                         f"pre-quantized qint8 activations are built for fc_plain / linear without a post-op on "
                         f"QINT8-family weights")
-    N, K = weight.weight_nk()
     if input.shape[-1] != K:
         raise TppxError(_lib.ESHAPE, f"input has {input.shape[-1]} features, weight expects {K}")
     x = input.contiguous()
@@ -515,11 +516,11 @@ def _qint8_scratch(x, M, K, qbs):
 ACT_FP8 = os.environ.get("TPPX_ACT_FP8", "0") == "1"
 
 
-def _mxfp4_flags_ws(x, M, K, flags=0):
+def _mxfp4_flags_ws(x, M, K, flags=0, ws=None):
     """(flags, workspace) of an MXFP4 call: the FP8-activation path keeps the quantised activations in the workspace."""
     if ACT_FP8 and M > 64:
         flags |= _lib.FLAG_ACT_FP8
-    ws = _lib.workspace(x)
+    ws = _lib.workspace(x) if ws is None else ws
     if flags & _lib.FLAG_ACT_FP8:
         Mp = (M + 63) // 64 * 64
         need = Mp * K + Mp * (K // 32)
@@ -770,20 +771,22 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
     row_sumsq: f32 [16][256] table that receives the row sums of squares of the output (see sums_table());
     only honoured where takes_row_sums() says so."""
     L = _lib.lib()
+    layout = weight.weight_layout() if isinstance(weight, QTensor) else None
+    w4a8 = layout is not None and layout[0] == "mxfp4_int8"
     other_type = isinstance(input, QTensor) or (isinstance(input, torch.Tensor) and input.dtype in (torch.float32, torch.float16))
-    if other_type and not _is_w4a8(weight):
+    if other_type and not w4a8:
         if row_sumsq is not None:
             raise TppxError(_lib.EUNSUPPORTED, "row sums of squares need bfloat16 activations")
         return _linear_other_types(input, weight, bias, post, flags, post_in, post_in2, post_scale)
-    if not isinstance(weight, QTensor) and isinstance(weight, torch.Tensor) and weight.dtype == torch.bfloat16:
+    if layout is None and isinstance(weight, torch.Tensor) and weight.dtype == torch.bfloat16:
         if row_sumsq is not None:
             raise TppxError(_lib.EUNSUPPORTED, "row sums of squares need an MXFP4 weight and at most 16 rows")
         return _linear_bf16(input, weight, bias, post, post_in, post_in2, post_scale, flags)
-    if _is_w4a8(weight):
+    if w4a8:
         if row_sumsq is not None:
             raise TppxError(_lib.EUNSUPPORTED, "row sums of squares need an MXFP4 weight in the default layout")
         return _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale)
-    x, M, N, K = _prep_input(input, weight)
+    x, M, N, K = _prep_input(input, weight, layout)
     out_shape = tuple(input.shape[:-1]) + (N,)
     y = torch.empty(out_shape, dtype=torch.bfloat16, device=x.device)
     if M == 0:
@@ -793,7 +796,7 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
     post_in2 = _prep_post(post_in2, M, N, "second post-op input", x.device)
     # QINT4 / QINT2 decode steps (up to 64 rows): the codes streamed at their own width and expanded in registers
     # (same bits as the expanded int8 tiles).  TPPX_PACKED_CODES=0 keeps the expanded tiles.
-    if PACKED_CODES and M <= 64 and weight.weight_kind() in ("qint4", "qint2") and weight.block_size == 256 \
+    if PACKED_CODES and M <= 64 and layout[0] in ("qint4", "qint2") and weight.block_size == 256 \
             and row_sumsq is None and not (flags & ~_lib.FLAG_XQ_REUSE):
         qp, sp, bits = weight.native_packed()
         xq, sa = _qint8_scratch(x, M, K, 256) if M > 16 else (None, None)
@@ -805,7 +808,7 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
             return y
     qn, sn = weight.native()
     st = _lib.stream_of(x)
-    ws = _lib.workspace(x)
+    ws = _lib.workspace(x, st)
     if row_sumsq is not None:
         if not takes_row_sums(weight, M):
             raise TppxError(_lib.EUNSUPPORTED, "row sums of squares need an MXFP4 weight and at most 16 rows")
@@ -814,7 +817,7 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
                                              post, post_scale, flags, ws.data_ptr(), ws.numel(),
                                              row_sumsq.data_ptr(), st))
     elif weight._qscheme == QSCHEME_MXFP:
-        flags, ws = _mxfp4_flags_ws(x, M, K, flags)
+        flags, ws = _mxfp4_flags_ws(x, M, K, flags, ws)
         _lib.check(L.tppx_linear_mxfp4(x.data_ptr(), qn.data_ptr(), sn.data_ptr(), _lib.ptr(bias),
                                        _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N, K,
                                        post, post_scale, flags, ws.data_ptr(), ws.numel(), st))
@@ -1071,14 +1074,14 @@ def qkv_gemm(input, weights, biases, norm=None):
     if M == 0:
         return outs
     st = _lib.stream_of(x)
-    ws = _lib.workspace(x)
+    ws = _lib.workspace(x, st)
     if scheme == QSCHEME_MXFP and norm is not None and _norm_table(norm) is not None:
         _lib.check(L.tppx_normsq_multi_linear_mxfp4(x.data_ptr(), _norm_table(norm).data_ptr(), norm[0].data_ptr(),
                                                     float(norm[1]), segs, n, M, K, 0, st))
     elif scheme == QSCHEME_MXFP and norm is not None:
         _lib.check(L.tppx_norm_multi_linear_mxfp4(x.data_ptr(), norm[0].data_ptr(), float(norm[1]), segs, n, M, K, 0, st))
     elif scheme == QSCHEME_MXFP:
-        fl, ws = _mxfp4_flags_ws(x, M, K)
+        fl, ws = _mxfp4_flags_ws(x, M, K, 0, ws)
         _lib.check(L.tppx_multi_linear_mxfp4(x.data_ptr(), segs, n, M, K, fl, ws.data_ptr(), ws.numel(), st))
     else:
         qbs = weights[0].block_size
@@ -1147,7 +1150,8 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
                                             _lib.ptr(bg), qu.data_ptr(), su.data_ptr(), _lib.ptr(bu), y.data_ptr(),
                                             M, N, K, 0, _lib.stream_of(x)))
         return y
-    fl, ws = _mxfp4_flags_ws(x, M, K)
+    st = _lib.stream_of(x)
+    fl, ws = _mxfp4_flags_ws(x, M, K, 0, _lib.workspace(x, st))
     if not fl and M > 64 and M * N * 2 > ws.numel():
         # prefill: room for the gate tile lets the library run gate and up as one grid (fuller last round)
         ws = torch.empty(M * N * 2, dtype=torch.uint8, device=x.device)
@@ -1159,7 +1163,7 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
             ws = torch.empty(need, dtype=torch.uint8, device=x.device)
     _lib.check(L.tppx_swiglu_mxfp4(x.data_ptr(), qg.data_ptr(), sg.data_ptr(), _lib.ptr(bg), qu.data_ptr(),
                                    su.data_ptr(), _lib.ptr(bu), y.data_ptr(), M, N, K, fl, ws.data_ptr(),
-                                   ws.numel(), _lib.stream_of(x)))
+                                   ws.numel(), st))
     return y
 
 

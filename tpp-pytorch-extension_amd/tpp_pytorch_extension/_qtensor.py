@@ -75,42 +75,47 @@ class QTensor(torch.Tensor):
         return pre, bsi, post, vnni
 
     # -- weight geometry -----------------------------------------------------
-    def weight_kind(self):
-        """Which linear-layer weight layout this is: "mxfp4" [N/32, K/64, 32, 32, 2], "mxfp4_int8" (the VNNI8-interleaved
+    def weight_layout(self):
+        """(kind, N, K) of a linear-layer weight: "mxfp4" [N/32, K/64, 32, 32, 2], "mxfp4_int8" (the VNNI8-interleaved
         W4A8 layout) [N/8, K/bc, bc/8, 8, 8], "qint8" [N/16, K/QBS, QBS/4, 16, 4], "qint4" (VNNI2) [N/16, K/QBS, QBS/2,
-        16, 2], "qint2" (interleaved ternary) [N/32, K/QBS, QBS/4, 32, 4]; None for any other layout (helper-only
-        tensors, quantized activations)."""
-        s = tuple(self.shape)
-        if len(s) != 5 or not self.is_vnni or self.axis != 2:
-            return None
+        16, 2], "qint2" (interleaved ternary) [N/32, K/QBS, QBS/4, 32, 4]; (None, 0, 0) for any other layout (helper-only
+        tensors, quantized activations).  An eager call asks once and passes the answer on: a tensor subclass takes
+        0.5-1 us to answer for its shape or type."""
+        if not self.is_vnni or self.axis != 2:
+            return None, 0, 0
+        s = self.shape
+        if len(s) != 5:
+            return None, 0, 0
+        nb, kb, a, b, c = s
+        bs = self.block_size
         if self._qscheme == QSCHEME_MXFP:
-            if s[2:] == (32, 32, 2) and self.block_size == 32:
-                return "mxfp4"
-            if s[3:] == (8, 8) and self.block_size == 32 and s[2] % 4 == 0 and (s[0] * 8) % 16 == 0:
-                return "mxfp4_int8"
-            return None
-        if self.dtype == torch.qint8 and s[3:] == (16, 4) and s[2] * 4 == self.block_size:
-            return "qint8"
-        if self.dtype == torch.quint4x2 and s[3:] == (16, 2) and s[2] * 2 == self.block_size and self.block_size % 64 == 0:
-            return "qint4"
-        if self.dtype == torch.quint2x4 and s[3:] == (32, 4) and s[2] * 4 == self.block_size and self.block_size % 64 == 0:
-            return "qint2"
-        return None
+            if bs == 32:
+                if a == 32 and b == 32 and c == 2:
+                    return "mxfp4", nb * 32, kb * 64
+                if b == 8 and c == 8 and a % 4 == 0 and (nb * 8) % 16 == 0:
+                    return "mxfp4_int8", nb * 8, kb * a * 8
+            return None, 0, 0
+        if b == 16 and c == 4 and a * 4 == bs and self.dtype == torch.qint8:
+            return "qint8", nb * 16, kb * bs
+        if b == 16 and c == 2 and a * 2 == bs and bs % 64 == 0 and self.dtype == torch.quint4x2:
+            return "qint4", nb * 16, kb * bs
+        if b == 32 and c == 4 and a * 4 == bs and bs % 64 == 0 and self.dtype == torch.quint2x4:
+            return "qint2", nb * 32, kb * bs
+        return None, 0, 0
+
+    def weight_kind(self):
+        """Which linear-layer weight layout this is, None for any other (weight_layout())."""
+        return self.weight_layout()[0]
 
     def is_weight(self):
         """True for the weight layouts the linear kernels consume."""
         return self.weight_kind() is not None
 
     def weight_nk(self):
-        s = self.shape
-        kind = self.weight_kind()
-        if kind == "mxfp4":
-            return s[0] * 32, s[1] * 64
-        if kind == "mxfp4_int8":
-            return s[0] * 8, s[1] * s[2] * 8
-        if kind == "qint2":
-            return s[0] * 32, s[1] * self.block_size
-        return s[0] * 16, s[1] * self.block_size
+        kind, N, K = self.weight_layout()
+        if kind is None:
+            return self.shape[0] * 16, self.shape[1] * self.block_size
+        return N, K
 
     def native(self):
         """(qdata_native, scales_for_kernel), built once."""

@@ -15,8 +15,9 @@
 //   skinny_mxfp4_xl_kernel  the wave's whole K slice staged once in LDS, up to
 //                           16 rows; optional RMSNorm in front
 //   skinny_mxfp4_x4_kernel  the same with only 4 rows kept, for long K
-//   skinny_mxfp4_mg_kernel  activations streamed through LDS one K tile at a
-//                           time, 1, 2 or 4 row groups of 16
+//   skinny_mxfp4_mg_kernel  activations streamed straight into LDS in units of
+//                           16 or 32 rows of a K tile, 1, 2 or 4 row groups of
+//                           16; skinny_bf16_kernel: the same on bf16 weights
 //
 // MFMA operand convention (A = activations, B = weights):
 //   lane l supplies row/col (l & 15) and K group (l >> 4);

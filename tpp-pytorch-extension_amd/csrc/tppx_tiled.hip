@@ -1039,8 +1039,8 @@ big_bf16_kernel(const BigParams P) {
 // MXFP4 launches whose workgroups are at most one or two to a CU: the same tiles, operand layout and order of sums as
 // big_gemm_body (the same bits), but BOTH operands and the scale bytes go from global memory straight into LDS, NB - 1
 // K steps ahead in a ring of NB stages.  With one workgroup per CU nothing else covers the latency of a step's loads:
-// requested one step ahead (weights half a step, into registers) a step of a 64 x 128 workgroup took 0.8 us where its
-// MFMAs take 0.25 and its bytes 0.45; now 0.5 (4096 x 11008 at 333 rows 74 -> 52 us, 3584 x 18944 122 -> 82).  Six
+// requested one step ahead (weights half a step, into registers) they stood in the way: 128 x 128, 3584 x 18944 at 800
+// rows 150 -> 131 us; 128 x 256 55 -> 52.  (64 x 128 workgroups went on to waves side by side, side_gemm_body.)  Six
 // stages measured as three.  All loads of the loop being of one kind they complete in issue order, so the
 // wait at the top of a step leaves the younger stages in flight; one barrier per step.
 // Stage: A [WM*MT row tiles][4096 B], swizzled as in big_gemm_body | B [4*WN native tiles][1 KiB] | scales [4*WN][64 B].
@@ -1223,7 +1223,7 @@ __device__ __forceinline__ void ring_gemm_body(const BigParams& P) {
     big_epilogue<MT>(p, acc, stage, m_wg + wm * (MT * 16), tile_base);
 }
 
-constexpr int RING_STAGES = 3; // (two 64 x 128 workgroups of three stages share a CU's LDS)
+constexpr int RING_STAGES = 3;
 template <int MT, bool DUAL, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
 big_mxfp4_kernel(const BigParams P) {

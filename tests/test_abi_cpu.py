@@ -260,7 +260,7 @@ def test_launch_plans_of_the_baseline_shapes():
                                                                              _lib.FLAG_FORCE_TILED, 0)[0]  # 128 x 512: eight waves anyway
     # from 65 rows on the 64-row forms take what the planner hands to a tiled kernel
     assert "big_mxfp4_kernel<2, false, 2, 2> grid=96x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 160, 4096, 4096, 0, 0)[0]
-    assert "skinny_mxfp4" in plan(L.tppx_plan_linear_mxfp4, 128, 4096, 4096, 0, ws)[0]
+    assert "big_mxfp4_kernel<2, false, 2, 2> grid=64x1x1" in plan(L.tppx_plan_linear_mxfp4, 128, 4096, 4096, 0, ws)[0]  # 17.0 us (rows 17.9)
     assert "big_qint8_small_kernel grid=129x1x1 block=512" in plan(L.tppx_plan_linear_qint8, 160, 11008, 4096, 256, 1, 0, ws)[-1]
     assert "big_mxfp4_kernel<2, false, 2, 2>" in plan(L.tppx_plan_linear_mxfp4, 100, 4096, 4096, _lib.FLAG_FORCE_TILED, 0)[0]
 
@@ -320,6 +320,15 @@ def test_kernel_family_of_short_prompts():
     assert "big_mxfp4" in one(192, 14336, 5120)                                                     # 42 us (65)
     assert "<2, false, 2, 2>" not in one(1800, 2560, 11008) and "<2, false, 2, 2>" in one(1500, 1536, 18944)
     assert "<8, true, 1, 8>" in pair(2048, 28672, 8192)                                             # 1254 us (128 x 256: 1283)
+
+    def qkv(M, N, K):
+        _lib.check(L.tppx_plan_multi_linear_mxfp4((ctypes.c_int64 * 3)(N, N, N), 3, M, K, 0, 0, 1 << 25, buf, len(buf)))
+        return buf.value.decode()
+
+    for M in (96, 127, 128, 129):  # nothing changes at whole block rows of 64
+        assert "<2, false, 2, 2>" in qkv(M, 4096, 4096), M                                          # 18.6 us (rows 35)
+        assert "<2, false, 2, 2>" in one(M, 12288, 4096) and "<2, false, 2, 2>" in one(M, 11008, 4096), M  # 18 us (26)
+        assert "skinny_mxfp4" in one(M, 1024, 4096), M                                              # 8 us (tiles 16)
 
     def per_weight(M, N, K, weight_bytes):
         return not L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, weight_bytes)

@@ -659,7 +659,7 @@ def test_launch_plan_names_the_kernels():
     assert "big_mxfp4_kernel" in buf.value.decode()
     _lib.check(L.tppx_plan_linear_mxfp4(100, 8192, 8192, _lib.FLAG_FORCE_TILED, 0, buf, len(buf)))
     assert "big_mxfp4_kernel<2, false, 2, 2>" in buf.value.decode()  # 64 x 128 workgroups from 65 rows on
-    _lib.check(L.tppx_plan_linear_mxfp4(128, 11008, 4096, 0, 0, buf, len(buf)))  # few tiles: block rows of 64
+    _lib.check(L.tppx_plan_linear_mxfp4(128, 1024, 4096, 0, 0, buf, len(buf)))  # few tiles: block rows of 64
     assert "skinny_mxfp4_mg_kernel" in buf.value.decode() and "x2x" in buf.value.decode()
 
 

@@ -234,13 +234,14 @@ static int kernel_family(int64_t M, int flags) {
 }
 
 // What the decode kernels take over block rows of 64 rows: rounds of 256 workgroups of nt channel tiles and one block row,
-// each round a fixed part and a part per input channel; the last one costs three quarters when it is all but empty.
+// each round a fixed part and a part per input channel, which has a share for the rows that the block rows are short of whole
+// (rows past the end repeat the last one, whose lines are at hand); the last one costs three quarters when it is all but empty.
 struct RowsCost {
-  double launch, round, per_k; // us, us, ns
+  double launch, round, per_k, per_k_rows; // us, us, ns, ns
 };
-static double rows_us(const RowsCost& c, int64_t wgs, int64_t K) {
-  const double r = (double)((wgs + 255) / 256), f = (double)wgs / 256.0 - (r - 1.0);
-  return c.launch + (r - 0.25 * (1.0 - f)) * (c.round + c.per_k * 1e-3 * (double)K);
+static double rows_us(const RowsCost& c, int64_t wgs, int64_t M, int64_t K) {
+  const double r = (double)((wgs + 255) / 256), f = (double)wgs / 256.0 - (r - 1.0), filled = (double)M / (double)((M + 63) / 64 * 64);
+  return c.launch + (r - 0.25 * (1.0 - f)) * (c.round + (c.per_k + c.per_k_rows * filled) * 1e-3 * (double)K);
 }
 
 // the tile x K-part kernel's shapes (33..64 rows per block row, K in 4 slices across workgroups, partial sums in ws)
@@ -250,9 +251,10 @@ static bool mxfp4_nk_fits(int64_t M, int total_tiles, int units, int64_t ws_byte
          (int64_t)4 * groups * 4 * 4 * 256 * (int64_t)sizeof(float) * ((M + 63) / 64) <= ws_bytes;
 }
 
-// MXFP4 (dual: `tiles` of each projection).  Both sides within 12 % of 3600 launches of 65 .. 640 rows; the family and
-// tile taken are within 0.5 % of the fastest on average (the fits before, one figure per block row whatever its rounds:
-// 4.6 %, and twice the time for pairs of 1024 channels or single GEMMs of 28672 x 2560).
+// MXFP4 (dual: `tiles` of each projection).  Fitted to 2800 launches of the decode kernels at 65 .. 1024 rows with weights that
+// come from memory, most of all to those that take about as long as the tiles.  On 2000 launches of other shapes the family and
+// tile taken are 0.14 % off the fastest on average and 7 % in the worst hundredth (fitted to the decode kernels before their
+// activations went straight to LDS: 1.3 % and 30 %, a 128-row q/k/v of 3 x 4096 x 4096 at 34.6 us where the tiles take 18.6).
 static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, bool dual, bool nk, int64_t ws_bytes) {
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
@@ -265,18 +267,14 @@ static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, boo
     return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
            (double)rows64 * (8.0 + (double)n_tiles16 * 16.0 * (double)K * (0.5 + 1.0 / 32) / 5.5e6 + (double)K * 0.0008);
   }
-  static constexpr RowsCost SINGLE[3] = {{1.84, 1.85, 1.78}, {1.78, 2.70, 2.03}, {2.49, 4.26, 2.17}};
-  static constexpr RowsCost DUAL[3] = {{1.91, 2.69, 1.94}, {1.57, 4.04, 2.64}, {1.88, 6.88, 3.42}};
-  static constexpr RowsCost NK = {1.78, 6.63, 0.734};
+  static constexpr RowsCost SINGLE[3] = {{3.13, 0.665, 0.939, 0.75}, {2.73, 1.78, 1.08, 0.939}, {2.3, 3.16, 1.58, 0.616}};
+  static constexpr RowsCost DUAL[3] = {{2.82, 1.16, 1.14, 0.883}, {2.92, 3.4, 1.51, 0.984}, {2.42, 5.0, 2.31, 1.02}};
+  static constexpr RowsCost NK = {3.18, 6.73, 0.392, 0.326};
   const double tiled = tiled_mxfp4_us(M, K, n_tiles16);
   if (nk && mxfp4_nk_fits(M, (int)tiles, (int)(K / 128), ws_bytes))
-    return tiled <= rows_us(NK, (tiles + 3) / 4 * 4 * rows64, K);
+    return tiled <= rows_us(NK, (tiles + 3) / 4 * 4 * rows64, M, K);
   const int nt = tiles <= 256 ? 1 : (tiles + 1) / 2 <= 256 ? 2 : 3; // channel tiles per workgroup, as the launch picks them
-  // (a single GEMM of two full block rows stays with the decode kernels up to an advantage of 1.56, as callers hold those
-  // launch plans: 28.1 against 17.7 us at 11008 x 4096 are left there, 20.6 against 17.0 at 4096 x 4096; 52 against 20 at
-  // 28672 x 2560 are not)
-  const double margin = !dual && M == 128 ? 1.56 : 1.0;
-  return tiled * margin <= rows_us((dual ? DUAL : SINGLE)[nt - 1], (tiles + nt - 1) / nt * rows64, K);
+  return tiled <= rows_us((dual ? DUAL : SINGLE)[nt - 1], (tiles + nt - 1) / nt * rows64, M, K);
 }
 
 // QINT8.  `tiles` of the whole launch.
@@ -287,7 +285,7 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
   if (family != BY_COST)
     return family == BY_TILES;
   const int64_t rows64 = (M + 63) / 64;
-  static constexpr RowsCost ROWS[3] = {{4.62, 2.33, 1.35}, {5.38, 4.48, 1.55}, {5.14, 5.03, 2.41}};
+  static constexpr RowsCost ROWS[3] = {{4.62, 2.33, 1.35, 0}, {5.38, 4.48, 1.55, 0}, {5.14, 5.03, 2.41, 0}};
   auto row_tiles = [](int64_t one) { return one < 512 ? 1 : one > 512 && one <= 768 ? 3 : 2; }; // as plan_skinny
   if (!dual && qbs == 256 && M >= big_min_rows() && env_int("TPPX_TILED_BIG_QINT8", 1) != 0 && env_int("TPPX_TILED_SMALL", 1) != 0) {
     // With half the CUs' worth of 64 x 256 workgroups and more the tiles were the faster side of every one of 682 shapes
@@ -299,8 +297,8 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
       return true;
     const int nt = row_tiles(tiles);
     const double k = 1e-3 * (double)K, wgs = (double)(rows64 * ((tiles + 7) / 8)), mk = 1e-6 * (double)M * (double)K;
-    static constexpr RowsCost R[3] = {{4.9, 2.26, 1.25}, {4.4, 3.96, 1.6}, {5.5, 4.25, 2.3}};
-    return 6.6 + k * (2.33 + 0.80 * wgs / 256.0) + 0.3 * mk <= rows_us(R[nt - 1], (tiles + nt - 1) / nt * rows64, K) + 0.8 * mk;
+    static constexpr RowsCost R[3] = {{4.9, 2.26, 1.25, 0}, {4.4, 3.96, 1.6, 0}, {5.5, 4.25, 2.3, 0}};
+    return 6.6 + k * (2.33 + 0.80 * wgs / 256.0) + 0.3 * mk <= rows_us(R[nt - 1], (tiles + nt - 1) / nt * rows64, M, K) + 0.8 * mk;
   }
   const int64_t wgs = ((M + 127) / 128) * ((tiles + 15) / 16);
   const bool small = wgs <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0;
@@ -311,7 +309,7 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
     const double one_us = wgs1 <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0 ? 8.0 + (double)K * 0.006
                                                                               : (double)((wgs1 + 255) / 256) * (10.0 + (double)K * 0.0075);
     const int nt = row_tiles(one);
-    if (!by_block_rows(one_us, one) && tiled_us > 1.15 * 2.0 * rows_us(ROWS[nt - 1], (one + nt - 1) / nt * rows64, K))
+    if (!by_block_rows(one_us, one) && tiled_us > 1.15 * 2.0 * rows_us(ROWS[nt - 1], (one + nt - 1) / nt * rows64, M, K))
       return false;
   }
   return by_block_rows(tiled_us, tiles);
@@ -322,7 +320,7 @@ static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tile
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
     return family == BY_TILES;
-  static constexpr RowsCost ROWS[2] = {{1.63, 2.01, 2.40}, {1.16, 3.71, 3.11}};
+  static constexpr RowsCost ROWS[2] = {{1.63, 2.01, 2.40, 0}, {1.16, 3.71, 3.11, 0}};
   const int64_t rows64 = (M + 63) / 64;
   int64_t all = 0;
   double rows = 0.0;
@@ -330,7 +328,7 @@ static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tile
   for (int i = 0; i < n; i++) {
     const int nt = tiles[i] > 512 ? 2 : 1;
     const int64_t wgs = (tiles[i] + nt - 1) / nt * rows64;
-    rows += rows_us(ROWS[nt - 1], wgs, K);
+    rows += rows_us(ROWS[nt - 1], wgs, M, K);
     one_round = one_round && wgs <= 256;
     all += tiles[i];
   }

@@ -330,6 +330,11 @@ def test_kernel_family_of_short_prompts():
         assert "<2, false, 2, 2>" in one(M, 12288, 4096) and "<2, false, 2, 2>" in one(M, 11008, 4096), M  # 18 us (26)
         assert "skinny_mxfp4" in one(M, 1024, 4096), M                                              # 8 us (tiles 16)
 
+    # 64 x 128 workgroups in whole columns per XCD drift apart from 21 row blocks on, also with an even number of them
+    assert "<2, false, 2, 2>" not in one(2048, 9088, 8704) and "<2, false, 2, 2>" not in one(1744, 6528, 10496)  # 250 us (342), 183 (251)
+    assert "<2, false, 2, 2>" not in qkv(2048, 1856, 13312) and "<2, true, 2, 2>" not in pair(2048, 2880, 7168)   # 230 us (339), 134 (180)
+    assert "<2, false, 2, 2>" in one(2048, 4800, 4096)                                              # rectangles: 63 us (74)
+
     def per_weight(M, N, K, weight_bytes):
         return not L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, weight_bytes)
 

@@ -1718,8 +1718,7 @@ static constexpr TileCost BF16_COST[N_TILES] = {
     {},
     {3.35, 0.708, 0.2, -2.67, 3.75, -0.226, 0.857, 0.388, 0.285, 0.076, 0.111},
 };
-static double tile_us(const TileCost& k, int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
-  const int64_t wgs = mb * nb;
+static double tile_us(const TileCost& k, int tile, int64_t wgs, double s, double weight_mb) {
   const double r = (double)((wgs + 255) / 256), f = (double)wgs / 256.0 - (r - 1.0);
   if (r <= 1.0)
     return k.a + (k.b + k.c * f) * s + k.g * weight_mb;
@@ -1727,15 +1726,38 @@ static double tile_us(const TileCost& k, int tile, int64_t mb, int64_t nb, doubl
   const double rs = std::min(r * s, 448.0 * 4096.0 / (TILE_ROWS[tile] * TILE_COLS16[tile]));
   return k.p + k.q * r + (k.u + k.v * r + k.w * f + k.z * 1e-3 * rs * r) * s + k.h * weight_mb;
 }
-static double mxfp4_tile_us(int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
-  const double us = tile_us(MXFP4_COST[tile], tile, mb, nb, s, weight_mb);
-  // An odd number of row blocks leaves no rectangles for the XCDs (tile_of_block), and columns of more row blocks than
-  // fit a CU set drift apart in K: 21 row blocks of 64 cost 10 % more, 27 and 29 29 % (K from 3072; 6 % up to 2048).
-  return tile == TILE_64_128 && mb * nb > 256 && (mb & 1) && mb >= 21
-             ? us * (1.0 + std::min(0.29, 0.1 + 0.031 * (double)(mb - 21)) * std::min(1.0, std::max(0.0, (s - 8.0) / 16.0))) : us;
+
+// How many of the 8 rectangles of tile_of_block lie along M: the split that moves the fewest bytes from memory into the L2s
+// (every XCD fetches 1/xm of the activations and xm/8 of the weights)
+static int xcd_split(int64_t mb, int64_t nb, double a_bytes, double w_bytes) {
+  double best = 8.0 * (a_bytes + w_bytes / 8.0); // xm = 1: an eighth of the channel blocks each, whether or not 8 divides them
+  int split = 1;
+  for (int xm = 2; xm <= 4; xm *= 2)
+    if (mb % xm == 0 && nb % (8 / xm) == 0) {
+      const double fill = 8.0 * (a_bytes / xm + w_bytes * xm / 8.0);
+      if (fill < best) {
+        best = fill;
+        split = xm;
+      }
+    }
+  return split;
 }
-static double bf16_tile_us(int tile, int64_t mb, int64_t nb, double s, double weight_mb) {
-  return tile_us(BF16_COST[tile], tile, mb, nb, s, weight_mb);
+
+constexpr double MXFP4_WEIGHT_BYTES = 0.53;
+static double mxfp4_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb) {
+  const int64_t mb = (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile];
+  const double us = tile_us(MXFP4_COST[tile], tile, mb * nb, s, weight_mb);
+  // Without a split along M an XCD walks whole columns, and from 21 row blocks of 64 on the columns of the workgroups that are
+  // resident together drift apart in K: 3 % more for each, 24 row blocks 12 .. 20 %, 29 25 .. 33 %, 32 30 .. 37 % (from K = 2560
+  // on; 10 % at 32 row blocks of K = 1536).  With rectangles (an even number of row blocks and channel blocks to go with it) 32
+  // row blocks are as fast as the estimate.  2048 x 9088 x 8704 342 us where 128 x 256 takes 250.
+  if (tile != TILE_64_128 || mb <= 20 || mb * nb <= 256 ||
+      xcd_split(mb, nb, (double)M * 2.0, (double)nb * TILE_COLS16[tile] * 16.0 * MXFP4_WEIGHT_BYTES) != 1)
+    return us;
+  return us * (1.0 + std::min(0.36, 0.03 * (double)(mb - 20)) * std::min(1.0, std::max(0.0, (s - 8.0) / 12.0)));
+}
+static double bf16_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb) {
+  return tile_us(BF16_COST[tile], tile, (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile] * nb, s, weight_mb);
 }
 
 // the tiles a launch may take, one bit each.  scales4: scale bytes on a 4-byte address (the ring forms move four at a time)
@@ -1763,7 +1785,7 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
     int64_t nb = 0;
     for (int g = 0; g < (dual ? 1 : n); g++)
       nb += (tiles[g] + tpw - 1) / tpw;
-    if (const double c = us(i, (M + TILE_ROWS[i] - 1) / TILE_ROWS[i], nb, (double)(K / 128), (double)(all * 32 * K) * 1e-6);
+    if (const double c = us(i, M, nb, (double)(K / 128), (double)(all * 32 * K) * 1e-6);
         c < (i >= TILE_64_128 ? 0.99 : 1.0) * best) { // (a tie goes to the larger tiles, which read less)
       best = c;
       shape = i;
@@ -1850,19 +1872,7 @@ static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int 
   for (int i = n; i <= TPPX_MAX_SEGS; i++)
     P.nb0[i] = nb;
   P.n_seg = n;
-  // XCD rectangles: the split that moves the fewest bytes from memory into the L2s (activations: rows x K bf16 per
-  // row block, fetched by 8 / xm XCDs... every XCD fetches 1/xm of them; weights xm/8 each)
-  const double a_bytes = (double)t[0].M * t[0].K * 2.0, w_bytes = (dual ? 2.0 : 1.0) * nb * tpw * 16.0 * t[0].K * bytes_per_weight;
-  double best = 8.0 * (a_bytes + w_bytes / 8.0); // xm = 1: an eighth of the channel blocks each, whether or not 8 divides them
-  P.xm = 1;
-  for (int xm = 2; xm <= 4; xm *= 2)
-    if (MB % xm == 0 && nb % (8 / xm) == 0) {
-      const double fill = 8.0 * (a_bytes / xm + w_bytes * xm / 8.0);
-      if (fill < best) {
-        best = fill;
-        P.xm = xm;
-      }
-    }
+  P.xm = xcd_split(MB, nb, (double)t[0].M * t[0].K * 2.0, (dual ? 2.0 : 1.0) * nb * tpw * 16.0 * t[0].K * bytes_per_weight);
   const int env_xm = env_int("TPPX_TILED_XCD_M", 0);
   if ((env_xm == 1 || env_xm == 2 || env_xm == 4) && MB % env_xm == 0 && nb % (8 / env_xm) == 0)
     P.xm = env_xm;
@@ -1897,7 +1907,7 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
   if (shape < 0 || shape > TILE_128_128 || (shape == TILE_128_128 && !scales4))
     shape = cheapest_tile(t, n, dual, mxfp4_tiles(scales4) & ~mxfp4_fixed_plans(t, n, dual), mxfp4_tile_us);
   BigParams P;
-  const int wgs = big_params(P, t, n, dual, shape, 0.53);
+  const int wgs = big_params(P, t, n, dual, shape, MXFP4_WEIGHT_BYTES);
   switch (shape) {
   case TILE_128_512:
     return dual ? big_launch<8, true, 1, 8>(P, wgs, stream) : big_launch<8, false, 1, 8>(P, wgs, stream);

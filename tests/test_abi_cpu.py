@@ -244,10 +244,15 @@ def test_launch_plans_of_the_baseline_shapes():
     assert "big_mxfp4_kernel<2, false, 2, 2> grid=256x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 512, 4096, 4096,
                                                                              _lib.FLAG_FORCE_TILED, 0)[0]
     assert "big_mxfp4_kernel<2, false, 2, 2>" in plan(L.tppx_plan_linear_mxfp4, 512, 4096, 4096, 0, 0)[0]   # and it is the choice
-    assert "big_mxfp4_kernel<4, false, 2, 4> grid=172x1x1 block=512" in plan(L.tppx_plan_linear_mxfp4, 512, 11008, 4096,
-                                                                             _lib.FLAG_FORCE_TILED, 0)[0]
+    assert "big_mxfp4_kernel<2, false, 2, 2> grid=688x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 512, 11008, 4096,
+                                                                             _lib.FLAG_FORCE_TILED, 0)[0]   # 42 us (172 of 128 x 256: 50)
+    assert "big_mxfp4_kernel<4, false, 2, 4> grid=256x1x1 block=512" in plan(L.tppx_plan_linear_mxfp4, 2048, 4096, 4096,
+                                                                             _lib.FLAG_FORCE_TILED, 0)[0]   # 50 us (64 x 128: 53)
     pair7 = (ctypes.c_int64 * 2)(11008, 11008)
-    assert "big_mxfp4_kernel<4, true, 2, 4> grid=172x1x1 block=512" in plan(L.tppx_plan_multi_linear_mxfp4, pair7, 2, 256, 4096, 1,
+    assert "big_mxfp4_kernel<2, true, 2, 2> grid=688x1x1 block=256" in plan(L.tppx_plan_multi_linear_mxfp4, pair7, 2, 256, 4096, 1,
+                                                                           _lib.FLAG_FORCE_TILED, 0)[0]     # 44 us (128 x 256: 51)
+    pair2 = (ctypes.c_int64 * 2)(2048, 2048)
+    assert "big_mxfp4_kernel<4, true, 2, 4> grid=256x1x1 block=512" in plan(L.tppx_plan_multi_linear_mxfp4, pair2, 2, 2048, 4096, 1,
                                                                            _lib.FLAG_FORCE_TILED, 0)[0]
     assert "big_qint8_small_kernel grid=128x1x1 block=512" in plan(L.tppx_plan_linear_qint8, 512, 4096, 4096, 256, 1,
                                                                     _lib.FLAG_FORCE_TILED, 1 << 25)[-1]
@@ -256,8 +261,10 @@ def test_launch_plans_of_the_baseline_shapes():
     pair1 = (ctypes.c_int64 * 2)(4096, 4096)
     assert "big_mxfp4_kernel<2, true, 2, 2> grid=256x1x1 block=256" in plan(L.tppx_plan_multi_linear_mxfp4, pair1, 2, 256, 4096, 1,
                                                                            _lib.FLAG_FORCE_TILED, 0)[0]
-    assert "big_mxfp4_kernel<8, false, 1, 8> grid=176x1x1 block=512" in plan(L.tppx_plan_linear_mxfp4, 1024, 11008, 4096,
-                                                                             _lib.FLAG_FORCE_TILED, 0)[0]  # 128 x 512: eight waves anyway
+    assert "big_mxfp4_kernel<2, false, 2, 2> grid=1376x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 1024, 11008, 4096,
+                                                                              _lib.FLAG_FORCE_TILED, 0)[0]  # 79 us (128 x 512: 81)
+    for M, other in ((511, 512), (1000, 1024)):  # whole 128-row blocks make no difference
+        assert plan(L.tppx_plan_linear_mxfp4, M, 11008, 4096, 0, 0) == plan(L.tppx_plan_linear_mxfp4, other, 11008, 4096, 0, 0)
     # from 65 rows on the 64-row forms take what the planner hands to a tiled kernel
     assert "big_mxfp4_kernel<2, false, 2, 2> grid=96x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 160, 4096, 4096, 0, 0)[0]
     assert "big_mxfp4_kernel<2, false, 2, 2> grid=64x1x1" in plan(L.tppx_plan_linear_mxfp4, 128, 4096, 4096, 0, ws)[0]  # 17.0 us (rows 17.9)

@@ -1879,23 +1879,6 @@ static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int 
   return MB * nb;
 }
 
-// Launches of whole 128-row blocks that fill between two thirds and seven tenths of the CUs as 128 x 256 or 128 x 512 keep
-// those tiles: callers hold their launch plans (512 or 1024 rows x 11008, pair of 256 rows).  64 x 128 would be the faster
-// one at the first and the last, 39.5 against 46.6 us and 41.5 against 48.8; 77.2 against 75.5 at the second.
-static unsigned mxfp4_fixed_plans(const TiledParams* t, int n, bool dual) {
-  if (t[0].M % 128 != 0)
-    return 0u;
-  for (int tile : {TILE_128_256, TILE_128_512}) {
-    const int tpw = TILE_COLS16[tile] / (dual ? 2 : 1);
-    int nb = 0;
-    for (int i = 0; i < (dual ? 1 : n); i++)
-      nb += (t[i].tiles + tpw - 1) / tpw;
-    if (const int64_t wgs = (int64_t)(t[0].M / 128) * nb; wgs >= 171 && wgs <= 179)
-      return 1u << TILE_64_128;
-  }
-  return 0u;
-}
-
 // dual: t[0] = gate, t[1] = up (equal shapes, n == 2); y[m][n] = silu(gate) * up goes to t[1].y
 hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
@@ -1905,7 +1888,7 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
     scales4 = scales4 && (reinterpret_cast<uintptr_t>(t[i].sw) & 3u) == 0;
   int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
   if (shape < 0 || shape > TILE_128_128 || (shape == TILE_128_128 && !scales4))
-    shape = cheapest_tile(t, n, dual, mxfp4_tiles(scales4) & ~mxfp4_fixed_plans(t, n, dual), mxfp4_tile_us);
+    shape = cheapest_tile(t, n, dual, mxfp4_tiles(scales4), mxfp4_tile_us);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, MXFP4_WEIGHT_BYTES);
   switch (shape) {

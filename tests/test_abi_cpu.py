@@ -347,7 +347,15 @@ def test_kernel_family_of_short_prompts():
 
     assert per_weight(200, 1024, 3584, 1) and per_weight(256, 1024, 4096, 1)    # 22 us (one launch 28), 26 (31)
     assert not per_weight(212, 1024, 2304, 1)                                   # 22 us (per weight 45)
-    assert per_weight(160, 1024, 5120, 2) and not per_weight(160, 4096, 5120, 2)
+    assert per_weight(160, 1024, 5120, 2) and not per_weight(160, 4096, 5120, 2)  # 25 us (one launch 29)
+
+    def bf16_tiles(M, N, K):
+        return L.tppx_group_is_one_launch((ctypes.c_int64 * 1)(N), 1, M, K, 2)
+
+    # single bf16 weights that come from memory: the decode kernels where they are few and K is long
+    assert not bf16_tiles(82, 2304, 10496) and not bf16_tiles(128, 2432, 11776) and not bf16_tiles(100, 3584, 18944)  # 39 us (55), 54 (70), 85 (106)
+    assert not bf16_tiles(160, 1536, 18944) and not bf16_tiles(105, 2304, 5376)                      # 70 us (91), 24 (32)
+    assert bf16_tiles(128, 11008, 4096) and bf16_tiles(300, 4096, 4096) and bf16_tiles(1000, 1024, 4096)
 
 
 def test_group_is_one_launch():

@@ -315,28 +315,24 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
   return by_block_rows(tiled_us, tiles);
 }
 
-// Unquantized bf16 weights: n of them as one launch of the large-M kernel against one decode launch each
+// Unquantized bf16 weights: n of them as one launch of the large-M kernel against one decode launch each.  Both sides fitted with
+// weights that come from memory: 2304 x 10496 at 82 rows 39 us on the decode kernels (tiles 55), 1024 x 5120 twice at 160 rows 25
+// as two decode launches (one of the tiles 29), 4096 x 4096 at 128 rows 23 (27), at 200 rows 41 (24).
 static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tiles, int n) {
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
     return family == BY_TILES;
-  static constexpr RowsCost ROWS[2] = {{1.63, 2.01, 2.40, 0}, {1.16, 3.71, 3.11, 0}};
+  static constexpr RowsCost ROWS[2] = {{1.98, 1.14, 1.73, 0.561}, {1.96, 1.97, 2.15, 1.2}};
   const int64_t rows64 = (M + 63) / 64;
   int64_t all = 0;
   double rows = 0.0;
-  bool one_round = true;
   for (int i = 0; i < n; i++) {
     const int nt = tiles[i] > 512 ? 2 : 1;
-    const int64_t wgs = (tiles[i] + nt - 1) / nt * rows64;
-    rows += rows_us(ROWS[nt - 1], wgs, M, K);
-    one_round = one_round && wgs <= 256;
+    rows += rows_us(ROWS[nt - 1], (tiles[i] + nt - 1) / nt * rows64, M, K);
     all += tiles[i];
   }
-  if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0) {
-    // A group whose every decode launch is a single round stays with one launch per weight up to an advantage of 1.42, as
-    // callers count on it for pairs of 1024 channels (2 x 1024 x 5120 at 160 rows: 28.3 us, one launch would take 22.5).
-    return tiled_bf16_us(M, K, all) * (n > 1 && one_round ? 1.42 : 1.0) <= rows;
-  }
+  if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
+    return tiled_bf16_us(M, K, all) <= rows;
   const int64_t wgs = ((M + 127) / 128) * ((all + 7) / 8); // tiled_bf16_kernel
   return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
          (double)rows64 * (8.0 + (double)all * 32.0 * (double)K / 5.5e6 + (double)K * 0.0008);

@@ -1695,12 +1695,15 @@ static constexpr int TILE_COLS16[N_TILES] = {16, 16, 32, 8, 8, 16}; // 16-channe
 //   one round     a + (b + c f) s
 //   more          p + q r + (u + v r + w f + z r s / 1000) s     (z: the clock falls under the power limit as a launch
 //                                                                 grows; measured up to 28672 x 8192 pairs of 2048 rows)
-// bf16 weights: and g (one round) or h us for each MB of them, which come from memory at whatever tile.
-// Fitted to 2736 launches of each format: 65 .. 2048 rows, linears and pairs of 1024 .. 28672 x 1024 .. 18944, every tile
-// forced, weights rotated through 2 GB.  On 792 others (random channels and K) the tile chosen is 0.4 % (MXFP4) and 0.75 %
-// (bf16) off the fastest on average, 11 and 15 % in the worst hundredth.
+// bf16 weights: and g (one round) or h us for each MB of them, and e us per round for the epilogue of a gate/up pair.
+// MXFP4: fitted to 2736 launches of 65 .. 2048 rows, linears and pairs of 1024 .. 28672 x 1024 .. 18944, every tile forced; on
+// 792 others (random channels and K) the tile chosen was 0.4 % off the fastest on average, 11 % in the worst hundredth.
+// bf16: fitted to 4100 launches, q/k/v groups among them, up to pairs of 28672 x 8192, most of all where the tile is within 20 %
+// of the fastest, and with weights that come from memory: 96 of them, or as many as fill 2 GB, in turn.  (With four in turn most
+// lie in the Infinity Cache, as they never do in a model, and the estimates came out 20 .. 30 % low.)  On 2600 others the family
+// and tile chosen are 0.3 % off the fastest on average and 9 % in the worst hundredth (1.7 % and 25 % before).
 struct TileCost {
-  double a, b, c, p, q, u, v, w, z, g, h;
+  double a, b, c, p, q, u, v, w, z, g, h, e;
 };
 static constexpr TileCost MXFP4_COST[N_TILES] = {
     {7.75, 1.88, 0.607, -6.18, 12.4, -0.498, 2.31, 0.768, 0.256, 0, 0},
@@ -1711,20 +1714,20 @@ static constexpr TileCost MXFP4_COST[N_TILES] = {
     {},
 };
 static constexpr TileCost BF16_COST[N_TILES] = {
-    {7.22, 1.96, 0.625, -8.28, 13.5, -0.615, 2.49, 0.883, 0.297, 0.0298, 0.0316},
-    {5.39, 1.02, 0.341, 1.28, 3.47, -0.41, 1.26, 0.607, 0.268, 0.0726, 0.0559},
-    {6.9, 1.91, 0.543, -15.3, 15.2, -0.583, 2.38, 1.15, 0.281, 0.0795, 0.089},
-    {3.26, 0.404, 0.148, 2.96, 0.221, -0.246, 0.539, 0.206, 0.134, 0.0443, 0.0668},
+    {9.19, 1.73, 0.784, 2.54, 6.07, -1.52, 2.92, 1.23, 0.155, 0.0249, 0.00722, 3.73},
+    {7.3, 1.13, 0.298, 2.01, 3.53, -0.41, 1.25, 0.708, 0.288, 0.043, 0.0481, 1.07},
+    {8.86, 1.81, 0.692, -1.47, 7.78, -1.4, 2.81, 1.4, 0.195, 0.0518, 0.0267, 3.63},
+    {3.7, 0.613, 0.0187, 2.24, 0.731, 0.0345, 0.498, 0.186, 0.041, 0.0584, 0.069, 0.555},
     {},
-    {3.35, 0.708, 0.2, -2.67, 3.75, -0.226, 0.857, 0.388, 0.285, 0.076, 0.111},
+    {4.61, 1.02, 0.051, 1.68, 3.15, -0.354, 0.929, 0.634, 0.195, 0.0614, 0.0625, 1.05},
 };
-static double tile_us(const TileCost& k, int tile, int64_t wgs, double s, double weight_mb) {
+static double tile_us(const TileCost& k, int tile, int64_t wgs, double s, double weight_mb, bool dual) {
   const double r = (double)((wgs + 255) / 256), f = (double)wgs / 256.0 - (r - 1.0);
   if (r <= 1.0)
-    return k.a + (k.b + k.c * f) * s + k.g * weight_mb;
+    return k.a + (k.b + k.c * f) * s + k.g * weight_mb + (dual ? k.e : 0.0);
   // (the z term at most as far as it was measured: 448 rounds x steps of 256 x 256, the same work in the other tiles)
   const double rs = std::min(r * s, 448.0 * 4096.0 / (TILE_ROWS[tile] * TILE_COLS16[tile]));
-  return k.p + k.q * r + (k.u + k.v * r + k.w * f + k.z * 1e-3 * rs * r) * s + k.h * weight_mb;
+  return k.p + k.q * r + (k.u + k.v * r + k.w * f + k.z * 1e-3 * rs * r) * s + k.h * weight_mb + (dual ? k.e * r : 0.0);
 }
 
 // How many of the 8 rectangles of tile_of_block lie along M: the split that moves the fewest bytes from memory into the L2s
@@ -1744,9 +1747,9 @@ static int xcd_split(int64_t mb, int64_t nb, double a_bytes, double w_bytes) {
 }
 
 constexpr double MXFP4_WEIGHT_BYTES = 0.53;
-static double mxfp4_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb) {
+static double mxfp4_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb, bool dual) {
   const int64_t mb = (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile];
-  const double us = tile_us(MXFP4_COST[tile], tile, mb * nb, s, weight_mb);
+  const double us = tile_us(MXFP4_COST[tile], tile, mb * nb, s, weight_mb, dual);
   // Without a split along M an XCD walks whole columns, and from 21 row blocks of 64 on the columns of the workgroups that are
   // resident together drift apart in K: 3 % more for each, 24 row blocks 10 % (K = 4096) .. 21 % (K = 16384), 29 25 .. 33 %, 32
   // 31 .. 37 % (from K = 2560 on; 12 % at 32 row blocks of K = 1536).  With rectangles (an even number of row blocks and channel
@@ -1758,8 +1761,8 @@ static double mxfp4_tile_us(int tile, int64_t M, int64_t nb, double s, double we
   return us * (1.0 + std::min(0.36, 0.03 * (double)(mb - 21) + 0.0007 * s) * std::min(1.0, std::max(0.0, (s - 8.0) / 12.0)) *
                          std::min(1.0, (double)(mb * nb + 256) / 1024.0));
 }
-static double bf16_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb) {
-  return tile_us(BF16_COST[tile], tile, (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile] * nb, s, weight_mb);
+static double bf16_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb, bool dual) {
+  return tile_us(BF16_COST[tile], tile, (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile] * nb, s, weight_mb, dual);
 }
 
 // the tiles a launch may take, one bit each.  scales4: scale bytes on a 4-byte address (the ring forms move four at a time)
@@ -1787,8 +1790,9 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
     int64_t nb = 0;
     for (int g = 0; g < (dual ? 1 : n); g++)
       nb += (tiles[g] + tpw - 1) / tpw;
-    if (const double c = us(i, M, nb, (double)(K / 128), (double)(all * 32 * K) * 1e-6);
-        c < (i >= TILE_64_128 ? 0.99 : 1.0) * best) { // (a tie goes to the larger tiles, which read less)
+    // (a tie goes to the larger tiles, which read less)
+    const double tie = i == TILE_64_256 && shape == TILE_64_128 ? 1.01 : i >= TILE_64_128 ? 0.99 : 1.0;
+    if (const double c = us(i, M, nb, (double)(K / 128), (double)(all * 32 * K) * 1e-6, dual); c < tie * best) {
       best = c;
       shape = i;
     }

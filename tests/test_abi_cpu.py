@@ -345,9 +345,20 @@ def test_kernel_family_of_short_prompts():
     def per_weight(M, N, K, weight_bytes):
         return not L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, weight_bytes)
 
-    assert per_weight(200, 1024, 3584, 1) and per_weight(256, 1024, 4096, 1)    # 22 us (one launch 28), 26 (31)
-    assert not per_weight(212, 1024, 2304, 1)                                   # 22 us (per weight 45)
+    # QINT8 pairs: one launch from 65 rows on, 18 us (per weight 24), 20 (26), 13 (21), 62 (96 on rows, 123 on tiles), 9 (17)
+    for M, N, K in ((200, 1024, 3584), (256, 1024, 4096), (212, 1024, 2304), (128, 2432, 16128), (65, 1024, 1024)):
+        assert not per_weight(M, N, K, 1), (M, N, K)
+    assert per_weight(64, 1024, 4096, 1)
     assert per_weight(160, 1024, 5120, 2) and not per_weight(160, 4096, 5120, 2)  # 25 us (one launch 29)
+
+    def qint8(M, N, K):
+        _lib.check(L.tppx_plan_linear_qint8(M, N, K, 256, 1, 0, 1 << 25, buf, len(buf)))
+        return buf.value.decode().strip().splitlines()[-1]
+
+    # single QINT8 weights that come from memory: the decode kernels where they are few, also for short K
+    assert "skinny_qint8" in qint8(192, 1408, 8448) and "skinny_qint8" in qint8(251, 1152, 11776)    # 28 us (35), 39 (47)
+    assert "skinny_qint8" in qint8(128, 2368, 12032) and "skinny_qint8" in qint8(96, 1024, 1024)      # 41 us (48), 8.1 (8.8)
+    assert "big_qint8" in qint8(300, 1024, 1024) and "big_qint8" in qint8(128, 11008, 4096)
 
     def bf16_tiles(M, N, K):
         return L.tppx_group_is_one_launch((ctypes.c_int64 * 1)(N), 1, M, K, 2)
@@ -373,7 +384,7 @@ def test_group_is_one_launch():
         assert one([11000] * 2, 333, 4096, bytes_per) == 0  # no whole tiles
         assert one([11008] * 2, 0, 4096, bytes_per) == 0 and one([], 333, 4096, bytes_per) == 0
         assert one([1 << 20] * 2, 333, 4096 // bytes_per, bytes_per) == 0  # weights of 4 GiB
-    assert one([5120] * 2, 66, 2048, 1) == 0 and one([5120] * 2, 129, 2048, 1) == 1  # per weight, then one launch
+    assert one([5120] * 2, 64, 2048, 1) == 0 and one([5120] * 2, 66, 2048, 1) == 1  # per weight, then one launch (14 us, per weight 26)
     assert one([11008] * 2, 333, 4096, 3) == 0
     assert one([4096, 1024, 1024], 2048, 4096, 2) == 1 and one([4096, 1024, 1024], 2048, 4096, 1) == 0  # bf16 only
 

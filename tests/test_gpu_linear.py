@@ -1061,10 +1061,13 @@ def test_prefill_qint8_pair_agrees_with_two_launches(fmt, M, N, K, monkeypatch):
 
 @pytest.mark.parametrize("fmt,M,N,K", [("qint8", 66, 5120, 2048), ("qint8", 128, 1536, 1024), ("bf16", 65, 64, 2048), ("bf16", 100, 32, 4096)])
 def test_groups_that_run_per_weight_are_asked_about_first(fmt, M, N, K, monkeypatch):
-    """Where the library would answer TPPX_EUNSUPPORTED to a gate/up pair or a q/k/v group (few rows on small weights),
-    the call is not made and nothing is prepared for it: the outputs are those of one call per weight."""
+    """Where the library would answer TPPX_EUNSUPPORTED to a gate/up pair or a q/k/v group (few rows on small weights;
+    QINT8: by the row threshold, its estimate takes every pair), the call is not made and nothing is prepared for it:
+    the outputs are those of one call per weight."""
     from tpp_pytorch_extension import _lib
     ops = _ops()
+    if fmt == "qint8":
+        monkeypatch.setenv("TPPX_TILED_MIN_M", "512")
     ws = [block_bf16(randn_bf16((N, K), 0.05, 775 + i), bc=256).cuda() for i in range(2)]
     if fmt == "qint8":
         ws = [ops.remap_and_quantize_qint8(w) for w in ws]

@@ -277,42 +277,34 @@ static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, boo
   return tiled <= rows_us((dual ? DUAL : SINGLE)[nt - 1], (tiles + nt - 1) / nt * rows64, M, K);
 }
 
-// QINT8.  `tiles` of the whole launch.
-// The gate/up pair (dual) stands against two launches behind a quantizer each, on figures of an earlier form of the tiles
-// (128 x 256, at most 128 of them twice as many of 64 x 256; blocks other than 256 wide still go by them).
+// QINT8.  `tiles` of the whole launch (dual: the gate/up pair, of both projections).
 static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, bool dual, int64_t qbs) {
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
     return family == BY_TILES;
   const int64_t rows64 = (M + 63) / 64;
-  static constexpr RowsCost ROWS[3] = {{4.62, 2.33, 1.35, 0}, {5.38, 4.48, 1.55, 0}, {5.14, 5.03, 2.41, 0}};
-  auto row_tiles = [](int64_t one) { return one < 512 ? 1 : one > 512 && one <= 768 ? 3 : 2; }; // as plan_skinny
-  if (!dual && qbs == 256 && M >= big_min_rows() && env_int("TPPX_TILED_BIG_QINT8", 1) != 0 && env_int("TPPX_TILED_SMALL", 1) != 0) {
-    // With half the CUs' worth of 64 x 256 workgroups and more the tiles were the faster side of every one of 682 shapes
-    // (65 .. 1000 rows, 512 .. 28672 channels, K 1024 .. 18944: up to four times).  Launches of fewer run as 64 x 128, in one
-    // round, against the decode kernels' rounds; both sides in us, the quantizer included, within 5 % on average: the choice
-    // is 0.02 % off the faster one, 7 % at worst (the fit before, to the earlier form of the tiles: 8.6 %, 132 %).
-    // (K up to 1024: both at what a launch takes, 8.5 .. 9.1 us)
-    if (K <= 1024 || rows64 * ((tiles + 15) / 16) >= 128)
+  if (qbs == 256 && M >= big_min_rows() && env_int("TPPX_TILED_BIG_QINT8", 1) != 0 && env_int("TPPX_TILED_SMALL", 1) != 0) {
+    // The pair as one launch against two launches behind a quantizer each, on whichever family: the faster side of 1429 of 1449
+    // pairs (65 .. 1024 rows, 1024 .. 14336 channels, K 1024 .. 18944), up to twice, 14 % slower at worst.  (An earlier form of
+    // the tiles left those of few workgroups per weight: 2 x 2432 x 16128 at 128 rows 125 us where one launch takes 63.)
+    // Linears and q/k/v groups: with half the CUs' worth of 64 x 256 workgroups and more the tiles were the faster side of each of
+    // 1216 launches, up to four times; with K up to 1024 both take what a launch takes from 129 rows on (8.5 us), the tiles less from
+    // 257 on.
+    if (dual || rows64 * ((tiles + 15) / 16) >= 128 || (K <= 1024 && rows64 > 2))
       return true;
-    const int nt = row_tiles(tiles);
+    // Fewer run as 64 x 128, in one round, against the decode kernels' rounds; both sides in us with weights that come from
+    // memory, the quantizer included.  On 1260 launches of other shapes the choice is 0.04 % off the faster one on average, 1 % in
+    // the worst hundredth (fitted to four weights in turn, which mostly lie in the Infinity Cache: 0.35 % and 15 %).
+    const int nt = tiles < 512 ? 1 : tiles > 512 && tiles <= 768 ? 3 : 2; // as plan_skinny
     const double k = 1e-3 * (double)K, wgs = (double)(rows64 * ((tiles + 7) / 8)), mk = 1e-6 * (double)M * (double)K;
-    static constexpr RowsCost R[3] = {{4.9, 2.26, 1.25, 0}, {4.4, 3.96, 1.6, 0}, {5.5, 4.25, 2.3, 0}};
-    return 6.6 + k * (2.33 + 0.80 * wgs / 256.0) + 0.3 * mk <= rows_us(R[nt - 1], (tiles + nt - 1) / nt * rows64, M, K) + 0.8 * mk;
+    static constexpr RowsCost ROWS[3] = {{5.06, 2.34, 1.30, 0}, {4.9, 3.96, 1.6, 0}, {5.5, 4.25, 2.3, 0}};
+    return 6.07 + k * (3.01 + 0.668 * wgs / 256.0) + 0.257 * mk <=
+           rows_us(ROWS[nt - 1], (tiles + nt - 1) / nt * rows64, M, K) + (nt == 1 ? 0.1 : 0.8) * mk;
   }
   const int64_t wgs = ((M + 127) / 128) * ((tiles + 15) / 16);
   const bool small = wgs <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0;
   const double tiled_us = small ? 8.0 + (double)K * 0.006 : (double)((wgs + 255) / 256) * (10.0 + (double)K * 0.0075);
-  auto by_block_rows = [&](double us, int64_t n) { return us <= (double)rows64 * (5.0 + (double)n * 16.0 * (double)K / 5.5e6 + (double)K * 0.0004); };
-  if (dual) {
-    const int64_t one = tiles / 2, wgs1 = ((M + 127) / 128) * ((one + 15) / 16);
-    const double one_us = wgs1 <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0 ? 8.0 + (double)K * 0.006
-                                                                              : (double)((wgs1 + 255) / 256) * (10.0 + (double)K * 0.0075);
-    const int nt = row_tiles(one);
-    if (!by_block_rows(one_us, one) && tiled_us > 1.15 * 2.0 * rows_us(ROWS[nt - 1], (one + nt - 1) / nt * rows64, M, K))
-      return false;
-  }
-  return by_block_rows(tiled_us, tiles);
+  return tiled_us <= (double)rows64 * (5.0 + (double)tiles * 16.0 * (double)K / 5.5e6 + (double)K * 0.0004);
 }
 
 // Unquantized bf16 weights: n of them as one launch of the large-M kernel against one decode launch each.  Both sides fitted with

@@ -1116,8 +1116,8 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
     if N2 != N or w_gate._qscheme != w_up._qscheme:
         raise TppxError(_lib.ESHAPE, "gate and up projections must have the same shape and format")
     if w_gate._qscheme != QSCHEME_MXFP:
-        # the large-M kernel (from 65 rows, where the library's estimate prefers it to the row kernels, blocks of 256)
-        # takes the pair as one launch behind one quantization: rounds(2w) <= 2 rounds(w), so it is never the slower way
+        # the large-M kernel (from 65 rows, blocks of 256) takes the pair as one launch behind one quantization: the faster
+        # way for 1429 of 1449 pairs of 65 .. 1024 rows, up to twice
         if M > 64 and w_gate.block_size == w_up.block_size == 256 and \
                 L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, 1):
             y = torch.empty(tuple(input.shape[:-1]) + (N,), dtype=torch.bfloat16, device=x.device)

@@ -254,8 +254,8 @@ def test_launch_plans_of_the_baseline_shapes():
     pair2 = (ctypes.c_int64 * 2)(2048, 2048)
     assert "big_mxfp4_kernel<4, true, 2, 4> grid=256x1x1 block=512" in plan(L.tppx_plan_multi_linear_mxfp4, pair2, 2, 2048, 4096, 1,
                                                                            _lib.FLAG_FORCE_TILED, 0)[0]
-    assert "big_qint8_small_kernel grid=128x1x1 block=512" in plan(L.tppx_plan_linear_qint8, 512, 4096, 4096, 256, 1,
-                                                                    _lib.FLAG_FORCE_TILED, 1 << 25)[-1]
+    assert "big_qint8_narrow_kernel grid=256x1x1 block=256" in plan(L.tppx_plan_linear_qint8, 512, 4096, 4096, 256, 1,
+                                                                     _lib.FLAG_FORCE_TILED, 1 << 25)[-1]     # 22 us (128 of 64 x 256: 30)
     assert "big_qint8_kernel grid=172x1x1 block=512" in plan(L.tppx_plan_linear_qint8, 512, 11008, 4096, 256, 1,
                                                               _lib.FLAG_FORCE_TILED, 1 << 25)[-1]
     pair1 = (ctypes.c_int64 * 2)(4096, 4096)

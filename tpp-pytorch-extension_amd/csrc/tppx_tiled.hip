@@ -2082,8 +2082,9 @@ hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t str
   };
   const int64_t wgs64 = (int64_t)((t[0].M + 63) / 64) * channel_blocks(8); // workgroups of 64 x 256
   const bool small = env_int("TPPX_TILED_SMALL", 1) != 0;
-  if (small && wgs64 < 128) { // less than half the CUs: 64 x 128, twice as many (4096 x 4096 at 333 rows 19.6 -> 15.0 us; from
-                              // 129 of 64 x 256 on, where they would take a second round, 64 x 128 loses: 24.5 against 25.7)
+  if (small && wgs64 <= 128) { // up to half the CUs: 64 x 128, twice as many, one round (4096 x 4096 at 333 rows 19.6 -> 15.0 us, at
+                               // 512, exactly a round, 29.9 -> 21.9 with the quantizer; with 129 of 64 x 256 and more, where they
+                               // take a second round, 64 x 128 loses: 24.5 against 25.7)
     channel_blocks(4);
     return dual ? go(big_qint8_narrow_dual_kernel, 64, 4, Qint8Geom<4, 4>::LDS) : go(big_qint8_narrow_kernel, 64, 4, Qint8Geom<4, 4>::LDS);
   }

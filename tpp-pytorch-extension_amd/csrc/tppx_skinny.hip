@@ -2420,18 +2420,19 @@ __device__ __forceinline__ void skinny_rows_body(const DecodeParams& p) {
   }
 }
 
-// WS = W / 4 waves per SIMD
-template <int MG, int NT, bool DUAL, int WS, int W, bool PAIRS>
-__global__ void __launch_bounds__(W * 64)
+// waves of a workgroup: two to a SIMD, with one row group (whose waves hold less) four
+constexpr int rows_waves(int mg) { return mg == 1 ? 16 : 8; }
+
+template <int MG, int NT, bool DUAL>
+__global__ void __launch_bounds__(rows_waves(MG) * 64)
 skinny_mxfp4_mg_kernel(const DecodeParams p) {
-  static_assert(WS * 4 == W, "four SIMDs");
-  skinny_rows_body<false, MG, NT, DUAL, W, PAIRS>(p);
+  skinny_rows_body<false, MG, NT, DUAL, rows_waves(MG), rows_in_pairs(false, MG)>(p);
 }
 
-template <int MG, int NT, int W, bool PAIRS>
-__global__ void __launch_bounds__(W * 64)
+template <int MG, int NT>
+__global__ void __launch_bounds__(rows_waves(MG) * 64)
 skinny_bf16_kernel(const DecodeParams p) {
-  skinny_rows_body<true, MG, NT, false, W, PAIRS>(p);
+  skinny_rows_body<true, MG, NT, false, rows_waves(MG), rows_in_pairs(true, MG)>(p);
 }
 
 // Scale blocks that `runs` consecutive runs of `deal` tiles can touch (slots of activation scales a wave keeps in LDS).
@@ -2832,9 +2833,9 @@ hipError_t launch_skinny_mxfp4_mg(DecodeParams& p, int mg, int nt, bool dual, hi
   dim3 grid(p.groups, (p.M + mg * 16 - 1) / (mg * 16), p.S);
   if (p.S > 1 && (p.S > 4 || (p.ticket0 = skinny_split_tickets((int)(grid.x * grid.y))) < 0))
     return hipErrorInvalidValue;
-  const int waves = mg == 1 ? 16 : 8;
+  const int waves = rows_waves(mg);
   const size_t lds = skinny_rows_lds(false, mg, nt, waves); // the gate/up pair is reduced one half at a time
-#define SKMG(MG, NT, DUAL) return sk_launch(skinny_mxfp4_mg_kernel<MG, NT, DUAL, MG == 1 ? 4 : 2, MG == 1 ? 16 : 8, rows_in_pairs(false, MG)>, p, grid, waves, lds, stream)
+#define SKMG(MG, NT, DUAL) return sk_launch(skinny_mxfp4_mg_kernel<MG, NT, DUAL>, p, grid, waves, lds, stream)
 #define SKMG_NT(MG, DUAL) \
   do {                    \
     if (nt == 3)          \
@@ -2867,9 +2868,9 @@ hipError_t launch_skinny_mxfp4_mg(DecodeParams& p, int mg, int nt, bool dual, hi
 // bf16 weights: mg row groups of 16 per block row (1, 2 or 4), nt channel tiles per workgroup (1 or 2)
 hipError_t launch_skinny_bf16(DecodeParams& p, int mg, int nt, hipStream_t stream) {
   dim3 grid(p.groups, (p.M + mg * 16 - 1) / (mg * 16), 1);
-  const int waves = mg == 1 ? 16 : 8;
+  const int waves = rows_waves(mg);
   const size_t lds = skinny_rows_lds(true, mg, nt, waves);
-#define SKBF(MG, NT) return sk_launch(skinny_bf16_kernel<MG, NT, MG == 1 ? 16 : 8, rows_in_pairs(true, MG)>, p, grid, waves, lds, stream)
+#define SKBF(MG, NT) return sk_launch(skinny_bf16_kernel<MG, NT>, p, grid, waves, lds, stream)
   if (mg == 1) {
     if (nt == 2)
       SKBF(1, 2);

@@ -692,6 +692,37 @@ def test_bf16_weight_linear(M, N, K, post, layout):
     assert torch.equal(y, y2)
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "mxfp4"])
+@pytest.mark.parametrize("M", [16, 40, 200])
+def test_outputs_round_to_nearest_even(fmt, M):
+    """The fp32 sum of a GEMM becomes bf16 by round to nearest, ties to even, in the epilogues of the decode kernels, the row
+    groups and the tiles: sums built from three bf16 parts (all 24 bits, in different MFMA steps, weights of 1) around every
+    tie, with carries into the exponent and past the largest value, infinities and NaN, against torch's conversion."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    K, N = 256, 64
+    low = torch.tensor([0x0000, 0x0001, 0x7fff, 0x8000, 0x8001, 0xffff])
+    high = torch.tensor([0x3f80, 0x3f81, 0x3fff, 0x4000, 0x1234, 0x7f7e, 0x7f7f, 0x0c01])
+    bits = ((high[:, None] << 16) | low[None, :]).flatten()
+    bits = torch.cat([bits, bits | 0x80000000, torch.tensor([0x7f800000, 0xff800000, 0x7fc00000, 0])])
+    values = torch.from_numpy(bits.numpy().astype(np.uint32).view(np.float32))
+    w = block_bf16(torch.ones((N, K), dtype=torch.bfloat16)).cuda()
+    if fmt == "mxfp4":
+        w = ops.remap_and_quantize_mxfp4(w)
+        assert bool((w.dequantize() == 1).all())
+    for start in range(0, values.numel(), M):
+        v = values[torch.arange(start, start + M) % values.numel()]
+        x, rest = torch.zeros((M, K)), v.double()
+        for k in (0, 96, 224):
+            x[:, k] = torch.from_numpy((rest.float().numpy().view(np.uint32) & np.uint32(0xffff0000)).view(np.float32))
+            rest = torch.where(torch.isfinite(v), rest - x[:, k].double(), torch.zeros_like(rest))
+        y = ops.linear(x.to(torch.bfloat16).cuda(), w, None, flags=_lib.FLAG_FORCE_TILED if M > 64 else 0).cpu()
+        want = v.to(torch.bfloat16)[:, None].expand(M, N).contiguous()
+        nan = torch.isnan(want)
+        assert torch.equal(torch.isnan(y), nan)
+        assert torch.equal(y.masked_fill(nan, 0).view(torch.int16), want.masked_fill(nan, 0).view(torch.int16)), start
+
+
 def test_bf16_weight_module_and_errors():
     import tpp_pytorch_extension  # noqa: F401
     from tpp_pytorch_extension.llm.llm_common import FixLinear, BlockedLinear

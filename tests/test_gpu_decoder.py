@@ -210,13 +210,13 @@ def _attn_prefill(q, kc, vc, past, mask=None):
 
 @pytest.mark.parametrize("B,S,Nq,Nkv,past,Smax", [(1, 256, 4, 4, 0, 256), (2, 77, 8, 2, 0, 128), (2, 5, 4, 4, 100, 128),
                                                   (1, 130, 2, 1, 63, 256), (3, 1, 4, 2, 40, 64)])
-@pytest.mark.parametrize("queries_per_wave", [16, 32])
-def test_attn_prefill(B, S, Nq, Nkv, past, Smax, queries_per_wave, monkeypatch):
+@pytest.mark.parametrize("queries", [64, 128])  # per workgroup
+def test_attn_prefill(B, S, Nq, Nkv, past, Smax, queries, monkeypatch):
     """Causal attention for S query tokens against the oracle (tolerance as for the single-query kernel: rel-L2
     5e-3, max-abs 2^-7 of the largest output) and against plain PyTorch fp32 causal softmax attention (1e-2), with
     both of the kernel's shapes (the library picks by launch size; the knob forces one)."""
     _llm()
-    monkeypatch.setenv("TPPX_ATTN_QG", str(queries_per_wave // 16))
+    monkeypatch.setenv("TPPX_ATTN_QG", str(queries // 64))
     L = past + S
     q = randn_bf16((B, S, Nq, 128), 1.0, 51)
     k = randn_bf16((B, Nkv, Smax, 128), 1.0, 52)
@@ -241,13 +241,13 @@ def test_attn_prefill(B, S, Nq, Nkv, past, Smax, queries_per_wave, monkeypatch):
 
 
 @pytest.mark.parametrize("rise", [0.5, 7.0, 40.0, -7.0])
-@pytest.mark.parametrize("queries_per_wave", [16, 32])
-def test_attn_prefill_running_maximum(rise, queries_per_wave, monkeypatch):
+@pytest.mark.parametrize("queries", [64, 128])  # per workgroup
+def test_attn_prefill_running_maximum(rise, queries, monkeypatch):
     """Sums are rescaled only in tiles where some query's running maximum moves: scores that rise along the keys by less and by
     more than a binade per key tile, and that fall, over grouped heads, one query of a workgroup far above the others, against
     softmax attention in float64 (probabilities and outputs rounded to bf16: 2^-8 each)."""
     _llm()
-    monkeypatch.setenv("TPPX_ATTN_QG", str(queries_per_wave // 16))
+    monkeypatch.setenv("TPPX_ATTN_QG", str(queries // 64))
     S, Nq, Nkv = 330, 6, 2
     q, v = randn_bf16((1, S, Nq, 128), 0.3, 66), randn_bf16((1, Nkv, 384, 128), 1.0, 67)
     k = randn_bf16((1, Nkv, 384, 128), 0.3, 68)
@@ -280,13 +280,13 @@ def test_attn_prefill_full_size_rows_equal_single_query_problem():
         assert np.abs(g - r).max() <= 2.0 ** -7 * np.abs(r).max(), i
 
 
-@pytest.mark.parametrize("S,Nq,queries_per_wave", [(600, 32, 16), (1100, 32, 32), (700, 48, 16)])
-def test_attn_prefill_more_than_256_workgroups(S, Nq, queries_per_wave, monkeypatch):
+@pytest.mark.parametrize("S,Nq,queries", [(600, 32, 64), (1100, 32, 128), (700, 48, 64)])
+def test_attn_prefill_more_than_256_workgroups(S, Nq, queries, monkeypatch):
     """Launches of more than 256 workgroups whose query blocks per head do not divide 256 (the heads of every other
     run of 256 workgroups walk their blocks in the other order; a run boundary inside a head must not change that
     head's order): EVERY row against plain PyTorch fp32 causal attention."""
     _llm()
-    monkeypatch.setenv("TPPX_ATTN_QG", str(queries_per_wave // 16))
+    monkeypatch.setenv("TPPX_ATTN_QG", str(queries // 64))
     q = randn_bf16((1, S, Nq, 128), 1.0, 61)
     k = randn_bf16((1, Nq, S, 128), 1.0, 62)
     v = randn_bf16((1, Nq, S, 128), 1.0, 63)
@@ -299,10 +299,10 @@ def test_attn_prefill_more_than_256_workgroups(S, Nq, queries_per_wave, monkeypa
     assert float(err.max()) <= 2e-2, (int(err.argmax()), float(err.max()))
 
 
-@pytest.mark.parametrize("queries_per_wave", [16, 32])
-def test_attn_prefill_mask_and_errors(queries_per_wave, monkeypatch):
+@pytest.mark.parametrize("queries", [64, 128])  # per workgroup
+def test_attn_prefill_mask_and_errors(queries, monkeypatch):
     F = _llm()
-    monkeypatch.setenv("TPPX_ATTN_QG", str(queries_per_wave // 16))
+    monkeypatch.setenv("TPPX_ATTN_QG", str(queries // 64))
     from tpp_pytorch_extension._lib import TppxError
     B, S, Nq, Smax = 2, 70, 4, 128
     q = randn_bf16((B, S, Nq, 128), 1.0, 61)

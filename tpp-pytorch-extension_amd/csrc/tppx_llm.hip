@@ -866,7 +866,9 @@ constexpr int AP_VP = 68; // LDS row pitch of the hd kernel's V^T tile (64 keys 
 // What bounds it is the chain scores -> softmax -> output of a wave, not one unit (MFMA a third busy, vector issue a half), so
 // waves per SIMD count more than operand reads per MFMA (32 queries per wave, half the reads: 57 us where 16 took 50).  The
 // tile's maximum is taken across lanes and the sums are rescaled only where some query's running maximum moves, everything
-// else being a factor of exactly 1: the bits of doing it in every tile.
+// else being a factor of exactly 1: the bits of doing it in every tile.  Two links of that chain stand still: the 16 operand
+// reads of 32 keys' V are waited for as they are issued, twice per tile (124 of 128 registers are taken, none are left to read
+// ahead), and with a mask its values, requested behind the next tile, arrive behind it.
 // Measured against registers in between, V transposed by byte permutes and a rescaling per tile: 2048 tokens x 32 heads
 // 74 -> 57.5 us, 64 heads on 8 of K/V 152 -> 88, 1000 x 32 28 -> 22.3, 333 x 32 12.6 -> 9.9, 3 x 600 behind 500 with a mask 107
 // -> 48.5 (the mask was read under a branch per key).

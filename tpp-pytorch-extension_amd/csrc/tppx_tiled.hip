@@ -1224,6 +1224,8 @@ __device__ __forceinline__ void ring_gemm_body(const BigParams& P) {
 }
 
 constexpr int RING_STAGES = 3;
+// MT = 2: 64 x 128, waves side by side (named, as in big_bf16_kernel, by the workgroup tile MT*16*WM rows x WN*64 channels and
+// the threads; its waves do not stand 2 x 2); MT = 4: the ring; MT = 8: the large tiles
 template <int MT, bool DUAL, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
 big_mxfp4_kernel(const BigParams P) {
@@ -1477,7 +1479,6 @@ big_qint8_narrow_dual_kernel(const BigParams P) {
   big_qint8_body<4, 4, true>(P);
 }
 
-// the large-M kernel addresses its operands with 32-bit byte offsets
 // ---------------------------------------------------------------------------
 // Large-M MXFP4 weights x MXFP8 activations on the block-scaled MFMA
 // (v_mfma_scale_f32_16x16x128_f8f6f4): the weights' E2M1 codes and E8M0 scales

@@ -253,7 +253,7 @@ static bool mxfp4_nk_fits(int64_t M, int total_tiles, int units, int64_t ws_byte
 
 // MXFP4 (dual: `tiles` of each projection).  Fitted to 2800 launches of the decode kernels at 65 .. 1024 rows with weights that
 // come from memory, most of all to those that take about as long as the tiles.  On 2000 launches of other shapes the family and
-// tile taken are 0.14 % off the fastest on average and 7 % in the worst hundredth (fitted to the decode kernels before their
+// tile taken are 0.13 % off the fastest on average and 6 % in the worst hundredth (fitted to the decode kernels before their
 // activations went straight to LDS: 1.3 % and 30 %, a 128-row q/k/v of 3 x 4096 x 4096 at 34.6 us where the tiles take 18.6).
 static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, bool dual, bool nk, int64_t ws_bytes) {
   const int family = kernel_family(M, flags);
@@ -267,9 +267,9 @@ static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, boo
     return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
            (double)rows64 * (8.0 + (double)n_tiles16 * 16.0 * (double)K * (0.5 + 1.0 / 32) / 5.5e6 + (double)K * 0.0008);
   }
-  static constexpr RowsCost SINGLE[3] = {{3.13, 0.665, 0.939, 0.75}, {2.73, 1.78, 1.08, 0.939}, {2.3, 3.16, 1.58, 0.616}};
+  static constexpr RowsCost SINGLE[3] = {{3.19, 0.678, 0.958, 0.765}, {2.78, 1.82, 1.10, 0.958}, {2.35, 3.22, 1.61, 0.628}};
   static constexpr RowsCost DUAL[3] = {{2.82, 1.16, 1.14, 0.883}, {2.92, 3.4, 1.51, 0.984}, {2.42, 5.0, 2.31, 1.02}};
-  static constexpr RowsCost NK = {3.18, 6.73, 0.392, 0.326};
+  static constexpr RowsCost NK = {3.24, 6.86, 0.400, 0.333};
   const double tiled = tiled_mxfp4_us(M, K, n_tiles16);
   if (nk && mxfp4_nk_fits(M, (int)tiles, (int)(K / 128), ws_bytes))
     return tiled <= rows_us(NK, (tiles + 3) / 4 * 4 * rows64, M, K);

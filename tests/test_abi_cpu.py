@@ -339,6 +339,7 @@ def test_kernel_family_of_short_prompts():
 
     # 64 x 128 workgroups in whole columns per XCD drift apart from 21 row blocks on, also with an even number of them
     assert "<2, false, 2, 2>" not in one(2048, 9088, 8704) and "<2, false, 2, 2>" not in one(1744, 6528, 10496)  # 250 us (342), 183 (251)
+    assert "<2, false, 2, 2>" not in one(1421, 4096, 11008) and "<2, false, 2, 2>" in one(1421, 4096, 4096)      # 111 us (125), 44 (50)
     assert "<2, false, 2, 2>" not in qkv(2048, 1856, 13312) and "<2, true, 2, 2>" not in pair(2048, 2880, 7168)   # 230 us (339), 134 (180)
     assert "<2, false, 2, 2>" in one(2048, 4800, 4096)                                              # rectangles: 63 us (74)
 

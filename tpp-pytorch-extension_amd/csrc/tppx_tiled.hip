@@ -1751,16 +1751,17 @@ constexpr double MXFP4_WEIGHT_BYTES = 0.53;
 static double mxfp4_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb, bool dual) {
   const int64_t mb = (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile];
   const double us = tile_us(MXFP4_COST[tile], tile, mb * nb, s, weight_mb, dual);
-  // Without a split along M an XCD walks whole columns, and from 21 row blocks of 64 on the columns of the workgroups that are
-  // resident together drift apart in K: 3 % more for each, 24 row blocks 10 % (K = 4096) .. 21 % (K = 16384), 29 25 .. 33 %, 32
-  // 31 .. 37 % (from K = 2560 on; 12 % at 32 row blocks of K = 1536).  With rectangles (an even number of row blocks and channel
+  // Without a split along M an XCD walks whole columns, and the columns of the workgroups that are resident together drift apart
+  // in K, the more so the more row blocks there are and the longer K is: 24 row blocks cost 10 % (K = 4096) .. 21 % (K = 16384),
+  // 29 25 .. 33 %, 32 31 .. 37 %, K up to 2048 half of that and less.  With rectangles (an even number of row blocks and channel
   // blocks to go with it) 32 row blocks are as fast as the estimate, and launches of up to 768 workgroups, three to a CU and so
-  // all of them resident, lose 5 .. 10 % less.  2048 x 9088 x 8704 342 us where 128 x 256 takes 250.
-  if (tile != TILE_64_128 || mb <= 20 || mb * nb <= 256 ||
+  // all of them resident, lose 5 .. 10 % less.  2048 x 9088 x 8704 342 us where 128 x 256 takes 250, 4096 x 11008 at 1421 rows
+  // 125 (111).  On 2600 launches of 1025 .. 2048 rows the tile taken is 0.3 % off the fastest on average.
+  if (tile != TILE_64_128 || mb <= 16 || mb * nb <= 256 ||
       xcd_split(mb, nb, (double)M * 2.0, (double)nb * TILE_COLS16[tile] * 16.0 * MXFP4_WEIGHT_BYTES) != 1)
     return us;
-  return us * (1.0 + std::min(0.36, 0.03 * (double)(mb - 21) + 0.0007 * s) * std::min(1.0, std::max(0.0, (s - 8.0) / 12.0)) *
-                         std::min(1.0, (double)(mb * nb + 256) / 1024.0));
+  const double drift = std::max(0.0, std::min(0.4, 0.025 * (double)(mb - 21) + 0.0014 * s));
+  return us * (1.0 + drift * std::min(1.0, std::max(0.0, (s - 8.0) / 12.0)) * std::min(1.0, (double)(mb * nb + 256) / 1024.0));
 }
 static double bf16_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb, bool dual) {
   return tile_us(BF16_COST[tile], tile, (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile] * nb, s, weight_mb, dual);

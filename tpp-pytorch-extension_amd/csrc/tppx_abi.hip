@@ -309,7 +309,8 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
 
 // Unquantized bf16 weights: n of them as one launch of the large-M kernel against one decode launch each.  Both sides fitted with
 // weights that come from memory: 2304 x 10496 at 82 rows 39 us on the decode kernels (tiles 55), 1024 x 5120 twice at 160 rows 25
-// as two decode launches (one of the tiles 29), 4096 x 4096 at 128 rows 23 (27), at 200 rows 41 (24).
+// as two decode launches (one of the tiles 29), 4096 x 4096 at 128 rows 22 (27), at 200 rows 41 (24).  (With the weights at hand in
+// the Infinity Cache the tiles take 18 at 128 rows, the decode kernels 21; those of a model are not.)
 static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tiles, int n) {
   const int family = kernel_family(M, flags);
   if (family != BY_COST)

@@ -293,13 +293,14 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
     if (dual || rows64 * ((tiles + 15) / 16) >= 128 || (K <= 1024 && rows64 > 2))
       return true;
     // Fewer run as 64 x 128, in one round, against the decode kernels' rounds; both sides in us with weights that come from
-    // memory, the quantizer included.  On 1260 launches of other shapes the choice is 0.04 % off the faster one on average, 1 % in
-    // the worst hundredth (fitted to four weights in turn, which mostly lie in the Infinity Cache: 0.35 % and 15 %).
+    // memory, the quantizer included, near ties to the tiles (which gain more from weights at hand in the Infinity Cache: 3008 x
+    // 5120 at 117 rows 23.4 and 23.1 us, then 19.1 and 22.4).  On 1260 launches of other shapes the choice is 0.04 % off the faster
+    // one on average, 1 % in the worst hundredth (fitted to four weights in turn, mostly at hand: 0.35 % and 15 %).
     const int nt = tiles < 512 ? 1 : tiles > 512 && tiles <= 768 ? 3 : 2; // as plan_skinny
     const double k = 1e-3 * (double)K, wgs = (double)(rows64 * ((tiles + 7) / 8)), mk = 1e-6 * (double)M * (double)K;
     static constexpr RowsCost ROWS[3] = {{5.06, 2.34, 1.30, 0}, {4.9, 3.96, 1.6, 0}, {5.5, 4.25, 2.3, 0}};
     return 6.07 + k * (3.01 + 0.668 * wgs / 256.0) + 0.257 * mk <=
-           rows_us(ROWS[nt - 1], (tiles + nt - 1) / nt * rows64, M, K) + (nt == 1 ? 0.1 : 0.8) * mk;
+           1.04 * (rows_us(ROWS[nt - 1], (tiles + nt - 1) / nt * rows64, M, K) + (nt == 1 ? 0.1 : 0.8) * mk);
   }
   const int64_t wgs = ((M + 127) / 128) * ((tiles + 15) / 16);
   const bool small = wgs <= 128 && env_int("TPPX_TILED_SMALL", 1) != 0;
@@ -309,8 +310,9 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
 
 // Unquantized bf16 weights: n of them as one launch of the large-M kernel against one decode launch each.  Both sides fitted with
 // weights that come from memory: 2304 x 10496 at 82 rows 39 us on the decode kernels (tiles 55), 1024 x 5120 twice at 160 rows 25
-// as two decode launches (one of the tiles 29), 4096 x 4096 at 128 rows 22 (27), at 200 rows 41 (24).  (With the weights at hand in
-// the Infinity Cache the tiles take 18 at 128 rows, the decode kernels 21; those of a model are not.)
+// as two decode launches (one of the tiles 29), 4096 x 4096 at 128 rows 22 (27), at 200 rows 41 (24).  A near tie goes to the tiles:
+// with weights at hand in the Infinity Cache, as those of one small layer or of a linear called again, they take up to a quarter
+// less (4096 x 4096 at 128 rows 18), the decode kernels hardly (21).
 static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tiles, int n) {
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
@@ -325,7 +327,7 @@ static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tile
     all += tiles[i];
   }
   if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
-    return tiled_bf16_us(M, K, all) <= rows;
+    return tiled_bf16_us(M, K, all) <= 1.04 * rows;
   const int64_t wgs = ((M + 127) / 128) * ((all + 7) / 8); // tiled_bf16_kernel
   return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
          (double)rows64 * (8.0 + (double)all * 32.0 * (double)K / 5.5e6 + (double)K * 0.0008);

@@ -120,7 +120,8 @@ def test_attn_decode_split_merge_in_launch_equals_second_kernel(monkeypatch):
 
 @pytest.mark.parametrize("kernel", ["rows", "wide"])
 @pytest.mark.parametrize("B,Nq,Nkv,L0,Smax,B_pos", [(1, 32, 32, 2048, 2304, 1), (3, 8, 2, 300, 512, 3), (2, 4, 4, 0, 64, 1),
-                                                     (16, 32, 32, 77, 128, 16), (1, 8, 8, 255, 256, 1), (2, 4, 2, 128, 512, 2)])
+                                                     (16, 32, 32, 77, 128, 16), (1, 8, 8, 255, 256, 1), (2, 4, 2, 128, 512, 2),
+                                                     (2, 28, 4, 95, 96, 2), (1, 40, 2, 1023, 1100, 1)])
 def test_attn_decode_with_rotary_and_append_in_the_launch(B, Nq, Nkv, L0, Smax, B_pos, kernel, monkeypatch):
     monkeypatch.setenv("TPPX_ATTN_WIDE", "1" if kernel == "wide" else "0")
     """tppx_attn_decode_rotary = tppx_rotary_kv_append_llama + tppx_attn_decode(kv_len_add = 1) in one launch: same
@@ -194,6 +195,36 @@ def test_attn_decode_mask(kernel, monkeypatch):
     g, r = bits2f(t2bits(got)).astype(np.float64), bits2f(ref).astype(np.float64)
     assert np.isfinite(g).all()
     assert np.sqrt(((g - r) ** 2).sum() / (r ** 2).sum()) <= 5e-3
+
+
+@pytest.mark.parametrize("Nq,Nkv", [(4, 2), (28, 4), (16, 2), (32, 2), (34, 2), (80, 4)])
+@pytest.mark.parametrize("B,L,Smax", [(1, 1, 1), (2, 31, 33), (1, 64, 64), (3, 65, 100), (1, 700, 900), (2, 2081, 2200), (48, 150, 160)])
+def test_attn_decode_grouped_heads(B, L, Smax, Nq, Nkv, monkeypatch):
+    """Query heads that share a K/V head, one workgroup for up to 16 of them (2, 7, 8, 16, 17, 20 here): lengths around the
+    tiles of 32 keys and the trips of 64, one split and many, with NaN behind the length and a mask shorter than it; the
+    in-launch merge gives the bits of the second kernel.  Bounds as for the kernels of one head."""
+    F = _llm()
+    q = randn_bf16((B, Nq, 128), 1.0, 131)
+    k = randn_bf16((B, Nkv, Smax, 128), 1.0, 132)
+    v = randn_bf16((B, Nkv, Smax, 128), 1.0, 133)
+    k[:, :, L:] = float("nan")
+    v[:, :, L:] = float("nan")
+    mask = torch.zeros((B, max(1, L - 3)), dtype=torch.bfloat16)
+    mask[:, : L // 3] = -10000.0
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    for m in (None, mask):
+        ref = bits2f(O.attn_decode(t2bits(q), t2bits(k[:, :, :L]), t2bits(v[:, :, :L]),
+                                   None if m is None else torch.nn.functional.pad(m, (0, L - m.shape[1])).float().numpy())).astype(np.float64)
+        outs = [_attn(F, qd, kd, vd, L, mask=None if m is None else m.cuda(), ws=ws) for ws in (True, True, False)]
+        monkeypatch.setenv("TPPX_ATTN_ONE_LAUNCH", "0")
+        outs.append(_attn(F, qd, kd, vd, L, mask=None if m is None else m.cuda()))
+        monkeypatch.delenv("TPPX_ATTN_ONE_LAUNCH")
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[3])
+        for o in outs:
+            got = bits2f(t2bits(o)).astype(np.float64)
+            assert np.isfinite(got).all()
+            assert np.sqrt(((got - ref) ** 2).sum() / (ref ** 2).sum()) <= 5e-3
+            assert np.abs(got - ref).max() <= 2.0 ** -7 * np.abs(ref).max()
 
 
 def _attn_prefill(q, kc, vc, past, mask=None):

@@ -1078,6 +1078,377 @@ attn_prefill_kernel(const AttnPrefillParams p) {
 }
 
 // ---------------------------------------------------------------------------
+// Single-query attention where several query heads share a K/V head (grouped-query attention), head size 128: a workgroup
+// per (sequence, K/V head, up to 16 of its query heads, split of the keys).  The query heads are the columns of the MFMA
+// operand that the prompt kernel above fills with queries, so a key row is read once for all of them.
+// What bounds it is the cache stream.  A wave works by itself on tiles of 32 keys (8 KiB of K and of V, in two stages of its
+// own LDS, brought by loads straight into LDS; no barrier in the loop), the first one requested before the length is known;
+// 2 waves = 64 KiB, so that two workgroups of a CU have 64 to 128 KiB under way.  Scores, maximum, probabilities and sums as in
+// attn_decode_wide_kernel; the waves and then the splits are merged in order, the latter by the last to arrive.
+// Against a workgroup per query head (attn_decode_wide_kernel), which reads every row Nq / Nkv times through the L2s and does
+// its arithmetic on the vector units each time, us per launch: 28 heads on 4 of K/V, 16 sequences of 2500 keys 101 -> 20.6,
+// 48 of 1500 169 -> 32.7, 4 of 2000 27.6 -> 10.4, 1 of 4000 15.7 -> 11.8, 1 of 100 6.9 -> 6.3; 64 heads on 8, 16 of 2048
+// 164 -> 28.7; 32 on 16, 16 of 1000 44 -> 26.4 (5 TB/s of cache).  With a head per K/V head the other kernel is the faster one
+// from some 30 MB of cache on (32 heads, 16 of 2048 87 against 96 us: more waves with requests of their own).
+// ---------------------------------------------------------------------------
+constexpr int AG_WAVES = 2, AG_KEYS = 32 * AG_WAVES; // keys per workgroup and trip
+
+// the K operands of 32 keys (2 runs of 16 keys x 4 steps of 32 dims), issued and waited for in one block
+template <int OFF>
+__device__ __forceinline__ void read_k_operands(i32x4 (&k)[2][4], const uint32_t (&a)[4]) {
+  asm volatile("ds_read_b128 %0, %8 offset:%12\n\tds_read_b128 %1, %9 offset:%12\n\t"
+               "ds_read_b128 %2, %10 offset:%12\n\tds_read_b128 %3, %11 offset:%12\n\t"
+               "ds_read_b128 %4, %8 offset:%13\n\tds_read_b128 %5, %9 offset:%13\n\t"
+               "ds_read_b128 %6, %10 offset:%13\n\tds_read_b128 %7, %11 offset:%13\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(k[0][0]), "=&v"(k[0][1]), "=&v"(k[0][2]), "=&v"(k[0][3]), "=&v"(k[1][0]), "=&v"(k[1][1]), "=&v"(k[1][2]), "=&v"(k[1][3])
+               : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "n"(OFF), "n"(OFF + 4096)
+               : "memory");
+}
+
+template <bool ROT>
+__global__ void __launch_bounds__(AG_WAVES * 64, 1)
+attn_decode_group_kernel(const AttnParams p) {
+  constexpr int STAGE = 16384, WAVE_LDS = 2 * STAGE; // per stage: K [32 keys][256 B] | V [32 keys][256 B]
+  constexpr int OP = 132;                            // pitch of a merged output row in floats
+  __shared__ __align__(16) uint8_t lds[AG_WAVES * WAVE_LDS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  const int G = p.Nq / p.Nkv, blocks = (G + 15) >> 4; // query heads of a K/V head, workgroups they take
+  const int gb = (int)blockIdx.x % blocks, bkv = (int)blockIdx.x / blocks, b = bkv / p.Nkv, hk = bkv - b * p.Nkv;
+  const int heads = min(16, G - gb * 16);             // of this workgroup
+  const int head0 = b * p.Nq + hk * G + gb * 16;      // the first of them
+  const int S = p.splits;
+
+  // rows past the cache's end repeat its last one; rows past the length are masked below
+  auto request = [&](int base, int stage) {
+    const int first = min(base, p.Smax - 1), rows = p.Smax - 1 - first;
+    const int64_t at = ((int64_t)bkv * p.Smax + first) * 128;
+    const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.kc + at), 0, 0xffffffffu, 0x00020000);
+    const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.vc + at), 0, 0xffffffffu, 0x00020000);
+    uint8_t* const dst = lds + wave * WAVE_LDS + stage * STAGE;
+#pragma unroll
+    for (int pc = 0; pc < 8; pc++) // pieces of 4 rows x 256 B
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (__attribute__((address_space(3))) void*)(dst + pc * 1024), 16,
+                                               (uint32_t)min(pc * 4 + g, rows) * 256u + (uint32_t)(c ^ ((pc & 3) * 4 + g)) * 16u, 0, 0, 0);
+#pragma unroll
+    for (int pc = 0; pc < 8; pc++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (__attribute__((address_space(3))) void*)(dst + 8192 + pc * 1024), 16,
+                                               (uint32_t)min(pc * 4 + g, rows) * 256u + (uint32_t)(c ^ (((pc & 1) * 4 + g) * 2)) * 16u, 0, 0, 0);
+  };
+  // the query: head c, dims j * 32 + g * 8 .. + 7 (columns past the heads repeat the last one, never stored)
+  i32x4 qw[4];
+  {
+    const uint16_t* qrow = p.q + (int64_t)(head0 + min(c, heads - 1)) * 128 + g * 8;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      qw[j] = *reinterpret_cast<const i32x4*>(qrow + j * 32);
+  }
+  const int64_t pp = ROT ? p.pos[p.B_pos == 1 ? 0 : b] : 0;
+  const bool rot = ROT && p.emb != nullptr && pp >= 0 && pp < p.MP; // positions outside the table are left unrotated
+  if (rot) { // rotation pairs (i, 64 + i): operands j and j + 2 of the same lane
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const f32x4* cp = reinterpret_cast<const f32x4*>(p.emb + pp * 128 + j * 32 + g * 8);
+      const f32x4* sp = reinterpret_cast<const f32x4*>(p.emb + ((int64_t)p.MP + pp) * 128 + j * 32 + g * 8);
+      const f32x4 cs[2] = {cp[0], cp[1]}, sn[2] = {sp[0], sp[1]};
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        uint32_t lo[2], hi[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          const float x1 = bf16_bits_to_f32(((uint32_t)qw[j][d] >> (16 * e)) & 0xffffu);
+          const float x2 = bf16_bits_to_f32(((uint32_t)qw[j + 2][d] >> (16 * e)) & 0xffffu);
+          const float cv = cs[d >> 1][(d & 1) * 2 + e], sv = sn[d >> 1][(d & 1) * 2 + e];
+          lo[e] = f32_to_bf16_bits(x1 * cv - x2 * sv);
+          hi[e] = f32_to_bf16_bits(x2 * cv + x1 * sv);
+        }
+        qw[j][d] = (int)(lo[0] | lo[1] << 16);
+        qw[j + 2][d] = (int)(hi[0] | hi[1] << 16);
+      }
+    }
+  }
+  request(blockIdx.y * AG_KEYS + wave * 32, 0);
+  const int len0 = *p.kv_len;
+  const int L = max(0, min(len0 + p.kv_len_add, p.Smax));
+  const int nk = (ROT && len0 >= 0 && len0 < p.Smax) ? len0 : -1; // cache position of the new token
+  const int trips = (L + AG_KEYS - 1) / AG_KEYS;
+  const uint16_t* mrow = p.mask ? p.mask + (int64_t)b * p.mask_ld : nullptr;
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + wave * WAVE_LDS;
+  uint32_t kaddr[4], vaddr[8]; // this lane's operands inside a stage: K chunk j * 4 + g of row c; V dims dt * 16 .. + 15
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    kaddr[j] = lds0 + (uint32_t)(c * 256 + (((j * 4 + g) ^ c) & 15) * 16);
+  {
+    const int r = g * 4 + (c >> 2); // key of this lane's 8 bytes inside a run of 16
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++)
+      vaddr[dt] = lds0 + (uint32_t)(r * 256 + ((dt * 2 + ((c >> 1) & 1)) ^ ((r & 7) * 2)) * 16 + (c & 1) * 8);
+  }
+  float m = -3.0e38f, l = 0.f;
+  f32x4 acc[8];
+#pragma unroll
+  for (int dt = 0; dt < 8; dt++)
+    acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto tile = [&](auto STAGE_, int base, bool more) {
+    constexpr int stage = decltype(STAGE_)::value;
+    if (more) // the next tile's 16 loads stay under way
+      asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (ROT && nk >= base && nk < base + 32) {
+      // the new token is not in the cache yet: its row of the tile becomes the rotated key (lane i: pair (i, 64 + i)) and the
+      // step's value; one workgroup per K/V head writes both into the cache
+      uint8_t* const st = lds + wave * WAVE_LDS + stage * STAGE;
+      const int r = nk - base;
+      const uint16_t* krow = p.k_new + (int64_t)bkv * 128;
+      const uint16_t* vrow = p.v_new + (int64_t)bkv * 128;
+      const float x1 = bf16_bits_to_f32(krow[lane]), x2 = bf16_bits_to_f32(krow[64 + lane]);
+      const float cv = rot ? p.emb[pp * 128 + lane] : 1.f, sv = rot ? p.emb[((int64_t)p.MP + pp) * 128 + lane] : 0.f;
+      const uint16_t k1 = (uint16_t)f32_to_bf16_bits(rot ? x1 * cv - x2 * sv : x1), k2 = (uint16_t)f32_to_bf16_bits(rot ? x2 * cv + x1 * sv : x2);
+      const i32x4 vn = *reinterpret_cast<const i32x4*>(vrow + c * 8);
+      uint16_t* const kt = reinterpret_cast<uint16_t*>(st + r * 256);
+      kt[((lane >> 3) ^ (r & 15)) * 8 + (lane & 7)] = k1;
+      kt[((8 + (lane >> 3)) ^ (r & 15)) * 8 + (lane & 7)] = k2;
+      if (g == 0)
+        *reinterpret_cast<i32x4*>(st + 8192 + r * 256 + (c ^ ((r & 7) * 2)) * 16) = vn;
+      if (gb == 0) {
+        const int64_t o = ((int64_t)bkv * p.Smax + nk) * 128;
+        uint16_t* const kd = const_cast<uint16_t*>(p.kc) + o;
+        kd[lane] = k1;
+        kd[64 + lane] = k2;
+        if (g == 0)
+          *reinterpret_cast<i32x4*>(const_cast<uint16_t*>(p.vc) + o + c * 8) = vn;
+      }
+      // (the builtin, so that the compiler knows these loads done: it would wait for the next tile at the join otherwise)
+      __builtin_amdgcn_s_waitcnt(0x0070); // vmcnt(0) lgkmcnt(0)
+      asm volatile("" ::: "memory");
+    }
+    f32x4 sc[2];
+    {
+      i32x4 kw[2][4];
+      read_k_operands<stage * STAGE>(kw, kaddr);
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        sc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kw[t][j]), __builtin_bit_cast(bf16x8, qw[j]), sc[t], 0, 0, 0);
+      }
+    }
+    const bool tail = base + 32 > L; // wave-uniform
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      sc[i >> 2][i & 3] = scaled(sc[i >> 2][i & 3], p.scale);
+    if (mrow) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int key = base + (i >> 2) * 16 + g * 4 + (i & 3);
+        const float mv = bf16_bits_to_f32(mrow[min(key, p.mask_ld - 1)]); // (no branch per key)
+        sc[i >> 2][i & 3] += key < p.mask_ld ? mv : 0.f;
+      }
+    }
+    if (tail) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) // past the end: -inf, whose exponential is exactly 0 against the finite maximum
+        sc[i >> 2][i & 3] = base + (i >> 2) * 16 + g * 4 + (i & 3) < L ? sc[i >> 2][i & 3] : -INFINITY;
+    }
+    float mx = m;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      mx = fmaxf(mx, sc[i >> 2][i & 3]);
+    if (__builtin_amdgcn_ballot_w64(mx > m) != 0) { // some head's maximum moves
+      mx = max_of_groups(mx);
+      const float alpha = __expf(m - mx);
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 8; dt++)
+        acc[dt] *= alpha;
+      m = mx;
+    }
+    bf16x8 pb;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float pr = __expf(sc[i >> 2][i & 3] - m);
+      l += pr;
+      pb[i] = (__bf16)pr;
+    }
+    // K slots g*8 .. +7 of the operand = keys g*4 .. +3 and 16 + g*4 .. +3, the keys pb holds in the same slots
+    i32x2 vv[8][2];
+    read_v_operands<stage * STAGE + 8192>(vv, vaddr);
+    if (tail) { // rows past the end may hold anything, NaN included
+      const int left = L - base - g * 4; // keys of this lane's first run that count
+      auto keep = [](int n) { return n <= 0 ? 0 : n == 1 ? 0xffff : -1; };
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int k0 = keep(left - h * 16), k1 = keep(left - h * 16 - 2);
+#pragma unroll
+        for (int dt = 0; dt < 8; dt++) {
+          vv[dt][h][0] &= k0;
+          vv[dt][h][1] &= k1;
+        }
+      }
+    }
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++) {
+      const i32x4 av = {vv[dt][0][0], vv[dt][0][1], vv[dt][1][0], vv[dt][1][1]};
+      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), pb, acc[dt], 0, 0, 0);
+    }
+  };
+  // Tiles of this wave: base + i * S * AG_KEYS while they begin before the end of the keys.  While tile i is worked on tile
+  // i + 1 is under way in the other stage; a stage is asked for again once its tile has been read.
+  const int step = S * AG_KEYS;
+  int base = blockIdx.y * AG_KEYS + wave * 32;
+  if (base + step < L)
+    request(base + step, 1);
+  for (; base < L; base += 2 * step) {
+    tile(std::integral_constant<int, 0>{}, base, base + step < L);
+    if (base + 2 * step < L)
+      request(base + 2 * step, 0);
+    if (base + step < L) {
+      tile(std::integral_constant<int, 1>{}, base + step, base + 2 * step < L);
+      if (base + 3 * step < L)
+        request(base + 3 * step, 1);
+    }
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+
+  // the waves' states through LDS (every load into it has landed, also a first tile that lies past the keys)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  float* const mo = reinterpret_cast<float*>(lds);           // [wave][head][OP]
+  float* const sm = mo + AG_WAVES * 16 * OP;                 // [wave][head] maximum
+  float* const sl = sm + AG_WAVES * 16;                      // [wave][head] sum
+  float* const sw = sl + AG_WAVES * 16;                      // [head][32] weight of a split
+  float* const sws = sw + 16 * 32;                           // [head][32] its sum
+  int* const arrived_last = reinterpret_cast<int*>(sws + 16 * 32);
+#pragma unroll
+  for (int dt = 0; dt < 8; dt++)
+    *reinterpret_cast<f32x4*>(mo + (wave * 16 + c) * OP + dt * 16 + g * 4) = acc[dt];
+  if (g == 0) {
+    sm[wave * 16 + c] = m;
+    sl[wave * 16 + c] = l;
+  }
+  __syncthreads();
+  float* const part_o = p.part;                                            // [head][split][128]
+  float* const part_ml = p.part + (int64_t)p.B * p.Nq * S * 128;           // [head][split][2]
+  auto store4 = [&](int h, int d4, f32x4 o, float Ls) {
+    uint32_t w[2];
+#pragma unroll
+    for (int e = 0; e < 2; e++)
+      w[e] = f32x2_to_bf16_bits(Ls > 0.f ? o[2 * e] / Ls : 0.f, Ls > 0.f ? o[2 * e + 1] / Ls : 0.f);
+    *reinterpret_cast<uint2*>(p.out + (int64_t)(head0 + h) * 128 + d4 * 4) = make_uint2(w[0], w[1]);
+  };
+  for (int i = tid; i < heads * 32; i += AG_WAVES * 64) {
+    const int h = i >> 5, d4 = i & 31;
+    float M = sm[h];
+#pragma unroll
+    for (int w = 1; w < AG_WAVES; w++)
+      M = fmaxf(M, sm[w * 16 + h]);
+    float Ls = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < AG_WAVES; w++) {
+      const float wt = __expf(sm[w * 16 + h] - M);
+      Ls = fmaf(wt, sl[w * 16 + h], Ls);
+      const f32x4 ow = *reinterpret_cast<const f32x4*>(mo + (w * 16 + h) * OP + d4 * 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        o[e] = fmaf(wt, ow[e], o[e]);
+    }
+    if (S == 1) {
+      store4(h, d4, o, Ls);
+      continue;
+    }
+    if (p.ticket0 < 0) { // attn_combine_kernel follows
+      float* const dst = p.part + ((int64_t)(head0 + h) * S + blockIdx.y) * 130;
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        dst[2 + d4 * 4 + e] = o[e];
+      if (d4 == 0) {
+        dst[0] = M;
+        dst[1] = Ls;
+      }
+      continue;
+    }
+    // device-scope stores: written through to the level all XCDs share
+    const int64_t at = (int64_t)(head0 + h) * S + blockIdx.y;
+    uint64_t* const dst = reinterpret_cast<uint64_t*>(part_o + at * 128 + d4 * 4);
+    __hip_atomic_store(dst, __builtin_bit_cast(uint64_t, make_float2(o[0], o[1])), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(dst + 1, __builtin_bit_cast(uint64_t, make_float2(o[2], o[3])), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (d4 == 0)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(part_ml + at * 2), __builtin_bit_cast(uint64_t, make_float2(M, Ls)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (S == 1 || p.ticket0 < 0)
+    return;
+  // The split that arrives last merges all of them, in split order; the ordering argument is attn_finish's: own stores
+  // acknowledged, barrier, ticket, device-scope loads.  Nobody waits for anybody.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const unsigned int last = (unsigned int)S - 1;
+    *arrived_last = atomicInc(&attn_tickets[(p.ticket0 + (int)blockIdx.x) * ATTN_TICKET_STRIDE], last) == last;
+  }
+  __syncthreads();
+  if (!*arrived_last)
+    return;
+  auto load2 = [](const float* src) {
+    return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t*>(src), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  };
+  // 16 lanes per head: every lane two splits at most
+  for (int i = tid; i < heads * 16; i += AG_WAVES * 64) {
+    const int h = i >> 4, s0 = i & 15;
+    float2 ml[2] = {{-3.0e38f, 0.f}, {-3.0e38f, 0.f}};
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+      if (s0 + 16 * u < S)
+        ml[u] = load2(part_ml + ((int64_t)(head0 + h) * S + s0 + 16 * u) * 2);
+    float M = fmaxf(ml[0].x, ml[1].x);
+    M = fmaxf(M, dpp_mov<0xB1>(M));
+    M = fmaxf(M, dpp_mov<0x4E>(M));
+    M = fmaxf(M, dpp_mov<0x141>(M));
+    M = fmaxf(M, dpp_mov<0x140>(M));
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      sw[h * 32 + s0 + 16 * u] = __expf(ml[u].x - M);
+      sws[h * 32 + s0 + 16 * u] = ml[u].y;
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < heads * 32; i += AG_WAVES * 64) {
+    const int h = i >> 5, d4 = i & 31;
+    const float* src = part_o + (int64_t)(head0 + h) * S * 128 + d4 * 4;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    float Ls = 0.f;
+    for (int s0 = 0; s0 < S; s0 += 8) { // eight splits' loads in flight
+      float2 a[8][2];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const float* at = src + (int64_t)min(s0 + u, S - 1) * 128;
+        a[u][0] = load2(at);
+        a[u][1] = load2(at + 2);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        if (s0 + u < S) {
+          const float wt = sw[h * 32 + s0 + u];
+          Ls = fmaf(wt, sws[h * 32 + s0 + u], Ls);
+          o[0] = fmaf(wt, a[u][0].x, o[0]);
+          o[1] = fmaf(wt, a[u][0].y, o[1]);
+          o[2] = fmaf(wt, a[u][1].x, o[2]);
+          o[3] = fmaf(wt, a[u][1].y, o[3]);
+        }
+      }
+    }
+    store4(h, d4, o, Ls);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Prompt attention at head sizes other than 128: attn_prefill_kernel with the head size padded to HD = 64, 128 or
 // 256 (H a multiple of 8, H <= HD; dims past H are staged as zeros and not stored), the K tile 64 x (HD + 8) and the
 // V^T tile HD x 68 in dynamic LDS, HD / 32 MFMAs per 16 keys for the scores and HD / 16 output tiles per query group.
@@ -1527,25 +1898,42 @@ static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t 
     splits = max_by_len;
   if (splits > 32)
     splits = 32;
+  const bool one_launch = env_int("TPPX_ATTN_ONE_LAUNCH", 1) != 0;
+  // Several query heads per K/V head: one workgroup for up to 16 of them.  Splits for about one workgroup per CU (16 groups of
+  // 2000 keys: 16 splits 10.4 us, 32 13.2: more states to merge); from 129 groups on as many as two workgroups per CU take
+  // in one round (160 groups of 900 keys: 3 splits 20.4, 2 21.8).  At least a trip each.
+  const int64_t groups = B * p.Nkv * ((Nq / p.Nkv + 15) / 16);
+  int64_t gsplits = target_env > 0 ? (target_env + groups - 1) / groups : groups <= 128 ? (256 + groups - 1) / groups : 500 / groups;
+  gsplits = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(gsplits, 32), (Smax + AG_KEYS - 1) / AG_KEYS));
+  if (gsplits > 1 && (B * Nq * gsplits * 130 * (int64_t)sizeof(float) > ws_bytes || !aligned16(ws)))
+    gsplits = 1;
+  const bool group = wide && Nq > p.Nkv && env_int("TPPX_ATTN_GROUP", 1) != 0;
+  if (group)
+    splits = gsplits;
   const int64_t need = B * Nq * splits * 130 * (int64_t)sizeof(float);
   if (splits > 1 && need > ws_bytes)
     splits = 1; // no room for partial results: one workgroup per head
   p.splits = (int)splits;
   p.part = (float*)ws;
   p.ticket0 = -1;
-  if (splits > 1 && B * Nq <= ATTN_TICKETS && env_int("TPPX_ATTN_ONE_LAUNCH", 1) != 0) {
-    // window of B * Nq arrival counters, handed out in rotation so that split launches in flight on different
+  const int64_t tickets = group ? groups : B * Nq;
+  if (splits > 1 && tickets <= ATTN_TICKETS && one_launch) {
+    // window of arrival counters, handed out in rotation so that split launches in flight on different
     // streams do not share counters
     static std::mutex mu;
     static int cursor = 0;
     std::lock_guard<std::mutex> lock(mu);
-    if (cursor + B * Nq > ATTN_TICKETS)
+    if (cursor + tickets > ATTN_TICKETS)
       cursor = 0;
     p.ticket0 = cursor;
-    cursor += (int)(B * Nq);
+    cursor += (int)tickets;
   }
-  const dim3 grid((unsigned)(B * Nq), (unsigned)splits);
-  if (wide && rot)
+  const dim3 grid((unsigned)(group ? groups : B * Nq), (unsigned)splits);
+  if (group && rot)
+    attn_decode_group_kernel<true><<<grid, dim3(AG_WAVES * 64), 0, stream>>>(p);
+  else if (group)
+    attn_decode_group_kernel<false><<<grid, dim3(AG_WAVES * 64), 0, stream>>>(p);
+  else if (wide && rot)
     attn_decode_wide_kernel<true><<<grid, dim3(256), 0, stream>>>(p);
   else if (wide)
     attn_decode_wide_kernel<false><<<grid, dim3(256), 0, stream>>>(p);
@@ -1556,7 +1944,7 @@ static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t 
   int rc = check_hip(hipGetLastError(), who);
   if (rc && p.ticket0 >= 0) {
     // the refused launch leaves its counter window as it found it, but whoever gets the window next relies on zeros
-    const int n = (int)(B * Nq);
+    const int n = (int)tickets;
     attn_clear_tickets_kernel<<<dim3((n + 255) / 256), dim3(256), 0, stream>>>(p.ticket0, n);
     (void)hipGetLastError();
   }

@@ -597,6 +597,18 @@ int tppx_linear_qint8_f32(const void* xq, const void* sa, const void* qw,
                           int64_t M, int64_t N, int64_t K, int64_t qbs,
                           tppx_stream_t stream);
 
+/* The whole call of that switch: quantizes the rows (x fp32 or fp16 [M][K] as
+ * dtype says, into xq / sa; NULL: xq / sa hold them already), runs the GEMM
+ * above, adds the bias ([N] of bias_dtype, any of the three, or NULL) in fp32,
+ * rounds to dtype and applies the post-op there; post_in / post_in2 and y
+ * [M][N] in dtype. */
+int tppx_linear_qint8_wide(const void* x, int dtype, void* xq, void* sa,
+                           const void* qw, const void* sw, const void* bias,
+                           int bias_dtype, const void* post_in,
+                           const void* post_in2, void* y, int64_t M, int64_t N,
+                           int64_t K, int64_t qbs, int post_op,
+                           float post_scale, tppx_stream_t stream);
+
 /* The same switch for MXFP4 and unquantized bf16 weights:
  * TppBlockedLinearW<Tin, uint8_t, Tout> / <Tin, bfloat16, Tout> with Tin =
  * float or half (src/csrc/fused_gemm.h:1519-1523, 1541-1550; 785-1073).  The
@@ -610,6 +622,15 @@ int tppx_linear_qint8_f32(const void* xq, const void* sa, const void* qw,
 int tppx_linear_wide(const void* x, int x_dtype, const void* w, const void* sw,
                      int w_kind, const void* bias_f32, void* y_f32, int64_t M,
                      int64_t N, int64_t K, tppx_stream_t stream);
+
+/* tppx_linear_wide with the bias in its own type, the rounding to x_dtype and
+ * the post-op in the same launch; post_in / post_in2 and y in x_dtype. */
+int tppx_linear_wide_post(const void* x, int x_dtype, const void* w,
+                          const void* sw, int w_kind, const void* bias,
+                          int bias_dtype, const void* post_in,
+                          const void* post_in2, void* y, int64_t M, int64_t N,
+                          int64_t K, int post_op, float post_scale,
+                          tppx_stream_t stream);
 
 /* Post-ops of call_gemm_with_post_op on a float or half output tile
  * (src/csrc/fused_gemm.h:1343-1488 with Tout = float / half): out[i] =

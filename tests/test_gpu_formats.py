@@ -688,3 +688,82 @@ def test_w4a8_takes_rows_at_any_address(M, off):
     assert torch.equal(ops.linear(xm, qt, moved(b), O.POST_ADD_SCALE, moved(r), None, 0.5),
                        ops.linear(x, qt, b, O.POST_ADD_SCALE, r, None, 0.5))
     assert torch.equal(ops.swiglu_gate_up(xm, qt, qt), ops.swiglu_gate_up(x, qt, qt))
+
+
+# edges of the row and channel tiles (15 / 16 / 17, 32 / 33, 64 / 65 rows; channels that do not fill a workgroup's last
+# tile), enough rows for the whole-chain kernel, and K with fewer blocks than a workgroup has waves
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("M,N,K,qbs", [(16, 112, 256, 256), (17, 48, 1792, 256), (33, 4128, 256, 256), (65, 4112, 512, 256),
+                                       (130, 8224, 1024, 64), (31, 96, 1024, 1024), (200, 4112, 384, 128), (150, 8208, 512, 512)])
+def test_float_and_half_rows_on_qint8_tile_edges(M, N, K, qbs, dtype):
+    """Bit-exact against the oracle's fp32 chain, whichever kernel runs."""
+    ops = _ops()
+    W = randn_bf16((N, K), 0.02, 91)
+    t = W.view(N // 16, 16, K // qbs, qbs // 4, 4).permute(0, 2, 3, 1, 4).contiguous()
+    qw = ops.quantize_int8sym(t.cuda(), qbs, 2, True)
+    q_or, s_or = O.quantize_int8sym(t.float().numpy(), qbs, 2, True)
+    s_or = s_or.reshape(N // 16, K // qbs, 1, 16)
+    g = torch.Generator().manual_seed(92)
+    x = (torch.randn((M, K), generator=g) * 1.7).to(dtype)
+    x[0, :qbs] = 0
+    bias = (torch.randn((N,), generator=g) * 0.1).to(dtype)
+    xq, sa = O.quantize_int8sym(x.float().numpy(), qbs, -1, False)
+    ref = torch.from_numpy(O.linear_qint8_f32(xq, sa, q_or, s_or, bias.float().numpy())).to(dtype)
+    assert torch.equal(ops.fc_plain(x.cuda(), qw, bias.cuda()).cpu(), ref)
+    # rows that do not lie on a 16-byte address
+    off = torch.empty(M * K + 1, dtype=dtype, device="cuda")[1:].view(M, K)
+    off.copy_(x)
+    assert off.data_ptr() % 16 and torch.equal(ops.fc_plain(off, qw, bias.cuda()).cpu(), ref)
+
+
+def test_float_rows_quantizer_on_nan_and_inf():
+    """A NaN in a block's first place sticks in its scale, any other is passed over, as in quantize_int8sym."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    M, N, K = 5, 32, 512
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(3))
+    x[0, 0] = x[1, 7] = x[2, 256] = float("nan")
+    x[3, 9] = float("inf")
+    q = ops.quantize_int8sym(x.cuda(), 256, -1, False)
+    qw = ops.remap_and_quantize_qint8(block_bf16(randn_bf16((N, K), 0.02, 4)).cuda())
+    qn, sn = qw.native()
+    for dtype, dt in ((torch.float32, _lib.DT_F32), (torch.float16, _lib.DT_F16)):
+        xd = x.to(dtype).cuda()
+        q = ops.quantize_int8sym(xd.float(), 256, -1, False)
+        xq = torch.zeros((M, K), dtype=torch.int8, device="cuda")
+        sa = torch.zeros((M, 2), dtype=torch.float32, device="cuda")
+        y = torch.empty((M, N), dtype=dtype, device="cuda")
+        _lib.check(_lib.lib().tppx_linear_qint8_wide(xd.data_ptr(), dt, xq.data_ptr(), sa.data_ptr(), qn.data_ptr(), sn.data_ptr(),
+                                                     None, 0, None, None, y.data_ptr(), M, N, K, 256, 0, 1.0, _lib.stream_of(xd)))
+        assert torch.equal(xq, q.qdata.view(M, K))
+        assert torch.equal(sa.nan_to_num(7.0, 8.0), q.scales.view(M, 2).nan_to_num(7.0, 8.0))
+
+
+@pytest.mark.parametrize("wkind", ["mxfp4", "bf16"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(15, 32, 128), (16, 8224, 256), (17, 96, 1152), (33, 4128, 384), (64, 64, 2304), (130, 8288, 256)])
+def test_float_and_half_activations_in_terms_of_bf16(M, N, K, dtype, wkind):
+    """The terms of an activation add up to it: against a float64 product the float result is within 4 fp32 ulps of
+    sum |x||w| (tests above say why), over 60 binary orders of activations; a row with an infinity, a NaN or the largest
+    float gives what float64 gives."""
+    ops = _ops()
+    W = randn_bf16((N, K), 0.05, 171)
+    g = torch.Generator().manual_seed(172)
+    lo, hi = (-30, 30) if dtype == torch.float32 else (-10, 5)
+    x = (torch.randn((M, K), generator=g) * torch.exp2(torch.randint(lo, hi, (M, 1), generator=g).float())).to(dtype)
+    if wkind == "mxfp4":
+        w = ops.remap_and_quantize_mxfp4(block_bf16(W).cuda())
+        Wd = torch.from_numpy(O.dequantize_mxfp4_plain(*O.remap_quantize_mxfp4(W.float().numpy()))).double()
+    else:
+        w, Wd = block_bf16(W).cuda(), W.double()
+    y = ops.fc_plain(x.cuda(), w, None).cpu().double()
+    ref, mag = x.double() @ Wd.T, x.double().abs() @ Wd.abs().T
+    eps = 2.0 ** -23 if dtype == torch.float32 else 2.0 ** -11
+    assert ((y - ref).abs() <= 4 * 2.0 ** -23 * mag + (eps * ref.abs() + 2.0 ** -25 if dtype == torch.float16 else 0)).all()
+    x[0, 3], x[1, 5], x[2, 7] = float("inf"), float("nan"), torch.finfo(dtype).max
+    y = ops.fc_plain(x.cuda(), w, None).cpu()
+    ref = (x.double() @ Wd.T).to(dtype)
+    assert torch.equal(y[1].isnan(), ref[1].isnan()) and torch.equal(y[0].isnan(), ref[0].isnan())
+    assert torch.equal(y[0].nan_to_num(0.0), ref[0].nan_to_num(0.0))
+    near = 1e-2 if dtype == torch.float16 else 1e-5
+    assert torch.allclose(y[2].double(), ref[2].double(), rtol=near, atol=near * float(ref[2].double().abs()[ref[2].isfinite()].max()), equal_nan=True)

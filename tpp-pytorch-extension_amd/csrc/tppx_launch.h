@@ -130,6 +130,8 @@ inline int big_min_rows() { return env_int("TPPX_TILED_BIG_MIN_M", 65); }
 hipError_t allow_dynamic_lds(const void* kern, size_t lds);
 
 // dynamic activation quantisation; mt > 0 writes xq in MFMA operand order (see DecodeParams::mt)
+hipError_t launch_quant_act_int8_wide(const void* x, int dtype, int64_t M, int64_t K, int64_t qbs, void* xq, void* sa,
+                                      hipStream_t stream);
 hipError_t launch_quant_act_int8(const void* x, int64_t M, int64_t K, int64_t qbs, void* xq, void* sa, int mt,
                                  hipStream_t stream);
 

@@ -617,6 +617,54 @@ quant_act_int8_rows_kernel(const uint16_t* __restrict__ x, int64_t M, int64_t K,
   }
 }
 
+// float / half rows, any block size in 64s: one wave per (row, block), VEC consecutive values per lane and trip (4 where
+// rows lie on 16-byte addresses).  The maximum follows the generic kernel's rule for NaN: |first|, then std::max, so one
+// in the first place sticks and any other is passed over.  Reads the rows twice where a block is longer than
+// 64 * VEC values.  (A thread per block, byte by byte, took 85 us for 2 x 9984 and 116 for 61 x 8704.)
+template <typename T, int VEC>
+__global__ void __launch_bounds__(256)
+quant_act_int8_wide_kernel(const T* __restrict__ x, int64_t blocks, int64_t qbs, int8_t* __restrict__ xq, float* __restrict__ sa) {
+  typedef T tv __attribute__((ext_vector_type(4)));
+  const int64_t blk = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int l = threadIdx.x & 63;
+  if (blk >= blocks) // whole waves
+    return;
+  const T* src = x + blk * qbs; // (m, b) -> m*K + b*qbs = blk*qbs
+  int8_t* dst = xq + blk * qbs;
+  float v[VEC];
+  auto load = [&](int64_t j) {
+    if constexpr (VEC == 4) {
+      const tv t = *reinterpret_cast<const tv*>(src + j);
+      v[0] = (float)t[0]; v[1] = (float)t[1]; v[2] = (float)t[2]; v[3] = (float)t[3];
+    } else {
+      v[0] = (float)src[j];
+    }
+  };
+  float amax = 0.0f;
+  for (int64_t j = (int64_t)l * VEC; j < qbs; j += 64 * VEC) {
+    load(j);
+#pragma unroll
+    for (int i = 0; i < VEC; i++)
+      amax = fmaxf(amax, fabsf(v[i]));
+  }
+  amax = wave_max(amax);
+  const float first = fabsf((float)src[0]);
+  if (first != first)
+    amax = first;
+  const float s = int8_scale_of(amax), inv = int8_inv_scale(s);
+  if (l == 0)
+    sa[blk] = s;
+  for (int64_t j = (int64_t)l * VEC; j < qbs; j += 64 * VEC) {
+    if (qbs > 64 * VEC)
+      load(j);
+    if constexpr (VEC == 4)
+      *reinterpret_cast<uint32_t*>(dst + j) = (uint32_t)(int8_q(v[0], inv) & 0xff) | ((uint32_t)(int8_q(v[1], inv) & 0xff) << 8) |
+          ((uint32_t)(int8_q(v[2], inv) & 0xff) << 16) | ((uint32_t)(int8_q(v[3], inv) & 0xff) << 24);
+    else
+      dst[j] = (int8_t)int8_q(v[0], inv);
+  }
+}
+
 // Scale blocks of several 256-wide runs (per-output-channel weights: one block = all of K): one workgroup per
 // (row, block), 16 lanes per run as above; the runs' maxima meet in LDS.  A lane group's first run stays in registers
 // between the two steps, further runs (blocks beyond 16 Ki channels) are read a second time.
@@ -1054,6 +1102,29 @@ pack_qint_tiles_kernel(const int8_t* __restrict__ nat, int64_t groups, uint8_t* 
 
 static inline unsigned grid_for(int64_t n, int block) {
   return (unsigned)((n + block - 1) / block);
+}
+
+hipError_t launch_quant_act_int8_wide(const void* x, int dtype, int64_t M, int64_t K, int64_t qbs, void* xq, void* sa,
+                                      hipStream_t stream) {
+  const bool vec = aligned16(x);
+  auto go = [&](auto t) {
+    typedef decltype(t) T;
+    const int64_t all = M * (K / qbs), most = 1 << 25; // blocks; a launch takes at most 2^32 work-items
+    for (int64_t at = 0; at < all; at += most) {
+      const int64_t n = all - at < most ? all - at : most;
+      const T* in = (const T*)x + at * qbs;
+      int8_t* q = (int8_t*)xq + at * qbs;
+      if (vec)
+        quant_act_int8_wide_kernel<T, 4><<<grid_for(n * 64, 256), 256, 0, stream>>>(in, n, qbs, q, (float*)sa + at);
+      else
+        quant_act_int8_wide_kernel<T, 1><<<grid_for(n * 64, 256), 256, 0, stream>>>(in, n, qbs, q, (float*)sa + at);
+    }
+  };
+  if (dtype == TPPX_DT_F16)
+    go((_Float16)0);
+  else
+    go(0.0f);
+  return hipGetLastError();
 }
 
 hipError_t launch_quant_act_int8(const void* x, int64_t M, int64_t K, int64_t qbs, void* xq, void* sa, int mt,

@@ -529,31 +529,34 @@ def _mxfp4_flags_ws(x, M, K, flags=0, ws=None):
     return flags, ws
 
 
-def _wide_post(acc, ctype, post, post_in, post_in2, post_scale, shape):
-    """fp32 GEMM tile (bias + dot) -> the activations' type with the post-op applied there (tppx_post_op_wide)."""
-    L = _lib.lib()
-    if ctype == torch.float32 and post == POST_NONE:
-        return acc.view(shape)
-    out = torch.empty(shape, dtype=ctype, device=acc.device)
+_WIDE_DT = {torch.float32: _lib.DT_F32, torch.float16: _lib.DT_F16, torch.bfloat16: _lib.DT_BF16}
+
+
+def _wide_bias(bias, N, dev):
+    """(bias, dtype id) of a float / half linear: read in its own type where the kernels know it."""
+    if bias is None or not bias.numel():
+        return None, _lib.DT_F32
+    if bias.numel() != N:
+        raise TppxError(_lib.ESHAPE, f"bias has {bias.numel()} elements, the weight {N} channels")
+    if bias.dtype not in _WIDE_DT or bias.device != dev:
+        bias = bias.to(device=dev, dtype=torch.float32)
+    return bias.contiguous(), _WIDE_DT[bias.dtype]
+
+
+def _wide_ins(ctype, post, post_in, post_in2, shape, dev):
+    """The post-op's inputs in the output's type, None where it has none."""
     ins = []
     for t, need in ((post_in, post in (POST_MUL, POST_ADD_SCALE, POST_ADD2_SCALE)), (post_in2, post == POST_ADD2_SCALE)):
-        if not need:
-            ins.append(None)
-            continue
-        if t is None or tuple(t.shape) != tuple(shape) or t.device != acc.device:
-            raise TppxError(_lib.ESHAPE, f"post-op {post} needs an input of the output's shape {tuple(shape)} on {acc.device}")
-        ins.append(t.to(ctype).contiguous())
-    if out.numel():
-        _lib.check(L.tppx_post_op_wide(acc.data_ptr(), _lib.DT_F16 if ctype == torch.float16 else _lib.DT_F32, post,
-                                       _lib.ptr(ins[0]), _lib.ptr(ins[1]), float(post_scale), out.data_ptr(),
-                                       out.numel(), _lib.stream_of(acc)))
-    return out
+        if need and (t is None or tuple(t.shape) != tuple(shape) or t.device != dev):
+            raise TppxError(_lib.ESHAPE, f"post-op {post} needs an input of the output's shape {tuple(shape)} on {dev}")
+        ins.append(t.to(ctype).contiguous() if need else None)
+    return ins
 
 
 def _linear_wide(input, weight, bias, post, post_in, post_in2, post_scale):
     """float / half activations on an MXFP4 or an unquantized bf16 weight: TppBlockedLinearW<Tin, uint8_t, Tout> /
     <Tin, bfloat16, Tout> with Tin = float or half (src/csrc/fused_gemm.h:1519-1523, 1541-1550).  The activations are
-    NOT rounded to bf16: fp32 products and sums (every weight value is exact in fp32), output and post-op in the
+    NOT rounded to bf16: exact products and fp32 sums (every weight value is a bf16), output and post-op in the
     activations' type."""
     L = _lib.lib()
     _lib.require_gpu(input, "input")
@@ -570,16 +573,14 @@ def _linear_wide(input, weight, bias, post, post_in, post_in2, post_scale):
     x = input.contiguous()
     M = x.numel() // K
     shape = tuple(input.shape[:-1]) + (N,)
-    acc = torch.empty((M, N), dtype=torch.float32, device=x.device)
+    y = torch.empty(shape, dtype=ctype, device=x.device)
+    ins = _wide_ins(ctype, post, post_in, post_in2, shape, x.device)
     if M:
-        b = None
-        if bias is not None and bias.numel():
-            if bias.numel() != N:
-                raise TppxError(_lib.ESHAPE, f"bias has {bias.numel()} elements, the weight {N} channels")
-            b = bias.to(device=x.device, dtype=torch.float32).contiguous()
-        _lib.check(L.tppx_linear_wide(x.data_ptr(), _lib.DT_F16 if ctype == torch.float16 else _lib.DT_F32, qn.data_ptr(),
-                                      _lib.ptr(sn), kind, _lib.ptr(b), acc.data_ptr(), M, N, K, _lib.stream_of(x)))
-    return _wide_post(acc, ctype, post, post_in, post_in2, post_scale, shape)
+        b, bdt = _wide_bias(bias, N, x.device)
+        _lib.check(L.tppx_linear_wide_post(x.data_ptr(), _WIDE_DT[ctype], qn.data_ptr(), _lib.ptr(sn), kind, _lib.ptr(b), bdt,
+                                           _lib.ptr(ins[0]), _lib.ptr(ins[1]), y.data_ptr(), M, N, K, post,
+                                           float(post_scale), _lib.stream_of(x)))
+    return y
 
 
 def _linear_other_types(input, weight, bias, post, flags, post_in=None, post_in2=None, post_scale=1.0):
@@ -613,20 +614,26 @@ def _linear_other_types(input, weight, bias, post, flags, post_in=None, post_in2
         ctype = input.dtype
         if input.shape[-1] != K:
             raise TppxError(_lib.ESHAPE, f"input has {input.shape[-1]} features, weight expects {K}")
-        act = quantize_int8sym(input.float().contiguous(), qbs, -1, False)
-    shape = tuple(act.shape)
+        act = None
+    shape = tuple(input.shape)
     if shape[-1] != K:
         raise TppxError(_lib.ESHAPE, f"input has {shape[-1]} features, weight expects {K}")
-    xq, sa = act.qdata.contiguous(), act.scales.contiguous()
-    M = xq.numel() // K
+    if act is None:
+        x = input.contiguous()
+        M, dev = x.numel() // K, x.device
+        xq = torch.empty((M, K), dtype=torch.int8, device=dev)
+        sa = torch.empty((M, K // qbs), dtype=torch.float32, device=dev)
+    else:
+        x, xq, sa = None, act.qdata.contiguous(), act.scales.contiguous()
+        M, dev = xq.numel() // K, xq.device
     qn, sn = weight.native()
     st = _lib.stream_of(xq)
     if ctype == torch.bfloat16:
-        y = torch.empty(shape[:-1] + (N,), dtype=torch.bfloat16, device=xq.device)
+        y = torch.empty(shape[:-1] + (N,), dtype=torch.bfloat16, device=dev)
         if M:
-            b = _prep_bias(bias, N, xq.device)
-            p1 = _prep_post(post_in, M, N, "post-op input", xq.device) if post in (POST_MUL, POST_ADD_SCALE, POST_ADD2_SCALE) else None
-            p2 = _prep_post(post_in2, M, N, "second post-op input", xq.device) if post == POST_ADD2_SCALE else None
+            b = _prep_bias(bias, N, dev)
+            p1 = _prep_post(post_in, M, N, "post-op input", dev) if post in (POST_MUL, POST_ADD_SCALE, POST_ADD2_SCALE) else None
+            p2 = _prep_post(post_in2, M, N, "second post-op input", dev) if post == POST_ADD2_SCALE else None
             ws = _lib.workspace(xq)
             _lib.check(L.tppx_linear_qint8(None, xq.data_ptr(), sa.data_ptr(), qn.data_ptr(), sn.data_ptr(), _lib.ptr(b),
                                            _lib.ptr(p1), _lib.ptr(p2), y.data_ptr(), M, N, K, qbs, post, float(post_scale),
@@ -634,16 +641,14 @@ def _linear_other_types(input, weight, bias, post, flags, post_in=None, post_in2
         return y
     if ctype not in (torch.float32, torch.float16):
         raise TppxError(_lib.EUNSUPPORTED, f"compute type {ctype} is not built")
-    y = torch.empty((M, N), dtype=torch.float32, device=xq.device)
+    y = torch.empty(shape[:-1] + (N,), dtype=ctype, device=dev)
+    ins = _wide_ins(ctype, post, post_in, post_in2, y.shape, dev)
     if M:
-        b = None
-        if bias is not None and bias.numel():
-            if bias.numel() != N:
-                raise TppxError(_lib.ESHAPE, f"bias has {bias.numel()} elements, the weight {N} channels")
-            b = bias.to(device=xq.device, dtype=torch.float32).contiguous()
-        _lib.check(L.tppx_linear_qint8_f32(xq.data_ptr(), sa.data_ptr(), qn.data_ptr(), sn.data_ptr(), _lib.ptr(b),
-                                           y.data_ptr(), M, N, K, qbs, st))
-    return _wide_post(y, ctype, post, post_in, post_in2, post_scale, shape[:-1] + (N,))
+        b, bdt = _wide_bias(bias, N, dev)
+        _lib.check(L.tppx_linear_qint8_wide(_lib.ptr(x), _WIDE_DT[ctype], xq.data_ptr(), sa.data_ptr(), qn.data_ptr(),
+                                            sn.data_ptr(), _lib.ptr(b), bdt, _lib.ptr(ins[0]), _lib.ptr(ins[1]), y.data_ptr(),
+                                            M, N, K, qbs, post, float(post_scale), st))
+    return y
 
 
 PACKED_CODES = os.environ.get("TPPX_PACKED_CODES", "1") == "1"

@@ -570,6 +570,18 @@ int tppx_attn_decode_rotary(const void* q, const void* k, const void* v,
                             int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
                             void* ws, int64_t ws_bytes, tppx_stream_t stream);
 
+/* The same for the other head sizes (H a multiple of 8 up to 256, not 128):
+ * tppx_rotary_kv_append_llama or, with gptj, _gptj for one token per sequence
+ * and tppx_attn_decode in one launch.  emb_pos f32 [2][MP][HR] cos / sin, with
+ * gptj [MP][HR] sin | cos, or NULL (append without rotation). */
+int tppx_attn_decode_append(const void* q, const void* k, const void* v,
+                            const void* emb_pos, int gptj, const void* pos,
+                            int64_t B_pos, int64_t MP, int64_t HR, void* kcache,
+                            void* vcache, const void* mask, int64_t mask_ld,
+                            const void* kv_len_dev, void* out, int64_t B,
+                            int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
+                            void* ws, int64_t ws_bytes, tppx_stream_t stream);
+
 /* The same attn<T> (src/csrc/llm/attn.cpp:781-955, isCausal) for S query tokens
  * per sequence (prompt processing, or several new tokens on a filled cache):
  * q / out bf16 [B][S][Nq][128]; the cache already holds the S new keys at

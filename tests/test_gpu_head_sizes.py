@@ -204,3 +204,71 @@ def test_attn_prefill_other_head_size_with_mask(H):
     g, r = bits2f(t2bits(got)).astype(np.float64), bits2f(ref).astype(np.float64)
     assert np.isfinite(g).all()
     assert np.sqrt(((g - r) ** 2).sum() / (r ** 2).sum()) <= 5e-3
+
+
+# around the edges of a trip (128 or 64 keys) and of a wave's keys (32 or 16), an empty and a full cache, one split and
+# several, query heads sharing a K/V head, no mask / mask
+@pytest.mark.parametrize("H,HR,style", [(256, 64, "gptj"), (80, 0, None), (64, 64, "llama"), (96, 96, "llama"), (200, 80, "llama"),
+                                        (16, 16, "gptj"), (8, 0, None), (72, 48, "gptj"), (136, 136 - 8, "llama")])
+@pytest.mark.parametrize("B,Nq,Nkv,past,Smax", [(1, 4, 4, 0, 700), (2, 8, 2, 31, 64), (1, 2, 2, 63, 64), (3, 4, 4, 128, 1024),
+                                                (1, 6, 3, 700, 1100), (2, 4, 4, 64, 64), (40, 16, 16, 97, 130)])
+def test_decode_step_with_rotary_and_append_in_the_launch(H, HR, style, B, Nq, Nkv, past, Smax):
+    """tppx_attn_decode_append against the two launches it stands for: the same cache (positions it must not touch
+    included), rotated values within one rounding, the context to the tolerance of the two orders of sums; every replay of a
+    captured step the same."""
+    from tpp_pytorch_extension import _lib
+    F = _llm()
+    L = _lib.lib()
+    g = torch.Generator(device="cuda").manual_seed(7 * H + past)
+
+    def rnd(*shape):
+        return torch.randn(shape, generator=g, device="cuda").to(torch.bfloat16)
+
+    q, k, v, kc, vc = rnd(B, Nq, H), rnd(B, Nkv, H), rnd(B, Nkv, H), rnd(B, Nkv, Smax, H), rnd(B, Nkv, Smax, H)
+    kc[:, :, past + 1:] = vc[:, :, past + 1:] = float("nan")
+    MP = 512
+    pos = torch.randint(0, MP + 20, (B, 1), generator=g, device="cuda")  # some past the table: not rotated
+    emb = None
+    if style == "llama":
+        emb = F.llama_rotary_table(MP, HR)
+    elif style == "gptj":
+        emb = torch.randn((MP, HR), generator=g, device="cuda")
+    mask = torch.where(torch.rand((B, past + 1), generator=g, device="cuda") < 0.2, -10000.0, 0.0).to(torch.bfloat16) if past > 40 else None
+    n = torch.tensor([past], dtype=torch.int32, device="cuda")
+    ws = _lib.workspace(q)
+    st = _lib.stream_of(q)
+    P = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    mld = mask.shape[1] if mask is not None else 0
+    q2, k2, kc2, vc2 = q.clone(), k.clone(), kc.clone(), vc.clone()
+    out, ref = torch.empty_like(q), torch.empty_like(q)
+
+    def step(stream):
+        _lib.check(L.tppx_attn_decode_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), P(emb), style == "gptj", pos.data_ptr(), B,
+                                             MP, HR, kc.data_ptr(), vc.data_ptr(), P(mask), mld, n.data_ptr(), out.data_ptr(),
+                                             B, Nq, Nkv, H, Smax, ws.data_ptr(), ws.numel(), stream))
+
+    q0, k0 = q.clone(), k.clone()
+    step(st)
+    fn = L.tppx_rotary_kv_append_gptj if style == "gptj" else L.tppx_rotary_kv_append_llama
+    _lib.check(fn(q2.data_ptr(), k2.data_ptr(), v.data_ptr(), P(emb), pos.data_ptr(), kc2.data_ptr(), vc2.data_ptr(), n.data_ptr(),
+                  B, 1, Nq, Nkv, H, MP, HR if emb is not None else H, B, Smax, st))
+    _lib.check(L.tppx_attn_decode(q2.data_ptr(), kc2.data_ptr(), vc2.data_ptr(), P(mask), mld, n.data_ptr(), 1, ref.data_ptr(),
+                                  B, Nq, Nkv, H, Smax, ws.data_ptr(), ws.numel(), st))
+    assert torch.equal(q, q0) and torch.equal(k, k0)
+    a, b = kc.float(), kc2.float()
+    assert torch.equal(a.isnan(), b.isnan()) and torch.equal(vc.view(torch.int16), vc2.view(torch.int16))
+    a, b = a.nan_to_num(0.0), b.nan_to_num(0.0)
+    assert ((a - b).abs() <= 2.0 ** -7 * b.abs()).all() and (a != b).float().mean() < 1e-3
+    assert out.isfinite().all()
+    assert (out.float() - ref.float()).norm() <= 5e-3 * ref.float().norm()
+    first = out.clone()
+    s2 = torch.cuda.Stream()
+    s2.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s2):
+        step(torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, first)

@@ -1871,6 +1871,19 @@ extern "C" int tppx_rotary_kv_append_gptj(void* q, void* k, const void* v, const
 }
 
 // shared tail of the two single-query entry points: split planning, counters, launch
+// window of arrival counters (at most ATTN_TICKETS), handed out in rotation so that split launches in flight on different
+// streams do not share counters
+static int attn_take_tickets(int64_t tickets) {
+  static std::mutex mu;
+  static int cursor = 0;
+  std::lock_guard<std::mutex> lock(mu);
+  if (cursor + tickets > ATTN_TICKETS)
+    cursor = 0;
+  const int first = cursor;
+  cursor += (int)tickets;
+  return first;
+}
+
 static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t B, int64_t Nq, int64_t Smax, void* ws,
                               int64_t ws_bytes, hipStream_t stream) {
   // The wide kernel (128 keys per workgroup and trip) is the default: measured against the row kernel (64 keys per
@@ -1917,17 +1930,8 @@ static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t 
   p.part = (float*)ws;
   p.ticket0 = -1;
   const int64_t tickets = group ? groups : B * Nq;
-  if (splits > 1 && tickets <= ATTN_TICKETS && one_launch) {
-    // window of arrival counters, handed out in rotation so that split launches in flight on different
-    // streams do not share counters
-    static std::mutex mu;
-    static int cursor = 0;
-    std::lock_guard<std::mutex> lock(mu);
-    if (cursor + tickets > ATTN_TICKETS)
-      cursor = 0;
-    p.ticket0 = cursor;
-    cursor += (int)tickets;
-  }
+  if (splits > 1 && tickets <= ATTN_TICKETS && one_launch)
+    p.ticket0 = attn_take_tickets(tickets);
   const dim3 grid((unsigned)(group ? groups : B * Nq), (unsigned)splits);
   if (group && rot)
     attn_decode_group_kernel<true><<<grid, dim3(AG_WAVES * 64), 0, stream>>>(p);
@@ -1957,7 +1961,7 @@ static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t 
 // ---------------------------------------------------------------------------
 // Attention for head sizes other than 128 (attn<T>, src/csrc/llm/attn.cpp:781-955, is generic in the head size; the
 // kernels above are built for 128), H a multiple of 8 up to 256.  The single-query step runs on
-// attn_generic_rows_kernel below, prompt passes on attn_prefill_hd_kernel above; this first, plain kernel serves
+// attn_hd_step_kernel below, prompt passes on attn_prefill_hd_kernel above; this first, plain kernel serves
 // both when those are switched off (TPPX_ATTN_GENERIC_ROWS=0, TPPX_ATTN_PREFILL_MFMA=0).  One wave per (sequence,
 // query token, query head), four per workgroup, no barrier: 64 keys per trip,
 // a lane takes the whole dot product of its key (16-byte loads along its row, the query as fp32 in wave-private
@@ -1975,8 +1979,16 @@ struct AttnGenParams {
   uint16_t* out;       // [B][S][Nq][H]
   int B, S, Nq, Nkv, H, Smax, mask_ld, past; // prompt pass: query i sees keys 0 .. past + i
   float scale;
-  int splits;          // single-query step (attn_generic_rows_kernel): workgroups per query, see there
+  // single-query step (attn_hd_step_kernel):
+  int splits;          // workgroups per query
+  int ticket0;         // splits > 1: first arrival counter of this launch
   float* part;         // splits > 1: [query][split][2 + H] floats (running maximum, sum, unnormalised output)
+  // APP: the query and the step's new key / value arrive unrotated and not yet in the cache
+  const uint16_t* k_new; // [B][Nkv][H]
+  const uint16_t* v_new;
+  const float* emb;      // cos / sin [2][MP][HR] (Llama pairs) or sin | cos [MP][HR] (gptj), or null: no rotation
+  const int64_t* pos;    // i64 [B_pos]
+  int MP, HR, B_pos, gptj;
 };
 
 __global__ void __launch_bounds__(256)
@@ -2050,173 +2062,282 @@ attn_generic_kernel(const AttnGenParams p) {
       orow[lane + 64 * i] = (uint16_t)f32_to_bf16_bits(l > 0.f ? acc[i] / l : 0.f);
 }
 
-// The single-query step at those head sizes, laid out like attn_decode_kernel: G = 8, 16 or 32 lanes share a key
-// (lane = key slot l / G, 16-byte chunk l % G; chunks past H / 8 idle), so a wave instruction reads 64 / G whole
-// rows; NU instructions per wave and trip with the next trip requested ahead; every lane group keeps its own
-// running (maximum, sum, 8 output dims per lane), merged at the end through LDS.  Grid (B * Nq, splits): split y
-// takes the trips y, y + splits, ...; several splits leave their states for attn_generic_merge_kernel.
-template <int G>
-__global__ void __launch_bounds__(256)
-attn_generic_rows_kernel(const AttnGenParams p) {
+// The single-query step at those head sizes, laid out like attn_decode_wide_kernel: G lanes share a key, a lane owns its
+// chunks j*G + c (8 dims of 16 bytes each; chunks past H / 8 idle) of NU keys, so a wave instruction reads 64 / G whole
+// (part) rows and a trip's K and V rows -- up to 16 KB a wave -- are requested at once, the first trip's before the length is
+// known.  q . k and p . v run on the bf16 dot instruction, the wave shares one running maximum, the lanes' outputs are added
+// up through LDS.  Grid (B * Nq, splits): split y takes the trips y, y + splits, ...; the split that arrives last merges all
+// of them in the launch.
+// APP: the launch also does what the rotary + append launch did before it (LayerCache::update, attn.h:198-222): wave 0
+// rotates the query and, in the split that reads its position, the new key -- rounded to bf16, as stored -- and that
+// position's lanes take key and value from there; one workgroup per KV head writes them into the cache.
+// What bounds a step of a few sequences is this chain of launches and of dependent loads, many the bytes.  In a graph of
+// steps, against rotary + append, attention and the merge as launches of their own: 16 heads of 256, 1 x 2000 keys
+// 24.2 -> 12.5 us, 4 x 700 18.1 -> 12.2, 16 x 2500 106.5 (6.2 TB/s) either way; 32 heads of 80, 1 x 2000 14.3 -> 9.7,
+// 4 x 140 7.8 -> 7.0, 48 x 1400 113.7 -> 108.3.  (80 as 8 lanes x 2 chunks, the second a quarter live, 117.4.)
+template <int G, int J, int NU, bool APP>
+__global__ void __launch_bounds__(256, 4)
+attn_hd_step_kernel(const AttnGenParams p) {
   constexpr int KPI = 64 / G;            // keys per wave instruction
-  constexpr int NU = G == 8 ? 2 : 4;     // instructions per wave and trip
   constexpr int WK = NU * KPI;           // keys per wave and trip
   constexpr int TRIP = 4 * WK;           // keys per workgroup and trip
-  constexpr int NG = 4 * KPI;            // lane groups per workgroup
-  __shared__ float sm[NG], sl[NG];
-  __shared__ float sacc[NG * G * 8];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int OP = G * J * 8 + 4;      // pitch of a lane group's output in floats
+  __shared__ __align__(16) uint16_t q_s[G * J * 8], k_s[G * J * 8];
+  __shared__ float sm[4], sl[4];
+  __shared__ __align__(16) float sacc[4][KPI][OP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = lane / G, c = lane % G;
-  const int H = p.H, C = H >> 3;
-  const bool live = c < C;               // this lane's chunk exists
-  const int cc = min(c, C - 1);
+  const int H = p.H, C = H >> 3, S = p.splits;
   const int bh = blockIdx.x, b = bh / p.Nq, hq = bh - b * p.Nq;
   const int hk = hq / (p.Nq / p.Nkv);
-  const uint16_t* kb = p.kc + ((int64_t)b * p.Nkv + hk) * (int64_t)p.Smax * H + cc * 8;
-  const uint16_t* vb = p.vc + ((int64_t)b * p.Nkv + hk) * (int64_t)p.Smax * H + cc * 8;
-  i32x4 kw[NU], vw[NU], kn[NU], vn[NU];
-  auto load_kv = [&](int base, i32x4 (&kd)[NU], i32x4 (&vd)[NU]) {
+  const int64_t kv_head = (int64_t)b * p.Nkv + hk;
+  const uint16_t* kb = p.kc + kv_head * p.Smax * H;
+  const uint16_t* vb = p.vc + kv_head * p.Smax * H;
+  bool live[J];                          // this lane's chunks that exist; the others re-read the last one
+  int at[J];
+#pragma unroll
+  for (int j = 0; j < J; j++) {
+    live[j] = j * G + c < C;
+    at[j] = min(j * G + c, C - 1) * 8;
+  }
+  i32x4 kr[NU][J], vr[NU][J];
+  auto load_rows = [&](const uint16_t* src, int base, i32x4 (&dst)[NU][J]) {
 #pragma unroll
     for (int u = 0; u < NU; u++) {
-      const int kk = min(base + u * KPI + grp, p.Smax - 1);
-      kd[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(kb + (int64_t)kk * H));
-      vd[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(vb + (int64_t)kk * H));
+      const int64_t row = (int64_t)min(base + u * KPI + grp, p.Smax - 1) * H; // past the end: read, never used
+#pragma unroll
+      for (int j = 0; j < J; j++)
+        dst[u][j] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(src + row + at[j]));
     }
   };
-  load_kv(blockIdx.y * TRIP + wave * WK, kw, vw); // the first trip does not depend on the length (a device scalar)
-  const int L = max(0, min(p.kv_len[0] + p.kv_len_add, p.Smax));
-  const int trips = (L + TRIP - 1) / TRIP;
-  float qf[8];
-  unpack8(*reinterpret_cast<const uint4*>(p.q + (int64_t)bh * H + cc * 8), qf);
+  // A wave's loads return in the order of their issue: wave 0 asks for the query and the new key first (dims lane + 64 i)
+  constexpr int D = G * J / 8;           // head dims per lane of wave 0
+  i32x4 qp[J];
+  float qx[D], qo[D], kx[D], ko[D], cs[D], sn[D]; // value, its pair's other half, cos, signed sin
+  bool turned[D];
+  if (!APP) {
 #pragma unroll
-  for (int e = 0; e < 8; e++)
-    qf[e] = live ? qf[e] * p.scale : 0.f;
-  const uint16_t* mrow = p.mask ? p.mask + (int64_t)b * p.mask_ld : nullptr;
-  float m = -3.0e38f, l = 0.f, acc[8];
+    for (int j = 0; j < J; j++)
+      qp[j] = *reinterpret_cast<const i32x4*>(p.q + (int64_t)bh * H + at[j]);
+  } else if (wave == 0) {
+    const uint16_t* qrow = p.q + (int64_t)bh * H;
+    const uint16_t* krow = p.k_new + kv_head * H;
+    const int64_t pp = p.emb ? p.pos[p.B_pos == 1 ? 0 : b] : -1;
+    const bool rot = pp >= 0 && pp < p.MP; // positions outside the table are left unrotated
+    const int half = p.HR >> 1;
 #pragma unroll
-  for (int e = 0; e < 8; e++)
-    acc[e] = 0.f;
-  for (int t = blockIdx.y; t < trips; t += p.splits) {
-    const int base = t * TRIP + wave * WK;
-    load_kv(base + p.splits * TRIP, kn, vn); // unconditional (rows are clamped): a branch here would drain the queue
-    float sc[NU];
-    int key[NU];
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      key[u] = base + u * KPI + grp;
-      float kf[8];
-      unpack8(as_uint4(kw[u]), kf);
-      float d = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        d = fmaf(qf[e], kf[e], d);
-      // sum over the G lanes of the key: DPP steps inside a row of 16, then the other half of a 32-lane group
-      d += dpp_mov<0xB1>(d);
-      d += dpp_mov<0x4E>(d);
-      d += dpp_mov<0x141>(d);
-      if (G >= 16)
-        d += dpp_mov<0x140>(d);
-      if (G == 32)
-        d += __shfl_xor(d, 16);
-      if (mrow && key[u] < p.mask_ld && key[u] < L)
-        d += bf16_bits_to_f32(mrow[key[u]]);
-      sc[u] = key[u] < L ? d : -3.0e38f;
-    }
-    if (t * TRIP + TRIP > L) { // the last trip only (wave-uniform): rows past the end may hold anything, NaN included
-#pragma unroll
-      for (int u = 0; u < NU; u++)
-        if (key[u] >= L)
-          vw[u] = i32x4{0, 0, 0, 0};
-    }
-    float mn = m;
-#pragma unroll
-    for (int u = 0; u < NU; u++)
-      mn = fmaxf(mn, sc[u]);
-    const float alpha = __expf(m - mn);
-    l *= alpha;
-#pragma unroll
-    for (int e = 0; e < 8; e++)
-      acc[e] *= alpha;
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      const float pr = key[u] < L ? __expf(sc[u] - mn) : 0.f;
-      l += pr;
-      const float pb = round_bf16(pr); // the probabilities that multiply V are bf16, the normaliser sums the unrounded
-      float vf[8];
-      unpack8(as_uint4(vw[u]), vf);
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        acc[e] = fmaf(pb, vf[e], acc[e]);
-    }
-    m = mn;
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      kw[u] = kn[u];
-      vw[u] = vn[u];
-    }
-  }
-  // merge the lane groups of the workgroup
-  const int gi = wave * KPI + grp;
-  if (c == 0) {
-    sm[gi] = m;
-    sl[gi] = l;
-  }
-  if (live) {
-#pragma unroll
-    for (int e = 0; e < 8; e++)
-      sacc[gi * (G * 8) + c * 8 + e] = acc[e];
-  }
-  __syncthreads();
-  if (tid < H) {
-    float M = -3.0e38f;
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-      M = fmaxf(M, sm[g]);
-    float Ls = 0.f, o = 0.f;
-#pragma unroll
-    for (int g = 0; g < NG; g++) {
-      const float w = __expf(sm[g] - M);
-      Ls = fmaf(w, sl[g], Ls);
-      o = fmaf(w, sacc[g * (G * 8) + tid], o);
-    }
-    if (p.splits == 1) {
-      p.out[(int64_t)bh * H + tid] = (uint16_t)f32_to_bf16_bits(Ls > 0.f ? o / Ls : 0.f);
-    } else {
-      float* st = p.part + ((int64_t)bh * p.splits + blockIdx.y) * (int64_t)(H + 2);
-      st[2 + tid] = o;
-      if (tid == 0) {
-        st[0] = M;
-        st[1] = Ls;
+    for (int i = 0; i < D; i++) {
+      const int d = min(lane + 64 * i, H - 1);
+      const bool turn = rot && d < p.HR;
+      const bool second = p.gptj ? (d & 1) : d >= half;
+      const int o = !turn ? d : p.gptj ? d ^ 1 : second ? d - half : d + half;
+      const int e = p.gptj ? d >> 1 : second ? d - half : d;
+      qx[i] = bf16_bits_to_f32(qrow[d]);
+      qo[i] = bf16_bits_to_f32(qrow[o]);
+      kx[i] = bf16_bits_to_f32(krow[d]);
+      ko[i] = bf16_bits_to_f32(krow[o]);
+      cs[i] = sn[i] = 0.f;
+      turned[i] = turn;
+      if (turn) {
+        cs[i] = p.gptj ? p.emb[pp * p.HR + half + e] : p.emb[pp * p.HR + e];
+        sn[i] = p.gptj ? p.emb[pp * p.HR + e] : p.emb[((int64_t)p.MP + pp) * p.HR + e];
+        if (!second)
+          sn[i] = -sn[i];
       }
     }
   }
-}
-
-// one wave per query: the splits' (maximum, sum, output) states, in split order, become the normalised output
-__global__ void __launch_bounds__(64)
-attn_generic_merge_kernel(const AttnGenParams p) {
-  const int lane = threadIdx.x;
-  const int64_t qi = blockIdx.x;
-  const int H = p.H;
-  const float* st = p.part + qi * p.splits * (int64_t)(H + 2);
-  float M = -3.0e38f;
-  for (int i = 0; i < p.splits; i++)
-    M = fmaxf(M, st[i * (H + 2)]);
-  float Ls = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < p.splits; i++) {
-    const float* si = st + i * (int64_t)(H + 2);
-    const float w = __expf(si[0] - M); // a split without keys carries sum 0 and output 0
-    Ls = fmaf(w, si[1], Ls);
+  load_rows(kb, blockIdx.y * TRIP + wave * WK, kr);
+  load_rows(vb, blockIdx.y * TRIP + wave * WK, vr);
+  const int len0 = *p.kv_len;
+  const int L = max(0, min(len0 + p.kv_len_add, p.Smax));
+  const int nk = (APP && len0 >= 0 && len0 < p.Smax) ? len0 : -1; // cache position of the new token
+  const int trips = (L + TRIP - 1) / TRIP;
+  // the split whose trips contain the new token's position (uniform over the workgroup)
+  const bool has_new = APP && nk >= 0 && nk < L && (nk / TRIP) % S == (int)blockIdx.y;
+  if (APP) {
+    if (wave == 0) {
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-      if (lane + 64 * j < H)
-        o[j] = fmaf(w, si[2 + lane + 64 * j], o[j]);
+      for (int i = 0; i < D; i++) {
+        const int d = lane + 64 * i;
+        if (d < H) {
+          q_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? qx[i] * cs[i] + qo[i] * sn[i] : qx[i]);
+          k_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? kx[i] * cs[i] + ko[i] * sn[i] : kx[i]);
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < J; j++)
+      qp[j] = *reinterpret_cast<const i32x4*>(q_s + at[j]);
+    // one workgroup per KV head appends: the first query head of the group, in the split that reads the position
+    if (has_new && hq == hk * (p.Nq / p.Nkv) && tid < C) {
+      const int64_t o = (kv_head * p.Smax + nk) * H + tid * 8;
+      *reinterpret_cast<i32x4*>(const_cast<uint16_t*>(p.kc) + o) = reinterpret_cast<const i32x4*>(k_s)[tid];
+      *reinterpret_cast<i32x4*>(const_cast<uint16_t*>(p.vc) + o) = reinterpret_cast<const i32x4*>(p.v_new + kv_head * H)[tid];
+    }
   }
-  uint16_t* orow = p.out + qi * H;
+  const uint16_t* mrow = p.mask ? p.mask + (int64_t)b * p.mask_ld : nullptr;
+  float m = -3.0e38f, l = 0.f; // m is the same in every lane of the wave
+  float acc[J * 8];
 #pragma unroll
-  for (int j = 0; j < 4; j++)
-    if (lane + 64 * j < H)
-      orow[lane + 64 * j] = (uint16_t)f32_to_bf16_bits(Ls > 0.f ? o[j] / Ls : 0.f);
+  for (int e = 0; e < J * 8; e++)
+    acc[e] = 0.f;
+  for (int t = blockIdx.y; t < trips; t += S) {
+    const int base = t * TRIP + wave * WK;
+    if (t != (int)blockIdx.y) {
+      load_rows(kb, base, kr);
+      load_rows(vb, base, vr);
+    }
+    if (has_new && nk >= base && nk < base + WK && grp == (nk - base) % KPI) {
+      const int u_new = (nk - base) / KPI;
+#pragma unroll
+      for (int u = 0; u < NU; u++)
+        if (u == u_new) {
+#pragma unroll
+          for (int j = 0; j < J; j++) {
+            kr[u][j] = *reinterpret_cast<const i32x4*>(k_s + at[j]);
+            vr[u][j] = *reinterpret_cast<const i32x4*>(p.v_new + kv_head * H + at[j]);
+          }
+        }
+    }
+    float sc[NU], mx = -3.0e38f;
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const int key = base + u * KPI + grp;
+      float d = 0.f;
+#pragma unroll
+      for (int j = 0; j < J; j++) {
+        float dj = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          dj = dot2_bf16((uint32_t)kr[u][j][r], (uint32_t)qp[j][r], dj);
+        d += live[j] ? dj : 0.f;
+      }
+      d += dpp_mov<0xB1>(d);  // the parts of the key: quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror, row_mirror
+      d += dpp_mov<0x4E>(d);
+      d += dpp_mov<0x141>(d);
+      if (G == 16)
+        d += dpp_mov<0x140>(d);
+      d *= p.scale;
+      if (mrow && key < p.mask_ld && key < L)
+        d += bf16_bits_to_f32(mrow[key]);
+      sc[u] = key < L ? d : -3.0e38f;
+      mx = fmaxf(mx, sc[u]);
+    }
+    const float mn = fmaxf(m, wave_max(mx));
+    if (mn > m) { // wave-uniform; rare once the first trips have passed
+      const float alpha = __expf(m - mn);
+      l *= alpha;
+#pragma unroll
+      for (int e = 0; e < J * 8; e++)
+        acc[e] *= alpha;
+      m = mn;
+    }
+    uint32_t pk[NU / 2]; // probabilities of the key pairs as packed bf16; the normaliser sums the unrounded ones
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const int key = base + u * KPI + grp;
+      const float pr = key < L ? __expf(sc[u] - m) : 0.f;
+      l += pr;
+      const uint32_t pb = f32_to_bf16_bits(pr);
+      if (u & 1)
+        pk[u >> 1] |= pb << 16;
+      else
+        pk[u >> 1] = pb;
+      if (base + WK > L && key >= L) { // rows past the end may hold anything, NaN included
+#pragma unroll
+        for (int j = 0; j < J; j++)
+          vr[u][j] = i32x4{0, 0, 0, 0};
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < NU / 2; h++)
+#pragma unroll
+      for (int j = 0; j < J; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const uint32_t va = (uint32_t)vr[2 * h][j][r], vb2 = (uint32_t)vr[2 * h + 1][j][r];
+          const uint32_t lo = __builtin_amdgcn_perm(vb2, va, 0x05040100u); // (a.dim 2r, b.dim 2r)
+          const uint32_t hi = __builtin_amdgcn_perm(vb2, va, 0x07060302u); // (a.dim 2r+1, b.dim 2r+1)
+          acc[j * 8 + 2 * r] = dot2_bf16(lo, pk[h], acc[j * 8 + 2 * r]);
+          acc[j * 8 + 2 * r + 1] = dot2_bf16(hi, pk[h], acc[j * 8 + 2 * r + 1]);
+        }
+  }
+#pragma unroll
+  for (int j = 0; j < J; j++) {
+    float* dst = &sacc[wave][grp][(j * G + c) * 8];
+    *reinterpret_cast<f32x4*>(dst) = f32x4{acc[j * 8], acc[j * 8 + 1], acc[j * 8 + 2], acc[j * 8 + 3]};
+    *reinterpret_cast<f32x4*>(dst + 4) = f32x4{acc[j * 8 + 4], acc[j * 8 + 5], acc[j * 8 + 6], acc[j * 8 + 7]};
+  }
+  const float lw = wave_sum(l) * (1.0f / G); // every key's l sits in its G lanes: counted G times, a power of two
+  if (lane == 0) {
+    sm[wave] = m;
+    sl[wave] = lw;
+  }
+  __syncthreads();
+  float M = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3])), Ls = 0.f, o = 0.f;
+  float* st = p.part + ((int64_t)bh * S + blockIdx.y) * (H + 2);
+  if (tid < H) {
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      float so = 0.f;
+#pragma unroll
+      for (int i = 0; i < KPI; i++)
+        so += sacc[w][i][tid];
+      const float wt = __expf(sm[w] - M);
+      Ls = fmaf(wt, sl[w], Ls);
+      o = fmaf(wt, so, o);
+    }
+    if (S == 1) {
+      p.out[(int64_t)bh * H + tid] = (uint16_t)f32_to_bf16_bits(Ls > 0.f ? o / Ls : 0.f);
+    } else { // device scope: written through to the level all XCDs share
+      __hip_atomic_store(st + 2 + tid, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) {
+        __hip_atomic_store(st, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(st + 1, Ls, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  }
+  if (S == 1)
+    return;
+  // as in attn_finish: own stores acknowledged, barrier, ticket, then the device-scope loads; nobody waits for anybody
+  __shared__ int arrived_last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const unsigned int last = (unsigned int)S - 1;
+    arrived_last = atomicInc(&attn_tickets[(p.ticket0 + bh) * ATTN_TICKET_STRIDE], last) == last;
+  }
+  __syncthreads();
+  if (!arrived_last || tid >= H)
+    return;
+  const float* src = p.part + (int64_t)bh * S * (H + 2);
+  float pm[32], pl[32], po[32]; // every load in flight at once (at most 32 splits)
+  M = -3.0e38f;
+#pragma unroll
+  for (int i = 0; i < 32; i++) {
+    pm[i] = -3.0e38f;
+    pl[i] = po[i] = 0.f;
+    if (i < S) {
+      pm[i] = __hip_atomic_load(src + i * (H + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      pl[i] = __hip_atomic_load(src + i * (H + 2) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      po[i] = __hip_atomic_load(src + i * (H + 2) + 2 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 32; i++)
+    if (i < S)
+      M = fmaxf(M, pm[i]);
+  Ls = 0.f;
+  o = 0.f;
+#pragma unroll
+  for (int i = 0; i < 32; i++)
+    if (i < S) {
+      const float w = __expf(pm[i] - M); // a split without keys carries sum 0 and output 0
+      Ls = fmaf(w, pl[i], Ls);
+      o = fmaf(w, po[i], o);
+    }
+  p.out[(int64_t)bh * H + tid] = (uint16_t)f32_to_bf16_bits(Ls > 0.f ? o / Ls : 0.f);
 }
 
 static int attn_generic_launch(const char* who, AttnGenParams& p, hipStream_t stream, void* ws = nullptr,
@@ -2226,35 +2347,41 @@ static int attn_generic_launch(const char* who, AttnGenParams& p, hipStream_t st
   const int64_t queries = (int64_t)p.B * p.S * p.Nq;
   p.splits = 1;
   if (p.kv_len && p.S == 1 && env_int("TPPX_ATTN_GENERIC_ROWS", 1) != 0) {
-    // Single-query steps: a workgroup per (query, split of the key range).  Up to 384 workgroups in all (measured at
-    // 2048 keys: 16 heads of 256 59.9 -> 21.1 us with 24 splits, 64 queries 57.8 -> 27.6 us with 6, 256 queries
-    // better unsplit), at least two trips each at the cache's capacity (the length itself is a device scalar: splits
-    // whose trips lie past the keys leave empty states), at most 32; one split for caches under 512 keys (the merge
-    // launch costs more than it saves) and when the caller's workspace cannot hold the states.
-    const int G = p.H <= 64 ? 8 : p.H <= 128 ? 16 : 32;
-    const int trip = G == 32 ? 32 : 64;
+    TPPX_REQUIRE(queries < ((int64_t)1 << 31), TPPX_ESHAPE, "%s: problem too large", who);
+    // Workgroups per (sequence, head), as for 128-wide heads: two trips each at the cache's capacity (the length itself is
+    // a device scalar: splits whose trips lie past the keys leave empty states), but no fewer than 288 workgroups and no
+    // more than 512 in all; at most one per trip and 32.  One for caches of three trips (50 keys in 178 of one sequence:
+    // 4.6 us against 6.5 with two), from 256 heads on (16 x 16 x 700 keys: 30.5 against 31.6 with two) and where the
+    // workspace cannot hold the states.
+    const int64_t trip = p.H <= 128 ? 128 : 64, most = ((int64_t)p.Smax + trip - 1) / trip;
     int64_t want = env_int("TPPX_ATTN_GENERIC_SPLITS", 0);
-    if (want <= 0)
-      want = p.Smax < 512 ? 1 : 384 / queries;
-    want = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 32), ((int64_t)p.Smax + 2 * trip - 1) / (2 * trip)));
-    if (want > 1 && ws && queries * want * (p.H + 2) * (int64_t)sizeof(float) <= ws_bytes) {
+    if (want <= 0 && (most <= 3 || queries >= 256))
+      want = 1;
+    else if (want <= 0)
+      want = std::max((288 + queries - 1) / queries, std::min((most + 1) / 2, (512 + queries - 1) / queries));
+    want = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 32), most));
+    if (want > 1 && queries <= ATTN_TICKETS && ws && queries * want * (p.H + 2) * (int64_t)sizeof(float) <= ws_bytes) {
       p.splits = (int)want;
       p.part = (float*)ws;
+      p.ticket0 = attn_take_tickets(queries);
     }
-    TPPX_REQUIRE(queries < ((int64_t)1 << 31), TPPX_ESHAPE, "%s: problem too large", who);
     const dim3 grid((unsigned)queries, (unsigned)p.splits);
-    if (G == 8)
-      attn_generic_rows_kernel<8><<<grid, dim3(256), 0, stream>>>(p);
-    else if (G == 16)
-      attn_generic_rows_kernel<16><<<grid, dim3(256), 0, stream>>>(p);
+    auto go = [&](auto app) {
+      constexpr bool APP = decltype(app)::value;
+      if (p.H <= 64)
+        attn_hd_step_kernel<8, 1, 4, APP><<<grid, dim3(256), 0, stream>>>(p);
+      else if (p.H <= 128)
+        attn_hd_step_kernel<16, 1, 8, APP><<<grid, dim3(256), 0, stream>>>(p);
+      else
+        attn_hd_step_kernel<16, 2, 4, APP><<<grid, dim3(256), 0, stream>>>(p);
+    };
+    if (p.k_new)
+      go(std::true_type{});
     else
-      attn_generic_rows_kernel<32><<<grid, dim3(256), 0, stream>>>(p);
-    int rc = check_hip(hipGetLastError(), who);
-    if (rc || p.splits == 1)
-      return rc;
-    attn_generic_merge_kernel<<<dim3((unsigned)queries), dim3(64), 0, stream>>>(p);
+      go(std::false_type{});
     return check_hip(hipGetLastError(), who);
   }
+  TPPX_REQUIRE(!p.k_new, TPPX_EUNSUPPORTED, "%s: the single-query kernel is switched off", who);
   const int64_t waves = queries;
   TPPX_REQUIRE(waves > 0 && (waves + 3) / 4 < ((int64_t)1 << 31), TPPX_ESHAPE, "%s: problem too large", who);
   attn_generic_kernel<<<dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream>>>(p);
@@ -2316,6 +2443,33 @@ extern "C" int tppx_attn_decode_rotary(const void* q, const void* k, const void*
   p.k_new = (const uint16_t*)k; p.v_new = (const uint16_t*)v; p.emb = (const float*)emb_pos; p.pos = (const int64_t*)pos;
   p.MP = (int)MP; p.B_pos = (int)B_pos;
   return attn_decode_launch(who, p, true, B, Nq, Smax, ws, ws_bytes, (hipStream_t)stream);
+}
+
+extern "C" int tppx_attn_decode_append(const void* q, const void* k, const void* v, const void* emb_pos, int gptj,
+                                       const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache, void* vcache,
+                                       const void* mask, int64_t mask_ld, const void* kv_len_dev, void* out, int64_t B,
+                                       int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes,
+                                       tppx_stream_t stream) {
+  const char* who = "tppx_attn_decode_append";
+  TPPX_REQUIRE(q && k && v && pos && kcache && vcache && kv_len_dev && out, TPPX_EINVAL, "%s: null pointer", who);
+  TPPX_REQUIRE(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(kcache) && aligned16(vcache) && aligned16(out),
+               TPPX_EINVAL, "%s: pointer not 16-byte aligned", who);
+  TPPX_REQUIRE(H != 128, TPPX_EUNSUPPORTED, "%s: 128-wide heads have kernels of their own", who);
+  TPPX_REQUIRE(B > 0 && Nq > 0 && Nkv > 0 && Nq % Nkv == 0 && Smax > 0 && B * Nq < (1 << 30) && (B_pos == 1 || B_pos == B),
+               TPPX_ESHAPE, "%s: bad shape B=%ld Nq=%ld Nkv=%ld Smax=%ld B_pos=%ld", who, (long)B, (long)Nq, (long)Nkv,
+               (long)Smax, (long)B_pos);
+  TPPX_REQUIRE(!emb_pos || (HR > 0 && HR <= H && HR % 16 == 0 && MP > 0), TPPX_ESHAPE,
+               "%s: rotary_dim=%ld must be a multiple of 16 and <= H=%ld", who, (long)HR, (long)H);
+  TPPX_REQUIRE(ws_bytes >= 0 && (ws_bytes == 0 || ws), TPPX_EINVAL, "%s: workspace size given with a null workspace", who);
+  AttnGenParams g;
+  memset(&g, 0, sizeof(g));
+  g.q = (const uint16_t*)q; g.kc = (const uint16_t*)kcache; g.vc = (const uint16_t*)vcache; g.mask = (const uint16_t*)mask;
+  g.kv_len = (const int32_t*)kv_len_dev; g.kv_len_add = 1; g.out = (uint16_t*)out;
+  g.B = (int)B; g.S = 1; g.Nq = (int)Nq; g.Nkv = (int)Nkv; g.H = (int)H; g.Smax = (int)Smax; g.mask_ld = (int)mask_ld;
+  g.scale = 1.0f / sqrtf((float)H);
+  g.k_new = (const uint16_t*)k; g.v_new = (const uint16_t*)v; g.emb = (const float*)emb_pos; g.pos = (const int64_t*)pos;
+  g.MP = (int)MP; g.HR = emb_pos ? (int)HR : 0; g.B_pos = (int)B_pos; g.gptj = gptj != 0;
+  return attn_generic_launch(who, g, (hipStream_t)stream, ws, ws_bytes);
 }
 
 extern "C" int tppx_attn_prefill(const void* q, const void* kcache, const void* vcache, const void* mask,

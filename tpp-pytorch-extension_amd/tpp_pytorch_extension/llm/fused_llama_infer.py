@@ -240,13 +240,24 @@ def rotate_append_attend(q, k, v, t_am, t_pid, cache, layer_idx, B, S, Nq, Nkv, 
     (fused_llm_infer.cpp:784-789, 1025-1027, 1252-1257): rotary embedding on q and k in place (style "llama":
     rotate-half with a [2][MP][HR] cos / sin table; "gptj": adjacent pairs with a [MP][HR] sin | cos table; None:
     no rotation, OPT), append of the S new keys and values at the cache length (LayerCache::update, attn.h:198-222),
-    attention over the cached and the new keys (attn<T>, attn.cpp:781-955).  Returns the context [B][S][Nq*H]."""
+    attention over the cached and the new keys (attn<T>, attn.cpp:781-955).  Returns the context [B][S][Nq*H].  Decode
+    steps of heads that are not 128 wide do all three in one launch and leave q and k as they are."""
     L = _lib.lib()
     st = _lib.stream_of(q)
     kc, vc = cache._ensure(layer_idx, B, Nkv, H, q.device)
     ws = _lib.workspace(q)
     mask_ptr = t_am.data_ptr() if t_am is not None and t_am.numel() else None
     mask_ld = t_am.shape[-1] if mask_ptr else 0
+    if S == 1 and FUSE_ROTARY and H != 128:
+        ctx = torch.empty_like(q)
+        table, MP, HR = (None, 1, H) if style is None else (t_EP.data_ptr(), *t_EP.shape[-2:])
+        rc = L.tppx_attn_decode_append(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), table, style == "gptj", t_pid.data_ptr(), t_pid.shape[0], MP, HR,
+            kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld, cache.seq_len_dev.data_ptr(), ctx.data_ptr(), B, Nq, Nkv, H,
+            cache.capacity, ws.data_ptr(), ws.numel(), st)
+        if rc != _lib.EUNSUPPORTED:  # (head sizes past 256, the kernel switched off)
+            _lib.check(rc)
+            return ctx
     if style == "gptj":
         _lib.check(L.tppx_rotary_kv_append_gptj(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), t_EP.data_ptr(), t_pid.data_ptr(), kc.data_ptr(), vc.data_ptr(),

@@ -151,7 +151,8 @@ def ptr(t):
 
 
 def stream_of(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # (the handle alone: torch.cuda.current_stream() makes a Stream object around it, 1.5 us of an eager call's 13)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 WORKSPACE_BYTES = 32 << 20

@@ -504,11 +504,18 @@ def _prep_post(t, M, N, name, dev):
     return t.contiguous()
 
 
+def _qint8_buffer(x, M, K, qbs):
+    """(buffer, address of the int8 rows, address of their scales): one allocation for both."""
+    rows = (M + 63) // 64 * 64  # the library may lay the quantized rows out in 64-row operand tiles
+    buf = torch.empty(rows * K + rows * (K // qbs) * 4, dtype=torch.uint8, device=x.device)
+    return buf, buf.data_ptr(), buf.data_ptr() + rows * K
+
+
 def _qint8_scratch(x, M, K, qbs):
-    # the library may lay the quantized rows out in 64-row operand tiles
-    xq = torch.empty(((M + 63) // 64 * 64, K), dtype=torch.int8, device=x.device)
-    sa = torch.empty(((M + 63) // 64 * 64, K // qbs), dtype=torch.float32, device=x.device)
-    return xq, sa
+    """The same as two tensors."""
+    buf = _qint8_buffer(x, M, K, qbs)[0]
+    rows = (M + 63) // 64 * 64
+    return buf[:rows * K], buf[rows * K:]
 
 
 # Opt-in (TPPX_ACT_FP8=1, or flags=FLAG_ACT_FP8 on linear()): MXFP4 GEMMs with more than 64 rows quantize their
@@ -804,8 +811,8 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
     if PACKED_CODES and M <= 64 and layout[0] in ("qint4", "qint2") and weight.block_size == 256 \
             and row_sumsq is None and not (flags & ~_lib.FLAG_XQ_REUSE):
         qp, sp, bits = weight.native_packed()
-        xq, sa = _qint8_scratch(x, M, K, 256) if M > 16 else (None, None)
-        rc = L.tppx_linear_qintx(x.data_ptr(), _lib.ptr(xq), _lib.ptr(sa), qp.data_ptr(), sp.data_ptr(), _lib.ptr(bias),
+        _buf, xq, sa = _qint8_buffer(x, M, K, 256) if M > 16 else (None, None, None)
+        rc = L.tppx_linear_qintx(x.data_ptr(), xq, sa, qp.data_ptr(), sp.data_ptr(), _lib.ptr(bias),
                                  _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N, K, bits, post, post_scale,
                                  flags, _lib.stream_of(x))
         if rc != _lib.EUNSUPPORTED:  # rows that do not fit the in-kernel quantisation fall through to the int8 tiles
@@ -828,8 +835,8 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
                                        post, post_scale, flags, ws.data_ptr(), ws.numel(), st))
     else:
         qbs = weight.block_size
-        xq, sa = _qint8_scratch(x, M, K, qbs)
-        _lib.check(L.tppx_linear_qint8(x.data_ptr(), xq.data_ptr(), sa.data_ptr(), qn.data_ptr(),
+        _buf, xq, sa = _qint8_buffer(x, M, K, qbs)
+        _lib.check(L.tppx_linear_qint8(x.data_ptr(), xq, sa, qn.data_ptr(),
                                        sn.data_ptr(), _lib.ptr(bias), _lib.ptr(post_in),
                                        _lib.ptr(post_in2), y.data_ptr(), M, N, K, qbs, post,
                                        post_scale, flags, ws.data_ptr(), ws.numel(), st))
@@ -1058,11 +1065,15 @@ def qkv_gemm(input, weights, biases, norm=None):
         return outs
     segs = (_lib.Seg * n)()
     outs, keep = [], []
+    lead = tuple(input.shape[:-1])
     for i, w in enumerate(weights):
-        xi, Mi, Ni, Ki = _prep_input(input, w)
+        kind, Ni, Ki = w.weight_layout()
+        if kind is None:
+            raise TppxError(_lib.EUNSUPPORTED, f"Unsupported qscheme / layout for a linear weight: {w!r}")
+        _lib.require_gpu(w.qdata, "weight")
         if w._qscheme != scheme or Ki != K or w.block_size != weights[0].block_size:
             raise TppxError(_lib.ESHAPE, "Fused QKV weight block mismatch")
-        y = torch.empty(tuple(input.shape[:-1]) + (Ni,), dtype=torch.bfloat16, device=x.device)
+        y = torch.empty(lead + (Ni,), dtype=torch.bfloat16, device=x.device)
         b = _prep_bias(biases[i], Ni, x.device)
         qn, sn = w.native()
         keep.append((b, qn, sn))
@@ -1090,8 +1101,8 @@ def qkv_gemm(input, weights, biases, norm=None):
         _lib.check(L.tppx_multi_linear_mxfp4(x.data_ptr(), segs, n, M, K, fl, ws.data_ptr(), ws.numel(), st))
     else:
         qbs = weights[0].block_size
-        xq, sa = _qint8_scratch(x, M, K, qbs)
-        _lib.check(L.tppx_multi_linear_qint8(x.data_ptr(), xq.data_ptr(), sa.data_ptr(), segs, n, M, K,
+        _buf, xq, sa = _qint8_buffer(x, M, K, qbs)
+        _lib.check(L.tppx_multi_linear_qint8(x.data_ptr(), xq, sa, segs, n, M, K,
                                              qbs, 0, ws.data_ptr(), ws.numel(), st))
     return outs
 
@@ -1128,8 +1139,8 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
             y = torch.empty(tuple(input.shape[:-1]) + (N,), dtype=torch.bfloat16, device=x.device)
             bg, bu = _prep_bias(b_gate, N, x.device), _prep_bias(b_up, N, x.device)
             (qg, sg), (qu, su) = w_gate.native(), w_up.native()
-            xq, sa = _qint8_scratch(x, M, K, 256)
-            rc = L.tppx_swiglu_qint8(x.data_ptr(), xq.data_ptr(), sa.data_ptr(), qg.data_ptr(), sg.data_ptr(), _lib.ptr(bg),
+            _buf, xq, sa = _qint8_buffer(x, M, K, 256)
+            rc = L.tppx_swiglu_qint8(x.data_ptr(), xq, sa, qg.data_ptr(), sg.data_ptr(), _lib.ptr(bg),
                                      qu.data_ptr(), su.data_ptr(), _lib.ptr(bu), y.data_ptr(), M, N, K, 256, 0,
                                      _lib.stream_of(x))
             if rc != _lib.EUNSUPPORTED:

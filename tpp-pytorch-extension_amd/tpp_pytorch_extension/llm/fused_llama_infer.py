@@ -245,7 +245,7 @@ def rotate_append_attend(q, k, v, t_am, t_pid, cache, layer_idx, B, S, Nq, Nkv, 
     L = _lib.lib()
     st = _lib.stream_of(q)
     kc, vc = cache._ensure(layer_idx, B, Nkv, H, q.device)
-    ws = _lib.workspace(q)
+    ws = _lib.workspace(q, st)
     mask_ptr = t_am.data_ptr() if t_am is not None and t_am.numel() else None
     mask_ld = t_am.shape[-1] if mask_ptr else 0
     if S == 1 and FUSE_ROTARY and H != 128:
@@ -413,7 +413,7 @@ class LlamaDecoderLayer(FormatSwitches):
         q, k, v = _ops.qkv_gemm(t_HS, [Wq, Wk, Wv], [self.t_Bq, self.t_Bk, self.t_Bv],
                                 norm=(self.t_Gi, self.eps, sums_in))
         kc, vc = cache._ensure(self.layer_idx, B, self.Nkv, self.H, t_HS.device)
-        ws = _lib.workspace(t_HS)
+        ws = _lib.workspace(t_HS, st)
         mask_ptr = t_am.data_ptr() if t_am is not None and t_am.numel() else None
         mask_ld = t_am.shape[-1] if mask_ptr else 0
         if S == 1 and FUSE_ROTARY and self.H == 128 and self.t_EP.shape[2] == 128:

@@ -405,9 +405,10 @@ int tppx_swiglu_mxfp4(const void* x, const void* qw_gate, const void* sw_gate,
 
 /* Unquantized bf16 weights: several over one activation (q/k/v), or the gate/up pair with
  * y = silu(gate) * up and the rounding points of fc_silu followed by fc_mul,
- * as ONE launch of the large-M kernel (segs[i].sw is not used; it repeats
- * segs[i].qw).  TPPX_EUNSUPPORTED where one tppx_linear_bf16 per weight is the
- * way: few rows, operands of 4 GiB and more. */
+ * as ONE launch (segs[i].sw is not used; it repeats segs[i].qw): of the decode
+ * kernel up to 64 rows, of the large-M kernel beyond.  TPPX_EUNSUPPORTED where
+ * one tppx_linear_bf16 per weight is the way: more than 64 rows that are still
+ * the decode kernels', operands of 4 GiB and more. */
 int tppx_multi_linear_bf16(const void* x, const tppx_seg* segs, int n_segs,
                            int64_t M, int64_t K, int flags,
                            tppx_stream_t stream);

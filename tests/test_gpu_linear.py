@@ -989,6 +989,29 @@ def test_prefill_bf16_groups_agree_with_single_launches(M, shape, monkeypatch):
     assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws, bs), got))
 
 
+# rows around the row groups (16, 32, 64), one K tile and fewer than a workgroup has waves, widths that take one, two and three
+# channel tiles per workgroup, the last of a GEMM ragged
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("shape", [((4112, 16, 48, 80), 128), ((4096, 4096, 4096), 256), ((5136, 5120), 640), ((1056, 64, 96), 2176)])
+def test_decode_bf16_groups_agree_with_single_launches(M, shape):
+    """q/k/v (a fourth with its GELU) and the gate/up pair on unquantized bf16 weights as one launch of the decode kernel:
+    the bits of one launch per weight, which other tests hold against the oracle."""
+    ops = _ops()
+    widths, K = shape
+    ws = [block_bf16(randn_bf16((n, K), 0.05, 1750 + i)).cuda() for i, n in enumerate(widths)]
+    bs = [randn_bf16((widths[0],), 0.5, 1755).cuda()] + [None] * (len(widths) - 1)
+    wu = block_bf16(randn_bf16((widths[0], K), 0.05, 1756)).cuda()
+    x = randn_bf16((M, K), 1.0, 1757).cuda()
+    got = ops._bf16_group(x, ws, bs)
+    pair = ops._bf16_group(x, [ws[0], wu], [bs[0], None], pair=True)
+    assert got is not None and pair is not None
+    for i, (w, b) in enumerate(zip(ws, bs)):
+        assert torch.equal(got[i], ops.linear(x, w, b, O.POST_GELU if i == 3 else O.POST_NONE)), i
+    assert torch.equal(pair, ops.fc_mul(x, wu, None, ops.fc_silu(x, ws[0], bs[0])))
+    want = x.double() @ randn_bf16((widths[1], K), 0.05, 1751).cuda().double().t()
+    assert ((got[1].double() - want).norm() / want.norm()).item() < 2.0 ** -8
+
+
 @pytest.mark.parametrize("tile,w8", [(1, 1), (2, 1), (2, 0), (3, 1), (4, 1)])
 @pytest.mark.parametrize("M,N,K", [(65, 160, 128), (129, 544, 256), (300, 544, 384), (200, 1056, 640)])
 def test_prefill_bf16_every_workgroup_tile_ragged(tile, w8, M, N, K, monkeypatch):

@@ -308,6 +308,9 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
   return tiled_us <= (double)rows64 * (5.0 + (double)tiles * 16.0 * (double)K / 5.5e6 + (double)K * 0.0004);
 }
 
+// Unquantized bf16 weights, by channel tiles per workgroup (three: fitted to 33 .. 64 rows of K = 2560 and 4096)
+static constexpr RowsCost BF16_ROWS[3] = {{1.98, 1.14, 1.73, 0.561}, {1.96, 1.97, 2.15, 1.2}, {2.0, 5.3, 2.2, 1.1}};
+
 // Unquantized bf16 weights: n of them as one launch of the large-M kernel against one decode launch each.  Both sides fitted with
 // weights that come from memory: 2304 x 10496 at 82 rows 39 us on the decode kernels (tiles 55), 1024 x 5120 twice at 160 rows 25
 // as two decode launches (one of the tiles 29), 4096 x 4096 at 128 rows 22 (27), at 200 rows 41 (24).  A near tie goes to the tiles:
@@ -317,13 +320,12 @@ static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tile
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
     return family == BY_TILES;
-  static constexpr RowsCost ROWS[2] = {{1.98, 1.14, 1.73, 0.561}, {1.96, 1.97, 2.15, 1.2}};
   const int64_t rows64 = (M + 63) / 64;
   int64_t all = 0;
   double rows = 0.0;
   for (int i = 0; i < n; i++) {
     const int nt = tiles[i] > 512 ? 2 : 1;
-    rows += rows_us(ROWS[nt - 1], (tiles[i] + nt - 1) / nt * rows64, M, K);
+    rows += rows_us(BF16_ROWS[nt - 1], (tiles[i] + nt - 1) / nt * rows64, M, K);
     all += tiles[i];
   }
   if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
@@ -757,6 +759,36 @@ extern "C" int tppx_linear_mxfp4(const void* x, const void* qw, const void* sw,
   return run_mxfp4("tppx_linear_mxfp4", x, &s, 1, M, K, flags, false, ws, ws_bytes, (hipStream_t)stream);
 }
 
+// bf16 weights on the decode kernels: the GEMMs of p.seg, or the gate/up pair, in one launch.  A launch per weight rounds each
+// up to whole rounds of 256 workgroups and pays its start and its drain: q/k/v of 3 x 4096 x 4096 at one row 21.7 -> 19.3 us,
+// 3584 + 2 x 512 channels of 3584 16.6 -> 8.9, with a fourth of 16384 48.8 -> 42.9; pair 2 x 11008 x 4096 43.0 -> 32.7, at 64
+// rows 63.7 -> 44.9 (6.5 TB/s: 27.7).
+static int run_bf16_rows(const char* who, DecodeParams& p, bool dual, hipStream_t stream) {
+  p.units = p.K / 128;
+  p.tpb = 1;
+  p.S = 1;
+  const int mg = p.M <= 16 ? 1 : (p.M <= 32 ? 2 : 4);
+  // Channel tiles per workgroup (dual: one of each GEMM).  One GEMM of up to 16 rows, or of more than 64: two once one each
+  // still leaves two rounds.  Else the fewest rounds, weighed by what a round takes (one: 1; measured up to 32 rows, M > 32 as
+  // fitted above; three spill registers up to 16 rows): 640 tiles of K = 2560 at 64 rows 23.3 / 21.4 / 15.6 us with 1 / 2 / 3,
+  // 768 tiles of K = 4096 at 17 rows 20.0 / 22.8 / 27.4, 288 of 3584 12.1 / 10.0 / 12.0.
+  int nt = dual || p.total_tiles <= 512 ? 1 : 2;
+  if (!dual && p.M <= 64 && (p.n_seg > 1 || p.M > 16)) {
+    static constexpr RowsCost UP_TO_32[3] = {{0, 1.0, 0, 0}, {0, 1.7, 0, 0}, {0, 2.7, 0, 0}};
+    double best = 1e30;
+    for (int n = 1; n <= (mg == 1 ? 2 : 3); n++) {
+      set_groups(p, n, false);
+      const double us = rows_us(mg == 4 ? BF16_ROWS[n - 1] : UP_TO_32[n - 1], p.groups, p.M, p.K);
+      if (us < best) {
+        best = us;
+        nt = n;
+      }
+    }
+  }
+  set_groups(p, nt, dual);
+  return check_hip(launch_skinny_bf16(p, mg, nt, dual, stream), who);
+}
+
 extern "C" int tppx_linear_bf16(const void* x, const void* w, const void* bias, const void* post_in,
                                 const void* post_in2, void* y, int64_t M, int64_t N, int64_t K, int post_op,
                                 float post_scale, int flags, tppx_stream_t stream) {
@@ -776,23 +808,17 @@ extern "C" int tppx_linear_bf16(const void* x, const void* w, const void* bias, 
   p.x = x;
   p.M = (int)M;
   p.K = (int)K;
-  p.units = (int)(K / 128);
-  p.tpb = 1;
-  p.S = 1;
   // more than 64 rows: the LDS-tiled kernel once it is the cheaper one
   const int64_t tiles = p.total_tiles;
   if (want_tiled_bf16(M, K, flags, &tiles, 1)) {
     TPPX_REQUIRE(aligned16(w), TPPX_EINVAL, "%s: weight not 16-byte aligned", who);
     return check_hip(launch_tiled_bf16(tiled_from_seg(p, 0), (hipStream_t)stream), who);
   }
-  const int mg = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-  const int nt = p.total_tiles > 512 ? 2 : 1; // two channel tiles per workgroup once one each still leaves two rounds
-  set_groups(p, nt, false);
-  return check_hip(launch_skinny_bf16(p, mg, nt, (hipStream_t)stream), who);
+  return run_bf16_rows(who, p, false, (hipStream_t)stream);
 }
 
-// n unquantized bf16 weights over one activation, or the gate/up pair, as one large-M launch; TPPX_EUNSUPPORTED where
-// one launch per weight is the way (few rows, operands of 4 GiB and more)
+// n unquantized bf16 weights over one activation, or the gate/up pair, in one launch; TPPX_EUNSUPPORTED where one launch per
+// weight is the way (beyond 64 rows: fewer than the large-M kernel wants, operands of 4 GiB and more)
 static int run_bf16_group(const char* who, const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,
                           bool dual, hipStream_t stream) {
   int rc = check_common(who, x, M, K, n_segs, flags, nullptr, 0);
@@ -821,7 +847,10 @@ static int run_bf16_group(const char* who, const void* x, const tppx_seg* segs, 
       t[i].post_op = TPPX_POST_NONE;
     group = group && tiled_bf16_takes_groups(t[i]);
   }
-  group = group && want_tiled_bf16(M, K, flags, tiles, n_segs);
+  const bool want = want_tiled_bf16(M, K, flags, tiles, n_segs);
+  if (!want && M <= 64)
+    return run_bf16_rows(who, p, dual, stream);
+  group = group && want;
   TPPX_REQUIRE(group, TPPX_EUNSUPPORTED, "%s: M=%ld runs as one launch per weight", who, (long)M);
   return check_hip(launch_tiled_bf16_group(t, n_segs, stream, dual), who);
 }

@@ -158,7 +158,7 @@ hipError_t launch_skinny_w4a8_mg(DecodeParams& p, bool ascending, hipStream_t st
 // xq mt * 16 * K bytes, sa mt * 16 * K / 32 floats
 hipError_t launch_quant_act_w4a8_rows(const void* x, int64_t M, int64_t K, int mt, void* xq, float* sa, hipStream_t stream);
 hipError_t launch_skinny_mxfp4_nk(DecodeParams& p, hipStream_t stream);
-hipError_t launch_skinny_bf16(DecodeParams& p, int mg, int nt, hipStream_t stream);
+hipError_t launch_skinny_bf16(DecodeParams& p, int mg, int nt, bool dual, hipStream_t stream);
 size_t skinny_mxfp4_xl_lds(int units, int nt, bool dual);
 hipError_t launch_skinny_mxfp4_x4(DecodeParams& p, int nt, bool dual, hipStream_t stream);
 hipError_t launch_skinny_mxfp4_mg(DecodeParams& p, int mg, int nt, bool dual, hipStream_t stream);

@@ -2429,10 +2429,10 @@ skinny_mxfp4_mg_kernel(const DecodeParams p) {
   skinny_rows_body<false, MG, NT, DUAL, rows_waves(MG), rows_in_pairs(false, MG)>(p);
 }
 
-template <int MG, int NT>
+template <int MG, int NT, bool DUAL>
 __global__ void __launch_bounds__(rows_waves(MG) * 64)
 skinny_bf16_kernel(const DecodeParams p) {
-  skinny_rows_body<true, MG, NT, false, rows_waves(MG), rows_in_pairs(true, MG)>(p);
+  skinny_rows_body<true, MG, NT, DUAL, rows_waves(MG), rows_in_pairs(true, MG)>(p);
 }
 
 // Scale blocks that `runs` consecutive runs of `deal` tiles can touch (slots of activation scales a wave keeps in LDS).
@@ -2865,25 +2865,28 @@ hipError_t launch_skinny_mxfp4_mg(DecodeParams& p, int mg, int nt, bool dual, hi
 #undef SKMG
 }
 
-// bf16 weights: mg row groups of 16 per block row (1, 2 or 4), nt channel tiles per workgroup (1 or 2)
-hipError_t launch_skinny_bf16(DecodeParams& p, int mg, int nt, hipStream_t stream) {
+// bf16 weights: mg row groups of 16 per block row (1, 2 or 4), nt channel tiles per workgroup (1 to 3; dual: one of each GEMM)
+hipError_t launch_skinny_bf16(DecodeParams& p, int mg, int nt, bool dual, hipStream_t stream) {
   dim3 grid(p.groups, (p.M + mg * 16 - 1) / (mg * 16), 1);
   const int waves = rows_waves(mg);
-  const size_t lds = skinny_rows_lds(true, mg, nt, waves);
-#define SKBF(MG, NT) return sk_launch(skinny_bf16_kernel<MG, NT>, p, grid, waves, lds, stream)
-  if (mg == 1) {
-    if (nt == 2)
-      SKBF(1, 2);
-    SKBF(1, 1);
-  }
-  if (mg == 2) {
-    if (nt == 2)
-      SKBF(2, 2);
-    SKBF(2, 1);
-  }
-  if (nt == 2)
-    SKBF(4, 2);
-  SKBF(4, 1);
+  const size_t lds = skinny_rows_lds(true, mg, nt, waves); // the gate/up pair is reduced one half at a time
+#define SKBF(MG, NT, DUAL) return sk_launch(skinny_bf16_kernel<MG, NT, DUAL>, p, grid, waves, lds, stream)
+#define SKBF_NT(MG)      \
+  do {                   \
+    if (dual)            \
+      SKBF(MG, 1, true); \
+    if (nt == 3)         \
+      SKBF(MG, 3, false); \
+    if (nt == 2)         \
+      SKBF(MG, 2, false); \
+    SKBF(MG, 1, false);  \
+  } while (0)
+  if (mg == 1)
+    SKBF_NT(1);
+  if (mg == 2)
+    SKBF_NT(2);
+  SKBF_NT(4);
+#undef SKBF_NT
 #undef SKBF
 }
 

@@ -444,21 +444,21 @@ def _linear_bf16(input, weight, bias, post, post_in, post_in2, post_scale, flags
 
 
 def _bf16_group(input, weights, biases, pair=False):
-    """q/k/v-like GEMMs (or, pair, the gate/up pair) with unquantized bf16 weights as one launch of the large-M kernel;
-    None where one call per weight is the way (few rows, other types, shapes that call refuses)."""
+    """q/k/v-like GEMMs (or, pair, the gate/up pair) with unquantized bf16 weights as one launch: any number of them up to
+    64 rows, what the large-M kernel takes together beyond; None where one call per weight is the way."""
     if isinstance(input, QTensor) or not isinstance(input, torch.Tensor) or input.dtype != torch.bfloat16 or not input.is_cuda:
         return None
     K = input.shape[-1] if input.dim() else 0
     M = input.numel() // K if K else 0
     n = len(weights)
-    if M <= 64 or not 2 <= n <= 4 or any(not _is_plain(w) or w.dtype != torch.bfloat16 or w.device != input.device
+    if M == 0 or not 2 <= n <= 4 or any(not _is_plain(w) or w.dtype != torch.bfloat16 or w.device != input.device
                                          for w in weights):
         return None
     geo = [_blocked_geometry(w)[:2] for w in weights]
     if any(k != K for _, k in geo) or (pair and geo[0] != geo[1]):
         return None
     L = _lib.lib()
-    if not L.tppx_group_is_one_launch((ctypes.c_int64 * n)(*(N for N, _ in geo)), n, M, K, 2):
+    if M > 64 and not L.tppx_group_is_one_launch((ctypes.c_int64 * n)(*(N for N, _ in geo)), n, M, K, 2):
         return None
     x = input.contiguous()
     keep = [(_prep_bias(b, N, x.device), _bf16_native(w)) for (N, _), b, w in zip(geo, biases, weights)]

@@ -416,6 +416,22 @@ int tppx_swiglu_bf16(const void* x, const void* w_gate, const void* bias_gate,
                      const void* w_up, const void* bias_up, void* y, int64_t M,
                      int64_t N, int64_t K, int flags, tppx_stream_t stream);
 
+/* The same three with a workspace (16-byte aligned; without one K stays whole):
+ * launches of few workgroups and a long K run K in slices whose fp32 sums are
+ * added by a second launch. */
+int tppx_linear_bf16_ws(const void* x, const void* w, const void* bias,
+                        const void* post_in, const void* post_in2, void* y,
+                        int64_t M, int64_t N, int64_t K, int post_op,
+                        float post_scale, int flags, void* ws, int64_t ws_bytes,
+                        tppx_stream_t stream);
+int tppx_multi_linear_bf16_ws(const void* x, const tppx_seg* segs, int n_segs,
+                              int64_t M, int64_t K, int flags, void* ws,
+                              int64_t ws_bytes, tppx_stream_t stream);
+int tppx_swiglu_bf16_ws(const void* x, const void* w_gate, const void* bias_gate,
+                        const void* w_up, const void* bias_up, void* y,
+                        int64_t M, int64_t N, int64_t K, int flags, void* ws,
+                        int64_t ws_bytes, tppx_stream_t stream);
+
 /* The gate/up pair of QINT8-family weights as one launch behind the activation
  * quantizer (xq / sa as in tppx_linear_qint8), the same bits as fc_silu
  * followed by fc_mul.  TPPX_EUNSUPPORTED (before any launch) where one

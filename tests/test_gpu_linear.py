@@ -1049,6 +1049,55 @@ def test_prefill_bf16_every_workgroup_tile_ragged(tile, w8, M, N, K, monkeypatch
     assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws[:4], bs), got[2:]))
 
 
+# ragged rows and channel blocks, slices of unequal and of the fewest steps (four), each number of slices
+@pytest.mark.parametrize("fmt", ["mxfp4", "bf16"])
+@pytest.mark.parametrize("S,M,N,K", [(2, 65, 160, 1152), (3, 200, 288, 1792), (4, 129, 2080, 2048), (6, 100, 32, 3072), (6, 333, 416, 4224)])
+def test_prompt_gemms_with_k_in_slices(fmt, S, M, N, K, monkeypatch):
+    """K in S slices whose fp32 sums a second launch adds, in slice order: linear with its residual and bias, a post-op that
+    goes through the general epilogue, and q/k/v with a fourth GELU GEMM, against the launch with K whole (another order of
+    the fp32 sums: one bf16 ulp here and there) and a float64 product; every replay of a captured call the same."""
+    ops = _ops()
+    flat = [randn_bf16((n, K), 0.05, 1800 + i) for i, n in enumerate((N, 64, 96, 160))]
+    ws = [block_bf16(w).cuda() for w in flat]
+    if fmt == "mxfp4":
+        ws = [ops.remap_and_quantize_mxfp4(w) for w in ws]
+    x, res, b = randn_bf16((M, K), 1.0, 1805).cuda(), randn_bf16((M, N), 1.0, 1806).cuda(), randn_bf16((N,), 0.5, 1807).cuda()
+
+    def run():
+        return [ops.fc_add(x, ws[0], b, res, 0.5), ops.fc_add2(x, ws[0], b, res, res, 0.5)] + list(ops.qkv_gemm(x, ws, [b, None, None, None]))
+
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
+    monkeypatch.setenv("TPPX_TILED_SPLIT", "0")
+    want = run()
+    monkeypatch.setenv("TPPX_TILED_SPLIT", str(S))
+    got = run()
+    for i, (a, w) in enumerate(zip(got, want)):
+        a, w = a.double(), w.double()
+        assert (a - w).norm() <= 2.0 ** -9 * w.norm(), i
+        # the bf16 GEMM tile differs by one ulp, 2^-7 of it at most, and is at most |out| + 1.5 |residual|; one more ulp for
+        # each of the two roundings behind it; sums near zero by the fp32 sums' own error
+        near = w.abs() + (1.5 * res.double().abs() if i < 2 else 0.0)
+        assert ((a - w).abs() <= 3 * 2.0 ** -7 * near + 2.0 ** -12 * w.abs().max()).all(), i
+    if fmt == "mxfp4":
+        import ctypes
+        from tpp_pytorch_extension import _lib
+        buf = ctypes.create_string_buffer(4096)
+        _lib.check(_lib.lib().tppx_plan_linear_mxfp4(M, N, K, 0, 1 << 25, buf, len(buf)))
+        assert f"side_split_kernel<false> grid={(M + 63) // 64 * ((N + 127) // 128)}x{S}x1" in buf.value.decode()
+    if fmt == "bf16":
+        ref = x.double() @ flat[1].cuda().double().t()
+        assert ((got[3].double() - ref).norm() / ref.norm()).item() < 2.0 ** -8
+    y = torch.empty(0)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = ops.fc_add(x, ws[0], b, res, 0.5)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, got[0])
+
+
 @pytest.mark.parametrize("fmt", ["mxfp4", "bf16"])
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 7])
 def test_prefill_side_by_side_forms_at_every_loop_remainder(fmt, steps, monkeypatch):

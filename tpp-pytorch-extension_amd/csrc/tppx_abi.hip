@@ -270,7 +270,8 @@ static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, boo
   static constexpr RowsCost SINGLE[3] = {{3.19, 0.678, 0.958, 0.765}, {2.78, 1.82, 1.10, 0.958}, {2.35, 3.22, 1.61, 0.628}};
   static constexpr RowsCost DUAL[3] = {{2.82, 1.16, 1.14, 0.883}, {2.92, 3.4, 1.51, 0.984}, {2.42, 5.0, 2.31, 1.02}};
   static constexpr RowsCost NK = {3.24, 6.86, 0.400, 0.333};
-  const double tiled = tiled_mxfp4_us(M, K, n_tiles16);
+  // (narrower ones, which the decode kernels run well, have not been measured with K in slices)
+  const double tiled = nk && tiles >= 128 ? tiled_mxfp4_split_us(M, K, tiles, ws_bytes) : tiled_mxfp4_us(M, K, n_tiles16);
   if (nk && mxfp4_nk_fits(M, (int)tiles, (int)(K / 128), ws_bytes))
     return tiled <= rows_us(NK, (tiles + 3) / 4 * 4 * rows64, M, K);
   const int nt = tiles <= 256 ? 1 : (tiles + 1) / 2 <= 256 ? 2 : 3; // channel tiles per workgroup, as the launch picks them
@@ -316,7 +317,7 @@ static constexpr RowsCost BF16_ROWS[3] = {{1.98, 1.14, 1.73, 0.561}, {1.96, 1.97
 // as two decode launches (one of the tiles 29), 4096 x 4096 at 128 rows 22 (27), at 200 rows 41 (24).  A near tie goes to the tiles:
 // with weights at hand in the Infinity Cache, as those of one small layer or of a linear called again, they take up to a quarter
 // less (4096 x 4096 at 128 rows 18), the decode kernels hardly (21).
-static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tiles, int n) {
+static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tiles, int n, int64_t ws_bytes = 0) {
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
     return family == BY_TILES;
@@ -329,7 +330,7 @@ static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tile
     all += tiles[i];
   }
   if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
-    return tiled_bf16_us(M, K, all) <= 1.04 * rows;
+    return (n == 1 && all >= 128 ? tiled_bf16_split_us(M, K, all, ws_bytes) : tiled_bf16_us(M, K, all)) <= 1.04 * rows;
   const int64_t wgs = ((M + 127) / 128) * ((all + 7) / 8); // tiled_bf16_kernel
   return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
          (double)rows64 * (8.0 + (double)all * 32.0 * (double)K / 5.5e6 + (double)K * 0.0008);
@@ -430,6 +431,7 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
   }
   if (want_tiled_mxfp4(M, K, flags, p.total_tiles, dual, !dual && n_segs == 1 && !row_sumsq, ws_bytes)) {
     TPPX_REQUIRE(!row_sumsq, TPPX_EUNSUPPORTED, "%s: row sums of squares are not produced by the large-M kernels", who);
+    float* part = aligned16(ws) ? (float*)ws : nullptr;
     // prefill shapes: one LDS-tiled launch per GEMM of the group; the fused
     // gate/up pair becomes silu(gate) followed by up * gate (same rounding)
     if (!dual && n_segs > 1) {
@@ -440,7 +442,7 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
         group = group && tiled_mxfp4_takes_groups(t[i]);
       }
       if (group) // fused q/k/v: one grid over the channel blocks of all GEMMs
-        return check_hip(launch_tiled_mxfp4_group(t, n_segs, stream), who);
+        return check_hip(launch_tiled_mxfp4_group(t, n_segs, stream, false, part, ws_bytes), who);
     }
     if (dual && env_int("TPPX_TILED_DUAL_FUSED", 1) != 0) {
       // Gate and up in ONE launch whose workgroups own 128 output channels each and compute both projections for
@@ -449,7 +451,7 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
       TiledParams t[2] = {tiled_from_seg(p, 0), tiled_from_seg(p, 1)};
       if (tiled_mxfp4_takes_groups(t[0])) {
         t[0].post_op = t[1].post_op = TPPX_POST_NONE;
-        return check_hip(launch_tiled_mxfp4_group(t, 2, stream, true), who);
+        return check_hip(launch_tiled_mxfp4_group(t, 2, stream, true, part, ws_bytes), who);
       }
     }
     if (dual) {
@@ -476,7 +478,7 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
         t.post_op = i == 0 ? TPPX_POST_SILU : TPPX_POST_MUL;
         t.post_in = i == 0 ? nullptr : (const uint16_t*)segs[0].y;
       }
-      rc = check_hip(launch_tiled_mxfp4(t, stream), who);
+      rc = check_hip(launch_tiled_mxfp4(t, stream, part, ws_bytes), who);
       if (rc)
         return rc;
     }
@@ -789,11 +791,10 @@ static int run_bf16_rows(const char* who, DecodeParams& p, bool dual, hipStream_
   return check_hip(launch_skinny_bf16(p, mg, nt, dual, stream), who);
 }
 
-extern "C" int tppx_linear_bf16(const void* x, const void* w, const void* bias, const void* post_in,
-                                const void* post_in2, void* y, int64_t M, int64_t N, int64_t K, int post_op,
-                                float post_scale, int flags, tppx_stream_t stream) {
-  const char* who = "tppx_linear_bf16";
-  int rc = check_common(who, x, M, K, 1, flags, nullptr, 0);
+static int run_linear_bf16(const char* who, const void* x, const void* w, const void* bias, const void* post_in,
+                           const void* post_in2, void* y, int64_t M, int64_t N, int64_t K, int post_op, float post_scale,
+                           int flags, void* ws, int64_t ws_bytes, tppx_stream_t stream) {
+  int rc = check_common(who, x, M, K, 1, flags, ws, ws_bytes);
   if (rc)
     return rc;
   TPPX_REQUIRE(K > 0 && K % 128 == 0, TPPX_ESHAPE, "%s: K=%ld must be a positive multiple of 128 (native bf16 tiles span 128 input channels)", who, (long)K);
@@ -810,18 +811,30 @@ extern "C" int tppx_linear_bf16(const void* x, const void* w, const void* bias, 
   p.K = (int)K;
   // more than 64 rows: the LDS-tiled kernel once it is the cheaper one
   const int64_t tiles = p.total_tiles;
-  if (want_tiled_bf16(M, K, flags, &tiles, 1)) {
+  if (want_tiled_bf16(M, K, flags, &tiles, 1, aligned16(ws) ? ws_bytes : 0)) {
     TPPX_REQUIRE(aligned16(w), TPPX_EINVAL, "%s: weight not 16-byte aligned", who);
-    return check_hip(launch_tiled_bf16(tiled_from_seg(p, 0), (hipStream_t)stream), who);
+    return check_hip(launch_tiled_bf16(tiled_from_seg(p, 0), (hipStream_t)stream, aligned16(ws) ? (float*)ws : nullptr, ws_bytes), who);
   }
   return run_bf16_rows(who, p, false, (hipStream_t)stream);
+}
+
+extern "C" int tppx_linear_bf16(const void* x, const void* w, const void* bias, const void* post_in,
+                                const void* post_in2, void* y, int64_t M, int64_t N, int64_t K, int post_op,
+                                float post_scale, int flags, tppx_stream_t stream) {
+  return run_linear_bf16("tppx_linear_bf16", x, w, bias, post_in, post_in2, y, M, N, K, post_op, post_scale, flags, nullptr, 0, stream);
+}
+
+extern "C" int tppx_linear_bf16_ws(const void* x, const void* w, const void* bias, const void* post_in,
+                                   const void* post_in2, void* y, int64_t M, int64_t N, int64_t K, int post_op,
+                                   float post_scale, int flags, void* ws, int64_t ws_bytes, tppx_stream_t stream) {
+  return run_linear_bf16("tppx_linear_bf16_ws", x, w, bias, post_in, post_in2, y, M, N, K, post_op, post_scale, flags, ws, ws_bytes, stream);
 }
 
 // n unquantized bf16 weights over one activation, or the gate/up pair, in one launch; TPPX_EUNSUPPORTED where one launch per
 // weight is the way (beyond 64 rows: fewer than the large-M kernel wants, operands of 4 GiB and more)
 static int run_bf16_group(const char* who, const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,
-                          bool dual, hipStream_t stream) {
-  int rc = check_common(who, x, M, K, n_segs, flags, nullptr, 0);
+                          bool dual, hipStream_t stream, void* ws = nullptr, int64_t ws_bytes = 0) {
+  int rc = check_common(who, x, M, K, n_segs, flags, ws, ws_bytes);
   if (rc)
     return rc;
   TPPX_REQUIRE(segs, TPPX_EINVAL, "%s: null segment table", who);
@@ -852,7 +865,7 @@ static int run_bf16_group(const char* who, const void* x, const tppx_seg* segs, 
     return run_bf16_rows(who, p, dual, stream);
   group = group && want;
   TPPX_REQUIRE(group, TPPX_EUNSUPPORTED, "%s: M=%ld runs as one launch per weight", who, (long)M);
-  return check_hip(launch_tiled_bf16_group(t, n_segs, stream, dual), who);
+  return check_hip(launch_tiled_bf16_group(t, n_segs, stream, dual, aligned16(ws) ? (float*)ws : nullptr, ws_bytes), who);
 }
 
 extern "C" int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M, int64_t K, int weight_bytes) {
@@ -886,6 +899,19 @@ extern "C" int tppx_swiglu_bf16(const void* x, const void* w_gate, const void* b
   tppx_seg s[2] = {{w_gate, w_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
                    {w_up, w_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
   return run_bf16_group("tppx_swiglu_bf16", x, s, 2, M, K, flags, true, (hipStream_t)stream);
+}
+
+extern "C" int tppx_multi_linear_bf16_ws(const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,
+                                         void* ws, int64_t ws_bytes, tppx_stream_t stream) {
+  return run_bf16_group("tppx_multi_linear_bf16_ws", x, segs, n_segs, M, K, flags, false, (hipStream_t)stream, ws, ws_bytes);
+}
+
+extern "C" int tppx_swiglu_bf16_ws(const void* x, const void* w_gate, const void* bias_gate, const void* w_up,
+                                   const void* bias_up, void* y, int64_t M, int64_t N, int64_t K, int flags, void* ws,
+                                   int64_t ws_bytes, tppx_stream_t stream) {
+  tppx_seg s[2] = {{w_gate, w_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
+                   {w_up, w_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
+  return run_bf16_group("tppx_swiglu_bf16_ws", x, s, 2, M, K, flags, true, (hipStream_t)stream, ws, ws_bytes);
 }
 
 extern "C" int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* qw_gate, const void* sw_gate,

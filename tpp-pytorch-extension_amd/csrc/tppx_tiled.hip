@@ -50,8 +50,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tl_rsrc(const void* q) {
 // time share operand tiles in its L2.  xm = how many of the 8 rectangles lie along M (1: an XCD owns NB/8 channel
 // blocks and all row blocks; 2, 4: 1/xm of the row blocks and xm/8 of the channel blocks).  Every XCD fetches
 // 1/xm of the activations and xm/8 of the weights from memory.  The host passes an xm that divides evenly.
-__device__ __forceinline__ void tile_of_block(int MB, int NB, int& bm, int& bn, int xm = 1) {
-  int id = blockIdx.x;
+__device__ __forceinline__ void tile_of_block(int MB, int NB, int& bm, int& bn, int xm, int id) {
   const int T = MB * NB;
   if ((T & 7) == 0 && xm > 1) {
     const int x = id & 7, r = id >> 3;
@@ -67,6 +66,9 @@ __device__ __forceinline__ void tile_of_block(int MB, int NB, int& bm, int& bn, 
   id = x * (T >> 3) + min(x, T & 7) + (id >> 3);
   bm = id % MB;
   bn = id / MB;
+}
+__device__ __forceinline__ void tile_of_block(int MB, int NB, int& bm, int& bn, int xm = 1) {
+  tile_of_block(MB, NB, bm, bn, xm, blockIdx.x);
 }
 
 template <typename Acc>
@@ -613,6 +615,8 @@ struct BigParams {
   int nb0[TPPX_MAX_SEGS + 1]; // first channel block of each segment, then the total
   int n_seg;
   int xm;                     // XCD rectangles along M (see tile_of_block)
+  int S;                      // K slices (grid y) whose sums go to `part`; side_gemm_body with SPLIT
+  float* part;                // [S][workgroup][wave][MT * 2 tiles][64 lanes][4]
 };
 
 // MT = 16-row tiles per wave along M (8).
@@ -867,7 +871,7 @@ struct SideGeom {
   static constexpr size_t LDS = (size_t)PD * STAGE > EP ? (size_t)PD * STAGE : EP;
 };
 
-template <int MT, int W, int PD, bool DUAL, bool WBF16>
+template <int MT, int W, int PD, bool DUAL, bool WBF16, bool SPLIT = false>
 __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
   using G = SideGeom<MT, W, PD, WBF16>;
   constexpr int WGM = G::WGM, STAGE = G::STAGE, NA = G::NA, LB = G::LB, L = G::L;
@@ -888,7 +892,8 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
       }
   }
   bn -= nb_first;
-  const int KT = p.K >> 7, last = KT - 1;
+  // K steps k0 .. k0 + KT - 1 of KA
+  const int KA = p.K >> 7, k0 = SPLIT ? KA * (int)blockIdx.y / P.S : 0, KT = SPLIT ? KA * ((int)blockIdx.y + 1) / P.S - k0 : KA, last = KT - 1;
   const int m_wg = bm * WGM;
   const int tile_base = DUAL ? bn * W + wave : bn * (W * 2) + wave * 2; // DUAL: gate and up tile of the same 16 channels
 
@@ -897,7 +902,7 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
 #pragma unroll
   for (int i = 0; i < NA; i++) {
     const int blk = wave * NA + i, r16 = (blk & 3) * 4 + (lane >> 4);
-    aoff[i] = (uint32_t)min(m_wg + blk * 4 + (lane >> 4), p.M - 1) * (uint32_t)p.K * 2u + (uint32_t)(((lane & 15) ^ r16) & 15) * 16u;
+    aoff[i] = (uint32_t)min(m_wg + blk * 4 + (lane >> 4), p.M - 1) * (uint32_t)p.K * 2u + (uint32_t)(((lane & 15) ^ r16) & 15) * 16u + (uint32_t)k0 * 256u;
   }
   __amdgpu_buffer_rsrc_t wr[2], swr[2];
   uint32_t woff[2], swoff[2];
@@ -905,9 +910,9 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
   for (int nt = 0; nt < 2; nt++) {
     const int tile = min(DUAL ? tile_base : tile_base + nt, p.tiles - 1);
     wr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].qw : p.qw);
-    swoff[nt] = (uint32_t)tile * (uint32_t)KT * 64u + (uint32_t)lane;
+    swoff[nt] = ((uint32_t)tile * (uint32_t)KA + (uint32_t)k0) * 64u + (uint32_t)lane;
     if constexpr (WBF16) {
-      woff[nt] = ((uint32_t)tile * (uint32_t)KT * 256u + (uint32_t)lane) * 16u;
+      woff[nt] = (((uint32_t)tile * (uint32_t)KA + (uint32_t)k0) * 256u + (uint32_t)lane) * 16u;
     } else {
       woff[nt] = swoff[nt] * 16u;
       swr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].sw : p.sw);
@@ -1016,12 +1021,55 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
       step(std::false_type{}, S, s + decltype(S)::value);
   });
   unit(std::integral_constant<int, NQ - 1>{});
+  if constexpr (SPLIT) { // (as they lie in the registers: a wave instruction is 1 KiB)
+    f32x4* out = reinterpret_cast<f32x4*>(P.part) + (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * W + wave) * (MT * 2 * 64) + lane;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      out[(mt * 2) * 64] = acc[mt][0];
+      out[(mt * 2 + 1) * 64] = acc[mt][1];
+    }
+    return;
+  }
   __syncthreads(); // (waits for the loads still under way: the ring is free for the epilogue staging)
   float* stage = reinterpret_cast<float*>(tl_lds) + wave * (MT < 4 ? MT * 16 : 64) * ep_ld(2);
   if (DUAL)
     big_epilogue_dual<MT, 2>(p, P.seg[1], acc, stage, m_wg, tile_base);
   else
     big_epilogue<MT, 2>(p, acc, stage, m_wg, tile_base);
+}
+
+// The other half of a launch split along K: a workgroup of one wave per wave tile adds the S slices' sums, in their order, and
+// goes through the same epilogue.  Bound by those bytes, S * 32 KiB per 64 x 128 outputs, and the launch.
+template <int MT, int W, int S>
+__global__ void __launch_bounds__(64)
+side_sum_kernel(const BigParams P) {
+  __shared__ __align__(16) float stage[MT * 16 * ep_ld(2)];
+  const int wg = (int)blockIdx.x / W, wave = (int)blockIdx.x % W, lane = threadIdx.x;
+  const int MB = (P.seg[0].M + MT * 16 - 1) / (MT * 16), wgs = (int)gridDim.x / W;
+  int bm, bn;
+  tile_of_block(MB, P.nb0[P.n_seg], bm, bn, P.xm, wg);
+  TiledParams p = P.seg[0];
+  int nb_first = 0;
+#pragma unroll
+  for (int i = 1; i < TPPX_MAX_SEGS; i++)
+    if (i < P.n_seg && bn >= P.nb0[i]) {
+      p = P.seg[i];
+      nb_first = P.nb0[i];
+    }
+  const f32x4* in = reinterpret_cast<const f32x4*>(P.part) + ((int64_t)wg * W + wave) * (MT * 2 * 64) + lane;
+  f32x4 acc[MT][2];
+#pragma unroll
+  for (int i = 0; i < MT * 2; i++) {
+    f32x4 v[S];
+#pragma unroll
+    for (int z = 0; z < S; z++)
+      v[z] = in[(int64_t)z * wgs * W * (MT * 2 * 64) + i * 64];
+    acc[i >> 1][i & 1] = v[0];
+#pragma unroll
+    for (int z = 1; z < S; z++)
+      acc[i >> 1][i & 1] += v[z];
+  }
+  big_epilogue<MT, 2>(p, acc, stage, bm * MT * 16, (bn - nb_first) * (W * 2) + wave * 2);
 }
 
 constexpr int SIDE_PD = 3;
@@ -1033,6 +1081,17 @@ big_bf16_kernel(const BigParams P) {
     side_gemm_body<MT * WM, WM * WN, SIDE_PD, DUAL, true>(P);
   else
     big_gemm_body<MT, DUAL, WM, WN, true>(P);
+}
+
+// 64 x 128 with K in P.S slices (grid y): launches of few workgroups and a long K.  A workgroup's time is its K steps (0.45 us
+// each, MXFP4) whatever else the chip does, so 64 .. 192 of them with 86 steps leave most of it idle; three resident to a CU
+// run S times as many with an S-th of the steps.  The sums go out as they lie in the registers, 32 KiB a workgroup, and a
+// second launch adds them: with it 4096 x 11008 at 100 / 200 / 333 rows 32.3 -> 18.7 / 40.1 -> 27.5 / 42.1 -> 38.0 us, 2560 x
+// 10240 at 200 rows 36.3 -> 21.1; bf16 weights 55 -> 29, 60 -> 40, 61 -> 59 and 55 -> 28.
+template <bool WBF16>
+__global__ void __launch_bounds__(256, 2)
+side_split_kernel(const BigParams P) {
+  side_gemm_body<4, 4, SIDE_PD, false, WBF16, true>(P);
 }
 
 // ---------------------------------------------------------------------------
@@ -1818,6 +1877,53 @@ double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16) {
   return us;
 }
 
+// K slices (1: whole) of a launch of n GEMMs that takes whole_us without them, *us: what it takes then.  The 64 x 128 tile's
+// estimate for S times the workgroups and an S-th of the steps, and the slices' sums out and in: 2.2 us and 8.5 .. 16.5 ns
+// (MXFP4, the more the shorter K is) or 11.5 ns (bf16 weights) for each 32 KiB of them.  Measured at 65 .. 800 rows of
+// 2560 .. 4096 channels and K = 2560 .. 16384 with 2, 3, 4, 6 and 8 slices: within 10 % but for the shortest K, where it is up to
+// 2 us low: up to K = 2560 (11.5 us whole, 11.3 in slices at 65 rows), MXFP4 4096 (17 whole, 15 .. 22), no launch is split.  Up to
+// one round of whole-K workgroups (bf16: a quarter more); 3 % for the estimate's sake.
+template <bool WBF16>
+static int best_split(int64_t M, int64_t K, const int* tiles, int n, int64_t part_bytes, double whole_us, double* us) {
+  const int forced = env_int("TPPX_TILED_SPLIT", 1);
+  int64_t nb = 0, all = 0;
+  for (int i = 0; i < n; i++) {
+    nb += (tiles[i] + 7) / 8;
+    all += tiles[i];
+  }
+  const int64_t wgs = (M + 63) / 64 * nb;
+  const double s = (double)K / 128.0, mb = (double)(all * 32 * K) * 1e-6;
+  const double ns = WBF16 ? 11.5 : 16.5 - 8.0 * std::min(1.0, std::max(0.0, (s - 32.0) / 48.0));
+  int best = 1;
+  double best_us = 0.97 * whole_us;
+  for (int S : {2, 3, 4, 6}) {
+    if (wgs * S * 32768 > part_bytes || K / 128 < 4 * S)
+      break;
+    const double c = tile_us((WBF16 ? BF16_COST : MXFP4_COST)[TILE_64_128], TILE_64_128, wgs * S, s / S, mb, false) + 2.2 + ns * 1e-3 * (double)(wgs * S);
+    if (forced == S || (forced == 1 && K > (WBF16 ? 2560 : 4096) && wgs <= (WBF16 ? 320 : 256) && c < best_us)) {
+      best_us = c;
+      best = S;
+    }
+  }
+  if (us && best > 1)
+    *us = best_us;
+  return best;
+}
+
+// the same for one GEMM of n_tiles16 channel tiles with room for the slices' sums
+double tiled_mxfp4_split_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes) {
+  const int tiles = (int)n_tiles16;
+  double us = tiled_mxfp4_us(M, K, n_tiles16);
+  best_split<false>(M, K, &tiles, 1, part_bytes, us, &us);
+  return us;
+}
+double tiled_bf16_split_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes) {
+  const int tiles = (int)n_tiles16;
+  double us = tiled_bf16_us(M, K, n_tiles16);
+  best_split<true>(M, K, &tiles, 1, part_bytes, us, &us);
+  return us;
+}
+
 static bool big_fits(const TiledParams& p) {
   return (int64_t)p.M * p.K * 2 < ((int64_t)1 << 32) && (int64_t)p.tiles * 8 * p.K < ((int64_t)1 << 32);
 }
@@ -1855,12 +1961,17 @@ static hipError_t big_bf16_launch(const BigParams& P, int wgs, hipStream_t strea
   return big_go(big_bf16_kernel<MT, DUAL, WM, WN>, P, wgs, WM * WN * 64, lds, stream);
 }
 
-template <typename Us>
-static int cheapest_tile(const TiledParams* t, int n, bool dual, unsigned allowed, Us&& us) {
+// S: K slices of the 64 x 128 tile, 1 where K stays whole
+template <bool WBF16, typename Us>
+static int cheapest_tile(const TiledParams* t, int n, bool dual, unsigned allowed, Us&& us, int64_t part_bytes, int* S) {
   int tiles[TPPX_MAX_SEGS];
   for (int i = 0; i < n; i++)
     tiles[i] = t[i].tiles;
-  return cheapest_tile(t[0].M, t[0].K, tiles, n, dual, allowed, us);
+  double best;
+  const int shape = cheapest_tile(t[0].M, t[0].K, tiles, n, dual, allowed, us, &best);
+  if (!dual && part_bytes > 0 && (allowed >> TILE_64_128 & 1u))
+    *S = best_split<WBF16>(t[0].M, t[0].K, tiles, n, part_bytes, best, nullptr);
+  return *S > 1 ? TILE_64_128 : shape;
 }
 
 // fills P for n GEMMs over one activation with this workgroup tile; returns the workgroups of the launch
@@ -1887,18 +1998,45 @@ static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int 
   return MB * nb;
 }
 
+template <bool WBF16>
+static hipError_t side_split_launch(BigParams& P, int wgs, int S, float* part, hipStream_t stream) {
+  P.S = S;
+  P.part = part;
+  const size_t lds = SideGeom<4, 4, SIDE_PD, WBF16>::LDS;
+  const auto kern = side_split_kernel<WBF16>;
+  auto gemm = [&]() -> hipError_t {
+    TPPX_PLAN_ONLY(kern, dim3(wgs, S), dim3(256), lds);
+    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds); e != hipSuccess)
+      return e;
+    kern<<<dim3(wgs, S), dim3(256), lds, stream>>>(P);
+    return hipGetLastError();
+  };
+  if (hipError_t e = gemm(); e != hipSuccess)
+    return e;
+  auto sum = [&](auto add) -> hipError_t {
+    TPPX_PLAN_ONLY(add, dim3(wgs * 4), dim3(64), 0);
+    add<<<dim3(wgs * 4), dim3(64), 0, stream>>>(P);
+    return hipGetLastError();
+  };
+  return S == 2 ? sum(side_sum_kernel<4, 4, 2>) : S == 3 ? sum(side_sum_kernel<4, 4, 3>) : S == 4 ? sum(side_sum_kernel<4, 4, 4>)
+                                                                                          : sum(side_sum_kernel<4, 4, 6>);
+}
+
 // dual: t[0] = gate, t[1] = up (equal shapes, n == 2); y[m][n] = silu(gate) * up goes to t[1].y
-hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
+hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual, float* part, int64_t part_bytes) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
   bool scales4 = true;
   for (int i = 0; i < n; i++)
     scales4 = scales4 && (reinterpret_cast<uintptr_t>(t[i].sw) & 3u) == 0;
   int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
+  int S = 1;
   if (shape < 0 || shape > TILE_128_128 || (shape == TILE_128_128 && !scales4))
-    shape = cheapest_tile(t, n, dual, mxfp4_tiles(scales4), mxfp4_tile_us);
+    shape = cheapest_tile<false>(t, n, dual, mxfp4_tiles(scales4), mxfp4_tile_us, part ? part_bytes : 0, &S);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, MXFP4_WEIGHT_BYTES);
+  if (S > 1)
+    return side_split_launch<false>(P, wgs, S, part, stream);
   switch (shape) {
   case TILE_128_512:
     return dual ? big_launch<8, true, 1, 8>(P, wgs, stream) : big_launch<8, false, 1, 8>(P, wgs, stream);
@@ -1961,9 +2099,9 @@ hipError_t launch_tiled_mxfp4_fp8_group(const TiledParams* t, int n, hipStream_t
   return dual ? fp8_launch<8, true>(P, MB8 * nb, stream) : fp8_launch<8, false>(P, MB8 * nb, stream);
 }
 
-hipError_t launch_tiled_mxfp4(const TiledParams& p, hipStream_t stream) {
+hipError_t launch_tiled_mxfp4(const TiledParams& p, hipStream_t stream, float* part, int64_t part_bytes) {
   if (tiled_mxfp4_takes_groups(p))
-    return launch_tiled_mxfp4_group(&p, 1, stream);
+    return launch_tiled_mxfp4_group(&p, 1, stream, false, part, part_bytes);
   const int MB = (p.M + 127) / 128, NB = (p.tiles + 7) / 8;
   const size_t lds = 2 * 2048 * 16;
   TPPX_PLAN_ONLY(tiled_mxfp4_kernel, dim3(MB * NB), dim3(256), lds);
@@ -2001,14 +2139,17 @@ bool tiled_bf16_takes_groups(const TiledParams& p) {
 
 // n GEMMs over one activation in one launch (fuller last rounds: q/k/v of 4096 channels at 2048 rows 207 -> 167 us), or
 // the gate/up pair (dual, as launch_tiled_mxfp4_group: 11008 x 4096 at 2048 rows 355 -> 310 us, 333 rows 148 -> 96)
-hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
+hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual, float* part, int64_t part_bytes) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
   int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 .. 4 as in launch_tiled_mxfp4_group, 6 = 64 x 256; 5 is not built for 2-byte weights
+  int S = 1;
   if (shape < 0 || shape >= N_TILES || shape == TILE_128_128)
-    shape = cheapest_tile(t, n, dual, bf16_tiles(), bf16_tile_us);
+    shape = cheapest_tile<true>(t, n, dual, bf16_tiles(), bf16_tile_us, part ? part_bytes : 0, &S);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 2.0);
+  if (S > 1)
+    return side_split_launch<true>(P, wgs, S, part, stream);
   switch (shape) {
   case TILE_128_512:
     return dual ? big_bf16_launch<8, true, 1, 8>(P, wgs, stream) : big_bf16_launch<8, false, 1, 8>(P, wgs, stream);
@@ -2025,9 +2166,9 @@ hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stre
   }
 }
 
-hipError_t launch_tiled_bf16(const TiledParams& p, hipStream_t stream) {
+hipError_t launch_tiled_bf16(const TiledParams& p, hipStream_t stream, float* part, int64_t part_bytes) {
   if (tiled_bf16_takes_groups(p))
-    return launch_tiled_bf16_group(&p, 1, stream, false);
+    return launch_tiled_bf16_group(&p, 1, stream, false, part, part_bytes);
   const int MB = (p.M + 127) / 128, NB = (p.tiles + 7) / 8;
   const dim3 grid((unsigned)(MB * NB));
   const size_t lds = 2 * 2048 * 16;

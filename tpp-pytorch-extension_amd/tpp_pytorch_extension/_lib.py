@@ -66,6 +66,9 @@ SIGNATURES = {
     "tppx_prepack_bf16": [_vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp],
     "tppx_linear_bf16": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _f32, _i32, _vp],
     "tppx_multi_linear_bf16": [_vp, ctypes.POINTER(Seg), _i32, _i64, _i64, _i32, _vp],
+    "tppx_linear_bf16_ws": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _f32, _i32, _vp, _i64, _vp],
+    "tppx_multi_linear_bf16_ws": [_vp, ctypes.POINTER(Seg), _i32, _i64, _i64, _i32, _vp, _i64, _vp],
+    "tppx_swiglu_bf16_ws": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp, _i64, _vp],
     "tppx_group_is_one_launch": [ctypes.POINTER(_i64), _i32, _i64, _i64, _i32],
     "tppx_swiglu_qint8": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp],
     "tppx_swiglu_bf16": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],

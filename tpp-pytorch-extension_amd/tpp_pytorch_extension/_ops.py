@@ -437,10 +437,22 @@ def _linear_bf16(input, weight, bias, post, post_in, post_in2, post_scale, flags
     post_in = _prep_post(post_in, M, N, "post-op input", x.device)
     post_in2 = _prep_post(post_in2, M, N, "second post-op input", x.device)
     nat = _bf16_native(weight)
-    _lib.check(_lib.lib().tppx_linear_bf16(x.data_ptr(), nat.data_ptr(), _lib.ptr(bias), _lib.ptr(post_in),
-                                           _lib.ptr(post_in2), y.data_ptr(), M, N, K, post, post_scale, flags,
-                                           _lib.stream_of(x)))
+    st = _lib.stream_of(x)
+    ws = _bf16_ws(x, M, st)
+    _lib.check(_lib.lib().tppx_linear_bf16_ws(x.data_ptr(), nat.data_ptr(), _lib.ptr(bias), _lib.ptr(post_in),
+                                              _lib.ptr(post_in2), y.data_ptr(), M, N, K, post, post_scale, flags,
+                                              _lib.ptr(ws), _lib.WORKSPACE_BYTES if M > 64 else 0, st))
     return y
+
+
+def _bf16_ws(x, M, st):
+    """Workspace for the K slices of prompt launches, None for decode steps.  A capture gets one from its own pool: replays
+    of different graphs need no order between them."""
+    if M <= 64:
+        return None
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(_lib.WORKSPACE_BYTES, dtype=torch.uint8, device=x.device)
+    return _lib.workspace(x, st)
 
 
 def _bf16_group(input, weights, biases, pair=False):
@@ -463,10 +475,13 @@ def _bf16_group(input, weights, biases, pair=False):
     x = input.contiguous()
     keep = [(_prep_bias(b, N, x.device), _bf16_native(w)) for (N, _), b, w in zip(geo, biases, weights)]
     lead = tuple(input.shape[:-1])
+    st = _lib.stream_of(x)
+    ws = _bf16_ws(x, M, st)
+    ws_ptr, ws_bytes = _lib.ptr(ws), _lib.WORKSPACE_BYTES if M > 64 else 0
     if pair:
         y = torch.empty(lead + (geo[0][0],), dtype=torch.bfloat16, device=x.device)
-        rc = L.tppx_swiglu_bf16(x.data_ptr(), keep[0][1].data_ptr(), _lib.ptr(keep[0][0]), keep[1][1].data_ptr(),
-                                _lib.ptr(keep[1][0]), y.data_ptr(), M, geo[0][0], K, 0, _lib.stream_of(x))
+        rc = L.tppx_swiglu_bf16_ws(x.data_ptr(), keep[0][1].data_ptr(), _lib.ptr(keep[0][0]), keep[1][1].data_ptr(),
+                                   _lib.ptr(keep[1][0]), y.data_ptr(), M, geo[0][0], K, 0, ws_ptr, ws_bytes, st)
     else:
         y = [torch.empty(lead + (N,), dtype=torch.bfloat16, device=x.device) for N, _ in geo]
         segs = (_lib.Seg * n)()
@@ -477,7 +492,7 @@ def _bf16_group(input, weights, biases, pair=False):
             segs[i].N = geo[i][0]
             segs[i].post_op = POST_GELU if (n == 4 and i == 3) else POST_NONE
             segs[i].post_scale = 1.0
-        rc = L.tppx_multi_linear_bf16(x.data_ptr(), segs, n, M, K, 0, _lib.stream_of(x))
+        rc = L.tppx_multi_linear_bf16_ws(x.data_ptr(), segs, n, M, K, 0, ws_ptr, ws_bytes, st)
     if rc == _lib.EUNSUPPORTED:
         return None
     _lib.check(rc)

@@ -1098,6 +1098,28 @@ def test_prompt_gemms_with_k_in_slices(fmt, S, M, N, K, monkeypatch):
         assert torch.equal(y, got[0])
 
 
+@pytest.mark.parametrize("S,M,N,K", [(2, 65, 160, 512), (2, 200, 288, 1792), (3, 129, 2080, 1792), (4, 100, 32, 2304), (6, 333, 416, 3328)])
+def test_prompt_qint8_gemms_with_k_in_slices(S, M, N, K, monkeypatch):
+    """QINT8 the same: K in S slices of whole scale blocks (one block a slice, an odd and an even number), against the oracle
+    to the tolerance of the launch with K whole."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")
+    monkeypatch.setenv("TPPX_TILED_SPLIT", str(S))
+    buf = ctypes.create_string_buffer(4096)
+    _lib.check(_lib.lib().tppx_plan_linear_qint8(M, N, K, 256, 1, 0, 1 << 25, buf, len(buf)))
+    assert f"big_qint8_split_kernel grid={(M + 63) // 64 * ((N + 127) // 128)}x{S}x1" in buf.value.decode()
+    y, _, _, ctx = _run("qint8", M, N, K, "add", True, 1900 + M)  # (checks against the oracle)
+    qw, _, _, x, bias, in1, in2, scale = ctx
+    other = _make("qint8", 64, K, 1901)[0]
+    q, k2 = ops.qkv_gemm(x.cuda(), [qw, other], [bias.cuda(), None])
+    monkeypatch.setenv("TPPX_TILED_SPLIT", "0")
+    for got, want in ((y, ops.linear(x.cuda(), qw, bias.cuda(), O.POST_ADD_SCALE, in1.cuda(), None, scale)),
+                      (q, ops.fc_plain(x.cuda(), qw, bias.cuda())), (k2, ops.fc_plain(x.cuda(), other, None))):
+        assert (got.double() - want.double()).norm() <= 2.0 ** -9 * want.double().norm()
+
+
 @pytest.mark.parametrize("fmt", ["mxfp4", "bf16"])
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 7])
 def test_prefill_side_by_side_forms_at_every_loop_remainder(fmt, steps, monkeypatch):

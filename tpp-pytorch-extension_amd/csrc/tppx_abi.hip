@@ -279,7 +279,7 @@ static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, boo
 }
 
 // QINT8.  `tiles` of the whole launch (dual: the gate/up pair, of both projections).
-static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, bool dual, int64_t qbs) {
+static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, bool dual, int64_t qbs, int64_t ws_bytes = 0) {
   const int family = kernel_family(M, flags);
   if (family != BY_COST)
     return family == BY_TILES;
@@ -300,7 +300,9 @@ static bool want_tiled_qint8(int64_t M, int64_t K, int flags, int64_t tiles, boo
     const int nt = tiles < 512 ? 1 : tiles > 512 && tiles <= 768 ? 3 : 2; // as plan_skinny
     const double k = 1e-3 * (double)K, wgs = (double)(rows64 * ((tiles + 7) / 8)), mk = 1e-6 * (double)M * (double)K;
     static constexpr RowsCost ROWS[3] = {{5.06, 2.34, 1.30, 0}, {4.9, 3.96, 1.6, 0}, {5.5, 4.25, 2.3, 0}};
-    return 6.07 + k * (3.01 + 0.668 * wgs / 256.0) + 0.257 * mk <=
+    // (in S slices a step of K counts once for S of them, and their sums go out and in: high by up to 5 us at 2560 channels)
+    const int S = tiles >= 160 ? qint8_split(M, K, (tiles + 7) / 8, ws_bytes) : 1;
+    return 6.07 + k / S * (3.01 + 0.668 * wgs * S / 256.0) + 0.257 * mk + (S > 1 ? 2.0 + 0.02 * wgs * S : 0.0) <=
            1.04 * (rows_us(ROWS[nt - 1], (tiles + nt - 1) / nt * rows64, M, K) + (nt == 1 ? 0.1 : 0.8) * mk);
   }
   const int64_t wgs = ((M + 127) / 128) * ((tiles + 15) / 16);
@@ -576,7 +578,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
   p.units = (int)(K / (64 * p.deal));
   p.spb_magic = (p.deal == 4 && p.tpb > 4) ? (unsigned int)((((uint64_t)1 << 32) + (uint64_t)(p.tpb / 4) - 1) / (uint64_t)(p.tpb / 4)) : 0u;
   const bool reuse = (flags & TPPX_FLAG_XQ_REUSE) != 0; // xq / sa still hold this x, quantized by an earlier call
-  const bool tiled = qbs % 128 == 0 && want_tiled_qint8(M, K, flags, (dual ? 2 : 1) * (int64_t)p.total_tiles, dual, qbs);
+  const bool tiled = qbs % 128 == 0 && want_tiled_qint8(M, K, flags, (dual ? 2 : 1) * (int64_t)p.total_tiles, dual, qbs, n_segs == 1 && aligned16(ws) ? ws_bytes : 0);
   TiledParams t[TPPX_MAX_SEGS];
   bool group = tiled && n_segs > 1; // one grid over the channel blocks of all GEMMs when the large-M kernel takes them
   for (int i = 0; i < n_segs && tiled; i++) {
@@ -592,9 +594,9 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
         return rc;
     }
     if (group)
-      return check_hip(launch_tiled_qint8_group(t, n_segs, stream, dual), who);
+      return check_hip(launch_tiled_qint8_group(t, n_segs, stream, dual, aligned16(ws) ? (float*)ws : nullptr, ws_bytes), who);
     for (int i = 0; i < n_segs; i++) {
-      rc = check_hip(launch_tiled_qint8(t[i], stream), who);
+      rc = check_hip(launch_tiled_qint8(t[i], stream, aligned16(ws) ? (float*)ws : nullptr, ws_bytes), who);
       if (rc)
         return rc;
     }

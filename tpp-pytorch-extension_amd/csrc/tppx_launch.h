@@ -114,7 +114,7 @@ bool tiled_mxfp4_takes_groups(const TiledParams& p);
 // dual: the gate/up pair (t[0] = gate, t[1] = up) with silu(gate) * up formed in the launch and written to t[1].y
 hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual = false, float* part = nullptr,
                                     int64_t part_bytes = 0);
-hipError_t launch_tiled_qint8(const TiledParams& p, hipStream_t stream);
+hipError_t launch_tiled_qint8(const TiledParams& p, hipStream_t stream, float* part = nullptr, int64_t part_bytes = 0);
 // unquantized bf16 weights (native bf16 tiles in p.qw), more than 64 rows
 hipError_t launch_tiled_bf16(const TiledParams& p, hipStream_t stream, float* part = nullptr, int64_t part_bytes = 0);
 double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16);
@@ -123,7 +123,10 @@ hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stre
                                    int64_t part_bytes = 0);
 hipError_t launch_tiled_mxfp4_fp8_group(const TiledParams* t, int n, hipStream_t stream, bool dual = false);
 bool tiled_qint8_takes_groups(const TiledParams& p);
-hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t stream, bool dual = false);
+// K slices of a launch of nb blocks of 128 channels, with that much workspace for their sums
+int qint8_split(int64_t M, int64_t K, int64_t nb, int64_t part_bytes);
+hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t stream, bool dual = false, float* part = nullptr,
+                                    int64_t part_bytes = 0);
 // y[i] = bf16( silu(gate[i]) * y[i] ) with the rounding points of SiluPostOp followed by MulPostOp; n % 8 == 0
 hipError_t launch_silu_mul(const uint16_t* gate, uint16_t* y, int64_t n, hipStream_t stream);
 

@@ -1335,7 +1335,7 @@ struct Qint8Geom {
   static constexpr size_t LDS = (size_t)NB * STAGE > EP ? (size_t)NB * STAGE : EP;
 };
 
-template <int MT, int W, bool DUAL>
+template <int MT, int W, bool DUAL, bool SPLIT = false>
 __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
   using G = Qint8Geom<MT, W>;
   constexpr int WGM = G::WGM, NB = G::NB, NA = G::NA, LA = G::LA, LB = G::LB, STAGE = G::STAGE;
@@ -1356,7 +1356,8 @@ __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
       }
   }
   bn -= nb_first;
-  const int KS = p.K >> 8;
+  // K steps k0 .. k0 + KS - 1 of KA
+  const int KA = p.K >> 8, k0 = SPLIT ? KA * (int)blockIdx.y / P.S : 0, KS = SPLIT ? KA * ((int)blockIdx.y + 1) / P.S - k0 : KA;
   const int m_wg = bm * WGM;
   const int tile_base = DUAL ? bn * W + wave : bn * (W * 2) + wave * 2; // DUAL: gate and up tile of the same 16 channels
 
@@ -1365,10 +1366,10 @@ __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
 #pragma unroll
   for (int i = 0; i < NA; i++) {
     const int blk = wave * NA + i, r16 = (blk & 3) * 4 + (lane >> 4);
-    aoff[i] = (uint32_t)min(m_wg + blk * 4 + (lane >> 4), p.M - 1) * (uint32_t)p.K + (uint32_t)(((lane & 15) ^ r16) & 15) * 16u;
+    aoff[i] = (uint32_t)min(m_wg + blk * 4 + (lane >> 4), p.M - 1) * (uint32_t)p.K + (uint32_t)(((lane & 15) ^ r16) & 15) * 16u + (uint32_t)k0 * 256u;
   }
   const int sp = wave % (WGM / 64);
-  const uint32_t saoff = (uint32_t)(min(m_wg + sp * 64 + lane, p.M - 1) * KS) * 4u;
+  const uint32_t saoff = (uint32_t)(min(m_wg + sp * 64 + lane, p.M - 1) * KA + k0) * 4u;
   auto load_a = [&](auto I, int s, int buf) {
     constexpr int i = decltype(I)::value;
     uint8_t* base = tl_lds + buf * STAGE;
@@ -1384,8 +1385,8 @@ __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
     const int tile = min(DUAL ? tile_base : tile_base + nt, p.tiles - 1);
     wr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].qw : p.qw);
     swr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].sw : p.sw);
-    woff[nt] = ((uint32_t)tile * (uint32_t)(KS * 4) * 64u + (uint32_t)lane) * 16u;
-    swoff[nt] = (uint32_t)(tile * KS * 16 + (lane & 15)) * 4u;
+    woff[nt] = (((uint32_t)tile * (uint32_t)KA + (uint32_t)k0) * 256u + (uint32_t)lane) * 16u;
+    swoff[nt] = (uint32_t)((tile * KA + k0) * 16 + (lane & 15)) * 4u;
   }
   i32x4 b[2][4][2]; // [set][j][nt]
   float swv[2][2];
@@ -1500,12 +1501,27 @@ __device__ __forceinline__ void big_qint8_body(const BigParams& P) {
   if (s < KS)
     step(std::integral_constant<int, 0>{}, s);
   fold(std::integral_constant<int, NG - 1>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 16>{}, swp);
+  if constexpr (SPLIT) { // (as they lie in the registers: a wave instruction is 1 KiB)
+    f32x4* out = reinterpret_cast<f32x4*>(P.part) + (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * W + wave) * (MT * 2 * 64) + lane;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      out[(mt * 2) * 64] = facc[mt][0];
+      out[(mt * 2 + 1) * 64] = facc[mt][1];
+    }
+    return;
+  }
   __syncthreads(); // (waits for the loads still under way: the ring is free for the epilogue staging)
   float* stage = reinterpret_cast<float*>(tl_lds) + wave * (MT < 4 ? MT * 16 : 64) * ep_ld(2);
   if (DUAL)
     big_epilogue_dual<MT, 2>(p, P.seg[1], facc, stage, m_wg, tile_base);
   else
     big_epilogue<MT, 2>(p, facc, stage, m_wg, tile_base);
+}
+
+// 64 x 128 with K in P.S slices (grid y), as side_split_kernel
+__global__ void __launch_bounds__(256, 2)
+big_qint8_split_kernel(const BigParams P) {
+  big_qint8_body<4, 4, false, true>(P);
 }
 
 __global__ void __launch_bounds__(512, 2)
@@ -1998,12 +2014,11 @@ static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int 
   return MB * nb;
 }
 
-template <bool WBF16>
-static hipError_t side_split_launch(BigParams& P, int wgs, int S, float* part, hipStream_t stream) {
+// kern: 64 x 128 workgroups of four waves with K in S slices; part: S * wgs * 32 KiB
+template <typename Kern>
+static hipError_t split_launch(Kern kern, size_t lds, BigParams& P, int wgs, int S, float* part, hipStream_t stream) {
   P.S = S;
   P.part = part;
-  const size_t lds = SideGeom<4, 4, SIDE_PD, WBF16>::LDS;
-  const auto kern = side_split_kernel<WBF16>;
   auto gemm = [&]() -> hipError_t {
     TPPX_PLAN_ONLY(kern, dim3(wgs, S), dim3(256), lds);
     if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds); e != hipSuccess)
@@ -2036,7 +2051,7 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, MXFP4_WEIGHT_BYTES);
   if (S > 1)
-    return side_split_launch<false>(P, wgs, S, part, stream);
+    return split_launch(side_split_kernel<false>, SideGeom<4, 4, SIDE_PD, false>::LDS, P, wgs, S, part, stream);
   switch (shape) {
   case TILE_128_512:
     return dual ? big_launch<8, true, 1, 8>(P, wgs, stream) : big_launch<8, false, 1, 8>(P, wgs, stream);
@@ -2149,7 +2164,7 @@ hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stre
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 2.0);
   if (S > 1)
-    return side_split_launch<true>(P, wgs, S, part, stream);
+    return split_launch(side_split_kernel<true>, SideGeom<4, 4, SIDE_PD, true>::LDS, P, wgs, S, part, stream);
   switch (shape) {
   case TILE_128_512:
     return dual ? big_bf16_launch<8, true, 1, 8>(P, wgs, stream) : big_bf16_launch<8, false, 1, 8>(P, wgs, stream);
@@ -2193,9 +2208,22 @@ bool tiled_qint8_takes_groups(const TiledParams& p) {
          (int64_t)p.M * p.K < ((int64_t)1 << 32) && (int64_t)p.tiles * 16 * p.K < ((int64_t)1 << 32);
 }
 
+// K slices (1: whole) of a QINT8 launch of nb blocks of 128 channels: as many as leave one round of 64 x 128 workgroups, for
+// K from 6144 on (4096 x 4096: whole 17.0 us, in slices 16.7 .. 20) and slices of 1536 and more.  4096 x 11008, quantizer included:
+// 100 rows (64 workgroups, 4 slices) 40.4 -> 25.1 us, 200 rows (128, 2) 42.3 -> 32.0, 333 rows (192) whole 43.3, in slices
+// 45 .. 50; 2560 x 10240: 100 rows (40, 6) 33.4 -> 18.2, 333 rows (120, 2) 33.9 -> 27.5; 4096 x 16384 at 100 rows 53.4 -> 32.2.
+int qint8_split(int64_t M, int64_t K, int64_t nb, int64_t part_bytes) {
+  const int forced = env_int("TPPX_TILED_SPLIT", 1);
+  const int64_t wgs = (M + 63) / 64 * nb;
+  for (int S : {6, 4, 3, 2})
+    if (wgs * S * 32768 <= part_bytes && (forced == S ? K / 256 >= S : forced == 1 && K >= 6144 && K >= 1536 * S && wgs * S <= 256))
+      return S;
+  return 1;
+}
+
 // n GEMMs over the same quantised activations (same M, K, xq, sa) in one launch of the large-M kernel
 // dual: t[0] = gate, t[1] = up, as in launch_tiled_mxfp4_group
-hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t stream, bool dual) {
+hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t stream, bool dual, float* part, int64_t part_bytes) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].xq != t[1].xq))
     return hipErrorInvalidValue;
   BigParams P;
@@ -2223,6 +2251,11 @@ hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t str
     P.n_seg = n;
     return nb;
   };
+  if (!dual && part) {
+    const int nb = channel_blocks(4), S = qint8_split(t[0].M, t[0].K, nb, part_bytes);
+    if (S > 1)
+      return split_launch(big_qint8_split_kernel, Qint8Geom<4, 4>::LDS, P, (t[0].M + 63) / 64 * nb, S, part, stream);
+  }
   const int64_t wgs64 = (int64_t)((t[0].M + 63) / 64) * channel_blocks(8); // workgroups of 64 x 256
   const bool small = env_int("TPPX_TILED_SMALL", 1) != 0;
   if (small && wgs64 <= 128) { // up to half the CUs: 64 x 128, twice as many, one round (4096 x 4096 at 333 rows 19.6 -> 15.0 us, at
@@ -2237,9 +2270,9 @@ hipError_t launch_tiled_qint8_group(const TiledParams* t, int n, hipStream_t str
   return dual ? go(big_qint8_dual_kernel, 128, 8, Qint8Geom<8, 8>::LDS) : go(big_qint8_kernel, 128, 8, Qint8Geom<8, 8>::LDS);
 }
 
-hipError_t launch_tiled_qint8(const TiledParams& p, hipStream_t stream) {
+hipError_t launch_tiled_qint8(const TiledParams& p, hipStream_t stream, float* part, int64_t part_bytes) {
   if (tiled_qint8_takes_groups(p))
-    return launch_tiled_qint8_group(&p, 1, stream);
+    return launch_tiled_qint8_group(&p, 1, stream, false, part, part_bytes);
   const int MB = (p.M + 127) / 128, NB = (p.tiles + 7) / 8;
   const size_t lds = 2 * 1024 * 16 + 2 * 128 * sizeof(float);
   TPPX_PLAN_ONLY(tiled_qint8_kernel, dim3(MB * NB), dim3(256), lds);

@@ -668,6 +668,33 @@ def test_w4a8_row_groups_equal_the_oracle_from_64_rows(M, N, K, bc, post):
     assert torch.equal(ops.linear(xg, qt, bg, posts[post], in1, in2, 0.5), want)
 
 
+# workgroups of one channel tile (at most 512 of 64 rows) and of two (33 x 16 of 64 rows; 37 tiles: the last one alone),
+# K tiles: less than a step of four, whole steps, a remainder behind them
+@pytest.mark.parametrize("M,N,K,bc", [(64, 48, 384, 64), (130, 272, 1024, 128), (1024, 528, 640, 32), (960, 592, 1920, 64),
+                                      (40, 272, 640, 64)])
+def test_w4a8_row_groups_of_any_weight_scale(M, N, K, bc):
+    """The row-group kernels start their integer sums from a float's bits where the weight scales of the K tiles at hand
+    lie between 2^-126 and 1, and convert and scale them otherwise: weights with blocks of scales from 2 up, of the
+    smallest ones and of zeros between ordinary ones equal the oracle (from 64 rows) or the two-step path."""
+    ops = _ops()
+    W = randn_bf16((N, K), 0.05, 3400 + M)
+    W[1, :32] *= 1000
+    W[N - 1, K - 32:] *= 30000
+    W[N // 2, 96:160] *= 1e-37
+    W[N // 2, K - 64:K - 32] *= 300
+    W[3, 64:96] = 0.0
+    t = W.view(N // 16, 16, K // bc, bc // 2, 2).permute(0, 2, 3, 1, 4).contiguous()
+    q_or, s_or = O.remap_quantize_mxfp4_int8(t.float().numpy())
+    assert s_or.min() == 0 and s_or.max() > 127
+    qt = ops.remap_and_quantize_mxfp4(t.cuda(), int8_layout=True)
+    x, b = randn_bf16((M, K), 1.0, 3410 + M), randn_bf16((N,), 0.1, 3420)
+    y = _w4a8_mid(qt, x.cuda(), b.cuda(), O.POST_NONE, None, None, 1.0)
+    if M >= 64:
+        assert np.array_equal(t2bits(y), O.linear_w4a8(t2bits(x), q_or, s_or, bc, t2bits(b)))
+    else:
+        assert torch.equal(y, _w4a8_two_steps(qt, x.cuda(), b.cuda(), O.POST_NONE, None, None, 1.0))
+
+
 @pytest.mark.parametrize("off", [1, 4])
 @pytest.mark.parametrize("M", [17, 40, 63])
 def test_w4a8_takes_rows_at_any_address(M, off):

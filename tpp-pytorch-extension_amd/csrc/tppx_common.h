@@ -128,14 +128,15 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // W4A8 (USE_MXFP4_INT8): the integer the reference multiplies for an E2M1 code = its value times 127 / 6, rounded
-// four 4-bit E2M1 codes (one per byte, bits 0..3) -> four int8 values
+// four 4-bit E2M1 codes (one per byte, the upper four bits clear) -> four int8 values {0 11 21 32 42 64 85 127} with sign.
+// Two byte permutes look up all sixteen codes: selector bytes 0..7 pick a table byte (0..3 from the second operand, 4..7
+// from the first), 8..11 give the sign of the pair's bytes 1, 3, 5, 7 in every bit, 12 zero, 13..15 0xFF.  So the first
+// lookup is a constant (0 or 0xFF) for codes 8..15 and the second one, on the code with its sign bit flipped, for codes
+// 0..7; the other table's bytes are stored with that constant folded in, and the exclusive or of the two is the value
+// (four instructions; a lookup of the magnitude, one of its negative and a select by the sign bit are eight).
 __device__ __forceinline__ uint32_t w4a8_expand(uint32_t codes) {
-  const uint32_t sel = codes & 0x07070707u;
-  // v_perm_b32: selector bytes 0..3 pick from the second operand, 4..7 from the first
-  const uint32_t pos = __builtin_amdgcn_perm(0x7F55402Au, 0x20150B00u, sel); // 0 11 21 32 | 42 64 85 127
-  const uint32_t neg = __builtin_amdgcn_perm(0x81ABC0D6u, 0xE0EBF500u, sel); // the same, negated
-  const uint32_t m = ((codes >> 3) & 0x01010101u) * 0xFFu;                   // 0xFF in the bytes with the sign bit
-  return (neg & m) | (pos & ~m);
+  return __builtin_amdgcn_perm(0x80AABF2Au, 0x20150BFFu, codes) ^
+         __builtin_amdgcn_perm(0x7E543FD6u, 0x1F14F500u, codes ^ 0x08080808u);
 }
 
 } // namespace tppx

@@ -1633,43 +1633,38 @@ skinny_w4a8_kernel(const DecodeParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// W4A8 between the kernel above and the prompt passes.  The rows arrive quantised in operand order
-// (quant_act_w4a8_rows_kernel): xq [K/128][mt][2 halves][64 lanes (g, m)][16 B], 8 bytes of each of two MX blocks per
-// lane, and scales sa [K/128][mt][16 m][4 blocks] f32, already times 6 / 127.  Weight tiles and their E8M0 dwords as in
-// skinny_w4a8_kernel.  The weights are the MFMA's FIRST operand, so a result tile is [channel][row]: a lane's four sums
-// belong to one row, whose four block scales of a K tile are one 16-byte load, and no scale goes through LDS.
-// A wave owns ONE channel tile, MG row tiles and one of KP parts of K; a workgroup T channel tiles and MG * R row tiles.
-//   KP = 4  the parts are linear_w4a8_kernel's, contiguous quarters of the MX blocks (a quarter may begin and end inside
-//           a K tile: its first and last tile skip the blocks outside), each folded in ascending order, added in part
-//           order and to the bias: that kernel's bits
-//   KP = 1  all of K in ascending order on top of the bias: the prompt kernel's (and the oracle's) bits
-// What bounds it: vector issue.  Every K = 32 MFMA (one MX block) leaves 4 sums per lane to convert, scale and add
-// (12 instructions) behind the expansion of the codes (about 18, shared by the wave's MG row tiles); the weight stream
-// hides behind that from 32 rows on.  Whole calls, quantizer included, weights from memory, in us, and in brackets the
-// kernel with the same bits (32 and 63 rows: the two-step path; from 64 rows: the prompt kernel):
-//   rows     4096 x 4096    11008 x 4096    4096 x 11008    3584 x 18944
-//   32       10 (35)        17 (52)         17 (63)         25 (104)
-//   63       13 (43)        24 (79)         23 (81)         35 (142)
-//   64       16 (38)        28 (47)         33 (94)         58 (152)
-//   128      23 (38)        39 (47)         52 (94)         82 (153)
-//   256      31 (39)        68 (67)         70 (93)         111 (151)
+// W4A8, 17 to 63 rows.  The rows arrive quantised in operand order (quant_act_w4a8_rows_kernel): xq [K/128][mt]
+// [2 halves][64 lanes (g, m)][16 B], 8 bytes of each of two MX blocks per lane, and scales sa [K/128][mt][16 m][4 blocks]
+// f32, already times 6 / 127.  Weight tiles and their E8M0 dwords as in skinny_w4a8_kernel.  The weights are the MFMA's
+// FIRST operand, so a result tile is [channel][row]: a lane's four sums belong to one row, whose four block scales of a K
+// tile are one 16-byte load, and no scale goes through LDS.
+// A wave owns one channel tile, MG row tiles and one of KP = 4 parts of K; a workgroup MG * R row tiles of one channel
+// tile.  The parts are linear_w4a8_kernel's, contiguous quarters of the MX blocks (a quarter may begin and end inside a K
+// tile: its first and last tile skip the blocks outside), each folded in ascending order, added in part order and to the
+// bias: that kernel's bits, except that a whole tile rounds once less where a product of two scales is subnormal (below).
+// What bounds it: vector issue in chains that few waves hide.  Every K = 32 MFMA (one MX block) leaves 4 sums per lane to
+// take off their start and to add (8 instructions; 12 where they are converted and scaled) behind the expansion of the
+// codes (11, shared by the wave's MG row tiles).  Two projections of 11008 x 4096 and one of 4096 x 11008 with their
+// quantizers, weights from memory: 32 rows 50.4 -> 49.2 us, 50 rows 67.5 -> 63.3 from a conversion per sum, an 18
+// instruction expansion and no order between the MFMAs and the folds.  (Weights four tiles ahead instead of two: 50.8 at
+// 32 rows; four row tiles per wave at 50 rows: 73; the expansion shared by the row tiles through LDS as in the kernel
+// below: 46 / 60 us at 32 rows of these / 3584 x 16128 where this one takes 49 / 57, and 70 at 50 rows.)
 // ---------------------------------------------------------------------------
-template <int MG, int T, int R, int KP, int PF>
-__global__ void __launch_bounds__(KP * T * R * 64)
+template <int MG, int R, int PF>
+__global__ void __launch_bounds__(4 * R * 64)
 skinny_w4a8_mg_kernel(const DecodeParams p) {
-  static_assert(KP == 1 || KP == 4, "K parts");
+  constexpr int KP = 4;
   extern __shared__ __align__(16) float sk_lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kp = wave % KP, rr = (wave / KP) % R, tt = wave / (KP * R);
+  const int kp = wave % KP, rr = wave / KP;
   const DecodeSeg& sg = p.seg[0];
-  const int ltile0 = blockIdx.x * T;
   const int m0 = blockIdx.y * (MG * R * 16);
   const int KT = p.units; // K tiles of 128 channels
   // MX blocks b0 .. b1 - 1 in K tiles t0 .. t1 - 1; `first`: where the first tile begins, `last`: where the last one ends
-  const int b0 = KP == 1 ? 0 : kp * KT, b1 = KP == 1 ? 4 * KT : b0 + KT;
+  const int b0 = kp * KT, b1 = b0 + KT;
   const int t0 = b0 >> 2, t1 = (b1 + 3) >> 2, first = b0 & 3, last = ((b1 - 1) & 3) + 1;
 
-  const int64_t lt = min(ltile0 + tt, sg.tiles - 1); // ragged last group: duplicate, not stored
+  const int64_t lt = blockIdx.x;
   const i32x4* wq = reinterpret_cast<const i32x4*>(sg.qw) + lt * KT * 64;
   const i32x4* ws = reinterpret_cast<const i32x4*>(sg.sw) + lt * KT * 4; // E8M0 dwords of four channels
   const int rt0 = (int)blockIdx.y * (MG * R) + rr * MG; // first row tile of this wave
@@ -1694,63 +1689,80 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
   for (int i = 0; i < PF; i++)
     load(i, t0 + i);
   __builtin_amdgcn_sched_barrier(0);
-  SkEpilogue<MG * R, T, false, KP * T * R, KP * T * R> ep; // KP == 4
-  uint16_t in1[MG][4], in2[MG][4];                         // KP == 1
+  SkEpilogue<MG * R, 1, false, KP * R, KP * R> ep;
   f32x4 facc[MG];
 #pragma unroll
   for (int mg = 0; mg < MG; mg++)
     facc[mg] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if constexpr (KP == 1) {
-    // (an absent input is read from the output, as in SkEpilogue::prefetch_flat: no branch around a load)
-    const uint16_t* pb = sg.bias ? sg.bias : sg.y;
-    const uint16_t* p1 = sg.post_in ? sg.post_in : sg.y;
-    const uint16_t* p2 = sg.post_in2 ? sg.post_in2 : sg.y;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int n = (int)lt * 16 + (lane >> 4) * 4 + r;
-      const uint32_t b = pb[n];
-#pragma unroll
-      for (int mg = 0; mg < MG; mg++) {
-        const int o = min(m0 + (rr * MG + mg) * 16 + (lane & 15), p.M - 1) * sg.N + n;
-        in1[mg][r] = p1[o];
-        in2[mg][r] = p2[o];
-        facc[mg][r] = sg.bias ? bf16_bits_to_f32(b) : 0.f;
-      }
-    }
-  } else {
-    ep.prefetch_flat(p, sg, ltile0, m0);
-  }
+  ep.prefetch_flat(p, sg, blockIdx.x, m0);
   __builtin_amdgcn_sched_barrier(0);
 
-  auto block = [&](int i, auto J) {
-    constexpr int j = decltype(J)::value;
+  auto weights = [&](int i, int j) {
     const uint32_t codes = (uint32_t)wreg[i][j];
     const uint32_t lo = w4a8_expand(codes & 0x0F0F0F0Fu), hi = w4a8_expand((codes >> 4) & 0x0F0F0F0Fu);
-    const long wb = (long)(((uint64_t)hi << 32) | lo);
+    return (long)(((uint64_t)hi << 32) | lo);
+  };
+  auto rows = [&](int i, int mg, int j) {
+    return (long)(((uint64_t)(uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2 + 1] << 32) |
+                  (uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2]);
+  };
+  auto block = [&](int i, int j) {
+    const long wb = weights(i, j);
     float wsc[4];
 #pragma unroll
     for (int r = 0; r < 4; r++)
       wsc[r] = e8m0_to_f32((uint32_t)sreg[i][r] >> (8 * j));
 #pragma unroll
     for (int mg = 0; mg < MG; mg++) {
-      const long xa = (long)(((uint64_t)(uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2 + 1] << 32) |
-                             (uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2]);
-      const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, xa, i32x4{0, 0, 0, 0}, 0, 0, 0);
+      const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, rows(i, mg, j), i32x4{0, 0, 0, 0}, 0, 0, 0);
       const float sav = areg[i][mg][j];
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        facc[mg][r] = KP == 1 ? fmaf((float)acc[r] * wsc[r], sav, facc[mg][r])
-                              : fmaf((float)acc[r], sav * wsc[r], facc[mg][r]); // (the roundings of the kernel it equals)
+        facc[mg][r] = fmaf((float)acc[r], sav * wsc[r], facc[mg][r]);
     }
   };
+  // A whole K tile whose weight scales are all below 2 (E8M0 bytes 1 .. 127; 0 is a scale of zero in every W4A8 kernel).
+  // The MFMA starts from the BITS of
+  // 1.5 * 2^(23 + e), whose last place is 2^e: an integer sum (below 2^19) added to them leaves the float
+  // 1.5 * 2^(23 + e) + sum * 2^e, and taking the start off again, which is exact, leaves sum * 2^e without a conversion
+  // or a multiplication.  The MFMAs of a block go out ahead of the fold of the block before it.
+  auto whole_tile = [&](int i) {
+    i32x4 start[2], acc[2][MG];
+    auto issue = [&](auto J) {
+      constexpr int j = decltype(J)::value;
+      const long wb = weights(i, j);
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        start[j & 1][r] = (int)((((uint32_t)sreg[i][r] >> (8 * j)) & 0xffu) << 23) + 0x0BC00000;
+#pragma unroll
+      for (int mg = 0; mg < MG; mg++)
+        acc[j & 1][mg] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, rows(i, mg, j), start[j & 1], 0, 0, 0);
+    };
+    issue(std::integral_constant<int, 0>{});
+    static_for<0, 4>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      if constexpr (j < 3)
+        issue(std::integral_constant<int, j + 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int mg = 0; mg < MG; mg++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          facc[mg][r] = fmaf(__int_as_float(acc[j & 1][mg][r]) - __int_as_float(start[j & 1][r]), areg[i][mg][j], facc[mg][r]);
+    });
+  };
   auto consume = [&](int i, int t) {
-    const int lo = KP > 1 && t == t0 ? first : 0, hi = KP > 1 && t == t1 - 1 ? last : 4;
-    if (KP == 1 || (lo == 0 && hi == 4)) {
-      static_for<0, 4>([&](auto J) { block(i, J); });
+    const int lo = t == t0 ? first : 0, hi = t == t1 - 1 ? last : 4;
+    uint32_t any = 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      any |= (uint32_t)sreg[i][r] | ((uint32_t)sreg[i][r] - 0x01010101u); // a top bit for a byte of 0 or from 128 on
+    if (!__any((any & 0x80808080u) != 0) && lo == 0 && hi == 4) {
+      whole_tile(i);
     } else {
       static_for<0, 4>([&](auto J) {
         if (decltype(J)::value >= lo && decltype(J)::value < hi)
-          block(i, J);
+          block(i, decltype(J)::value);
       });
     }
   };
@@ -1767,22 +1779,188 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
   for (int i = 0; i < PF - 1; i++) // fewer than PF left: their tiles are in the stages a trip would use
     if (t + i < t1)
       consume(i, t + i);
-  if constexpr (KP == 1) {
-    if (ltile0 + tt >= sg.tiles)
-      return;
+  ep.template finish_parts<KP, MG>(sg, facc, sk_lds, kp, rr * MG);
+}
+
+// ---------------------------------------------------------------------------
+// W4A8 from 64 rows up to the prompt kernel: rows, scales and weight tiles as above, all of K in ascending order on top
+// of the bias -- the prompt kernel's (and the oracle's) bits, so K cannot be split.
+// A workgroup owns NT channel tiles x 64 rows, a wave NT x 16 rows.  K moves in steps of four K tiles: each wave expands
+// the codes of ONE of them (per channel tile) into LDS for all four, a step ahead of their use in the other of two
+// buffers, one barrier per step; its own rows come from the L2 into registers, a step ahead as well.  A wave's units of
+// (K tile, channel tile) are pipelined: LDS reads of the next, MFMAs of this one, fold of the last one.
+// What bounds it: vector issue, 8 instructions per four sums and block, and below 512 workgroups the chain itself.
+// Against waves that expand the codes themselves (27 instructions per four sums at one row tile per wave, 17 at two), whole
+// calls with the quantizer, weights from memory, in us, and in brackets the prompt kernel (the same bits):
+//   rows     4096 x 4096          11008 x 4096         4096 x 11008         3584 x 16128
+//   64       17.2 -> 14.2 (38)    30.2 -> 22.6 (45)    35.0 -> 28.1 (93)    49.3 -> 38.3 (131)
+//   128      23.9 -> 18.1 (39)    49.6 -> 34.5 (45)    52.4 -> 36.4 (93)    70.9 -> 49.2 (131)
+//   256      38.0 -> 24.6 (39)    85.2 -> 58.9 (67)    86.4 -> 55.2 (92)    123 -> 73.5 (130)
+// ---------------------------------------------------------------------------
+template <int NT>
+__global__ void __launch_bounds__(256)
+skinny_w4a8_rows_kernel(const DecodeParams p) {
+  constexpr uint32_t START = 0x0BC00000u; // E8M0 byte e << 23 plus this: the bits of 1.5 * 2^(23 + e - 127)
+  constexpr int KS = 4; // K tiles per step: each of the four waves expands one (of every channel tile)
+  __shared__ __align__(16) long w_s[2][NT][KS][4][64]; // [buffer][channel tile][K tile][block][lane] codes, operand order
+  __shared__ __align__(16) int e_s[2][NT][KS][4][16];  // [block][channel] where the sum starts, or the scale
+  __shared__ __align__(16) int large_s[2][KS];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const DecodeSeg& sg = p.seg[0];
+  const int rt = (int)blockIdx.y * 4 + wave; // this wave's row tile (p.mt is a multiple of four)
+  const int KT = p.units, steps = (KT + KS - 1) / KS;
+
+  const i32x4* wq[NT];
+  const uint32_t* ws[NT];
 #pragma unroll
-    for (int mg = 0; mg < MG; mg++) {
-      const int m = m0 + (rr * MG + mg) * 16 + (lane & 15);
-      if (m >= p.M)
-        continue;
-      uint32_t h[4];
+  for (int a = 0; a < NT; a++) {
+    const int64_t lt = min((int)blockIdx.x * NT + a, sg.tiles - 1); // ragged last group: duplicate, not stored
+    wq[a] = reinterpret_cast<const i32x4*>(sg.qw) + lt * KT * 64 + lane;
+    ws[a] = reinterpret_cast<const uint32_t*>(sg.sw) + lt * KT * 16 + (lane & 15);
+  }
+  const i32x4* xop = reinterpret_cast<const i32x4*>(p.xq) + (int64_t)rt * 128 + lane;
+  const f32x4* sop = reinterpret_cast<const f32x4*>(p.sa) + (int64_t)rt * 16 + (lane & 15);
+  const int64_t xstride = p.mt * 128, sstride = p.mt * 16;
+
+  // (past the end: re-read a valid tile that is never consumed -- no branch around a load)
+  i32x4 wreg[NT], xreg[KS][2];
+  uint32_t sreg[NT];
+  f32x4 areg[KS];
+  auto load_w = [&](int s) {
+    const int64_t t = min(s * KS + wave, KT - 1);
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-        h[r] = apply_post_bits(facc[mg][r], sg.post_op, in1[mg][r], in2[mg][r], sg.post_scale) & 0xffffu;
-      *reinterpret_cast<uint2*>(sg.y + (int64_t)m * sg.N + lt * 16 + (lane >> 4) * 4) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    for (int a = 0; a < NT; a++) {
+      wreg[a] = wq[a][t * 64];
+      sreg[a] = ws[a][t * 16];
     }
-  } else {
-    ep.template finish_parts<KP, MG>(sg, facc, sk_lds, kp, tt * (MG * R) + rr * MG);
+  };
+  auto load_x = [&](int i, int t) {
+    t = min(t, KT - 1);
+    xreg[i][0] = xop[t * xstride];
+    xreg[i][1] = xop[t * xstride + 64];
+    areg[i] = sop[t * sstride];
+  };
+  load_w(0);
+#pragma unroll
+  for (int i = 0; i < KS; i++)
+    load_x(i, i);
+  __builtin_amdgcn_sched_barrier(0);
+  // (an absent input is read from the output, as in SkEpilogue::prefetch_flat: no branch around a load)
+  const uint16_t* pb = sg.bias ? sg.bias : sg.y;
+  const uint16_t* p1 = sg.post_in ? sg.post_in : sg.y;
+  const uint16_t* p2 = sg.post_in2 ? sg.post_in2 : sg.y;
+  const int m = rt * 16 + (lane & 15);
+  uint16_t in1[NT][4], in2[NT][4];
+  f32x4 facc[NT];
+#pragma unroll
+  for (int a = 0; a < NT; a++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int n = min((int)blockIdx.x * NT + a, sg.tiles - 1) * 16 + (lane >> 4) * 4 + r, o = min(m, p.M - 1) * sg.N + n;
+      const uint32_t b = pb[n];
+      in1[a][r] = p1[o];
+      in2[a][r] = p2[o];
+      facc[a][r] = sg.bias ? bf16_bits_to_f32(b) : 0.f;
+    }
+  __builtin_amdgcn_sched_barrier(0);
+
+  auto expand = [&](int s) {
+    const int buf = s & 1;
+    uint32_t scales = 0;
+#pragma unroll
+    for (int a = 0; a < NT; a++) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const uint32_t codes = (uint32_t)wreg[a][j];
+        const uint32_t lo = w4a8_expand(codes & 0x0F0F0F0Fu), hi = w4a8_expand((codes >> 4) & 0x0F0F0F0Fu);
+        w_s[buf][a][wave][j][lane] = (long)(((uint64_t)hi << 32) | lo);
+      }
+      e_s[buf][a][wave][lane >> 4][lane & 15] = (int)((((sreg[a] >> (8 * (lane >> 4))) & 0xffu) << 23) + START);
+      scales |= sreg[a] | (sreg[a] - 0x01010101u);
+    }
+    large_s[buf][wave] = __any((scales & 0x80808080u) != 0);
+  };
+  constexpr int U = KS * NT; // units of a step: (K tile, channel tile)
+  long wb[2][4];
+  i32x4 st[3][4], acc[2][4];
+  auto read = [&](int buf, int u) {
+    const long* wl = &w_s[buf][u % NT][u / NT][0][lane];
+    const i32x4* el = reinterpret_cast<const i32x4*>(&e_s[buf][u % NT][u / NT][0][(lane >> 4) * 4]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      wb[u & 1][j] = wl[j * 64];
+      st[u % 3][j] = el[j * 4];
+    }
+  };
+  auto rows = [&](int i, int j) {
+    return (long)(((uint64_t)(uint32_t)xreg[i][j >> 1][(j & 1) * 2 + 1] << 32) | (uint32_t)xreg[i][j >> 1][(j & 1) * 2]);
+  };
+  expand(0);
+  load_w(1);
+  __syncthreads();
+  for (int s = 0; s < steps; s++) {
+    const int buf = s & 1;
+    const i32x4 lg = *reinterpret_cast<const i32x4*>(large_s[buf]);
+    read(buf, 0);
+    if (s + 1 < steps) {
+      expand(s + 1);
+      load_w(s + 2);
+    }
+    if (s * KS + KS <= KT && __builtin_amdgcn_readfirstlane(lg[0] | lg[1] | lg[2] | lg[3]) == 0) {
+      static_for<0, U + 1>([&](auto UI) {
+        constexpr int u = decltype(UI)::value;
+        if constexpr (u + 1 < U)
+          read(buf, u + 1);
+        if constexpr (u < U) {
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            acc[u & 1][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb[u & 1][j], rows(u / NT, j), st[u % 3][j], 0, 0, 0);
+        }
+        if constexpr (u > 0) {
+          constexpr int v = u - 1, i = v / NT, a = v % NT;
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+              facc[a][r] = fmaf(__int_as_float(acc[v & 1][j][r]) - __int_as_float(st[v % 3][j][r]), areg[i][j], facc[a][r]);
+          if constexpr (a == NT - 1)
+            load_x(i, (s + 1) * KS + i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    } else { // a scale of zero, or of 2 or more, or fewer than KS K tiles left: convert and scale the sums
+      static_for<0, KS>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        if (s * KS + i < KT) {
+          static_for<0, NT>([&](auto A) {
+            constexpr int a = decltype(A)::value, u = i * NT + a;
+            read(buf, u);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              const i32x4 sum = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb[u & 1][j], rows(i, j), i32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+              for (int r = 0; r < 4; r++)
+                facc[a][r] = fmaf((float)sum[r] * __int_as_float(st[u % 3][j][r] - (int)START), areg[i][j], facc[a][r]);
+            }
+          });
+        }
+        load_x(i, (s + 1) * KS + i);
+      });
+    }
+    __syncthreads();
+  }
+  if (m >= p.M)
+    return;
+#pragma unroll
+  for (int a = 0; a < NT; a++) {
+    const int lt = (int)blockIdx.x * NT + a;
+    if (lt >= sg.tiles)
+      continue;
+    uint32_t h[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      h[r] = apply_post_bits(facc[a][r], sg.post_op, in1[a][r], in2[a][r], sg.post_scale) & 0xffffu;
+    *reinterpret_cast<uint2*>(sg.y + (int64_t)m * sg.N + lt * 16 + (lane >> 4) * 4) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
   }
 }
 
@@ -2699,23 +2877,26 @@ hipError_t launch_skinny_w4a8(DecodeParams& p, int ntw, hipStream_t stream) {
 }
 
 // W4A8 between decode and the prompt passes; p.mt, p.units set by the caller
-template <int MG, int T, int R, int KP, int PF>
+template <int MG, int R, int PF>
 static hipError_t sk_launch_w4a8_mg(DecodeParams& p, hipStream_t stream) {
-  const dim3 grid((p.total_tiles + T - 1) / T, (p.M + MG * R * 16 - 1) / (MG * R * 16), 1);
-  const size_t lds = KP == 1 ? 0 : (size_t)KP * T * MG * R * 256 * sizeof(float);
-  return sk_launch(skinny_w4a8_mg_kernel<MG, T, R, KP, PF>, p, grid, KP * T * R, lds, stream);
+  const dim3 grid(p.total_tiles, (p.M + MG * R * 16 - 1) / (MG * R * 16), 1);
+  return sk_launch(skinny_w4a8_mg_kernel<MG, R, PF>, p, grid, 4 * R, (size_t)4 * MG * R * 256 * sizeof(float), stream);
 }
 hipError_t launch_skinny_w4a8_mg(DecodeParams& p, bool ascending, hipStream_t stream) {
   if (p.S != 1 || p.mt <= 0 || p.n_seg != 1)
     return hipErrorInvalidValue;
-  if (ascending) // one row tile per wave while that leaves at most one workgroup per CU, else two (the codes expanded
-                 // once for both): 4096 x 4096 at 64 rows (256 workgroups) 13.3 us against 18.8, at 128 rows 21.0 against 19.1
-    return p.total_tiles * ((p.M + 63) / 64) <= 256 ? sk_launch_w4a8_mg<1, 1, 4, 1, 2>(p, stream)
-                                                    : sk_launch_w4a8_mg<2, 2, 2, 1, 2>(p, stream);
-  // one channel tile per workgroup: more of them lose except at 11008 x 4096, 32 rows (three: 14.0 us against 14.2)
+  if (ascending) {
+    // One channel tile per workgroup while those all run at once (two per CU: registers), else two, which read the rows
+    // half as often: 512 workgroups of one at 128 rows of 4096 x 11008 36.4 us against 39.8, 4096 x 4096 18.1 against
+    // 18.4; 768 (192 rows) 56.0 against 50.1 and 26.5 against 23.2.
+    const int by = (p.M + 63) / 64;
+    if ((int64_t)p.total_tiles * by <= 512)
+      return sk_launch(skinny_w4a8_rows_kernel<1>, p, dim3(p.total_tiles, by, 1), 4, 0, stream);
+    return sk_launch(skinny_w4a8_rows_kernel<2>, p, dim3((p.total_tiles + 1) / 2, by, 1), 4, 0, stream);
+  }
   if (p.M <= 16)
-    return sk_launch_w4a8_mg<1, 1, 1, 4, 4>(p, stream);
-  return p.M <= 32 ? sk_launch_w4a8_mg<2, 1, 1, 4, 2>(p, stream) : sk_launch_w4a8_mg<2, 1, 2, 4, 2>(p, stream);
+    return sk_launch_w4a8_mg<1, 1, 4>(p, stream);
+  return p.M <= 32 ? sk_launch_w4a8_mg<2, 1, 2>(p, stream) : sk_launch_w4a8_mg<2, 2, 2>(p, stream);
 }
 
 // MXFP4, 33..64 rows per block row: four channel tiles x four K parts per workgroup, K in p.S slices across workgroups

@@ -10,7 +10,7 @@
 // first four of its eight MFMA operand bytes, the high nibbles the last four; scales u8 [N/8][K/bc][bc/32][8].
 // A workgroup owns a 16 x 16 output tile; its four waves split the MX blocks of K and add their partial sums in
 // wave order: the simple shape of the calls that the prepacked kernels do not take (K no multiple of 128), not a tuned
-// kernel.  skinny_w4a8_mg_kernel computes the same sums in the same order on the prepacked tiles.
+// kernel.  skinny_w4a8_mg_kernel (fewer than 64 rows) computes the same sums in the same order on the prepacked tiles.
 #include <hip/hip_runtime.h>
 
 #include "tppx.h"
@@ -144,7 +144,7 @@ quant_act_w4a8_wide_kernel(const uint16_t* __restrict__ x, int M, int K, int MT1
     sa[((((int64_t)kt * (MT16 >> 2) + (mt >> 2)) * 4 + b) * 16 + m16) * 4 + (mt & 3)] = __fmul_rn(sc, (float)(6.0 / 127.0));
 }
 
-// The same bytes for skinny_w4a8_mg_kernel: int8 in its operand order, see there.
+// The same values for skinny_w4a8_mg_kernel and skinny_w4a8_rows_kernel: int8 in their operand order, see there.
 __global__ void __launch_bounds__(256)
 quant_act_w4a8_rows_kernel(const uint16_t* __restrict__ x, int M, int K, int mtiles, uint2* __restrict__ xq,
                            float* __restrict__ sa) {

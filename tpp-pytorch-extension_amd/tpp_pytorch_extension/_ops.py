@@ -682,23 +682,25 @@ W4A8_WIDE_ROWS = int(os.environ.get("TPPX_W4A8_WIDE_ROWS", "64"))
 def _w4a8_row_groups(M, N, K):
     """Does a W4A8 call of 64 or more rows run on the row-group kernel (4-bit weights, once per 64 rows) rather than on
     the prompt kernel (2 bytes per weight)?  The same bits either way.  Both in us, the row quantizer included, fitted
-    to 64 .. 2048 rows of fifteen shapes from 64 x 4096 to 28672 x 8192 (the choice is within 8 % of the faster one
-    down to K = 2304): row groups by rounds of 256 workgroups of 64 rows x 32 channels (16 channels while those are one
-    round); the prompt kernel by its workgroups of 64 x 128, one or two per CU, and beyond 256 of 128 x 128, two per CU,
-    by rounds of 512 of those, the last one rarely full.  7B shapes hand over at about 200 (11008 x 4096) to 300 rows,
-    28672 x 8192 at 128: 2048 rows there take 1250 us on the prompt kernel, 2260 in row groups."""
+    to 64 .. 512 rows of eight shapes from 1024 x 4096 to 20480 x 6656: row groups of 64 rows x 16 channels while at most
+    512 workgroups of those run (two per CU), else of 64 rows x 32 channels by rounds of 512 (a round begun costs 0.4 of
+    one whatever it holds); the prompt kernel by its workgroups of 64 x 128, one or two per CU, and beyond 256 of
+    128 x 128, two per CU, by rounds of 512 of those, the last one rarely full.  They hand over at 256 rows (20480 x 6656:
+    154 us in row groups, 144 on the prompt kernel, and 78 against 118 at 128 rows) to 512 rows (4096 x 4096: 44 and 42)."""
     rows64 = (M + 63) // 64
-    if rows64 * (N // 16) <= 256:
-        groups = 2.0 + 0.00272 * K
+    wgs = rows64 * (N // 16)
+    if wgs <= 512:
+        groups = 5.5 + 0.0021 * K if wgs <= 256 else 6.5 + 0.0027 * K
     else:
-        rounds = (rows64 * ((N + 31) // 32) + 255) // 256
-        groups = 3.0 + 0.00376 * K if rounds == 1 else 4.3 + 0.00516 * K + (rounds - 2) * (0.4 + 0.00227 * K)
+        rounds, rest = divmod(rows64 * ((N + 31) // 32), 512)
+        part = 0.0 if not rest else 0.4 + 0.6 * rest / 512 if rounds else 0.75 + 0.25 * rest / 512
+        groups = 6.0 + 0.0044 * K * (rounds + part)
     wgs = (M + 127) // 128 * ((N + 127) // 128)
     if wgs <= 256:
         prompt = (5.0 + 0.0072 * K + N * K / 4.5e6) * (1.0 if wgs <= 128 else 1.45)
     else:
         prompt = (1.0 if wgs <= 512 else 0.8 * ((wgs + 511) // 512)) * (12.0 + 0.0205 * K)
-    return groups + 3.0 + M * K * 1.5e-6 < prompt
+    return groups < prompt
 
 
 def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=None):

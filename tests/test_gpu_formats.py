@@ -794,3 +794,28 @@ def test_float_and_half_activations_in_terms_of_bf16(M, N, K, dtype, wkind):
     assert torch.equal(y[0].nan_to_num(0.0), ref[0].nan_to_num(0.0))
     near = 1e-2 if dtype == torch.float16 else 1e-5
     assert torch.allclose(y[2].double(), ref[2].double(), rtol=near, atol=near * float(ref[2].double().abs()[ref[2].isfinite()].max()), equal_nan=True)
+
+
+def _qint(kind, W):
+    ops = _ops()
+    if kind == "qint8":
+        return ops.remap_and_quantize_qint8(block_bf16(W).cuda())
+    if kind == "qint2":
+        return ops.remap_and_quantize_qint2_intlv(block_bf16(W).cuda())
+    N, K = W.shape
+    return ops.quantize_int4sym(W.view(N // 16, 16, K // 256, 128, 2).permute(0, 2, 3, 1, 4).contiguous().cuda(), 256, 2, True)
+
+
+# 4096 channels of 11008: K in slices; 640 channels are no blocks of 256, so 96 rows are two launches there (a pair of 65 or
+# more rows of such blocks is one launch of another kernel)
+@pytest.mark.parametrize("fmt,M,N,K", [("qint8", 16, 272, 1024), ("qint8", 17, 272, 1024), ("qint8", 33, 4096, 11008), ("qint8", 64, 1040, 2560),
+                                       ("qint8", 96, 272, 640), ("qint4", 9, 272, 1024), ("qint4", 40, 1040, 2560), ("qint2", 64, 288, 1024)])
+def test_int8_gate_up_quantizes_its_rows_once(fmt, M, N, K):
+    """The gate/up pair of QINT8-family weights where it runs as two launches behind ONE quantization of the rows: equal to
+    the two calls that quantize them each."""
+    ops = _ops()
+    W = [_qint(fmt, randn_bf16((N, K), 0.05, 3500 + i)) for i in range(2)]
+    assert M <= 64 or W[0].block_size != 256
+    x, b = randn_bf16((M, K), 1.0, 3510 + M).cuda(), randn_bf16((N,), 0.1, 3520).cuda()
+    want = ops.fc_mul(x, W[1], None, ops.fc_silu(x, W[0], b))
+    assert torch.equal(ops.swiglu_gate_up(x, W[0], W[1], b, None), want)

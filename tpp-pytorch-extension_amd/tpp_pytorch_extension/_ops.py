@@ -794,11 +794,13 @@ def _one_launch_group(weights):
 
 
 def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None, post_scale=1.0, flags=0,
-           row_sumsq=None):
+           row_sumsq=None, rows=None):
     """One quantized GEMM with a fused post-op
     (call_gemm_with_post_op, src/csrc/fused_gemm.h:1510-1597).
     row_sumsq: f32 [16][256] table that receives the row sums of squares of the output (see sums_table());
-    only honoured where takes_row_sums() says so."""
+    only honoured where takes_row_sums() says so.
+    rows: a list shared by consecutive calls of ONE input against QINT8 / QINT4 / QINT2 weights of one shape and format;
+    the quantized rows are left in it and the later calls' quantizer launch is left out."""
     L = _lib.lib()
     layout = weight.weight_layout() if isinstance(weight, QTensor) else None
     w4a8 = layout is not None and layout[0] == "mxfp4_int8"
@@ -828,12 +830,14 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
     if PACKED_CODES and M <= 64 and layout[0] in ("qint4", "qint2") and weight.block_size == 256 \
             and row_sumsq is None and not (flags & ~_lib.FLAG_XQ_REUSE):
         qp, sp, bits = weight.native_packed()
-        _buf, xq, sa = _qint8_buffer(x, M, K, 256) if M > 16 else (None, None, None)
+        _buf, xq, sa = (rows[0] if rows else _qint8_buffer(x, M, K, 256)) if M > 16 else (None, None, None)
         rc = L.tppx_linear_qintx(x.data_ptr(), xq, sa, qp.data_ptr(), sp.data_ptr(), _lib.ptr(bias),
                                  _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N, K, bits, post, post_scale,
-                                 flags, _lib.stream_of(x))
+                                 flags | _lib.FLAG_XQ_REUSE if rows and M > 16 else flags, _lib.stream_of(x))
         if rc != _lib.EUNSUPPORTED:  # rows that do not fit the in-kernel quantisation fall through to the int8 tiles
             _lib.check(rc)
+            if rows is not None and not rows and M > 16:
+                rows.append((_buf, xq, sa))
             return y
     qn, sn = weight.native()
     st = _lib.stream_of(x)
@@ -852,7 +856,12 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
                                        post, post_scale, flags, ws.data_ptr(), ws.numel(), st))
     else:
         qbs = weight.block_size
-        _buf, xq, sa = _qint8_buffer(x, M, K, qbs)
+        if rows:
+            (_buf, xq, sa), flags = rows[0], flags | _lib.FLAG_XQ_REUSE
+        else:
+            _buf, xq, sa = _qint8_buffer(x, M, K, qbs)
+            if rows is not None:
+                rows.append((_buf, xq, sa))
         _lib.check(L.tppx_linear_qint8(x.data_ptr(), xq, sa, qn.data_ptr(),
                                        sn.data_ptr(), _lib.ptr(bias), _lib.ptr(post_in),
                                        _lib.ptr(post_in2), y.data_ptr(), M, N, K, qbs, post,
@@ -1163,8 +1172,12 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
             if rc != _lib.EUNSUPPORTED:
                 _lib.check(rc)
                 return y
-        g = fc_silu(input, w_gate, b_gate)
-        return fc_mul(input, w_up, b_up, g)
+        # one quantization of the rows for both projections: the two calls are of one shape, so of one plan and layout of
+        # the quantized rows (17 .. 64 rows; up to 16 the GEMM quantizes its rows itself).  Gate, up and down projections of
+        # 4096 / 11008 at 32 / 64 rows 47.4 -> 44.7 / 57.7 -> 54.8 us, of 4096 / 4096 33.3 -> 30.6.
+        rows = [] if w_gate.block_size == w_up.block_size and w_gate.weight_kind() == w_up.weight_kind() else None
+        g = linear(input, w_gate, b_gate, POST_SILU, rows=rows)
+        return linear(input, w_up, b_up, POST_MUL, g, rows=rows)
     y = torch.empty(tuple(input.shape[:-1]) + (N,), dtype=torch.bfloat16, device=x.device)
     if M == 0:
         return y

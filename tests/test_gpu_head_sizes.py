@@ -206,6 +206,39 @@ def test_attn_prefill_other_head_size_with_mask(H):
     assert np.sqrt(((g - r) ** 2).sum() / (r ** 2).sum()) <= 5e-3
 
 
+# five and six tiles of 64 keys (one team has one more, or as many), a last tile of one key and a full one, one query block
+# whose last tile lies past its own last key; sequence 0 masked over its first tiles (both teams' first ones), or over all
+# keys of its first queries
+@pytest.mark.parametrize("H", [64, 8, 72, 120])
+@pytest.mark.parametrize("B,S,Nq,Nkv,past,hidden", [(1, 257, 4, 4, 0, 0), (2, 70, 4, 2, 314, 0), (2, 5, 8, 8, 252, 130), (2, 300, 4, 4, 0, 70)])
+def test_attn_prefill_in_two_teams(H, B, S, Nq, Nkv, past, hidden, monkeypatch):
+    """Prompt attention of few workgroups over many keys: two teams of waves take every other key tile.  Equal to the oracle
+    within the bounds of the other tests here, and to one team within the rounding of the probabilities: each is rounded to
+    bf16 against its own team's maximum (2^-8 relative, independent errors)."""
+    F = _llm()
+    L, Smax = past + S, 448
+    q = randn_bf16((B, S, Nq, H), 1.0, 281 + H)
+    k = randn_bf16((B, Nkv, Smax, H), 1.0, 282 + H)
+    v = randn_bf16((B, Nkv, Smax, H), 1.0, 283 + H)
+    k[:, :, L:] = float("nan")
+    v[:, :, L:] = float("nan")
+    mask = None
+    if hidden:
+        keep = torch.ones(B, L, dtype=torch.int64)
+        keep[0, :hidden] = 0
+        mask = F.TppCache(Smax).align_and_invert_mask(keep.to(torch.bfloat16))
+    got = _attn_prefill(q.cuda(), k.cuda(), v.cuda(), past, mask=None if mask is None else mask.cuda())
+    monkeypatch.setenv("TPPX_ATTN_TEAMS", "1")
+    one = _attn_prefill(q.cuda(), k.cuda(), v.cuda(), past, mask=None if mask is None else mask.cuda())
+    ref = O.attn_prefill(t2bits(q), t2bits(k[:, :, :L]), t2bits(v[:, :, :L]), None if mask is None else mask.float().numpy())
+    g, r, o = (bits2f(a).astype(np.float64) for a in (t2bits(got), ref, t2bits(one)))
+    assert np.isfinite(g).all()
+    rows = slice(hidden if past == 0 else 0, None)  # (queries that see no key at all: whatever the mask's finite values leave)
+    g, r, o = g[:, rows], r[:, rows], o[:, rows]
+    assert np.sqrt(((g - r) ** 2).sum() / (r ** 2).sum()) <= 5e-3
+    assert np.sqrt(((g - o) ** 2).sum() / (o ** 2).sum()) <= 2.0 ** -8
+
+
 # around the edges of a trip (128 or 64 keys) and of a wave's keys (32 or 16), an empty and a full cache, one split and
 # several, query heads sharing a K/V head, no mask / mask
 @pytest.mark.parametrize("H,HR,style", [(256, 64, "gptj"), (80, 0, None), (64, 64, "llama"), (96, 96, "llama"), (200, 80, "llama"),

@@ -1453,18 +1453,25 @@ attn_decode_group_kernel(const AttnParams p) {
 // 256 (H a multiple of 8, H <= HD; dims past H are staged as zeros and not stored), the K tile 64 x (HD + 8) and the
 // V^T tile HD x 68 in dynamic LDS, HD / 32 MFMAs per 16 keys for the scores and HD / 16 output tiles per query group.
 // Same arithmetic and rounding points as the kernel for 128.
+// TEAMS = 2: launches of few workgroups, where four waves walk one key tile after another and wait for each: two teams of four
+// waves take every other tile, with K and V tiles of their own, and the second one's sums (fp32, with the row maxima) meet the
+// first one's in LDS at the end.  96 workgroups of 80 wide behind 13 tiles 20.9 -> 17.4 us, 192 of 64 wide over 16 tiles
+// 17.9 -> 14.0.
 // ---------------------------------------------------------------------------
-template <int QG, int HD>
-__global__ void __launch_bounds__(256)
+template <int QG, int HD, int TEAMS>
+__global__ void __launch_bounds__(256 * TEAMS)
 attn_prefill_hd_kernel(const AttnPrefillParams p) {
   extern __shared__ __align__(16) uint16_t ap_lds[];
   constexpr int KP = HD + 8, VP = AP_VP, NJ = HD / 32, NDT = HD / 16, CH = HD / 8;
   constexpr int VI = (CH + 15) / 16; // value chunks per thread: 16 threads (key quads) x 16 chunks per pass
-  uint16_t* ks = ap_lds;           // [64 keys][KP]
-  uint16_t* vt = ap_lds + 64 * KP; // [HD dims][VP]
+  static_assert(TEAMS == 1 || QG == 1, "teams hand over one query group");
+  constexpr int TILE = 64 * KP + HD * VP; // elements of a team's tiles
+  const int team = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+  uint16_t* ks = ap_lds + team * TILE; // [64 keys][KP]
+  uint16_t* vt = ks + 64 * KP;         // [HD dims][VP]
   constexpr int QB = 64 * QG;
   const int H = p.H, HC = H >> 3;  // real 8-dim chunks per row
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int bh = blockIdx.y, b = bh / p.Nq, hq = bh - b * p.Nq;
   const int hk = hq / (p.Nq / p.Nkv);
@@ -1548,13 +1555,16 @@ attn_prefill_hd_kernel(const AttnPrefillParams p) {
       acc[qg][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const int nkb = (p.past + min(qblk * QB + QB - 1, p.S - 1)) / 64 + 1;
-  load_tile(0);
-  for (int kb = 0; kb < nkb; kb++) {
+  load_tile(team); // (past the last tile: the last key again, never used)
+  for (int kb0 = 0; kb0 < nkb; kb0 += TEAMS) {
+    const int kb = kb0 + team;
     __syncthreads(); // the previous tile has been read by every wave
     store_tile();
     __syncthreads();
-    if (kb + 1 < nkb)
-      load_tile(kb + 1); // in flight during the arithmetic below
+    if (kb + TEAMS < nkb)
+      load_tile(kb + TEAMS); // in flight during the arithmetic below
+    if (TEAMS > 1 && kb >= nkb)
+      continue; // the last round of a team without a tile (its barriers are behind it)
 
     f32x4 sc[QG][4];
 #pragma unroll
@@ -1636,9 +1646,48 @@ attn_prefill_hd_kernel(const AttnPrefillParams p) {
   }
 #pragma unroll
   for (int qg = 0; qg < QG; qg++) {
-    float ls = l[qg];
-    ls += __shfl_xor(ls, 16);
-    ls += __shfl_xor(ls, 32);
+    l[qg] += __shfl_xor(l[qg], 16);
+    l[qg] += __shfl_xor(l[qg], 32);
+  }
+  if constexpr (TEAMS > 1) {
+    // the other teams leave their sums where their tiles were ([wave][dim tile][lane] x 16 bytes, then maximum and sum per
+    // query); the first one adds them in team order
+    float* sums = reinterpret_cast<float*>(ks);
+    float* ml = sums + HD * 64;
+    static_assert(HD * 256 + 512 <= TILE * 2, "a team's sums fit its tiles");
+    __syncthreads();
+    if (team > 0) {
+#pragma unroll
+      for (int dt = 0; dt < NDT; dt++)
+        *reinterpret_cast<f32x4*>(sums + ((wave * NDT + dt) * 64 + lane) * 4) = acc[0][dt];
+      if (g == 0) {
+        ml[(wave * 16 + c) * 2] = m[0];
+        ml[(wave * 16 + c) * 2 + 1] = l[0];
+      }
+    }
+    __syncthreads();
+    if (team > 0)
+      return;
+#pragma unroll
+    for (int t = 1; t < TEAMS; t++) {
+      const float* ot = reinterpret_cast<const float*>(ap_lds + t * TILE);
+      const float om = ot[HD * 64 + (wave * 16 + c) * 2], ol = ot[HD * 64 + (wave * 16 + c) * 2 + 1];
+      const float mn = fmaxf(m[0], om);
+      const float wa = __builtin_amdgcn_exp2f(m[0] - mn), wb = __builtin_amdgcn_exp2f(om - mn);
+#pragma unroll
+      for (int dt = 0; dt < NDT; dt++) {
+        const f32x4 o = *reinterpret_cast<const f32x4*>(ot + ((wave * NDT + dt) * 64 + lane) * 4);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          acc[0][dt][r] = acc[0][dt][r] * wa + o[r] * wb;
+      }
+      l[0] = l[0] * wa + ol * wb;
+      m[0] = mn;
+    }
+  }
+#pragma unroll
+  for (int qg = 0; qg < QG; qg++) {
+    const float ls = l[qg];
     const int qi = q0 + qg * 16 + c;
     if (qi < p.S) {
       uint16_t* orow = p.out + (((int64_t)b * p.S + qi) * p.Nq + hq) * H;
@@ -2510,25 +2559,36 @@ extern "C" int tppx_attn_prefill(const void* q, const void* kcache, const void* 
     const int hd = H <= 64 ? 64 : H <= 128 ? 128 : 256;
     const long wgs2h = ((S + 127) / 128) * B * Nq;
     const bool two = hd != 256 && S > 64 && env_int("TPPX_ATTN_QG", wgs2h >= 512 ? 2 : 1) == 2;
-    const size_t lds = (size_t)(64 * (hd + 8) + hd * AP_VP) * sizeof(uint16_t);
     const dim3 grid((unsigned)((S + (two ? 127 : 63)) / (two ? 128 : 64)), (unsigned)(B * Nq));
+    const int64_t tiles = (past_len + S + 63) / 64;
+    // One workgroup per CU or less: two teams over the key tiles from five of them on (3: 6.0 us either way at 64 wide, 7.4
+    // against 7.5 at 80; 5: 8.0 -> 7.4 and 10.2 -> 9.7).  Beyond 256 workgroups they share CUs as it is (512 of 80 wide 26.6
+    // us, in teams 31.6), and at 256 wide the LDS reads of one team fill a CU (13 tiles 35.0 against 33.8, 5 tiles 17.6
+    // against 18.4).
+    const bool teams = hd != 256 && !two && tiles > 1 &&
+                       env_int("TPPX_ATTN_TEAMS", (int64_t)grid.x * grid.y <= 256 && tiles >= 5 ? 2 : 1) == 2;
     hipError_t e = hipSuccess;
-#define TPPX_AP_HD(QG_, HD_)                                                                                          \
+#define TPPX_AP_HD(QG_, HD_, T_)                                                                                      \
   do {                                                                                                               \
-    e = allow_dynamic_lds(reinterpret_cast<const void*>(attn_prefill_hd_kernel<QG_, HD_>), lds);                     \
+    const size_t lds = (size_t)T_ * (64 * (HD_ + 8) + HD_ * AP_VP) * sizeof(uint16_t);                               \
+    e = allow_dynamic_lds(reinterpret_cast<const void*>(attn_prefill_hd_kernel<QG_, HD_, T_>), lds);                 \
     if (e == hipSuccess)                                                                                             \
-      attn_prefill_hd_kernel<QG_, HD_><<<grid, dim3(256), lds, (hipStream_t)stream>>>(p);                            \
+      attn_prefill_hd_kernel<QG_, HD_, T_><<<grid, dim3(256 * T_), lds, (hipStream_t)stream>>>(p);                   \
   } while (0)
     if (hd == 64 && two)
-      TPPX_AP_HD(2, 64);
+      TPPX_AP_HD(2, 64, 1);
+    else if (hd == 64 && teams)
+      TPPX_AP_HD(1, 64, 2);
     else if (hd == 64)
-      TPPX_AP_HD(1, 64);
+      TPPX_AP_HD(1, 64, 1);
     else if (hd == 128 && two)
-      TPPX_AP_HD(2, 128);
+      TPPX_AP_HD(2, 128, 1);
+    else if (hd == 128 && teams)
+      TPPX_AP_HD(1, 128, 2);
     else if (hd == 128)
-      TPPX_AP_HD(1, 128);
+      TPPX_AP_HD(1, 128, 1);
     else
-      TPPX_AP_HD(1, 256);
+      TPPX_AP_HD(1, 256, 1);
 #undef TPPX_AP_HD
     if (e != hipSuccess)
       return check_hip(e, who);

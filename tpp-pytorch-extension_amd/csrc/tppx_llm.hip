@@ -2399,15 +2399,24 @@ static int attn_generic_launch(const char* who, AttnGenParams& p, hipStream_t st
     TPPX_REQUIRE(queries < ((int64_t)1 << 31), TPPX_ESHAPE, "%s: problem too large", who);
     // Workgroups per (sequence, head), as for 128-wide heads: two trips each at the cache's capacity (the length itself is
     // a device scalar: splits whose trips lie past the keys leave empty states), but no fewer than 288 workgroups and no
-    // more than 512 in all; at most one per trip and 32.  One for caches of three trips (50 keys in 178 of one sequence:
-    // 4.6 us against 6.5 with two), from 256 heads on (16 x 16 x 700 keys: 30.5 against 31.6 with two) and where the
-    // workspace cannot hold the states.
+    // more than 512 in all; at most one per trip and 32; of that count, one less and one more the one that fills the rounds
+    // of 256 best (192 heads of 80, 3000 keys: three 39.0 us, four 34.2; 160: four 31.4, three 29.1; 224 heads of 64: three
+    // 33.0, two 31.6).  One for caches of three trips (50 keys in 178 of one sequence: 4.6 us against 6.5 with two), from
+    // 256 heads on (16 x 16 x 700 keys: 30.5 against 31.6 with two), more than 128 wide, where a workgroup moves twice the
+    // bytes, from 160 on (208 heads of 256, 3000 keys: 98 against 108 with three, 160 heads 80 against 83 with four; 96
+    // heads 76 against 49 with five), and where the workspace cannot hold the states.
     const int64_t trip = p.H <= 128 ? 128 : 64, most = ((int64_t)p.Smax + trip - 1) / trip;
     int64_t want = env_int("TPPX_ATTN_GENERIC_SPLITS", 0);
-    if (want <= 0 && (most <= 3 || queries >= 256))
+    if (want <= 0 && (most <= 3 || queries >= (p.H > 128 ? 160 : 256))) {
       want = 1;
-    else if (want <= 0)
-      want = std::max((288 + queries - 1) / queries, std::min((most + 1) / 2, (512 + queries - 1) / queries));
+    } else if (want <= 0) {
+      const int64_t least = (288 + queries - 1) / queries, w = std::max(least, std::min((most + 1) / 2, (512 + queries - 1) / queries));
+      const auto fill = [&](int64_t n) { return (double)(n * queries) / (double)((n * queries + 255) / 256); };
+      want = w;
+      for (int64_t n = std::max(least, w - 1); n <= std::min(w + 1, std::max(w, (most + 1) / 2)); n++)
+        if (n < want ? fill(n) >= fill(want) : fill(n) > fill(want))
+          want = n;
+    }
     want = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 32), most));
     if (want > 1 && queries <= ATTN_TICKETS && ws && queries * want * (p.H + 2) * (int64_t)sizeof(float) <= ws_bytes) {
       p.splits = (int)want;

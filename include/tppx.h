@@ -298,8 +298,9 @@ int tppx_linear_mxfp4_int8_rows(const void* x, const void* q_nat,
 /* W4A8 between decode calls and prompt passes, on the same prepacked weights (s_nat 16-byte aligned).  The rows are
  * quantized into xq / sa first (operand order, private to the library): xq holds roundup(M, 64) * K bytes, sa
  * roundup(M, 64) * K / 32 floats, both 16-byte aligned.  TPPX_FLAG_XQ_REUSE: xq / sa still hold this x from an earlier
- * call with the same M and K.  The same bits as the quantizer followed by tppx_linear_mxfp4_int8 with fewer than 64 rows,
- * as tppx_linear_mxfp4_int8_wide from 64 rows on.  TPPX_EUNSUPPORTED (before any launch): 2^31 outputs and more, K above
+ * call with the same M and K.  The same bits as the quantizer followed by tppx_linear_mxfp4_int8 with fewer than 64 rows
+ * (where a product of two scales is subnormal this one rounds once less), as tppx_linear_mxfp4_int8_wide from 64 rows on.
+ * TPPX_EUNSUPPORTED (before any launch): 2^31 outputs and more, K above
  * 65535 * 128, more than 2^25 channels or 2^21 rows. */
 int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa,
                                const void* q_nat, const void* s_nat,

@@ -305,3 +305,19 @@ def test_decode_step_with_rotary_and_append_in_the_launch(H, HR, style, B, Nq, N
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, first)
+
+
+@pytest.mark.parametrize("H,Nq,Nkv", [(64, 8, 2), (80, 4, 4), (256, 2, 2), (8, 2, 1), (200, 4, 2)])
+@pytest.mark.parametrize("B,L,Smax", [(2, 77, 128), (1, 1000, 1100)])
+def test_decode_step_rounds_the_output_only(H, Nq, Nkv, B, L, Smax):
+    """The probabilities keep 16 bits on their way into p . v: against float64 the output is off by its own rounding to bf16,
+    half an ulp, and what fp32 scores and sums leave -- 2^-16 of a probability, an exponential good to about 2^-20 of scores up
+    to 2^3, so 2^-14 of sum p |v| is far above it.  (With bf16 probabilities the second part would be up to 2^-9.)"""
+    F = _llm()
+    q, k, v = randn_bf16((B, Nq, H), 1.0, 331 + H), randn_bf16((B, Nkv, Smax, H), 1.0, 332 + H), randn_bf16((B, Nkv, Smax, H), 1.0, 333 + H)
+    got = _attn(F, q.cuda(), k.cuda(), v.cuda(), L).cpu().double()
+    kk, vv = (t[:, :, :L].double().repeat_interleave(Nq // Nkv, dim=1) for t in (k, v))
+    p = torch.softmax((q.double().unsqueeze(2) * kk).sum(-1) / H ** 0.5, -1).unsqueeze(-1)
+    ref, mag = (p * vv).sum(2), (p * vv.abs()).sum(2)
+    half_ulp = torch.exp2(torch.floor(torch.log2(ref.abs().clamp_min(1e-30))) - 8)
+    assert ((got.view_as(ref) - ref).abs() <= half_ulp * (1 + 2.0 ** -8) + 2.0 ** -14 * mag).all()

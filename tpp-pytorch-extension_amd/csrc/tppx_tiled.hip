@@ -1086,8 +1086,8 @@ big_bf16_kernel(const BigParams P) {
 // 64 x 128 with K in P.S slices (grid y): launches of few workgroups and a long K.  A workgroup's time is its K steps (0.45 us
 // each, MXFP4) whatever else the chip does, so 64 .. 192 of them with 86 steps leave most of it idle; three resident to a CU
 // run S times as many with an S-th of the steps.  The sums go out as they lie in the registers, 32 KiB a workgroup, and a
-// second launch adds them: with it 4096 x 11008 at 100 / 200 / 333 rows 32.3 -> 18.7 / 40.1 -> 27.5 / 42.1 -> 38.0 us, 2560 x
-// 10240 at 200 rows 36.3 -> 21.1; bf16 weights 55 -> 29, 60 -> 40, 61 -> 59 and 55 -> 28.
+// second launch adds them: with it 4096 x 11008 at 100 / 200 / 300 rows 32.9 -> 20.8 / 40.5 -> 29.1 / 40.9 -> 34.9 us, 2560 x
+// 10240 at 200 rows 35.6 -> 21.7; bf16 weights 56.9 -> 32.3, 61.2 -> 40.7, 66.4 -> 53.4 and 55.3 -> 28.5 (weights from memory).
 template <bool WBF16>
 __global__ void __launch_bounds__(256, 2)
 side_split_kernel(const BigParams P) {
@@ -1895,10 +1895,16 @@ double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16) {
 
 // K slices (1: whole) of a launch of n GEMMs that takes whole_us without them, *us: what it takes then.  The 64 x 128 tile's
 // estimate for S times the workgroups and an S-th of the steps, and the slices' sums out and in: 2.2 us and 8.5 .. 16.5 ns
-// (MXFP4, the more the shorter K is) or 11.5 ns (bf16 weights) for each 32 KiB of them.  Measured at 65 .. 800 rows of
-// 2560 .. 4096 channels and K = 2560 .. 16384 with 2, 3, 4, 6 and 8 slices: within 10 % but for the shortest K, where it is up to
-// 2 us low: up to K = 2560 (11.5 us whole, 11.3 in slices at 65 rows), MXFP4 4096 (17 whole, 15 .. 22), no launch is split.  Up to
-// one round of whole-K workgroups (bf16: a quarter more); 3 % for the estimate's sake.
+// (MXFP4, the more the shorter K is) or 11.5 ns (bf16 weights) for each 32 KiB of them.  Up to K = 2560 (11.5 us whole, 11.3 in
+// slices at 65 rows), MXFP4 4096 (17 whole, 15 .. 22), no launch is split; up to one round of whole-K workgroups (bf16: a quarter
+// more).  Measured on 250 launches of 65 .. 1024 rows of 1024 .. 11000 channels and K = 2816 .. 16384:
+//   MXFP4  the slices' estimate is 3 .. 5 % high, but 2 % low with two slices of more than 160 workgroups or more than 730
+//          workgroups in all, and 1 % lower with each row block from the fifth on (more of them read the same weights).  With
+//          that, 6 % for the estimate's sake: none is slower than whole by more than 2 % (1408 x 9216 at 1024 rows, 34.0 us
+//          whole, 37.8 in slices without it; 4096 x 11008 at 400 rows 41.8 and 45.1), the best forgone is 6 % faster in slices.
+//   bf16   right to 3 % with weights from memory; at hand in the Infinity Cache whole K is up to a quarter faster, slices hardly
+//          (8640 x 4608 at 124 rows 32.9 and 32.1 us from memory, 22.4 and 25.8 at hand), so a near tie goes to whole K: 5 %,
+//          10 % beyond a round.
 template <bool WBF16>
 static int best_split(int64_t M, int64_t K, const int* tiles, int n, int64_t part_bytes, double whole_us, double* us) {
   const int forced = env_int("TPPX_TILED_SPLIT", 1);
@@ -1910,12 +1916,15 @@ static int best_split(int64_t M, int64_t K, const int* tiles, int n, int64_t par
   const int64_t wgs = (M + 63) / 64 * nb;
   const double s = (double)K / 128.0, mb = (double)(all * 32 * K) * 1e-6;
   const double ns = WBF16 ? 11.5 : 16.5 - 8.0 * std::min(1.0, std::max(0.0, (s - 32.0) / 48.0));
+  const double rows = 0.01 * (double)std::max<int64_t>(0, (M + 63) / 64 - 4);
   int best = 1;
-  double best_us = 0.97 * whole_us;
+  double best_us = (WBF16 ? wgs > 256 ? 0.90 : 0.95 : 0.94) * whole_us;
   for (int S : {2, 3, 4, 6}) {
     if (wgs * S * 32768 > part_bytes || K / 128 < 4 * S)
       break;
-    const double c = tile_us((WBF16 ? BF16_COST : MXFP4_COST)[TILE_64_128], TILE_64_128, wgs * S, s / S, mb, false) + 2.2 + ns * 1e-3 * (double)(wgs * S);
+    double c = tile_us((WBF16 ? BF16_COST : MXFP4_COST)[TILE_64_128], TILE_64_128, wgs * S, s / S, mb, false) + 2.2 + ns * 1e-3 * (double)(wgs * S);
+    if (!WBF16)
+      c *= 1.0 + rows + ((S == 2 ? wgs > 160 : wgs * S > 730) ? 0.02 : -0.04);
     if (forced == S || (forced == 1 && K > (WBF16 ? 2560 : 4096) && wgs <= (WBF16 ? 320 : 256) && c < best_us)) {
       best_us = c;
       best = S;

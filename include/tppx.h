@@ -561,10 +561,17 @@ int tppx_rotary_kv_append_gptj(void* q, void* k, const void* v,
  * sequence: q bf16 [B][Nq][128], cache bf16 [B][Nkv][Smax][128], additive mask
  * bf16 [B][mask_ld] or NULL; valid keys = *kv_len_dev (device i32) + kv_len_add
  * (the counter may still hold the length before this step's append); out bf16
- * [B][Nq][128].  ws: optional scratch for split-KV partial results.  Head sizes
- * H other than 128 (multiples of 8 up to 256, tensors [..][H]) run a kernel of
- * the same layout with 8, 16 or 32 lanes per key (not the rotary-fused form);
- * anything else returns TPPX_EUNSUPPORTED. */
+ * [B][Nq][128].  ws: optional scratch for split-KV partial results, B * Nq *
+ * splits * (H + 2) floats for up to 32 splits (too small: unsplit); launches
+ * that share it must be ordered.  Head sizes H other than 128 (multiples of 8
+ * up to 256, tensors [..][H]) run a kernel of the same layout with 8 or 16
+ * lanes per key; anything else returns TPPX_EUNSUPPORTED.
+ * The splits' results are merged by the workgroup that arrives last, found by
+ * arrival counters of the library (4096 per device, one per (sequence, head) of
+ * a launch, handed out in rotation: launches on different streams are safe only
+ * while fewer counters than that are taken by launches issued and not done, a
+ * captured graph keeps its counters for good); other head sizes than 128: by a
+ * second launch.  The _counted forms below need neither. */
 int tppx_attn_decode(const void* q, const void* kcache, const void* vcache,
                      const void* mask, int64_t mask_ld, const void* kv_len_dev,
                      int64_t kv_len_add, void* out, int64_t B, int64_t Nq,
@@ -599,6 +606,35 @@ int tppx_attn_decode_append(const void* q, const void* k, const void* v,
                             const void* kv_len_dev, void* out, int64_t B,
                             int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
                             void* ws, int64_t ws_bytes, tppx_stream_t stream);
+
+/* The three above with arrival counters of the caller's: counters holds u32
+ * words 256 bytes apart, one per (sequence, head), zero before its first launch;
+ * every launch leaves it zero.  Launches that share it must be ordered, as those
+ * that share ws, so a caller keeps one beside each workspace; then any number
+ * of streams, threads and replayed graphs may overlap, for every head size, and
+ * the merge is part of the launch.  NULL or fewer than B * Nq * 256 bytes: as
+ * the form without. */
+int tppx_attn_decode_counted(const void* q, const void* kcache,
+                             const void* vcache, const void* mask,
+                             int64_t mask_ld, const void* kv_len_dev,
+                             int64_t kv_len_add, void* out, int64_t B,
+                             int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
+                             void* ws, int64_t ws_bytes, void* counters,
+                             int64_t counter_bytes, tppx_stream_t stream);
+int tppx_attn_decode_rotary_counted(
+    const void* q, const void* k, const void* v, const void* emb_pos,
+    const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache,
+    void* vcache, const void* mask, int64_t mask_ld, const void* kv_len_dev,
+    void* out, int64_t B, int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
+    void* ws, int64_t ws_bytes, void* counters, int64_t counter_bytes,
+    tppx_stream_t stream);
+int tppx_attn_decode_append_counted(
+    const void* q, const void* k, const void* v, const void* emb_pos, int gptj,
+    const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache,
+    void* vcache, const void* mask, int64_t mask_ld, const void* kv_len_dev,
+    void* out, int64_t B, int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
+    void* ws, int64_t ws_bytes, void* counters, int64_t counter_bytes,
+    tppx_stream_t stream);
 
 /* The same attn<T> (src/csrc/llm/attn.cpp:781-955, isCausal) for S query tokens
  * per sequence (prompt processing, or several new tokens on a filled cache):

@@ -321,3 +321,88 @@ def test_decode_step_rounds_the_output_only(H, Nq, Nkv, B, L, Smax):
     ref, mag = (p * vv).sum(2), (p * vv.abs()).sum(2)
     half_ulp = torch.exp2(torch.floor(torch.log2(ref.abs().clamp_min(1e-30))) - 8)
     assert ((got.view_as(ref) - ref).abs() <= half_ulp * (1 + 2.0 ** -8) + 2.0 ** -14 * mag).all()
+
+
+@pytest.mark.parametrize("H,Nq,Nkv,B", [(80, 32, 32, 4), (256, 16, 16, 4), (128, 28, 4, 2), (128, 32, 32, 2)])
+def test_steps_on_two_streams_and_in_a_replayed_graph(H, Nq, Nkv, B):
+    """Decode attention with split keys, from two threads on streams of their own beside a replayed graph: launches that
+    share arrival counters are the ones that share a workspace, which are ordered, so every output has the bits of the same
+    call alone, and the counters are zero again.  96 launches a thread: 4096 counters in rotation, one per (sequence, head),
+    would have come round several times.  Without counters: the same bits."""
+    import threading
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+    Smax, past = 1600, 1500
+    g = torch.Generator(device="cuda").manual_seed(H + Nq)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    kc, vc = rnd(B, Nkv, Smax, H), rnd(B, Nkv, Smax, H)
+    qs = [rnd(B, Nq, H) for _ in range(3)]
+    n = torch.tensor([past], dtype=torch.int32, device="cuda")
+
+    def step(q, counted=True):
+        ws, st, out = _lib.workspace(q), _lib.stream_of(q), torch.empty_like(q)
+        args = (q.data_ptr(), kc.data_ptr(), vc.data_ptr(), None, 0, n.data_ptr(), 0, out.data_ptr(), B, Nq, Nkv, H, Smax)
+        scratch = _lib.with_counters(ws)
+        _lib.check(L.tppx_attn_decode_counted(*args, *scratch, st) if counted else L.tppx_attn_decode(*args, *scratch[:2], st))
+        return out
+
+    alone = [step(q) for q in qs]
+    assert all(torch.equal(step(q, False), a) for q, a in zip(qs, alone))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step(qs[2])
+    torch.cuda.synchronize()
+    outs, errors, buffers = [[], []], [], [None, None]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+
+    def worker(i):
+        try:
+            with torch.cuda.stream(streams[i]):
+                for _ in range(96):
+                    outs[i].append(step(qs[i]))
+                buffers[i] = _lib.workspace(qs[i])
+        except Exception as e:  # reported by the main thread
+            errors.append(repr(e))
+
+    threads = [threading.Thread(target=worker, args=(i,)) for i in range(2)]
+    replays = []
+    for t in threads:
+        t.start()
+    for _ in range(48):
+        graph.replay()
+        replays.append(captured.clone())
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i in range(2):
+        assert all(torch.equal(y, alone[i]) for y in outs[i]), i
+    assert all(torch.equal(y, alone[2]) for y in replays)
+    assert buffers[0].data_ptr() != buffers[1].data_ptr()
+    for ws in buffers:
+        at = _lib.with_counters(ws)[2] - ws.untyped_storage().data_ptr()
+        whole = torch.empty(0, dtype=torch.uint8, device="cuda").set_(ws.untyped_storage())
+        assert whole.numel() >= at + _lib.COUNTER_BYTES and not whole[at:at + _lib.COUNTER_BYTES].any()
+
+
+def test_decoder_blocks_count_arrivals_in_their_own_workspace(monkeypatch):
+    """The Python layer calls no form of decode attention that shares counters between streams."""
+    from tpp_pytorch_extension import _lib
+    F = _llm()
+    lib, seen = _lib.lib(), []
+
+    class Watch:
+        def __getattr__(self, name):
+            if name.startswith("tppx_attn_decode"):
+                assert name.endswith("_counted"), name
+                seen.append(name)
+            return getattr(lib, name)
+
+    monkeypatch.setattr(_lib, "lib", lambda: Watch())
+    for H, N, style in ((80, 4, None), (256, 2, "gptj"), (128, 4, "gptj")):
+        cache = F.TppCache(64)
+        table = None if style is None else torch.zeros((64, 64), device="cuda")
+        qkv = [torch.randn((1, 1, N * H), device="cuda").to(torch.bfloat16) for _ in range(3)]
+        F.rotate_append_attend(*qkv, None, torch.zeros((1, 1), dtype=torch.int64, device="cuda"), cache, 0, 1, 1, N, N, H, table, style)
+    torch.cuda.synchronize()
+    assert seen == ["tppx_attn_decode_append_counted"] * 2 + ["tppx_attn_decode_counted"]

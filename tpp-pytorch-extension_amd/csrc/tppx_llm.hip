@@ -286,7 +286,8 @@ struct AttnParams {
   uint16_t* out;        // [B][Nq][128]
   float* part;          // [B*Nq][splits][130]
   int B, Nq, Nkv, Smax, mask_ld, splits;
-  int ticket0;          // >= 0: first arrival counter of this launch (the last split to arrive merges); < 0: second kernel
+  unsigned int* counters; // the caller's arrival counters, or null:
+  int ticket0;          // >= 0: first of the library's (the last split to arrive merges); < 0: second kernel
   float scale;
   // ROT: the query and the step's new key / value arrive unrotated and not yet in the cache
   const uint16_t* k_new; // [B][Nkv][128]
@@ -297,7 +298,10 @@ struct AttnParams {
 };
 
 // Arrival counters of the split launches, one per (sequence, head): zero between launches (the counting
-// instruction wraps on the last arrival); a launch takes a window handed out in rotation by the host.
+// instruction wraps on the last arrival).  A caller that gives counters with its workspace orders its launches on both
+// alike.  Without them a launch of 128-wide heads takes a window of the library's, handed out in rotation by the host:
+// windows come round again after 4096 counters, so launches queued on other streams, and graphs replayed beside eager
+// work, can hold the same one.
 // The counters of a launch are all hit within a microsecond or two; side by side they would queue up at the atomic
 // unit of one memory channel, so each one has 256 bytes to itself.
 constexpr int ATTN_TICKETS = 4096;
@@ -308,6 +312,13 @@ __global__ void attn_clear_tickets_kernel(int first, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n)
     attn_tickets[(first + i) * ATTN_TICKET_STRIDE] = 0;
+}
+
+// Counts an arrival of group `i` of a launch; true for the last of `splits`.
+__device__ __forceinline__ bool attn_arrive(unsigned int* counters, int ticket0, int i, int splits) {
+  unsigned int* c = counters ? counters : attn_tickets + (int64_t)ticket0 * ATTN_TICKET_STRIDE;
+  const unsigned int last = (unsigned int)splits - 1;
+  return atomicInc(c + (int64_t)i * ATTN_TICKET_STRIDE, last) == last;
 }
 
 __device__ __forceinline__ uint4 as_uint4(const i32x4& v) {
@@ -321,7 +332,7 @@ __device__ __forceinline__ void attn_finish(const AttnParams& p, int bh, int tid
   if (tid < 128) {
     if (p.splits == 1) {
       p.out[(int64_t)bh * 128 + tid] = (uint16_t)f32_to_bf16_bits(Ls > 0.f ? o / Ls : 0.f);
-    } else if (p.ticket0 < 0) {
+    } else if (p.ticket0 < 0 && !p.counters) {
       float* dst = p.part + ((int64_t)bh * p.splits + blockIdx.y) * 130;
       dst[2 + tid] = o;
       if (tid == 0) {
@@ -338,7 +349,7 @@ __device__ __forceinline__ void attn_finish(const AttnParams& p, int bh, int tid
       }
     }
   }
-  if (p.splits == 1 || p.ticket0 < 0)
+  if (p.splits == 1 || (p.ticket0 < 0 && !p.counters))
     return;
   // The split that arrives last merges all of them, in split order (the same sums whichever split that is).
   // Order: every thread waits until its own stores above have been acknowledged (vmcnt counts stores on this
@@ -347,10 +358,8 @@ __device__ __forceinline__ void attn_finish(const AttnParams& p, int bh, int tid
   __shared__ int arrived_last;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (tid == 0) {
-    const unsigned int last = (unsigned int)p.splits - 1;
-    arrived_last = atomicInc(&attn_tickets[(p.ticket0 + bh) * ATTN_TICKET_STRIDE], last) == last;
-  }
+  if (tid == 0)
+    arrived_last = attn_arrive(p.counters, p.ticket0, bh, p.splits);
   __syncthreads();
   if (!arrived_last || tid >= 128)
     return;
@@ -1364,7 +1373,7 @@ attn_decode_group_kernel(const AttnParams p) {
       store4(h, d4, o, Ls);
       continue;
     }
-    if (p.ticket0 < 0) { // attn_combine_kernel follows
+    if (p.ticket0 < 0 && !p.counters) { // attn_combine_kernel follows
       float* const dst = p.part + ((int64_t)(head0 + h) * S + blockIdx.y) * 130;
 #pragma unroll
       for (int e = 0; e < 4; e++)
@@ -1383,16 +1392,14 @@ attn_decode_group_kernel(const AttnParams p) {
     if (d4 == 0)
       __hip_atomic_store(reinterpret_cast<uint64_t*>(part_ml + at * 2), __builtin_bit_cast(uint64_t, make_float2(M, Ls)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (S == 1 || p.ticket0 < 0)
+  if (S == 1 || (p.ticket0 < 0 && !p.counters))
     return;
   // The split that arrives last merges all of them, in split order; the ordering argument is attn_finish's: own stores
   // acknowledged, barrier, ticket, device-scope loads.  Nobody waits for anybody.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (tid == 0) {
-    const unsigned int last = (unsigned int)S - 1;
-    *arrived_last = atomicInc(&attn_tickets[(p.ticket0 + (int)blockIdx.x) * ATTN_TICKET_STRIDE], last) == last;
-  }
+  if (tid == 0)
+    *arrived_last = attn_arrive(p.counters, p.ticket0, (int)blockIdx.x, S);
   __syncthreads();
   if (!*arrived_last)
     return;
@@ -1919,9 +1926,22 @@ extern "C" int tppx_rotary_kv_append_gptj(void* q, void* k, const void* v, const
   return rotary_common(who, p, (hipStream_t)stream);
 }
 
-// shared tail of the two single-query entry points: split planning, counters, launch
-// window of arrival counters (at most ATTN_TICKETS), handed out in rotation so that split launches in flight on different
-// streams do not share counters
+// a caller's arrival counters: zero before their first launch, zero again behind every launch
+struct AttnCounters {
+  void* p = nullptr;
+  int64_t bytes = 0;
+  unsigned int* of(int64_t groups) const { // null: too few
+    return groups * ATTN_TICKET_STRIDE * (int64_t)sizeof(unsigned int) <= bytes ? (unsigned int*)p : nullptr;
+  }
+};
+
+static int check_counters(const char* who, const AttnCounters& c) {
+  TPPX_REQUIRE(c.bytes >= 0 && (c.bytes == 0 || c.p), TPPX_EINVAL, "%s: size of the counters given with a null pointer", who);
+  TPPX_REQUIRE(((uintptr_t)c.p & 3u) == 0, TPPX_EINVAL, "%s: counters not 4-byte aligned", who);
+  return TPPX_OK;
+}
+
+// window of the library's arrival counters (at most ATTN_TICKETS), handed out in rotation
 static int attn_take_tickets(int64_t tickets) {
   static std::mutex mu;
   static int cursor = 0;
@@ -1933,8 +1953,9 @@ static int attn_take_tickets(int64_t tickets) {
   return first;
 }
 
+// shared tail of the single-query entry points for 128-wide heads: split planning, counters, launch
 static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t B, int64_t Nq, int64_t Smax, void* ws,
-                              int64_t ws_bytes, hipStream_t stream) {
+                              int64_t ws_bytes, AttnCounters counters, hipStream_t stream) {
   // The wide kernel (128 keys per workgroup and trip) is the default: measured against the row kernel (64 keys per
   // trip) over 32 heads, it is faster at every batch size from 1 to 64 and context from 100 to 8000 keys once its
   // workgroups make about two trips each (batch 16, 2048 keys: 3660 -> 3739 tokens/s for the whole decode step;
@@ -1979,8 +2000,11 @@ static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t 
   p.part = (float*)ws;
   p.ticket0 = -1;
   const int64_t tickets = group ? groups : B * Nq;
-  if (splits > 1 && tickets <= ATTN_TICKETS && one_launch)
-    p.ticket0 = attn_take_tickets(tickets);
+  if (splits > 1 && one_launch) {
+    p.counters = counters.of(tickets);
+    if (!p.counters && tickets <= ATTN_TICKETS)
+      p.ticket0 = attn_take_tickets(tickets);
+  }
   const dim3 grid((unsigned)(group ? groups : B * Nq), (unsigned)splits);
   if (group && rot)
     attn_decode_group_kernel<true><<<grid, dim3(AG_WAVES * 64), 0, stream>>>(p);
@@ -2001,7 +2025,7 @@ static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t 
     attn_clear_tickets_kernel<<<dim3((n + 255) / 256), dim3(256), 0, stream>>>(p.ticket0, n);
     (void)hipGetLastError();
   }
-  if (rc || splits == 1 || p.ticket0 >= 0)
+  if (rc || splits == 1 || p.ticket0 >= 0 || p.counters)
     return rc;
   attn_combine_kernel<<<dim3((unsigned)(B * Nq)), dim3(128), 0, stream>>>(p);
   return check_hip(hipGetLastError(), who);
@@ -2030,7 +2054,7 @@ struct AttnGenParams {
   float scale;
   // single-query step (attn_hd_step_kernel):
   int splits;          // workgroups per query
-  int ticket0;         // splits > 1: first arrival counter of this launch
+  unsigned int* counters; // splits > 1: the caller's arrival counters, or null: attn_hd_merge_kernel follows
   float* part;         // splits > 1: [query][split][2 + H] floats (running maximum, sum, unnormalised output)
   // APP: the query and the step's new key / value arrive unrotated and not yet in the cache
   const uint16_t* k_new; // [B][Nkv][H]
@@ -2119,8 +2143,8 @@ attn_generic_kernel(const AttnGenParams p) {
 // made the relative error against float64 1.98 / 2.02 / 1.98e-3 for heads of 256 / 80 / 64, where rounding it against the maximum
 // of a lane group (the larger ones are then the 1 that bf16 holds exactly) gives 1.87 / 1.82 / 1.80e-3; in two terms it is 1.65 /
 // 1.63 / 1.63e-3, the rounding of the output, for at most 1 % of the time (64 heads of 80, 2500 keys 67.1 -> 68.0 us).
-// Grid (B * Nq, splits): split y takes the trips y, y + splits, ...; the split that arrives last merges all
-// of them in the launch.
+// Grid (B * Nq, splits): split y takes the trips y, y + splits, ...; where the caller gives arrival counters the split that
+// arrives last merges all of them in the launch.
 // APP: the launch also does what the rotary + append launch did before it (LayerCache::update, attn.h:198-222): wave 0
 // rotates the query and, in the split that reads its position, the new key -- rounded to bf16, as stored -- and that
 // position's lanes take key and value from there; one workgroup per KV head writes them into the cache.
@@ -2354,16 +2378,14 @@ attn_hd_step_kernel(const AttnGenParams p) {
       }
     }
   }
-  if (S == 1)
+  if (S == 1 || !p.counters) // (without counters attn_hd_merge_kernel follows)
     return;
   // as in attn_finish: own stores acknowledged, barrier, ticket, then the device-scope loads; nobody waits for anybody
   __shared__ int arrived_last;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (tid == 0) {
-    const unsigned int last = (unsigned int)S - 1;
-    arrived_last = atomicInc(&attn_tickets[(p.ticket0 + bh) * ATTN_TICKET_STRIDE], last) == last;
-  }
+  if (tid == 0)
+    arrived_last = attn_arrive(p.counters, 0, bh, S);
   __syncthreads();
   if (!arrived_last || tid >= H)
     return;
@@ -2396,8 +2418,36 @@ attn_hd_step_kernel(const AttnGenParams p) {
   p.out[(int64_t)bh * H + tid] = (uint16_t)f32_to_bf16_bits(Ls > 0.f ? o / Ls : 0.f);
 }
 
+// Without arrival counters: one wave per query, the splits' (maximum, sum, output) states, in split order, become the
+// normalised output -- the sums of the merge above.
+__global__ void __launch_bounds__(64)
+attn_hd_merge_kernel(const AttnGenParams p) {
+  const int lane = threadIdx.x;
+  const int64_t qi = blockIdx.x;
+  const int H = p.H;
+  const float* st = p.part + qi * p.splits * (int64_t)(H + 2);
+  float M = -3.0e38f;
+  for (int i = 0; i < p.splits; i++)
+    M = fmaxf(M, st[i * (H + 2)]);
+  float Ls = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < p.splits; i++) {
+    const float* si = st + i * (int64_t)(H + 2);
+    const float w = __expf(si[0] - M); // a split without keys carries sum 0 and output 0
+    Ls = fmaf(w, si[1], Ls);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (lane + 64 * j < H)
+        o[j] = fmaf(w, si[2 + lane + 64 * j], o[j]);
+  }
+  uint16_t* orow = p.out + qi * H;
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    if (lane + 64 * j < H)
+      orow[lane + 64 * j] = (uint16_t)f32_to_bf16_bits(Ls > 0.f ? o[j] / Ls : 0.f);
+}
+
 static int attn_generic_launch(const char* who, AttnGenParams& p, hipStream_t stream, void* ws = nullptr,
-                               int64_t ws_bytes = 0) {
+                               int64_t ws_bytes = 0, AttnCounters counters = {}) {
   TPPX_REQUIRE(p.H >= 8 && p.H <= 256 && p.H % 8 == 0, TPPX_EUNSUPPORTED,
                "%s: head size %d (128 on the tuned kernels, other multiples of 8 up to 256 on the plain one)", who, p.H);
   const int64_t queries = (int64_t)p.B * p.S * p.Nq;
@@ -2425,10 +2475,10 @@ static int attn_generic_launch(const char* who, AttnGenParams& p, hipStream_t st
           want = n;
     }
     want = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 32), most));
-    if (want > 1 && queries <= ATTN_TICKETS && ws && queries * want * (p.H + 2) * (int64_t)sizeof(float) <= ws_bytes) {
+    if (want > 1 && ws && queries * want * (p.H + 2) * (int64_t)sizeof(float) <= ws_bytes) {
       p.splits = (int)want;
       p.part = (float*)ws;
-      p.ticket0 = attn_take_tickets(queries);
+      p.counters = env_int("TPPX_ATTN_ONE_LAUNCH", 1) != 0 ? counters.of(queries) : nullptr;
     }
     const dim3 grid((unsigned)queries, (unsigned)p.splits);
     auto go = [&](auto app) {
@@ -2444,6 +2494,10 @@ static int attn_generic_launch(const char* who, AttnGenParams& p, hipStream_t st
       go(std::true_type{});
     else
       go(std::false_type{});
+    int rc = check_hip(hipGetLastError(), who);
+    if (rc || p.splits == 1 || p.counters)
+      return rc;
+    attn_hd_merge_kernel<<<dim3((unsigned)queries), dim3(64), 0, stream>>>(p);
     return check_hip(hipGetLastError(), who);
   }
   TPPX_REQUIRE(!p.k_new, TPPX_EUNSUPPORTED, "%s: the single-query kernel is switched off", who);
@@ -2453,11 +2507,12 @@ static int attn_generic_launch(const char* who, AttnGenParams& p, hipStream_t st
   return check_hip(hipGetLastError(), who);
 }
 
-extern "C" int tppx_attn_decode(const void* q, const void* kcache, const void* vcache, const void* mask,
-                                int64_t mask_ld, const void* kv_len_dev, int64_t kv_len_add, void* out, int64_t B, int64_t Nq,
-                                int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes,
-                                tppx_stream_t stream) {
-  const char* who = "tppx_attn_decode";
+static int run_attn_decode(const char* who, const void* q, const void* kcache, const void* vcache, const void* mask,
+                           int64_t mask_ld, const void* kv_len_dev, int64_t kv_len_add, void* out, int64_t B, int64_t Nq,
+                           int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes, const AttnCounters& counters,
+                           tppx_stream_t stream) {
+  if (int rc = check_counters(who, counters))
+    return rc;
   TPPX_REQUIRE(q && kcache && vcache && kv_len_dev && out, TPPX_EINVAL, "%s: null pointer", who);
   TPPX_REQUIRE(aligned16(q) && aligned16(kcache) && aligned16(vcache) && aligned16(out), TPPX_EINVAL,
                "%s: pointer not 16-byte aligned", who);
@@ -2471,7 +2526,7 @@ extern "C" int tppx_attn_decode(const void* q, const void* kcache, const void* v
     g.kv_len = (const int32_t*)kv_len_dev; g.kv_len_add = (int)kv_len_add; g.out = (uint16_t*)out;
     g.B = (int)B; g.S = 1; g.Nq = (int)Nq; g.Nkv = (int)Nkv; g.H = (int)H; g.Smax = (int)Smax; g.mask_ld = (int)mask_ld;
     g.scale = 1.0f / sqrtf((float)H);
-    return attn_generic_launch(who, g, (hipStream_t)stream, ws, ws_bytes);
+    return attn_generic_launch(who, g, (hipStream_t)stream, ws, ws_bytes, counters);
   }
   AttnParams p;
   memset(&p, 0, sizeof(p));
@@ -2479,15 +2534,16 @@ extern "C" int tppx_attn_decode(const void* q, const void* kcache, const void* v
   p.mask = (const uint16_t*)mask; p.kv_len = (const int32_t*)kv_len_dev; p.kv_len_add = (int)kv_len_add; p.out = (uint16_t*)out;
   p.B = (int)B; p.Nq = (int)Nq; p.Nkv = (int)Nkv; p.Smax = (int)Smax; p.mask_ld = (int)mask_ld;
   p.scale = 1.0f / sqrtf((float)H);
-  return attn_decode_launch(who, p, false, B, Nq, Smax, ws, ws_bytes, (hipStream_t)stream);
+  return attn_decode_launch(who, p, false, B, Nq, Smax, ws, ws_bytes, counters, (hipStream_t)stream);
 }
 
-extern "C" int tppx_attn_decode_rotary(const void* q, const void* k, const void* v, const void* emb_pos,
-                                       const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache,
-                                       void* vcache, const void* mask, int64_t mask_ld, const void* kv_len_dev,
-                                       void* out, int64_t B, int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
-                                       void* ws, int64_t ws_bytes, tppx_stream_t stream) {
-  const char* who = "tppx_attn_decode_rotary";
+static int run_attn_decode_rotary(const char* who, const void* q, const void* k, const void* v, const void* emb_pos,
+                                  const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache, void* vcache,
+                                  const void* mask, int64_t mask_ld, const void* kv_len_dev, void* out, int64_t B,
+                                  int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes,
+                                  const AttnCounters& counters, tppx_stream_t stream) {
+  if (int rc = check_counters(who, counters))
+    return rc;
   TPPX_REQUIRE(q && k && v && pos && kcache && vcache && kv_len_dev && out, TPPX_EINVAL, "%s: null pointer", who);
   TPPX_REQUIRE(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(kcache) && aligned16(vcache) && aligned16(out) &&
                    (!emb_pos || aligned16(emb_pos)),
@@ -2507,15 +2563,16 @@ extern "C" int tppx_attn_decode_rotary(const void* q, const void* k, const void*
   p.scale = 1.0f / sqrtf((float)H);
   p.k_new = (const uint16_t*)k; p.v_new = (const uint16_t*)v; p.emb = (const float*)emb_pos; p.pos = (const int64_t*)pos;
   p.MP = (int)MP; p.B_pos = (int)B_pos;
-  return attn_decode_launch(who, p, true, B, Nq, Smax, ws, ws_bytes, (hipStream_t)stream);
+  return attn_decode_launch(who, p, true, B, Nq, Smax, ws, ws_bytes, counters, (hipStream_t)stream);
 }
 
-extern "C" int tppx_attn_decode_append(const void* q, const void* k, const void* v, const void* emb_pos, int gptj,
-                                       const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache, void* vcache,
-                                       const void* mask, int64_t mask_ld, const void* kv_len_dev, void* out, int64_t B,
-                                       int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes,
-                                       tppx_stream_t stream) {
-  const char* who = "tppx_attn_decode_append";
+static int run_attn_decode_append(const char* who, const void* q, const void* k, const void* v, const void* emb_pos,
+                                  int gptj, const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache,
+                                  void* vcache, const void* mask, int64_t mask_ld, const void* kv_len_dev, void* out,
+                                  int64_t B, int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes,
+                                  const AttnCounters& counters, tppx_stream_t stream) {
+  if (int rc = check_counters(who, counters))
+    return rc;
   TPPX_REQUIRE(q && k && v && pos && kcache && vcache && kv_len_dev && out, TPPX_EINVAL, "%s: null pointer", who);
   TPPX_REQUIRE(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(kcache) && aligned16(vcache) && aligned16(out),
                TPPX_EINVAL, "%s: pointer not 16-byte aligned", who);
@@ -2534,7 +2591,62 @@ extern "C" int tppx_attn_decode_append(const void* q, const void* k, const void*
   g.scale = 1.0f / sqrtf((float)H);
   g.k_new = (const uint16_t*)k; g.v_new = (const uint16_t*)v; g.emb = (const float*)emb_pos; g.pos = (const int64_t*)pos;
   g.MP = (int)MP; g.HR = emb_pos ? (int)HR : 0; g.B_pos = (int)B_pos; g.gptj = gptj != 0;
-  return attn_generic_launch(who, g, (hipStream_t)stream, ws, ws_bytes);
+  return attn_generic_launch(who, g, (hipStream_t)stream, ws, ws_bytes, counters);
+}
+
+extern "C" int tppx_attn_decode(const void* q, const void* kcache, const void* vcache, const void* mask, int64_t mask_ld,
+                                const void* kv_len_dev, int64_t kv_len_add, void* out, int64_t B, int64_t Nq, int64_t Nkv,
+                                int64_t H, int64_t Smax, void* ws, int64_t ws_bytes, tppx_stream_t stream) {
+  return run_attn_decode("tppx_attn_decode", q, kcache, vcache, mask, mask_ld, kv_len_dev, kv_len_add, out, B, Nq, Nkv, H,
+                         Smax, ws, ws_bytes, {}, stream);
+}
+
+extern "C" int tppx_attn_decode_counted(const void* q, const void* kcache, const void* vcache, const void* mask,
+                                        int64_t mask_ld, const void* kv_len_dev, int64_t kv_len_add, void* out, int64_t B,
+                                        int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes,
+                                        void* counters, int64_t counter_bytes, tppx_stream_t stream) {
+  return run_attn_decode("tppx_attn_decode_counted", q, kcache, vcache, mask, mask_ld, kv_len_dev, kv_len_add, out, B, Nq,
+                         Nkv, H, Smax, ws, ws_bytes, {counters, counter_bytes}, stream);
+}
+
+extern "C" int tppx_attn_decode_rotary(const void* q, const void* k, const void* v, const void* emb_pos, const void* pos,
+                                       int64_t B_pos, int64_t MP, int64_t HR, void* kcache, void* vcache,
+                                       const void* mask, int64_t mask_ld, const void* kv_len_dev, void* out, int64_t B,
+                                       int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes,
+                                       tppx_stream_t stream) {
+  return run_attn_decode_rotary("tppx_attn_decode_rotary", q, k, v, emb_pos, pos, B_pos, MP, HR, kcache, vcache, mask,
+                                mask_ld, kv_len_dev, out, B, Nq, Nkv, H, Smax, ws, ws_bytes, {}, stream);
+}
+
+extern "C" int tppx_attn_decode_rotary_counted(const void* q, const void* k, const void* v, const void* emb_pos,
+                                               const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache,
+                                               void* vcache, const void* mask, int64_t mask_ld, const void* kv_len_dev,
+                                               void* out, int64_t B, int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
+                                               void* ws, int64_t ws_bytes, void* counters, int64_t counter_bytes,
+                                               tppx_stream_t stream) {
+  return run_attn_decode_rotary("tppx_attn_decode_rotary_counted", q, k, v, emb_pos, pos, B_pos, MP, HR, kcache, vcache,
+                                mask, mask_ld, kv_len_dev, out, B, Nq, Nkv, H, Smax, ws, ws_bytes,
+                                {counters, counter_bytes}, stream);
+}
+
+extern "C" int tppx_attn_decode_append(const void* q, const void* k, const void* v, const void* emb_pos, int gptj,
+                                       const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache, void* vcache,
+                                       const void* mask, int64_t mask_ld, const void* kv_len_dev, void* out, int64_t B,
+                                       int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax, void* ws, int64_t ws_bytes,
+                                       tppx_stream_t stream) {
+  return run_attn_decode_append("tppx_attn_decode_append", q, k, v, emb_pos, gptj, pos, B_pos, MP, HR, kcache, vcache,
+                                mask, mask_ld, kv_len_dev, out, B, Nq, Nkv, H, Smax, ws, ws_bytes, {}, stream);
+}
+
+extern "C" int tppx_attn_decode_append_counted(const void* q, const void* k, const void* v, const void* emb_pos, int gptj,
+                                               const void* pos, int64_t B_pos, int64_t MP, int64_t HR, void* kcache,
+                                               void* vcache, const void* mask, int64_t mask_ld, const void* kv_len_dev,
+                                               void* out, int64_t B, int64_t Nq, int64_t Nkv, int64_t H, int64_t Smax,
+                                               void* ws, int64_t ws_bytes, void* counters, int64_t counter_bytes,
+                                               tppx_stream_t stream) {
+  return run_attn_decode_append("tppx_attn_decode_append_counted", q, k, v, emb_pos, gptj, pos, B_pos, MP, HR, kcache,
+                                vcache, mask, mask_ld, kv_len_dev, out, B, Nq, Nkv, H, Smax, ws, ws_bytes,
+                                {counters, counter_bytes}, stream);
 }
 
 extern "C" int tppx_attn_prefill(const void* q, const void* kcache, const void* vcache, const void* mask,

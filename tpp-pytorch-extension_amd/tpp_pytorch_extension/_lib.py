@@ -111,6 +111,11 @@ SIGNATURES = {
     "tppx_attn_decode_rotary": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp],
     "tppx_attn_decode_append": [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64,
                                 _i64, _i64, _vp, _i64, _vp],
+    "tppx_attn_decode_counted": [_vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp],
+    "tppx_attn_decode_rotary_counted": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64,
+                                        _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp],
+    "tppx_attn_decode_append_counted": [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _i64,
+                                        _i64, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp],
     "tppx_attn_prefill": [_vp, _vp, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp],
     "tppx_plan_linear_mxfp4": [_i64, _i64, _i64, _i32, _i64, ctypes.c_char_p, _i64],
     "tppx_plan_linear_qint8": [_i64, _i64, _i64, _i64, _i32, _i32, _i64, ctypes.c_char_p, _i64],
@@ -159,6 +164,7 @@ def stream_of(t):
 
 
 WORKSPACE_BYTES = 32 << 20
+COUNTER_BYTES = 1 << 20  # behind it: arrival counters of split-KV attention, 256 bytes per (sequence, head)
 MAX_STREAM_WORKSPACES = 8  # per device; the least recently used one beyond that is released
 _workspaces = {}
 _workspaces_lock = threading.Lock()
@@ -177,7 +183,8 @@ def workspace(t, stream=None):
     these ops with respect to each other.  A device keeps at most
     MAX_STREAM_WORKSPACES per-stream buffers: beyond that the least recently
     used one goes back to torch's allocator (it was allocated on its own stream,
-    so work still queued there keeps it valid)."""
+    so work still queued there keeps it valid).  with_counters(): arrival
+    counters behind the buffer, under the same ordering."""
     global _tick
     dev = t.device.index
     if torch.cuda.is_current_stream_capturing():
@@ -193,7 +200,7 @@ def workspace(t, stream=None):
             ws = _workspaces.get(key)
             if ws is None:
                 if (dev, "capture") not in _workspaces:
-                    cap = torch.zeros(WORKSPACE_BYTES, dtype=torch.uint8, device=t.device)
+                    cap = torch.zeros(WORKSPACE_BYTES + COUNTER_BYTES, dtype=torch.uint8, device=t.device)[:WORKSPACE_BYTES]
                     torch.cuda.current_stream(t.device).synchronize()  # zeroed before any capture stream sees it
                     _workspaces[(dev, "capture")] = cap
                 mine = [k for k in _workspace_use if k[0] == dev]
@@ -201,11 +208,18 @@ def workspace(t, stream=None):
                     old = min(mine, key=_workspace_use.get)
                     _workspace_use.pop(old)
                     _workspaces.pop(old, None)
-                ws = torch.zeros(WORKSPACE_BYTES, dtype=torch.uint8, device=t.device)
+                ws = torch.zeros(WORKSPACE_BYTES + COUNTER_BYTES, dtype=torch.uint8, device=t.device)[:WORKSPACE_BYTES]
                 _workspaces[key] = ws
     _tick += 1
     _workspace_use[key] = _tick
     return ws
+
+
+def with_counters(ws):
+    """(address, bytes, address of its arrival counters, their bytes) of a workspace() buffer.  The counters are zeros outside
+    of the launches that count on them, and no other launch writes there."""
+    at = ws.data_ptr()
+    return at, WORKSPACE_BYTES, at + WORKSPACE_BYTES, COUNTER_BYTES
 
 
 def require_gpu(t, what):

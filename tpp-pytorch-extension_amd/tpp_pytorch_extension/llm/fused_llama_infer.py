@@ -251,10 +251,10 @@ def rotate_append_attend(q, k, v, t_am, t_pid, cache, layer_idx, B, S, Nq, Nkv, 
     if S == 1 and FUSE_ROTARY and H != 128:
         ctx = torch.empty_like(q)
         table, MP, HR = (None, 1, H) if style is None else (t_EP.data_ptr(), *t_EP.shape[-2:])
-        rc = L.tppx_attn_decode_append(
+        rc = L.tppx_attn_decode_append_counted(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), table, style == "gptj", t_pid.data_ptr(), t_pid.shape[0], MP, HR,
             kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld, cache.seq_len_dev.data_ptr(), ctx.data_ptr(), B, Nq, Nkv, H,
-            cache.capacity, ws.data_ptr(), ws.numel(), st)
+            cache.capacity, *_lib.with_counters(ws), st)
         if rc != _lib.EUNSUPPORTED:  # (head sizes past 256, the kernel switched off)
             _lib.check(rc)
             return ctx
@@ -271,9 +271,9 @@ def rotate_append_attend(q, k, v, t_am, t_pid, cache, layer_idx, B, S, Nq, Nkv, 
             t_pid.shape[0], cache.capacity, st))
     ctx = torch.empty_like(q)
     if S == 1:
-        _lib.check(L.tppx_attn_decode(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld,
-                                      cache.seq_len_dev.data_ptr(), 1, ctx.data_ptr(), B, Nq, Nkv, H, cache.capacity,
-                                      ws.data_ptr(), ws.numel(), st))
+        _lib.check(L.tppx_attn_decode_counted(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld,
+                                              cache.seq_len_dev.data_ptr(), 1, ctx.data_ptr(), B, Nq, Nkv, H, cache.capacity,
+                                              *_lib.with_counters(ws), st))
     else:
         _lib.check(L.tppx_attn_prefill(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld,
                                        cache.get_seq_length(), ctx.data_ptr(), B, S, Nq, Nkv, H, cache.capacity, st))
@@ -306,8 +306,8 @@ def attn(t_QL, t_KL, t_VL, t_AM, cache, layer_idx, isCausal=True):
     mask_ptr, mask_ld = (mask.data_ptr(), mask.shape[-1]) if mask is not None else (None, 0)
     klen = torch.full((1,), key_len, dtype=torch.int32, device=q.device)
     if Sq == 1:
-        _lib.check(L.tppx_attn_decode(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld, klen.data_ptr(), 0,
-                                      out.data_ptr(), B, Nkv * R, Nkv, H, core.capacity, ws.data_ptr(), ws.numel(), st))
+        _lib.check(L.tppx_attn_decode_counted(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld, klen.data_ptr(),
+                                              0, out.data_ptr(), B, Nkv * R, Nkv, H, core.capacity, *_lib.with_counters(ws), st))
     else:
         _lib.check(L.tppx_attn_prefill(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld, key_len - Sq,
                                        out.data_ptr(), B, Sq, Nkv * R, Nkv, H, core.capacity, st))
@@ -419,11 +419,11 @@ class LlamaDecoderLayer(FormatSwitches):
         if S == 1 and FUSE_ROTARY and self.H == 128 and self.t_EP.shape[2] == 128:
             # decode step: rotary, cache append and attention in one launch
             ctx = torch.empty_like(q)
-            _lib.check(L.tppx_attn_decode_rotary(
+            _lib.check(L.tppx_attn_decode_rotary_counted(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), self.t_EP.data_ptr(), t_pid.data_ptr(), t_pid.shape[0],
                 self.t_EP.shape[1], self.t_EP.shape[2], kc.data_ptr(), vc.data_ptr(), mask_ptr, mask_ld,
                 cache.seq_len_dev.data_ptr(), ctx.data_ptr(), B, self.Nq, self.Nkv, self.H, cache.capacity,
-                ws.data_ptr(), ws.numel(), st))
+                *_lib.with_counters(ws), st))
             return self._after_attention(ctx, t_res, empty, cache, sums_attn, sums_out, Wp, Wg, Wu, Wd)
         ctx = rotate_append_attend(q, k, v, t_am, t_pid, cache, self.layer_idx, B, S, self.Nq, self.Nkv, self.H,
                                    self.t_EP, "llama")

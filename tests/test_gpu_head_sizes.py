@@ -406,3 +406,32 @@ def test_decoder_blocks_count_arrivals_in_their_own_workspace(monkeypatch):
         F.rotate_append_attend(*qkv, None, torch.zeros((1, 1), dtype=torch.int64, device="cuda"), cache, 0, 1, 1, N, N, H, table, style)
     torch.cuda.synchronize()
     assert seen == ["tppx_attn_decode_append_counted"] * 2 + ["tppx_attn_decode_counted"]
+
+
+@pytest.mark.parametrize("H,Nq,Nkv", [(128, 28, 4), (128, 4, 4), (80, 8, 2)])
+def test_a_mask_of_no_keys_masks_nothing(H, Nq, Nkv):
+    """A mask pointer with mask_ld 0 is as good as none: nothing is read there, by tppx_attn_decode and by the forms that
+    append the new token (all of them read the pointer's surroundings here: valid memory that would mask every key)."""
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+    q, k, v = (randn_bf16(s, 1.0, 341 + i).cuda() for i, s in enumerate(((2, Nq, H), (2, Nkv, 128, H), (2, Nkv, 128, H))))
+    k0, v0 = k[:, :, 0].contiguous(), v[:, :, 0].contiguous()
+    low = torch.full((4096,), -1e30, dtype=torch.bfloat16, device="cuda")
+    n, pos = torch.tensor([76], dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda")
+    ws, st = _lib.workspace(q), _lib.stream_of(q)
+    for append in (False, True):
+        outs = []
+        for mask in (None, low[2048:].data_ptr()):
+            kc, vc, out = k.clone(), v.clone(), torch.empty_like(q)
+            end = (n.data_ptr(),) + ((out.data_ptr(),) if append else (1, out.data_ptr())) + (2, Nq, Nkv, H, 128, ws.data_ptr(), ws.numel(), st)
+            new = (q.data_ptr(), k0.data_ptr(), v0.data_ptr(), None)
+            at = (pos.data_ptr(), 1, 1, H, kc.data_ptr(), vc.data_ptr(), mask, 0)
+            if not append:
+                _lib.check(L.tppx_attn_decode(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), mask, 0, *end))
+            elif H == 128:
+                _lib.check(L.tppx_attn_decode_rotary(*new, *at, *end))
+            else:
+                _lib.check(L.tppx_attn_decode_append(*new, 0, *at, *end))
+            outs.append(out)
+        torch.cuda.synchronize()
+        assert torch.equal(*outs)

@@ -1991,6 +1991,8 @@ static int attn_decode_launch(const char* who, AttnParams& p, bool rot, int64_t 
   if (gsplits > 1 && (B * Nq * gsplits * 130 * (int64_t)sizeof(float) > ws_bytes || !aligned16(ws)))
     gsplits = 1;
   const bool group = wide && Nq > p.Nkv && env_int("TPPX_ATTN_GROUP", 1) != 0;
+  if (p.mask_ld <= 0)
+    p.mask = nullptr; // a mask of no keys: the grouped kernel clamps its reads to the mask's last key
   if (group)
     splits = gsplits;
   const int64_t need = B * Nq * splits * 130 * (int64_t)sizeof(float);

@@ -796,6 +796,37 @@ def test_float_and_half_activations_in_terms_of_bf16(M, N, K, dtype, wkind):
     assert torch.allclose(y[2].double(), ref[2].double(), rtol=near, atol=near * float(ref[2].double().abs()[ref[2].isfinite()].max()), equal_nan=True)
 
 
+@pytest.mark.parametrize("wkind", ["mxfp4", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1, 32, 128), (16, 8224, 256), (17, 96, 1152), (33, 4128, 384), (64, 64, 2304), (130, 8288, 256)])
+def test_float_rows_of_any_size_keep_their_bits(M, N, K, wkind):
+    """Rows of 2^-112 down to 2^-130, whose values have bits below bf16's smallest number, next to ordinary rows and one with an
+    infinity: the bound of ordinary rows, 4 fp32 ulps of sum |x||w|, and fp32's own last place (2^-149) per product; the
+    ordinary rows have the bits that they have among their like."""
+    ops = _ops()
+    W = randn_bf16((N, K), 0.5, 181)
+    if wkind == "mxfp4":
+        w = ops.remap_and_quantize_mxfp4(block_bf16(W).cuda())
+        Wd = torch.from_numpy(O.dequantize_mxfp4_plain(*O.remap_quantize_mxfp4(W.float().numpy()))).double()
+    else:
+        w, Wd = block_bf16(W).cuda(), W.double()
+    g = torch.Generator().manual_seed(182)
+    x = torch.randn((M, K), generator=g)
+    plain = ops.fc_plain(x.cuda(), w, None).cpu()
+    rows = torch.arange(M)
+    small = x * torch.exp2(-112.0 - (rows % 19).float()).unsqueeze(1)
+    tiny = rows % 3 != 1
+    mixed = torch.where(tiny.unsqueeze(1), small, x)
+    if M > 4:
+        mixed[4, K - 1] = float("inf")
+    y = ops.fc_plain(mixed.cuda(), w, None).cpu()
+    ref, mag = mixed.double() @ Wd.T, mixed.double().abs() @ Wd.abs().T
+    fine = mag.isfinite().all(1)
+    assert ((y[fine].double() - ref[fine]).abs() <= 4 * 2.0 ** -23 * mag[fine] + K * 2.0 ** -149).all()
+    assert torch.equal(y[~fine].isnan(), ref[~fine].isnan()) and not y[~fine].isfinite().any()
+    same = fine & ~tiny
+    assert torch.equal(y[same], plain[same])
+
+
 def _qint(kind, W):
     ops = _ops()
     if kind == "qint8":

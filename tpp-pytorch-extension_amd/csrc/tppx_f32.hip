@@ -318,8 +318,10 @@ linear_qint8_wide_rows_kernel(const F32OutParams p) {
 // Every weight value is a bf16.  An activation is cut into bf16 terms that add up to it exactly -- its leading 8
 // significant bits, the next 8, and for fp32 the last 8 -- so two (half) or three (float) bf16 MFMAs form the products
 // that an fp32 MFMA would, at 16 times its rate each; terms are cut off, not rounded, so none is larger than the value.
-// An infinite or NaN activation has no such terms (Inf - Inf), and 0 * Inf weights give a NaN that is not there: an
-// output that comes out non-finite is computed again by its thread, value by value.
+// Two kinds of activations have no such terms.  Below 2^-110 the last ones would lie under the smallest bf16, 2^-133: what the
+// three terms of a value leave over shows in the lower half of the third one's float.  And an infinity or NaN gives Inf - Inf:
+// outputs that come out non-finite.  Rows and outputs with either are formed again by the workgroup on the fp32 MFMA, from the
+// values as they are; the others keep the sums they have, so a row does not depend on its neighbours.
 // Native layouts: lane (g, n) of a 128-channel K tile holds the 32 weights k = g*32 .. g*32 + 31 of channel n; MFMA j
 // multiplies channels g*32 + j*8 .. + 7 of each group g.
 // ---------------------------------------------------------------------------
@@ -335,9 +337,9 @@ __device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) {
   return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 
-// eight activations -> TERMS bf16 operands
+// eight activations -> TERMS bf16 operands; over: its low half collects what they leave over
 template <bool XHALF>
-__device__ __forceinline__ void split_terms(const i32x4* raw, bf16x8* out) {
+__device__ __forceinline__ void split_terms(const i32x4* raw, bf16x8* out, uint32_t& over) {
   constexpr int TERMS = XHALF ? 2 : 3;
   uint32_t part[TERMS][4];
 #pragma unroll
@@ -357,6 +359,8 @@ __device__ __forceinline__ void split_terms(const i32x4* raw, bf16x8* out) {
       if (t + 1 < TERMS) {
         v[0] -= __uint_as_float(__float_as_uint(v[0]) & 0xffff0000u);
         v[1] -= __uint_as_float(__float_as_uint(v[1]) & 0xffff0000u);
+      } else if (!XHALF) {
+        asm("v_or3_b32 %0, %1, %2, %0" : "+v"(over) : "v"(v[0]), "v"(v[1]));
       }
     }
   }
@@ -372,33 +376,20 @@ __device__ __forceinline__ bf16x8 expand_codes(uint32_t c, float sc) {
   return bf16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
 
-// one output, value by value in ascending k
-template <bool XHALF, bool WBF16>
-__device__ __noinline__ float wide_dot(const WideParams& p, int m, int n) {
-  float s = 0.f;
-  const int KT = p.o.K / 128;
-  for (int c = 0; c < p.o.K / 32; c++) { // 32 channels: K group c % 4 of K tile c / 4
-    const int64_t slot = ((int64_t)(n / 16) * KT + (c >> 2)) * (WBF16 ? 256 : 64) + (c & 3) * 16 + (n & 15);
-    for (int j = 0; j < 4; j++) {
-      const bf16x8 w = WBF16 ? __builtin_bit_cast(bf16x8, reinterpret_cast<const i32x4*>(p.qw)[slot + j * 64])
-                             : expand_codes(reinterpret_cast<const uint32_t*>(p.qw)[slot * 4 + j], e8m0_to_f32(p.sw[slot]));
-      for (int e = 0; e < 8; e++)
-        s = fmaf(load_elem(p.x, XHALF ? TPPX_DT_F16 : TPPX_DT_F32, (int64_t)m * p.o.K + c * 32 + j * 8 + e), (float)w[e], s);
-    }
-  }
-  return s;
-}
-
 // MT row tiles x NT channel tiles per workgroup, its eight waves on every eighth K tile, partial tiles summed through
-// LDS in wave order.  Bound by the chain of a wave's K tiles with few rows (16 x 4096 x 4096 12.5 us in half, 16 in
+// LDS in wave order.  Bound by the chain of a wave's K tiles with few rows (16 x 4096 x 4096 12.2 us in half, 12.5 in
 // float), by cutting the activations and by the LDS sums with many.  Its error against float64 is a fifth of that of
 // one wave per 16 x 16 outputs on the fp32 MFMA (61 x 3264 x 8704 in float: 3.1e-7 relative against 1.6e-6), as eight
-// partial sums of 32 products at a time round less often than one of four.
+// partial sums of 32 products at a time round less often than one of four.  A workgroup that forms its outputs again takes the
+// time of the fp32 MFMA on top (one infinity in 61 x 3264 x 8704 in half 21 -> 67 us, a row of 2^-118 in float 38 -> 90;
+// all on the fp32 MFMA 64 and 104).
 template <bool XHALF, bool WBF16, int MT, int NT>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, MT * NT <= 2 ? 4 : 2) // two workgroups to a CU while their tiles are small
 linear_wide_kernel(const WideParams p) {
   constexpr int W = 8, T = MT * NT, TERMS = XHALF ? 2 : 3, XV = XHALF ? 1 : 2, BV = WBF16 ? 4 : 1;
-  __shared__ float part[W][T * 256];
+  __shared__ __align__(16) float part[W][T * 256];
+  __shared__ __align__(16) uint16_t rows_over[MT][W]; // bit r: row r of the tile has activations beyond three terms
+  __shared__ int again;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
   const int tiles = p.o.N / 16, tile0 = blockIdx.x * NT, m0 = blockIdx.y * MT * 16, KT = p.o.K / 128;
   const i32x4* wq[NT];
@@ -420,6 +411,7 @@ linear_wide_kernel(const WideParams p) {
 #pragma unroll
     for (int ni = 0; ni < NT; ni++)
       acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint32_t over[MT] = {};
   i32x4 wb[NT][BV];
   uint32_t sb[NT];
   auto request = [&](int kt) {
@@ -462,7 +454,7 @@ linear_wide_kernel(const WideParams p) {
 #pragma unroll
       for (int mi = 0; mi < MT; mi++) {
         bf16x8 x[TERMS];
-        split_terms<XHALF>(xv[j][mi], x);
+        split_terms<XHALF>(xv[j][mi], x, over[mi]);
 #pragma unroll
         for (int t = TERMS - 1; t >= 0; t--)
 #pragma unroll
@@ -476,20 +468,119 @@ linear_wide_kernel(const WideParams p) {
 #pragma unroll
     for (int ni = 0; ni < NT; ni++)
       *reinterpret_cast<f32x4*>(&part[wave][(mi * NT + ni) * 256 + lane * 4]) = acc[mi][ni];
-  __syncthreads();
-  for (int o = threadIdx.x; o < T * 256; o += 512) {
-    const int t = o >> 8, l = (o & 255) >> 2;
-    const int m = m0 + (t / NT) * 16 + (l >> 4) * 4 + (o & 3), n = (tile0 + t % NT) * 16 + (l & 15);
-    if (m >= p.o.M || n >= p.o.N)
-      continue;
-    float s = part[0][o];
+  if (!XHALF) {
 #pragma unroll
-    for (int w = 1; w < W; w++)
-      s += part[w][o];
-    if (!(fabsf(s) <= 3.4028234663852886e38f))
-      s = wide_dot<XHALF, WBF16>(p, m, n);
-    wide_store(p.o, m, n, p.o.bias ? load_elem(p.o.bias, p.o.bias_dtype, n) + s : s);
+    for (int mi = 0; mi < MT; mi++) {
+      uint64_t rows = __builtin_amdgcn_ballot_w64((over[mi] & 0xffffu) != 0); // lane (g, row)
+      rows |= rows >> 32;
+      rows |= rows >> 16;
+      if (lane == 0)
+        rows_over[mi][wave] = (uint16_t)rows;
+    }
   }
+  if (threadIdx.x == 0)
+    again = 0;
+  __syncthreads();
+  uint32_t overs[MT] = {}, any_over = 0; // per row tile, of all waves
+  if (!XHALF) {
+#pragma unroll
+    for (int mi = 0; mi < MT; mi++) {
+      const i32x4 r = *reinterpret_cast<const i32x4*>(rows_over[mi]);
+      const uint32_t u = (uint32_t)(r[0] | r[1] | r[2] | r[3]);
+      overs[mi] = (u | u >> 16) & 0xffffu;
+      any_over |= overs[mi];
+    }
+  }
+  constexpr int OPT = (T * 256 + 511) / 512; // outputs per thread
+  auto each = [&](auto&& f) {
+#pragma unroll
+    for (int i = 0; i < OPT; i++) {
+      const int o = threadIdx.x + i * 512, t = o >> 8, l = (o & 255) >> 2, r = (l >> 4) * 4 + (o & 3);
+      const int m = m0 + (t / NT) * 16 + r, n = (tile0 + t % NT) * 16 + (l & 15);
+      if (o >= T * 256 || m >= p.o.M || n >= p.o.N)
+        continue;
+      float s = part[0][o];
+#pragma unroll
+      for (int w = 1; w < W; w++)
+        s += part[w][o];
+      f(i, t / NT, r, m, n, s);
+    }
+  };
+  auto store = [&](int m, int n, float s) { wide_store(p.o, m, n, p.o.bias ? load_elem(p.o.bias, p.o.bias_dtype, n) + s : s); };
+  uint32_t redo = 0; // bit i: this thread's i-th output
+  each([&](int i, int mi, int r, int m, int n, float s) {
+    bool over_row = false;
+    if (any_over) {
+#pragma unroll
+      for (int k = 0; k < MT; k++)
+        over_row |= k == mi && (overs[k] >> r & 1u);
+    }
+    if (over_row || !(fabsf(s) <= 3.4028234663852886e38f))
+      redo |= 1u << i;
+    else
+      store(m, n, s);
+  });
+  if (redo)
+    again = 1;
+  __syncthreads();
+  if (!again) // the same for the whole workgroup
+    return;
+#pragma unroll
+  for (int mi = 0; mi < MT; mi++)
+#pragma unroll
+    for (int ni = 0; ni < NT; ni++)
+      acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int ln = lane; // (hidden from the compiler, which would keep the operands' addresses in registers through the loop above)
+  asm volatile("" : "+v"(ln));
+#pragma unroll 1
+  for (int kt = wave; kt < KT; kt += W) {
+#pragma unroll 1
+    for (int j = 0; j < 4; j++) { // MFMA e: channels g * 32 + j * 8 + e of the four groups
+      float x[MT][8], w[NT][8];
+#pragma unroll
+      for (int mi = 0; mi < MT; mi++) {
+        const i32x4* src = reinterpret_cast<const i32x4*>(reinterpret_cast<const char*>(p.x) +
+            ((int64_t)min(m0 + mi * 16 + (ln & 15), p.o.M - 1) * p.o.K + kt * 128 + (ln >> 4) * 32 + j * 8) * (XHALF ? 2 : 4));
+        i32x4 v[XV];
+#pragma unroll
+        for (int k = 0; k < XV; k++)
+          v[k] = src[k];
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          x[mi][e] = XHALF ? (float)__builtin_bit_cast(_Float16, (uint16_t)((uint32_t)v[0][e >> 1] >> (16 * (e & 1))))
+                           : __int_as_float(v[XHALF ? 0 : e >> 2][e & 3]);
+      }
+#pragma unroll
+      for (int ni = 0; ni < NT; ni++) {
+        const int64_t slot = (int64_t)min(tile0 + ni, tiles - 1) * KT + kt;
+        bf16x8 b;
+        if constexpr (WBF16)
+          b = __builtin_bit_cast(bf16x8, reinterpret_cast<const i32x4*>(p.qw)[(slot * 4 + j) * 64 + ln]);
+        else
+          b = expand_codes(reinterpret_cast<const uint32_t*>(p.qw)[(slot * 64 + ln) * 4 + j], e8m0_to_f32(p.sw[slot * 64 + ln]));
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          w[ni][e] = (float)b[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+#pragma unroll
+        for (int mi = 0; mi < MT; mi++)
+#pragma unroll
+          for (int ni = 0; ni < NT; ni++)
+            acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[mi][e], w[ni][e], acc[mi][ni], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int mi = 0; mi < MT; mi++)
+#pragma unroll
+    for (int ni = 0; ni < NT; ni++)
+      *reinterpret_cast<f32x4*>(&part[wave][(mi * NT + ni) * 256 + lane * 4]) = acc[mi][ni];
+  __syncthreads();
+  each([&](int i, int, int, int m, int n, float s) {
+    if (redo >> i & 1u)
+      store(m, n, s);
+  });
 }
 
 template <bool HALF>
@@ -549,8 +640,9 @@ static int run_linear_wide(const char* who, const void* x, int x_dtype, const vo
     // One row tile: two channel tiles once one each would be more than two rounds of workgroups.  Otherwise 32 rows x 16
     // channels while those fit one round, else x 32, and from a few rounds of those the largest tile whose operands and
     // partial sums still leave two waves per SIMD (64 x 64 with 4-bit weights, 64 x 32 with the four times wider bf16
-    // ones).  MXFP4 x half: 64 rows of 1088 x 9984 27 us on 32 x 16, 29 on 32 x 32, 54 on 64 x 64; 128 rows of
-    // 11008 x 4096 72 on 32 x 32, 61 on 64 x 64; float, with three terms to cut, at 512 rows of 11008 x 4096 489 and 390.
+    // ones).  MXFP4 x half: 64 rows of 1088 x 9984 21.3 us on 32 x 16, 22.4 on 32 x 32, 53.9 on 64 x 64; 128 rows of
+    // 11008 x 4096 51.2 on 32 x 32, 50.5 on 64 x 64; float, with three terms to cut, at 128 rows 105 and 112, at 512 rows 379
+    // and 327; bf16 weights x half at 128 rows 79.6 on 32 x 32, 65.6 on 64 x 32.
     typedef std::integral_constant<int, 1> one;
     typedef std::integral_constant<int, 2> two;
     typedef std::integral_constant<int, 4> four;

@@ -534,6 +534,16 @@ def test_w4a8_prompts_take_the_prompt_kernel():
             assert not _ops._w4a8_row_groups(m, n, k), (m, n, k)
 
 
+def test_w4a8_calls_run_on_the_faster_kernel():
+    """Calls where one of the two kernels was measured faster by 10 to 40 % (us in row groups, on the prompt kernel)."""
+    from tpp_pytorch_extension import _ops
+
+    for m, n, k in ((1957, 5056, 1280), (1398, 4416, 1024), (1555, 5056, 1280), (964, 8256, 1280), (512, 11008, 1024), (672, 8128, 1024)):
+        assert not _ops._w4a8_row_groups(m, n, k), (m, n, k)  # 80 / 60, 42 / 34, 66 / 54, 69 / 57, 39 / 33, 39 / 33
+    for m, n, k in ((400, 5120, 5120), (384, 7808, 10752), (323, 7360, 4096), (541, 5184, 9216), (1024, 2560, 10240), (600, 4864, 14336)):
+        assert _ops._w4a8_row_groups(m, n, k), (m, n, k)      # 59 / 80, 133 / 186, 56 / 78, 117 / 153, 114 / 149, 180 / 233
+
+
 def test_mxfp4_prompts_run_k_in_slices_where_that_pays():
     """Launch plans: K in slices where few workgroups have many steps; whole where the launch with whole K was measured
     faster, by 3 to 11 % (most of a round of workgroups, many row blocks) or as fast (4096 x 11008 at 333 rows)."""

@@ -681,25 +681,28 @@ W4A8_WIDE_ROWS = int(os.environ.get("TPPX_W4A8_WIDE_ROWS", "64"))
 
 def _w4a8_row_groups(M, N, K):
     """Does a W4A8 call of 64 or more rows run on the row-group kernel (4-bit weights, once per 64 rows) rather than on
-    the prompt kernel (2 bytes per weight)?  The same bits either way.  Both in us, the row quantizer included, fitted
-    to 64 .. 512 rows of eight shapes from 1024 x 4096 to 20480 x 6656: row groups of 64 rows x 16 channels while at most
-    512 workgroups of those run (two per CU), else of 64 rows x 32 channels by rounds of 512 (a round begun costs 0.4 of
-    one whatever it holds); the prompt kernel by its workgroups of 64 x 128, one or two per CU, and beyond 256 of
-    128 x 128, two per CU, by rounds of 512 of those, the last one rarely full.  They hand over at 256 rows (20480 x 6656:
-    154 us in row groups, 144 on the prompt kernel, and 78 against 118 at 128 rows) to 512 rows (4096 x 4096: 44 and 42)."""
+    the prompt kernel (2 bytes per weight)?  The same bits either way.  Both in us, the row quantizer included: row groups
+    of 64 rows x 16 channels while at most 512 workgroups of those run (two per CU), else of 64 rows x 32 channels by
+    rounds of 512, a round begun at 0.45 of one whatever it holds; the prompt kernel by its workgroups of 64 x 128, one or
+    two per CU, and beyond 256 of 128 x 128, two per CU, by rounds of 512 of those, half of one for up to 256.  Fitted to
+    720 calls of 64 .. 2048 rows, 1024 .. 20480 channels and K = 1024 .. 18944: the choice costs 0.3 % on average, over
+    10 % at five of them (4672 x 1536 at 292 rows, 18.9 us in row groups, 23.5 on the prompt kernel).  They hand over at 256 rows
+    (20480 x 6656: 138 us in row groups, 143 on the prompt kernel, and 80 against 122 at 128 rows), 512 rows (4096 x 4096: 41
+    and 42) or 1300 (5056 x 1280 at 1957: 80 and 60)."""
     rows64 = (M + 63) // 64
     wgs = rows64 * (N // 16)
     if wgs <= 512:
         groups = 5.5 + 0.0021 * K if wgs <= 256 else 6.5 + 0.0027 * K
     else:
         rounds, rest = divmod(rows64 * ((N + 31) // 32), 512)
-        part = 0.0 if not rest else 0.4 + 0.6 * rest / 512 if rounds else 0.75 + 0.25 * rest / 512
-        groups = 6.0 + 0.0044 * K * (rounds + part)
+        part = 0.0 if not rest else 0.45 + 0.55 * rest / 512 if rounds else 0.75 + 0.25 * rest / 512
+        groups = 6.5 + (2.0 + 0.0038 * K) * (rounds + part)
     wgs = (M + 127) // 128 * ((N + 127) // 128)
     if wgs <= 256:
-        prompt = (5.0 + 0.0072 * K + N * K / 4.5e6) * (1.0 if wgs <= 128 else 1.45)
+        prompt = (5.5 + 0.0072 * K + N * K / 3.3e6) * (1.0 if wgs <= 128 else 1.5)
     else:
-        prompt = (1.0 if wgs <= 512 else 0.8 * ((wgs + 511) // 512)) * (12.0 + 0.0205 * K)
+        rounds, rest = divmod(wgs, 512)
+        prompt = (12.5 + 0.0202 * K) * (rounds + (0.0 if not rest else 0.5 if rest <= 256 else 0.9 + 0.1 * rest / 512))
     return groups < prompt
 
 

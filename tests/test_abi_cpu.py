@@ -371,7 +371,7 @@ def test_kernel_family_of_short_prompts():
 
 
 def test_group_is_one_launch():
-    """Which groups the large-M launches take, by sizes alone: rows, blocks of whole tiles, operands below 4 GiB."""
+    """Which groups run as one launch, by sizes alone: rows, blocks of whole tiles, operands below 4 GiB."""
     import ctypes
     from tpp_pytorch_extension import _lib
     L = _lib.lib()
@@ -381,13 +381,16 @@ def test_group_is_one_launch():
 
     for bytes_per in (1, 2):
         assert one([11008] * 2, 333, 4096, bytes_per) == 1 and one([11008] * 2, 2048, 4096, bytes_per) == 1
-        assert one([11008] * 2, 64, 4096, bytes_per) == 0   # the decode kernels' rows
+        assert one([11008] * 2, 64, 4096, bytes_per) == bytes_per - 1  # the decode kernels' rows: bf16 weights in one launch
         assert one([11000] * 2, 333, 4096, bytes_per) == 0  # no whole tiles
         assert one([11008] * 2, 0, 4096, bytes_per) == 0 and one([], 333, 4096, bytes_per) == 0
         assert one([1 << 20] * 2, 333, 4096 // bytes_per, bytes_per) == 0  # weights of 4 GiB
     assert one([5120] * 2, 64, 2048, 1) == 0 and one([5120] * 2, 66, 2048, 1) == 1  # per weight, then one launch (14 us, per weight 26)
     assert one([11008] * 2, 333, 4096, 3) == 0
     assert one([4096, 1024, 1024], 2048, 4096, 2) == 1 and one([4096, 1024, 1024], 2048, 4096, 1) == 0  # bf16 only
+    for M in (1, 17, 64):
+        assert one([4096, 1024, 1024], M, 4096, 2) == 1 and one([1 << 20] * 2, M, 2048, 2) == 1  # (weights of 4 GiB too)
+        assert one([4096, 1024], M, 4032, 2) == 0  # K in no whole tiles
 
 
 def test_environment_switches_are_read_once(monkeypatch):

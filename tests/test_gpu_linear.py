@@ -1212,7 +1212,7 @@ def test_groups_that_run_per_weight_are_asked_about_first(fmt, M, N, K, monkeypa
         assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws, [None] * 2), qkv))
 
 
-@pytest.mark.parametrize("M", [65, 128, 129, 300])
+@pytest.mark.parametrize("M", [1, 17, 64, 65, 128, 129, 300])
 @pytest.mark.parametrize("N,K", [(64, 2048), (1536, 1024), (5120, 2048)])
 def test_group_is_one_launch_answers_as_the_calls_do(M, N, K):
     """tppx_group_is_one_launch against what tppx_swiglu_bf16 and tppx_swiglu_qint8 do with the same shape."""

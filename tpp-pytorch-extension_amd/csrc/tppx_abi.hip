@@ -875,6 +875,7 @@ extern "C" int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M
       (weight_bytes == 1 ? n_segs != 2 || Ns[0] != Ns[1] : weight_bytes != 2))
     return 0;
   int64_t tiles[TPPX_MAX_SEGS];
+  bool large = true; // the large-M kernel takes them together
   for (int i = 0; i < n_segs; i++) {
     if (Ns[i] <= 0 || Ns[i] % 16 != 0 || Ns[i] > (1 << 25))
       return 0;
@@ -884,11 +885,14 @@ extern "C" int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M
     t.K = (int)K;
     t.tiles = (int)(Ns[i] / 16);
     t.qbs = 256;
-    if (!(weight_bytes == 1 ? tiled_qint8_takes_groups(t) : tiled_bf16_takes_groups(t)))
+    if (weight_bytes == 2 && (K % 128 != 0 || M * Ns[i] >= ((int64_t)1 << 31)))
       return 0;
+    large = large && (weight_bytes == 1 ? tiled_qint8_takes_groups(t) : tiled_bf16_takes_groups(t));
     tiles[i] = t.tiles;
   }
-  return weight_bytes == 1 ? want_tiled_qint8(M, K, 0, 2 * tiles[0], true, 256) : want_tiled_bf16(M, K, 0, tiles, n_segs);
+  if (weight_bytes == 1)
+    return large && want_tiled_qint8(M, K, 0, 2 * tiles[0], true, 256);
+  return want_tiled_bf16(M, K, 0, tiles, n_segs) ? large : M <= 64; // (up to 64 rows the decode kernel takes any group)
 }
 
 extern "C" int tppx_multi_linear_bf16(const void* x, const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int flags,

@@ -470,6 +470,7 @@ def _bf16_group(input, weights, biases, pair=False):
     if any(k != K for _, k in geo) or (pair and geo[0] != geo[1]):
         return None
     L = _lib.lib()
+    # (up to 64 rows the answer is yes: not asked, a call less in an eager step)
     if M > 64 and not L.tppx_group_is_one_launch((ctypes.c_int64 * n)(*(N for N, _ in geo)), n, M, K, 2):
         return None
     x = input.contiguous()

@@ -1098,6 +1098,56 @@ def test_prompt_gemms_with_k_in_slices(fmt, S, M, N, K, monkeypatch):
         assert torch.equal(y, got[0])
 
 
+@pytest.mark.parametrize("fmt", ["mxfp4", "qint8", "bf16"])
+def test_captured_prompt_gemms_keep_their_slices_in_the_graphs_own_memory(fmt, monkeypatch):
+    """K slices of a captured prompt leave their sums in a buffer of the graph's own, so that replays of two graphs on two
+    streams need no order; decode steps use the device's capture buffer.  Every replay has the eager call's bits."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    K, N = 6144, 256
+    ws = [block_bf16(randn_bf16((N, K), 0.05, 1850 + i)).cuda() for i in range(2)]
+    if fmt != "bf16":
+        ws = [{"mxfp4": ops.remap_and_quantize_mxfp4, "qint8": ops.remap_and_quantize_qint8}[fmt](w) for w in ws]
+    lib, seen = _lib.lib(), []
+
+    class Watch:
+        def __getattr__(self, name):
+            f = getattr(lib, name)
+            if "linear" not in name:
+                return f
+
+            def call(*args):  # (every one of them ends in ws, ws_bytes, stream)
+                seen.append((args[-3], args[-2]))
+                return f(*args)
+            return call
+
+    for M, prompt in ((200, True), (64, False)):
+        x = randn_bf16((M, K), 1.0, 1860).cuda()
+
+        def run():
+            return [ops.linear(x, ws[0], None)] + list(ops.qkv_gemm(x, ws, [None, None]))
+
+        want = run()
+        _lib.workspace(x)
+        shared = _lib._workspaces[(x.device.index, "capture")]
+        g, seen[:] = torch.cuda.CUDAGraph(), []
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "lib", lambda: Watch())
+            with torch.cuda.graph(g):
+                got = run()
+        assert seen
+        if prompt:
+            assert all(at != shared.data_ptr() and n == _lib.WORKSPACE_BYTES for at, n in seen)
+        elif fmt != "bf16":
+            assert all(at == shared.data_ptr() for at, n in seen)
+        for _ in range(3):
+            for y in got:
+                y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("S,M,N,K", [(2, 65, 160, 512), (2, 200, 288, 1792), (3, 129, 2080, 1792), (4, 100, 32, 2304), (6, 333, 416, 3328)])
 def test_prompt_qint8_gemms_with_k_in_slices(S, M, N, K, monkeypatch):
     """QINT8 the same: K in S slices of whole scale blocks (one block a slice, an odd and an even number), against the oracle

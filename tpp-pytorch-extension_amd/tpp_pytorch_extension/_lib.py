@@ -172,15 +172,18 @@ _workspace_use = {}  # (device, stream) -> tick of its last use
 _tick = 0
 
 
-def workspace(t, stream=None):
-    """Split-K / staging scratch for an op on `t`'s device (see include/tppx.h); stream: stream_of(t), where it is known.
+def workspace(t, stream=None, rows=0):
+    """Split-K / staging scratch for an op on `t`'s device (see include/tppx.h); stream: stream_of(t), where it is known;
+    rows: those of a GEMM.
     One zero-initialised buffer per (device, stream): every op orders itself on
     the caller's current stream, so threads that work on streams of their own
     never share scratch and need no ordering between them. Work recorded under
     stream capture uses one more buffer per device, created together with the
     device's first eager one (a capture cannot allocate it): run the op once
     eagerly before capturing, and order replays of different graphs that use
-    these ops with respect to each other.  A device keeps at most
+    these ops with respect to each other.  Prompt GEMMs (more than 64 rows, which
+    may leave sums of K slices there) get one from the capture's own pool
+    instead: their replays need no such order.  A device keeps at most
     MAX_STREAM_WORKSPACES per-stream buffers: beyond that the least recently
     used one goes back to torch's allocator (it was allocated on its own stream,
     so work still queued there keeps it valid).  with_counters(): arrival
@@ -192,7 +195,7 @@ def workspace(t, stream=None):
         if ws is None:
             raise TppxError(EINVAL, "first call on this device happens inside graph capture: run the op once "
                                     "eagerly before capturing so that its workspace exists")
-        return ws
+        return ws if rows <= 64 else torch.empty(WORKSPACE_BYTES, dtype=torch.uint8, device=t.device)
     key = (dev, stream_of(t) if stream is None else stream)
     ws = _workspaces.get(key)
     if ws is None:

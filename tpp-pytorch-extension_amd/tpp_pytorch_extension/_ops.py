@@ -446,8 +446,8 @@ def _linear_bf16(input, weight, bias, post, post_in, post_in2, post_scale, flags
 
 
 def _bf16_ws(x, M, st):
-    """Workspace for the K slices of prompt launches, None for decode steps.  A capture gets one from its own pool: replays
-    of different graphs need no order between them."""
+    """Workspace for the K slices of prompt launches, None for decode steps.  (A capture's own, as _lib.workspace() gives to
+    prompts; here without an eager call before it, which bf16 weights never asked for.)"""
     if M <= 64:
         return None
     if torch.cuda.is_current_stream_capturing():
@@ -543,7 +543,7 @@ def _mxfp4_flags_ws(x, M, K, flags=0, ws=None):
     """(flags, workspace) of an MXFP4 call: the FP8-activation path keeps the quantised activations in the workspace."""
     if ACT_FP8 and M > 64:
         flags |= _lib.FLAG_ACT_FP8
-    ws = _lib.workspace(x) if ws is None else ws
+    ws = _lib.workspace(x, rows=M) if ws is None else ws
     if flags & _lib.FLAG_ACT_FP8:
         Mp = (M + 63) // 64 * 64
         need = Mp * K + Mp * (K // 32)
@@ -657,7 +657,7 @@ def _linear_other_types(input, weight, bias, post, flags, post_in=None, post_in2
             b = _prep_bias(bias, N, dev)
             p1 = _prep_post(post_in, M, N, "post-op input", dev) if post in (POST_MUL, POST_ADD_SCALE, POST_ADD2_SCALE) else None
             p2 = _prep_post(post_in2, M, N, "second post-op input", dev) if post == POST_ADD2_SCALE else None
-            ws = _lib.workspace(xq)
+            ws = _lib.workspace(xq, st, M)
             _lib.check(L.tppx_linear_qint8(None, xq.data_ptr(), sa.data_ptr(), qn.data_ptr(), sn.data_ptr(), _lib.ptr(b),
                                            _lib.ptr(p1), _lib.ptr(p2), y.data_ptr(), M, N, K, qbs, post, float(post_scale),
                                            flags, ws.data_ptr(), ws.numel(), st))
@@ -845,7 +845,7 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
             return y
     qn, sn = weight.native()
     st = _lib.stream_of(x)
-    ws = _lib.workspace(x, st)
+    ws = _lib.workspace(x, st, M)
     if row_sumsq is not None:
         if not takes_row_sums(weight, M):
             raise TppxError(_lib.EUNSUPPORTED, "row sums of squares need an MXFP4 weight and at most 16 rows")
@@ -1120,7 +1120,7 @@ def qkv_gemm(input, weights, biases, norm=None):
     if M == 0:
         return outs
     st = _lib.stream_of(x)
-    ws = _lib.workspace(x, st)
+    ws = _lib.workspace(x, st, M)
     if scheme == QSCHEME_MXFP and norm is not None and _norm_table(norm) is not None:
         _lib.check(L.tppx_normsq_multi_linear_mxfp4(x.data_ptr(), _norm_table(norm).data_ptr(), norm[0].data_ptr(),
                                                     float(norm[1]), segs, n, M, K, 0, st))
@@ -1201,7 +1201,7 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
                                             M, N, K, 0, _lib.stream_of(x)))
         return y
     st = _lib.stream_of(x)
-    fl, ws = _mxfp4_flags_ws(x, M, K, 0, _lib.workspace(x, st))
+    fl, ws = _mxfp4_flags_ws(x, M, K, 0, _lib.workspace(x, st, M))
     if not fl and M > 64 and M * N * 2 > ws.numel():
         # prefill: room for the gate tile lets the library run gate and up as one grid (fuller last round)
         ws = torch.empty(M * N * 2, dtype=torch.uint8, device=x.device)

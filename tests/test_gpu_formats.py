@@ -743,6 +743,19 @@ def test_float_and_half_rows_on_qint8_tile_edges(M, N, K, qbs, dtype):
     assert off.data_ptr() % 16 and torch.equal(ops.fc_plain(off, qw, bias.cuda()).cpu(), ref)
 
 
+def test_half_rows_beyond_65535_blocks_of_32():
+    """More rows of a narrow weight than a launch with 32 rows to a workgroup has blocks for (up to 65535 blocks of 64 are
+    accepted): the bits of the same rows in a call of their own."""
+    ops = _ops()
+    w = ops.remap_and_quantize_qint8(block_bf16(randn_bf16((32, 64), 0.5, 185)).cuda())
+    M = 65535 * 32 + 7
+    x = torch.randn((M, 64), generator=torch.Generator(device="cuda").manual_seed(186), device="cuda").half()
+    y = ops.fc_plain(x, w, None)
+    for rows in (slice(0, 70), slice(M - 70, M)):
+        assert torch.equal(y[rows], ops.fc_plain(x[rows].contiguous(), w, None))
+    assert y.isfinite().all()
+
+
 def test_float_rows_quantizer_on_nan_and_inf():
     """A NaN in a block's first place sticks in its scale, any other is passed over, as in quantize_int8sym."""
     from tpp_pytorch_extension import _lib

@@ -708,7 +708,7 @@ static int run_linear_qint8(const char* who, const void* xq, const void* sa, con
     launch(one{}, one{});
   else if (M <= 32 || rows32 * tiles <= 256)
     launch(two{}, one{});
-  else if (5.0 + 0.0027 * K * small < 15.0 + 0.0073 * K * large)
+  else if (rows32 <= 65535 && 5.0 + 0.0027 * K * small < 15.0 + 0.0073 * K * large) // (the grid: rows come in twice as many blocks)
     launch(two{}, two{});
   else {
     const dim3 grid((unsigned)((tiles + 7) / 8), (unsigned)((M + 63) / 64));

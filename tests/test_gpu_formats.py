@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import oracle as O
-from util import t2bits, randn_bf16, block_bf16, assert_close_bf16
+from util import t2bits, randn_bf16, block_bf16, assert_close_bf16, qint8_scratch
 
 pytestmark = pytest.mark.gpu
 
@@ -341,7 +341,7 @@ def test_packed_code_kernel_block_rows(kind, M):
     x = randn_bf16((M, K), 1.0, 2810 + M).cuda()
     r = randn_bf16((M, N), 1.0, 2830).cuda()
     packed, sn, bits = qt.native_packed()
-    xq, sa = ops._qint8_scratch(x, M, K, 256)
+    xq, sa = qint8_scratch(x, M, K, 256)
     y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
     _lib.check(_lib.lib().tppx_linear_qintx(x.data_ptr(), xq.data_ptr(), sa.data_ptr(), packed.data_ptr(), sn.data_ptr(), None,
                                             r.data_ptr(), None, y.data_ptr(), M, N, K, bits, O.POST_ADD_SCALE, 1.0, 0,
@@ -486,7 +486,7 @@ def test_packed_code_decode_kernel_equals_expanded_weight(kind, M, N, K, post, m
     assert packed.numel() == N * K * bits // 8
     # the packed path really ran: the entry point accepts the call (no fall-through) and gives the op's bits
     y2 = torch.empty_like(y)
-    xq, sa = ops._qint8_scratch(x, M, K, 256)
+    xq, sa = qint8_scratch(x, M, K, 256)
     _lib.check(_lib.lib().tppx_linear_qintx(x.data_ptr(), xq.data_ptr(), sa.data_ptr(), packed.data_ptr(), sn.data_ptr(),
                                             b.data_ptr(), r.data_ptr(), None, y2.data_ptr(), M, N, K, bits, posts[post], 0.5,
                                             0, _lib.stream_of(x)))
@@ -743,6 +743,37 @@ def test_float_and_half_rows_on_qint8_tile_edges(M, N, K, qbs, dtype):
     assert off.data_ptr() % 16 and torch.equal(ops.fc_plain(off, qw, bias.cuda()).cpu(), ref)
 
 
+@pytest.mark.parametrize("post", [O.POST_NONE, O.POST_SILU, O.POST_ADD2_SCALE])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("M", [3, 40])
+def test_float_linears_in_steps(M, dtype, post):
+    """The GEMMs with fp32 output (tppx_linear_wide, tppx_linear_qint8_f32) followed by tppx_post_op_wide: the bits of the
+    calls that do both in one launch."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    L, N, K = _lib.lib(), 160, 512
+    dt, st = {torch.float32: _lib.DT_F32, torch.float16: _lib.DT_F16}[dtype], torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(191)
+    x, in1, in2 = (torch.randn(s, generator=g).to(dtype).cuda() for s in ((M, K), (M, N), (M, N)))
+    b = torch.randn((N,), generator=g).cuda()
+    W = block_bf16(randn_bf16((N, K), 0.05, 192)).cuda()
+    acc, y = torch.empty((M, N), device="cuda"), torch.empty((M, N), dtype=dtype, device="cuda")
+    for w in (ops.remap_and_quantize_mxfp4(W), W, ops.remap_and_quantize_qint8(W)):
+        if w is W:
+            _lib.check(L.tppx_linear_wide(x.data_ptr(), dt, ops._bf16_native(W).data_ptr(), None, _lib.W_BF16, b.data_ptr(), acc.data_ptr(),
+                                          M, N, K, st))
+        elif w.weight_kind() == "mxfp4":
+            qn, sn = w.native()
+            _lib.check(L.tppx_linear_wide(x.data_ptr(), dt, qn.data_ptr(), sn.data_ptr(), _lib.W_MXFP4, b.data_ptr(), acc.data_ptr(), M, N, K,
+                                          st))
+        else:
+            (qn, sn), q = w.native(), ops.quantize_int8sym(x.float(), w.block_size, -1, False)
+            _lib.check(L.tppx_linear_qint8_f32(q.qdata.data_ptr(), q.scales.data_ptr(), qn.data_ptr(), sn.data_ptr(), b.data_ptr(),
+                                               acc.data_ptr(), M, N, K, w.block_size, st))
+        _lib.check(L.tppx_post_op_wide(acc.data_ptr(), dt, post, in1.data_ptr(), in2.data_ptr(), 0.5, y.data_ptr(), M * N, st))
+        assert torch.equal(y, ops.linear(x, w, b, post, in1, in2, 0.5))
+
+
 def test_half_rows_beyond_65535_blocks_of_32():
     """More rows of a narrow weight than a launch with 32 rows to a workgroup has blocks for (up to 65535 blocks of 64 are
     accepted): the bits of the same rows in a call of their own."""
@@ -854,12 +885,34 @@ def _qint(kind, W):
 # more rows of such blocks is one launch of another kernel)
 @pytest.mark.parametrize("fmt,M,N,K", [("qint8", 16, 272, 1024), ("qint8", 17, 272, 1024), ("qint8", 33, 4096, 11008), ("qint8", 64, 1040, 2560),
                                        ("qint8", 96, 272, 640), ("qint4", 9, 272, 1024), ("qint4", 40, 1040, 2560), ("qint2", 64, 288, 1024)])
-def test_int8_gate_up_quantizes_its_rows_once(fmt, M, N, K):
+def test_int8_gate_up_quantizes_its_rows_once(fmt, M, N, K, monkeypatch):
     """The gate/up pair of QINT8-family weights where it runs as two launches behind ONE quantization of the rows: equal to
-    the two calls that quantize them each."""
+    the two calls that quantize them each.  The second call says that the rows are there (up to 16 rows the GEMM quantizes
+    them itself)."""
+    from tpp_pytorch_extension import _lib
     ops = _ops()
     W = [_qint(fmt, randn_bf16((N, K), 0.05, 3500 + i)) for i in range(2)]
     assert M <= 64 or W[0].block_size != 256
     x, b = randn_bf16((M, K), 1.0, 3510 + M).cuda(), randn_bf16((N,), 0.1, 3520).cuda()
     want = ops.fc_mul(x, W[1], None, ops.fc_silu(x, W[0], b))
-    assert torch.equal(ops.swiglu_gate_up(x, W[0], W[1], b, None), want)
+    lib, calls = _lib.lib(), []
+
+    class Watch:
+        def __getattr__(self, name):
+            f = getattr(lib, name)
+            if name not in ("tppx_linear_qint8", "tppx_linear_qintx"):
+                return f
+
+            def call(*args):  # (x, xq, sa, ..., flags[, ws, ws_bytes], stream)
+                rc = f(*args)
+                if rc == _lib.OK:
+                    calls.append((args[1], args[2], args[-4 if name == "tppx_linear_qint8" else -2]))
+                return rc
+            return call
+
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "lib", lambda: Watch())
+        got = ops.swiglu_gate_up(x, W[0], W[1], b, None)
+    assert torch.equal(got, want) and len(calls) == 2
+    if M > 16:
+        assert calls[0][:2] == calls[1][:2] and [c[2] & _lib.FLAG_XQ_REUSE for c in calls] == [0, _lib.FLAG_XQ_REUSE]

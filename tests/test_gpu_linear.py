@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import oracle as O
-from util import t2bits, randn_bf16, block_bf16, assert_close_bf16, err_stats
+from util import t2bits, randn_bf16, block_bf16, assert_close_bf16, err_stats, qint8_scratch
 
 pytestmark = pytest.mark.gpu
 
@@ -1049,6 +1049,31 @@ def test_prefill_bf16_every_workgroup_tile_ragged(tile, w8, M, N, K, monkeypatch
     assert all(torch.equal(a, b) for a, b in zip(ops.qkv_gemm(x, ws[:4], bs), got[2:]))
 
 
+@pytest.mark.parametrize("M", [5, 200])
+def test_bf16_entry_points_without_a_workspace(M):
+    """tppx_linear_bf16, tppx_multi_linear_bf16 and tppx_swiglu_bf16: the bits of the forms with a workspace, given none."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    L, N, K = _lib.lib(), 4096, 3072
+    nat = [ops._bf16_native(block_bf16(randn_bf16((N, K), 0.05, 1870 + i)).cuda()) for i in range(2)]
+    x, st = randn_bf16((M, K), 1.0, 1872).cuda(), torch.cuda.current_stream().cuda_stream
+
+    def run(ws):
+        y = [torch.empty((M, N), dtype=torch.bfloat16, device="cuda") for _ in range(4)]
+        segs = (_lib.Seg * 2)()
+        for s, w, o in zip(segs, nat, y[1:]):
+            s.qw = s.sw = w.data_ptr()
+            s.y, s.N, s.post_op, s.post_scale = o.data_ptr(), N, O.POST_NONE, 1.0
+        end = (None, 0, st) if ws else (st,)
+        f = [getattr(L, f"tppx_{name}_bf16{'_ws' if ws else ''}") for name in ("linear", "multi_linear", "swiglu")]
+        _lib.check(f[0](x.data_ptr(), nat[0].data_ptr(), None, None, None, y[0].data_ptr(), M, N, K, O.POST_SILU, 1.0, 0, *end))
+        _lib.check(f[1](x.data_ptr(), segs, 2, M, K, 0, *end))
+        _lib.check(f[2](x.data_ptr(), nat[0].data_ptr(), None, nat[1].data_ptr(), None, y[3].data_ptr(), M, N, K, 0, *end))
+        return y
+
+    assert all(torch.equal(a, b) for a, b in zip(run(False), run(True)))
+
+
 # ragged rows and channel blocks, slices of unequal and of the fewest steps (four), each number of slices
 @pytest.mark.parametrize("fmt", ["mxfp4", "bf16"])
 @pytest.mark.parametrize("S,M,N,K", [(2, 65, 160, 1152), (3, 200, 288, 1792), (4, 129, 2080, 2048), (6, 100, 32, 3072), (6, 333, 416, 4224)])
@@ -1056,6 +1081,7 @@ def test_prompt_gemms_with_k_in_slices(fmt, S, M, N, K, monkeypatch):
     """K in S slices whose fp32 sums a second launch adds, in slice order: linear with its residual and bias, a post-op that
     goes through the general epilogue, and q/k/v with a fourth GELU GEMM, against the launch with K whole (another order of
     the fp32 sums: one bf16 ulp here and there) and a float64 product; every replay of a captured call the same."""
+    from tpp_pytorch_extension import _lib
     ops = _ops()
     flat = [randn_bf16((n, K), 0.05, 1800 + i) for i, n in enumerate((N, 64, 96, 160))]
     ws = [block_bf16(w).cuda() for w in flat]
@@ -1066,10 +1092,19 @@ def test_prompt_gemms_with_k_in_slices(fmt, S, M, N, K, monkeypatch):
     def run():
         return [ops.fc_add(x, ws[0], b, res, 0.5), ops.fc_add2(x, ws[0], b, res, res, 0.5)] + list(ops.qkv_gemm(x, ws, [b, None, None, None]))
 
+    def left_sums():  # the slices' sums are what these launches write to the workspace
+        return bool(_lib.workspace(x).any())
+
     monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
     monkeypatch.setenv("TPPX_TILED_SPLIT", "0")
+    _lib.workspace(x).zero_()
     want = run()
+    assert not left_sums()
     monkeypatch.setenv("TPPX_TILED_SPLIT", str(S))
+    for call in (lambda: ops.fc_add(x, ws[0], b, res, 0.5), lambda: ops.qkv_gemm(x, ws, [b, None, None, None])):
+        _lib.workspace(x).zero_()
+        call()
+        assert left_sums()
     got = run()
     for i, (a, w) in enumerate(zip(got, want)):
         a, w = a.double(), w.double()
@@ -1080,7 +1115,6 @@ def test_prompt_gemms_with_k_in_slices(fmt, S, M, N, K, monkeypatch):
         assert ((a - w).abs() <= 3 * 2.0 ** -7 * near + 2.0 ** -12 * w.abs().max()).all(), i
     if fmt == "mxfp4":
         import ctypes
-        from tpp_pytorch_extension import _lib
         buf = ctypes.create_string_buffer(4096)
         _lib.check(_lib.lib().tppx_plan_linear_mxfp4(M, N, K, 0, 1 << 25, buf, len(buf)))
         assert f"side_split_kernel<false> grid={(M + 63) // 64 * ((N + 127) // 128)}x{S}x1" in buf.value.decode()
@@ -1229,7 +1263,7 @@ def test_prefill_qint8_pair_agrees_with_two_launches(fmt, M, N, K, monkeypatch):
     b = randn_bf16((N,), 0.5, 762).cuda()
     x = randn_bf16((M, K), 1.0, 763).cuda()
     with monkeypatch.context() as m:
-        m.setattr(ops, "fc_silu", None)  # (the two launches would call it)
+        m.setattr(ops, "linear", None)  # (the two launches would call it)
         got = ops.swiglu_gate_up(x, ws[0], ws[1], b, None)
     assert torch.equal(got, ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], b)))
 
@@ -1253,7 +1287,7 @@ def test_groups_that_run_per_weight_are_asked_about_first(fmt, M, N, K, monkeypa
 
     class Without:
         def __getattr__(self, name):
-            assert name not in ("tppx_swiglu_qint8", "tppx_swiglu_bf16", "tppx_multi_linear_bf16"), name
+            assert not name.startswith(("tppx_swiglu_qint8", "tppx_swiglu_bf16", "tppx_multi_linear_bf16")), name
             return getattr(lib, name)
 
     monkeypatch.setattr(_lib, "lib", lambda: Without())
@@ -1274,7 +1308,7 @@ def test_group_is_one_launch_answers_as_the_calls_do(M, N, K):
     nat, (q, s) = ops._bf16_native(w), ops.remap_and_quantize_qint8(w).native()
     x = randn_bf16((M, K), 1.0, 779).cuda()
     y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
-    xq, sa = ops._qint8_scratch(x, M, K, 256)
+    xq, sa = qint8_scratch(x, M, K, 256)
     st, ns = _lib.stream_of(x), (ctypes.c_int64 * 2)(N, N)
     rc = L.tppx_swiglu_bf16(x.data_ptr(), nat.data_ptr(), None, nat.data_ptr(), None, y.data_ptr(), M, N, K, 0, st)
     assert rc in (_lib.OK, _lib.EUNSUPPORTED) and (rc == _lib.OK) == bool(L.tppx_group_is_one_launch(ns, 2, M, K, 2))

@@ -29,6 +29,13 @@ def block_bf16(W, bk=16, bc=64):
     return W.view(N // bk, bk, K // bc, bc // 2, 2).permute(0, 2, 3, 1, 4).contiguous()
 
 
+def qint8_scratch(x, M, K, qbs):
+    """Buffers for the int8 rows of a QINT8 call and their scales, with the room of whole operand tiles of 64 rows."""
+    rows = (M + 63) // 64 * 64
+    return (torch.empty((rows, K), dtype=torch.int8, device=x.device),
+            torch.empty((rows, K // qbs), dtype=torch.float32, device=x.device))
+
+
 def err_stats(got_bits, ref_bits):
     g = bits2f(got_bits).astype(np.float64)
     r = bits2f(ref_bits).astype(np.float64)

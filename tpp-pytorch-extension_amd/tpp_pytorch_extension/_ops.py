@@ -527,13 +527,6 @@ def _qint8_buffer(x, M, K, qbs):
     return buf, buf.data_ptr(), buf.data_ptr() + rows * K
 
 
-def _qint8_scratch(x, M, K, qbs):
-    """The same as two tensors."""
-    buf = _qint8_buffer(x, M, K, qbs)[0]
-    rows = (M + 63) // 64 * 64
-    return buf[:rows * K], buf[rows * K:]
-
-
 # Opt-in (TPPX_ACT_FP8=1, or flags=FLAG_ACT_FP8 on linear()): MXFP4 GEMMs with more than 64 rows quantize their
 # activations to MXFP8 and run on the block-scaled MFMA.  Not the reference's arithmetic (its activations stay bf16).
 ACT_FP8 = os.environ.get("TPPX_ACT_FP8", "0") == "1"

@@ -207,6 +207,8 @@ int tppx_quant_act_int8(const void* x, int64_t M, int64_t K, int64_t qbs,
  * scratch, 256-byte aligned, that lets decode-shape launches with more than 16
  * rows split K across workgroups (fp32 partial tiles, summed inside the same
  * launch by whichever workgroup of a tile finishes last, in a fixed order).
+ * Prompt launches (more than 64 rows) of few workgroups and a long K leave the
+ * sums of 2 to 6 K slices there, added by a second launch in slice order.
  * It needs no initialisation and carries no state between calls.
  * Launches that share a workspace must be ordered on one stream.  With
  * ws == NULL (or too small) the kernels simply do not split K.  32 MiB covers
@@ -251,8 +253,8 @@ int tppx_quant_act_mxfp8(const void* x, int64_t M, int64_t K, void* xq, void* xs
  * bc=K, vnni=1 = a plain [N][K] matrix) -> native bf16 tiles
  * [N/16][K/128][4][64][8] (N*K*2 bytes).  N%16==0, K%128==0.
  * tppx_linear_bf16: y = post( bf16( bias[n] + sum_k x[m][k]*W[n][k] ) ) with
- * the row-group kernel at any M (beyond 64 rows every block of 64 rows
- * streams the weights again: meant for lm_head-sized M, not for prefill). */
+ * the row-group kernel up to 64 rows, beyond with that (every block of 64 rows
+ * streams the weights again) or the large-M kernel, whichever is faster. */
 int tppx_prepack_bf16(const void* w_ref, int64_t N, int64_t K, int64_t bk,
                       int64_t bc, int vnni, void* w_nat, tppx_stream_t stream);
 int tppx_linear_bf16(const void* x, const void* w_nat, const void* bias,
@@ -417,9 +419,9 @@ int tppx_swiglu_bf16(const void* x, const void* w_gate, const void* bias_gate,
                      const void* w_up, const void* bias_up, void* y, int64_t M,
                      int64_t N, int64_t K, int flags, tppx_stream_t stream);
 
-/* The same three with a workspace (16-byte aligned; without one K stays whole):
- * launches of few workgroups and a long K run K in slices whose fp32 sums are
- * added by a second launch. */
+/* The same three with a workspace (256-byte aligned; NULL: K stays whole): from
+ * 65 rows on launches of few workgroups and a long K run K in slices whose fp32
+ * sums are added by a second launch. */
 int tppx_linear_bf16_ws(const void* x, const void* w, const void* bias,
                         const void* post_in, const void* post_in2, void* y,
                         int64_t M, int64_t N, int64_t K, int post_op,
@@ -435,7 +437,8 @@ int tppx_swiglu_bf16_ws(const void* x, const void* w_gate, const void* bias_gate
 
 /* The gate/up pair of QINT8-family weights as one launch behind the activation
  * quantizer (xq / sa as in tppx_linear_qint8), the same bits as fc_silu
- * followed by fc_mul.  TPPX_EUNSUPPORTED (before any launch) where one
+ * followed by fc_mul with K whole (with a workspace those two may run a K of
+ * 6144 and more in slices, another order of the fp32 sums).  TPPX_EUNSUPPORTED (before any launch) where one
  * tppx_linear_qint8 per weight is the way: few rows, block sizes other than
  * 256, operands of 4 GiB and more. */
 int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* qw_gate,

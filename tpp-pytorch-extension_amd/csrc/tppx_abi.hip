@@ -433,7 +433,7 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
   }
   if (want_tiled_mxfp4(M, K, flags, p.total_tiles, dual, !dual && n_segs == 1 && !row_sumsq, ws_bytes)) {
     TPPX_REQUIRE(!row_sumsq, TPPX_EUNSUPPORTED, "%s: row sums of squares are not produced by the large-M kernels", who);
-    float* part = aligned16(ws) ? (float*)ws : nullptr;
+    float* part = (float*)ws;
     // prefill shapes: one LDS-tiled launch per GEMM of the group; the fused
     // gate/up pair becomes silu(gate) followed by up * gate (same rounding)
     if (!dual && n_segs > 1) {
@@ -578,7 +578,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
   p.units = (int)(K / (64 * p.deal));
   p.spb_magic = (p.deal == 4 && p.tpb > 4) ? (unsigned int)((((uint64_t)1 << 32) + (uint64_t)(p.tpb / 4) - 1) / (uint64_t)(p.tpb / 4)) : 0u;
   const bool reuse = (flags & TPPX_FLAG_XQ_REUSE) != 0; // xq / sa still hold this x, quantized by an earlier call
-  const bool tiled = qbs % 128 == 0 && want_tiled_qint8(M, K, flags, (dual ? 2 : 1) * (int64_t)p.total_tiles, dual, qbs, n_segs == 1 && aligned16(ws) ? ws_bytes : 0);
+  const bool tiled = qbs % 128 == 0 && want_tiled_qint8(M, K, flags, (dual ? 2 : 1) * (int64_t)p.total_tiles, dual, qbs, n_segs == 1 ? ws_bytes : 0);
   TiledParams t[TPPX_MAX_SEGS];
   bool group = tiled && n_segs > 1; // one grid over the channel blocks of all GEMMs when the large-M kernel takes them
   for (int i = 0; i < n_segs && tiled; i++) {
@@ -594,9 +594,9 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
         return rc;
     }
     if (group)
-      return check_hip(launch_tiled_qint8_group(t, n_segs, stream, dual, aligned16(ws) ? (float*)ws : nullptr, ws_bytes), who);
+      return check_hip(launch_tiled_qint8_group(t, n_segs, stream, dual, (float*)ws, ws_bytes), who);
     for (int i = 0; i < n_segs; i++) {
-      rc = check_hip(launch_tiled_qint8(t[i], stream, aligned16(ws) ? (float*)ws : nullptr, ws_bytes), who);
+      rc = check_hip(launch_tiled_qint8(t[i], stream, (float*)ws, ws_bytes), who);
       if (rc)
         return rc;
     }
@@ -813,9 +813,9 @@ static int run_linear_bf16(const char* who, const void* x, const void* w, const 
   p.K = (int)K;
   // more than 64 rows: the LDS-tiled kernel once it is the cheaper one
   const int64_t tiles = p.total_tiles;
-  if (want_tiled_bf16(M, K, flags, &tiles, 1, aligned16(ws) ? ws_bytes : 0)) {
+  if (want_tiled_bf16(M, K, flags, &tiles, 1, ws_bytes)) {
     TPPX_REQUIRE(aligned16(w), TPPX_EINVAL, "%s: weight not 16-byte aligned", who);
-    return check_hip(launch_tiled_bf16(tiled_from_seg(p, 0), (hipStream_t)stream, aligned16(ws) ? (float*)ws : nullptr, ws_bytes), who);
+    return check_hip(launch_tiled_bf16(tiled_from_seg(p, 0), (hipStream_t)stream, (float*)ws, ws_bytes), who);
   }
   return run_bf16_rows(who, p, false, (hipStream_t)stream);
 }
@@ -867,7 +867,7 @@ static int run_bf16_group(const char* who, const void* x, const tppx_seg* segs, 
     return run_bf16_rows(who, p, dual, stream);
   group = group && want;
   TPPX_REQUIRE(group, TPPX_EUNSUPPORTED, "%s: M=%ld runs as one launch per weight", who, (long)M);
-  return check_hip(launch_tiled_bf16_group(t, n_segs, stream, dual, aligned16(ws) ? (float*)ws : nullptr, ws_bytes), who);
+  return check_hip(launch_tiled_bf16_group(t, n_segs, stream, dual, (float*)ws, ws_bytes), who);
 }
 
 extern "C" int tppx_group_is_one_launch(const int64_t* Ns, int n_segs, int64_t M, int64_t K, int weight_bytes) {

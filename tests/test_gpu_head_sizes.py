@@ -307,7 +307,7 @@ def test_decode_step_with_rotary_and_append_in_the_launch(H, HR, style, B, Nq, N
         assert torch.equal(out, first)
 
 
-@pytest.mark.parametrize("H,Nq,Nkv", [(64, 8, 2), (80, 4, 4), (256, 2, 2), (8, 2, 1), (200, 4, 2), (128, 28, 4), (128, 4, 2), (128, 34, 2)])
+@pytest.mark.parametrize("H,Nq,Nkv", [(64, 8, 2), (80, 4, 4), (256, 2, 2), (8, 2, 1), (200, 4, 2)])
 @pytest.mark.parametrize("B,L,Smax", [(2, 77, 128), (1, 1000, 1100)])
 def test_decode_step_rounds_the_output_only(H, Nq, Nkv, B, L, Smax):
     """The probabilities keep 16 bits on their way into p . v: against float64 the output is off by its own rounding to bf16,

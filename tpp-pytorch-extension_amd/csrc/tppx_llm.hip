@@ -1093,15 +1093,15 @@ attn_prefill_kernel(const AttnPrefillParams p) {
 // operand that the prompt kernel above fills with queries, so a key row is read once for all of them.
 // What bounds it is the cache stream.  A wave works by itself on tiles of 32 keys (8 KiB of K and of V, in two stages of its
 // own LDS, brought by loads straight into LDS; no barrier in the loop), the first one requested before the length is known;
-// 2 waves = 64 KiB, so that two workgroups of a CU have 64 to 128 KiB under way.  Scores, maximum and sums as in
-// attn_decode_wide_kernel; the waves and then the splits are merged in order, the latter by the last to arrive.  A probability
-// enters p . v as two bf16 terms, as in attn_hd_step_kernel: rounded to one, against a maximum that a whole wave shares, the
-// relative error against float64 was up to 1.02 times that of attn_decode_wide_kernel (32 heads on 16, 16 x 700 keys 2.15e-3 against
-// 2.11e-3), in two it is 1.66e-3, for 1 to 2 % of the time (28 on 4, 16 x 2500 19.6 -> 19.9 us).
+// 2 waves = 64 KiB, so that two workgroups of a CU have 64 to 128 KiB under way.  Scores, maximum, probabilities and sums as in
+// attn_decode_wide_kernel; the waves and then the splits are merged in order, the latter by the last to arrive.
+// The relative error against float64 is that kernel's (28 heads on 4, 64 on 8: 0.98 .. 1.00 of it over 33 .. 2500 keys), up to
+// 1.02 times it where fewer splits leave more keys to a running maximum (32 on 16, 16 x 700: 2.15e-3 and 2.11e-3).  With the
+// probabilities as two bf16 terms it would be 1.66e-3, for 1 to 2 % of the time.
 // Against a workgroup per query head (attn_decode_wide_kernel), which reads every row Nq / Nkv times through the L2s and does
-// its arithmetic on the vector units each time, us per launch: 28 heads on 4 of K/V, 16 sequences of 2500 keys 97 -> 19.9,
-// 48 of 1500 167 -> 34.6, 4 of 2000 30.6 -> 11.0, 1 of 4000 15.3 -> 12.2, 1 of 100 7.1 -> 6.1; 64 heads on 8, 16 of 2048
-// 157 -> 29.6; 32 on 16, 16 of 1000 44.6 -> 27.1 (4.8 TB/s of cache).  With a head per K/V head the other kernel is the faster one
+// its arithmetic on the vector units each time, us per launch: 28 heads on 4 of K/V, 16 sequences of 2500 keys 101 -> 20.6,
+// 48 of 1500 169 -> 32.7, 4 of 2000 27.6 -> 10.4, 1 of 4000 15.7 -> 11.8, 1 of 100 6.9 -> 6.3; 64 heads on 8, 16 of 2048
+// 164 -> 28.7; 32 on 16, 16 of 1000 44 -> 26.4 (5 TB/s of cache).  With a head per K/V head the other kernel is the faster one
 // from some 30 MB of cache on (32 heads, 16 of 2048 87 against 96 us: more waves with requests of their own).
 // ---------------------------------------------------------------------------
 constexpr int AG_WAVES = 2, AG_KEYS = 32 * AG_WAVES; // keys per workgroup and trip
@@ -1282,16 +1282,12 @@ attn_decode_group_kernel(const AttnParams p) {
         acc[dt] *= alpha;
       m = mx;
     }
-    i32x4 pb;     // the probabilities' leading bits, two to a word
-    bf16x8 pr2;   // the rest of them
+    bf16x8 pb;
 #pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      const float a = __expf(sc[i >> 2][i & 3] - m), b = __expf(sc[i >> 2][(i & 3) + 1] - m);
-      l += a;
-      l += b;
-      pb[i >> 1] = (int)__builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
-      pr2[i] = (__bf16)(a - __uint_as_float(__float_as_uint(a) & 0xffff0000u));
-      pr2[i + 1] = (__bf16)(b - __uint_as_float(__float_as_uint(b) & 0xffff0000u));
+    for (int i = 0; i < 8; i++) {
+      const float pr = __expf(sc[i >> 2][i & 3] - m);
+      l += pr;
+      pb[i] = (__bf16)pr;
     }
     // K slots g*8 .. +7 of the operand = keys g*4 .. +3 and 16 + g*4 .. +3, the keys pb holds in the same slots
     i32x2 vv[8][2];
@@ -1312,8 +1308,7 @@ attn_decode_group_kernel(const AttnParams p) {
 #pragma unroll
     for (int dt = 0; dt < 8; dt++) {
       const i32x4 av = {vv[dt][0][0], vv[dt][0][1], vv[dt][1][0], vv[dt][1][1]};
-      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), pr2, acc[dt], 0, 0, 0);
-      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, pb), acc[dt], 0, 0, 0);
+      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), pb, acc[dt], 0, 0, 0);
     }
   };
   // Tiles of this wave: base + i * S * AG_KEYS while they begin before the end of the keys.  While tile i is worked on tile

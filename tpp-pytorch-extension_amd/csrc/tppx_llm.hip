@@ -2455,7 +2455,7 @@ attn_hd_merge_kernel(const AttnGenParams p) {
 static int attn_generic_launch(const char* who, AttnGenParams& p, hipStream_t stream, void* ws = nullptr,
                                int64_t ws_bytes = 0, AttnCounters counters = {}) {
   TPPX_REQUIRE(p.H >= 8 && p.H <= 256 && p.H % 8 == 0, TPPX_EUNSUPPORTED,
-               "%s: head size %d (128 on the tuned kernels, other multiples of 8 up to 256 on the plain one)", who, p.H);
+               "%s: head size %d (multiples of 8 up to 256)", who, p.H);
   const int64_t queries = (int64_t)p.B * p.S * p.Nq;
   p.splits = 1;
   if (p.kv_len && p.S == 1 && env_int("TPPX_ATTN_GENERIC_ROWS", 1) != 0) {

@@ -197,6 +197,21 @@ def test_fix_vnni_and_block_size_rule():
     assert _ops.qint8_block_size_for(192) == 64 and _ops.qint8_block_size_for(384) == 128
 
 
+def test_a_quantized_tensor_finds_its_layout_when_asked(monkeypatch):
+    """Making a quantized tensor (loading a model, quantizing activations) does not ask for its weight layout, a microsecond of
+    a short call; the first question does, the later ones are answered from it."""
+    from tpp_pytorch_extension import _qtensor as Q
+
+    asked, find = [], Q.QTensor._find_layout
+    monkeypatch.setattr(Q.QTensor, "_find_layout", lambda self: asked.append(1) or find(self))
+    w = Q.QTensor(torch.zeros(4, 2, 32, 32, 2, dtype=torch.uint8), torch.zeros(1), (4, 2, 32, 32, 2), torch.quint4x2, Q.QSCHEME_MXFP, 32, 2, True, 2)
+    x = Q.QTensor(torch.zeros(3, 256, dtype=torch.int8), torch.zeros(3, 1), (3, 256), torch.qint8, Q.QSCHEME_AFFINE, 256, 1, False, 1)
+    assert not asked
+    for _ in range(3):
+        assert w.weight_layout() == ("mxfp4", 128, 128) and x.weight_layout() == (None, 0, 0)
+    assert len(asked) == 2
+
+
 def test_launch_plans_of_the_baseline_shapes():
     """Host-side planning (no GPU work): which kernel and grid the library would launch for the BASELINE shapes --
     decode GEMMs fill one round of 256 workgroups, the prefill GEMMs get the workgroup tile whose rounds are full, the

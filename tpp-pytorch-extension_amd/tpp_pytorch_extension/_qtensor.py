@@ -33,7 +33,7 @@ class QTensor(torch.Tensor):
         r.is_vnni = bool(is_vnni)
         r.pack_size = int(pack_size)
         r._native = None
-        r._layout = r._find_layout()
+        r._layout = None
         return r
 
     # -- observable surface of a quantized at::Tensor ------------------------
@@ -80,8 +80,10 @@ class QTensor(torch.Tensor):
         """(kind, N, K) of a linear-layer weight: "mxfp4" [N/32, K/64, 32, 32, 2], "mxfp4_int8" (the VNNI8-interleaved
         W4A8 layout) [N/8, K/bc, bc/8, 8, 8], "qint8" [N/16, K/QBS, QBS/4, 16, 4], "qint4" (VNNI2) [N/16, K/QBS, QBS/2,
         16, 2], "qint2" (interleaved ternary) [N/32, K/QBS, QBS/4, 32, 4]; (None, 0, 0) for any other layout (helper-only
-        tensors, quantized activations).  Found once, when the tensor is made: a tensor subclass takes 0.5-1 us to answer
-        for its shape or type, and a decoder layer's step asks some twenty times."""
+        tensors, quantized activations).  Found once, when it is first asked for: a tensor subclass takes 0.5-1 us to answer
+        for its shape or type, a decoder layer's step asks some twenty times, quantizing a tensor never does."""
+        if self._layout is None:
+            self._layout = self._find_layout()
         return self._layout
 
     def _find_layout(self):

@@ -578,5 +578,5 @@ def test_mxfp4_prompts_run_k_in_slices_where_that_pays():
                   (8512, 6400, 65), (7360, 9216, 155)):
         assert split(*shape), shape
     for shape in ((1408, 9216, 1024), (1408, 11520, 970), (9024, 10496, 183), (4096, 11008, 400), (6400, 9984, 234), (2496, 13056, 725),
-                  (1600, 9984, 847), (4096, 11008, 333)):
+                  (1600, 9984, 847), (4096, 11008, 333), (4096, 16384, 420), (3584, 18944, 480)):
         assert not split(*shape), shape

@@ -1896,8 +1896,10 @@ double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16) {
 // K slices (1: whole) of a launch of n GEMMs that takes whole_us without them, *us: what it takes then.  The 64 x 128 tile's
 // estimate for S times the workgroups and an S-th of the steps, and the slices' sums out and in: 2.2 us and 8.5 .. 16.5 ns
 // (MXFP4, the more the shorter K is) or 11.5 ns (bf16 weights) for each 32 KiB of them.  Up to K = 2560 (11.5 us whole, 11.3 in
-// slices at 65 rows), MXFP4 4096 (17 whole, 15 .. 22), no launch is split; up to one round of whole-K workgroups (bf16: a quarter
-// more).  Measured on 250 launches of 65 .. 1024 rows of 1024 .. 11000 channels and K = 2816 .. 16384:
+// slices at 65 rows), MXFP4 4096 (17 whole, 15 .. 22), no launch is split; bf16 up to one round of whole-K workgroups and a
+// quarter more, MXFP4 up to 200 of them: beyond, slices are a little faster by themselves (4096 x 16384 at 420 rows, 224
+// workgroups, 61.9 us, whole 64.4), but behind and before other kernels they are not (the GPT-J pass it is part of, three
+// layers, 699 .. 731 us, whole 677 .. 688; three Qwen2 layers at 420 .. 512 rows within 1.4 %).  Measured on 250 launches of 65 .. 1024 rows of 1024 .. 11000 channels and K = 2816 .. 16384:
 //   MXFP4  the slices' estimate is 3 .. 5 % high, but 2 % low with two slices of more than 160 workgroups or more than 730
 //          workgroups in all, and 1 % lower with each row block from the fifth on (more of them read the same weights).  With
 //          that, 6 % for the estimate's sake: none is slower than whole by more than 2 % (1408 x 9216 at 1024 rows, 34.0 us
@@ -1925,7 +1927,7 @@ static int best_split(int64_t M, int64_t K, const int* tiles, int n, int64_t par
     double c = tile_us((WBF16 ? BF16_COST : MXFP4_COST)[TILE_64_128], TILE_64_128, wgs * S, s / S, mb, false) + 2.2 + ns * 1e-3 * (double)(wgs * S);
     if (!WBF16)
       c *= 1.0 + rows + ((S == 2 ? wgs > 160 : wgs * S > 730) ? 0.02 : -0.04);
-    if (forced == S || (forced == 1 && K > (WBF16 ? 2560 : 4096) && wgs <= (WBF16 ? 320 : 256) && c < best_us)) {
+    if (forced == S || (forced == 1 && K > (WBF16 ? 2560 : 4096) && wgs <= (WBF16 ? 320 : 200) && c < best_us)) {
       best_us = c;
       best = S;
     }

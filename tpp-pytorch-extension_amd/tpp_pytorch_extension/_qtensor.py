@@ -82,9 +82,10 @@ class QTensor(torch.Tensor):
         16, 2], "qint2" (interleaved ternary) [N/32, K/QBS, QBS/4, 32, 4]; (None, 0, 0) for any other layout (helper-only
         tensors, quantized activations).  Found once, when it is first asked for: a tensor subclass takes 0.5-1 us to answer
         for its shape or type, a decoder layer's step asks some twenty times, quantizing a tensor never does."""
-        if self._layout is None:
-            self._layout = self._find_layout()
-        return self._layout
+        have = self._layout
+        if have is None:
+            have = self._layout = self._find_layout()
+        return have
 
     def _find_layout(self):
         if not self.is_vnni or self.axis != 2:

@@ -255,36 +255,36 @@ def test_launch_plans_of_the_baseline_shapes():
     assert len(lines) == 1 and "big_mxfp4_kernel<8, true, 1, 8> grid=1792x1x1" in lines[0]       # silu*mul in the epilogue
     lines = plan(L.tppx_plan_multi_linear_mxfp4, pair, 2, 2048, 8192, 1, _lib.FLAG_ACT_FP8, 1 << 28)
     assert any("big_fp8_kernel<8, true> grid=1792x1x1" in l for l in lines), lines
-    # prompts of a few hundred tokens: 64 x 128 workgroups, or 128 x 256 ones of eight waves while one per CU is enough
-    assert "big_mxfp4_kernel<2, false, 2, 2> grid=256x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 512, 4096, 4096,
-                                                                             _lib.FLAG_FORCE_TILED, 0)[0]
-    assert "big_mxfp4_kernel<2, false, 2, 2>" in plan(L.tppx_plan_linear_mxfp4, 512, 4096, 4096, 0, 0)[0]   # and it is the choice
-    assert "big_mxfp4_kernel<2, false, 2, 2> grid=688x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 512, 11008, 4096,
-                                                                             _lib.FLAG_FORCE_TILED, 0)[0]   # 42 us (172 of 128 x 256: 50)
-    assert "big_mxfp4_kernel<4, false, 2, 4> grid=256x1x1 block=512" in plan(L.tppx_plan_linear_mxfp4, 2048, 4096, 4096,
-                                                                             _lib.FLAG_FORCE_TILED, 0)[0]   # 50 us (64 x 128: 53)
+    # prompts of a few hundred tokens: the wave tile whose workgroups fill one round of the CUs best
+    assert "wide_kernel<4, 2, 4, false, false, false> grid=256x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 512, 4096, 4096,
+                                                                                      _lib.FLAG_FORCE_TILED, 0)[0]
+    assert "wide_kernel<4, 2, 4, false, false, false>" in plan(L.tppx_plan_linear_mxfp4, 512, 4096, 4096, 0, 0)[0]   # and it is the choice
+    assert "wide_kernel<4, 3, 8, false, false, false> grid=232x1x1 block=512" in plan(L.tppx_plan_linear_mxfp4, 512, 11008, 4096,
+                                                                                      _lib.FLAG_FORCE_TILED, 0)[0]
+    assert "wide_kernel<6, 3, 8, false, false, false> grid=242x1x1 block=512" in plan(L.tppx_plan_linear_mxfp4, 2048, 4096, 4096,
+                                                                                      _lib.FLAG_FORCE_TILED, 0)[0]
     pair7 = (ctypes.c_int64 * 2)(11008, 11008)
-    assert "big_mxfp4_kernel<2, true, 2, 2> grid=688x1x1 block=256" in plan(L.tppx_plan_multi_linear_mxfp4, pair7, 2, 256, 4096, 1,
-                                                                           _lib.FLAG_FORCE_TILED, 0)[0]     # 44 us (128 x 256: 51)
+    assert "wide_kernel<4, 3, 8, true, false, false> grid=232x1x1 block=512" in plan(L.tppx_plan_multi_linear_mxfp4, pair7, 2, 256, 4096, 1,
+                                                                                     _lib.FLAG_FORCE_TILED, 0)[0]
     pair2 = (ctypes.c_int64 * 2)(2048, 2048)
-    assert "big_mxfp4_kernel<4, true, 2, 4> grid=256x1x1 block=512" in plan(L.tppx_plan_multi_linear_mxfp4, pair2, 2, 2048, 4096, 1,
-                                                                           _lib.FLAG_FORCE_TILED, 0)[0]
+    assert "wide_kernel<6, 3, 8, true, false, false> grid=242x1x1 block=512" in plan(L.tppx_plan_multi_linear_mxfp4, pair2, 2, 2048, 4096, 1,
+                                                                                     _lib.FLAG_FORCE_TILED, 0)[0]
     assert "big_qint8_narrow_kernel grid=256x1x1 block=256" in plan(L.tppx_plan_linear_qint8, 512, 4096, 4096, 256, 1,
                                                                      _lib.FLAG_FORCE_TILED, 1 << 25)[-1]     # 22 us (128 of 64 x 256: 30)
     assert "big_qint8_kernel grid=172x1x1 block=512" in plan(L.tppx_plan_linear_qint8, 512, 11008, 4096, 256, 1,
                                                               _lib.FLAG_FORCE_TILED, 1 << 25)[-1]
     pair1 = (ctypes.c_int64 * 2)(4096, 4096)
-    assert "big_mxfp4_kernel<2, true, 2, 2> grid=256x1x1 block=256" in plan(L.tppx_plan_multi_linear_mxfp4, pair1, 2, 256, 4096, 1,
-                                                                           _lib.FLAG_FORCE_TILED, 0)[0]
-    assert "big_mxfp4_kernel<2, false, 2, 2> grid=1376x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 1024, 11008, 4096,
-                                                                              _lib.FLAG_FORCE_TILED, 0)[0]  # 79 us (128 x 512: 81)
+    assert "wide_kernel<4, 2, 4, true, false, false> grid=256x1x1 block=256" in plan(L.tppx_plan_multi_linear_mxfp4, pair1, 2, 256, 4096, 1,
+                                                                                     _lib.FLAG_FORCE_TILED, 0)[0]
+    assert "wide_kernel<6, 2, 8, false, false, false> grid=473x1x1 block=512" in plan(L.tppx_plan_linear_mxfp4, 1024, 11008, 4096,
+                                                                                      _lib.FLAG_FORCE_TILED, 0)[0]
     for M, other in ((511, 512), (1000, 1024)):  # whole 128-row blocks make no difference
         assert plan(L.tppx_plan_linear_mxfp4, M, 11008, 4096, 0, 0) == plan(L.tppx_plan_linear_mxfp4, other, 11008, 4096, 0, 0)
-    # from 65 rows on the 64-row forms take what the planner hands to a tiled kernel
-    assert "big_mxfp4_kernel<2, false, 2, 2> grid=96x1x1 block=256" in plan(L.tppx_plan_linear_mxfp4, 160, 4096, 4096, 0, 0)[0]
-    assert "big_mxfp4_kernel<2, false, 2, 2> grid=64x1x1" in plan(L.tppx_plan_linear_mxfp4, 128, 4096, 4096, 0, ws)[0]  # 17.0 us (rows 17.9)
+    # from 65 rows on the small wave tiles take what the planner hands to a tiled kernel
+    assert "wide_kernel<2, 1, 8, false, false, false> grid=160x1x1 block=512" in plan(L.tppx_plan_linear_mxfp4, 160, 4096, 4096, 0, 0)[0]
+    assert "wide_kernel<2, 1, 8, false, false, false> grid=128x1x1" in plan(L.tppx_plan_linear_mxfp4, 128, 4096, 4096, 0, ws)[0]  # 12 us (rows 17.9)
     assert "big_qint8_small_kernel grid=129x1x1 block=512" in plan(L.tppx_plan_linear_qint8, 160, 11008, 4096, 256, 1, 0, ws)[-1]
-    assert "big_mxfp4_kernel<2, false, 2, 2>" in plan(L.tppx_plan_linear_mxfp4, 100, 4096, 4096, _lib.FLAG_FORCE_TILED, 0)[0]
+    assert "wide_kernel<2, 1, 8, false, false, false>" in plan(L.tppx_plan_linear_mxfp4, 100, 4096, 4096, _lib.FLAG_FORCE_TILED, 0)[0]
 
 
 def test_launch_plans_of_per_output_channel_qint8():
@@ -335,12 +335,11 @@ def test_kernel_family_of_short_prompts():
 
     for M in (65, 128):
         assert "skinny_mxfp4" in pair(M, 1024, 4096) and "skinny_mxfp4" in pair(M, 1536, 18944), M  # 11 us (tiles 22), 38 (79)
-        assert "big_mxfp4" in one(M, 28672, 2560) and "big_mxfp4" in one(M, 18944, 1024), M         # 25 us (rows 52), 14 (26)
-        assert "big_mxfp4" in pair(M, 11008, 4096), M                                              # 34 us (rows 42)
-    for M in (160, 256):
-        assert "skinny_mxfp4" in one(M, 1024, 18944) and "skinny_mxfp4" in pair(M, 1024, 8192), M    # 36 us (77), 19 (38)
-    assert "big_mxfp4" in one(192, 14336, 5120)                                                     # 42 us (65)
-    assert "<2, false, 2, 2>" not in one(1800, 2560, 11008) and "<2, false, 2, 2>" in one(1500, 1536, 18944)
+        assert "wide_kernel" in one(M, 28672, 2560) and "wide_kernel" in one(M, 18944, 1024), M     # (rows 52 us, 26)
+        assert "wide_kernel" in pair(M, 11008, 4096), M                                            # (rows 42 us)
+    assert "skinny_mxfp4" in pair(160, 1024, 8192)                                                  # 19 us (tiles 38)
+    assert "wide_kernel" in one(192, 14336, 5120)                                                   # (rows 65 us)
+    assert "<5, 2, 8," in one(1800, 2560, 11008) and "<5, 2, 4," in one(1500, 1536, 18944)
     assert "<8, true, 1, 8>" in pair(2048, 28672, 8192)                                             # 1254 us (128 x 256: 1283)
 
     def qkv(M, N, K):
@@ -348,15 +347,14 @@ def test_kernel_family_of_short_prompts():
         return buf.value.decode()
 
     for M in (96, 127, 128, 129):  # nothing changes at whole block rows of 64
-        assert "<2, false, 2, 2>" in qkv(M, 4096, 4096), M                                          # 18.6 us (rows 35)
-        assert "<2, false, 2, 2>" in one(M, 12288, 4096) and "<2, false, 2, 2>" in one(M, 11008, 4096), M  # 18 us (26)
+        assert "wide_kernel" in qkv(M, 4096, 4096), M                                               # 17 us (rows 35)
+        assert "wide_kernel" in one(M, 12288, 4096) and "wide_kernel" in one(M, 11008, 4096), M     # 17 us (26)
         assert "skinny_mxfp4" in one(M, 1024, 4096), M                                              # 8 us (tiles 16)
 
-    # 64 x 128 workgroups in whole columns per XCD drift apart from 21 row blocks on, also with an even number of them
-    assert "<2, false, 2, 2>" not in one(2048, 9088, 8704) and "<2, false, 2, 2>" not in one(1744, 6528, 10496)  # 250 us (342), 183 (251)
-    assert "<2, false, 2, 2>" not in one(1421, 4096, 11008) and "<2, false, 2, 2>" in one(1421, 4096, 4096)      # 111 us (125), 44 (50)
-    assert "<2, false, 2, 2>" not in qkv(2048, 1856, 13312) and "<2, true, 2, 2>" not in pair(2048, 2880, 7168)   # 230 us (339), 134 (180)
-    assert "<2, false, 2, 2>" in one(2048, 4800, 4096)                                              # rectangles: 63 us (74)
+    # long prompts: not the small wave tiles, whose workgroups drift apart in K where the XCDs get whole columns
+    for shape in ((2048, 9088, 8704), (1744, 6528, 10496), (1421, 4096, 11008), (1421, 4096, 4096), (2048, 4800, 4096)):
+        assert not any(small in one(*shape) for small in ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,")), shape
+    assert "<3, 2, 4," not in qkv(2048, 1856, 13312) and "<4, 2, 4," not in pair(2048, 2880, 7168)
 
     def per_weight(M, N, K, weight_bytes):
         return not L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, weight_bytes)
@@ -572,10 +570,9 @@ def test_mxfp4_prompts_run_k_in_slices_where_that_pays():
     def split(n, k, m):
         buf = ctypes.create_string_buffer(4096)
         _lib.check(L.tppx_plan_linear_mxfp4(m, n, k, 0, 32 << 20, buf, len(buf)))
-        return "side_split_kernel" in buf.value.decode()
+        return "wide_sum_kernel" in buf.value.decode()
 
-    for shape in ((4096, 11008, 100), (4096, 11008, 200), (4096, 11008, 300), (2560, 10240, 200), (3584, 18944, 333), (2112, 4608, 381),
-                  (8512, 6400, 65), (7360, 9216, 155)):
+    for shape in ((4096, 11008, 100), (4096, 11008, 200), (2560, 10240, 200), (3584, 18944, 333)):
         assert split(*shape), shape
     for shape in ((1408, 9216, 1024), (1408, 11520, 970), (9024, 10496, 183), (4096, 11008, 400), (6400, 9984, 234), (2496, 13056, 725),
                   (1600, 9984, 847), (4096, 11008, 333), (4096, 16384, 420), (3584, 18944, 480)):

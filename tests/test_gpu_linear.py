@@ -658,7 +658,7 @@ def test_launch_plan_names_the_kernels():
     _lib.check(L.tppx_plan_linear_mxfp4(2048, 8192, 8192, 0, 0, buf, len(buf)))
     assert "big_mxfp4_kernel" in buf.value.decode()
     _lib.check(L.tppx_plan_linear_mxfp4(100, 8192, 8192, _lib.FLAG_FORCE_TILED, 0, buf, len(buf)))
-    assert "big_mxfp4_kernel<2, false, 2, 2>" in buf.value.decode()  # 64 x 128 workgroups from 65 rows on
+    assert "wide_kernel<2, 1, 8, false, false, false>" in buf.value.decode()  # small wave tiles from 65 rows on
     _lib.check(L.tppx_plan_linear_mxfp4(128, 1024, 4096, 0, 0, buf, len(buf)))  # few tiles: block rows of 64
     assert "skinny_mxfp4_mg_kernel" in buf.value.decode() and "x2x" in buf.value.decode()
 
@@ -1117,7 +1117,7 @@ def test_prompt_gemms_with_k_in_slices(fmt, S, M, N, K, monkeypatch):
         import ctypes
         buf = ctypes.create_string_buffer(4096)
         _lib.check(_lib.lib().tppx_plan_linear_mxfp4(M, N, K, 0, 1 << 25, buf, len(buf)))
-        assert f"side_split_kernel<false> grid={(M + 63) // 64 * ((N + 127) // 128)}x{S}x1" in buf.value.decode()
+        assert "false, true> grid=" in buf.value.decode() and f"x{S}x1" in buf.value.decode()
     if fmt == "bf16":
         ref = x.double() @ flat[1].cuda().double().t()
         assert ((got[3].double() - ref).norm() / ref.norm()).item() < 2.0 ** -8
@@ -1207,7 +1207,7 @@ def test_prompt_qint8_gemms_with_k_in_slices(S, M, N, K, monkeypatch):
 @pytest.mark.parametrize("fmt", ["mxfp4", "bf16"])
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 7])
 def test_prefill_side_by_side_forms_at_every_loop_remainder(fmt, steps, monkeypatch):
-    """The forms whose waves keep the weights in registers (64 x 128; bf16: 64 x 256 and 128 x 256 as well) run their K steps
+    """The forms whose waves keep the weights in registers (bf16: 64 x 128, 64 x 256 and 128 x 256 as well) run their K steps
     of 128 by threes with a tail: one step up to two rounds and a remainder, rows and channel blocks ragged, against the
     256 x 256 form (the same sums in the same order, hence the same bits): linear, q/k/v, pair."""
     ops = _ops()
@@ -1230,6 +1230,57 @@ def test_prefill_side_by_side_forms_at_every_loop_remainder(fmt, steps, monkeypa
         monkeypatch.setenv("TPPX_TILED_BIG_TILE", tile)
         for i, (a, w) in enumerate(zip(run(), want)):
             assert torch.equal(a, w), (tile, i)
+
+
+@pytest.mark.parametrize("fmt,forms", [("mxfp4", range(7, 18)), ("bf16", (11, 15))])
+@pytest.mark.parametrize("M,N,K", [(65, 1056, 128), (70, 288, 640), (97, 1568, 896), (201, 352, 1152), (333, 800, 512)])
+def test_prefill_wave_tiles_agree(fmt, forms, M, N, K, monkeypatch):
+    """Every wave tile of the launches of up to a few workgroups per CU: 1 .. 9 K steps (rings of three and four stages), rows and
+    channel blocks ragged (row tiles of a block past the end, one live channel tile of a wave's three), a pair dealt out over
+    the waves, the residual's read-ahead, against the 256 x 256 form: the same sums in the same order, hence the same bits."""
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    if fmt == "mxfp4":
+        ws = [_make("mxfp4", n, K, 950 + i)[0] for i, n in enumerate((N, 32, 160, N))]
+    else:
+        ws = [block_bf16(randn_bf16((n, K), 0.05, 950 + i)).cuda() for i, n in enumerate((N, 32, 160, N))]
+    x, res, b = randn_bf16((M, K), 1.0, 955).cuda(), randn_bf16((M, N), 1.0, 956).cuda(), randn_bf16((N,), 0.5, 957).cuda()
+
+    def run():
+        return [ops.fc_add(x, ws[0], b, res, 0.5), ops.fc_gelu(x, ws[0], b), ops.swiglu_gate_up(x, ws[0], ws[3], b, None)] + \
+            list(ops.qkv_gemm(x, ws[:3], [b, None, None]))
+
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")  # the LDS-tiled family whatever the cost estimate says
+    monkeypatch.setenv("TPPX_TILED_SPLIT", "0")
+    monkeypatch.setenv("TPPX_TILED_BIG_TILE", "1")
+    want = run()
+    for form in forms:
+        monkeypatch.setenv("TPPX_TILED_BIG_TILE", str(form))
+        for i, (a, w) in enumerate(zip(run(), want)):
+            assert torch.equal(a, w), (form, i)
+
+
+@pytest.mark.parametrize("S", [2, 3, 4, 6])
+@pytest.mark.parametrize("form", [7, 8, 9])
+def test_prefill_wave_tiles_with_k_in_slices(form, S, monkeypatch):
+    """Slices of unequal steps on each wave tile that has them, and without room for their sums (K whole, the same call)."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    M, N, K = 77, 288, 128 * (4 * S + 3)
+    w = _make("mxfp4", N, K, 960 + S)[0]
+    x, res = randn_bf16((M, K), 1.0, 961).cuda(), randn_bf16((M, N), 1.0, 962).cuda()
+    monkeypatch.setenv("TPPX_TILED_MIN_M", "0")
+    monkeypatch.setenv("TPPX_TILED_BIG_TILE", str(form))
+    monkeypatch.setenv("TPPX_TILED_SPLIT", "0")
+    want = ops.fc_add(x, w, None, res, 1.0).double()
+    monkeypatch.setenv("TPPX_TILED_SPLIT", str(S))
+    got = ops.fc_add(x, w, None, res, 1.0).double()
+    assert (got - want).norm() <= 2.0 ** -9 * want.norm()
+    buf = ctypes.create_string_buffer(4096)
+    for ws_bytes, slices in ((1 << 25, True), (1 << 12, False)):
+        _lib.check(_lib.lib().tppx_plan_linear_mxfp4(M, N, K, 0, ws_bytes, buf, len(buf)))
+        assert ("wide_sum_kernel" in buf.value.decode()) == slices, ws_bytes
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 16, 256), (64 * 3, 272, 512), (129, 4080, 768), (300, 8208, 1024), (1000, 1040, 1280)])

@@ -270,8 +270,7 @@ static bool want_tiled_mxfp4(int64_t M, int64_t K, int flags, int64_t tiles, boo
   static constexpr RowsCost SINGLE[3] = {{3.19, 0.678, 0.958, 0.765}, {2.78, 1.82, 1.10, 0.958}, {2.35, 3.22, 1.61, 0.628}};
   static constexpr RowsCost DUAL[3] = {{2.82, 1.16, 1.14, 0.883}, {2.92, 3.4, 1.51, 0.984}, {2.42, 5.0, 2.31, 1.02}};
   static constexpr RowsCost NK = {3.24, 6.86, 0.400, 0.333};
-  // (narrower ones, which the decode kernels run well, have not been measured with K in slices)
-  const double tiled = nk && tiles >= 128 ? tiled_mxfp4_split_us(M, K, tiles, ws_bytes) : tiled_mxfp4_us(M, K, n_tiles16);
+  const double tiled = tiled_mxfp4_us(M, K, n_tiles16, dual ? 0 : ws_bytes);
   if (nk && mxfp4_nk_fits(M, (int)tiles, (int)(K / 128), ws_bytes))
     return tiled <= rows_us(NK, (tiles + 3) / 4 * 4 * rows64, M, K);
   const int nt = tiles <= 256 ? 1 : (tiles + 1) / 2 <= 256 ? 2 : 3; // channel tiles per workgroup, as the launch picks them
@@ -332,7 +331,7 @@ static bool want_tiled_bf16(int64_t M, int64_t K, int flags, const int64_t* tile
     all += tiles[i];
   }
   if (M >= big_min_rows() && env_int("TPPX_BF16_BIG", 1) != 0)
-    return (n == 1 && all >= 128 ? tiled_bf16_split_us(M, K, all, ws_bytes) : tiled_bf16_us(M, K, all)) <= 1.04 * rows;
+    return tiled_bf16_us(M, K, all, n == 1 && all >= 128 ? ws_bytes : 0) <= 1.04 * rows;
   const int64_t wgs = ((M + 127) / 128) * ((all + 7) / 8); // tiled_bf16_kernel
   return (double)((wgs + 255) / 256) * (double)K * 0.0203 <=
          (double)rows64 * (8.0 + (double)all * 32.0 * (double)K / 5.5e6 + (double)K * 0.0008);

@@ -127,6 +127,17 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
+// LDS image of bf16 MFMA operands: the 16-byte chunk c (0..15) of row m's 128 K values lies at position c ^ swz16(m) of 16.
+// Lane (g, m) of a read takes chunk g * 4 + j of row m.  A ds_read_b128 is served in four sets of 16 lanes, 64 banks each,
+// and a set takes the lanes m = 0..3 and 12..15 of an even g together with m = 4..11 of the next (lanes 0-3, 12-15, 20-27).
+// With c ^ m the bits of g and m cancel, the second half of a set has the banks of the first, and every read takes twice
+// its cycles (SQ_LDS_BANK_CONFLICT 0.5 of SQ_LDS_IDX_ACTIVE); with bit 3 of m flipped where bit 2 is set they do not.
+// The four chunks of an aligned quad stay together: loads into LDS fetch 64 bytes per four lanes (another order that read
+// without conflicts, (j * 4 + g) ^ m, spread them over the row and cost 7 % of the whole kernel at 333 rows).
+__device__ __forceinline__ constexpr int swz16(int m) {
+  return (m ^ ((m & 4) << 1)) & 15;
+}
+
 // W4A8 (USE_MXFP4_INT8): the integer the reference multiplies for an E2M1 code = its value times 127 / 6, rounded
 // four 4-bit E2M1 codes (one per byte, the upper four bits clear) -> four int8 values {0 11 21 32 42 64 85 127} with sign.
 // Two byte permutes look up all sixteen codes: selector bytes 0..7 pick a table byte (0..3 from the second operand, 4..7

@@ -104,11 +104,9 @@ struct TiledParams {
 
 // part (of the single GEMM and group launches): room for the fp32 sums of K slices, or null: K stays whole
 hipError_t launch_tiled_mxfp4(const TiledParams& p, hipStream_t stream, float* part = nullptr, int64_t part_bytes = 0);
-// what the large-M launches take for n_tiles16 tiles of 16 output channels, in us (estimate)
-double tiled_mxfp4_us(int64_t M, int64_t K, int64_t n_tiles16);
-// one GEMM, with that much workspace for K slices
-double tiled_mxfp4_split_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes);
-double tiled_bf16_split_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes);
+// what the large-M launches take for n_tiles16 tiles of 16 output channels, with that much workspace for K slices, in us (estimate)
+double tiled_mxfp4_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes);
+double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes);
 // large-M kernel: several GEMMs over one activation in one launch
 bool tiled_mxfp4_takes_groups(const TiledParams& p);
 // dual: the gate/up pair (t[0] = gate, t[1] = up) with silu(gate) * up formed in the launch and written to t[1].y
@@ -117,7 +115,6 @@ hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t str
 hipError_t launch_tiled_qint8(const TiledParams& p, hipStream_t stream, float* part = nullptr, int64_t part_bytes = 0);
 // unquantized bf16 weights (native bf16 tiles in p.qw), more than 64 rows
 hipError_t launch_tiled_bf16(const TiledParams& p, hipStream_t stream, float* part = nullptr, int64_t part_bytes = 0);
-double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16);
 bool tiled_bf16_takes_groups(const TiledParams& p);
 hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual, float* part = nullptr,
                                    int64_t part_bytes = 0);

@@ -26,50 +26,9 @@
 
 #include "tppx_common.h"
 #include "tppx_launch.h"
+#include "tppx_tiled.h"
 
 namespace tppx {
-
-__device__ __forceinline__ bf16x8 tl_cvt_fp4x8(uint32_t codes, float scale) {
-  bf16x2 c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, scale, 0);
-  bf16x2 c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, scale, 1);
-  bf16x2 c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, scale, 2);
-  bf16x2 c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, scale, 3);
-  bf16x8 w;
-  w[0] = c0[0]; w[1] = c0[1]; w[2] = c1[0]; w[3] = c1[1];
-  w[4] = c2[0]; w[5] = c2[1]; w[6] = c3[0]; w[7] = c3[1];
-  return w;
-}
-
-// buffer descriptor of an operand below 4 GiB (addresses checked by the host, so without a bound of its own)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t tl_rsrc(const void* q) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(q), 0, 0xffffffffu, 0x00020000);
-}
-
-// XCD-aware tile order: returns (bm, bn) of this workgroup.  Workgroup ids go round the 8 XCDs; XCD x gets a
-// rectangle of the tile space and walks it row block fastest, so that the workgroups resident on an XCD at the same
-// time share operand tiles in its L2.  xm = how many of the 8 rectangles lie along M (1: an XCD owns NB/8 channel
-// blocks and all row blocks; 2, 4: 1/xm of the row blocks and xm/8 of the channel blocks).  Every XCD fetches
-// 1/xm of the activations and xm/8 of the weights from memory.  The host passes an xm that divides evenly.
-__device__ __forceinline__ void tile_of_block(int MB, int NB, int& bm, int& bn, int xm, int id) {
-  const int T = MB * NB;
-  if ((T & 7) == 0 && xm > 1) {
-    const int x = id & 7, r = id >> 3;
-    const int xn = 8 / xm;                // rectangles along N
-    const int mb = MB / xm, nb = NB / xn; // the rectangle of XCD x: mb x nb tiles at (x % xm, x / xm)
-    bm = (x % xm) * mb + r % mb;
-    bn = (x / xm) * nb + r / mb;
-    return;
-  }
-  // an eighth of the tiles in column-major order, whether or not NB divides by 8 (the first T mod 8 XCDs own one more);
-  // dealt round the XCDs instead, each of them fetches most of the weights
-  const int x = id & 7;
-  id = x * (T >> 3) + min(x, T & 7) + (id >> 3);
-  bm = id % MB;
-  bn = id / MB;
-}
-__device__ __forceinline__ void tile_of_block(int MB, int NB, int& bm, int& bn, int xm = 1) {
-  tile_of_block(MB, NB, bm, bn, xm, blockIdx.x);
-}
 
 template <typename Acc>
 __device__ __forceinline__ void tiled_epilogue(const TiledParams& p, Acc& acc, int m_base, int tile_base) {
@@ -439,161 +398,6 @@ tiled_qint8_kernel(const TiledParams p) {
 // LDS byte address of chunk ck of row m of row tile mt:
 //   mt*4096 + (m>>2)*1024 + (m&3)*256 + ((ck ^ m) & 15)*16.
 // ---------------------------------------------------------------------------
-// Epilogue of a 128 x 64 wave tile through a wave-private LDS region: the
-// fp32 sums of 64 rows at a time are written there (statically indexed, so the
-// accumulators stay in registers), then read back row-contiguously; every
-// lane finishes 8 adjacent channels and writes them with one 16-byte store.
-// It is a chain at the end of every workgroup, so what bounds it is latency: the post-op is chosen once in front of it
-// (chosen per output, every one of the 8 x 16 sat behind branches of its own) and its input is requested whole before
-// the first sum is staged (requested in the loop, each of 16 rounds waited for memory).  QINT8 4096 x 4096 with residual
-// at 1000 / 2048 rows 33.1 -> 28.7 / 51.6 -> 44.0 us, 11008 x 4096 at 1000 rows 87.8 -> 71.5; a four-layer prompt on bf16
-// weights at 2048 tokens 3478 -> 3277, MXFP4 at 333 989 -> 919.
-constexpr int EP_LD = 68; // floats per staged row of 64 channels: 64 + 4 keeps the 4-row lane groups on distinct banks
-constexpr int ep_ld(int nt) { return nt * 16 + 4; }
-template <int MT, int POST, int NT> // POST < 0: whatever p.post_op says; NT = 16-channel tiles of the wave tile (4 or 2)
-__device__ __forceinline__ void big_epilogue_post(const TiledParams& p, f32x4 (&acc)[MT][NT], float* stage, int m_base,
-                                                  int tile_base) {
-  constexpr bool INPUT = POST == TPPX_POST_MUL || POST == TPPX_POST_ADD_SCALE;
-  const int lane = threadIdx.x & 63;
-  constexpr int LPR = NT * 2, RPI = 64 / LPR, LD = ep_ld(NT); // lanes per row, rows per wave instruction
-  const int cx = (lane % LPR) * 8; // first of this lane's 8 channels inside the wave tile
-  const int tile = tile_base + (cx >> 4);
-  const bool tile_ok = tile < p.tiles;
-  const int n = min(tile, p.tiles - 1) * 16 + (cx & 15);
-  constexpr int MH = MT < 4 ? MT : 4; // row tiles staged at a time (64 rows, or the whole wave tile when it has fewer)
-  // every input of the post-op is requested before the first sum is staged (rows past the end read the last one)
-  constexpr int NI = MH * 16 / RPI;
-  uint4 in[INPUT ? MT / MH * NI : 1];
-  if constexpr (INPUT) {
-#pragma unroll
-    for (int it = 0; it < MT / MH * NI; it++)
-      in[it] = *reinterpret_cast<const uint4*>(p.post_in + (int64_t)min(m_base + it * RPI + lane / LPR, p.M - 1) * p.N + n);
-  }
-  float bias[8];
-#pragma unroll
-  for (int e = 0; e < 8; e++)
-    bias[e] = p.bias ? bf16_bits_to_f32(p.bias[n + e]) : 0.0f;
-#pragma unroll
-  for (int h = 0; h < MT / MH; h++) {
-#pragma unroll
-    for (int mt = 0; mt < MH; mt++)
-#pragma unroll
-      for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          stage[(mt * 16 + (lane >> 4) * 4 + r) * LD + nt * 16 + (lane & 15)] = acc[h * MH + mt][nt][r];
-    // same wave wrote and reads: no barrier, the compiler orders the LDS accesses
-    auto rows8 = [&](int it) {
-      const int row = it * RPI + lane / LPR;
-      const int m = m_base + h * (MH * 16) + row;
-      const f32x4 v0 = *reinterpret_cast<const f32x4*>(stage + row * LD + cx);
-      const f32x4 v1 = *reinterpret_cast<const f32x4*>(stage + row * LD + cx + 4);
-      const int64_t o = (int64_t)m * p.N + n;
-      uint32_t out[4];
-      if constexpr (POST >= 0) {
-        const uint4 i1 = INPUT ? in[INPUT ? h * NI + it : 0] : make_uint4(0, 0, 0, 0);
-        const uint32_t w1[4] = {i1.x, i1.y, i1.z, i1.w};
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-          out[e] = apply_post_pair<POST>((e < 2 ? v0[2 * e] : v1[2 * e - 4]) + bias[2 * e],
-                                         (e < 2 ? v0[2 * e + 1] : v1[2 * e - 3]) + bias[2 * e + 1], w1[e], p.post_scale);
-        if (tile_ok && m < p.M)
-          *reinterpret_cast<uint4*>(p.y + o) = make_uint4(out[0], out[1], out[2], out[3]);
-      } else if (tile_ok && m < p.M) {
-        uint4 i1 = make_uint4(0, 0, 0, 0), i2 = make_uint4(0, 0, 0, 0);
-        if (p.post_in)
-          i1 = *reinterpret_cast<const uint4*>(p.post_in + o);
-        if (p.post_in2)
-          i2 = *reinterpret_cast<const uint4*>(p.post_in2 + o);
-        const uint32_t w1[4] = {i1.x, i1.y, i1.z, i1.w}, w2[4] = {i2.x, i2.y, i2.z, i2.w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const float lo = (e < 2 ? v0[2 * e] : v1[2 * e - 4]) + bias[2 * e];
-          const float hi = (e < 2 ? v0[2 * e + 1] : v1[2 * e - 3]) + bias[2 * e + 1];
-          const uint32_t a = apply_post_bits(lo, p.post_op, w1[e] & 0xffffu, w2[e] & 0xffffu, p.post_scale);
-          const uint32_t b = apply_post_bits(hi, p.post_op, w1[e] >> 16, w2[e] >> 16, p.post_scale);
-          out[e] = (a & 0xffffu) | (b << 16);
-        }
-        *reinterpret_cast<uint4*>(p.y + o) = make_uint4(out[0], out[1], out[2], out[3]);
-      }
-    };
-    if constexpr (POST >= 0) {
-#pragma unroll
-      for (int it = 0; it < NI; it++)
-        rows8(it);
-    } else {
-      for (int it = 0; it < NI; it++)
-        rows8(it);
-    }
-  }
-}
-
-template <int MT, int NT = 4>
-__device__ __forceinline__ void big_epilogue(const TiledParams& p, f32x4 (&acc)[MT][NT], float* stage, int m_base,
-                                             int tile_base) {
-  switch (p.post_op) {
-  case TPPX_POST_NONE: return big_epilogue_post<MT, TPPX_POST_NONE, NT>(p, acc, stage, m_base, tile_base);
-  case TPPX_POST_SILU: return big_epilogue_post<MT, TPPX_POST_SILU, NT>(p, acc, stage, m_base, tile_base);
-  case TPPX_POST_MUL: return big_epilogue_post<MT, TPPX_POST_MUL, NT>(p, acc, stage, m_base, tile_base);
-  case TPPX_POST_ADD_SCALE: return big_epilogue_post<MT, TPPX_POST_ADD_SCALE, NT>(p, acc, stage, m_base, tile_base);
-  default: return big_epilogue_post<MT, -1, NT>(p, acc, stage, m_base, tile_base);
-  }
-}
-
-// The gate/up pair: the first half of the wave tile's channels are gate sums and the second the up sums of the SAME
-// output channels, so silu(gate) * up is formed here, with the rounding points of SiluPostOp followed by MulPostOp, and
-// only the product is written: a lane finishes 8 adjacent channels of one row (16-byte store, NT lanes per row).
-template <int MT, int NT = 4>
-__device__ __forceinline__ void big_epilogue_dual(const TiledParams& pg, const TiledParams& pu, f32x4 (&acc)[MT][NT],
-                                                  float* stage, int m_base, int tile_base) {
-  const int lane = threadIdx.x & 63;
-  constexpr int LPR = NT, RPI = 64 / LPR, LD = ep_ld(NT);
-  const int cx = (lane % LPR) * 8; // first of this lane's 8 channels among the wave's NT * 8
-  const int tile = tile_base + (cx >> 4);
-  const bool tile_ok = tile < pg.tiles;
-  const int n = min(tile, pg.tiles - 1) * 16 + (cx & 15);
-  float bg[8], bu[8];
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    bg[e] = pg.bias ? bf16_bits_to_f32(pg.bias[n + e]) : 0.0f;
-    bu[e] = pu.bias ? bf16_bits_to_f32(pu.bias[n + e]) : 0.0f;
-  }
-  constexpr int MH = MT < 4 ? MT : 4; // row tiles staged at a time
-#pragma unroll
-  for (int h = 0; h < MT / MH; h++) {
-#pragma unroll
-    for (int mt = 0; mt < MH; mt++)
-#pragma unroll
-      for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          stage[(mt * 16 + (lane >> 4) * 4 + r) * LD + nt * 16 + (lane & 15)] = acc[h * MH + mt][nt][r];
-    // same wave wrote and reads: no barrier, the compiler orders the LDS accesses
-#pragma unroll
-    for (int it = 0; it < MH * 16 / RPI; it++) {
-      const int row = it * RPI + lane / LPR;
-      const int m = m_base + h * (MH * 16) + row;
-      const f32x4 g0 = *reinterpret_cast<const f32x4*>(stage + row * LD + cx);
-      const f32x4 g1 = *reinterpret_cast<const f32x4*>(stage + row * LD + cx + 4);
-      const f32x4 u0 = *reinterpret_cast<const f32x4*>(stage + row * LD + NT * 8 + cx);
-      const f32x4 u1 = *reinterpret_cast<const f32x4*>(stage + row * LD + NT * 8 + cx + 4);
-      if (tile_ok && m < pg.M) {
-        uint32_t out[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const float glo = (e < 2 ? g0[2 * e] : g1[2 * e - 4]) + bg[2 * e];
-          const float ghi = (e < 2 ? g0[2 * e + 1] : g1[2 * e - 3]) + bg[2 * e + 1];
-          const float ulo = (e < 2 ? u0[2 * e] : u1[2 * e - 4]) + bu[2 * e];
-          const float uhi = (e < 2 ? u0[2 * e + 1] : u1[2 * e - 3]) + bu[2 * e + 1];
-          const uint32_t gate = apply_post_pair<TPPX_POST_SILU>(glo, ghi, 0, 1.0f);
-          out[e] = apply_post_pair<TPPX_POST_MUL>(ulo, uhi, gate, 1.0f);
-        }
-        *reinterpret_cast<uint4*>(pu.y + (int64_t)m * pu.N + n) = make_uint4(out[0], out[1], out[2], out[3]);
-      }
-    }
-  }
-}
-
 // LDS operand reads issued by hand, so that they can be kept several MFMA
 // groups ahead of their use: the compiler does not track them, the waits are
 // explicit (LDS operations complete in issue order, so "at most N younger
@@ -607,17 +411,6 @@ template <int N>
 __device__ __forceinline__ void lds_wait_keep(i32x4& r) {
   asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(N));
 }
-
-// Several GEMMs over one activation (fused q/k/v) share a launch: the channel
-// blocks of all segments form one grid.
-struct BigParams {
-  TiledParams seg[TPPX_MAX_SEGS];
-  int nb0[TPPX_MAX_SEGS + 1]; // first channel block of each segment, then the total
-  int n_seg;
-  int xm;                     // XCD rectangles along M (see tile_of_block)
-  int S;                      // K slices (grid y) whose sums go to `part`; side_gemm_body with SPLIT
-  float* part;                // [S][workgroup][wave][MT * 2 tiles][64 lanes][4]
-};
 
 // MT = 16-row tiles per wave along M (8).
 // DUAL: the gate/up pair (seg[0] = gate, seg[1] = up, equal shapes).  A workgroup owns 128 output channels and
@@ -682,31 +475,31 @@ __device__ __forceinline__ void big_gemm_body(const BigParams& P) {
   // global memory straight into LDS, one wave instruction per block (lane =
   // row r of the block, 16-byte chunk).  The LDS image of an instruction is
   // lane-linear, so the swizzle is applied on the global side: the lane at
-  // position ch of row m fetches chunk ch ^ (m & 15).  Operand reads of one K
-  // group (16 rows, same chunk) then fall on 16 different bank groups.
+  // position ch of row m fetches chunk ch ^ swz16(m & 15); operand reads
+  // then fall on all the banks (see swz16).
   //   LDS byte address of chunk ck of row m of row tile mt:
-  //     mt*4096 + (m>>2)*1024 + (m&3)*256 + ((ck ^ m) & 15)*16
+  //     mt*4096 + (m>>2)*1024 + (m&3)*256 + (ck ^ swz16(m))*16
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(tl_lds); // LDS byte address of the buffers
   uint32_t rdb[4]; // byte offset of this lane's operand for step j (+ mt*4096): chunk ck = g*4 + j
   {
     const int m = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int j = 0; j < 4; j++)
-      rdb[j] = (uint32_t)((m >> 2) * 1024 + (m & 3) * 256 + (((g * 4 + j) ^ m) & 15) * 16);
+      rdb[j] = (uint32_t)((m >> 2) * 1024 + (m & 3) * 256 + ((g * 4 + j) ^ swz16(m)) * 16);
   }
   const char* xbase = reinterpret_cast<const char*>(p.x);
   // this wave's NBLK blocks: blk = wave*NBLK + i -> rows blk*4 + (lane>>4)
   const int rin = (lane >> 4);          // row inside the block
   const int ch = lane & 15;             // chunk position of this lane inside the row
   // source byte offset of block i at K step ks:
-  //   row(i) * K * 2 + ((ch ^ m16(i)) & 15) * 16 + ks * 256, row(i) = m_wg + (wave*8 + i)*4 + rin,
+  //   row(i) * K * 2 + (ch ^ swz16(m16(i))) * 16 + ks * 256, row(i) = m_wg + (wave*8 + i)*4 + rin,
   //   m16(i) = (i & 3)*4 + rin (wave*8 is a multiple of 4)
   const bool full = m_wg + WGM <= p.M; // uniform
   const uint32_t xrow0 = (uint32_t)((m_wg + wave * (NBLK * 4) + rin) * p.K) * 2u;
   const uint32_t blk_stride = (uint32_t)(4 * p.K) * 2u; // uniform
   auto load_a_one = [&](auto I, int ks, int buf) {
     constexpr int i = decltype(I)::value;
-    const uint32_t sw = (uint32_t)((ch ^ ((i & 3) * 4 + rin)) & 15) * 16u;
+    const uint32_t sw = (uint32_t)(ch ^ swz16((i & 3) * 4 + rin)) * 16u;
     uint32_t off;
     if (full) {
       off = xrow0 + (uint32_t)i * blk_stride + sw + (uint32_t)ks * 256u;
@@ -848,32 +641,30 @@ __device__ __forceinline__ void big_gemm_body(const BigParams& P) {
 }
 
 // ---------------------------------------------------------------------------
-// The same sums for launches of a few workgroups per CU (bf16 weights: and for those of 128 x 256 that stand one to a CU):
+// The same sums on bf16 weights, for launches of a few workgroups per CU and those of 128 x 256 that stand one to a CU:
 // W waves side by side, each with a wave tile of MT*16 rows x 32 channels, K steps of 128, PD steps in flight.
-// What bounds such a launch is what a step of one workgroup takes with nothing beside it: the LDS (128 B/clk out, about half
-// of that in), the expansion of the codes and the latency of the step's loads.  So the weights of a wave are its own: they
-// go straight to its registers, expanded once per workgroup (a 2 x 2 grid of 32 x 64 wave tiles expanded each twice and took
-// codes and scales through the LDS), only the activations go through LDS, and everything is requested PD - 1 steps ahead.
+// What bounds such a launch is what a step of one workgroup takes with nothing beside it: its intake and the latency of the
+// step's loads.  So the weights of a wave are its own: they go straight to its registers, only the activations go through LDS,
+// and everything is requested PD - 1 steps ahead.
 // All loads are buffer loads: scalar addresses, and the compiler counts them exactly beside the loads into LDS (flat-
 // addressed loads into LDS make it wait for everything).  Loads of the two kinds complete in issue order, so a step waits
-// until at most those of the PD - 2 younger steps are left; one barrier per step.  Scale bytes at any address.
-// Measured at 333 rows, MXFP4: 4096 x 4096 with residual 20.9 -> 17.8 us, 4096 x 11008 48.9 -> 41.6, 12288 x 4096
-// 46 -> 37, pair 2 x 11008 x 4096 73.5 -> 61 (three workgroups to a CU with PD = 3: 61.1, two with PD = 4: 64.8).  bf16
-// weights: 25.4 -> 19.3, 76.9 -> 58.2; 64 x 256 at 1000 rows 4096 x 11008 152 -> 103; 128 x 256 at 2048 rows 167 -> 144.
+// until at most those of the PD - 2 younger steps are left; one barrier per step.
+// Measured at 333 rows: 4096 x 4096 with residual 25.4 -> 19.3 us, 4096 x 11008 76.9 -> 58.2; 64 x 256 at 1000 rows 4096 x 11008
+// 152 -> 103; 128 x 256 at 2048 rows 167 -> 144.
 // ---------------------------------------------------------------------------
-template <int MT, int W, int PD, bool WBF16>
+template <int MT, int W, int PD>
 struct SideGeom {
   static constexpr int WGM = MT * 16, STAGE = WGM * 256;
   static constexpr int NA = MT * 4 / W;             // 4-row pieces of A a wave fetches per step
-  static constexpr int LB = WBF16 ? 8 : 4;          // weight (and scale) loads of a wave per step
+  static constexpr int LB = 8;                      // weight loads of a wave per step
   static constexpr int L = NA + LB;
   static constexpr size_t EP = (size_t)W * (MT < 4 ? MT * 16 : 64) * ep_ld(2) * sizeof(float);
   static constexpr size_t LDS = (size_t)PD * STAGE > EP ? (size_t)PD * STAGE : EP;
 };
 
-template <int MT, int W, int PD, bool DUAL, bool WBF16, bool SPLIT = false>
+template <int MT, int W, int PD, bool DUAL, bool SPLIT = false>
 __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
-  using G = SideGeom<MT, W, PD, WBF16>;
+  using G = SideGeom<MT, W, PD>;
   constexpr int WGM = G::WGM, STAGE = G::STAGE, NA = G::NA, LB = G::LB, L = G::L;
   extern __shared__ __align__(16) uint8_t tl_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -902,36 +693,23 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
 #pragma unroll
   for (int i = 0; i < NA; i++) {
     const int blk = wave * NA + i, r16 = (blk & 3) * 4 + (lane >> 4);
-    aoff[i] = (uint32_t)min(m_wg + blk * 4 + (lane >> 4), p.M - 1) * (uint32_t)p.K * 2u + (uint32_t)(((lane & 15) ^ r16) & 15) * 16u + (uint32_t)k0 * 256u;
+    aoff[i] = (uint32_t)min(m_wg + blk * 4 + (lane >> 4), p.M - 1) * (uint32_t)p.K * 2u + (uint32_t)((lane & 15) ^ swz16(r16)) * 16u + (uint32_t)k0 * 256u;
   }
-  __amdgpu_buffer_rsrc_t wr[2], swr[2];
-  uint32_t woff[2], swoff[2];
+  __amdgpu_buffer_rsrc_t wr[2];
+  uint32_t woff[2];
 #pragma unroll
   for (int nt = 0; nt < 2; nt++) {
     const int tile = min(DUAL ? tile_base : tile_base + nt, p.tiles - 1);
     wr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].qw : p.qw);
-    swoff[nt] = ((uint32_t)tile * (uint32_t)KA + (uint32_t)k0) * 64u + (uint32_t)lane;
-    if constexpr (WBF16) {
-      woff[nt] = (((uint32_t)tile * (uint32_t)KA + (uint32_t)k0) * 256u + (uint32_t)lane) * 16u;
-    } else {
-      woff[nt] = swoff[nt] * 16u;
-      swr[nt] = tl_rsrc(DUAL && nt ? P.seg[1].sw : p.sw);
-    }
+    woff[nt] = (((uint32_t)tile * (uint32_t)KA + (uint32_t)k0) * 256u + (uint32_t)lane) * 16u;
   }
-  constexpr int BJ = WBF16 ? 4 : 1;
-  i32x4 bw[PD][BJ][2]; // raw weights of PD steps: packed codes, or the operands of the four MFMA steps
-  uint32_t sc[PD][2];
+  i32x4 bw[PD][4][2]; // weights of PD steps: the operands of the four MFMA steps
   // load i of step s (clamped to the last one: what is read past it is never used)
   auto load = [&](auto I, int s, auto SET) {
     constexpr int i = decltype(I)::value, set = decltype(SET)::value;
     s = min(s, last);
     if constexpr (i < LB) {
-      if constexpr (WBF16)
-        bw[set][i >> 1][i & 1] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[i & 1], woff[i & 1] + (i >> 1) * 1024, s * 4096, 0));
-      else if constexpr (i < 2)
-        bw[set][0][i] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[i], woff[i], s * 1024, 0));
-      else
-        sc[set][i - 2] = __builtin_amdgcn_raw_buffer_load_b8(swr[i - 2], swoff[i - 2], s * 64, 0);
+      bw[set][i >> 1][i & 1] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[i & 1], woff[i & 1] + (i >> 1) * 1024, s * 4096, 0));
     } else {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(tl_lds + set * STAGE + (wave * NA + i - LB) * 1024), 16,
                                                aoff[i - LB], s * 256, 0, 0);
@@ -942,7 +720,7 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
     const int m = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int j = 0; j < 4; j++)
-      rdb[j] = (uint32_t)((m >> 2) * 1024 + (m & 3) * 256 + (((g * 4 + j) ^ m) & 15) * 16);
+      rdb[j] = (uint32_t)((m >> 2) * 1024 + (m & 3) * 256 + ((g * 4 + j) ^ swz16(m)) * 16);
   }
   f32x4 acc[MT][2];
 #pragma unroll
@@ -952,7 +730,7 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
     static_for<0, L>([&](auto I) { load(I, decltype(S)::value, S); });
     __builtin_amdgcn_sched_barrier(0); // (in this order: the waits count the loads behind those they wait for)
   });
-  // Units of MU row tiles and one MFMA step j; the operands of unit q are read (and its weights expanded) under the MFMAs
+  // Units of MU row tiles and one MFMA step j; the operands of unit q are read under the MFMAs
   // of unit q - 1, so the last unit of a step runs in the next one, under its first operand reads.
   constexpr int MU = 4, UJ = MT / MU, NQ = 4 * UJ;
   bf16x8 a[2][MU], b[2][2];
@@ -978,7 +756,6 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
     __builtin_amdgcn_s_waitcnt((vm & 15) | 7 << 4 | vm >> 4 << 14); // step s has landed, the reads of step s - 1 have returned
     asm volatile("s_barrier" : : : "memory");
     const uint8_t* ab = tl_lds + set * STAGE;
-    float scale[2];
     static_for<0, NQ>([&](auto Q) {
       constexpr int q = decltype(Q)::value, j = q / UJ, mu = q % UJ;
 #pragma unroll
@@ -987,22 +764,9 @@ __device__ __forceinline__ void side_gemm_body(const BigParams& P) {
       __builtin_amdgcn_sched_barrier(0);
       unit(std::integral_constant<int, (q + NQ - 1) % NQ>{});
       if constexpr (mu == 0) {
-        if constexpr (q == 0 && !WBF16) {
-          scale[0] = e8m0_to_f32(sc[set][0]);
-          scale[1] = e8m0_to_f32(sc[set][1]);
-        }
 #pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-          if constexpr (WBF16)
-            b[j & 1][nt] = __builtin_bit_cast(bf16x8, bw[set][j][nt]);
-          else
-            b[j & 1][nt] = tl_cvt_fp4x8((uint32_t)bw[set][0][nt][j], scale[nt]);
-        }
-        if constexpr (!WBF16)
-          static_for<0, MU * 2>([&](auto) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
-          });
+        for (int nt = 0; nt < 2; nt++)
+          b[j & 1][nt] = __builtin_bit_cast(bf16x8, bw[set][j][nt]);
       }
       __builtin_amdgcn_sched_barrier(0);
       // the loads PD - 1 steps ahead, a few behind each unit (in one burst, a wave stands at its load instructions while
@@ -1078,222 +842,25 @@ template <int MT, bool DUAL, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64, 2)
 big_bf16_kernel(const BigParams P) {
   if constexpr (MT <= 4)
-    side_gemm_body<MT * WM, WM * WN, SIDE_PD, DUAL, true>(P);
+    side_gemm_body<MT * WM, WM * WN, SIDE_PD, DUAL>(P);
   else
     big_gemm_body<MT, DUAL, WM, WN, true>(P);
 }
 
-// 64 x 128 with K in P.S slices (grid y): launches of few workgroups and a long K.  A workgroup's time is its K steps (0.45 us
-// each, MXFP4) whatever else the chip does, so 64 .. 192 of them with 86 steps leave most of it idle; three resident to a CU
+// 64 x 128 with K in P.S slices (grid y), bf16 weights: launches of few workgroups and a long K.  A workgroup's time is its K
+// steps whatever else the chip does, so 64 .. 192 of them with 86 steps leave most of it idle; several resident to a CU
 // run S times as many with an S-th of the steps.  The sums go out as they lie in the registers, 32 KiB a workgroup, and a
-// second launch adds them: with it 4096 x 11008 at 100 / 200 / 300 rows 32.9 -> 20.8 / 40.5 -> 29.1 / 40.9 -> 34.9 us, 2560 x
-// 10240 at 200 rows 35.6 -> 21.7; bf16 weights 56.9 -> 32.3, 61.2 -> 40.7, 66.4 -> 53.4 and 55.3 -> 28.5 (weights from memory).
-template <bool WBF16>
+// second launch adds them: with it 4096 x 11008 at 100 / 200 / 300 rows 56.9 -> 32.3, 61.2 -> 40.7, 66.4 -> 53.4 us, 2560 x 10240 at
+// 200 rows 55.3 -> 28.5 (weights from memory).
 __global__ void __launch_bounds__(256, 2)
 side_split_kernel(const BigParams P) {
-  side_gemm_body<4, 4, SIDE_PD, false, WBF16, true>(P);
+  side_gemm_body<4, 4, SIDE_PD, false, true>(P);
 }
 
-// ---------------------------------------------------------------------------
-// MXFP4 launches whose workgroups are at most one or two to a CU: the same tiles, operand layout and order of sums as
-// big_gemm_body (the same bits), but BOTH operands and the scale bytes go from global memory straight into LDS, NB - 1
-// K steps ahead in a ring of NB stages.  With one workgroup per CU nothing else covers the latency of a step's loads:
-// requested one step ahead (weights half a step, into registers) they stood in the way: 128 x 128, 3584 x 18944 at 800
-// rows 150 -> 131 us; 128 x 256 55 -> 52.  (64 x 128 workgroups went on to waves side by side, side_gemm_body.)  Six
-// stages measured as three.  All loads of the loop being of one kind they complete in issue order, so the
-// wait at the top of a step leaves the younger stages in flight; one barrier per step.
-// Stage: A [WM*MT row tiles][4096 B], swizzled as in big_gemm_body | B [4*WN native tiles][1 KiB] | scales [4*WN][64 B].
-// ---------------------------------------------------------------------------
-template <int MT, int WM, int WN, int NB>
-struct RingGeom {
-  static constexpr int A_BYTES = WM * MT * 4096;
-  static constexpr int B_OFF = A_BYTES;
-  static constexpr int S_OFF = B_OFF + WN * 4096;
-  static constexpr int STAGE = S_OFF + WN * 256;
-  static constexpr int NBLK = MT * 4 / WN; // blocks of 4 rows x 256 B a wave fetches per step
-  static constexpr int NBT = 4 / WM;       // weight tiles a wave fetches per step
-  static constexpr int LPS = NBLK + NBT + 1;
-  static constexpr size_t EP = (size_t)WM * WN * (MT < 4 ? MT * 16 : 64) * EP_LD * sizeof(float); // epilogue staging
-  static constexpr size_t LDS = (size_t)NB * STAGE > EP ? (size_t)NB * STAGE : EP;
-  static_assert(NBLK % 4 == 0, "the swizzle takes a wave's first block to be a multiple of 4");
-};
-
-template <int MT, bool DUAL, int WM, int WN, int NB>
-__device__ __forceinline__ void ring_gemm_body(const BigParams& P) {
-  using G = RingGeom<MT, WM, WN, NB>;
-  constexpr int WGM = MT * 16 * WM, NBLK = G::NBLK, NBT = G::NBT, LPS = G::LPS, STAGE = G::STAGE;
-  extern __shared__ __align__(16) uint8_t tl_lds[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % WM, wn = wave / WM;
-  const int MB = (P.seg[0].M + WGM - 1) / WGM;
-  int bm, bn;
-  tile_of_block(MB, P.nb0[P.n_seg], bm, bn, P.xm);
-  TiledParams p = P.seg[0];
-  int nb_first = 0;
-  if (!DUAL) {
-#pragma unroll
-    for (int i = 1; i < TPPX_MAX_SEGS; i++)
-      if (i < P.n_seg && bn >= P.nb0[i]) {
-        p = P.seg[i];
-        nb_first = P.nb0[i];
-      }
-  }
-  bn -= nb_first;
-  const int KT = p.K >> 7;
-  const int m_wg = bm * WGM;
-  const int tile_base = DUAL ? bn * (WN * 2) + wn * 2 : bn * (WN * 4) + wn * 4;
-  // weight tile behind slot t (0 .. 4*WN-1) of a stage; DUAL: slots 2, 3 of a wave column are the up projection's
-  auto slot_tile = [&](int t) { return min(DUAL ? bn * (WN * 2) + (t >> 2) * 2 + (t & 1) : bn * (WN * 4) + t, p.tiles - 1); };
-
-  // this wave's share of a stage: uniform bases that move with the step + 32-bit offsets per lane (operands < 4 GiB)
-  const char* xbase = reinterpret_cast<const char*>(p.x);
-  uint32_t aoff[NBLK];
-#pragma unroll
-  for (int i = 0; i < NBLK; i++) {
-    const int rin = lane >> 4, ch = lane & 15;
-    const int row = min(m_wg + (wave * NBLK + i) * 4 + rin, p.M - 1); // past the end: re-read the last row (never stored)
-    aoff[i] = (uint32_t)row * (uint32_t)p.K * 2u + (uint32_t)((ch ^ ((i & 3) * 4 + rin)) & 15) * 16u;
-  }
-  const char* bbase[NBT];
-  uint32_t boff[NBT];
-#pragma unroll
-  for (int i = 0; i < NBT; i++) {
-    const int t = wave * NBT + i;
-    bbase[i] = reinterpret_cast<const char*>(DUAL && (t & 2) ? P.seg[1].qw : p.qw);
-    boff[i] = ((uint32_t)slot_tile(t) * (uint32_t)KT * 64u + (uint32_t)lane) * 16u;
-  }
-  const int sp = wave % WN; // scales of slots 4*sp .. 4*sp+3; the waves of a row fetch the same ones, so that every
-                            // wave issues LPS loads per stage
-  const int st = sp * 4 + (lane >> 4);
-  const char* ssrc = reinterpret_cast<const char*>(DUAL && (st & 2) ? P.seg[1].sw : p.sw) +
-                     (size_t)slot_tile(st) * KT * 64 + (size_t)(lane & 15) * 4;
-  auto dma_one = [&](auto I, int ks, int buf) {
-    constexpr int i = decltype(I)::value;
-    uint8_t* base = tl_lds + buf * STAGE;
-    if constexpr (i < NBLK)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xbase + (size_t)ks * 256 + (size_t)aoff[i]),
-                                       (__attribute__((address_space(3))) void*)(base + (wave * NBLK + i) * 1024), 16, 0, 0);
-    else if constexpr (i < NBLK + NBT)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(bbase[i - NBLK] + (size_t)ks * 1024 + (size_t)boff[i - NBLK]),
-                                       (__attribute__((address_space(3))) void*)(base + G::B_OFF + (wave * NBT + i - NBLK) * 1024), 16, 0, 0);
-    else
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(ssrc + (size_t)ks * 64),
-                                       (__attribute__((address_space(3))) void*)(base + G::S_OFF + sp * 256), 4, 0, 0);
-  };
-
-  uint32_t rdb[4]; // byte offset of this lane's activation operand of step j in a row tile
-  {
-    const int m = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      rdb[j] = (uint32_t)((m >> 2) * 1024 + (m & 3) * 256 + (((g * 4 + j) ^ m) & 15) * 16);
-  }
-  f32x4 acc[MT][4];
-#pragma unroll
-  for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++)
-      acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-#pragma unroll
-  for (int s = 0; s < NB - 1; s++)
-    if (s < KT)
-      static_for<0, LPS>([&](auto I) { dma_one(I, s, s); });
-  // Operands of two MFMA steps j: those of (ks, j) are read and expanded under the MFMAs of the step before, so the
-  // MFMAs of (ks, 3) are issued in the next K step, under its first operand reads.  (The set of (-1, 3) is zeros.)
-  bf16x8 a[2][MT], b[2][4];
-#pragma unroll
-  for (int mt = 0; mt < MT; mt++)
-    a[1][mt] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int nt = 0; nt < 4; nt++)
-    b[1][nt] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-  auto mfmas = [&](int set) {
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++)
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[set][mt], b[set][nt], acc[mt][nt], 0, 0, 0);
-  };
-  int buf = 0;
-  auto step = [&](auto MORE, int ks) {
-    constexpr bool more = decltype(MORE)::value;
-    // stage ks has landed for this wave (in the main loop the NB - 2 younger ones may still be in flight; the last
-    // NB - 1 steps wait for all that is left) and its reads of stage ks - 1 have returned ...
-    // (the builtin, so that the compiler knows the operands of (ks - 1, 3) to be there)
-    constexpr int vm = more ? LPS * (NB - 2) : 0;
-    asm volatile("" : : : "memory");
-    __builtin_amdgcn_s_waitcnt((vm & 15) | 7 << 4 | vm >> 4 << 14); // vmcnt(vm) lgkmcnt(0), expcnt open
-    // ... and for every wave: the stage of step ks - 1 is free for the next loads
-    asm volatile("s_barrier" : : : "memory");
-    const int nbuf = buf == 0 ? NB - 1 : buf - 1;
-    const uint8_t* base = tl_lds + buf * STAGE;
-    const uint8_t* ab = base + wm * MT * 4096;
-    i32x4 bw[4];
-    uint32_t sc[4];
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      bw[nt] = *reinterpret_cast<const i32x4*>(base + G::B_OFF + (wn * 4 + nt) * 1024 + lane * 16);
-      sc[nt] = base[G::S_OFF + (wn * 4 + nt) * 64 + lane];
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-      a[0][mt] = *reinterpret_cast<const bf16x8*>(ab + mt * 4096 + rdb[0]);
-    __builtin_amdgcn_sched_barrier(0);
-    mfmas(1);
-    __builtin_amdgcn_sched_barrier(0);
-    static_for<0, 4>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      // the next stage's loads a few at a time (issued in one burst, a wave stands at its load instructions while the
-      // memory pipeline's queue drains)
-      if constexpr (more)
-        static_for<j * LPS / 4, (j + 1) * LPS / 4>([&](auto I) { dma_one(I, ks + NB - 1, nbuf); });
-      if constexpr (j > 0) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-          a[j & 1][mt] = *reinterpret_cast<const bf16x8*>(ab + mt * 4096 + rdb[j]);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas((j - 1) & 1);
-      }
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++)
-        b[j & 1][nt] = tl_cvt_fp4x8((uint32_t)bw[nt][j], e8m0_to_f32(sc[nt]));
-      if constexpr (j > 0)
-        static_for<0, MT * 4>([&](auto) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);          // an MFMA
-          __builtin_amdgcn_sched_group_barrier(0x002, 16 / (MT * 4) > 0 ? 16 / (MT * 4) : 1, 0); // its share of the 16 expansions
-        });
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    buf = buf == NB - 1 ? 0 : buf + 1;
-  };
-  int ks = 0;
-  for (; ks + NB - 1 < KT; ks++)
-    step(std::true_type{}, ks);
-  for (; ks < KT; ks++)
-    step(std::false_type{}, ks);
-  mfmas(1);
-  __syncthreads(); // the ring is free for the epilogue staging
-  float* stage = reinterpret_cast<float*>(tl_lds) + wave * (MT < 4 ? MT * 16 : 64) * EP_LD;
-  if (DUAL)
-    big_epilogue_dual<MT>(p, P.seg[1], acc, stage, m_wg + wm * (MT * 16), tile_base);
-  else
-    big_epilogue<MT>(p, acc, stage, m_wg + wm * (MT * 16), tile_base);
-}
-
-constexpr int RING_STAGES = 3;
-// MT = 2: 64 x 128, waves side by side (named, as in big_bf16_kernel, by the workgroup tile MT*16*WM rows x WN*64 channels and
-// the threads; its waves do not stand 2 x 2); MT = 4: the ring; MT = 8: the large tiles
 template <int MT, bool DUAL, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
 big_mxfp4_kernel(const BigParams P) {
-  if constexpr (MT == 2)
-    side_gemm_body<MT * WM, WM * WN, SIDE_PD, DUAL, false>(P);
-  else if constexpr (MT == 4)
-    ring_gemm_body<MT, DUAL, WM, WN, RING_STAGES>(P);
-  else
-    big_gemm_body<MT, DUAL, WM, WN, false>(P);
+  big_gemm_body<MT, DUAL, WM, WN, false>(P);
 }
 
 // ---------------------------------------------------------------------------
@@ -1758,51 +1325,78 @@ big_fp8_kernel(const BigParams P) {
 
 // Workgroup tiles of the MXFP4 and bf16 launches:
 //   256 x 256, 128 x 512  eight waves, one workgroup per CU; for launches that fill the chip several times over
-//   128 x 256             up to 256 of them one per CU (MXFP4: the ring kernel, bf16: waves side by side), beyond that four
-//                         waves and two per CU
-//   128 x 128             MXFP4 only: ring kernel, one per CU
-//   64 x 128              waves side by side; three (MXFP4) or two (bf16) per CU
-//   64 x 256              bf16 only: eight waves side by side
-enum { TILE_256_256 = 0, TILE_128_256, TILE_128_512, TILE_64_128, TILE_128_128, TILE_64_256, N_TILES };
-static constexpr int TILE_ROWS[N_TILES] = {256, 128, 128, 64, 128, 64};
-static constexpr int TILE_COLS16[N_TILES] = {16, 16, 32, 8, 8, 16}; // 16-channel weight tiles (the pair: gate + up)
+//   128 x 256             four waves and two per CU; bf16 weights: up to 256 of them eight waves side by side, one per CU
+//   64 x 128, 64 x 256    bf16 only: waves side by side
+//   the rest              WIDE_FORMS: launches of up to a few workgroups per CU
+enum { TILE_256_256 = 0, TILE_128_256, TILE_128_512, TILE_64_128, TILE_64_256, TILE_WIDE, N_TILES = TILE_WIDE + N_WIDE };
+static constexpr int tile_rows(int tile) {
+  constexpr int rows[TILE_WIDE] = {256, 128, 128, 64, 64};
+  return tile < TILE_WIDE ? rows[tile] : WIDE_FORMS[tile - TILE_WIDE].mt * 16;
+}
+static constexpr int tile_cols16(int tile) { // 16-channel weight tiles (the pair: gate + up)
+  constexpr int cols[TILE_WIDE] = {16, 16, 32, 8, 16};
+  return tile < TILE_WIDE ? cols[tile] : WIDE_FORMS[tile - TILE_WIDE].nt * WIDE_FORMS[tile - TILE_WIDE].w;
+}
 
-// What a launch takes, in us, with r = its rounds of 256 workgroups, f = the filled part of the last one and s = K / 128:
-//   one round     a + (b + c f) s
-//   more          p + q r + (u + v r + w f + z r s / 1000) s     (z: the clock falls under the power limit as a launch
-//                                                                 grows; measured up to 28672 x 8192 pairs of 2048 rows)
-// bf16 weights: and g (one round) or h us for each MB of them, and e us per round for the epilogue of a gate/up pair.
-// MXFP4: fitted to 2736 launches of 65 .. 2048 rows, linears and pairs of 1024 .. 28672 x 1024 .. 18944, every tile forced; on
-// 792 others (random channels and K) the tile chosen was 0.4 % off the fastest on average, 11 % in the worst hundredth.
-// bf16: fitted to 4100 launches, q/k/v groups among them, up to pairs of 28672 x 8192, most of all where the tile is within 20 %
-// of the fastest, and with weights that come from memory: 96 of them, or as many as fill 2 GB, in turn.  (With four in turn most
-// lie in the Infinity Cache, as they never do in a model, and the estimates came out 20 .. 30 % low.)  On 2600 others the family
-// and tile chosen are 0.3 % off the fastest on average and 9 % in the worst hundredth (1.7 % and 25 % before).
+// What a launch takes, in us, with r = its rounds of 256 workgroups, f = the filled part of the last one, s = K / 128 and w = the
+// weights as MB of bf16:
+//   one round     a + (b + c f) s + g w
+//   more          p + q r + (u + v r + w f + z r s / 1000) s + h w     (z: the clock falls under the power limit as a launch grows)
+//   K in slices   that for S times the workgroups and an S-th of the steps, and c0 + c1 us for each 32 KiB of the slices' sums
+// and e us per round for the epilogue of a gate/up pair.  (Rounds also where several workgroups share a CU: three of one round's
+// take about three times as long together.)
+// MXFP4: fitted to 888 of 1184 shapes of 65 .. 2048 rows, 768 .. 37888 channels and K = 1024 .. 18944 with every tile forced, whole
+// and in slices, weights in turn from 320 MB; on the others the tile and slices taken are 0.8 % off the fastest on average, 11 % in
+// the worst hundredth.  Larger launches (28672 x 8192 pairs) are extrapolated and stay with the large tiles.
+// bf16: the large tiles, 64 x 128 and 64 x 256 fitted to 4100 launches, q/k/v groups among them, up to pairs of 28672 x 8192, most of
+// all where the tile is within 20 % of the fastest, and with weights that come from memory: 96 of them, or as many as fill 2 GB, in
+// turn.  (With four in turn most lie in the Infinity Cache, as they never do in a model, and the estimates came out 20 .. 30 %
+// low.)  96 rows: fitted to 2956 more, times 0.96, which those take on the same shapes.
 struct TileCost {
-  double a, b, c, p, q, u, v, w, z, g, h, e;
+  double a, b, c, p, q, u, v, w, z, g, h, e, c0, c1;
 };
 static constexpr TileCost MXFP4_COST[N_TILES] = {
-    {7.75, 1.88, 0.607, -6.18, 12.4, -0.498, 2.31, 0.768, 0.256, 0, 0},
-    {6.07, 1.09, 0.302, 4.03, 3.96, -0.337, 1.18, 0.442, 0.0994, 0, 0},
-    {7.71, 1.85, 0.573, -8.21, 13, -0.546, 2.27, 0.864, 0.281, 0, 0},
-    {4.02, 0.385, 0.091, 3.36, 1.09, -0.0981, 0.352, 0.145, 0.029, 0, 0},
-    {4.88, 0.75, 0.146, 0.348, 3.97, -0.157, 0.871, 0.18, 0.00761, 0, 0},
-    {},
+    {9.24, 1.85, 0.843, 2.85, 7.11, -1.18, 2.6, 1.32, 0.182, 0.0166, 0.0562, 0}, // 256 x 256
+    {8.13, 1.15, 0.429, 2.31, 4.18, -0.632, 1.35, 0.85, 0, 0.0177, 0.00405, 0}, // 128 x 256
+    {8.78, 1.83, 0.835, 1.79, 7.7, -1.27, 2.56, 1.42, 0, 0.0236, 0.0681, 0}, // 128 x 512
+    {}, // 64 x 128
+    {}, // 64 x 256
+    {3.52, 0.203, 0.105, 3.27, 0.706, -0.0854, 0.243, 0.162, 0, 0.0109, 0.00497, 0, 2.91, 0.00848}, // 32 x 128
+    {3.98, 0.254, 0.119, 3.01, 1.43, -0.0935, 0.289, 0.192, 0.037, 0.00615, 0.00283, 0, 3.05, 0.00707}, // 48 x 128
+    {4.38, 0.277, 0.165, 2.79, 1.93, -0.191, 0.391, 0.21, 0.0643, 0.0034, 0, 0, 3.34, 0.00632}, // 64 x 128
+    {4.33, 0.346, 0.196, 1.27, 2.63, -0.243, 0.472, 0.328, 0.0483, 0.0033, 0, 0}, // 80 x 128
+    {}, // 96 x 128
+    {5.36, 0.375, 0.235, 4.15, 2.87, -0.371, 0.647, 0.332, 0.00103, 0.00239, 0, 0}, // 64 x 192
+    {5.54, 0.454, 0.247, 3.08, 3.4, -0.416, 0.758, 0.414, 0, 0.00417, 0, 0}, // 80 x 192
+    {6.04, 0.498, 0.396, 2.68, 3.55, -0.583, 0.967, 0.565, 0, 0.00161, 0, 0}, // 80 x 256
+    {6.4, 0.597, 0.463, 1.86, 4.66, -0.617, 1.08, 0.664, 0.0657, 0, 0, 0}, // 96 x 256
+    {7.41, 0.585, 0.473, 2.65, 4.99, -0.639, 1.11, 0.671, 0, 0, 0, 0}, // 64 x 384
+    {8.25, 0.935, 0.577, 1.79, 6.14, -0.789, 1.54, 0.962, 0, 0.00469, 0.00688, 0}, // 96 x 384
 };
 static constexpr TileCost BF16_COST[N_TILES] = {
-    {9.19, 1.73, 0.784, 2.54, 6.07, -1.52, 2.92, 1.23, 0.155, 0.0249, 0.00722, 3.73},
-    {7.3, 1.13, 0.298, 2.01, 3.53, -0.41, 1.25, 0.708, 0.288, 0.043, 0.0481, 1.07},
-    {8.86, 1.81, 0.692, -1.47, 7.78, -1.4, 2.81, 1.4, 0.195, 0.0518, 0.0267, 3.63},
-    {3.7, 0.613, 0.0187, 2.24, 0.731, 0.0345, 0.498, 0.186, 0.041, 0.0584, 0.069, 0.555},
-    {},
-    {4.61, 1.02, 0.051, 1.68, 3.15, -0.354, 0.929, 0.634, 0.195, 0.0614, 0.0625, 1.05},
+    {9.19, 1.73, 0.784, 2.54, 6.07, -1.52, 2.92, 1.23, 0.155, 0.0249, 0.00722, 3.73}, // 256 x 256
+    {7.3, 1.13, 0.298, 2.01, 3.53, -0.41, 1.25, 0.708, 0.288, 0.043, 0.0481, 1.07}, // 128 x 256
+    {8.86, 1.81, 0.692, -1.47, 7.78, -1.4, 2.81, 1.4, 0.195, 0.0518, 0.0267, 3.63}, // 128 x 512
+    {3.7, 0.613, 0.0187, 2.24, 0.731, 0.0345, 0.498, 0.186, 0.041, 0.0584, 0.069, 0.555, 2.2, 0.0115}, // 64 x 128
+    {4.61, 1.02, 0.051, 1.68, 3.15, -0.354, 0.929, 0.634, 0.195, 0.0614, 0.0625, 1.05}, // 64 x 256
+    {}, // 32 x 128
+    {}, // 48 x 128
+    {}, // 64 x 128
+    {}, // 80 x 128
+    {4.65, 0.631, 0.124, 3.46, 1.99, -0.287, 0.669, 0.398, 0.135, 0.0652, 0.0644, 0.6}, // 96 x 128
+    {}, // 64 x 192
+    {}, // 80 x 192
+    {}, // 80 x 256
+    {6.57, 1.09, 0.123, 0.575, 6.07, -0.269, 1.08, 0.729, 0.271, 0.0695, 0.0719, 0.6}, // 96 x 256
+    {}, // 64 x 384
+    {}, // 96 x 384
 };
 static double tile_us(const TileCost& k, int tile, int64_t wgs, double s, double weight_mb, bool dual) {
   const double r = (double)((wgs + 255) / 256), f = (double)wgs / 256.0 - (r - 1.0);
   if (r <= 1.0)
     return k.a + (k.b + k.c * f) * s + k.g * weight_mb + (dual ? k.e : 0.0);
   // (the z term at most as far as it was measured: 448 rounds x steps of 256 x 256, the same work in the other tiles)
-  const double rs = std::min(r * s, 448.0 * 4096.0 / (TILE_ROWS[tile] * TILE_COLS16[tile]));
+  const double rs = std::min(r * s, 448.0 * 4096.0 / (tile_rows(tile) * tile_cols16(tile)));
   return k.p + k.q * r + (k.u + k.v * r + k.w * f + k.z * 1e-3 * rs * r) * s + k.h * weight_mb + (dual ? k.e * r : 0.0);
 }
 
@@ -1823,55 +1417,68 @@ static int xcd_split(int64_t mb, int64_t nb, double a_bytes, double w_bytes) {
 }
 
 constexpr double MXFP4_WEIGHT_BYTES = 0.53;
-static double mxfp4_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb, bool dual) {
-  const int64_t mb = (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile];
-  const double us = tile_us(MXFP4_COST[tile], tile, mb * nb, s, weight_mb, dual);
-  // Without a split along M an XCD walks whole columns, and the columns of the workgroups that are resident together drift apart
-  // in K, the more so the more row blocks there are and the longer K is: 24 row blocks cost 10 % (K = 4096) .. 21 % (K = 16384),
-  // 29 25 .. 33 %, 32 31 .. 37 %, K up to 2048 half of that and less.  With rectangles (an even number of row blocks and channel
-  // blocks to go with it) 32 row blocks are as fast as the estimate, and launches of up to 768 workgroups, three to a CU and so
-  // all of them resident, lose 5 .. 10 % less.  2048 x 9088 x 8704 342 us where 128 x 256 takes 250, 4096 x 11008 at 1421 rows
-  // 125 (111).  On 2600 launches of 1025 .. 2048 rows the tile taken is 0.3 % off the fastest on average.
-  if (tile != TILE_64_128 || mb <= 16 || mb * nb <= 256 ||
-      xcd_split(mb, nb, (double)M * 2.0, (double)nb * TILE_COLS16[tile] * 16.0 * MXFP4_WEIGHT_BYTES) != 1)
-    return us;
-  const double drift = std::max(0.0, std::min(0.4, 0.025 * (double)(mb - 21) + 0.0014 * s));
-  return us * (1.0 + drift * std::min(1.0, std::max(0.0, (s - 8.0) / 12.0)) * std::min(1.0, (double)(mb * nb + 256) / 1024.0));
-}
-static double bf16_tile_us(int tile, int64_t M, int64_t nb, double s, double weight_mb, bool dual) {
-  return tile_us(BF16_COST[tile], tile, (M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile] * nb, s, weight_mb, dual);
+// the tiles a launch may take, one bit each
+template <bool WBF16>
+static unsigned big_tiles() {
+  unsigned tiles = 1u << TILE_256_256 | 1u << TILE_128_256 | 1u << TILE_128_512;
+  if (env_int("TPPX_TILED_SMALL", 1) == 0)
+    return tiles;
+  if (WBF16)
+    tiles |= 1u << TILE_64_128 | 1u << TILE_64_256;
+  for (int i = 0; i < N_WIDE; i++)
+    if (WBF16 ? WIDE_FORMS[i].bf16 : WIDE_FORMS[i].mxfp4)
+      tiles |= 1u << (TILE_WIDE + i);
+  return tiles;
 }
 
-// the tiles a launch may take, one bit each.  scales4: scale bytes on a 4-byte address (the ring forms move four at a time)
-static unsigned mxfp4_tiles(bool scales4) {
-  const unsigned large = 1u << TILE_256_256 | 1u << TILE_128_256 | 1u << TILE_128_512;
-  return env_int("TPPX_TILED_SMALL", 1) == 0 ? large : large | 1u << TILE_64_128 | (scales4 ? 1u << TILE_128_128 : 0u);
-}
-static unsigned bf16_tiles() {
-  const unsigned large = 1u << TILE_256_256 | 1u << TILE_128_256 | 1u << TILE_128_512;
-  return env_int("TPPX_TILED_SMALL", 1) == 0 ? large : large | 1u << TILE_64_128 | 1u << TILE_64_256;
-}
+// bytes of the sums of one K slice of a workgroup
+static int64_t slice_bytes(int tile) { return (int64_t)tile_rows(tile) * tile_cols16(tile) * 16 * 4; }
 
-// the cheapest of them for n GEMMs of tiles[i] channel tiles over one activation (dual: the gate/up pair, tiles[0] each)
-template <typename Us>
-static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dual, unsigned allowed, Us&& us, double* best_us = nullptr) {
+// The cheapest tile for n GEMMs of tiles[i] channel tiles over one activation (dual: the gate/up pair, tiles[0] each), *S its K
+// slices (1: whole; only with room for their sums in part_bytes).  Slices have to look 3 % faster (bf16 weights 5 %, in more than
+// a round 10 %): they are a second launch, behind and before other kernels (a GPT-J pass of three layers 699 .. 731 us in slices
+// where whole K looked 4 % slower, whole 677 .. 688), and weights at hand in the Infinity Cache gain them less (bf16 8640 x 4608
+// at 124 rows 32.9 and 32.1 us from memory, 22.4 and 25.8 at hand).  Fewer than 2048 channels are not sliced: the decode kernels
+// run those well (1024 x 4096 at 160 .. 256 rows 9 us, slices 10).
+template <bool WBF16>
+static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dual, int64_t part_bytes, int* S, double* best_us = nullptr) {
+  constexpr const TileCost* COST = WBF16 ? BF16_COST : MXFP4_COST;
+  const unsigned allowed = big_tiles<WBF16>();
+  const int forced = env_int("TPPX_TILED_SPLIT", 1);
   int64_t all = 0;
   for (int i = 0; i < n; i++)
     all += tiles[i];
+  const double s = (double)(K / 128), mb = (double)(all * 32 * K) * 1e-6;
   int shape = 0;
   double best = 1e300;
+  *S = 1;
   for (int i = 0; i < N_TILES; i++) {
-    if (!(allowed >> i & 1u))
+    if (!(allowed >> i & 1u) || (WBF16 && i >= TILE_WIDE && all < 48)) // (fewer than 768 channels: not measured)
       continue;
-    const int tpw = TILE_COLS16[i] / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
+    const int tpw = tile_cols16(i) / (dual ? 2 : 1); // channel tiles of a workgroup (of each projection for the pair)
     int64_t nb = 0;
     for (int g = 0; g < (dual ? 1 : n); g++)
       nb += (tiles[g] + tpw - 1) / tpw;
-    // (a tie goes to the larger tiles, which read less)
-    const double tie = i == TILE_64_256 && shape == TILE_64_128 ? 1.01 : i >= TILE_64_128 ? 0.99 : 1.0;
-    if (const double c = us(i, M, nb, (double)(K / 128), (double)(all * 32 * K) * 1e-6, dual); c < tie * best) {
+    const int64_t wgs = (M + tile_rows(i) - 1) / tile_rows(i) * nb;
+    // (a near tie goes to the large tiles, which read less)
+    double c = tile_us(COST[i], i, wgs, s, mb, dual) * (i >= TILE_64_128 && i != TILE_64_256 ? 1.01 : 1.0);
+    if (c < best && !(forced > 1 && *S > 1)) {
       best = c;
       shape = i;
+      *S = 1;
+    }
+    if (dual || forced == 0 || !(COST[i].c0 > 0.0) || (forced == 1 && (WBF16 ? K <= 2560 || wgs > 320 : all < 128)))
+      continue;
+    for (int z : {2, 3, 4, 6}) {
+      if (wgs * z * slice_bytes(i) > part_bytes || K / 128 < 4 * z || (forced == 1 && wgs * z > 1024)) // (as far as was measured)
+        break;
+      c = tile_us(COST[i], i, wgs * z, s / z, mb, false) + COST[i].c0 + COST[i].c1 * (double)(wgs * z * slice_bytes(i)) / 32768.0;
+      c *= !WBF16 ? 1.03 : wgs <= 256 ? 1.05 : 1.10;
+      if (forced == z ? *S != z || c < best : forced == 1 && c < best) {
+        best = c;
+        shape = i;
+        *S = z;
+      }
     }
   }
   if (best_us)
@@ -1879,75 +1486,19 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
   return shape;
 }
 
-double tiled_mxfp4_us(int64_t M, int64_t K, int64_t n_tiles16) {
+double tiled_mxfp4_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes) {
   const int tiles = (int)n_tiles16;
   double us;
-  cheapest_tile(M, K, &tiles, 1, false, mxfp4_tiles(true), mxfp4_tile_us, &us);
+  int S;
+  cheapest_tile<false>(M, K, &tiles, 1, false, part_bytes, &S, &us);
   return us;
 }
 
-double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16) {
+double tiled_bf16_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes) {
   const int tiles = (int)n_tiles16;
   double us;
-  cheapest_tile(M, K, &tiles, 1, false, bf16_tiles(), bf16_tile_us, &us);
-  return us;
-}
-
-// K slices (1: whole) of a launch of n GEMMs that takes whole_us without them, *us: what it takes then.  The 64 x 128 tile's
-// estimate for S times the workgroups and an S-th of the steps, and the slices' sums out and in: 2.2 us and 8.5 .. 16.5 ns
-// (MXFP4, the more the shorter K is) or 11.5 ns (bf16 weights) for each 32 KiB of them.  Up to K = 2560 (11.5 us whole, 11.3 in
-// slices at 65 rows), MXFP4 4096 (17 whole, 15 .. 22), no launch is split; bf16 up to one round of whole-K workgroups and a
-// quarter more, MXFP4 up to 200 of them: beyond, slices are a little faster by themselves (4096 x 16384 at 420 rows, 224
-// workgroups, 61.9 us, whole 64.4), but behind and before other kernels they are not (the GPT-J pass it is part of, three
-// layers, 699 .. 731 us, whole 677 .. 688; three Qwen2 layers at 420 .. 512 rows within 1.4 %).  Measured on 250 launches of 65 .. 1024 rows of 1024 .. 11000 channels and K = 2816 .. 16384:
-//   MXFP4  the slices' estimate is 3 .. 5 % high, but 2 % low with two slices of more than 160 workgroups or more than 730
-//          workgroups in all, and 1 % lower with each row block from the fifth on (more of them read the same weights).  With
-//          that, 6 % for the estimate's sake: none is slower than whole by more than 2 % (1408 x 9216 at 1024 rows, 34.0 us
-//          whole, 37.8 in slices without it; 4096 x 11008 at 400 rows 41.8 and 45.1), the best forgone is 6 % faster in slices.
-//   bf16   right to 3 % with weights from memory; at hand in the Infinity Cache whole K is up to a quarter faster, slices hardly
-//          (8640 x 4608 at 124 rows 32.9 and 32.1 us from memory, 22.4 and 25.8 at hand), so a near tie goes to whole K: 5 %,
-//          10 % beyond a round.
-template <bool WBF16>
-static int best_split(int64_t M, int64_t K, const int* tiles, int n, int64_t part_bytes, double whole_us, double* us) {
-  const int forced = env_int("TPPX_TILED_SPLIT", 1);
-  int64_t nb = 0, all = 0;
-  for (int i = 0; i < n; i++) {
-    nb += (tiles[i] + 7) / 8;
-    all += tiles[i];
-  }
-  const int64_t wgs = (M + 63) / 64 * nb;
-  const double s = (double)K / 128.0, mb = (double)(all * 32 * K) * 1e-6;
-  const double ns = WBF16 ? 11.5 : 16.5 - 8.0 * std::min(1.0, std::max(0.0, (s - 32.0) / 48.0));
-  const double rows = 0.01 * (double)std::max<int64_t>(0, (M + 63) / 64 - 4);
-  int best = 1;
-  double best_us = (WBF16 ? wgs > 256 ? 0.90 : 0.95 : 0.94) * whole_us;
-  for (int S : {2, 3, 4, 6}) {
-    if (wgs * S * 32768 > part_bytes || K / 128 < 4 * S)
-      break;
-    double c = tile_us((WBF16 ? BF16_COST : MXFP4_COST)[TILE_64_128], TILE_64_128, wgs * S, s / S, mb, false) + 2.2 + ns * 1e-3 * (double)(wgs * S);
-    if (!WBF16)
-      c *= 1.0 + rows + ((S == 2 ? wgs > 160 : wgs * S > 730) ? 0.02 : -0.04);
-    if (forced == S || (forced == 1 && K > (WBF16 ? 2560 : 4096) && wgs <= (WBF16 ? 320 : 200) && c < best_us)) {
-      best_us = c;
-      best = S;
-    }
-  }
-  if (us && best > 1)
-    *us = best_us;
-  return best;
-}
-
-// the same for one GEMM of n_tiles16 channel tiles with room for the slices' sums
-double tiled_mxfp4_split_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes) {
-  const int tiles = (int)n_tiles16;
-  double us = tiled_mxfp4_us(M, K, n_tiles16);
-  best_split<false>(M, K, &tiles, 1, part_bytes, us, &us);
-  return us;
-}
-double tiled_bf16_split_us(int64_t M, int64_t K, int64_t n_tiles16, int64_t part_bytes) {
-  const int tiles = (int)n_tiles16;
-  double us = tiled_bf16_us(M, K, n_tiles16);
-  best_split<true>(M, K, &tiles, 1, part_bytes, us, &us);
+  int S;
+  cheapest_tile<true>(M, K, &tiles, 1, false, part_bytes, &S, &us);
   return us;
 }
 
@@ -1970,12 +1521,8 @@ static hipError_t big_go(Kern kern, const BigParams& P, int wgs, int threads, si
 
 template <int MT, bool DUAL, int WM, int WN>
 static hipError_t big_launch(const BigParams& P, int wgs, hipStream_t stream) {
-  size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float); // epilogue staging per wave; >= the two A buffers
-  static_assert(MT <= 4 || (size_t)WM * WN * 64 * EP_LD * sizeof(float) >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
-  if constexpr (MT == 2)
-    lds = SideGeom<MT * WM, WM * WN, SIDE_PD, false>::LDS;
-  else if constexpr (MT == 4)
-    lds = RingGeom<MT, WM, WN, RING_STAGES>::LDS;
+  constexpr size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float); // epilogue staging per wave; >= the two A buffers
+  static_assert(lds >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
   return big_go(big_mxfp4_kernel<MT, DUAL, WM, WN>, P, wgs, WM * WN * 64, lds, stream);
 }
 
@@ -1984,26 +1531,21 @@ static hipError_t big_bf16_launch(const BigParams& P, int wgs, hipStream_t strea
   size_t lds = (size_t)WM * WN * 64 * EP_LD * sizeof(float);
   static_assert(MT <= 4 || (size_t)WM * WN * 64 * EP_LD * sizeof(float) >= (size_t)2 * MT * 16 * WM * 256, "LDS plan");
   if constexpr (MT <= 4)
-    lds = SideGeom<MT * WM, WM * WN, SIDE_PD, true>::LDS;
+    lds = SideGeom<MT * WM, WM * WN, SIDE_PD>::LDS;
   return big_go(big_bf16_kernel<MT, DUAL, WM, WN>, P, wgs, WM * WN * 64, lds, stream);
 }
 
-// S: K slices of the 64 x 128 tile, 1 where K stays whole
-template <bool WBF16, typename Us>
-static int cheapest_tile(const TiledParams* t, int n, bool dual, unsigned allowed, Us&& us, int64_t part_bytes, int* S) {
+template <bool WBF16>
+static int cheapest_tile(const TiledParams* t, int n, bool dual, int64_t part_bytes, int* S) {
   int tiles[TPPX_MAX_SEGS];
   for (int i = 0; i < n; i++)
     tiles[i] = t[i].tiles;
-  double best;
-  const int shape = cheapest_tile(t[0].M, t[0].K, tiles, n, dual, allowed, us, &best);
-  if (!dual && part_bytes > 0 && (allowed >> TILE_64_128 & 1u))
-    *S = best_split<WBF16>(t[0].M, t[0].K, tiles, n, part_bytes, best, nullptr);
-  return *S > 1 ? TILE_64_128 : shape;
+  return cheapest_tile<WBF16>(t[0].M, t[0].K, tiles, n, dual, part_bytes, S);
 }
 
 // fills P for n GEMMs over one activation with this workgroup tile; returns the workgroups of the launch
 static int big_params(BigParams& P, const TiledParams* t, int n, bool dual, int tile, double bytes_per_weight) {
-  const int tpw = TILE_COLS16[tile] / (dual ? 2 : 1), MB = (t[0].M + TILE_ROWS[tile] - 1) / TILE_ROWS[tile];
+  const int tpw = tile_cols16(tile) / (dual ? 2 : 1), MB = (t[0].M + tile_rows(tile) - 1) / tile_rows(tile);
   memset(&P, 0, sizeof(P));
   int nb = 0;
   for (int i = 0; i < n; i++) {
@@ -2048,33 +1590,44 @@ static hipError_t split_launch(Kern kern, size_t lds, BigParams& P, int wgs, int
                                                                                           : sum(side_sum_kernel<4, 4, 6>);
 }
 
+// TPPX_TILED_BIG_TILE: 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128 and 6 = 64 x 256 (bf16 weights), from 7 on
+// WIDE_FORMS; what is not built for the weights, 5 too, is left to the estimates
+static int forced_tile() {
+  const int t = env_int("TPPX_TILED_BIG_TILE", 0);
+  return t >= 1 && t <= 4 ? t - 1 : t == 6 ? TILE_64_256 : t >= 7 && t < 7 + N_WIDE ? TILE_WIDE + t - 7 : -1;
+}
+
+// K slices of a tile that TPPX_TILED_BIG_TILE forces: TPPX_TILED_SPLIT's, where the kernels are built and their sums have room
+static int forced_slices(bool can, const TiledParams* t, int n, int tile, int64_t part_bytes) {
+  const int S = env_int("TPPX_TILED_SPLIT", 1);
+  int64_t nb = 0;
+  for (int i = 0; i < n; i++)
+    nb += (t[i].tiles + tile_cols16(tile) - 1) / tile_cols16(tile);
+  const int64_t wgs = (t[0].M + tile_rows(tile) - 1) / tile_rows(tile) * nb;
+  return can && (S == 2 || S == 3 || S == 4 || S == 6) && t[0].K / 128 >= 4 * S && wgs * S * slice_bytes(tile) <= part_bytes ? S : 1;
+}
+
 // dual: t[0] = gate, t[1] = up (equal shapes, n == 2); y[m][n] = silu(gate) * up goes to t[1].y
 hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual, float* part, int64_t part_bytes) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
-  bool scales4 = true;
-  for (int i = 0; i < n; i++)
-    scales4 = scales4 && (reinterpret_cast<uintptr_t>(t[i].sw) & 3u) == 0;
-  int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 5 = 128 x 128
-  int S = 1;
-  if (shape < 0 || shape > TILE_128_128 || (shape == TILE_128_128 && !scales4))
-    shape = cheapest_tile<false>(t, n, dual, mxfp4_tiles(scales4), mxfp4_tile_us, part ? part_bytes : 0, &S);
+  int shape = forced_tile(), S = 1;
+  if (shape < 0 || shape >= N_TILES || !(MXFP4_COST[shape].b > 0.0))
+    shape = cheapest_tile<false>(t, n, dual, part ? part_bytes : 0, &S);
+  else if (shape >= TILE_WIDE)
+    S = forced_slices(WIDE_FORMS[shape - TILE_WIDE].split && !dual, t, n, shape, part ? part_bytes : 0);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, MXFP4_WEIGHT_BYTES);
-  if (S > 1)
-    return split_launch(side_split_kernel<false>, SideGeom<4, 4, SIDE_PD, false>::LDS, P, wgs, S, part, stream);
+  if (shape >= TILE_WIDE) {
+    P.S = S;
+    P.part = part;
+    const hipError_t e = launch_wide_mxfp4(P, shape - TILE_WIDE, wgs, dual, stream);
+    return S > 1 && e == hipSuccess ? launch_wide_sum(P, shape - TILE_WIDE, wgs, stream) : e;
+  }
   switch (shape) {
   case TILE_128_512:
     return dual ? big_launch<8, true, 1, 8>(P, wgs, stream) : big_launch<8, false, 1, 8>(P, wgs, stream);
-  case TILE_64_128:
-    return dual ? big_launch<2, true, 2, 2>(P, wgs, stream) : big_launch<2, false, 2, 2>(P, wgs, stream);
-  case TILE_128_128:
-    return dual ? big_launch<4, true, 2, 2>(P, wgs, stream) : big_launch<4, false, 2, 2>(P, wgs, stream);
   case TILE_128_256:
-    // at most one workgroup per CU: eight waves of 64 x 64, two per SIMD, so that one wave's waits are another's issue
-    // slots; else four of 128 x 64, two workgroups per CU
-    if (scales4 && wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0)
-      return dual ? big_launch<4, true, 2, 4>(P, wgs, stream) : big_launch<4, false, 2, 4>(P, wgs, stream);
     return dual ? big_launch<8, true, 1, 4>(P, wgs, stream) : big_launch<8, false, 1, 4>(P, wgs, stream);
   default:
     return dual ? big_launch<8, true, 2, 4>(P, wgs, stream) : big_launch<8, false, 2, 4>(P, wgs, stream);
@@ -2168,14 +1721,15 @@ bool tiled_bf16_takes_groups(const TiledParams& p) {
 hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual, float* part, int64_t part_bytes) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
-  int shape = env_int("TPPX_TILED_BIG_TILE", 0) - 1; // 1 .. 4 as in launch_tiled_mxfp4_group, 6 = 64 x 256; 5 is not built for 2-byte weights
-  int S = 1;
-  if (shape < 0 || shape >= N_TILES || shape == TILE_128_128)
-    shape = cheapest_tile<true>(t, n, dual, bf16_tiles(), bf16_tile_us, part ? part_bytes : 0, &S);
+  int shape = forced_tile(), S = 1;
+  if (shape < 0 || shape >= N_TILES || !(BF16_COST[shape].b > 0.0))
+    shape = cheapest_tile<true>(t, n, dual, part ? part_bytes : 0, &S);
   BigParams P;
   const int wgs = big_params(P, t, n, dual, shape, 2.0);
+  if (shape >= TILE_WIDE)
+    return launch_wide_bf16(P, shape - TILE_WIDE, wgs, dual, stream);
   if (S > 1)
-    return split_launch(side_split_kernel<true>, SideGeom<4, 4, SIDE_PD, true>::LDS, P, wgs, S, part, stream);
+    return split_launch(side_split_kernel, SideGeom<4, 4, SIDE_PD>::LDS, P, wgs, S, part, stream);
   switch (shape) {
   case TILE_128_512:
     return dual ? big_bf16_launch<8, true, 1, 8>(P, wgs, stream) : big_bf16_launch<8, false, 1, 8>(P, wgs, stream);

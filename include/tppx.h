@@ -312,6 +312,16 @@ int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa,
                                float post_scale, int flags,
                                tppx_stream_t stream);
 
+/* The gate/up pair on W4A8 weights as one launch behind the row quantizer (xq / sa and flags as above):
+ * silu(gate) * up with the rounding points, and the bits, of tppx_linear_mxfp4_int8_mid with TPPX_POST_SILU followed by
+ * one with TPPX_POST_MUL. */
+int tppx_swiglu_mxfp4_int8_mid(const void* x, void* xq, void* sa,
+                               const void* q_gate, const void* s_gate,
+                               const void* bias_gate, const void* q_up,
+                               const void* s_up, const void* bias_up, void* y,
+                               int64_t M, int64_t N, int64_t K, int flags,
+                               tppx_stream_t stream);
+
 /* W4A8 with many rows (prompt passes): the same arithmetic on the bf16 MFMA.  An int8 activation and a weight
  * integer times its block's power of two are exact in bf16 and so is the fp32 sum of one MX block's 32 products, so
  * one K = 32 MFMA per block gives float(int32 block sum) * 2^(e - 127) and the fold is one fp32 multiply-add with

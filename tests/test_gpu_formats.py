@@ -668,6 +668,41 @@ def test_w4a8_row_groups_equal_the_oracle_from_64_rows(M, N, K, bc, post):
     assert torch.equal(ops.linear(xg, qt, bg, posts[post], in1, in2, 0.5), want)
 
 
+# row tiles 2 / 3 / 4 of a wave and their edges, then the row-group kernel; K tiles 1, 2, 5, 9 (quarters inside a tile), 4 and 8
+@pytest.mark.parametrize("M,N,K,bc", [(17, 96, 128, 32), (32, 272, 640, 64), (33, 144, 1152, 128), (48, 1040, 1024, 64),
+                                      (49, 272, 256, 64), (63, 4096, 640, 64), (64, 112, 384, 64), (130, 272, 1024, 128)])
+def test_w4a8_pair_has_the_bits_of_two_calls(M, N, K, bc):
+    """silu(gate) * up of W4A8 weights in one launch equals the call of the gate followed by the one of the up projection:
+    ordinary weight scales and ones that the integer sums' float start does not cover, rows with zeros, with and without
+    biases, rows off a 16-byte address (the pair is not taken), and an infinity and a NaN in the rows."""
+    ops = _ops()
+    W = randn_bf16((N, K), 0.05, 3700 + M)
+    W[1, :32] *= 1000
+    W[N - 1, K - 32:] *= 30000
+    W[3, 64:96] = 0.0
+    t = W.view(N // 16, 16, K // bc, bc // 2, 2).permute(0, 2, 3, 1, 4).contiguous()
+    up, gate = ops.remap_and_quantize_mxfp4(t.cuda(), int8_layout=True), _w4a8(N, K, bc, 3710 + M)[0]
+    x = randn_bf16((M, K), 1.0, 3720 + M)
+    x[M - 1, :64] = 0.0
+    bg, bu = randn_bf16((N,), 0.1, 3730).cuda(), randn_bf16((N,), 0.1, 3740).cuda()
+
+    def two(x, bg, bu):
+        return _w4a8_mid(up, x, bu, O.POST_MUL, _w4a8_mid(gate, x, bg, O.POST_SILU, None, None, 1.0), None, 1.0)
+
+    for special in (False, True):
+        if special:
+            x[0, 5], x[M - 1, 40] = float("inf"), float("nan")
+        xg = x.cuda()
+        for a, b in ((bg, bu), (None, None), (bg, None)):
+            y, want = ops._w4a8_pair(xg, gate, up, a, b), two(xg, a, b)
+            assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.nan_to_num(y), torch.nan_to_num(want))
+            assert special or torch.equal(y, want) and not torch.isnan(y).any()
+    x[0, 5], x[M - 1, 40] = 0.5, 0.5
+    off = torch.empty(M * K + 1, dtype=torch.bfloat16, device="cuda")[1:].view(M, K).copy_(x)
+    assert ops._w4a8_pair(off, gate, up, None, None) is None
+    assert torch.equal(ops.swiglu_gate_up(x.cuda(), gate, up), two(x.cuda(), None, None))
+
+
 # workgroups of one channel tile (at most 512 of 64 rows) and of two (33 x 16 of 64 rows; 37 tiles: the last one alone),
 # K tiles: less than a step of four, whole steps, a remainder behind them
 @pytest.mark.parametrize("M,N,K,bc", [(64, 48, 384, 64), (130, 272, 1024, 128), (1024, 528, 640, 32), (960, 592, 1920, 64),

@@ -1105,11 +1105,10 @@ extern "C" int tppx_linear_mxfp4_int8_rows(const void* x, const void* q_nat, con
   return check_hip(launch_skinny_w4a8(p, ntw, (hipStream_t)stream), who);
 }
 
-extern "C" int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa, const void* q_nat, const void* s_nat,
-                                          const void* bias, const void* post_in, const void* post_in2, void* y,
-                                          int64_t M, int64_t N, int64_t K, int post_op, float post_scale, int flags,
-                                          tppx_stream_t stream) {
-  const char* who = "tppx_linear_mxfp4_int8_mid";
+// one W4A8 weight, or the gate/up pair (dual), behind the quantizer of the rows
+static int run_w4a8_mid(const char* who, const void* x, void* xq, void* sa, const tppx_seg* segs, bool dual, int64_t M,
+                        int64_t K, int flags, hipStream_t stream) {
+  const int64_t N = segs[0].N;
   TPPX_REQUIRE(M <= 0 || (K / 128 <= 65535 && (M + 63) / 64 <= 32767 && N <= (1 << 25) && N < ((int64_t)1 << 31) / M),
                TPPX_EUNSUPPORTED, "%s: M=%ld N=%ld K=%ld is too large for this kernel's 32-bit offsets and grid", who, (long)M,
                (long)N, (long)K);
@@ -1119,11 +1118,11 @@ extern "C" int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa, con
   TPPX_REQUIRE((flags & ~TPPX_FLAG_XQ_REUSE) == 0, TPPX_EINVAL, "%s: flags 0x%x not taken here (TPPX_FLAG_XQ_REUSE only)", who, flags);
   TPPX_REQUIRE(K > 0 && K % 128 == 0, TPPX_ESHAPE, "%s: K=%ld must be a positive multiple of 128", who, (long)K);
   TPPX_REQUIRE(xq && sa && aligned16(xq) && aligned16(sa), TPPX_EINVAL, "%s: null or misaligned xq / sa scratch", who);
-  TPPX_REQUIRE(aligned16(s_nat), TPPX_EINVAL, "%s: scales not 16-byte aligned", who);
-  tppx_seg s = {q_nat, s_nat, bias, post_in, post_in2, y, N, post_op, post_scale};
+  for (int i = 0; i < 1 + (int)dual; i++)
+    TPPX_REQUIRE(aligned16(segs[i].sw), TPPX_EINVAL, "%s: scales not 16-byte aligned", who);
   DecodeParams p;
   memset(&p, 0, sizeof(p));
-  rc = fill_all(who, &s, 1, 16, false, p);
+  rc = fill_all(who, segs, 1 + (int)dual, 16, dual, p);
   if (rc)
     return rc;
   p.x = x;
@@ -1136,11 +1135,27 @@ extern "C" int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa, con
   p.S = 1;
   p.mt = (int)((M + 63) / 64 * 4);
   if (!(flags & TPPX_FLAG_XQ_REUSE)) {
-    rc = check_hip(launch_quant_act_w4a8_rows(x, M, K, p.mt, xq, (float*)sa, (hipStream_t)stream), who);
+    rc = check_hip(launch_quant_act_w4a8_rows(x, M, K, p.mt, xq, (float*)sa, stream), who);
     if (rc)
       return rc;
   }
-  return check_hip(launch_skinny_w4a8_mg(p, M >= 64, (hipStream_t)stream), who);
+  return check_hip(launch_skinny_w4a8_mg(p, M >= 64, dual, stream), who);
+}
+
+extern "C" int tppx_linear_mxfp4_int8_mid(const void* x, void* xq, void* sa, const void* q_nat, const void* s_nat,
+                                          const void* bias, const void* post_in, const void* post_in2, void* y,
+                                          int64_t M, int64_t N, int64_t K, int post_op, float post_scale, int flags,
+                                          tppx_stream_t stream) {
+  tppx_seg s = {q_nat, s_nat, bias, post_in, post_in2, y, N, post_op, post_scale};
+  return run_w4a8_mid("tppx_linear_mxfp4_int8_mid", x, xq, sa, &s, false, M, K, flags, (hipStream_t)stream);
+}
+
+extern "C" int tppx_swiglu_mxfp4_int8_mid(const void* x, void* xq, void* sa, const void* q_gate, const void* s_gate,
+                                          const void* bias_gate, const void* q_up, const void* s_up, const void* bias_up,
+                                          void* y, int64_t M, int64_t N, int64_t K, int flags, tppx_stream_t stream) {
+  tppx_seg s[2] = {{q_gate, s_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
+                   {q_up, s_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
+  return run_w4a8_mid("tppx_swiglu_mxfp4_int8_mid", x, xq, sa, s, true, M, K, flags, (hipStream_t)stream);
 }
 
 extern "C" void tppx_reload_env(void) {

@@ -158,8 +158,9 @@ hipError_t launch_skinny_qintx(DecodeParams& p, int mg, int ntw, hipStream_t str
 // W4A8 decode kernel (M <= 16): does it fit (LDS), and with how many channel tiles per workgroup; p.units = K / 128
 bool skinny_w4a8_fits(int64_t M, int total_tiles, int ktiles, int* ntw_out);
 hipError_t launch_skinny_w4a8(DecodeParams& p, int ntw, hipStream_t stream);
-// rows already quantised (p.xq, p.sa, p.mt a multiple of 4); ascending: K in one ascending sum per output, else four parts
-hipError_t launch_skinny_w4a8_mg(DecodeParams& p, bool ascending, hipStream_t stream);
+// rows already quantised (p.xq, p.sa, p.mt a multiple of 4); ascending: K in one ascending sum per output, else four parts;
+// dual: seg[0] = gate, seg[1] = up, silu(gate) * up to seg[0].y
+hipError_t launch_skinny_w4a8_mg(DecodeParams& p, bool ascending, bool dual, hipStream_t stream);
 // W4A8 rows quantised into that kernel's operand order, mt row tiles of 16 (rows past M repeat the last one):
 // xq mt * 16 * K bytes, sa mt * 16 * K / 32 floats
 hipError_t launch_quant_act_w4a8_rows(const void* x, int64_t M, int64_t K, int mt, void* xq, float* sa, hipStream_t stream);

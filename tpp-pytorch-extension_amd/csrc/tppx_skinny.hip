@@ -394,18 +394,20 @@ struct SkEpilogue {
       leave_row_sums(ov, sumsq, M);
   }
 
-  // The waves of a K part own different result tiles (channel tile a, row tile mg) of the workgroup: this wave has the
-  // OWN tiles slot0, slot0 + 1, .. (slot = a * MG + mg) of part kp.  The tiles are transposed: lane l holds channels
-  // (l >> 4) * 4 + r of row l & 15 (weights as the MFMA's first operand).  The KP parts are added in part order.
+  // The waves of a K part own different row tiles of the workgroup: this wave has the row tiles mg0 .. mg0 + OWN - 1 of
+  // part kp, for each of the NACC channel tiles.  The tiles are transposed: lane l holds channels (l >> 4) * 4 + r of row
+  // l & 15 (weights as the MFMA's first operand).  The KP parts are added in part order.
   template <int KP, int OWN>
-  __device__ __forceinline__ void finish_parts(const DecodeSeg& sg, f32x4 (&acc)[OWN], float* red, int kp, int slot0) {
-    static_assert(!DUAL && OUT % (FIXW * 64) == 0, "every thread finishes the same number of outputs");
+  __device__ __forceinline__ void finish_parts(const DecodeSeg& sg, f32x4 (&acc)[NACC][OWN], float* red, int kp, int mg0) {
+    static_assert(OUT % (FIXW * 64) == 0, "every thread finishes the same number of outputs");
     settle();
     const int lane = threadIdx.x & 63;
-    float* mine = red + kp * ELEMS + slot0 * 256 + (lane & 3) * 64 + ((lane >> 2) & 3) * 16 + (lane >> 4) * 4;
+    float* mine = red + kp * ELEMS + mg0 * 256 + (lane & 3) * 64 + ((lane >> 2) & 3) * 16 + (lane >> 4) * 4;
 #pragma unroll
-    for (int o = 0; o < OWN; o++)
-      *reinterpret_cast<f32x4*>(mine + o * 256) = acc[o];
+    for (int a = 0; a < NACC; a++)
+#pragma unroll
+      for (int o = 0; o < OWN; o++)
+        *reinterpret_cast<f32x4*>(mine + (a * MG + o) * 256) = acc[a][o];
     __syncthreads();
     uint32_t out[MAXE];
 #pragma unroll
@@ -415,7 +417,16 @@ struct SkEpilogue {
 #pragma unroll
       for (int k = 1; k < KP; k++)
         v += red[k * ELEMS + e];
-      out[i] = apply_post_bits(bf16_bits_to_f32(bias[i]) + v, sg.post_op, in1[i], in2[i], sg.post_scale);
+      if constexpr (DUAL) { // silu(gate) * up, the rounding points of the two calls
+        float u = red[OUT + e];
+#pragma unroll
+        for (int k = 1; k < KP; k++)
+          u += red[k * ELEMS + OUT + e];
+        const uint32_t gact = apply_post_bits(bf16_bits_to_f32(bias[i]) + v, TPPX_POST_SILU, 0, 0, 1.0f);
+        out[i] = apply_post_bits(bf16_bits_to_f32(bias2[i]) + u, TPPX_POST_MUL, gact & 0xffffu, 0, 1.0f);
+      } else {
+        out[i] = apply_post_bits(bf16_bits_to_f32(bias[i]) + v, sg.post_op, in1[i], in2[i], sg.post_scale);
+      }
     }
 #pragma unroll
     for (int i = 0; i < MAXE; i++)
@@ -1633,7 +1644,7 @@ skinny_w4a8_kernel(const DecodeParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// W4A8, 17 to 63 rows.  The rows arrive quantised in operand order (quant_act_w4a8_rows_kernel): xq [K/128][mt]
+// W4A8, 17 to 63 rows, one weight or the gate/up pair (DUAL).  The rows arrive quantised in operand order (quant_act_w4a8_rows_kernel): xq [K/128][mt]
 // [2 halves][64 lanes (g, m)][16 B], 8 bytes of each of two MX blocks per lane, and scales sa [K/128][mt][16 m][4 blocks]
 // f32, already times 6 / 127.  Weight tiles and their E8M0 dwords as in skinny_w4a8_kernel.  The weights are the MFMA's
 // FIRST operand, so a result tile is [channel][row]: a lane's four sums belong to one row, whose four block scales of a K
@@ -1649,11 +1660,20 @@ skinny_w4a8_kernel(const DecodeParams p) {
 // instruction expansion and no order between the MFMAs and the folds.  (Weights four tiles ahead instead of two: 50.8 at
 // 32 rows; four row tiles per wave at 50 rows: 73; the expansion shared by the row tiles through LDS as in the kernel
 // below: 46 / 60 us at 32 rows of these / 3584 x 16128 where this one takes 49 / 57, and 70 at 50 rows.)
+// DUAL, the gate/up pair: a wave holds the gate and the up tile of its channels, so a row's codes and scales, 3 of the
+// 4 KiB that a row tile takes through the vector memory path per K tile, are read once for both, there are twice the
+// independent chains in a wave, and one launch's start and end are gone: two launches -> one, quantizer included, in us
+//   rows     2048 x 5120      4096 x 11008     3584 x 16128     5120 x 13824
+//   32       15.9 -> 11.3     31.1 -> 22.0     35.1 -> 25.3     44.1 -> 31.3
+//   48       20.6 -> 13.5     47.5 -> 28.7     54.3 -> 32.6     71.7 -> 39.9
+//   63       21.2 -> 15.7     48.5 -> 34.3     55.9 -> 38.2     72.2 -> 47.3
+// (Three or four K tiles ahead: 24.3 / 26.1 at 32 rows of 4096 x 11008; the requests past the end of a wave's 8 tiles
+// are then 3 or 4 in 11 or 12.)
 // ---------------------------------------------------------------------------
-template <int MG, int R, int PF>
+template <int MG, int R, int PF, bool DUAL>
 __global__ void __launch_bounds__(4 * R * 64)
 skinny_w4a8_mg_kernel(const DecodeParams p) {
-  constexpr int KP = 4;
+  constexpr int KP = 4, NP = DUAL ? 2 : 1;
   extern __shared__ __align__(16) float sk_lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kp = wave % KP, rr = wave / KP;
@@ -1665,19 +1685,26 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
   const int t0 = b0 >> 2, t1 = (b1 + 3) >> 2, first = b0 & 3, last = ((b1 - 1) & 3) + 1;
 
   const int64_t lt = blockIdx.x;
-  const i32x4* wq = reinterpret_cast<const i32x4*>(sg.qw) + lt * KT * 64;
-  const i32x4* ws = reinterpret_cast<const i32x4*>(sg.sw) + lt * KT * 4; // E8M0 dwords of four channels
+  const i32x4 *wq[NP], *ws[NP];
+#pragma unroll
+  for (int q = 0; q < NP; q++) {
+    wq[q] = reinterpret_cast<const i32x4*>(p.seg[q].qw) + lt * KT * 64;
+    ws[q] = reinterpret_cast<const i32x4*>(p.seg[q].sw) + lt * KT * 4; // E8M0 dwords of four channels
+  }
   const int rt0 = (int)blockIdx.y * (MG * R) + rr * MG; // first row tile of this wave
   const i32x4* xop = reinterpret_cast<const i32x4*>(p.xq) + (int64_t)rt0 * 128;
   const f32x4* sop = reinterpret_cast<const f32x4*>(p.sa) + (int64_t)rt0 * 16;
   const int64_t xstride = p.mt * 128, sstride = p.mt * 16;
 
-  i32x4 wreg[PF], sreg[PF], xreg[PF][MG][2];
+  i32x4 wreg[PF][NP], sreg[PF][NP], xreg[PF][MG][2];
   f32x4 areg[PF][MG];
   auto load = [&](int st, int t) {
     t = min(t, t1 - 1); // (past the end: re-read a valid tile that is never consumed -- no branch around a load)
-    wreg[st] = R == 1 ? __builtin_nontemporal_load(wq + (int64_t)t * 64 + lane) : wq[(int64_t)t * 64 + lane];
-    sreg[st] = (ws + (int64_t)t * 4)[lane >> 4];
+#pragma unroll
+    for (int q = 0; q < NP; q++) {
+      wreg[st][q] = R == 1 ? __builtin_nontemporal_load(wq[q] + (int64_t)t * 64 + lane) : wq[q][(int64_t)t * 64 + lane];
+      sreg[st][q] = (ws[q] + (int64_t)t * 4)[lane >> 4];
+    }
 #pragma unroll
     for (int mg = 0; mg < MG; mg++) {
       xreg[st][mg][0] = (xop + t * xstride + mg * 128)[lane];
@@ -1689,16 +1716,18 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
   for (int i = 0; i < PF; i++)
     load(i, t0 + i);
   __builtin_amdgcn_sched_barrier(0);
-  SkEpilogue<MG * R, 1, false, KP * R, KP * R> ep;
-  f32x4 facc[MG];
+  SkEpilogue<MG * R, NP, DUAL, KP * R, KP * R> ep;
+  f32x4 facc[NP][MG];
 #pragma unroll
-  for (int mg = 0; mg < MG; mg++)
-    facc[mg] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int q = 0; q < NP; q++)
+#pragma unroll
+    for (int mg = 0; mg < MG; mg++)
+      facc[q][mg] = f32x4{0.f, 0.f, 0.f, 0.f};
   ep.prefetch_flat(p, sg, blockIdx.x, m0);
   __builtin_amdgcn_sched_barrier(0);
 
-  auto weights = [&](int i, int j) {
-    const uint32_t codes = (uint32_t)wreg[i][j];
+  auto weights = [&](int i, int q, int j) {
+    const uint32_t codes = (uint32_t)wreg[i][q][j];
     const uint32_t lo = w4a8_expand(codes & 0x0F0F0F0Fu), hi = w4a8_expand((codes >> 4) & 0x0F0F0F0Fu);
     return (long)(((uint64_t)hi << 32) | lo);
   };
@@ -1706,19 +1735,19 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
     return (long)(((uint64_t)(uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2 + 1] << 32) |
                   (uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2]);
   };
-  auto block = [&](int i, int j) {
-    const long wb = weights(i, j);
+  auto block = [&](int i, int q, int j) {
+    const long wb = weights(i, q, j);
     float wsc[4];
 #pragma unroll
     for (int r = 0; r < 4; r++)
-      wsc[r] = e8m0_to_f32((uint32_t)sreg[i][r] >> (8 * j));
+      wsc[r] = e8m0_to_f32((uint32_t)sreg[i][q][r] >> (8 * j));
 #pragma unroll
     for (int mg = 0; mg < MG; mg++) {
       const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, rows(i, mg, j), i32x4{0, 0, 0, 0}, 0, 0, 0);
       const float sav = areg[i][mg][j];
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        facc[mg][r] = fmaf((float)acc[r], sav * wsc[r], facc[mg][r]);
+        facc[q][mg][r] = fmaf((float)acc[r], sav * wsc[r], facc[q][mg][r]);
     }
   };
   // A whole K tile whose weight scales are all below 2 (E8M0 bytes 1 .. 127; 0 is a scale of zero in every W4A8 kernel).
@@ -1728,41 +1757,46 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
   // or a multiplication.  The MFMAs of a block go out ahead of the fold of the block before it.
   auto whole_tile = [&](int i) {
     i32x4 start[2], acc[2][MG];
-    auto issue = [&](auto J) {
-      constexpr int j = decltype(J)::value;
-      const long wb = weights(i, j);
+    auto issue = [&](auto U) { // unit u: block u / NP of weight tile u % NP
+      constexpr int u = decltype(U)::value, j = u / NP, q = u % NP;
+      const long wb = weights(i, q, j);
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        start[j & 1][r] = (int)((((uint32_t)sreg[i][r] >> (8 * j)) & 0xffu) << 23) + 0x0BC00000;
+        start[u & 1][r] = (int)((((uint32_t)sreg[i][q][r] >> (8 * j)) & 0xffu) << 23) + 0x0BC00000;
 #pragma unroll
       for (int mg = 0; mg < MG; mg++)
-        acc[j & 1][mg] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, rows(i, mg, j), start[j & 1], 0, 0, 0);
+        acc[u & 1][mg] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, rows(i, mg, j), start[u & 1], 0, 0, 0);
     };
     issue(std::integral_constant<int, 0>{});
-    static_for<0, 4>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      if constexpr (j < 3)
-        issue(std::integral_constant<int, j + 1>{});
+    static_for<0, 4 * NP>([&](auto U) {
+      constexpr int u = decltype(U)::value, j = u / NP, q = u % NP;
+      if constexpr (u < 4 * NP - 1)
+        issue(std::integral_constant<int, u + 1>{});
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int mg = 0; mg < MG; mg++)
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          facc[mg][r] = fmaf(__int_as_float(acc[j & 1][mg][r]) - __int_as_float(start[j & 1][r]), areg[i][mg][j], facc[mg][r]);
+          facc[q][mg][r] = fmaf(__int_as_float(acc[u & 1][mg][r]) - __int_as_float(start[u & 1][r]), areg[i][mg][j], facc[q][mg][r]);
     });
   };
   auto consume = [&](int i, int t) {
     const int lo = t == t0 ? first : 0, hi = t == t1 - 1 ? last : 4;
     uint32_t any = 0;
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-      any |= (uint32_t)sreg[i][r] | ((uint32_t)sreg[i][r] - 0x01010101u); // a top bit for a byte of 0 or from 128 on
+    for (int q = 0; q < NP; q++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        any |= (uint32_t)sreg[i][q][r] | ((uint32_t)sreg[i][q][r] - 0x01010101u); // a top bit for a byte of 0 or from 128 on
     if (!__any((any & 0x80808080u) != 0) && lo == 0 && hi == 4) {
       whole_tile(i);
     } else {
       static_for<0, 4>([&](auto J) {
-        if (decltype(J)::value >= lo && decltype(J)::value < hi)
-          block(i, decltype(J)::value);
+        if (decltype(J)::value >= lo && decltype(J)::value < hi) {
+#pragma unroll
+          for (int q = 0; q < NP; q++)
+            block(i, q, decltype(J)::value);
+        }
       });
     }
   };
@@ -1796,10 +1830,13 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
 //   64       17.2 -> 14.2 (38)    30.2 -> 22.6 (45)    35.0 -> 28.1 (93)    49.3 -> 38.3 (131)
 //   128      23.9 -> 18.1 (39)    49.6 -> 34.5 (45)    52.4 -> 36.4 (93)    70.9 -> 49.2 (131)
 //   256      38.0 -> 24.6 (39)    85.2 -> 58.9 (67)    86.4 -> 55.2 (92)    123 -> 73.5 (130)
+// DUAL, the gate/up pair: the two channel tiles of a workgroup are a gate and an up tile.  Two launches -> one, in us, at
+// 64 / 128 / 200 rows of 4096 x 11008 43.5 -> 33.2 / 66.5 -> 56.7 / 110 -> 97.5, of 3584 x 16128 42.9 -> 38.8 / 74.7 -> 66.0 / 133 -> 122.
 // ---------------------------------------------------------------------------
-template <int NT>
+template <int NT, bool DUAL>
 __global__ void __launch_bounds__(256)
 skinny_w4a8_rows_kernel(const DecodeParams p) {
+  static_assert(!DUAL || NT == 2, "the pair: a gate tile and the up tile of the same channels");
   constexpr uint32_t START = 0x0BC00000u; // E8M0 byte e << 23 plus this: the bits of 1.5 * 2^(23 + e - 127)
   constexpr int KS = 4; // K tiles per step: each of the four waves expands one (of every channel tile)
   __shared__ __align__(16) long w_s[2][NT][KS][4][64]; // [buffer][channel tile][K tile][block][lane] codes, operand order
@@ -1814,9 +1851,10 @@ skinny_w4a8_rows_kernel(const DecodeParams p) {
   const uint32_t* ws[NT];
 #pragma unroll
   for (int a = 0; a < NT; a++) {
-    const int64_t lt = min((int)blockIdx.x * NT + a, sg.tiles - 1); // ragged last group: duplicate, not stored
-    wq[a] = reinterpret_cast<const i32x4*>(sg.qw) + lt * KT * 64 + lane;
-    ws[a] = reinterpret_cast<const uint32_t*>(sg.sw) + lt * KT * 16 + (lane & 15);
+    const int64_t lt = DUAL ? (int)blockIdx.x : min((int)blockIdx.x * NT + a, sg.tiles - 1); // ragged last group: duplicate, not stored
+    const DecodeSeg& sa = p.seg[DUAL ? a : 0];
+    wq[a] = reinterpret_cast<const i32x4*>(sa.qw) + lt * KT * 64 + lane;
+    ws[a] = reinterpret_cast<const uint32_t*>(sa.sw) + lt * KT * 16 + (lane & 15);
   }
   const i32x4* xop = reinterpret_cast<const i32x4*>(p.xq) + (int64_t)rt * 128 + lane;
   const f32x4* sop = reinterpret_cast<const f32x4*>(p.sa) + (int64_t)rt * 16 + (lane & 15);
@@ -1846,22 +1884,25 @@ skinny_w4a8_rows_kernel(const DecodeParams p) {
     load_x(i, i);
   __builtin_amdgcn_sched_barrier(0);
   // (an absent input is read from the output, as in SkEpilogue::prefetch_flat: no branch around a load)
-  const uint16_t* pb = sg.bias ? sg.bias : sg.y;
   const uint16_t* p1 = sg.post_in ? sg.post_in : sg.y;
   const uint16_t* p2 = sg.post_in2 ? sg.post_in2 : sg.y;
   const int m = rt * 16 + (lane & 15);
   uint16_t in1[NT][4], in2[NT][4];
   f32x4 facc[NT];
 #pragma unroll
-  for (int a = 0; a < NT; a++)
+  for (int a = 0; a < NT; a++) {
+    const uint16_t* bias = p.seg[DUAL ? a : 0].bias;
+    const uint16_t* pb = bias ? bias : sg.y;
+    const int tile = DUAL ? (int)blockIdx.x : min((int)blockIdx.x * NT + a, sg.tiles - 1);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int n = min((int)blockIdx.x * NT + a, sg.tiles - 1) * 16 + (lane >> 4) * 4 + r, o = min(m, p.M - 1) * sg.N + n;
+      const int n = tile * 16 + (lane >> 4) * 4 + r, o = min(m, p.M - 1) * sg.N + n;
       const uint32_t b = pb[n];
-      in1[a][r] = p1[o];
-      in2[a][r] = p2[o];
-      facc[a][r] = sg.bias ? bf16_bits_to_f32(b) : 0.f;
+      in1[a][r] = DUAL ? 0 : p1[o];
+      in2[a][r] = DUAL ? 0 : p2[o];
+      facc[a][r] = bias ? bf16_bits_to_f32(b) : 0.f;
     }
+  }
   __builtin_amdgcn_sched_barrier(0);
 
   auto expand = [&](int s) {
@@ -1951,6 +1992,16 @@ skinny_w4a8_rows_kernel(const DecodeParams p) {
   }
   if (m >= p.M)
     return;
+  if constexpr (DUAL) { // silu(gate) * up, the rounding points of the two calls
+    uint32_t h[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const uint32_t gact = apply_post_bits(facc[0][r], TPPX_POST_SILU, 0, 0, 1.0f) & 0xffffu;
+      h[r] = apply_post_bits(facc[1][r], TPPX_POST_MUL, gact, 0, 1.0f) & 0xffffu;
+    }
+    *reinterpret_cast<uint2*>(sg.y + (int64_t)m * sg.N + blockIdx.x * 16 + (lane >> 4) * 4) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    return;
+  }
 #pragma unroll
   for (int a = 0; a < NT; a++) {
     const int lt = (int)blockIdx.x * NT + a;
@@ -2876,26 +2927,36 @@ hipError_t launch_skinny_w4a8(DecodeParams& p, int ntw, hipStream_t stream) {
 }
 
 // W4A8 between decode and the prompt passes; p.mt, p.units set by the caller
-template <int MG, int R, int PF>
+template <int MG, int R, int PF, bool DUAL>
 static hipError_t sk_launch_w4a8_mg(DecodeParams& p, hipStream_t stream) {
   const dim3 grid(p.total_tiles, (p.M + MG * R * 16 - 1) / (MG * R * 16), 1);
-  return sk_launch(skinny_w4a8_mg_kernel<MG, R, PF>, p, grid, 4 * R, (size_t)4 * MG * R * 256 * sizeof(float), stream);
+  return sk_launch(skinny_w4a8_mg_kernel<MG, R, PF, DUAL>, p, grid, 4 * R, (size_t)4 * (DUAL ? 2 : 1) * MG * R * 256 * sizeof(float),
+                   stream);
 }
-hipError_t launch_skinny_w4a8_mg(DecodeParams& p, bool ascending, hipStream_t stream) {
-  if (p.S != 1 || p.mt <= 0 || p.n_seg != 1)
+hipError_t launch_skinny_w4a8_mg(DecodeParams& p, bool ascending, bool dual, hipStream_t stream) {
+  if (p.S != 1 || p.mt <= 0 || p.n_seg != (dual ? 2 : 1))
     return hipErrorInvalidValue;
   if (ascending) {
     // One channel tile per workgroup while those all run at once (two per CU: registers), else two, which read the rows
     // half as often: 512 workgroups of one at 128 rows of 4096 x 11008 36.4 us against 39.8, 4096 x 4096 18.1 against
     // 18.4; 768 (192 rows) 56.0 against 50.1 and 26.5 against 23.2.
     const int by = (p.M + 63) / 64;
+    if (dual)
+      return sk_launch(skinny_w4a8_rows_kernel<2, true>, p, dim3(p.total_tiles, by, 1), 4, 0, stream);
     if ((int64_t)p.total_tiles * by <= 512)
-      return sk_launch(skinny_w4a8_rows_kernel<1>, p, dim3(p.total_tiles, by, 1), 4, 0, stream);
-    return sk_launch(skinny_w4a8_rows_kernel<2>, p, dim3((p.total_tiles + 1) / 2, by, 1), 4, 0, stream);
+      return sk_launch(skinny_w4a8_rows_kernel<1, false>, p, dim3(p.total_tiles, by, 1), 4, 0, stream);
+    return sk_launch(skinny_w4a8_rows_kernel<2, false>, p, dim3((p.total_tiles + 1) / 2, by, 1), 4, 0, stream);
+  }
+  // The pair: one wave per K quarter with all of the rows.  At 63 rows of 4096 x 11008 / 3584 x 16128 34.3 / 38.2 us;
+  // two waves of two row tiles, which leave one workgroup per CU, 39.0 / 46.7 (50 rows), four of one 52.3 / 62.4.
+  if (dual) {
+    if (p.M <= 32)
+      return sk_launch_w4a8_mg<2, 1, 2, true>(p, stream);
+    return p.M <= 48 ? sk_launch_w4a8_mg<3, 1, 2, true>(p, stream) : sk_launch_w4a8_mg<4, 1, 2, true>(p, stream);
   }
   if (p.M <= 16)
-    return sk_launch_w4a8_mg<1, 1, 4>(p, stream);
-  return p.M <= 32 ? sk_launch_w4a8_mg<2, 1, 2>(p, stream) : sk_launch_w4a8_mg<2, 2, 2>(p, stream);
+    return sk_launch_w4a8_mg<1, 1, 4, false>(p, stream);
+  return p.M <= 32 ? sk_launch_w4a8_mg<2, 1, 2, false>(p, stream) : sk_launch_w4a8_mg<2, 2, 2, false>(p, stream);
 }
 
 // MXFP4, 33..64 rows per block row: four channel tiles x four K parts per workgroup, K in p.S slices across workgroups

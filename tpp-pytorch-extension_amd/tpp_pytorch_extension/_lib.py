@@ -97,6 +97,7 @@ SIGNATURES = {
     "tppx_prepack_mxfp4_int8": [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp],
     "tppx_linear_mxfp4_int8_rows": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _f32, _vp],
     "tppx_linear_mxfp4_int8_mid": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _f32, _i32, _vp],
+    "tppx_swiglu_mxfp4_int8_mid": [_vp] * 10 + [_i64, _i64, _i64, _i32, _vp],
     "tppx_prepack_mxfp4_int8_wide": [_vp, _vp, _i64, _i64, _i64, _vp, _vp],
     "tppx_linear_mxfp4_int8_wide": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _f32, _vp, _i64, _vp],
     "tppx_linear_qintx": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _f32, _i32, _vp],

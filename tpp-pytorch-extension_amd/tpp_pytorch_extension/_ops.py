@@ -700,6 +700,12 @@ def _w4a8_row_groups(M, N, K):
     return groups < prompt
 
 
+def _w4a8_takes_groups(M, N, K):
+    if M >= W4A8_WIDE_ROWS:
+        return M >= 64 and _w4a8_row_groups(M, N, K)
+    return M < 64 and W4A8_DECODE
+
+
 def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=None):
     """TppBlockedLinearW<int8_t, uint8_t, Tout> (src/csrc/fused_gemm.h:965-978, 1523-1526): bf16 activations are
     quantized to int8 over blocks of 32 (quantize_int8sym with the weight's block size), the scales multiplied by
@@ -726,9 +732,7 @@ def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=
     # From TPPX_W4A8_WIDE_ROWS rows: K in one ascending sum per output, by the prompt kernel (its weights are a second
     # copy, 2 bytes per value) or, with the same bits, by row groups on the 4-bit tiles.
     wide_rows = M >= W4A8_WIDE_ROWS
-    nat = None
-    if (M >= 64 and _w4a8_row_groups(M, N, K)) if wide_rows else (M < 64 and W4A8_DECODE):
-        nat = weight.native_w4a8()
+    nat = weight.native_w4a8() if _w4a8_takes_groups(M, N, K) else None
     if nat is not None and M <= 16:
         rc = L.tppx_linear_mxfp4_int8_rows(x.data_ptr(), nat[0].data_ptr(), nat[1].data_ptr(), _lib.ptr(bias),
                                            _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N, K, post, post_scale,
@@ -764,6 +768,32 @@ def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=
     _lib.check(L.tppx_linear_mxfp4_int8(act.qdata.data_ptr(), sa.data_ptr(), weight.qdata.data_ptr(),
                                         weight.scales.data_ptr(), _lib.ptr(bias), _lib.ptr(post_in), _lib.ptr(post_in2),
                                         y.data_ptr(), M, N, K, weight.shape[2] * 8, post, post_scale, _lib.stream_of(x)))
+    return y
+
+
+def _w4a8_pair(input, w_gate, w_up, b_gate, b_up):
+    """silu(gate) * up of W4A8 weights in one launch behind the row quantizer, the bits of the two calls; None where those
+    do not both run on the row-group kernels (their own checks and messages then)."""
+    N, K = w_gate.weight_nk()
+    if input.dtype != torch.bfloat16 or input.device.type != "cuda" or input.shape[-1] != K or w_up.weight_nk() != (N, K):
+        return None
+    M = input.numel() // K
+    if M <= 16 or not _w4a8_takes_groups(M, N, K):
+        return None
+    x = input.contiguous()
+    nat_g, nat_u = w_gate.native_w4a8(), w_up.native_w4a8()
+    if nat_g is None or nat_u is None or x.data_ptr() % 16:
+        return None
+    y = torch.empty(tuple(input.shape[:-1]) + (N,), dtype=torch.bfloat16, device=x.device)
+    bg, bu = _prep_bias(b_gate, N, x.device), _prep_bias(b_up, N, x.device)
+    mp = (M + 63) // 64 * 64
+    held = torch.empty(mp * K + mp * (K // 8), dtype=torch.uint8, device=x.device)
+    rc = _lib.lib().tppx_swiglu_mxfp4_int8_mid(x.data_ptr(), held.data_ptr(), held.data_ptr() + mp * K, nat_g[0].data_ptr(),
+                                               nat_g[1].data_ptr(), _lib.ptr(bg), nat_u[0].data_ptr(), nat_u[1].data_ptr(),
+                                               _lib.ptr(bu), y.data_ptr(), M, N, K, 0, _lib.stream_of(x))
+    if rc == _lib.EUNSUPPORTED:
+        return None
+    _lib.check(rc)
     return y
 
 
@@ -1139,6 +1169,9 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
         if norm is not None:
             input = rms_norm(input, norm[0], norm[1])
         if _is_w4a8(w_gate) and _is_w4a8(w_up):
+            y = _w4a8_pair(input, w_gate, w_up, b_gate, b_up)
+            if y is not None:
+                return y
             rows = []  # one quantization of the rows for both projections
             gate = _linear_w4a8(input, w_gate, b_gate, POST_SILU, None, None, 1.0, rows)
             return _linear_w4a8(input, w_up, b_up, POST_MUL, gate, None, 1.0, rows)

@@ -102,6 +102,37 @@ def test_attn_decode(B, Nq, Nkv, L, Smax, kernel, monkeypatch):
     assert np.sqrt(((g - t) ** 2).sum() / (t ** 2).sum()) <= 1e-2
 
 
+@pytest.mark.parametrize("H", [128, 256, 80, 64])
+@pytest.mark.parametrize("L", [65, 128, 129, 256, 257, 415, 640, 1153])
+def test_attn_decode_several_trips(H, L):
+    """One workgroup per head walks all the keys, the next trip's rows requested during this one: lengths around the ends of
+    trips (128 or 64 keys) and of a wave's part of them, the new key in the first, a middle and the last trip, NaN behind the
+    length; against float64 and, with the new key still outside the cache, against the launch that finds it there."""
+    F = _llm()
+    from tpp_pytorch_extension import _lib
+    Lb = _lib.lib()
+    B, N, Smax = 2, 3, 1200
+    q, k, v = (randn_bf16((B, N) + d + (H,), 1.0, 40 + i).cuda() for i, d in enumerate(((), (Smax,), (Smax,))))
+    k[:, :, L:] = v[:, :, L:] = float("nan")
+    got = _attn(F, q, k, v, L, ws=False)
+    s = torch.matmul(k[:, :, :L].double(), q.double().unsqueeze(-1)).squeeze(-1) / np.sqrt(H)
+    ref = torch.matmul(torch.softmax(s, -1).unsqueeze(2), v[:, :, :L].double()).squeeze(2)
+    assert float((got.double() - ref).norm() / ref.norm()) <= 5e-3 and got.isfinite().all()
+    kc, vc, n = k.clone(), v.clone(), torch.tensor([L - 1], dtype=torch.int32, device="cuda")
+    pos = torch.full((B, 1), L, dtype=torch.int64, device="cuda")
+    kn, vn = k[:, :, L - 1].contiguous(), v[:, :, L - 1].contiguous()
+    kc[:, :, L - 1] = vc[:, :, L - 1] = float("nan")
+    out = torch.empty_like(q)
+    tail = (kc.data_ptr(), vc.data_ptr(), None, 0, n.data_ptr(), out.data_ptr(), B, N, N, H, Smax, None, 0, _lib.stream_of(q))
+    if H == 128:  # (positions past the table are left unrotated)
+        _lib.check(Lb.tppx_attn_decode_rotary(q.data_ptr(), kn.data_ptr(), vn.data_ptr(), F.llama_rotary_table(64, 128).data_ptr(),
+                                              pos.data_ptr(), B, 64, H, *tail))
+    else:
+        _lib.check(Lb.tppx_attn_decode_append(q.data_ptr(), kn.data_ptr(), vn.data_ptr(), None, 0, pos.data_ptr(), B, 4096, H, *tail))
+    assert torch.equal(out, got)
+    assert torch.equal(kc[:, :, :L], k[:, :, :L]) and torch.equal(vc[:, :, :L], v[:, :, :L])
+
+
 def test_attn_decode_split_merge_in_launch_equals_second_kernel(monkeypatch):
     """With a workspace the keys are split over several workgroups per head; the split that arrives last merges
     them inside the launch.  Twenty launches in a row (the arrival counters must return to zero) give the bits of

@@ -609,8 +609,13 @@ attn_decode_kernel(const AttnParams p) {
 //     split that reads its position.
 // The per-lane outputs (16 dims, partial over the lane's keys) are added up
 // through LDS at the end.  The first trip's K and V rows (16 KB per wave) are
-// requested before anything else; later trips request theirs when they start
-// (the launch planner sends long loops to the kernel above).
+// requested before anything else, a later trip's K rows once this trip's scores
+// have freed their registers and its V rows behind this trip's sums, so that a
+// workgroup of many trips never stands without requests; lanes past the length
+// share its last row (a last trip of one key fetched 128).  Against requests at
+// the start of a trip, rows up to the cache's end, 32 heads: 16 sequences of 2048
+// keys 90 -> 85 us (6.3 TB/s, ends of the launch included), a step of four layers
+// of 32 of 1300 741 -> 707, 2 of 2048 229 -> 222, 1 of 2000 201 -> 199.
 // ---------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
 __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
@@ -645,10 +650,10 @@ attn_decode_wide_kernel(const AttnParams p) {
   const char* vb = reinterpret_cast<const char*>(p.vc + ((int64_t)b * p.Nkv + hk) * p.Smax * 128) + q8 * 16;
   // key set s of a trip: keys base + s*8 + kq; register [s][j] holds dims (j*8 + q8)*8 .. +7 as four bf16 pairs
   i32x4 kr[4][2], vr[4][2];
-  auto load_rows = [&](const char* src, int base, i32x4 (&dst)[4][2]) {
+  auto load_rows = [&](const char* src, int base, int end, i32x4 (&dst)[4][2]) {
 #pragma unroll
     for (int s = 0; s < 4; s++) {
-      const int key = min(base + s * 8 + kq, p.Smax - 1); // past the end: read, never used
+      const int key = min(base + s * 8 + kq, end - 1); // past the end: read, never used
 #pragma unroll
       for (int j = 0; j < 2; j++)
         dst[s][j] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(src + (int64_t)key * 256 + j * 128));
@@ -678,8 +683,8 @@ attn_decode_wide_kernel(const AttnParams p) {
       sn = p.emb[((int64_t)p.MP + pp) * 128 + lane];
     }
   }
-  load_rows(kb, blockIdx.y * ATTN_WIDE_KEYS + wave * 32, kr);
-  load_rows(vb, blockIdx.y * ATTN_WIDE_KEYS + wave * 32, vr);
+  load_rows(kb, blockIdx.y * ATTN_WIDE_KEYS + wave * 32, p.Smax, kr);
+  load_rows(vb, blockIdx.y * ATTN_WIDE_KEYS + wave * 32, p.Smax, vr);
   const int len0 = *p.kv_len;
   const int L = max(0, min(len0 + p.kv_len_add, p.Smax));
   const int nk = (ROT && len0 >= 0 && len0 < p.Smax) ? len0 : -1; // cache position of the new token
@@ -715,29 +720,25 @@ attn_decode_wide_kernel(const AttnParams p) {
 #pragma unroll
   for (int e = 0; e < 16; e++)
     acc[e] = 0.f;
-  for (int t = blockIdx.y; t < trips; t += S) {
-    const int base = t * ATTN_WIDE_KEYS + wave * 32;
-    if (t != (int)blockIdx.y) { // the workgroups of this kernel make few trips: no request queue across trips
-      load_rows(kb, base, kr);
-      load_rows(vb, base, vr);
-    }
+  // a trip in two halves: the scores of its keys, which frees the K registers, then the sums, which free the V registers
+  float sc[4];
+  auto scores = [&](int base) {
     if (has_new && nk >= base && nk < base + 32) {
       // the new token is not in the cache yet (or is being written right now): its lanes take the rotated key from
       // LDS and the value from the step's input
-      const int s_new = (nk - base) >> 3;
-      if (kq == ((nk - base) & 7)) {
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const i32x4 kv = reinterpret_cast<const i32x4*>(k_s)[j * 8 + q8];
+        const i32x4 vv = *reinterpret_cast<const i32x4*>(p.v_new + ((int64_t)b * p.Nkv + hk) * 128 + (j * 8 + q8) * 8);
 #pragma unroll
         for (int s = 0; s < 4; s++)
-          if (s == s_new) {
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-              kr[s][j] = reinterpret_cast<const i32x4*>(k_s)[j * 8 + q8];
-              vr[s][j] = *reinterpret_cast<const i32x4*>(p.v_new + ((int64_t)b * p.Nkv + hk) * 128 + (j * 8 + q8) * 8);
-            }
+          for (int r = 0; r < 4; r++) { // (selects: stores under a condition end up indexed, and the rows in scratch memory)
+            kr[s][j][r] = nk == base + s * 8 + kq ? kv[r] : kr[s][j][r];
+            vr[s][j][r] = nk == base + s * 8 + kq ? vv[r] : vr[s][j][r];
           }
       }
     }
-    float sc[4];
 #pragma unroll
     for (int s = 0; s < 4; s++) {
       const int key = base + s * 8 + kq;
@@ -755,6 +756,8 @@ attn_decode_wide_kernel(const AttnParams p) {
         d += bf16_bits_to_f32(mrow[key]);
       sc[s] = key < L ? d : -3.0e38f;
     }
+  };
+  auto sums = [&](int base) {
     const float mn = fmaxf(m, wave_max(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]))));
     if (mn > m) { // wave-uniform; rare once the first trips have passed
       const float alpha = __expf(m - mn);
@@ -790,6 +793,22 @@ attn_decode_wide_kernel(const AttnParams p) {
           acc[j * 8 + 2 * r] = dot2_bf16(lo, pk[h], acc[j * 8 + 2 * r]);
           acc[j * 8 + 2 * r + 1] = dot2_bf16(hi, pk[h], acc[j * 8 + 2 * r + 1]);
         }
+  };
+  int t = blockIdx.y;
+  for (; t + S < trips; t += S) { // (the last trip on its own: a load under a condition would make every wait one for all)
+    const int base = t * ATTN_WIDE_KEYS + wave * 32, next = (t + S) * ATTN_WIDE_KEYS + wave * 32;
+    scores(base);
+    __builtin_amdgcn_sched_barrier(0);
+    load_rows(kb, next, L, kr); // lanes past the end share the last row: a trip of one key fetches one
+    __builtin_amdgcn_sched_barrier(0);
+    sums(base);
+    __builtin_amdgcn_sched_barrier(0);
+    load_rows(vb, next, L, vr);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (t < trips) {
+    scores(t * ATTN_WIDE_KEYS + wave * 32);
+    sums(t * ATTN_WIDE_KEYS + wave * 32);
   }
   // add up the lanes' partial outputs: [wave][kq][dim], rows padded against bank conflicts
 #pragma unroll
@@ -2158,6 +2177,8 @@ attn_generic_kernel(const AttnGenParams p) {
 // steps, against rotary + append, attention and the merge as launches of their own: 16 heads of 256, 1 x 2000 keys
 // 24.2 -> 12.5 us, 4 x 700 18.1 -> 12.2, 16 x 2500 106.5 (6.2 TB/s) either way; 32 heads of 80, 1 x 2000 14.3 -> 9.7,
 // 4 x 140 7.8 -> 7.0, 48 x 1400 113.7 -> 108.3.  (80 as 8 lanes x 2 chunks, the second a quarter live, 117.4.)
+// Later trips' rows are requested as in attn_decode_wide_kernel: a graph of four layers with 16 heads of 256, 1 x 2000 keys
+// 205.8 -> 199.4 us, 16 x 2500 619.8 -> 607.2, with 32 heads of 80, 1 x 2000 181.9 -> 176.1, 48 x 1400 677.7 -> 671.3.
 template <int G, int J, int NU, bool APP>
 __global__ void __launch_bounds__(256, 4)
 attn_hd_step_kernel(const AttnGenParams p) {
@@ -2184,10 +2205,10 @@ attn_hd_step_kernel(const AttnGenParams p) {
     at[j] = min(j * G + c, C - 1) * 8;
   }
   i32x4 kr[NU][J], vr[NU][J];
-  auto load_rows = [&](const uint16_t* src, int base, i32x4 (&dst)[NU][J]) {
+  auto load_rows = [&](const uint16_t* src, int base, int end, i32x4 (&dst)[NU][J]) {
 #pragma unroll
     for (int u = 0; u < NU; u++) {
-      const int64_t row = (int64_t)min(base + u * KPI + grp, p.Smax - 1) * H; // past the end: read, never used
+      const int64_t row = (int64_t)min(base + u * KPI + grp, end - 1) * H; // past the end: read, never used
 #pragma unroll
       for (int j = 0; j < J; j++)
         dst[u][j] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(src + row + at[j]));
@@ -2229,8 +2250,8 @@ attn_hd_step_kernel(const AttnGenParams p) {
       }
     }
   }
-  load_rows(kb, blockIdx.y * TRIP + wave * WK, kr);
-  load_rows(vb, blockIdx.y * TRIP + wave * WK, vr);
+  load_rows(kb, blockIdx.y * TRIP + wave * WK, p.Smax, kr);
+  load_rows(vb, blockIdx.y * TRIP + wave * WK, p.Smax, vr);
   const int len0 = *p.kv_len;
   const int L = max(0, min(len0 + p.kv_len_add, p.Smax));
   const int nk = (APP && len0 >= 0 && len0 < p.Smax) ? len0 : -1; // cache position of the new token
@@ -2243,8 +2264,9 @@ attn_hd_step_kernel(const AttnGenParams p) {
       for (int i = 0; i < D; i++) {
         const int d = lane + 64 * i;
         if (d < H) {
-          q_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? qx[i] * cs[i] + qo[i] * sn[i] : qx[i]);
-          k_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? kx[i] * cs[i] + ko[i] * sn[i] : kx[i]);
+          // (which product is fused is left to chance in a plain sum of two; rotary_append_kernel fuses the cosine's)
+          q_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(qx[i], cs[i], __fmul_rn(qo[i], sn[i])) : qx[i]);
+          k_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(kx[i], cs[i], __fmul_rn(ko[i], sn[i])) : kx[i]);
         }
       }
     }
@@ -2265,25 +2287,24 @@ attn_hd_step_kernel(const AttnGenParams p) {
 #pragma unroll
   for (int e = 0; e < J * 8; e++)
     acc[e] = 0.f;
-  for (int t = blockIdx.y; t < trips; t += S) {
-    const int base = t * TRIP + wave * WK;
-    if (t != (int)blockIdx.y) {
-      load_rows(kb, base, kr);
-      load_rows(vb, base, vr);
-    }
-    if (has_new && nk >= base && nk < base + WK && grp == (nk - base) % KPI) {
-      const int u_new = (nk - base) / KPI;
+  // a trip in two halves, as in attn_decode_wide_kernel
+  float sc[NU], mx;
+  auto scores = [&](int base) {
+    if (has_new && nk >= base && nk < base + WK) {
 #pragma unroll
-      for (int u = 0; u < NU; u++)
-        if (u == u_new) {
+      for (int j = 0; j < J; j++) {
+        const i32x4 kv = *reinterpret_cast<const i32x4*>(k_s + at[j]);
+        const i32x4 vv = *reinterpret_cast<const i32x4*>(p.v_new + kv_head * H + at[j]);
 #pragma unroll
-          for (int j = 0; j < J; j++) {
-            kr[u][j] = *reinterpret_cast<const i32x4*>(k_s + at[j]);
-            vr[u][j] = *reinterpret_cast<const i32x4*>(p.v_new + kv_head * H + at[j]);
+        for (int u = 0; u < NU; u++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) { // (selects, not stores under a condition)
+            kr[u][j][r] = nk == base + u * KPI + grp ? kv[r] : kr[u][j][r];
+            vr[u][j][r] = nk == base + u * KPI + grp ? vv[r] : vr[u][j][r];
           }
-        }
+      }
     }
-    float sc[NU], mx = -3.0e38f;
+    mx = -3.0e38f;
 #pragma unroll
     for (int u = 0; u < NU; u++) {
       const int key = base + u * KPI + grp;
@@ -2307,6 +2328,8 @@ attn_hd_step_kernel(const AttnGenParams p) {
       sc[u] = key < L ? d : -3.0e38f;
       mx = fmaxf(mx, sc[u]);
     }
+  };
+  auto sums = [&](int base) {
     const float mn = fmaxf(m, wave_max(mx));
     if (mn > m) { // wave-uniform; rare once the first trips have passed
       const float alpha = __expf(m - mn);
@@ -2348,6 +2371,22 @@ attn_hd_step_kernel(const AttnGenParams p) {
           acc[j * 8 + 2 * r] = dot2_bf16(lo, pk[h], dot2_bf16(lo, pk2[h], acc[j * 8 + 2 * r]));
           acc[j * 8 + 2 * r + 1] = dot2_bf16(hi, pk[h], dot2_bf16(hi, pk2[h], acc[j * 8 + 2 * r + 1]));
         }
+  };
+  int t = blockIdx.y;
+  for (; t + S < trips; t += S) {
+    const int base = t * TRIP + wave * WK, next = (t + S) * TRIP + wave * WK;
+    scores(base);
+    __builtin_amdgcn_sched_barrier(0);
+    load_rows(kb, next, L, kr);
+    __builtin_amdgcn_sched_barrier(0);
+    sums(base);
+    __builtin_amdgcn_sched_barrier(0);
+    load_rows(vb, next, L, vr);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (t < trips) {
+    scores(t * TRIP + wave * WK);
+    sums(t * TRIP + wave * WK);
   }
 #pragma unroll
   for (int j = 0; j < J; j++) {

@@ -190,8 +190,8 @@ def workspace(t, stream=None, rows=0):
     so work still queued there keeps it valid).  with_counters(): arrival
     counters behind the buffer, under the same ordering."""
     global _tick
-    dev = t.device.index
-    if torch.cuda.is_current_stream_capturing():
+    dev = t.get_device()
+    if torch._C._cuda_isCurrentStreamCapturing():
         ws = _workspaces.get((dev, "capture"))
         if ws is None:
             raise TppxError(EINVAL, "first call on this device happens inside graph capture: run the op once "

@@ -13,7 +13,7 @@ import torch
 from . import _lib
 from ._lib import (POST_NONE, POST_SILU, POST_MUL, POST_ADD_SCALE, POST_ADD2_SCALE, POST_GELU,
                    POST_RELU, TppxError)
-from ._qtensor import QTensor, QSCHEME_MXFP, QSCHEME_AFFINE
+from ._qtensor import DISPATCH, QTensor, QSCHEME_MXFP, QSCHEME_AFFINE
 
 # QINT8_BLOCK_SIZE is read once at import like the reference's file-static
 # (src/csrc/qtypes.cpp:28).
@@ -820,6 +820,9 @@ def _one_launch_group(weights):
                w.weight_kind() == weights[0].weight_kind() for w in weights)
 
 
+OTHER_TYPES = (torch.float32, torch.float16)
+
+
 def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None, post_scale=1.0, flags=0,
            row_sumsq=None, rows=None):
     """One quantized GEMM with a fused post-op
@@ -831,7 +834,7 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
     L = _lib.lib()
     layout = weight.weight_layout() if isinstance(weight, QTensor) else None
     w4a8 = layout is not None and layout[0] == "mxfp4_int8"
-    other_type = isinstance(input, QTensor) or (isinstance(input, torch.Tensor) and input.dtype in (torch.float32, torch.float16))
+    other_type = isinstance(input, QTensor) or (isinstance(input, torch.Tensor) and input.dtype in OTHER_TYPES)
     if other_type and not w4a8:
         if row_sumsq is not None:
             raise TppxError(_lib.EUNSUPPORTED, "row sums of squares need bfloat16 activations")
@@ -845,13 +848,15 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
             raise TppxError(_lib.EUNSUPPORTED, "row sums of squares need an MXFP4 weight in the default layout")
         return _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale)
     x, M, N, K = _prep_input(input, weight, layout)
-    out_shape = tuple(input.shape[:-1]) + (N,)
-    y = torch.empty(out_shape, dtype=torch.bfloat16, device=x.device)
+    y = x.new_empty((*input.shape[:-1], N))
     if M == 0:
         return y
-    bias = _prep_bias(bias, N, x.device)
-    post_in = _prep_post(post_in, M, N, "post-op input", x.device)
-    post_in2 = _prep_post(post_in2, M, N, "second post-op input", x.device)
+    dev = x.device
+    bias = _prep_bias(bias, N, dev)
+    if post_in is not None:
+        post_in = _prep_post(post_in, M, N, "post-op input", dev)
+    if post_in2 is not None:
+        post_in2 = _prep_post(post_in2, M, N, "second post-op input", dev)
     # QINT4 / QINT2 decode steps (up to 64 rows): the codes streamed at their own width and expanded in registers
     # (same bits as the expanded int8 tiles).  TPPX_PACKED_CODES=0 keeps the expanded tiles.
     if PACKED_CODES and M <= 64 and layout[0] in ("qint4", "qint2") and weight.block_size == 256 \
@@ -877,7 +882,8 @@ def linear(input, weight, bias=None, post=POST_NONE, post_in=None, post_in2=None
                                              post, post_scale, flags, ws.data_ptr(), ws.numel(),
                                              row_sumsq.data_ptr(), st))
     elif weight._qscheme == QSCHEME_MXFP:
-        flags, ws = _mxfp4_flags_ws(x, M, K, flags, ws)
+        if ACT_FP8 or flags & _lib.FLAG_ACT_FP8:
+            flags, ws = _mxfp4_flags_ws(x, M, K, flags, ws)
         _lib.check(L.tppx_linear_mxfp4(x.data_ptr(), qn.data_ptr(), sn.data_ptr(), _lib.ptr(bias),
                                        _lib.ptr(post_in), _lib.ptr(post_in2), y.data_ptr(), M, N, K,
                                        post, post_scale, flags, ws.data_ptr(), ws.numel(), st))
@@ -1276,4 +1282,4 @@ for _name, _fn in _IMPLS.items():
     _libdef.impl(_name, _fn, "CompositeExplicitAutograd")
 
 # QTensor.__torch_dispatch__ routes the ops here
-DISPATCH = {getattr(torch.ops.tpp_llm, n).default: f for n, f in _IMPLS.items()}
+DISPATCH.update({getattr(torch.ops.tpp_llm, n).default: f for n, f in _IMPLS.items()})

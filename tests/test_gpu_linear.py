@@ -91,6 +91,26 @@ def test_qint8_few_rows_quantised_in_the_gemm_ring_forms(M, N, K):
     _run("qint8", M, N, K, "add", True, 9100 + M + K)
 
 
+# one to eight channel tiles per workgroup (256, 512, .. tiles and one more; two rounds), ragged last groups, one run of K,
+# fewer runs than waves, one per wave; rows around the eight of two quantization passes
+@pytest.mark.parametrize("M,N,K", [(1, 16, 256), (8, 4096, 512), (9, 4112, 256), (16, 8192, 256), (3, 8208, 768), (8, 12304, 256),
+                                   (16, 16400, 256), (9, 20496, 256), (4, 24592, 256), (16, 32784, 256), (1, 1024, 4096),
+                                   (16, 272, 4096), (7, 8208, 3584), (2, 528, 4352)])
+def test_qint8_few_rows_tile_by_tile(M, N, K):
+    """Up to 16 rows and 4096 input channels: the channel tiles of a workgroup one after the other (and 4352 channels, which
+    are not)."""
+    _run("qint8", M, N, K, "add" if M % 2 else "none", True, 230 + M)
+
+
+def test_qint8_group_of_few_rows_counts_its_workgroups_by_weight():
+    """q/k/v and the first MLP projection as one launch: each weight's last workgroup may be short of tiles."""
+    ops = _ops()
+    ws = [_make("qint8", N, 512, 240 + i)[0] for i, N in enumerate((4096, 272, 272, 16384))]
+    x = randn_bf16((5, 512), 1.0, 250).cuda()
+    for y, w, post in zip(ops.qkv_gemm(x, ws, [None] * 4), ws, (O.POST_NONE,) * 3 + (O.POST_GELU,)):
+        assert torch.equal(y, ops.linear(x, w, None, post))
+
+
 def test_cfg1_mxfp4_fc_plain():
     """M=16, K=N=4096, MXFP4, bias."""
     _run("mxfp4", 16, 4096, 4096, "none", True, 1235)

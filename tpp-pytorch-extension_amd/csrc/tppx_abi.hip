@@ -603,6 +603,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
   }
   p.S = 1;
   SkinnyPlan sp = plan_skinny(M, p.total_tiles, p.units, p.tpb, p.deal, x != nullptr && qbs % 256 == 0);
+  plan_skinny_long(p, sp);
   // 33..64 rows, few channel tiles and a long K: every workgroup would pull all of the int8 activations (M x K)
   // through its CU.  Two K parts of two channel tiles each halve that (measured at N = 4096, 64 rows: K = 11008
   // 20.4 -> 18.5 us, K = 14336 25.1 -> 21.6 us; K = 8192 and shorter lose to the extra pass over the partial sums).

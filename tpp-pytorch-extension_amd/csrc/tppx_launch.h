@@ -148,6 +148,8 @@ hipError_t launch_quant_act_mxfp8(const void* x, int64_t M, int64_t K, void* xq,
 // units = runs of K dealt to waves (DecodeParams::units), tpb / deal as in DecodeParams;
 // can_fuse_quant: bf16 activations at hand and blocks of a multiple of 256 (the in-kernel quantisation's case)
 SkinnyPlan plan_skinny(int64_t M, int total_tiles, int units, int tpb, int deal, bool can_fuse_quant);
+// the quantising form's channel tiles per workgroup where three would take more than one round of workgroups
+void plan_skinny_long(const DecodeParams& p, SkinnyPlan& pl);
 // scale blocks a wave that owns `runs` consecutive runs of K can touch
 int skinny_qint8_blocks_per_wave(int runs, int tpb, int deal, int nblk);
 hipError_t launch_skinny_qint8(DecodeParams& p, const SkinnyPlan& pl, hipStream_t stream);

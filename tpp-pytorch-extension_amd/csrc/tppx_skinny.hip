@@ -1069,6 +1069,14 @@ template <int NTW, int PF, int MAXW, int MINW, int XB, bool BIGB, int WBITS = 8>
 __global__ void __launch_bounds__(MAXW * 64)
 skinny_qint8_fq_kernel(const DecodeParams p) {
   constexpr int G = 8 / WBITS; // K tiles per 16-byte weight load of a lane
+  // PF < 4: a wave has at most one run of K (K up to 4096).  It walks the workgroup's channel tiles one after the other,
+  // PF of them under way (the four K tiles of each), the run's rows in registers: the first products start with the first
+  // tile's arrival, and a launch's code, which every CU fetches anew, is half as long.  1 / 8 / 16 rows against the
+  // form below, us: 1024 channels of 4096 4.8 -> 4.0 / 5.5 -> 4.7 / 7.1 -> 6.7, 4096 of 4096 5.7 -> 5.1 / 6.1 -> 5.4 / 7.6 -> 7.3,
+  // 8192 of 4096 8.5 -> 7.8 / 8.8 -> 7.9 / 9.7 -> 9.1.  As the registers hold PF tiles whatever their number, eight fit, and up to
+  // 2048 tiles run in one round of workgroups (plan_skinny_long).
+  constexpr bool SEQ = WBITS == 8 && PF < 4;
+  static_assert(!SEQ || (PF <= NTW && !BIGB), "whole int8 tiles in blocks of one run");
   static_assert(WBITS == 8 || !BIGB, "the packed formats run 256-wide blocks");
   extern __shared__ __align__(16) float sk_lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1083,11 +1091,12 @@ skinny_qint8_fq_kernel(const DecodeParams p) {
   const unsigned int magic = p.spb_magic;
   auto blk_of_run = [&](int u) { return BIGB ? (int)__umulhi((unsigned int)u, magic) : u; };
 
-  const i32x4* wq[NTW];
-  const float* ws[NTW];
+  constexpr int WP = SEQ ? 1 : NTW;
+  const i32x4* wq[WP];
+  const float* ws[WP];
 #pragma unroll
-  for (int nt = 0; nt < NTW; nt++) {
-    const int64_t lt = min(ltile0 + nt, sg.tiles - 1);
+  for (int nt = 0; nt < WP; nt++) {
+    const int64_t lt = SEQ ? 0 : min(ltile0 + nt, sg.tiles - 1);
     wq[nt] = reinterpret_cast<const i32x4*>(sg.qw) + lt * (KT / G) * 64 + lane;
     ws[nt] = reinterpret_cast<const float*>(sg.sw) + lt * NB * 16 + (lane & 15);
   }
@@ -1119,13 +1128,22 @@ skinny_qint8_fq_kernel(const DecodeParams p) {
   __builtin_amdgcn_sched_barrier(0);
 
   // ring stage = weight tiles + their block scale (see skinny_qint8_kernel)
-  i32x4 wreg[PF][NTW];
-  float sreg[PF][NTW];
+  i32x4 wreg[PF][SEQ ? 4 : NTW]; // (SEQ: the four K tiles of a channel tile)
+  float sreg[PF][WP];
   // (WBITS < 8: `t` counts 16-byte loads = groups of G tiles; t0, t1 are multiples of 4, so of G)
   auto load_stage = [&](int st, int t) {
+    if constexpr (SEQ) { // `t` counts channel tiles of the workgroup; a wave without a run reads the last one, never consumed
+      const int64_t lt = min(ltile0 + t, sg.tiles - 1);
+      const int u = min(u0, NR - 1);
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        wreg[st][j] = __builtin_nontemporal_load(wq[0] + (lt * KT + u * 4 + j) * 64);
+      sreg[st][0] = ws[0][(lt * NB + u) * 16];
+      return;
+    }
     t = max(min(t, t1 / G - 1), 0); // past the end (or a wave without K blocks): re-read a valid tile, never consumed
 #pragma unroll
-    for (int nt = 0; nt < NTW; nt++) {
+    for (int nt = 0; nt < WP; nt++) {
       wreg[st][nt] = __builtin_nontemporal_load(wq[nt] + (int64_t)t * 64);
       sreg[st][nt] = ws[nt][blk_of_run((t * G) >> 2) * 16];
     }
@@ -1134,7 +1152,7 @@ skinny_qint8_fq_kernel(const DecodeParams p) {
   // activations and waits for the whole ring before it lets the quantisation start.
 #pragma unroll
   for (int i = 0; i < PF; i++)
-    load_stage(i, t0 / G + i);
+    load_stage(i, SEQ ? i : t0 / G + i);
   __builtin_amdgcn_sched_barrier(0);
 
   // wave-private LDS: xq [tile][g][M rows][16 B], then sa [unit][16]; the region of the cross-wave reduction
@@ -1226,7 +1244,7 @@ skinny_qint8_fq_kernel(const DecodeParams p) {
       __builtin_amdgcn_sched_barrier(0); // one pass after the other: interleaved, their temporaries spill
   };
   static_for<0, XB>([&](auto PS) { quant_pass(PS, 0); });
-  if (!BIGB)
+  if (!BIGB && !SEQ) // (SEQ: XB passes hold the run of every row)
     for (int base = XB; base * 4 < nitems; base += XB) { // more than 4 * XB items per wave
       static_for<0, XB>([&](auto PS) { load_pass(PS, base); });
       static_for<0, XB>([&](auto PS) { quant_pass(PS, base); });
@@ -1260,7 +1278,28 @@ skinny_qint8_fq_kernel(const DecodeParams p) {
         }
     }
   };
-  if constexpr (WBITS == 8) {
+  if constexpr (SEQ) {
+    if (t0 < t1) {
+      i32x4 xa[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        xa[j] = *reinterpret_cast<const i32x4*>(xq_s + j * 16 * M + xoff);
+      const f32x4 sav = *reinterpret_cast<const f32x4*>(sa_s + (lane >> 4) * 4);
+      static_for<0, NTW>([&](auto NT) {
+        constexpr int nt = decltype(NT)::value, st = nt % PF;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          iacc[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[j], wreg[st][j], iacc[nt], 0, 0, 0);
+        const float swv = sreg[st][0];
+        if constexpr (nt + PF < NTW)
+          load_stage(st, nt + PF);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          facc[nt][0][r] = fmaf((float)iacc[nt][r], sav[r] * swv, facc[nt][0][r]);
+      });
+    }
+  } else if constexpr (WBITS == 8) {
     int t = t0;
     for (; t + 2 * PF <= t1; t += PF) { // branch-free full groups (PF is a multiple of 4): every reload is a real tile
 #pragma unroll
@@ -2728,6 +2767,29 @@ SkinnyPlan plan_skinny(int64_t M, int total_tiles, int units, int tpb, int deal,
   return pl;
 }
 
+// A workgroup of the quantising form fills its CU, so rounds of them stand one behind the other: a start (rows, their
+// quantization, the first weights) and an end (sums over the waves) each, about what two channel tiles take.  Three, four,
+// five, six and eight tiles at 4 rows, us: 32000 channels of 4096 25.9, 23.1, 24.6, 27.3, 22.1; 4096 + 4096 + 4096 + 16384 25.0, 21.2,
+// 24.1, 27.2, 20.4; 16384 16.4, 12.6, 12.9, 13.5, 15.1; 37888 of 3584 30.8, 27.5, 24.6, 26.1, 30.9; 64000 of 4096 50.6, 44.9, 50.2, 45.1,
+// 42.5 (the rule takes the best of each).  At 16 rows 31.6 -> 23.1 for 32000 of 4096.
+void plan_skinny_long(const DecodeParams& p, SkinnyPlan& pl) {
+  if (!pl.fused_quant || pl.ntw != 3 || p.wbits == 4 || p.wbits == 2 || p.tpb != 4 || p.units > 16)
+    return;
+  int best = 1 << 30;
+  for (int n : {3, 4, 5, 6, 8}) {
+    int groups = 0;
+    for (int i = 0; i < p.n_seg; i++)
+      groups += (p.seg[i].tiles + n - 1) / n;
+    const int cost = ((groups + 255) / 256) * (n + 2);
+    if (cost < best) {
+      best = cost;
+      pl.ntw = n;
+    }
+  }
+  const size_t xbytes = (size_t)16 * pl.max_units * (256 * (size_t)p.M + 64), rbytes = (size_t)16 * pl.ntw * 1024;
+  pl.lds_overlap = xbytes + rbytes > 160 * 1024;
+}
+
 int skinny_split_tickets(int n) {
   static std::mutex mu;
   static int cursor = 0;
@@ -2801,11 +2863,27 @@ hipError_t launch_skinny_qint8(DecodeParams& p, const SkinnyPlan& pl, hipStream_
         return sk_launch(skinny_qint8_fq_kernel<1, 4, 16, 16, 6, true>, p, grid, 16, lds, stream);
       return sk_launch(skinny_qint8_fq_kernel<1, 8, 16, 16, 6, true>, p, grid, 16, lds, stream);
     }
+    if (p.units <= 16) { // at most a run per wave: the channel tiles one after the other
+      const auto go = [&](auto NT) {
+        constexpr int n = decltype(NT)::value, pf = n < 3 ? n : 3;
+        return p.M <= 8 ? sk_launch(skinny_qint8_fq_kernel<n, pf, 16, 16, 2, false>, p, grid, 16, lds, stream)
+                        : sk_launch(skinny_qint8_fq_kernel<n, pf, 16, 16, 4, false>, p, grid, 16, lds, stream);
+      };
+      switch (pl.ntw) {
+        case 1: return go(std::integral_constant<int, 1>{});
+        case 2: return go(std::integral_constant<int, 2>{});
+        case 3: return go(std::integral_constant<int, 3>{});
+        case 4: return go(std::integral_constant<int, 4>{});
+        case 5: return go(std::integral_constant<int, 5>{});
+        case 6: return go(std::integral_constant<int, 6>{});
+        default: return go(std::integral_constant<int, 8>{});
+      }
+    }
     if (pl.ntw == 3)
       return sk_launch(skinny_qint8_fq_kernel<3, 4, 16, 16, 2, false>, p, grid, 16, lds, stream);
     if (pl.ntw == 2)
       return sk_launch(skinny_qint8_fq_kernel<2, 4, 16, 16, 4, false>, p, grid, 16, lds, stream);
-    // Up to three K blocks (12 weight tiles) per wave: a ring of four tiles; one of eight would hold most of the
+    // Two or three K blocks (8 or 12 weight tiles) per wave: a ring of four tiles; one of eight would hold most of the
     // wave's K range and only delays its first MFMA (4096 x 4096 at one row 6.9 -> 5.9 us).  With more than 16
     // (row, block) items per wave, six quantisation passes are in flight, so that up to 24 items (8 rows x 3 blocks
     // of the K = 11008 down-projection) are requested before the weight ring and none queues behind it

@@ -111,6 +111,22 @@ def test_qint8_group_of_few_rows_counts_its_workgroups_by_weight():
         assert torch.equal(y, ops.linear(x, w, None, post))
 
 
+# waves with one or two K tiles of 128 (17, 20, 28, 31 in all), one to four channel tiles per workgroup, ragged last groups
+@pytest.mark.parametrize("M,N,K", [(1, 96, 2176), (4, 4128, 2560), (3, 8224, 3584), (2, 12320, 3968), (4, 32, 3584), (5, 96, 3584)])
+def test_mxfp4_few_rows_of_uneven_wave_slices(M, N, K):
+    """Up to 4 rows and K between 2048 and 4096 on the LDS-staged kernel (5 rows: the tile-by-tile one), single, grouped and
+    as the gate/up pair."""
+    ops = _ops()
+    y, _, _, ctx = _run("mxfp4", M, N, K, "add" if M % 2 else "none", True, 260 + M)
+    if N > 4200:
+        return
+    x = ctx[3].cuda()
+    ws = [ctx[0], _make("mxfp4", N, K, 270)[0], _make("mxfp4", 32, K, 271)[0]]
+    for o, w in zip(ops.qkv_gemm(x, ws, [None] * 3), ws):
+        assert torch.equal(o, ops.linear(x, w, None))
+    assert torch.equal(ops.swiglu_gate_up(x, ws[0], ws[1]), ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], None)))
+
+
 def test_cfg1_mxfp4_fc_plain():
     """M=16, K=N=4096, MXFP4, bias."""
     _run("mxfp4", 16, 4096, 4096, "none", True, 1235)

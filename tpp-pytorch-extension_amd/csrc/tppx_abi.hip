@@ -158,7 +158,7 @@ static void set_groups(DecodeParams& p, int tiles_per_group, bool dual) {
 
 // LDS-staged decode kernel (M <= 16): channel tiles per workgroup = the fewest that keep the grid within one round of
 // 256 workgroups (the kernel runs one workgroup per CU).  False when the K slice of a wave does not fit its staging.
-static bool plan_xl(DecodeParams& p, bool dual, int* nt_out) {
+static bool plan_xl(DecodeParams& p, bool dual, int* nt_out, bool uneven = false) {
   const int nt_max = dual ? 3 : 4;
   int nt = 1;
   for (; nt < nt_max; nt++) {
@@ -168,8 +168,9 @@ static bool plan_xl(DecodeParams& p, bool dual, int* nt_out) {
   }
   set_groups(p, nt, dual);
   *nt_out = nt;
-  // staging per wave: 16 rows x 32 chunks of 16 bytes, so at most 2 K tiles per wave and slices of 16 or 32 chunks
-  return p.units <= 32 && (p.units % 16 == 0 || p.units <= 16) && skinny_mxfp4_xl_lds(p.units, nt, dual) <= 160 * 1024;
+  // staging per wave: 16 rows x 32 chunks of 16 bytes, so at most 2 K tiles per wave and slices of 16 or 32 chunks;
+  // uneven: some waves one tile, some two
+  return p.units <= 32 && (uneven || p.units % 16 == 0 || p.units <= 16) && skinny_mxfp4_xl_lds(p.units, nt, dual) <= 160 * 1024;
 }
 
 // K split of the single-kernel decode paths for more than 16 rows: the largest S in {4, 2} (at most max_s) such that
@@ -486,7 +487,9 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
     return TPPX_OK;
   }
   int nt_xl = 1;
-  if (M <= 16 && env_int("TPPX_MXFP4_XL", 1) == 1 && plan_xl(p, dual, &nt_xl)) {
+  // K between 2048 and 4096: up to 4 rows (against the form that keeps 4 rows 2560 x 2560 4.6 -> 3.4 us, 4608 x 3584 5.9 -> 4.6,
+  // 10240 x 2560 6.3 -> 5.7); with 5 to 16 the tile-by-tile kernel is as fast or faster (2560 x 2560 at 8 rows 3.8, here 4.3).
+  if (M <= 16 && env_int("TPPX_MXFP4_XL", 1) == 1 && plan_xl(p, dual, &nt_xl, M <= 4)) {
     TPPX_REQUIRE(!row_sumsq || p.groups <= 256, TPPX_EUNSUPPORTED, "%s: N=%ld needs more than 256 workgroups; the table of row sums has 256 slots", who, (long)segs[0].N);
     return check_hip(launch_skinny_mxfp4_xl(p, nt_xl, dual, stream), who);
   }

@@ -72,6 +72,17 @@ def _attn(F, q, kc, vc, L, mask=None, ws=True):
     return out
 
 
+# one to four 16-byte chunks per thread and their edges, and beyond; a single thread's row
+@pytest.mark.parametrize("K", [8, 2040, 2048, 2056, 4104, 6136, 8192, 8200])
+@pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
+def test_rms_norm_row_lengths(K, gdt):
+    F = _llm()
+    x, g = randn_bf16((3, K), 2.0, 50), (torch.randn(K, generator=torch.Generator().manual_seed(51)) * 0.2 + 1.0).to(gdt)
+    y = F.rms_norm(x.cuda(), g.cuda(), 1e-5).cpu()
+    ref = x.double() * torch.rsqrt((x.double() ** 2).mean(-1, keepdim=True) + 1e-5) * g.double()
+    assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-30).all()  # one rounding to bf16 of a value within 1e-6
+
+
 @pytest.mark.parametrize("kernel", ["auto", "rows", "wide"])
 @pytest.mark.parametrize("B,Nq,Nkv,L,Smax", [(1, 32, 32, 2048, 2304), (3, 8, 2, 77, 128), (2, 4, 4, 1, 64),
                                              (16, 32, 32, 300, 512), (1, 32, 32, 129, 4096), (2, 8, 8, 1000, 1000)])

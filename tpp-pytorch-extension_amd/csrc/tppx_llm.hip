@@ -95,6 +95,70 @@ rms_norm_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma, 
   }
 }
 
+// The same for K up to 8192 (NC = 16-byte chunks per thread, 1 .. 4): row and gamma are requested together and stay in
+// registers, so that only one memory latency stands in the launch's way instead of two.  The same sums in the same order.
+// Rows of 4096, us: 1 2.5 -> 2.1, 16 2.7 -> 2.3, 333 3.1 -> 2.9, 1000 5.2 -> 4.7, 2048 7.6 -> 6.8 (4.9 TB/s, what a copy moves); of
+// 8192, 16 3.5 -> 2.6, 333 5.1 -> 4.2, 2048 15.7 -> 14.5.
+template <bool GAMMA_F32, int NC>
+__global__ void __launch_bounds__(256)
+rms_norm_regs_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma, uint16_t* __restrict__ y, int K, float eps) {
+  __shared__ float red[4];
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const uint4* xr = reinterpret_cast<const uint4*>(x + (int64_t)row * K);
+  uint4* yr = reinterpret_cast<uint4*>(y + (int64_t)row * K);
+  const int nchunk = K >> 3;
+  uint4 w[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) // (threads past the end repeat the last chunk: no branch around a load)
+    w[c] = xr[min(tid + c * 256, nchunk - 1)];
+  float4 g4[NC][2];
+  uint4 gb[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    const int i = min(tid + c * 256, nchunk - 1);
+    if (GAMMA_F32) {
+      g4[c][0] = reinterpret_cast<const float4*>(gamma)[2 * i];
+      g4[c][1] = reinterpret_cast<const float4*>(gamma)[2 * i + 1];
+    } else {
+      gb[c] = reinterpret_cast<const uint4*>(gamma)[i];
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    float f[8];
+    unpack8(w[c], f);
+    if (tid + c * 256 < nchunk) {
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        ss = fmaf(f[e], f[e], ss);
+    }
+  }
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0)
+    red[tid >> 6] = ss;
+  __syncthreads();
+  const float v = ((red[0] + red[1]) + (red[2] + red[3])) * (1.0f / (float)K);
+  const float s = 1.0f / sqrtf(v + eps);
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    if (tid + c * 256 >= nchunk)
+      break;
+    float f[8], g[8];
+    unpack8(w[c], f);
+    if (GAMMA_F32) {
+      g[0] = g4[c][0].x; g[1] = g4[c][0].y; g[2] = g4[c][0].z; g[3] = g4[c][0].w;
+      g[4] = g4[c][1].x; g[5] = g4[c][1].y; g[6] = g4[c][1].z; g[7] = g4[c][1].w;
+    } else {
+      unpack8(gb[c], g);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      f[e] = (f[e] * s) * g[e];
+    yr[tid + c * 256] = pack8(f);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // LayerNorm (lyr_norm, fused_llm_infer.cpp:254-306; LayerNormFwdTPP,
 // xsmm_functors.h:4749-4786): m = mean(x), v = max(mean(x^2) - m^2, 0),
@@ -1826,12 +1890,23 @@ extern "C" int tppx_rms_norm(const void* x, const void* gamma, int gamma_dtype, 
   TPPX_REQUIRE(gamma_dtype == TPPX_DT_F32 || gamma_dtype == TPPX_DT_BF16, TPPX_EINVAL, "tppx_rms_norm: unknown gamma dtype %d", gamma_dtype);
   TPPX_REQUIRE(rows > 0 && rows < ((int64_t)1 << 31) && K > 0 && K % 8 == 0 && K < (1 << 24), TPPX_ESHAPE,
                "tppx_rms_norm: bad shape rows=%ld K=%ld (K must be a multiple of 8)", (long)rows, (long)K);
+  const auto go = [&](auto F32) {
+    constexpr bool f32 = decltype(F32)::value;
+    const dim3 grid((unsigned)rows), block(256);
+    const uint16_t* xp = (const uint16_t*)x;
+    const hipStream_t st = (hipStream_t)stream;
+    switch ((K + 2047) / 2048) {
+      case 1: rms_norm_regs_kernel<f32, 1><<<grid, block, 0, st>>>(xp, gamma, (uint16_t*)y, (int)K, eps); break;
+      case 2: rms_norm_regs_kernel<f32, 2><<<grid, block, 0, st>>>(xp, gamma, (uint16_t*)y, (int)K, eps); break;
+      case 3: rms_norm_regs_kernel<f32, 3><<<grid, block, 0, st>>>(xp, gamma, (uint16_t*)y, (int)K, eps); break;
+      case 4: rms_norm_regs_kernel<f32, 4><<<grid, block, 0, st>>>(xp, gamma, (uint16_t*)y, (int)K, eps); break;
+      default: rms_norm_kernel<f32><<<grid, block, 0, st>>>(xp, gamma, (uint16_t*)y, (int)K, eps);
+    }
+  };
   if (gamma_dtype == TPPX_DT_F32)
-    rms_norm_kernel<true><<<dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream>>>(
-        (const uint16_t*)x, gamma, (uint16_t*)y, (int)K, eps);
+    go(std::true_type{});
   else
-    rms_norm_kernel<false><<<dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream>>>(
-        (const uint16_t*)x, gamma, (uint16_t*)y, (int)K, eps);
+    go(std::false_type{});
   return check_hip(hipGetLastError(), "tppx_rms_norm");
 }
 

@@ -457,6 +457,22 @@ int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* qw_gate,
                       const void* bias_up, void* y, int64_t M, int64_t N,
                       int64_t K, int64_t qbs, int flags, tppx_stream_t stream);
 
+/* tppx_multi_linear_qint8 and tppx_swiglu_qint8 with RMSNorm of the rows (gamma f32 or bf16 [K], 16-byte aligned) in the
+ * quantizer's launch: the bits of tppx_rms_norm followed by those calls.  TPPX_EUNSUPPORTED (before any launch) where that
+ * is not built: blocks other than 256, K above 8192, rows that the GEMM quantizes itself or that are few. */
+int tppx_norm_multi_linear_qint8(const void* x, const void* gamma,
+                                 int gamma_dtype, float eps, void* xq, void* sa,
+                                 const tppx_seg* segs, int n_segs, int64_t M,
+                                 int64_t K, int64_t qbs, int flags, void* ws,
+                                 int64_t ws_bytes, tppx_stream_t stream);
+int tppx_norm_swiglu_qint8(const void* x, const void* gamma, int gamma_dtype,
+                           float eps, void* xq, void* sa, const void* qw_gate,
+                           const void* sw_gate, const void* bias_gate,
+                           const void* qw_up, const void* sw_up,
+                           const void* bias_up, void* y, int64_t M, int64_t N,
+                           int64_t K, int64_t qbs, int flags,
+                           tppx_stream_t stream);
+
 /* 1 where the calls above run n_segs bf16 weights of Ns[i] x K (weight_bytes 2),
  * or the pair of QINT8 weights in blocks of 256 (weight_bytes 1, two equal Ns),
  * over M rows as one launch, 0 where they answer TPPX_EUNSUPPORTED or refuse

@@ -127,6 +127,32 @@ def test_mxfp4_few_rows_of_uneven_wave_slices(M, N, K):
     assert torch.equal(ops.swiglu_gate_up(x, ws[0], ws[1]), ops.fc_mul(x, ws[1], None, ops.fc_silu(x, ws[0], None)))
 
 
+# 17 rows and more behind the operand-order quantizer, 128 and more behind the row-major one; between them, from 65 rows, and
+# for K above 8192 the two launches; one to four chunks of 8 values per thread and their edges; gamma in both types
+@pytest.mark.parametrize("M,K,gdt", [(17, 256, torch.float32), (64, 2304, torch.bfloat16), (40, 4096, torch.float32),
+                                     (100, 1024, torch.float32), (128, 2048, torch.float32), (300, 6144, torch.bfloat16),
+                                     (1100, 512, torch.float32), (130, 8192, torch.float32), (130, 8448, torch.float32),
+                                     (3, 512, torch.float32)])
+def test_qint8_norm_in_the_quantizer(M, K, gdt):
+    """q/k/v and gate/up projections with RMSNorm in front equal rms_norm followed by them: ordinary rows, a row of zeros,
+    rows with an infinity and with a NaN."""
+    ops = _ops()
+    ws = [_make("qint8", N, K, 280 + i)[0] for i, N in enumerate((256, 128, 256))]
+    assert all(w.block_size == 256 for w in ws)
+    g = (torch.randn(K, generator=torch.Generator().manual_seed(283)) * 0.3 + 1.0).to(gdt).cuda()
+    x = randn_bf16((M, K), 2.0, 284)
+    x[1] = 0.0
+    for special in (False, True):
+        if special:
+            x[0, 3], x[2, K - 1] = float("inf"), float("nan")
+        xg = x.cuda()
+        n = ops.rms_norm(xg, g, 1e-5)
+        for y, w in zip(ops.qkv_gemm(xg, ws, [None] * 3, norm=(g, 1e-5)), ops.qkv_gemm(n, ws, [None] * 3)):
+            assert torch.equal(y.view(torch.int16), w.view(torch.int16))
+        y, w = ops.swiglu_gate_up(xg, ws[0], ws[2], norm=(g, 1e-5)), ops.swiglu_gate_up(n, ws[0], ws[2])
+        assert torch.equal(y.view(torch.int16), w.view(torch.int16))
+
+
 def test_cfg1_mxfp4_fc_plain():
     """M=16, K=N=4096, MXFP4, bias."""
     _run("mxfp4", 16, 4096, 4096, "none", True, 1235)

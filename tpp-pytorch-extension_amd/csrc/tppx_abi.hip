@@ -551,7 +551,12 @@ static int run_mxfp4(const char* who, const void* x, const tppx_seg* segs, int n
 
 static int run_qint8(const char* who, const void* x, void* xq, void* sa, const tppx_seg* segs,
                      int n_segs, int64_t M, int64_t K, int64_t qbs, int flags, void* ws,
-                     int64_t ws_bytes, hipStream_t stream, bool dual = false) {
+                     int64_t ws_bytes, hipStream_t stream, bool dual = false, const ActNorm* norm = nullptr) {
+  // norm: RMSNorm of x in the quantizer's launch
+  const auto quantize = [&](int mt) {
+    return norm ? launch_rms_norm_quant_int8(x, *norm, M, K, xq, sa, mt, stream)
+                : launch_quant_act_int8(x, M, K, qbs, xq, sa, mt, stream);
+  };
   // x == NULL: xq / sa already hold quantized activations (the reference's
   // pre-quantized input case, src/csrc/fused_gemm.h:1244-1246)
   int rc = check_common(who, x ? x : xq, M, K, n_segs, flags, ws, ws_bytes);
@@ -589,9 +594,11 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
     group = group && tiled_qint8_takes_groups(t[i]);
   }
   TPPX_REQUIRE(!dual || group, TPPX_EUNSUPPORTED, "%s: M=%ld runs as one launch per weight", who, (long)M);
+  TPPX_REQUIRE(!norm || (qbs == 256 && K <= 8192 && (tiled ? M >= 128 : M > 16) && !reuse && env_int("TPPX_QUANT_ROWS16", 1) != 0),
+               TPPX_EUNSUPPORTED, "%s: M=%ld rows of K=%ld channels are normalised in a launch of their own", who, (long)M, (long)K);
   if (tiled) {
     if (x && !reuse) {
-      rc = check_hip(launch_quant_act_int8(x, M, K, qbs, xq, sa, 0, stream), who);
+      rc = check_hip(quantize(0), who);
       if (rc)
         return rc;
     }
@@ -626,7 +633,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
       p.S = S;
       p.part = (float*)ws;
       p.mt = sp.grid_y * sp.mg;
-      rc = reuse ? TPPX_OK : check_hip(launch_quant_act_int8(x, M, K, qbs, xq, sa, p.mt, stream), who);
+      rc = reuse ? TPPX_OK : check_hip(quantize(p.mt), who);
       if (rc)
         return rc;
       return check_hip(launch_skinny_qint8_nk(p, sp.mg, stream), who);
@@ -643,7 +650,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
     // quantise straight into MFMA operand order: the GEMM then reads one
     // contiguous 1 KiB per operand instead of 16 rows x 64 B
     p.mt = sp.grid_y * sp.mg;
-    rc = reuse ? TPPX_OK : check_hip(launch_quant_act_int8(x, M, K, qbs, xq, sa, p.mt, stream), who);
+    rc = reuse ? TPPX_OK : check_hip(quantize(p.mt), who);
     if (rc)
       return rc;
   }
@@ -930,6 +937,33 @@ extern "C" int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* 
   tppx_seg s[2] = {{qw_gate, sw_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
                    {qw_up, sw_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
   return run_qint8(who, x, xq, sa, s, 2, M, K, qbs, flags, nullptr, 0, (hipStream_t)stream, true);
+}
+
+static int check_norm(const char* who, const void* x, const void* gamma, int gamma_dtype) {
+  TPPX_REQUIRE(x && gamma && aligned16(x) && aligned16(gamma), TPPX_EINVAL, "%s: rows or gamma null or not 16-byte aligned", who);
+  TPPX_REQUIRE(gamma_dtype == TPPX_DT_F32 || gamma_dtype == TPPX_DT_BF16, TPPX_EINVAL, "%s: unknown gamma dtype %d", who, gamma_dtype);
+  return TPPX_OK;
+}
+
+extern "C" int tppx_norm_multi_linear_qint8(const void* x, const void* gamma, int gamma_dtype, float eps, void* xq, void* sa,
+                                            const tppx_seg* segs, int n_segs, int64_t M, int64_t K, int64_t qbs, int flags,
+                                            void* ws, int64_t ws_bytes, tppx_stream_t stream) {
+  const char* who = "tppx_norm_multi_linear_qint8";
+  const int rc = check_norm(who, x, gamma, gamma_dtype);
+  const ActNorm n = {gamma, gamma_dtype, eps};
+  return rc ? rc : run_qint8(who, x, xq, sa, segs, n_segs, M, K, qbs, flags, ws, ws_bytes, (hipStream_t)stream, false, &n);
+}
+
+extern "C" int tppx_norm_swiglu_qint8(const void* x, const void* gamma, int gamma_dtype, float eps, void* xq, void* sa,
+                                      const void* qw_gate, const void* sw_gate, const void* bias_gate, const void* qw_up,
+                                      const void* sw_up, const void* bias_up, void* y, int64_t M, int64_t N, int64_t K,
+                                      int64_t qbs, int flags, tppx_stream_t stream) {
+  const char* who = "tppx_norm_swiglu_qint8";
+  const int rc = check_norm(who, x, gamma, gamma_dtype);
+  const ActNorm n = {gamma, gamma_dtype, eps};
+  tppx_seg s[2] = {{qw_gate, sw_gate, bias_gate, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f},
+                   {qw_up, sw_up, bias_up, nullptr, nullptr, y, N, TPPX_POST_NONE, 1.0f}};
+  return rc ? rc : run_qint8(who, x, xq, sa, s, 2, M, K, qbs, flags, nullptr, 0, (hipStream_t)stream, true, &n);
 }
 
 extern "C" int tppx_multi_linear_mxfp4(const void* x, const tppx_seg* segs,

@@ -617,6 +617,129 @@ quant_act_int8_rows_kernel(const uint16_t* __restrict__ x, int64_t M, int64_t K,
   }
 }
 
+// sum over the wave in tppx_rms_norm's order
+__device__ __forceinline__ float norm_wave_sum(float v) {
+  auto dpp = [](float v, auto CTRL) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(CTRL)::value, 0xf, 0xf, true));
+  };
+  v += dpp(v, std::integral_constant<int, 0xB1>{});  // quad_perm [1,0,3,2]
+  v += dpp(v, std::integral_constant<int, 0x4E>{});  // quad_perm [2,3,0,1]
+  v += dpp(v, std::integral_constant<int, 0x141>{}); // row_half_mirror
+  v += dpp(v, std::integral_constant<int, 0x140>{}); // row_mirror
+  const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
+  const float b = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
+  const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
+  const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
+  return (a + b) + (c + d);
+}
+
+// RMSNorm and the kernel above in one pass: y = bf16((x * rsqrt(mean(x^2) + eps)) * gamma) stays in registers and leaves as
+// int8 values and scales only, the bits of tppx_rms_norm followed by the quantizer.  A workgroup of 256 threads per row, NC
+// chunks of 8 values per thread (K up to 8192); 32 consecutive threads share a block of 256.  Bound by what it reads and
+// writes once (1000 rows of 4096: 4.7 + 4.3 us as two launches, which write and read the normalised row between them).
+template <bool GAMMA_F32, int NC>
+__global__ void __launch_bounds__(256)
+rms_norm_quant_int8_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma, int K, float eps,
+                           int8_t* __restrict__ xq, float* __restrict__ sa, int mt) {
+  __shared__ float red[4];
+  const int64_t m = blockIdx.x;
+  const int tid = threadIdx.x, nchunk = K >> 3, nb = K >> 8;
+  const uint4* xr = reinterpret_cast<const uint4*>(x + m * K);
+  uint4 w[NC], gb[NC];
+  float4 g4[NC][2];
+#pragma unroll
+  for (int c = 0; c < NC; c++) // (threads past the end repeat the last chunk: no branch around a load)
+    w[c] = xr[min(tid + c * 256, nchunk - 1)];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    const int i = min(tid + c * 256, nchunk - 1);
+    if (GAMMA_F32) {
+      g4[c][0] = reinterpret_cast<const float4*>(gamma)[2 * i];
+      g4[c][1] = reinterpret_cast<const float4*>(gamma)[2 * i + 1];
+    } else {
+      gb[c] = reinterpret_cast<const uint4*>(gamma)[i];
+    }
+  }
+  auto unpack = [](const uint4& v, float (&f)[8]) {
+    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      f[2 * i] = bf16_bits_to_f32(d[i] & 0xffffu);
+      f[2 * i + 1] = bf16_bits_to_f32(d[i] >> 16);
+    }
+  };
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    float f[8];
+    unpack(w[c], f);
+    if (tid + c * 256 < nchunk) {
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        ss = fmaf(f[e], f[e], ss);
+    }
+  }
+  ss = norm_wave_sum(ss);
+  if ((tid & 63) == 0)
+    red[tid >> 6] = ss;
+  __syncthreads();
+  const float v = ((red[0] + red[1]) + (red[2] + red[3])) * (1.0f / (float)K);
+  const float s = 1.0f / sqrtf(v + eps);
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    const int i = tid + c * 256;
+    if (i >= nchunk) // (whole blocks of 32 threads: K is a multiple of 256)
+      break;
+    float f[8], g[8];
+    unpack(w[c], f);
+    if (GAMMA_F32) {
+      g[0] = g4[c][0].x; g[1] = g4[c][0].y; g[2] = g4[c][0].z; g[3] = g4[c][0].w;
+      g[4] = g4[c][1].x; g[5] = g4[c][1].y; g[6] = g4[c][1].z; g[7] = g4[c][1].w;
+    } else {
+      unpack(gb[c], g);
+    }
+    float amax = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      f[e] = bf16_bits_to_f32(f32_to_bf16_bits((f[e] * s) * g[e]) & 0xffffu);
+      amax = fmaxf(amax, fabsf(f[e]));
+    }
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1)
+      amax = fmaxf(amax, __shfl_xor(amax, d, 32));
+    const float sc = int8_scale_of(amax), inv = int8_inv_scale(sc);
+    const int b = i >> 5;
+    if ((i & 31) == 0)
+      sa[mt > 0 ? b * (int64_t)mt * 16 + m : m * nb + b] = sc;
+    uint32_t o[2];
+#pragma unroll
+    for (int d = 0; d < 2; d++)
+      o[d] = (uint32_t)(int8_q(f[4 * d], inv) & 0xff) | ((uint32_t)(int8_q(f[4 * d + 1], inv) & 0xff) << 8) |
+             ((uint32_t)(int8_q(f[4 * d + 2], inv) & 0xff) << 16) | ((uint32_t)(int8_q(f[4 * d + 3], inv) & 0xff) << 24);
+    // operand order: half a slot of [K / 64][mt row tiles][4 K groups][16 rows][16 B]; else row-major
+    const int64_t at = mt > 0 ? (((int64_t)(i >> 3) * mt + (m >> 4)) * 64 + ((i >> 1) & 3) * 16 + (m & 15)) * 16 + (i & 1) * 8
+                              : m * K + i * 8;
+    *reinterpret_cast<uint2*>(xq + at) = make_uint2(o[0], o[1]);
+  }
+}
+
+hipError_t launch_rms_norm_quant_int8(const void* x, const ActNorm& n, int64_t M, int64_t K, void* xq, void* sa, int mt,
+                                      hipStream_t stream) {
+  const auto go = [&](auto kern) {
+    TPPX_PLAN_ONLY(kern, dim3((unsigned)M), dim3(256), 0);
+    kern<<<dim3((unsigned)M), dim3(256), 0, stream>>>((const uint16_t*)x, n.gamma, (int)K, n.eps, (int8_t*)xq, (float*)sa, mt);
+    return hipGetLastError();
+  };
+  const bool f32 = n.dtype == TPPX_DT_F32;
+  switch ((K + 2047) / 2048) {
+    case 1: return f32 ? go(rms_norm_quant_int8_kernel<true, 1>) : go(rms_norm_quant_int8_kernel<false, 1>);
+    case 2: return f32 ? go(rms_norm_quant_int8_kernel<true, 2>) : go(rms_norm_quant_int8_kernel<false, 2>);
+    case 3: return f32 ? go(rms_norm_quant_int8_kernel<true, 3>) : go(rms_norm_quant_int8_kernel<false, 3>);
+    case 4: return f32 ? go(rms_norm_quant_int8_kernel<true, 4>) : go(rms_norm_quant_int8_kernel<false, 4>);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 // float / half rows, any block size in 64s: one wave per (row, block), VEC consecutive values per lane and trip (4 where
 // rows lie on 16-byte addresses).  The maximum follows the generic kernel's rule for NaN: |first|, then std::max, so one
 // in the first place sticks and any other is passed over.  Reads the rows twice where a block is longer than

@@ -78,6 +78,8 @@ SIGNATURES = {
     "tppx_linear_qint8_noalloc": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _f32, _i32, _vp],
     "tppx_multi_linear_mxfp4": [_vp, ctypes.POINTER(Seg), _i32, _i64, _i64, _i32, _vp, _i64, _vp],
     "tppx_multi_linear_qint8": [_vp, _vp, _vp, ctypes.POINTER(Seg), _i32, _i64, _i64, _i64, _i32, _vp, _i64, _vp],
+    "tppx_norm_multi_linear_qint8": [_vp, _vp, _i32, _f32, _vp, _vp, ctypes.POINTER(Seg), _i32, _i64, _i64, _i64, _i32, _vp, _i64, _vp],
+    "tppx_norm_swiglu_qint8": [_vp, _vp, _i32, _f32] + [_vp] * 9 + [_i64, _i64, _i64, _i64, _i32, _vp],
     "tppx_swiglu_mxfp4": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp, _i64, _vp],
     "tppx_norm_multi_linear_mxfp4": [_vp, _vp, ctypes.c_float, ctypes.POINTER(Seg), _i32, _i64, _i64, _i32, _vp],
     "tppx_norm_swiglu_mxfp4": [_vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],

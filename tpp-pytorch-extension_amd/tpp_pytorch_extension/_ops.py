@@ -1019,6 +1019,18 @@ def _norm_fusable(norm, scheme, M, K):
     return _norm_fits(norm, scheme, M, K)
 
 
+def _norm_quantizes(norm, weight, M, K):
+    """Can RMSNorm ride in the quantizer's launch in front of a W8A8 GEMM (the library has the last word)?"""
+    gamma = norm[0]
+    return (weight._qscheme != QSCHEME_MXFP and weight.block_size == 256 and M > 16 and K <= 8192
+            and gamma.dtype in (torch.float32, torch.bfloat16) and gamma.numel() == K and gamma.is_cuda
+            and gamma.is_contiguous() and gamma.data_ptr() % 16 == 0)
+
+
+def _gamma_dt(norm):
+    return _lib.DT_F32 if norm[0].dtype == torch.float32 else _lib.DT_BF16
+
+
 def _norm_table(norm):
     return norm[2] if (len(norm) > 2 and norm[2] is not None and NORM_FROM_SUMS) else None
 
@@ -1106,9 +1118,12 @@ def qkv_gemm(input, weights, biases, norm=None):
             return outs
         return [linear(input, w, b, POST_GELU if (len(weights) == 4 and i == 3) else POST_NONE)
                 for i, (w, b) in enumerate(zip(weights, biases))]
+    quant_norm = None
     if norm is not None:
         xin, Min, _, Kin = _prep_input(input, list(weights)[0])
-        if not _norm_fusable(norm, list(weights)[0]._qscheme, Min, Kin):
+        if _norm_quantizes(norm, list(weights)[0], Min, Kin):
+            quant_norm, norm = norm, None
+        elif not _norm_fusable(norm, list(weights)[0]._qscheme, Min, Kin):
             input, norm = rms_norm(input, norm[0], norm[1]), None
     weights = list(weights)
     biases = list(biases) if biases is not None else []
@@ -1161,6 +1176,13 @@ def qkv_gemm(input, weights, biases, norm=None):
     else:
         qbs = weights[0].block_size
         _buf, xq, sa = _qint8_buffer(x, M, K, qbs)
+        if quant_norm is not None:
+            rc = L.tppx_norm_multi_linear_qint8(x.data_ptr(), quant_norm[0].data_ptr(), _gamma_dt(quant_norm), float(quant_norm[1]),
+                                                xq, sa, segs, n, M, K, qbs, 0, ws.data_ptr(), ws.numel(), st)
+            if rc != _lib.EUNSUPPORTED:
+                _lib.check(rc)
+                return outs
+            x = rms_norm(x, quant_norm[0], quant_norm[1])
         _lib.check(L.tppx_multi_linear_qint8(x.data_ptr(), xq, sa, segs, n, M, K,
                                              qbs, 0, ws.data_ptr(), ws.numel(), st))
     return outs
@@ -1185,9 +1207,12 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
         if y is not None:
             return y
         return fc_mul(input, w_up, b_up, fc_silu(input, w_gate, b_gate))
+    quant_norm = None
     if norm is not None:
         _, M0, _, K0 = _prep_input(input, w_gate)
-        if not _norm_fusable(norm, w_gate._qscheme, M0, K0):
+        if M0 > 64 and _norm_quantizes(norm, w_gate, M0, K0):
+            quant_norm, norm = norm, None
+        elif not _norm_fusable(norm, w_gate._qscheme, M0, K0):
             input, norm = rms_norm(input, norm[0], norm[1]), None
     x, M, N, K = _prep_input(input, w_gate)
     x2, M2, N2, K2 = _prep_input(input, w_up)
@@ -1202,12 +1227,23 @@ def swiglu_gate_up(input, w_gate, w_up, b_gate=None, b_up=None, norm=None):
             bg, bu = _prep_bias(b_gate, N, x.device), _prep_bias(b_up, N, x.device)
             (qg, sg), (qu, su) = w_gate.native(), w_up.native()
             _buf, xq, sa = _qint8_buffer(x, M, K, 256)
+            if quant_norm is not None:
+                rc = L.tppx_norm_swiglu_qint8(x.data_ptr(), quant_norm[0].data_ptr(), _gamma_dt(quant_norm), float(quant_norm[1]), xq, sa,
+                                              qg.data_ptr(), sg.data_ptr(), _lib.ptr(bg), qu.data_ptr(), su.data_ptr(), _lib.ptr(bu),
+                                              y.data_ptr(), M, N, K, 256, 0, _lib.stream_of(x))
+                if rc != _lib.EUNSUPPORTED:
+                    _lib.check(rc)
+                    return y
+                x = input = rms_norm(x, quant_norm[0], quant_norm[1])
+                quant_norm = None
             rc = L.tppx_swiglu_qint8(x.data_ptr(), xq, sa, qg.data_ptr(), sg.data_ptr(), _lib.ptr(bg),
                                      qu.data_ptr(), su.data_ptr(), _lib.ptr(bu), y.data_ptr(), M, N, K, 256, 0,
                                      _lib.stream_of(x))
             if rc != _lib.EUNSUPPORTED:
                 _lib.check(rc)
                 return y
+        if quant_norm is not None:
+            input = rms_norm(input, quant_norm[0], quant_norm[1])
         # one quantization of the rows for both projections: the two calls are of one shape, so of one plan and layout of
         # the quantized rows (17 .. 64 rows; up to 16 the GEMM quantizes its rows itself).  Gate, up and down projections of
         # 4096 / 11008 at 32 / 64 rows 47.4 -> 44.7 / 57.7 -> 54.8 us, of 4096 / 4096 33.3 -> 30.6.

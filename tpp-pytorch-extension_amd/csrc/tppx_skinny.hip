@@ -946,7 +946,7 @@ skinny_mxfp4_nk_kernel(const DecodeParams p) {
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int cj = (lane >> 4) * 4 + j;
-    rdo[j] = cj * MPAD + ((lane & 15) ^ swz16(cj));
+    rdo[j] = cj * MPAD + ((lane & 15) ^ cj);
   }
   f32x4 acc[TPW][MG];
 #pragma unroll
@@ -962,7 +962,8 @@ skinny_mxfp4_nk_kernel(const DecodeParams p) {
       i32x4* stage = xs + (size_t)((s & 1) * KPW + kp) * (MPAD * 16);
 #pragma unroll
       for (int it = 0; it < XI; it++)
-        stage[c16 * MPAD + ((wc * (RGW * 16) + it * 4 + r4) ^ swz16(c16))] = xr[xi][it];
+        // (with row ^ swz16(chunk), which reads without bank conflicts, 4096 x 11008 at 50 rows took 17.34 us, so 17.14)
+        stage[c16 * MPAD + ((wc * (RGW * 16) + it * 4 + r4) ^ c16)] = xr[xi][it];
       if (s + XPF < nsteps)
         load_x(xi, s + XPF);
       // one barrier per step: a wave that reaches the barrier of step s + 1 has finished reading the stage of

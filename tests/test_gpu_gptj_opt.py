@@ -49,6 +49,18 @@ def test_layer_norm(K, pdt):
         F.lyr_norm(x.cuda(), g.cuda(), b.float().cuda() if pdt == torch.bfloat16 else b.bfloat16().cuda(), 1e-5)
 
 
+# one to four 16-byte chunks per thread and their edges, shorter rows and longer ones
+@pytest.mark.parametrize("K", [1024, 1032, 2048, 2056, 4104, 6136, 8192, 8200])
+@pytest.mark.parametrize("pdt", [torch.float32, torch.bfloat16])
+def test_layer_norm_row_lengths(K, pdt):
+    F = _gj()
+    rng = torch.Generator().manual_seed(13)
+    x = randn_bf16((3, K), 1.5, 14)
+    g, b = (torch.randn(K, generator=rng) * 0.2 + 1.0).to(pdt), (torch.randn(K, generator=rng) * 0.3).to(pdt)
+    y = F.lyr_norm(x.cuda(), g.cuda(), b.cuda(), 1e-5)
+    assert_close_bf16(t2bits(y), O.layer_norm(t2bits(x), g.float().numpy(), b.float().numpy(), 1e-5), what=f"layer_norm K={K}")
+
+
 @pytest.mark.parametrize("H,HR", [(128, 64), (256, 64), (64, 64), (32, 16), (80, 32), (200, 64)])
 def test_rotary_gptj(H, HR):
     F = _gj()

@@ -221,6 +221,85 @@ layer_norm_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma
   }
 }
 
+// The same for K up to 8192, row and parameters in registers, as rms_norm_regs_kernel.  Rows of 4096, us: 1 2.7 -> 2.1, 16 2.8 -> 2.4,
+// 333 3.4 -> 3.0, 2048 8.5 -> 7.3; of 2560, 2048 6.7 -> 6.2.  (Rows of 1024 and less leave half of the threads idle: 1000 of them 3.0,
+// here 3.1, so they stay with the kernel above.)
+template <bool PARAMS_F32, int NC>
+__global__ void __launch_bounds__(256)
+layer_norm_regs_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma, const void* __restrict__ beta,
+                       uint16_t* __restrict__ y, int K, float eps) {
+  __shared__ float red[2][4];
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const uint4* xr = reinterpret_cast<const uint4*>(x + (int64_t)row * K);
+  uint4* yr = reinterpret_cast<uint4*>(y + (int64_t)row * K);
+  const int nchunk = K >> 3;
+  constexpr int P = PARAMS_F32 ? 2 : 1; // 16-byte words of 8 parameters
+  uint4 w[NC], g4[NC][P], b4[NC][P];
+#pragma unroll
+  for (int c = 0; c < NC; c++) // (threads past the end repeat the last chunk: no branch around a load)
+    w[c] = xr[min(tid + c * 256, nchunk - 1)];
+#pragma unroll
+  for (int c = 0; c < NC; c++)
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      const int i = min(tid + c * 256, nchunk - 1) * P + q;
+      g4[c][q] = reinterpret_cast<const uint4*>(gamma)[i];
+      b4[c][q] = reinterpret_cast<const uint4*>(beta)[i];
+    }
+  auto param = [](const uint4 (&p)[P], float (&f)[8]) {
+    if constexpr (PARAMS_F32) {
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        f[4 * q] = __uint_as_float(p[q].x);
+        f[4 * q + 1] = __uint_as_float(p[q].y);
+        f[4 * q + 2] = __uint_as_float(p[q].z);
+        f[4 * q + 3] = __uint_as_float(p[q].w);
+      }
+    } else {
+      unpack8(p[0], f);
+    }
+  };
+  float sm = 0.f, ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    float f[8];
+    unpack8(w[c], f);
+    if (tid + c * 256 < nchunk) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        sm += f[e];
+        ss = fmaf(f[e], f[e], ss);
+      }
+    }
+  }
+  sm = wave_sum(sm);
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) {
+    red[0][tid >> 6] = sm;
+    red[1][tid >> 6] = ss;
+  }
+  __syncthreads();
+  const float c1 = 1.0f / (float)K;
+  const float m = ((red[0][0] + red[0][1]) + (red[0][2] + red[0][3])) * c1;
+  float v = ((red[1][0] + red[1][1]) + (red[1][2] + red[1][3])) * c1;
+  v = fmaxf(v - m * m, 0.0f);
+  const float s = 1.0f / sqrtf(v + eps);
+  const float b = -1.0f * s * m;
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    if (tid + c * 256 >= nchunk)
+      break;
+    float f[8], g[8], bt[8];
+    unpack8(w[c], f);
+    param(g4[c], g);
+    param(b4[c], bt);
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      f[e] = (f[e] * s + b) * g[e] + bt[e];
+    yr[tid + c * 256] = pack8(f);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Llama rotary embedding, in place on t [B][S][N][H] (rotate-half pairs
 // (h2, HR/2 + h2)), cos/sin table f32 [2][MP][HR], positions i64 [B_pos][S].
@@ -1919,12 +1998,23 @@ extern "C" int tppx_layer_norm(const void* x, const void* gamma, const void* bet
                "tppx_layer_norm: unknown gamma / beta dtype %d", param_dtype);
   TPPX_REQUIRE(rows > 0 && rows < ((int64_t)1 << 31) && K > 0 && K % 8 == 0 && K < (1 << 24), TPPX_ESHAPE,
                "tppx_layer_norm: bad shape rows=%ld K=%ld (K must be a multiple of 8)", (long)rows, (long)K);
+  const auto go = [&](auto F32) {
+    constexpr bool f32 = decltype(F32)::value;
+    const dim3 grid((unsigned)rows), block(256);
+    const uint16_t* xp = (const uint16_t*)x;
+    const hipStream_t st = (hipStream_t)stream;
+    switch (K > 1024 ? (K + 2047) / 2048 : 0) {
+      case 1: layer_norm_regs_kernel<f32, 1><<<grid, block, 0, st>>>(xp, gamma, beta, (uint16_t*)y, (int)K, eps); break;
+      case 2: layer_norm_regs_kernel<f32, 2><<<grid, block, 0, st>>>(xp, gamma, beta, (uint16_t*)y, (int)K, eps); break;
+      case 3: layer_norm_regs_kernel<f32, 3><<<grid, block, 0, st>>>(xp, gamma, beta, (uint16_t*)y, (int)K, eps); break;
+      case 4: layer_norm_regs_kernel<f32, 4><<<grid, block, 0, st>>>(xp, gamma, beta, (uint16_t*)y, (int)K, eps); break;
+      default: layer_norm_kernel<f32><<<grid, block, 0, st>>>(xp, gamma, beta, (uint16_t*)y, (int)K, eps);
+    }
+  };
   if (param_dtype == TPPX_DT_F32)
-    layer_norm_kernel<true><<<dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream>>>(
-        (const uint16_t*)x, gamma, beta, (uint16_t*)y, (int)K, eps);
+    go(std::true_type{});
   else
-    layer_norm_kernel<false><<<dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream>>>(
-        (const uint16_t*)x, gamma, beta, (uint16_t*)y, (int)K, eps);
+    go(std::false_type{});
   return check_hip(hipGetLastError(), "tppx_layer_norm");
 }
 

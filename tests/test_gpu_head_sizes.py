@@ -307,6 +307,61 @@ def test_decode_step_with_rotary_and_append_in_the_launch(H, HR, style, B, Nq, N
         assert torch.equal(out, first)
 
 
+# 128-wide heads: the kernel of long loops, the wide one, the one of grouped heads
+@pytest.mark.parametrize("H,HR,style,Nq,wide", [(128, 128, "llama", 4, "0"), (128, 128, "llama", 4, "1"), (128, 128, "llama", 32, "1"),
+                                                (64, 64, "llama", 4, "1"), (80, 32, "gptj", 4, "1"), (256, 64, "gptj", 4, "1"), (200, 80, "llama", 8, "1")])
+def test_every_rotation_leaves_the_same_key(H, HR, style, Nq, wide, monkeypatch):
+    """The launches that rotate a new key agree in every bit: the second value's product rounded, the first one's fused into
+    it.  The table is made so that each pair's first (even pairs) or second (odd pairs) value nearly cancels and what is left is
+    the products' rounding; the keys are one row scaled by powers of two."""
+    from tpp_pytorch_extension import _lib
+    _llm()
+    monkeypatch.setenv("TPPX_ATTN_WIDE", wide)
+    L = _lib.lib()
+    B, Nkv, Smax, past, MP, pairs = 3, 4 if Nq < 32 else 2, 64, 17, 8, HR // 2
+    g = torch.Generator().manual_seed(HR + H)
+    base = (1.0 + torch.rand(H, generator=g)).to(torch.bfloat16)  # 1 .. 2: all products within a few binades
+    k = base * 2.0 ** torch.randint(-3, 4, (B, Nkv, 1), generator=g).to(torch.bfloat16)
+    i1 = torch.arange(pairs) * 2 if style == "gptj" else torch.arange(pairs)
+    i2 = i1 + (1 if style == "gptj" else pairs)
+    x1, x2 = base[i1].double(), base[i2].double()
+    t = (0.5 + 0.5 * torch.rand(pairs, generator=g)).double().float()
+    even = torch.arange(pairs) % 2 == 0
+    cos = torch.where(even, (x2 * t.double() / x1).float(), t)      # x1 cos - x2 sin ~ 0
+    sin = torch.where(even, t, (-x2 * t.double() / x1).float())     # x2 cos + x1 sin ~ 0
+    table = torch.zeros((MP, HR) if style == "gptj" else (2, MP, HR))
+    if style == "gptj":
+        table[5] = torch.cat([sin, cos])
+    else:
+        table[0, 5], table[1, 5] = torch.cat([cos, cos]), torch.cat([sin, sin])
+    want = k.clone()
+    k1, k2 = k[..., i1].double(), k[..., i2].double()  # (24 + 8 bits: products exact, and so are the sums, in float64)
+    want[..., i1] = (k1 * cos.double() - (k2 * sin.double()).float().double()).float().to(torch.bfloat16)
+    want[..., i2] = (k1 * sin.double() + (k2 * cos.double()).float().double()).float().to(torch.bfloat16)
+    own = (k2 * cos.double() + (k1 * sin.double()).float().double()).float().to(torch.bfloat16)
+    assert (own != want[..., i2]).float().mean() > 0.2  # (the other order is told apart)
+
+    dev = lambda a: a.cuda().contiguous()  # noqa: E731
+    k, v, q, table = dev(k), torch.zeros((B, Nkv, H), dtype=torch.bfloat16, device="cuda"), dev(base.expand(B, Nq, H)), dev(table)
+    kc, vc = (torch.zeros((B, Nkv, Smax, H), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    n, pos = torch.tensor([past], dtype=torch.int32, device="cuda"), torch.full((B, 1), 5, dtype=torch.int64, device="cuda")
+    st, out = _lib.stream_of(k), torch.empty_like(q)
+    cache = (kc.data_ptr(), vc.data_ptr())
+    head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr())
+    tail = (None, 0, n.data_ptr(), out.data_ptr(), B, Nq, Nkv, H, Smax, None, 0, st)
+    if H == 128:
+        _lib.check(L.tppx_attn_decode_rotary(*head, pos.data_ptr(), B, MP, HR, *cache, *tail))
+    else:
+        _lib.check(L.tppx_attn_decode_append(*head, style == "gptj", pos.data_ptr(), B, MP, HR, *cache, *tail))
+    assert torch.equal(kc[:, :, past].cpu(), want)
+    q2, k2 = q.clone(), k.clone()
+    fn = L.tppx_rotary_kv_append_gptj if style == "gptj" else L.tppx_rotary_kv_append_llama
+    kc.zero_()
+    _lib.check(fn(q2.data_ptr(), k2.data_ptr(), v.data_ptr(), table.data_ptr(), pos.data_ptr(), *cache, n.data_ptr(), B, 1, Nq, Nkv, H,
+                  MP, HR, B, Smax, st))
+    assert torch.equal(kc[:, :, past].cpu(), want) and torch.equal(k2.cpu(), want)
+
+
 @pytest.mark.parametrize("H,Nq,Nkv", [(64, 8, 2), (80, 4, 4), (256, 2, 2), (8, 2, 1), (200, 4, 2)])
 @pytest.mark.parametrize("B,L,Smax", [(2, 77, 128), (1, 1000, 1100)])
 def test_decode_step_rounds_the_output_only(H, Nq, Nkv, B, L, Smax):

@@ -369,8 +369,8 @@ rotary_append_kernel(const RotaryParams p) {
       const float* cs = sn + (p.HR >> 1);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        r[2 * e] = a[2 * e] * cs[e] - a[2 * e + 1] * sn[e];
-        r[2 * e + 1] = a[2 * e + 1] * cs[e] + a[2 * e] * sn[e];
+        r[2 * e] = rotate_first(a[2 * e], a[2 * e + 1], cs[e], sn[e]);
+        r[2 * e + 1] = rotate_second(a[2 * e], a[2 * e + 1], cs[e], sn[e]);
       }
       w = pack8(r);
       row[u] = w;
@@ -388,8 +388,8 @@ rotary_append_kernel(const RotaryParams p) {
     const float* sn = p.emb + ((int64_t)p.MP + pp) * p.HR + u * 8;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
-      r0[e] = a[e] * cs[e] - o[e] * sn[e];
-      r1[e] = o[e] * cs[e] + a[e] * sn[e];
+      r0[e] = rotate_first(a[e], o[e], cs[e], sn[e]);
+      r1[e] = rotate_second(a[e], o[e], cs[e], sn[e]);
     }
     w0 = pack8(r0);
     w1 = pack8(r1);
@@ -612,7 +612,7 @@ attn_decode_kernel(const AttnParams p) {
       unpack8(wo, o);
 #pragma unroll
       for (int e = 0; e < 8; e++)
-        r[e] = first ? a[e] * cs[e] - o[e] * sn[e] : a[e] * cs[e] + o[e] * sn[e];
+        r[e] = first ? rotate_first(a[e], o[e], cs[e], sn[e]) : rotate_second(o[e], a[e], cs[e], sn[e]);
       const uint4 out = pack8(r);
       unpack8(out, r); // the rotated row is a bf16 tensor
       return out;
@@ -837,11 +837,11 @@ attn_decode_wide_kernel(const AttnParams p) {
 
   if (ROT) {
     if (wave == 0) {
-      q_s[lane] = (uint16_t)f32_to_bf16_bits(rot ? qx1 * cs - qx2 * sn : qx1);
-      q_s[64 + lane] = (uint16_t)f32_to_bf16_bits(rot ? qx2 * cs + qx1 * sn : qx2);
+      q_s[lane] = (uint16_t)f32_to_bf16_bits(rot ? rotate_first(qx1, qx2, cs, sn) : qx1);
+      q_s[64 + lane] = (uint16_t)f32_to_bf16_bits(rot ? rotate_second(qx1, qx2, cs, sn) : qx2);
       if (has_new) {
-        k_s[lane] = (uint16_t)f32_to_bf16_bits(rot ? kx1 * cs - kx2 * sn : kx1);
-        k_s[64 + lane] = (uint16_t)f32_to_bf16_bits(rot ? kx2 * cs + kx1 * sn : kx2);
+        k_s[lane] = (uint16_t)f32_to_bf16_bits(rot ? rotate_first(kx1, kx2, cs, sn) : kx1);
+        k_s[64 + lane] = (uint16_t)f32_to_bf16_bits(rot ? rotate_second(kx1, kx2, cs, sn) : kx2);
       }
     }
     __syncthreads();
@@ -1336,8 +1336,8 @@ attn_decode_group_kernel(const AttnParams p) {
           const float x1 = bf16_bits_to_f32(((uint32_t)qw[j][d] >> (16 * e)) & 0xffffu);
           const float x2 = bf16_bits_to_f32(((uint32_t)qw[j + 2][d] >> (16 * e)) & 0xffffu);
           const float cv = cs[d >> 1][(d & 1) * 2 + e], sv = sn[d >> 1][(d & 1) * 2 + e];
-          lo[e] = f32_to_bf16_bits(x1 * cv - x2 * sv);
-          hi[e] = f32_to_bf16_bits(x2 * cv + x1 * sv);
+          lo[e] = f32_to_bf16_bits(rotate_first(x1, x2, cv, sv));
+          hi[e] = f32_to_bf16_bits(rotate_second(x1, x2, cv, sv));
         }
         qw[j][d] = (int)(lo[0] | lo[1] << 16);
         qw[j + 2][d] = (int)(hi[0] | hi[1] << 16);
@@ -1383,7 +1383,7 @@ attn_decode_group_kernel(const AttnParams p) {
       const uint16_t* vrow = p.v_new + (int64_t)bkv * 128;
       const float x1 = bf16_bits_to_f32(krow[lane]), x2 = bf16_bits_to_f32(krow[64 + lane]);
       const float cv = rot ? p.emb[pp * 128 + lane] : 1.f, sv = rot ? p.emb[((int64_t)p.MP + pp) * 128 + lane] : 0.f;
-      const uint16_t k1 = (uint16_t)f32_to_bf16_bits(rot ? x1 * cv - x2 * sv : x1), k2 = (uint16_t)f32_to_bf16_bits(rot ? x2 * cv + x1 * sv : x2);
+      const uint16_t k1 = (uint16_t)f32_to_bf16_bits(rot ? rotate_first(x1, x2, cv, sv) : x1), k2 = (uint16_t)f32_to_bf16_bits(rot ? rotate_second(x1, x2, cv, sv) : x2);
       const i32x4 vn = *reinterpret_cast<const i32x4*>(vrow + c * 8);
       uint16_t* const kt = reinterpret_cast<uint16_t*>(st + r * 256);
       kt[((lane >> 3) ^ (r & 15)) * 8 + (lane & 7)] = k1;
@@ -2382,7 +2382,7 @@ attn_hd_step_kernel(const AttnGenParams p) {
   // A wave's loads return in the order of their issue: wave 0 asks for the query and the new key first (dims lane + 64 i)
   constexpr int D = G * J / 8;           // head dims per lane of wave 0
   i32x4 qp[J];
-  float qx[D], qo[D], kx[D], ko[D], cs[D], sn[D]; // value, its pair's other half, cos, signed sin
+  float q1[D], q2[D], k1[D], k2[D], f1[D], f2[D]; // the pair of dim d and what its two values are multiplied with
   bool turned[D];
   if (!APP) {
 #pragma unroll
@@ -2398,20 +2398,20 @@ attn_hd_step_kernel(const AttnGenParams p) {
     for (int i = 0; i < D; i++) {
       const int d = min(lane + 64 * i, H - 1);
       const bool turn = rot && d < p.HR;
-      const bool second = p.gptj ? (d & 1) : d >= half;
+      const bool second = turn && (p.gptj ? (d & 1) : d >= half);
       const int o = !turn ? d : p.gptj ? d ^ 1 : second ? d - half : d + half;
       const int e = p.gptj ? d >> 1 : second ? d - half : d;
-      qx[i] = bf16_bits_to_f32(qrow[d]);
-      qo[i] = bf16_bits_to_f32(qrow[o]);
-      kx[i] = bf16_bits_to_f32(krow[d]);
-      ko[i] = bf16_bits_to_f32(krow[o]);
-      cs[i] = sn[i] = 0.f;
+      q1[i] = bf16_bits_to_f32(qrow[second ? o : d]);
+      q2[i] = bf16_bits_to_f32(qrow[second ? d : o]);
+      k1[i] = bf16_bits_to_f32(krow[second ? o : d]);
+      k2[i] = bf16_bits_to_f32(krow[second ? d : o]);
+      f1[i] = f2[i] = 0.f;
       turned[i] = turn;
       if (turn) {
-        cs[i] = p.gptj ? p.emb[pp * p.HR + half + e] : p.emb[pp * p.HR + e];
-        sn[i] = p.gptj ? p.emb[pp * p.HR + e] : p.emb[((int64_t)p.MP + pp) * p.HR + e];
-        if (!second)
-          sn[i] = -sn[i];
+        const float cs = p.gptj ? p.emb[pp * p.HR + half + e] : p.emb[pp * p.HR + e];
+        const float sn = p.gptj ? p.emb[pp * p.HR + e] : p.emb[((int64_t)p.MP + pp) * p.HR + e];
+        f1[i] = second ? sn : cs;
+        f2[i] = second ? cs : -sn;
       }
     }
   }
@@ -2429,9 +2429,9 @@ attn_hd_step_kernel(const AttnGenParams p) {
       for (int i = 0; i < D; i++) {
         const int d = lane + 64 * i;
         if (d < H) {
-          // (which product is fused is left to chance in a plain sum of two; rotary_append_kernel fuses the cosine's)
-          q_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(qx[i], cs[i], __fmul_rn(qo[i], sn[i])) : qx[i]);
-          k_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(kx[i], cs[i], __fmul_rn(ko[i], sn[i])) : kx[i]);
+          // rotate_first or rotate_second, as one form (the first value's product is the fused one in both)
+          q_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(q1[i], f1[i], __fmul_rn(q2[i], f2[i])) : q1[i]);
+          k_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(k1[i], f1[i], __fmul_rn(k2[i], f2[i])) : k1[i]);
         }
       }
     }

@@ -703,6 +703,28 @@ def test_w4a8_pair_has_the_bits_of_two_calls(M, N, K, bc):
     assert torch.equal(ops.swiglu_gate_up(x.cuda(), gate, up), two(x.cuda(), None, None))
 
 
+# two, three and four row tiles per wave, whole K tiles and quarters that begin and end inside one
+@pytest.mark.parametrize("M,K", [(20, 1024), (40, 2048), (63, 640)])
+@pytest.mark.parametrize("swap", [False, True])
+def test_w4a8_pair_rounds_as_two_calls_where_scales_differ(M, K, swap):
+    """One projection with scales of 2 and more, whose sums are converted and scaled, beside one whose products of weight and
+    row scale are subnormal, where that way rounds once more than the integer sums' float start does: each goes its own way,
+    as in the two calls."""
+    ops = _ops()
+    N = 96
+
+    def make(size, seed):
+        w = (randn_bf16((N, K), 1.0, seed).float() * 2.0 ** size).to(torch.bfloat16)
+        return ops.remap_and_quantize_mxfp4(w.view(N // 16, 16, K // 64, 32, 2).permute(0, 2, 3, 1, 4).contiguous().cuda(), int8_layout=True)
+
+    large, small = make(60, 3750), make(-66, 3751)
+    x = (randn_bf16((M, K), 1.0, 3752).float() * 2.0 ** -60).to(torch.bfloat16).cuda()
+    gate, up = (small, large) if swap else (large, small)
+    want = _w4a8_mid(up, x, None, O.POST_MUL, _w4a8_mid(gate, x, None, O.POST_SILU, None, None, 1.0), None, 1.0)
+    assert want.isfinite().all() and (want != 0).float().mean() > 0.3
+    assert torch.equal(ops._w4a8_pair(x, gate, up, None, None), want)
+
+
 # workgroups of one channel tile (at most 512 of 64 rows) and of two (33 x 16 of 64 rows; 37 tiles: the last one alone),
 # K tiles: less than a step of four, whole steps, a remainder behind them
 @pytest.mark.parametrize("M,N,K,bc", [(64, 48, 384, 64), (130, 272, 1024, 128), (1024, 528, 640, 32), (960, 592, 1920, 64),

@@ -1775,19 +1775,24 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
     return (long)(((uint64_t)(uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2 + 1] << 32) |
                   (uint32_t)xreg[i][mg][j >> 1][(j & 1) * 2]);
   };
-  auto block = [&](int i, int q, int j) {
+  // exact: the sums times the weight scale first, exact for scales below 2 and so with the rounding of a whole tile -- for the
+  // pair's projection whose tile would be one, beside one whose tile is not: each has the bits of a launch of its own
+  auto block = [&](int i, int q, int j, bool exact) {
     const long wb = weights(i, q, j);
-    float wsc[4];
+    float wsc[4], usc[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-      wsc[r] = e8m0_to_f32((uint32_t)sreg[i][q][r] >> (8 * j));
+    for (int r = 0; r < 4; r++) {
+      const float w = e8m0_to_f32((uint32_t)sreg[i][q][r] >> (8 * j));
+      usc[r] = exact ? w : 1.f;
+      wsc[r] = exact ? 1.f : w;
+    }
 #pragma unroll
     for (int mg = 0; mg < MG; mg++) {
       const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, rows(i, mg, j), i32x4{0, 0, 0, 0}, 0, 0, 0);
       const float sav = areg[i][mg][j];
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        facc[q][mg][r] = fmaf((float)acc[r], sav * wsc[r], facc[q][mg][r]);
+        facc[q][mg][r] = fmaf(DUAL ? (float)acc[r] * usc[r] : (float)acc[r], sav * wsc[r], facc[q][mg][r]);
     }
   };
   // A whole K tile whose weight scales are all below 2 (E8M0 bytes 1 .. 127; 0 is a scale of zero in every W4A8 kernel).
@@ -1822,20 +1827,25 @@ skinny_w4a8_mg_kernel(const DecodeParams p) {
   };
   auto consume = [&](int i, int t) {
     const int lo = t == t0 ? first : 0, hi = t == t1 - 1 ? last : 4;
-    uint32_t any = 0;
-#pragma unroll
-    for (int q = 0; q < NP; q++)
+    auto odd = [&](int q) { // a top bit for a scale byte of 0 or from 128 on
+      uint32_t any = 0;
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        any |= (uint32_t)sreg[i][q][r] | ((uint32_t)sreg[i][q][r] - 0x01010101u); // a top bit for a byte of 0 or from 128 on
-    if (!__any((any & 0x80808080u) != 0) && lo == 0 && hi == 4) {
+        any |= (uint32_t)sreg[i][q][r] | ((uint32_t)sreg[i][q][r] - 0x01010101u);
+      return any & 0x80808080u;
+    };
+    if (!__any((odd(0) | odd(NP - 1)) != 0) && lo == 0 && hi == 4) {
       whole_tile(i);
     } else {
+      bool exact[NP];
+#pragma unroll
+      for (int q = 0; q < NP; q++)
+        exact[q] = DUAL && lo == 0 && hi == 4 && !__any(odd(q) != 0);
       static_for<0, 4>([&](auto J) {
         if (decltype(J)::value >= lo && decltype(J)::value < hi) {
 #pragma unroll
           for (int q = 0; q < NP; q++)
-            block(i, q, decltype(J)::value);
+            block(i, q, decltype(J)::value, exact[q]);
         }
       });
     }

@@ -471,8 +471,9 @@ __device__ __forceinline__ uint4 as_uint4(const i32x4& v) {
 
 // Shared end of the single-query kernels.  Threads tid < 128 hold output dimension tid of this workgroup's state: the
 // running max M, the sum Ls and the unnormalised output o.  One split: normalise and store.  Several: store the state;
-// with arrival counters the split that arrives last merges all of them inside the launch.
-__device__ __forceinline__ void attn_finish(const AttnParams& p, int bh, int tid, float M, float Ls, float o) {
+// with arrival counters the split that arrives last merges all of them inside the launch.  hold(): right before the arrival.
+template <typename Hold>
+__device__ __forceinline__ void attn_finish(const AttnParams& p, int bh, int tid, float M, float Ls, float o, Hold&& hold) {
   if (tid < 128) {
     if (p.splits == 1) {
       p.out[(int64_t)bh * 128 + tid] = (uint16_t)f32_to_bf16_bits(Ls > 0.f ? o / Ls : 0.f);
@@ -500,6 +501,7 @@ __device__ __forceinline__ void attn_finish(const AttnParams& p, int bh, int tid
   // target; a workgroup barrier by itself does not wait for the global stores of the other waves), then the
   // barrier, then the ticket, then the device-scope loads of the other splits' results.  Nobody waits for anybody.
   __shared__ int arrived_last;
+  hold();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (tid == 0)
@@ -731,7 +733,7 @@ attn_decode_kernel(const AttnParams p) {
       o = fmaf(w, sacc[i][tid], o);
     }
   }
-  attn_finish(p, bh, tid, M, Ls, o);
+  attn_finish(p, bh, tid, M, Ls, o, [] {});
 }
 
 // ---------------------------------------------------------------------------
@@ -981,7 +983,17 @@ attn_decode_wide_kernel(const AttnParams p) {
       o = fmaf(wt, so, o);
     }
   }
-  attn_finish(p, bh, tid, M, Ls, o);
+  // A workgroup without keys gets here with its rows still on their way.  Their registers stay taken until its state is
+  // stored: the first reuse of one would wait for all of them in front of the sums over the waves, and the last of the nine
+  // or so workgroups of a head would arrive that much later (32 heads, 130 keys of 2048: 7.36 us, so 6.99; 12 of 64, 4 x 300 of 1024: 5.91, so 5.60).
+  auto hold = [&] {
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        asm volatile("" : : "v"(kr[s][j]), "v"(vr[s][j]), "v"(qp[j]));
+  };
+  attn_finish(p, bh, tid, M, Ls, o, hold);
 }
 
 __global__ void __launch_bounds__(128)
@@ -2592,6 +2604,11 @@ attn_hd_step_kernel(const AttnGenParams p) {
     return;
   // as in attn_finish: own stores acknowledged, barrier, ticket, then the device-scope loads; nobody waits for anybody
   __shared__ int arrived_last;
+#pragma unroll
+  for (int u = 0; u < NU; u++)
+#pragma unroll
+    for (int j = 0; j < J; j++)
+      asm volatile("" : : "v"(kr[u][j]), "v"(vr[u][j]), "v"(qp[j])); // (see attn_decode_wide_kernel)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (tid == 0)

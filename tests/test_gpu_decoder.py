@@ -83,6 +83,15 @@ def test_rms_norm_row_lengths(K, gdt):
     assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-30).all()  # one rounding to bf16 of a value within 1e-6
 
 
+@pytest.mark.parametrize("K", [8, 256, 1016, 1024, 1032])
+def test_rms_norm_has_the_same_bits_for_few_and_many_rows(K):
+    """Rows of up to 1024 run on one kernel up to 512 of them and on another beyond; the same sums in the same order."""
+    F = _llm()
+    g = (torch.randn(K, generator=torch.Generator().manual_seed(52)) * 0.2 + 1.0).cuda()
+    x = randn_bf16((600, K), 2.0, 53).cuda()
+    assert torch.equal(F.rms_norm(x, g, 1e-5), torch.cat([F.rms_norm(x[:512], g, 1e-5), F.rms_norm(x[512:], g, 1e-5)]))
+
+
 @pytest.mark.parametrize("kernel", ["auto", "rows", "wide"])
 @pytest.mark.parametrize("B,Nq,Nkv,L,Smax", [(1, 32, 32, 2048, 2304), (3, 8, 2, 77, 128), (2, 4, 4, 1, 64),
                                              (16, 32, 32, 300, 512), (1, 32, 32, 129, 4096), (2, 8, 8, 1000, 1000)])

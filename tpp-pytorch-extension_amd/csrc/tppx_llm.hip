@@ -98,7 +98,11 @@ rms_norm_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma, 
 // The same for K up to 8192 (NC = 16-byte chunks per thread, 1 .. 4): row and gamma are requested together and stay in
 // registers, so that only one memory latency stands in the launch's way instead of two.  The same sums in the same order.
 // Rows of 4096, us: 1 2.5 -> 2.1, 16 2.7 -> 2.3, 333 3.1 -> 2.9, 1000 5.2 -> 4.7, 2048 7.6 -> 6.8 (4.9 TB/s, what a copy moves); of
-// 8192, 16 3.5 -> 2.6, 333 5.1 -> 4.2, 2048 15.7 -> 14.5.
+// 8192, 16 3.5 -> 2.6, 333 5.1 -> 4.2, 2048 15.7 -> 14.5.  Many rows of up to 1024 leave half of the threads or more to ask for the
+// last chunk and its gamma again, and those run on the kernel above (f32 gamma, 8192 rows of 256 / 1024: 4.5 / 6.8 there, here
+// 5.3 / 7.1; 1000 of 512 2.22, 2.30; 200 of 1024 2.11 either way, 16 2.04, here 1.90).  Waves past the end without requests, behind a
+// branch: 2048 rows of 4096 5.6 -> 6.0, 1000 of 8192 5.8 -> 6.4.  2048 rows of 2304 and 2560 with f32 gamma lose 3 %, 1000 and 4096
+// of them do not.
 template <bool GAMMA_F32, int NC>
 __global__ void __launch_bounds__(256)
 rms_norm_regs_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma, uint16_t* __restrict__ y, int K, float eps) {
@@ -1986,7 +1990,7 @@ extern "C" int tppx_rms_norm(const void* x, const void* gamma, int gamma_dtype, 
     const dim3 grid((unsigned)rows), block(256);
     const uint16_t* xp = (const uint16_t*)x;
     const hipStream_t st = (hipStream_t)stream;
-    switch ((K + 2047) / 2048) {
+    switch (K > 1024 || rows <= 512 ? (K + 2047) / 2048 : 0) {
       case 1: rms_norm_regs_kernel<f32, 1><<<grid, block, 0, st>>>(xp, gamma, (uint16_t*)y, (int)K, eps); break;
       case 2: rms_norm_regs_kernel<f32, 2><<<grid, block, 0, st>>>(xp, gamma, (uint16_t*)y, (int)K, eps); break;
       case 3: rms_norm_regs_kernel<f32, 3><<<grid, block, 0, st>>>(xp, gamma, (uint16_t*)y, (int)K, eps); break;

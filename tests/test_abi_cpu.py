@@ -356,6 +356,11 @@ def test_kernel_family_of_short_prompts():
         assert not any(small in one(*shape) for small in ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,")), shape
     assert "<3, 2, 4," not in qkv(2048, 1856, 13312) and "<4, 2, 4," not in pair(2048, 2880, 7168)
 
+    # the wave tiles of up to 80 rows drift from 18 row blocks on, in more than a round of workgroups and without rectangles
+    assert "<6, 3, 8," in one(1978, 3136, 10240)                                                    # 111 us (80 x 128: 127)
+    for M, N, K in ((1740, 4160, 9216), (1990, 3136, 12288), (1850, 2112, 6400)):
+        assert not any(small in one(M, N, K) for small in ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,", "<5, 2, 4,")), (M, N, K)
+
     def per_weight(M, N, K, weight_bytes):
         return not L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, weight_bytes)
 

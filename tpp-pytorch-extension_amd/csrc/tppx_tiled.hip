@@ -1417,6 +1417,26 @@ static int xcd_split(int64_t mb, int64_t nb, double a_bytes, double w_bytes) {
 }
 
 constexpr double MXFP4_WEIGHT_BYTES = 0.53;
+
+// What the fits above do not have; a factor on tile_us.
+// MXFP4, the wave tiles of up to 80 rows, more than a round of workgroups: without a split along M an XCD walks whole columns, and
+// the columns of the workgroups that are resident together drift apart in K.  Against the estimate, with a split and up to 17 row
+// blocks 0.92, 22 1.08, 25 1.12, from 28 on 1.15 .. 1.24; no such drift on the larger tiles.  1978 x 3136 x 10240 127.5 us, with it
+// (96 x 384) 111.5; on 100 shapes of 390 .. 2048 rows with every tile forced the tile taken is 0.4 % off the fastest on average, 0.5
+// without, 7.6 % in the worst case, 14 without.
+// bf16, a single row block, all weights from memory once: 128 x 256 takes 1.13 of the estimate (1.3 in more than a round), 96 x 128
+// in more than a round, where the last workgroups have the chip alone, 1.27, 96 x 256 1.2.  q/k/v of 3 x 10944 x 2304 at 93 rows
+// 47.6 us, with it 40.0; 33024 x 5376 at 95 rows 103.6, 86.0; on 48 shapes 0.7 % off the fastest on average, 2.3 without.
+template <bool WBF16>
+static double tile_factor(int tile, int64_t mb, double s, int64_t wgs, int xm) {
+  const bool more = wgs > 256;
+  if (WBF16)
+    return mb > 1 ? 1.0 : tile == TILE_128_256 ? (more ? 1.3 : 1.1) : tile < TILE_WIDE || !more ? 1.0 : tile_cols16(tile) == 8 ? 1.25 : 1.2;
+  if (tile < TILE_WIDE || tile_cols16(tile) != 8 || !more || xm != 1)
+    return 1.0;
+  return 1.0 + std::max(0.0, std::min(0.33, 0.03 * (double)(mb - 17))) * std::min(1.0, std::max(0.0, (s - 8.0) / 12.0));
+}
+
 // the tiles a launch may take, one bit each
 template <bool WBF16>
 static unsigned big_tiles() {
@@ -1450,7 +1470,7 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
     all += tiles[i];
   const double s = (double)(K / 128), mb = (double)(all * 32 * K) * 1e-6;
   int shape = 0;
-  double best = 1e300;
+  double best = 1e300, us = 1e300; // (us: without tile_factor, as the decode kernels' estimates were weighed against it)
   *S = 1;
   for (int i = 0; i < N_TILES; i++) {
     if (!(allowed >> i & 1u) || (WBF16 && i >= TILE_WIDE && all < 48)) // (fewer than 768 channels: not measured)
@@ -1459,9 +1479,11 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
     int64_t nb = 0;
     for (int g = 0; g < (dual ? 1 : n); g++)
       nb += (tiles[g] + tpw - 1) / tpw;
-    const int64_t wgs = (M + tile_rows(i) - 1) / tile_rows(i) * nb;
+    const int64_t rows = (M + tile_rows(i) - 1) / tile_rows(i), wgs = rows * nb;
     // (a near tie goes to the large tiles, which read less)
     double c = tile_us(COST[i], i, wgs, s, mb, dual) * (i >= TILE_64_128 && i != TILE_64_256 ? 1.01 : 1.0);
+    us = std::min(us, c);
+    c *= tile_factor<WBF16>(i, rows, s, wgs, xcd_split(rows, nb, (double)M, (double)nb * tile_cols16(i) * (WBF16 ? 16.0 : 8.0 * MXFP4_WEIGHT_BYTES)));
     if (c < best && !(forced > 1 && *S > 1)) {
       best = c;
       shape = i;
@@ -1475,6 +1497,7 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
       c = tile_us(COST[i], i, wgs * z, s / z, mb, false) + COST[i].c0 + COST[i].c1 * (double)(wgs * z * slice_bytes(i)) / 32768.0;
       c *= !WBF16 ? 1.03 : wgs <= 256 ? 1.05 : 1.10;
       if (forced == z ? *S != z || c < best : forced == 1 && c < best) {
+        us = std::min(us, c);
         best = c;
         shape = i;
         *S = z;
@@ -1482,7 +1505,7 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
     }
   }
   if (best_us)
-    *best_us = best;
+    *best_us = us;
   return shape;
 }
 

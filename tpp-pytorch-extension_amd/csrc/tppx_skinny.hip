@@ -2075,9 +2075,11 @@ skinny_w4a8_rows_kernel(const DecodeParams p) {
 // row-contiguous 16-byte loads (a wave instruction covers whole 256-byte row
 // segments; the operand-shaped reads of the register path touch 16 cache
 // lines per 16 lanes) and writes it to its private LDS region as
-// [chunk][row ^ swz16(chunk)] x 16 B: conflict free on the way in and as MFMA
-// operand reads (lane = row, 4 K groups) on the way out.  The main loop then
-// streams only weights.  RMSNorm needs the whole row: the 16 waves exchange
+// [chunk][row ^ (chunk & 15)] x 16 B: conflict free on the way in; the MFMA
+// operand reads (lane = row, 4 K groups) on the way out take two turns at the
+// banks (row ^ swz16(chunk), one turn, measured the same: 16 shapes of up to 16
+// rows 1.001 in the mean, 0.97 .. 1.03).  The main loop then streams only
+// weights.  RMSNorm needs the whole row: the 16 waves exchange
 // per-(row, K tile) partial sums of squares through LDS and add them in a
 // fixed order.  The reduction scratch of the epilogue reuses the x regions.
 // ---------------------------------------------------------------------------
@@ -2256,9 +2258,9 @@ skinny_mxfp4_xl_kernel(const DecodeParams p) {
         const float hi = (bf16_bits_to_f32(d >> 16) * sc) * (e < 2 ? gm0[2 * e + 1] : gm1[2 * e - 3]);
         o[e] = (int)sk_pack_bf16(lo, hi);
       }
-      *reinterpret_cast<i32x4*>(&xs[ck * 16 + (row ^ swz16(ck))]) = o;
+      *reinterpret_cast<i32x4*>(&xs[ck * 16 + (row ^ (ck & 15))]) = o;
     } else {
-      *reinterpret_cast<i32x4*>(&xs[ck * 16 + (row ^ swz16(ck))]) = raw[it];
+      *reinterpret_cast<i32x4*>(&xs[ck * 16 + (row ^ (ck & 15))]) = raw[it];
     }
   });
   if (XMODE == 1) {
@@ -2279,7 +2281,7 @@ skinny_mxfp4_xl_kernel(const DecodeParams p) {
 #pragma unroll 1
     for (int i = lane; i < items; i += 64) {
       const int row = i >> nsh, ck = i & cmask;
-      i32x4* slot = reinterpret_cast<i32x4*>(&xs[ck * 16 + (row ^ swz16(ck))]);
+      i32x4* slot = reinterpret_cast<i32x4*>(&xs[ck * 16 + (row ^ (ck & 15))]);
       const i32x4 w = *slot;
       const float sc = srow[row];
       i32x4 o;
@@ -2313,7 +2315,7 @@ skinny_mxfp4_xl_kernel(const DecodeParams p) {
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int cj = (lane >> 4) * 4 + j;
-    rdo[j] = cj * 16 + ((lane & 15) ^ swz16(cj));
+    rdo[j] = cj * 16 + ((lane & 15) ^ cj);
   }
   auto consume = [&](int i, int tl) {
     bf16x8 xa[4];
@@ -2356,7 +2358,7 @@ skinny_mxfp4_xl_kernel(const DecodeParams p) {
 // ---------------------------------------------------------------------------
 // MXFP4 weight-only, up to 4 rows, long K (the Llama down-projection of a
 // batch-1 decode step): the LDS-staged kernel above with only the 4 rows kept
-// -- slot (chunk g*4 + j, row) = (j*4 + g)*4 + (row ^ j): four g side by side, on all the banks; the 16 MFMA rows read
+// -- slot (chunk, row) = chunk*4 + (row ^ (chunk & 3)); the 16 MFMA rows read
 // row m & 3 -- so that K up to 16384 fits (cht KiB per wave instead of 4*cht).
 // Sixteen waves split K; x and the weight ring are requested as there.
 // ---------------------------------------------------------------------------
@@ -2422,7 +2424,7 @@ skinny_mxfp4_x4_kernel(const DecodeParams p) {
     const i32x4 v = raw[it];
     const int row = it >> 1, ck = (it & 1) * 64 + lane2;
     if (row < p.M && ck < nch)
-      xs[(ck & ~15) * 4 + ((ck & 3) * 4 + (ck >> 2 & 3)) * 4 + (row ^ (ck & 3))] = v;
+      xs[ck * 4 + (row ^ (ck & 3))] = v;
   });
   // the wave reads only what it wrote itself: program order is enough
 
@@ -2436,7 +2438,8 @@ skinny_mxfp4_x4_kernel(const DecodeParams p) {
   int rdo[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    rdo[j] = (j * 4 + (lane >> 4)) * 4 + ((lane & 3) ^ j);
+    const int cj = (lane >> 4) * 4 + j;
+    rdo[j] = cj * 4 + ((lane & 3) ^ (cj & 3));
   }
   auto consume = [&](int i, int tl) {
     bf16x8 xa[4];
@@ -2483,8 +2486,9 @@ skinny_mxfp4_x4_kernel(const DecodeParams p) {
 // [N/16][K/128][4 j][64 lanes][16 B]: four 1 KB loads per K tile and wave.  W waves split K.  A wave walks its K tiles in units of UG row groups: the bf16 activations of a unit
 // (UG*16 rows x 256 B) go straight from global memory to one of the two slots of the wave's private LDS region, no
 // registers in between, and are read back as A operands; the weights of two K tiles are in registers or under way.
-// LDS image of a row group: row r at r*256, its 16-byte chunk c at (c ^ swz16(r))*16 -- a load instruction fills four rows
-// from eight whole 128-byte lines, and operand reads fall on all the banks.
+// LDS image of a row group: row r at r*256, its 16-byte chunk c at (c ^ r)*16 -- a load instruction fills four rows from eight
+// whole 128-byte lines.  (c ^ swz16(r), whose operand reads have no bank conflicts, took as long -- 42 shapes of both weights
+// within 1 %, 1.00 in the mean -- and three channel tiles of bf16 weights spilled 60 registers instead of 56.)
 // No barrier before the final cross-wave reduction, whose scratch reuses the activation regions.
 // What bounds it: at 50 rows of a 4096 -> 2 x 11008 pair the loop's 768 MFMAs per SIMD are 7 us and the 720 KB a CU takes
 // in 6, side by side; the rest of 20.3 us is the launch, the first loads' latency, and the sums over the waves.  Activations
@@ -2544,7 +2548,7 @@ __device__ __forceinline__ void skinny_rows_body(const DecodeParams& p) {
     for (int i = 0; i < NX; i++) {
       const int row = min(decltype(H)::value * UG * 16 + i * 4 + r, mlast); // (row and K are below 2^24)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(xs + (slot * NX + i) * 1024), 16,
-                                               (__umul24((uint32_t)row * 2u, (uint32_t)p.K) + (uint32_t)((c ^ swz16((i & 3) * 4 + r)) * 16)), t * 256, 0, 0);
+                                               (__umul24((uint32_t)row * 2u, (uint32_t)p.K) + (uint32_t)((c ^ ((i & 3) * 4 + r)) * 16)), t * 256, 0, 0);
     }
   };
   i32x4 wreg[2][NTW][BJ];
@@ -2563,7 +2567,7 @@ __device__ __forceinline__ void skinny_rows_body(const DecodeParams& p) {
   uint32_t rdo[4]; // operand of this lane for step j: chunk g*4 + j of row m
 #pragma unroll
   for (int j = 0; j < 4; j++)
-    rdo[j] = (lane & 15) * 256 + ((((lane >> 4) * 4 + j) ^ swz16(lane)) * 16);
+    rdo[j] = (lane & 15) * 256 + ((((lane >> 4) * 4 + j) ^ (lane & 15)) * 16);
 
   // post-op inputs early, except where registers are scarcest (the gate/up pair has none but its biases)
   constexpr bool LATE_EP = DUAL && MG == 4;

@@ -459,7 +459,7 @@ int tppx_swiglu_qint8(const void* x, void* xq, void* sa, const void* qw_gate,
 
 /* tppx_multi_linear_qint8 and tppx_swiglu_qint8 with RMSNorm of the rows (gamma f32 or bf16 [K], 16-byte aligned) in the
  * quantizer's launch: the bits of tppx_rms_norm followed by those calls.  TPPX_EUNSUPPORTED (before any launch) where that
- * is not built: blocks other than 256, K above 8192, rows that the GEMM quantizes itself or that are few. */
+ * is not built: blocks other than 256, K above 8192, up to 16 rows, which the GEMM quantizes itself. */
 int tppx_norm_multi_linear_qint8(const void* x, const void* gamma,
                                  int gamma_dtype, float eps, void* xq, void* sa,
                                  const tppx_seg* segs, int n_segs, int64_t M,

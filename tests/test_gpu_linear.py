@@ -153,6 +153,45 @@ def test_qint8_norm_in_the_quantizer(M, K, gdt):
         assert torch.equal(y.view(torch.int16), w.view(torch.int16))
 
 
+@pytest.mark.parametrize("M,K", [(3, 512), (17, 512), (64, 1024), (65, 512), (100, 2048), (127, 1024), (128, 512), (300, 1024), (130, 8448)])
+def test_qint8_norm_in_the_quantizer_is_one_launch_where_it_is_built(M, K, monkeypatch):
+    """From 17 rows on (the pair: from 65, as one launch) and up to 8192 input channels the normalisation is part of the
+    quantizer's launch; the library refuses none of those calls, and rms_norm runs once in front of the others.  The bits of
+    the two launches, for rows of zeros, with an infinity and with a NaN too."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    ops = _ops()
+    ws = [_make("qint8", 2048, K, 286 + i)[0] for i in range(2)]
+    x, g = randn_bf16((M, K), 2.0, 288), torch.ones(K, device="cuda")
+    x[0], x[1, 3], x[2, K - 1] = 0.0, float("inf"), float("nan")
+    x = x.cuda()
+    n = ops.rms_norm(x, g, 1e-5)
+    want = [list(ops.qkv_gemm(n, ws, [None] * 2)), [ops.swiglu_gate_up(n, *ws)]]
+    answers, norms, lib, rms = [], [], _lib.lib(), ops.rms_norm
+
+    class Watch:
+        def __getattr__(self, name):
+            f = getattr(lib, name)
+            if "_norm_" not in name:
+                return f
+
+            def call(*args):
+                rc = f(*args)
+                answers.append(rc)
+                return rc
+            return call
+
+    monkeypatch.setattr(_lib, "lib", lambda: Watch())
+    monkeypatch.setattr(ops, "rms_norm", lambda *a: norms.append(1) or rms(*a))
+    pair = M > 64 and lib.tppx_group_is_one_launch((ctypes.c_int64 * 2)(2048, 2048), 2, M, K, 1)
+    for call, fused, ref in ((lambda n: list(ops.qkv_gemm(x, ws, [None] * 2, norm=n)), M > 16 and K <= 8192, want[0]),
+                             (lambda n: [ops.swiglu_gate_up(x, *ws, norm=n)], pair and K <= 8192, want[1])):
+        answers.clear(), norms.clear()
+        for y, w in zip(call((g, 1e-5)), ref):
+            assert torch.equal(y.view(torch.int16), w.view(torch.int16))
+        assert answers == [0] * fused and len(norms) == 1 - fused, (answers, norms)
+
+
 def test_cfg1_mxfp4_fc_plain():
     """M=16, K=N=4096, MXFP4, bias."""
     _run("mxfp4", 16, 4096, 4096, "none", True, 1235)

@@ -594,7 +594,7 @@ static int run_qint8(const char* who, const void* x, void* xq, void* sa, const t
     group = group && tiled_qint8_takes_groups(t[i]);
   }
   TPPX_REQUIRE(!dual || group, TPPX_EUNSUPPORTED, "%s: M=%ld runs as one launch per weight", who, (long)M);
-  TPPX_REQUIRE(!norm || (qbs == 256 && K <= 8192 && (tiled ? M >= 128 : M > 16) && !reuse && env_int("TPPX_QUANT_ROWS16", 1) != 0),
+  TPPX_REQUIRE(!norm || (qbs == 256 && K <= 8192 && M > 16 && !reuse && env_int("TPPX_QUANT_ROWS16", 1) != 0),
                TPPX_EUNSUPPORTED, "%s: M=%ld rows of K=%ld channels are normalised in a launch of their own", who, (long)M, (long)K);
   if (tiled) {
     if (x && !reuse) {

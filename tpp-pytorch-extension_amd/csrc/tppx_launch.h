@@ -138,8 +138,7 @@ hipError_t allow_dynamic_lds(const void* kern, size_t lds);
 // dynamic activation quantisation; mt > 0 writes xq in MFMA operand order (see DecodeParams::mt)
 hipError_t launch_quant_act_int8_wide(const void* x, int dtype, int64_t M, int64_t K, int64_t qbs, void* xq, void* sa,
                                       hipStream_t stream);
-// RMSNorm in front of the quantizer, in its launch: blocks of 256, K up to 8192; the bits of the two launches where
-// launch_quant_act_int8 takes its many-rows form (from 128 rows, or mt > 0)
+// RMSNorm in front of the quantizer, in its launch: blocks of 256, K up to 8192; the bits of the two launches
 struct ActNorm {
   const void* gamma;
   int dtype; // TPPX_DT_F32 or TPPX_DT_BF16

@@ -637,10 +637,11 @@ __device__ __forceinline__ float norm_wave_sum(float v) {
 // int8 values and scales only, the bits of tppx_rms_norm followed by the quantizer.  A workgroup of 256 threads per row, NC
 // chunks of 8 values per thread (K up to 8192); 32 consecutive threads share a block of 256.  Bound by what it reads and
 // writes once (1000 rows of 4096: 4.7 + 4.3 us as two launches, which write and read the normalised row between them).
+// all_nan: a block of nothing but NaN has a NaN scale, as in quant_act_int8_kernel; else a scale of zero, as in the kernel above.
 template <bool GAMMA_F32, int NC>
 __global__ void __launch_bounds__(256)
 rms_norm_quant_int8_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma, int K, float eps,
-                           int8_t* __restrict__ xq, float* __restrict__ sa, int mt) {
+                           int8_t* __restrict__ xq, float* __restrict__ sa, int mt, bool all_nan) {
   __shared__ float red[4];
   const int64_t m = blockIdx.x;
   const int tid = threadIdx.x, nchunk = K >> 3, nb = K >> 8;
@@ -698,12 +699,13 @@ rms_norm_quant_int8_kernel(const uint16_t* __restrict__ x, const void* __restric
     } else {
       unpack(gb[c], g);
     }
-    float amax = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
+    for (int e = 0; e < 8; e++)
       f[e] = bf16_bits_to_f32(f32_to_bf16_bits((f[e] * s) * g[e]) & 0xffffu);
+    float amax = all_nan ? fabsf(f[0]) : 0.f; // (a maximum passes over NaN where there is anything else)
+#pragma unroll
+    for (int e = 0; e < 8; e++)
       amax = fmaxf(amax, fabsf(f[e]));
-    }
 #pragma unroll
     for (int d = 1; d < 32; d <<= 1)
       amax = fmaxf(amax, __shfl_xor(amax, d, 32));
@@ -727,7 +729,8 @@ hipError_t launch_rms_norm_quant_int8(const void* x, const ActNorm& n, int64_t M
                                       hipStream_t stream) {
   const auto go = [&](auto kern) {
     TPPX_PLAN_ONLY(kern, dim3((unsigned)M), dim3(256), 0);
-    kern<<<dim3((unsigned)M), dim3(256), 0, stream>>>((const uint16_t*)x, n.gamma, (int)K, n.eps, (int8_t*)xq, (float*)sa, mt);
+    kern<<<dim3((unsigned)M), dim3(256), 0, stream>>>((const uint16_t*)x, n.gamma, (int)K, n.eps, (int8_t*)xq, (float*)sa, mt,
+                                                      mt == 0 && M < 128); // (launch_quant_act_int8's choice)
     return hipGetLastError();
   };
   const bool f32 = n.dtype == TPPX_DT_F32;

@@ -436,6 +436,52 @@ def test_environment_switches_are_read_once(monkeypatch):
     assert "skinny_qint8_fq_kernel" in plan()
 
 
+def test_forced_prompt_tiles(monkeypatch):
+    """TPPX_TILED_BIG_TILE by number, with the workgroups that the tile makes of the launch: 1 .. 4 and, from 7 on, the wave tiles
+    of MXFP4 weights, whole and, on the three that have them, with K in slices; what is not built is left to the estimates."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+    buf = ctypes.create_string_buffer(4096)
+    M, N, K = 300, 4512, 4096
+
+    def plan(tile, split=0):
+        monkeypatch.setenv("TPPX_TILED_MIN_M", "0")
+        monkeypatch.setenv("TPPX_TILED_BIG_TILE", str(tile))
+        monkeypatch.setenv("TPPX_TILED_SPLIT", str(split))
+        L.tppx_reload_env()
+        _lib.check(L.tppx_plan_linear_mxfp4(M, N, K, 0, 1 << 25, buf, len(buf)))
+        return buf.value.decode()
+
+    def grid(rows, cols, slices=1):
+        return f"grid={(M + rows - 1) // rows * ((N + cols - 1) // cols)}x{slices}x1"
+
+    try:
+        for tile, name, rows, cols in ((1, "big_mxfp4_kernel<8, false, 2, 4>", 256, 256), (2, "big_mxfp4_kernel<8, false, 1, 4>", 128, 256),
+                                       (3, "big_mxfp4_kernel<8, false, 1, 8>", 128, 512), (4, "wide_kernel<4, 2, 4, false, false, false>", 64, 128)):
+            assert f"{name} {grid(rows, cols)}" in plan(tile), tile
+        forms = ((2, 1, 8), (3, 2, 4), (4, 2, 4), (5, 2, 4), None, (4, 3, 4), (5, 3, 4), (5, 2, 8), (6, 2, 8), (4, 3, 8), (6, 3, 8))
+        free = plan(0)
+        for tile, form in enumerate(forms, 7):
+            if form is None:
+                assert plan(tile) == free
+                continue
+            mt, nt, w = form
+            assert f"wide_kernel<{mt}, {nt}, {w}, false, false, false> {grid(mt * 16, nt * w * 16)} block={w * 64}" in plan(tile), tile
+        assert plan(5) == free and plan(6) == free and plan(18) == free
+        for tile, (mt, nt, w) in ((4, (4, 2, 4)), (7, (2, 1, 8)), (8, (3, 2, 4)), (9, (4, 2, 4))):
+            for S in (2, 3, 4, 6):
+                lines = plan(tile, S).splitlines()
+                rows, cols = mt * 16, nt * w * 16
+                fits = (M + rows - 1) // rows * ((N + cols - 1) // cols) * S * rows * cols * 4 <= 1 << 25
+                assert f"wide_kernel<{mt}, {nt}, {w}, false, false, {'true' if fits else 'false'}> {grid(rows, cols, S if fits else 1)}" in lines[0]
+                assert len(lines) == 1 + fits and (not fits or f"wide_sum_kernel<{mt}, {nt}, {w}, {S}>" in lines[1])
+        assert len(plan(10, 4).splitlines()) == 1  # 80 x 128: K whole
+    finally:
+        monkeypatch.undo()
+        L.tppx_reload_env()
+
+
 def test_cache_lengths_after_graph_replayed_steps():
     """Steps replayed from a graph move the device counter themselves; the host bookkeeping that follows them must
     move every layer's length, so that get_seq_length(layer) and a later update() on any layer see the new keys."""

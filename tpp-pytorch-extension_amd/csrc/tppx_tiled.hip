@@ -1613,10 +1613,21 @@ static hipError_t split_launch(Kern kern, size_t lds, BigParams& P, int wgs, int
                                                                                           : sum(side_sum_kernel<4, 4, 6>);
 }
 
-// TPPX_TILED_BIG_TILE: 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128 and 6 = 64 x 256 (bf16 weights), from 7 on
+// TPPX_TILED_BIG_TILE: 1 = 256 x 256, 2 = 128 x 256, 3 = 128 x 512, 4 = 64 x 128, 6 = 64 x 256 (bf16 weights), from 7 on
 // WIDE_FORMS; what is not built for the weights, 5 too, is left to the estimates
+constexpr int wide_form(int mt, int nt, int w) {
+  for (int i = 0; i < N_WIDE; i++)
+    if (WIDE_FORMS[i].mt == mt && WIDE_FORMS[i].nt == nt && WIDE_FORMS[i].w == w)
+      return i;
+  return -1;
+}
+template <bool WBF16>
 static int forced_tile() {
+  constexpr int small = wide_form(4, 2, 4); // MXFP4's 64 x 128
+  static_assert(small >= 0 && WIDE_FORMS[small].mxfp4);
   const int t = env_int("TPPX_TILED_BIG_TILE", 0);
+  if (!WBF16 && t == 4)
+    return TILE_WIDE + small;
   return t >= 1 && t <= 4 ? t - 1 : t == 6 ? TILE_64_256 : t >= 7 && t < 7 + N_WIDE ? TILE_WIDE + t - 7 : -1;
 }
 
@@ -1634,7 +1645,7 @@ static int forced_slices(bool can, const TiledParams* t, int n, int tile, int64_
 hipError_t launch_tiled_mxfp4_group(const TiledParams* t, int n, hipStream_t stream, bool dual, float* part, int64_t part_bytes) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
-  int shape = forced_tile(), S = 1;
+  int shape = forced_tile<false>(), S = 1;
   if (shape < 0 || shape >= N_TILES || !(MXFP4_COST[shape].b > 0.0))
     shape = cheapest_tile<false>(t, n, dual, part ? part_bytes : 0, &S);
   else if (shape >= TILE_WIDE)
@@ -1744,7 +1755,7 @@ bool tiled_bf16_takes_groups(const TiledParams& p) {
 hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stream, bool dual, float* part, int64_t part_bytes) {
   if (dual && (n != 2 || t[0].tiles != t[1].tiles || t[0].K != t[1].K || t[0].M != t[1].M || t[0].x != t[1].x))
     return hipErrorInvalidValue;
-  int shape = forced_tile(), S = 1;
+  int shape = forced_tile<true>(), S = 1;
   if (shape < 0 || shape >= N_TILES || !(BF16_COST[shape].b > 0.0))
     shape = cheapest_tile<true>(t, n, dual, part ? part_bytes : 0, &S);
   BigParams P;
@@ -1761,7 +1772,7 @@ hipError_t launch_tiled_bf16_group(const TiledParams* t, int n, hipStream_t stre
   case TILE_64_256:
     return dual ? big_bf16_launch<2, true, 2, 4>(P, wgs, stream) : big_bf16_launch<2, false, 2, 4>(P, wgs, stream);
   case TILE_128_256:
-    if (wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0) // at most one workgroup per CU: eight waves, as for MXFP4
+    if (wgs <= 256 && env_int("TPPX_TILED_W8", 1) != 0) // at most one workgroup per CU: eight waves side by side
       return dual ? big_bf16_launch<4, true, 2, 4>(P, wgs, stream) : big_bf16_launch<4, false, 2, 4>(P, wgs, stream);
     return dual ? big_bf16_launch<8, true, 1, 4>(P, wgs, stream) : big_bf16_launch<8, false, 1, 4>(P, wgs, stream);
   default:

@@ -337,7 +337,9 @@ def test_kernel_family_of_short_prompts():
         assert "skinny_mxfp4" in pair(M, 1024, 4096) and "skinny_mxfp4" in pair(M, 1536, 18944), M  # 11 us (tiles 22), 38 (79)
         assert "wide_kernel" in one(M, 28672, 2560) and "wide_kernel" in one(M, 18944, 1024), M     # (rows 52 us, 26)
         assert "wide_kernel" in pair(M, 11008, 4096), M                                            # (rows 42 us)
-    assert "skinny_mxfp4" in pair(160, 1024, 8192)                                                  # 19 us (tiles 38)
+    assert "skinny_mxfp4" in pair(160, 1024, 8192)                                                  # 15.4 us
+    assert "wide_kernel<2, 1, 8, true, false, false>" in pair(256, 1024, 8192)                      # 21.3 us (rows 20.7: a near tie)
+    assert "skinny_mxfp4" in one(160, 1024, 18944) and "skinny_mxfp4" in one(256, 1024, 18944)      # 38 us, 33
     assert "wide_kernel" in one(192, 14336, 5120)                                                   # (rows 65 us)
     assert "<5, 2, 8," in one(1800, 2560, 11008) and "<5, 2, 4," in one(1500, 1536, 18944)
     assert "<8, true, 1, 8>" in pair(2048, 28672, 8192)                                             # 1254 us (128 x 256: 1283)
@@ -354,7 +356,8 @@ def test_kernel_family_of_short_prompts():
     # long prompts: not the small wave tiles, whose workgroups drift apart in K where the XCDs get whole columns
     for shape in ((2048, 9088, 8704), (1744, 6528, 10496), (1421, 4096, 11008), (1421, 4096, 4096), (2048, 4800, 4096)):
         assert not any(small in one(*shape) for small in ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,")), shape
-    assert "<3, 2, 4," not in qkv(2048, 1856, 13312) and "<4, 2, 4," not in pair(2048, 2880, 7168)
+    for small in ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,", "<5, 2, 4,"):
+        assert small not in qkv(2048, 1856, 13312) and small not in pair(2048, 2880, 7168), small   # 226 us, 131
 
     # the wave tiles of up to 80 rows drift from 18 row blocks on, in more than a round of workgroups and without rectangles
     assert "<6, 3, 8," in one(1978, 3136, 10240)                                                    # 111 us (80 x 128: 127)
@@ -434,6 +437,23 @@ def test_environment_switches_are_read_once(monkeypatch):
         del os.environ["TPPX_SKINNY_FUSEDQ"]
         L.tppx_reload_env()
     assert "skinny_qint8_fq_kernel" in plan()
+
+
+def test_kernels_of_few_rows_and_uneven_wave_slices():
+    """K between 2048 and 4096 whose tiles do not divide by the sixteen waves: the LDS-staged kernel for up to 4 rows, the
+    tile-by-tile one for more; single, grouped and as the pair."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+    buf = ctypes.create_string_buffer(4096)
+    for M, N, K in ((1, 96, 2176), (4, 4128, 2560), (3, 8224, 3584), (2, 12320, 3968), (4, 32, 3584), (5, 96, 3584), (16, 4128, 2560)):
+        name = "skinny_mxfp4_xl_kernel<" if M <= 4 else "skinny_mxfp4_mg_kernel<"
+        plans = [(L.tppx_plan_linear_mxfp4, (M, N, K, 0, 1 << 25))]
+        for ns, dual in (((N, 32, N), 0), ((N, N), 1)):
+            plans.append((L.tppx_plan_multi_linear_mxfp4, ((ctypes.c_int64 * len(ns))(*ns), len(ns), M, K, dual, 0, 1 << 25)))
+        for fn, args in plans:
+            _lib.check(fn(*args, buf, len(buf)))
+            assert name in buf.value.decode(), (M, N, K, buf.value)
 
 
 def test_forced_prompt_tiles(monkeypatch):
@@ -626,5 +646,6 @@ def test_mxfp4_prompts_run_k_in_slices_where_that_pays():
     for shape in ((4096, 11008, 100), (4096, 11008, 200), (2560, 10240, 200), (3584, 18944, 333)):
         assert split(*shape), shape
     for shape in ((1408, 9216, 1024), (1408, 11520, 970), (9024, 10496, 183), (4096, 11008, 400), (6400, 9984, 234), (2496, 13056, 725),
-                  (1600, 9984, 847), (4096, 11008, 333), (4096, 16384, 420), (3584, 18944, 480)):
+                  (1600, 9984, 847), (4096, 11008, 333), (4096, 16384, 420), (3584, 18944, 480),
+                  (4096, 11008, 300), (2112, 4608, 381), (8512, 6400, 65)):  # 44.7 us (in slices 43.7), 16.7 (19.6), 26.8 (28.7)
         assert not split(*shape), shape

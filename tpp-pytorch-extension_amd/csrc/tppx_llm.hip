@@ -10,38 +10,10 @@
 
 #include "tppx_common.h"
 #include "tppx_launch.h"
+#include "tppx_norm.h"
 
 namespace tppx {
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_mov(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
-}
-// sum / max over the 16 lanes of a DPP row; every lane of the row gets the result
-__device__ __forceinline__ float row16_sum(float v) {
-  v += dpp_mov<0xB1>(v);  // quad_perm [1,0,3,2]
-  v += dpp_mov<0x4E>(v);  // quad_perm [2,3,0,1]
-  v += dpp_mov<0x141>(v); // row_half_mirror
-  v += dpp_mov<0x140>(v); // row_mirror
-  return v;
-}
-__device__ __forceinline__ float wave_sum(float v) {
-  v = row16_sum(v);
-  float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-  float b = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
-  float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-  float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
-  return (a + b) + (c + d);
-}
-
-__device__ __forceinline__ void unpack8(const uint4& w, float (&f)[8]) {
-  const uint32_t d[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    f[2 * i] = bf16_bits_to_f32(d[i] & 0xffffu);
-    f[2 * i + 1] = bf16_bits_to_f32(d[i] >> 16);
-  }
-}
 __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   uint32_t d[4];
 #pragma unroll
@@ -71,12 +43,7 @@ rms_norm_kernel(const uint16_t* __restrict__ x, const void* __restrict__ gamma, 
     for (int e = 0; e < 8; e++)
       ss = fmaf(f[e], f[e], ss);
   }
-  ss = wave_sum(ss);
-  if ((tid & 63) == 0)
-    red[tid >> 6] = ss;
-  __syncthreads();
-  const float v = ((red[0] + red[1]) + (red[2] + red[3])) * (1.0f / (float)K);
-  const float s = 1.0f / sqrtf(v + eps);
+  const float s = rms_scale(ss, red, K, eps);
   for (int i = tid; i < nchunk; i += 256) {
     float f[8], g[8];
     unpack8(xr[i], f); // second read hits L2/L1
@@ -138,12 +105,7 @@ rms_norm_regs_kernel(const uint16_t* __restrict__ x, const void* __restrict__ ga
         ss = fmaf(f[e], f[e], ss);
     }
   }
-  ss = wave_sum(ss);
-  if ((tid & 63) == 0)
-    red[tid >> 6] = ss;
-  __syncthreads();
-  const float v = ((red[0] + red[1]) + (red[2] + red[3])) * (1.0f / (float)K);
-  const float s = 1.0f / sqrtf(v + eps);
+  const float s = rms_scale(ss, red, K, eps);
 #pragma unroll
   for (int c = 0; c < NC; c++) {
     if (tid + c * 256 >= nchunk)

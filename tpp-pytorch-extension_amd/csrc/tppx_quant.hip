@@ -2,6 +2,7 @@
 // weight except for the activation quantizer which runs on every QINT8 call).
 #include "tppx_common.h"
 #include "tppx_launch.h"
+#include "tppx_norm.h"
 
 namespace tppx {
 
@@ -617,22 +618,6 @@ quant_act_int8_rows_kernel(const uint16_t* __restrict__ x, int64_t M, int64_t K,
   }
 }
 
-// sum over the wave in tppx_rms_norm's order
-__device__ __forceinline__ float norm_wave_sum(float v) {
-  auto dpp = [](float v, auto CTRL) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(CTRL)::value, 0xf, 0xf, true));
-  };
-  v += dpp(v, std::integral_constant<int, 0xB1>{});  // quad_perm [1,0,3,2]
-  v += dpp(v, std::integral_constant<int, 0x4E>{});  // quad_perm [2,3,0,1]
-  v += dpp(v, std::integral_constant<int, 0x141>{}); // row_half_mirror
-  v += dpp(v, std::integral_constant<int, 0x140>{}); // row_mirror
-  const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-  const float b = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
-  const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-  const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
-  return (a + b) + (c + d);
-}
-
 // RMSNorm and the kernel above in one pass: y = bf16((x * rsqrt(mean(x^2) + eps)) * gamma) stays in registers and leaves as
 // int8 values and scales only, the bits of tppx_rms_norm followed by the quantizer.  A workgroup of 256 threads per row, NC
 // chunks of 8 values per thread (K up to 8192); 32 consecutive threads share a block of 256.  Bound by what it reads and
@@ -661,43 +646,30 @@ rms_norm_quant_int8_kernel(const uint16_t* __restrict__ x, const void* __restric
       gb[c] = reinterpret_cast<const uint4*>(gamma)[i];
     }
   }
-  auto unpack = [](const uint4& v, float (&f)[8]) {
-    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      f[2 * i] = bf16_bits_to_f32(d[i] & 0xffffu);
-      f[2 * i + 1] = bf16_bits_to_f32(d[i] >> 16);
-    }
-  };
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < NC; c++) {
     float f[8];
-    unpack(w[c], f);
+    unpack8(w[c], f);
     if (tid + c * 256 < nchunk) {
 #pragma unroll
       for (int e = 0; e < 8; e++)
         ss = fmaf(f[e], f[e], ss);
     }
   }
-  ss = norm_wave_sum(ss);
-  if ((tid & 63) == 0)
-    red[tid >> 6] = ss;
-  __syncthreads();
-  const float v = ((red[0] + red[1]) + (red[2] + red[3])) * (1.0f / (float)K);
-  const float s = 1.0f / sqrtf(v + eps);
+  const float s = rms_scale(ss, red, K, eps);
 #pragma unroll
   for (int c = 0; c < NC; c++) {
     const int i = tid + c * 256;
     if (i >= nchunk) // (whole blocks of 32 threads: K is a multiple of 256)
       break;
     float f[8], g[8];
-    unpack(w[c], f);
+    unpack8(w[c], f);
     if (GAMMA_F32) {
       g[0] = g4[c][0].x; g[1] = g4[c][0].y; g[2] = g4[c][0].z; g[3] = g4[c][0].w;
       g[4] = g4[c][1].x; g[5] = g4[c][1].y; g[6] = g4[c][1].z; g[7] = g4[c][1].w;
     } else {
-      unpack(gb[c], g);
+      unpack8(gb[c], g);
     }
 #pragma unroll
     for (int e = 0; e < 8; e++)

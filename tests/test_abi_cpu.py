@@ -337,9 +337,7 @@ def test_kernel_family_of_short_prompts():
         assert "skinny_mxfp4" in pair(M, 1024, 4096) and "skinny_mxfp4" in pair(M, 1536, 18944), M  # 11 us (tiles 22), 38 (79)
         assert "wide_kernel" in one(M, 28672, 2560) and "wide_kernel" in one(M, 18944, 1024), M     # (rows 52 us, 26)
         assert "wide_kernel" in pair(M, 11008, 4096), M                                            # (rows 42 us)
-    assert "skinny_mxfp4" in pair(160, 1024, 8192)                                                  # 15.4 us
-    assert "wide_kernel<2, 1, 8, true, false, false>" in pair(256, 1024, 8192)                      # 21.3 us (rows 20.7: a near tie)
-    assert "skinny_mxfp4" in one(160, 1024, 18944) and "skinny_mxfp4" in one(256, 1024, 18944)      # 38 us, 33
+    assert "skinny_mxfp4" in pair(160, 1024, 8192)                                                  # 19 us (tiles 38)
     assert "wide_kernel" in one(192, 14336, 5120)                                                   # (rows 65 us)
     assert "<5, 2, 8," in one(1800, 2560, 11008) and "<5, 2, 4," in one(1500, 1536, 18944)
     assert "<8, true, 1, 8>" in pair(2048, 28672, 8192)                                             # 1254 us (128 x 256: 1283)
@@ -356,13 +354,7 @@ def test_kernel_family_of_short_prompts():
     # long prompts: not the small wave tiles, whose workgroups drift apart in K where the XCDs get whole columns
     for shape in ((2048, 9088, 8704), (1744, 6528, 10496), (1421, 4096, 11008), (1421, 4096, 4096), (2048, 4800, 4096)):
         assert not any(small in one(*shape) for small in ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,")), shape
-    for small in ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,", "<5, 2, 4,"):
-        assert small not in qkv(2048, 1856, 13312) and small not in pair(2048, 2880, 7168), small   # 226 us, 131
-
-    # the wave tiles of up to 80 rows drift from 18 row blocks on, in more than a round of workgroups and without rectangles
-    assert "<6, 3, 8," in one(1978, 3136, 10240)                                                    # 111 us (80 x 128: 127)
-    for M, N, K in ((1740, 4160, 9216), (1990, 3136, 12288), (1850, 2112, 6400)):
-        assert not any(small in one(M, N, K) for small in ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,", "<5, 2, 4,")), (M, N, K)
+    assert "<3, 2, 4," not in qkv(2048, 1856, 13312) and "<4, 2, 4," not in pair(2048, 2880, 7168)
 
     def per_weight(M, N, K, weight_bytes):
         return not L.tppx_group_is_one_launch((ctypes.c_int64 * 2)(N, N), 2, M, K, weight_bytes)
@@ -412,6 +404,47 @@ def test_group_is_one_launch():
     for M in (1, 17, 64):
         assert one([4096, 1024, 1024], M, 4096, 2) == 1 and one([1 << 20] * 2, M, 2048, 2) == 1  # (weights of 4 GiB too)
         assert one([4096, 1024], M, 4032, 2) == 0  # K in no whole tiles
+
+
+def test_prompt_plans_by_tile_and_grid(monkeypatch):
+    """What the tests above leave open of MXFP4 prompts: the family of few channels at a long K, which of the small wave tiles,
+    whole K where slices measured slower or as fast, and the launches of a forced number of slices."""
+    import ctypes
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+    buf = ctypes.create_string_buffer(4096)
+
+    def one(M, N, K):
+        _lib.check(L.tppx_plan_linear_mxfp4(M, N, K, 0, 1 << 25, buf, len(buf)))
+        return buf.value.decode()
+
+    def group(M, ns, K, dual):
+        _lib.check(L.tppx_plan_multi_linear_mxfp4((ctypes.c_int64 * len(ns))(*ns), len(ns), M, K, dual, 0, 1 << 25, buf, len(buf)))
+        return buf.value.decode()
+
+    assert "skinny_mxfp4" in one(160, 1024, 18944) and "skinny_mxfp4" in one(256, 1024, 18944)      # 38 us, 33
+    assert "wide_kernel<2, 1, 8, true, false, false>" in group(256, (1024, 1024), 8192, 1)          # 21.3 us (rows 20.7: a near tie)
+    # the wave tiles of up to 80 rows drift from 18 row blocks on, in more than a round of workgroups and without rectangles
+    small = ("<2, 1, 8,", "<3, 2, 4,", "<4, 2, 4,", "<5, 2, 4,")
+    assert "<6, 3, 8," in one(1978, 3136, 10240)                                                    # 111 us (80 x 128: 127)
+    for plan in (group(2048, (1856,) * 3, 13312, 0), group(2048, (2880,) * 2, 7168, 1),             # 226 us, 131
+                 one(1740, 4160, 9216), one(1990, 3136, 12288), one(1850, 2112, 6400)):
+        assert not any(t in plan for t in small), plan
+    for M, N, K in ((300, 4096, 11008), (381, 2112, 4608), (65, 8512, 6400)):  # 44.7 us (in slices 43.7), 16.7 (19.6), 26.8 (28.7)
+        assert "wide_sum_kernel" not in one(M, N, K), (M, N, K)
+    try:
+        monkeypatch.setenv("TPPX_TILED_MIN_M", "0")
+        for S, M, N, K in ((2, 65, 160, 1152), (3, 200, 288, 1792), (4, 129, 2080, 2048), (6, 100, 32, 3072), (6, 333, 416, 4224)):
+            monkeypatch.setenv("TPPX_TILED_SPLIT", str(S))
+            L.tppx_reload_env()
+            mt, nt, w = (3, 2, 4) if N * M > 100000 else (2, 1, 8)  # (row tiles and channel tiles of a wave, waves)
+            wgs = -(-M // (mt * 16)) * -(-N // (nt * w * 16))
+            gemm, add = one(M, N, K).splitlines()
+            assert f"wide_kernel<{mt}, {nt}, {w}, false, false, true> grid={wgs}x{S}x1 block={w * 64}" in gemm
+            assert f"wide_sum_kernel<{mt}, {nt}, {w}, {S}> grid={wgs * w}x1x1" in add
+    finally:
+        monkeypatch.undo()
+        L.tppx_reload_env()
 
 
 def test_environment_switches_are_read_once(monkeypatch):
@@ -646,6 +679,5 @@ def test_mxfp4_prompts_run_k_in_slices_where_that_pays():
     for shape in ((4096, 11008, 100), (4096, 11008, 200), (2560, 10240, 200), (3584, 18944, 333)):
         assert split(*shape), shape
     for shape in ((1408, 9216, 1024), (1408, 11520, 970), (9024, 10496, 183), (4096, 11008, 400), (6400, 9984, 234), (2496, 13056, 725),
-                  (1600, 9984, 847), (4096, 11008, 333), (4096, 16384, 420), (3584, 18944, 480),
-                  (4096, 11008, 300), (2112, 4608, 381), (8512, 6400, 65)):  # 44.7 us (in slices 43.7), 16.7 (19.6), 26.8 (28.7)
+                  (1600, 9984, 847), (4096, 11008, 333), (4096, 16384, 420), (3584, 18944, 480)):
         assert not split(*shape), shape

@@ -311,9 +311,9 @@ def test_decode_step_with_rotary_and_append_in_the_launch(H, HR, style, B, Nq, N
 @pytest.mark.parametrize("H,HR,style,Nq,wide", [(128, 128, "llama", 4, "0"), (128, 128, "llama", 4, "1"), (128, 128, "llama", 32, "1"),
                                                 (64, 64, "llama", 4, "1"), (80, 32, "gptj", 4, "1"), (256, 64, "gptj", 4, "1"), (200, 80, "llama", 8, "1")])
 def test_every_rotation_leaves_the_same_key(H, HR, style, Nq, wide, monkeypatch):
-    """The launches that rotate a new key agree in every bit: the second value's product rounded, the first one's fused into
-    it.  The table is made so that each pair's first (even pairs) or second (odd pairs) value nearly cancels and what is left is
-    the products' rounding; the keys are one row scaled by powers of two."""
+    """The launches that rotate a new key agree in every bit: the sine's product rounded, the cosine's fused into it.  The table is
+    made so that each pair's first (even pairs) or second (odd pairs) value nearly cancels and what is left is the products'
+    rounding; the keys are one row scaled by powers of two."""
     from tpp_pytorch_extension import _lib
     _llm()
     monkeypatch.setenv("TPPX_ATTN_WIDE", wide)
@@ -337,8 +337,8 @@ def test_every_rotation_leaves_the_same_key(H, HR, style, Nq, wide, monkeypatch)
     want = k.clone()
     k1, k2 = k[..., i1].double(), k[..., i2].double()  # (24 + 8 bits: products exact, and so are the sums, in float64)
     want[..., i1] = (k1 * cos.double() - (k2 * sin.double()).float().double()).float().to(torch.bfloat16)
-    want[..., i2] = (k1 * sin.double() + (k2 * cos.double()).float().double()).float().to(torch.bfloat16)
-    own = (k2 * cos.double() + (k1 * sin.double()).float().double()).float().to(torch.bfloat16)
+    want[..., i2] = (k2 * cos.double() + (k1 * sin.double()).float().double()).float().to(torch.bfloat16)
+    own = (k1 * sin.double() + (k2 * cos.double()).float().double()).float().to(torch.bfloat16)
     assert (own != want[..., i2]).float().mean() > 0.2  # (the other order is told apart)
 
     dev = lambda a: a.cuda().contiguous()  # noqa: E731

@@ -62,14 +62,14 @@ __device__ __forceinline__ float round_bf16(float f) {
   return bf16_bits_to_f32(f32_to_bf16_bits(f));
 }
 
-// Rotation of a pair by (c, s): x1 c - x2 s and x2 c + x1 s, the first value's product fused into the rounded product of the
-// second.  In a plain sum of two products the compiler chooses which one is fused, by kernel; the launches that rotate have to
-// agree in every bit, also where the two nearly cancel, for a cache filled by one of them and read behind another.
+// Rotation of a pair by (c, s): x1 c - x2 s and x2 c + x1 s, the cosine's product fused into the rounded product of the sine.  In
+// a plain sum of two products the compiler chooses which one is fused, by kernel; the launches that rotate have to agree in
+// every bit, also where the two nearly cancel, for a cache filled by one of them and read behind another.
 __device__ __forceinline__ float rotate_first(float x1, float x2, float c, float s) {
   return fmaf(x1, c, -__fmul_rn(x2, s));
 }
 __device__ __forceinline__ float rotate_second(float x1, float x2, float c, float s) {
-  return fmaf(x1, s, __fmul_rn(x2, c));
+  return fmaf(x2, c, __fmul_rn(x1, s));
 }
 
 // ---- post-ops on the bf16-rounded GEMM result -------------------------------

@@ -2360,7 +2360,7 @@ attn_hd_step_kernel(const AttnGenParams p) {
   // A wave's loads return in the order of their issue: wave 0 asks for the query and the new key first (dims lane + 64 i)
   constexpr int D = G * J / 8;           // head dims per lane of wave 0
   i32x4 qp[J];
-  float q1[D], q2[D], k1[D], k2[D], f1[D], f2[D]; // the pair of dim d and what its two values are multiplied with
+  float qx[D], qo[D], kx[D], ko[D], cs[D], sn[D]; // value, its pair's other half, cos, signed sin
   bool turned[D];
   if (!APP) {
 #pragma unroll
@@ -2376,20 +2376,20 @@ attn_hd_step_kernel(const AttnGenParams p) {
     for (int i = 0; i < D; i++) {
       const int d = min(lane + 64 * i, H - 1);
       const bool turn = rot && d < p.HR;
-      const bool second = turn && (p.gptj ? (d & 1) : d >= half);
+      const bool second = p.gptj ? (d & 1) : d >= half;
       const int o = !turn ? d : p.gptj ? d ^ 1 : second ? d - half : d + half;
       const int e = p.gptj ? d >> 1 : second ? d - half : d;
-      q1[i] = bf16_bits_to_f32(qrow[second ? o : d]);
-      q2[i] = bf16_bits_to_f32(qrow[second ? d : o]);
-      k1[i] = bf16_bits_to_f32(krow[second ? o : d]);
-      k2[i] = bf16_bits_to_f32(krow[second ? d : o]);
-      f1[i] = f2[i] = 0.f;
+      qx[i] = bf16_bits_to_f32(qrow[d]);
+      qo[i] = bf16_bits_to_f32(qrow[o]);
+      kx[i] = bf16_bits_to_f32(krow[d]);
+      ko[i] = bf16_bits_to_f32(krow[o]);
+      cs[i] = sn[i] = 0.f;
       turned[i] = turn;
       if (turn) {
-        const float cs = p.gptj ? p.emb[pp * p.HR + half + e] : p.emb[pp * p.HR + e];
-        const float sn = p.gptj ? p.emb[pp * p.HR + e] : p.emb[((int64_t)p.MP + pp) * p.HR + e];
-        f1[i] = second ? sn : cs;
-        f2[i] = second ? cs : -sn;
+        cs[i] = p.gptj ? p.emb[pp * p.HR + half + e] : p.emb[pp * p.HR + e];
+        sn[i] = p.gptj ? p.emb[pp * p.HR + e] : p.emb[((int64_t)p.MP + pp) * p.HR + e];
+        if (!second)
+          sn[i] = -sn[i];
       }
     }
   }
@@ -2407,9 +2407,9 @@ attn_hd_step_kernel(const AttnGenParams p) {
       for (int i = 0; i < D; i++) {
         const int d = lane + 64 * i;
         if (d < H) {
-          // rotate_first or rotate_second, as one form (the first value's product is the fused one in both)
-          q_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(q1[i], f1[i], __fmul_rn(q2[i], f2[i])) : q1[i]);
-          k_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(k1[i], f1[i], __fmul_rn(k2[i], f2[i])) : k1[i]);
+          // rotate_first and rotate_second, the sign in sn
+          q_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(qx[i], cs[i], __fmul_rn(qo[i], sn[i])) : qx[i]);
+          k_s[d] = (uint16_t)f32_to_bf16_bits(turned[i] ? fmaf(kx[i], cs[i], __fmul_rn(ko[i], sn[i])) : kx[i]);
         }
       }
     }

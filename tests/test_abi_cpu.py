@@ -447,6 +447,24 @@ def test_prompt_plans_by_tile_and_grid(monkeypatch):
         L.tppx_reload_env()
 
 
+def test_mxfp4_prompts_of_few_channels_run_a_long_k_in_slices():
+    """Fewer than 2048 channels: in slices where the decode kernels end and a few dozen workgroups would walk a long K, whole for
+    many row blocks, up to K = 4096 and, on the decode kernels, for few rows."""
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+    buf = ctypes.create_string_buffer(4096)
+
+    def plan(m, n, k):
+        _lib.check(L.tppx_plan_linear_mxfp4(m, n, k, 0, 32 << 20, buf, len(buf)))
+        return buf.value.decode()
+
+    for shape in ((320, 1024, 18176), (677, 512, 12288), (257, 1920, 8192), (512, 768, 18176), (400, 1344, 12288), (320, 1024, 8192)):
+        assert "wide_sum_kernel" in plan(*shape), shape  # whole 40.1 us, 24.6, 18.1, 35.0, 24.8, 17.6; in slices 22.5, 17.8, 17.5, 21.9, 22.5, 14.9
+    for shape in ((1400, 768, 12288), (1400, 512, 8192), (677, 512, 4096), (1024, 1408, 9216)):
+        assert "wide_kernel" in plan(*shape) and "wide_sum_kernel" not in plan(*shape), shape
+    assert "skinny_mxfp4" in plan(256, 1024, 18944) and "skinny_mxfp4" in plan(200, 512, 8192)
+
+
 def test_environment_switches_are_read_once(monkeypatch):
     """The library keeps a TPPX_* switch after its first read (no getenv per launch, and a captured graph's kernel
     choice cannot drift); tppx_reload_env() makes it read again."""

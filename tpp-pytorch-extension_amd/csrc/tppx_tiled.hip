@@ -1458,8 +1458,12 @@ static int64_t slice_bytes(int tile) { return (int64_t)tile_rows(tile) * tile_co
 // slices (1: whole; only with room for their sums in part_bytes).  Slices have to look 3 % faster (bf16 weights 5 %, in more than
 // a round 10 %): they are a second launch, behind and before other kernels (a GPT-J pass of three layers 699 .. 731 us in slices
 // where whole K looked 4 % slower, whole 677 .. 688), and weights at hand in the Infinity Cache gain them less (bf16 8640 x 4608
-// at 124 rows 32.9 and 32.1 us from memory, 22.4 and 25.8 at hand).  Fewer than 2048 channels are not sliced: the decode kernels
-// run those well (1024 x 4096 at 160 .. 256 rows 9 us, slices 10).
+// at 124 rows 32.9 and 32.1 us from memory, 22.4 and 25.8 at hand).
+// Fewer than 2048 channels, MXFP4: up to K = 4096 not sliced (1024 channels at 160 .. 256 rows: decode kernels 9 us, slices 10), and
+// the estimate that is weighed against the decode kernels is the one of whole K.  With a longer K and more rows than those run
+// well a few dozen workgroups have all of it to walk: 1024 x 18176 at 320 rows 40.1 us whole, 22.5 in slices, 512 x 12288 at 677
+// 24.6 and 17.8, 1920 x 8192 at 257 18.1 and 17.5.  More row blocks read the same weights: 1 % for each of 64 rows from the fifth
+// on (768 x 12288 at 1400 rows 33.6 whole, 40.4 in slices).  On 156 shapes of 512 .. 1920 channels 1.2 % off the fastest on average.
 template <bool WBF16>
 static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dual, int64_t part_bytes, int* S, double* best_us = nullptr) {
   constexpr const TileCost* COST = WBF16 ? BF16_COST : MXFP4_COST;
@@ -1489,15 +1493,19 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
       shape = i;
       *S = 1;
     }
-    if (dual || forced == 0 || !(COST[i].c0 > 0.0) || (forced == 1 && (WBF16 ? K <= 2560 || wgs > 320 : all < 128)))
+    const bool narrow = !WBF16 && all < 128;
+    if (dual || forced == 0 || !(COST[i].c0 > 0.0) || (forced == 1 && (WBF16 ? K <= 2560 || wgs > 320 : narrow && K <= 4096)))
       continue;
     for (int z : {2, 3, 4, 6}) {
       if (wgs * z * slice_bytes(i) > part_bytes || K / 128 < 4 * z || (forced == 1 && wgs * z > 1024)) // (as far as was measured)
         break;
       c = tile_us(COST[i], i, wgs * z, s / z, mb, false) + COST[i].c0 + COST[i].c1 * (double)(wgs * z * slice_bytes(i)) / 32768.0;
       c *= !WBF16 ? 1.03 : wgs <= 256 ? 1.05 : 1.10;
+      if (narrow)
+        c *= 1.0 + 0.01 * (double)std::max<int64_t>(0, (M + 63) / 64 - 4);
       if (forced == z ? *S != z || c < best : forced == 1 && c < best) {
-        us = std::min(us, c);
+        if (!narrow || forced > 1)
+          us = std::min(us, c);
         best = c;
         shape = i;
         *S = z;

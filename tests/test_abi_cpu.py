@@ -458,8 +458,9 @@ def test_mxfp4_prompts_of_few_channels_run_a_long_k_in_slices():
         _lib.check(L.tppx_plan_linear_mxfp4(m, n, k, 0, 32 << 20, buf, len(buf)))
         return buf.value.decode()
 
-    for shape in ((320, 1024, 18176), (677, 512, 12288), (257, 1920, 8192), (512, 768, 18176), (400, 1344, 12288), (320, 1024, 8192)):
-        assert "wide_sum_kernel" in plan(*shape), shape  # whole 40.1 us, 24.6, 18.1, 35.0, 24.8, 17.6; in slices 22.5, 17.8, 17.5, 21.9, 22.5, 14.9
+    for shape in ((320, 1024, 18176), (677, 512, 12288), (257, 1920, 8192), (512, 768, 18176), (400, 1344, 12288), (320, 1024, 8192),
+                  (3421, 64, 12288)):
+        assert "wide_sum_kernel" in plan(*shape), shape  # whole 40.1 us, 24.6, 18.1, 35.0, 24.8, 17.6; in slices 22.5, 17.8, 17.5, 21.9, 22.5, 14.9 (64 x 12288 24.4, 19.3)
     for shape in ((1400, 768, 12288), (1400, 512, 8192), (677, 512, 4096), (1024, 1408, 9216)):
         assert "wide_kernel" in plan(*shape) and "wide_sum_kernel" not in plan(*shape), shape
     assert "skinny_mxfp4" in plan(256, 1024, 18944) and "skinny_mxfp4" in plan(200, 512, 8192)

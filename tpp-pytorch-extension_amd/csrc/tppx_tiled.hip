@@ -1462,8 +1462,10 @@ static int64_t slice_bytes(int tile) { return (int64_t)tile_rows(tile) * tile_co
 // Fewer than 2048 channels, MXFP4: up to K = 4096 not sliced (1024 channels at 160 .. 256 rows: decode kernels 9 us, slices 10), and
 // the estimate that is weighed against the decode kernels is the one of whole K.  With a longer K and more rows than those run
 // well a few dozen workgroups have all of it to walk: 1024 x 18176 at 320 rows 40.1 us whole, 22.5 in slices, 512 x 12288 at 677
-// 24.6 and 17.8, 1920 x 8192 at 257 18.1 and 17.5.  More row blocks read the same weights: 1 % for each of 64 rows from the fifth
-// on (768 x 12288 at 1400 rows 33.6 whole, 40.4 in slices).  On 156 shapes of 512 .. 1920 channels 1.2 % off the fastest on average.
+// 24.6 and 17.8, 1920 x 8192 at 257 18.1 and 17.5.  Row blocks read the same weights: 1.5 % for each of 64 rows from the fifth to the
+// sixteenth (768 x 12288 at 1400 rows 33.6 whole, 40.4 in slices; 64 x 12288 at 3421 24.4 and 19.3), and 8 % for six slices (1024 x
+// 12288 at 320 rows 18.0, three 15.4).  On 228 shapes of 64 .. 1920 channels and 200 .. 6000 rows the one taken is 1 % off the fastest
+// on average and at most 1.2 % slower than whole K.
 template <bool WBF16>
 static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dual, int64_t part_bytes, int* S, double* best_us = nullptr) {
   constexpr const TileCost* COST = WBF16 ? BF16_COST : MXFP4_COST;
@@ -1502,7 +1504,7 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
       c = tile_us(COST[i], i, wgs * z, s / z, mb, false) + COST[i].c0 + COST[i].c1 * (double)(wgs * z * slice_bytes(i)) / 32768.0;
       c *= !WBF16 ? 1.03 : wgs <= 256 ? 1.05 : 1.10;
       if (narrow)
-        c *= 1.0 + 0.01 * (double)std::max<int64_t>(0, (M + 63) / 64 - 4);
+        c *= 1.0 + 0.015 * (double)std::min<int64_t>(12, std::max<int64_t>(0, (M + 63) / 64 - 4)) + (z == 6 ? 0.08 : 0.0);
       if (forced == z ? *S != z || c < best : forced == 1 && c < best) {
         if (!narrow || forced > 1)
           us = std::min(us, c);

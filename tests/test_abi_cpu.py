@@ -466,6 +466,15 @@ def test_mxfp4_prompts_of_few_channels_run_a_long_k_in_slices():
     assert "skinny_mxfp4" in plan(256, 1024, 18944) and "skinny_mxfp4" in plan(200, 512, 8192)
 
 
+def test_bf16_prompts_near_the_line_between_the_kernels_run_on_tiles():
+    """Launches whose two estimates nearly meet go to the tiles: what decides between two tiles is not weighed against the decode
+    kernels."""
+    from tpp_pytorch_extension import _lib
+    L = _lib.lib()
+    for Ns, M, K in (((1120, 1120), 156, 3584), ((192, 192), 541, 2816), ((1184,), 220, 512)):  # 20.3 us (rows 24.0), 14.0 (16.7), 6.1 (7.6)
+        assert L.tppx_group_is_one_launch((ctypes.c_int64 * len(Ns))(*Ns), len(Ns), M, K, 2), (Ns, M, K)
+
+
 def test_environment_switches_are_read_once(monkeypatch):
     """The library keeps a TPPX_* switch after its first read (no getenv per launch, and a captured graph's kernel
     choice cannot drift); tppx_reload_env() makes it read again."""

@@ -1476,7 +1476,7 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
     all += tiles[i];
   const double s = (double)(K / 128), mb = (double)(all * 32 * K) * 1e-6;
   int shape = 0;
-  double best = 1e300, us = 1e300; // (us: without tile_factor, as the decode kernels' estimates were weighed against it)
+  double best = 1e300, us = 1e300; // (us: without tile_factor, bf16 without what decides ties, as the decode kernels' estimates were weighed against it)
   *S = 1;
   for (int i = 0; i < N_TILES; i++) {
     if (!(allowed >> i & 1u) || (WBF16 && i >= TILE_WIDE && all < 48)) // (fewer than 768 channels: not measured)
@@ -1487,8 +1487,9 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
       nb += (tiles[g] + tpw - 1) / tpw;
     const int64_t rows = (M + tile_rows(i) - 1) / tile_rows(i), wgs = rows * nb;
     // (a near tie goes to the large tiles, which read less)
-    double c = tile_us(COST[i], i, wgs, s, mb, dual) * (i >= TILE_64_128 && i != TILE_64_256 ? 1.01 : 1.0);
-    us = std::min(us, c);
+    const double whole = tile_us(COST[i], i, wgs, s, mb, dual);
+    double c = whole * (i >= TILE_64_128 && i != TILE_64_256 ? 1.01 : 1.0);
+    us = std::min(us, WBF16 ? whole : c);
     c *= tile_factor<WBF16>(i, rows, s, wgs, xcd_split(rows, nb, (double)M, (double)nb * tile_cols16(i) * (WBF16 ? 16.0 : 8.0 * MXFP4_WEIGHT_BYTES)));
     if (c < best && !(forced > 1 && *S > 1)) {
       best = c;
@@ -1501,13 +1502,13 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
     for (int z : {2, 3, 4, 6}) {
       if (wgs * z * slice_bytes(i) > part_bytes || K / 128 < 4 * z || (forced == 1 && wgs * z > 1024)) // (as far as was measured)
         break;
-      c = tile_us(COST[i], i, wgs * z, s / z, mb, false) + COST[i].c0 + COST[i].c1 * (double)(wgs * z * slice_bytes(i)) / 32768.0;
-      c *= !WBF16 ? 1.03 : wgs <= 256 ? 1.05 : 1.10;
+      const double sliced = tile_us(COST[i], i, wgs * z, s / z, mb, false) + COST[i].c0 + COST[i].c1 * (double)(wgs * z * slice_bytes(i)) / 32768.0;
+      c = sliced * (!WBF16 ? 1.03 : wgs <= 256 ? 1.05 : 1.10);
       if (narrow)
         c *= 1.0 + 0.015 * (double)std::min<int64_t>(12, std::max<int64_t>(0, (M + 63) / 64 - 4)) + (z == 6 ? 0.08 : 0.0);
       if (forced == z ? *S != z || c < best : forced == 1 && c < best) {
         if (!narrow || forced > 1)
-          us = std::min(us, c);
+          us = std::min(us, WBF16 ? sliced : c);
         best = c;
         shape = i;
         *S = z;

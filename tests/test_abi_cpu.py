@@ -430,6 +430,9 @@ def test_prompt_plans_by_tile_and_grid(monkeypatch):
     for plan in (group(2048, (1856,) * 3, 13312, 0), group(2048, (2880,) * 2, 7168, 1),             # 226 us, 131
                  one(1740, 4160, 9216), one(1990, 3136, 12288), one(1850, 2112, 6400)):
         assert not any(t in plan for t in small), plan
+    # a short K in more than a round: two workgroups to a CU (286 us on 256 x 256, 246; 92, 75; 111, 99)
+    for plan in (group(3309, (31616,) * 2, 512, 1), group(1981, (20544,) * 2, 256, 1), group(6543, (5280,) * 3, 384, 0)):
+        assert "big_mxfp4_kernel<8, " in plan and ", 1, 4>" in plan, plan
     for M, N, K in ((300, 4096, 11008), (381, 2112, 4608), (65, 8512, 6400)):  # 44.7 us (in slices 43.7), 16.7 (19.6), 26.8 (28.7)
         assert "wide_sum_kernel" not in one(M, N, K), (M, N, K)
     try:

@@ -1348,6 +1348,10 @@ static constexpr int tile_cols16(int tile) { // 16-channel weight tiles (the pai
 // MXFP4: fitted to 888 of 1184 shapes of 65 .. 2048 rows, 768 .. 37888 channels and K = 1024 .. 18944 with every tile forced, whole
 // and in slices, weights in turn from 320 MB; on the others the tile and slices taken are 0.8 % off the fastest on average, 11 % in
 // the worst hundredth.  Larger launches (28672 x 8192 pairs) are extrapolated and stay with the large tiles.
+// MXFP4, K below 1024, more than a round: a workgroup is its first loads and its epilogue, which one alone on its CU has nothing
+// beside.  Of 852 shapes of 65 .. 8192 rows and K = 128 .. 896 with every tile forced 256 x 256 is the fastest in 3 and by its estimate in
+// 72, 128 x 512 in 34 and 81, so there they are not taken: 2 x 31616 x 512 at 3309 rows 285.9 us, on 128 x 256 246.2, 2 x 20544 x 256 at 1981
+// 92 and 75; 1.4 % off the fastest on average, with them 2.4, and none more than 2.5 % slower for it.
 // bf16: the large tiles, 64 x 128 and 64 x 256 fitted to 4100 launches, q/k/v groups among them, up to pairs of 28672 x 8192, most of
 // all where the tile is within 20 % of the fastest, and with weights that come from memory: 96 of them, or as many as fill 2 GB, in
 // turn.  (With four in turn most lie in the Infinity Cache, as they never do in a model, and the estimates came out 20 .. 30 %
@@ -1486,6 +1490,8 @@ static int cheapest_tile(int64_t M, int64_t K, const int* tiles, int n, bool dua
     for (int g = 0; g < (dual ? 1 : n); g++)
       nb += (tiles[g] + tpw - 1) / tpw;
     const int64_t rows = (M + tile_rows(i) - 1) / tile_rows(i), wgs = rows * nb;
+    if (!WBF16 && K < 1024 && wgs > 256 && (i == TILE_256_256 || i == TILE_128_512)) // (two workgroups to a CU instead: see above)
+      continue;
     // (a near tie goes to the large tiles, which read less)
     const double whole = tile_us(COST[i], i, wgs, s, mb, dual);
     double c = whole * (i >= TILE_64_128 && i != TILE_64_256 ? 1.01 : 1.0);

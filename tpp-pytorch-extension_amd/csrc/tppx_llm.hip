@@ -722,8 +722,9 @@ attn_decode_kernel(const AttnParams p) {
 // through LDS at the end.  The first trip's K and V rows (16 KB per wave) are
 // requested before anything else, a later trip's K rows once this trip's scores
 // have freed their registers and its V rows behind this trip's sums, so that a
-// workgroup of many trips never stands without requests; lanes past the length
-// share its last row (a last trip of one key fetched 128).  Against requests at
+// workgroup of many trips never stands without requests; in those lanes past the
+// length share its last row (a last trip of one key fetched 128), while the first
+// is requested before the length is known, up to the cache's end.  Against requests at
 // the start of a trip, rows up to the cache's end, 32 heads: 16 sequences of 2048
 // keys 90 -> 85 us (6.3 TB/s, ends of the launch included), a step of four layers
 // of 32 of 1300 741 -> 707, 2 of 2048 229 -> 222, 1 of 2000 201 -> 199.

@@ -3034,7 +3034,7 @@ hipError_t launch_skinny_w4a8_mg(DecodeParams& p, bool ascending, bool dual, hip
     // half as often: 512 workgroups of one at 128 rows of 4096 x 11008 36.4 us against 39.8, 4096 x 4096 18.1 against
     // 18.4; 768 (192 rows) 56.0 against 50.1 and 26.5 against 23.2.
     const int by = (p.M + 63) / 64;
-    if (dual)
+    if (dual) // (80 pairs of 17 .. 700 rows, 512 .. 16384 channels: 1.30 times as fast as two launches in the mean, 0.99 at worst)
       return sk_launch(skinny_w4a8_rows_kernel<2, true>, p, dim3(p.total_tiles, by, 1), 4, 0, stream);
     if ((int64_t)p.total_tiles * by <= 512)
       return sk_launch(skinny_w4a8_rows_kernel<1, false>, p, dim3(p.total_tiles, by, 1), 4, 0, stream);

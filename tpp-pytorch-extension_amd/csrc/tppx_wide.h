@@ -36,8 +36,8 @@ struct WideGeom {
   static constexpr size_t LDS = (size_t)PD * STAGE > EPB ? (size_t)PD * STAGE : EPB;
 };
 
-// The same with the pairs of a workgroup of four waves dealt out over all of them (an odd NT): slot t = wave * NT + nt is the
-// gate (t even) or the up tile of channel tile t / 2, so the sums of up to 64 rows meet in LDS, two buffers in turn.
+// The gate/up epilogue with the pairs of a workgroup dealt out over its four or eight waves (an odd NT): slot t = wave * NT + nt is the
+// gate (t even) or the up tile of channel tile t / 2, so the sums of 256 / W rows at a time meet in LDS, two buffers in turn.
 template <int MT, int NT, int W>
 __device__ __forceinline__ void wide_epilogue_dual(const TiledParams& pg, const TiledParams& pu, f32x4 (&acc)[MT][NT],
                                                    float* lds, int m_base, int tile_base) {

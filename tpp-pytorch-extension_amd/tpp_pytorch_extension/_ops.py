@@ -774,11 +774,13 @@ def _linear_w4a8(input, weight, bias, post, post_in, post_in2, post_scale, rows=
 def _w4a8_pair(input, w_gate, w_up, b_gate, b_up):
     """silu(gate) * up of W4A8 weights in one launch behind the row quantizer, the bits of the two calls; None where those
     do not both run on the row-group kernels (their own checks and messages then)."""
+    if input.numel() <= 16 * input.shape[-1]:
+        return None
     N, K = w_gate.weight_nk()
     if input.dtype != torch.bfloat16 or input.device.type != "cuda" or input.shape[-1] != K or w_up.weight_nk() != (N, K):
         return None
     M = input.numel() // K
-    if M <= 16 or not _w4a8_takes_groups(M, N, K):
+    if not _w4a8_takes_groups(M, N, K):
         return None
     x = input.contiguous()
     nat_g, nat_u = w_gate.native_w4a8(), w_up.native_w4a8()
